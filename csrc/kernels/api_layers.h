@@ -162,6 +162,10 @@ struct MoeGroupedParams {
   int f32;
 };
 
+// Shapes that the pipelined expert GEMMs take (moe_pipe.hip): reduction lengths of whole 64-element steps, two at least;
+// 16-byte-aligned operands; every operand inside a 2 GiB buffer range; and enough rows to be worth it.
+bool moe_pipe_ok(const MoeGroupedParams& p);
+
 // Router, choice and work list of a decode-sized step in one launch.
 struct MoeRouteRowsParams {
   const float* x;        // [M, W]
@@ -179,6 +183,7 @@ struct MoeRouteRowsParams {
 }  // namespace dsse
 
 extern "C" {
+hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st);  // the GEMMs alone: the work list is ready
 hipError_t dsse_gemm_rm(const dsse::GemmRmParams* p, hipStream_t st);
 hipError_t dsse_scalar_norm(const dsse::ScalarNormParams* p, hipStream_t st);
 // resid = embed[ids] * scale + table[positions] (table fp32 [table_len, W] or null); xb (or null) the same rounded

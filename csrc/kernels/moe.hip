@@ -10,6 +10,7 @@
 #include "api_layers.h"
 #include "api_memory.h"
 #include "frag.h"
+#include "moe_rows.h"
 
 namespace dsse {
 namespace {
@@ -152,24 +153,6 @@ __global__ __launch_bounds__(256) void moe_ffn_kernel(MoeFfnParams p) {
 //   moe_gate_up   h[id, f] = silu(gate_e[f] . x[row]) * (up_e[f] . x[row])       (element type)
 //   moe_down      o[id, :] = weight(id) * down_e . h[id]                          (fp32)
 // The residual norm that follows sums a row's S slots (scalar_norm nsum).
-
-// Weights: by default a routed expert's weight multiplies its output (moe_down).  weight_in moves it to the expert's
-// input; the gate and up products are linear in it, so it multiplies their fp32 sums (moe_gate_up).  The shared expert's
-// weight, when topk_w has a column for it, always multiplies its output.
-
-DEV float slot_weight(const MoeGroupedParams& p, int row, int k) {
-  return k < p.ldw ? p.topk_w[(int64_t)row * p.ldw + k] : 1.0f;
-}
-DEV float out_weight(const MoeGroupedParams& p, int row, int k) {
-  return p.weight_in && k < p.top ? 1.0f : slot_weight(p, row, k);
-}
-DEV float in_weight(const MoeGroupedParams& p, int id) {
-  if (!p.weight_in) return 1.0f;
-  const int row = id / p.S, k = id - row * p.S;
-  return k < p.top ? slot_weight(p, row, k) : 1.0f;
-}
-
-constexpr int kMoeRows = 64;  // rows of one expert per workgroup tile: four 16-row MFMA tiles share every weight fragment
 
 // The work list from the choices, by one workgroup; sm holds 3 NE + 1 ints.  choice(row, k): expert k of a row.
 template <typename Choice>
@@ -528,7 +511,8 @@ void launch_expert_gemms(const MoeGroupedParams& p, dim3 g1, dim3 g2, hipStream_
   hipLaunchKernelGGL((moe_down_kernel<T, SUBS>), g2, dim3(256), 0, st, p);
 }
 
-// Prompt-sized row counts (bf16, widths multiples of 8): the same two GEMMs with both operands staged through LDS.
+// Prompt-sized row counts (bf16, widths multiples of 8) whose shapes the pipelined form (moe_pipe.hip) does not take: the
+// same two GEMMs with both operands staged through LDS.
 // A workgroup owns a 64-row tile of one expert times 128 weight rows (MODE 0: 64 hidden units' gate rows and the same
 // units' up rows; MODE 1: 128 output columns of the down projection) and walks K in chunks of 64: 256 threads copy the
 // next chunk global -> registers while the MFMAs read the current one from LDS (two buffers, rows padded to 144 bytes so
@@ -694,7 +678,8 @@ extern "C" hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStrea
     hipLaunchKernelGGL(dsse::moe_align_kernel, dim3(1), dim3(256), sizeof(int) * (3 * NE + 1), st, *p);
   const int fmax = p->F > p->Fs ? p->F : p->Fs;
   dim3 g1((fmax + 15) / 16, p->max_tiles), g2((p->W + 15) / 16, p->max_tiles);
-  // prompt-sized steps in bf16 with 16-byte-aligned rows: operands staged through LDS
+  if (dsse::moe_pipe_ok(*p)) return dsse_moe_pipe(p, st);
+  // other prompt-sized steps in bf16 with rows of whole 16-byte pieces: operands staged through registers and LDS
   if (!p->f32 && p->lds_tiles && p->W % 8 == 0 && p->F % 8 == 0 && p->Fs % 8 == 0 && p->ldh % 8 == 0) {
     dim3 l1((fmax + 63) / 64, p->max_tiles), l2((p->W + 127) / 128, p->max_tiles), l3((fmax + 127) / 128, p->max_tiles);
     if (p->gate) hipLaunchKernelGGL(dsse::moe_tile_lds_kernel<0>, l1, dim3(256), 0, st, *p);

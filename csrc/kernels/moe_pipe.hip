@@ -1,0 +1,403 @@
+// Expert GEMMs of prompt-sized steps (bf16): up to 256 rows of one expert x 256 weight rows per workgroup, deep LDS-DMA
+// pipeline.
+//
+// What bounds it: at hundreds of rows per expert both products are compute-sized (muderax-wide, 3000 rows: 705 + 352 GFLOP
+// per layer on 0.7 GB of weights).  The 64-row tiles of moe.hip re-read each weight panel once per 64 rows and wait for
+// their register-staged loads at every chunk; here the schedule of gemm_pipe.hip runs on gathered rows and row-major
+// expert weights:
+//
+//   * 8 waves = 2 wave rows x 4 wave columns of 64; a K step of 64 is four phases, one quadrant of the wave's tile each,
+//     with one half-tile of LDS-DMA issued per phase and retired five phases later by a counted vmcnt, the two wave rows
+//     one barrier apart (one row's MFMA cluster covers the other's LDS reads);
+//   * both operands are row-major, so both LDS images are [row][64 k] with 16-byte pieces swizzled by (row >> 1) & 5 on the
+//     source address (conflict-free fragment reads); rows and columns that do not exist load as zeros without traffic;
+//   * a tile's height follows its expert: the expert's T = ceil(rows / 256) tiles take ceil(k / T) of its k 64-row list
+//     tiles each, and a tile of 64 q rows fills 16 q of every 64-row quadrant: q of the four MFMA row tiles per phase, none
+//     for rows that are not there;
+//   * MODE 0: a column tile pair is (gate rows, up rows) of the same 16 hidden units, so silu(gate) * up needs no exchange;
+//   * order: the shared expert's tiles first (the tallest), then the routed ones; each XCD owns a contiguous eighth of both,
+//     row tiles fastest within groups of 8, so a weight panel's readers share an L2 at about the same time.
+//
+// Every workgroup finds its tile by itself from the work list of 64-row tiles (the experts ascend, so ballots over the list
+// give every expert's place); the host knows only a bound of the tile count.
+//
+// Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
+// experts, top 2, shared 7168: 2369 -> 1014 us (1042 TFLOP/s); 2048 rows: 1695 -> 775; 1024 rows of 2048 x 1408, shared
+// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Never slower from 256 ids on.
+#include <algorithm>
+#include <cmath>
+
+#include "moe_rows.h"
+
+namespace dsse {
+namespace {
+namespace mp {
+
+constexpr int kA = 256 * 128;   // row image of one K step: 256 rows x 64 bf16
+constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 bf16
+constexpr int kBuf = kA + kB;
+constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), then their weights (256 floats)
+constexpr size_t kLDS = kIds + 2 * 256 * 4;
+constexpr uint32_t kOOB = 0x80000000u;  // buffer offset past every range: zeros, no traffic
+
+typedef __attribute__((address_space(3))) void* lds_t;
+
+DEV void dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, 0);
+}
+DEV int swizzle(int row) { return (row >> 1) & 5; }
+
+struct Place {
+  int first;  // the expert's first list tile
+  int tiles;  // its list tiles
+  int at;     // workgroup index inside the expert
+};
+
+// The list's experts in chunks of 64 tiles, a tile per lane: the first four chunks stay in registers
+struct List {
+  const int* tile_expert;
+  int n, lane;
+  int v[4];
+  DEV int chunk(int c) const {
+    const int i = 64 * c + lane;
+    return i < n ? ld_global<int>(tile_expert + i) : 0x7fffffff;
+  }
+  template <typename F>
+  DEV void each(F f) const {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f(c, v[c]);
+    for (int c = 4; 64 * c < n; ++c) f(c, chunk(c));
+  }
+};
+
+}  // namespace mp
+
+// MODE 0: h = silu(gate x) * (up x); 1: o = weight * down h; 2: h = relu(up x)^2
+template <int MODE>
+__global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int tall) {
+  using namespace mp;  // tall: most list tiles in a row tile, 1, 2 or 4
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr int kCols = MODE == 0 ? 128 : 256;  // hidden units or output columns per tile
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int wm = w >> 2, wn = w & 3;
+  auto blocks = [&](int F) { return ((MODE == 1 ? p.W : F) + kCols - 1) / kCols; };
+
+  List list{p.tile_expert, __builtin_amdgcn_readfirstlane(ld_global<int>(p.num_tiles)), lane, {}};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) list.v[c] = list.chunk(c);
+  // list tiles of routed experts, and the row tiles they make: one per started `tall` list tiles of an expert
+  int routed = 0, row_tiles = 0;
+  auto walk = [&](auto f) {  // f(tile, its expert, its index inside the expert, it opens a row tile, row tiles before it)
+    int last = -1, first = 0, before = 0;
+    list.each([&](int c, int v) {
+      const int i = 64 * c + lane;
+      int prev = __shfl_up(v, 1);
+      if (lane == 0) prev = last;
+      const uint64_t starts = __ballot(v != prev && i < list.n), upto = starts & (~0ull >> (63 - lane));
+      const int mine = upto ? 64 * c + 63 - __clzll((long long)upto) : first;
+      const bool opens = v < p.E && ((i - mine) & (tall - 1)) == 0;
+      const uint64_t open = __ballot(opens);
+      f(i, v, i - mine, opens, before + __popcll(open & ((1ull << lane) - 1)));
+      before += __popcll(open);
+      last = __builtin_amdgcn_readlane(v, 63);
+      first = starts ? 64 * c + 63 - __clzll((long long)starts) : first;
+    });
+    return before;
+  };
+  row_tiles = walk([&](int, int v, int, bool, int) { routed += __popcll(__ballot(v < p.E)); });
+  const int shared = list.n - routed;
+  const int nb_r = blocks(p.F), nb_s = blocks(p.Fs);
+  const int total_s = (shared + tall - 1) / tall * nb_s, total_r = row_tiles * nb_r;
+
+  for (int v = blockIdx.x; ; v += gridDim.x) {  // one tile; a second round only if a choice list is not what it should be
+    const int x = v & 7, u = v >> 3;
+    const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0;
+    const int r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
+    if (u >= (total_s + 7) / 8 + (total_r + 7) / 8) return;  // past every XCD's share
+    if (u >= ns + nr) continue;
+    const bool sh = u < ns;
+    Place pl;
+    int e;
+    if (sh) {
+      pl = Place{routed, shared, s0 + u};
+      e = p.E;
+    } else {
+      const int at = r0 + u - ns, want = at / nb_r;
+      int found = 0, opener = 0;
+      walk([&](int i, int ve, int idx, bool opens, int before) {
+        const uint64_t hit = __ballot(opens && before == want);
+        if (hit) {
+          const int l = __builtin_ctzll(hit);
+          found = __builtin_amdgcn_readlane(ve, l);
+          pl.first = __builtin_amdgcn_readlane(i - idx, l);
+          opener = want - __builtin_amdgcn_readlane(idx, l) / tall;  // row tiles before this expert
+        }
+      });
+      e = found;
+      pl.tiles = 0;
+      list.each([&](int, int ve) { pl.tiles += __popcll(__ballot(ve == e)); });
+      pl.at = at - opener * nb_r;
+    }
+    // groups of 8 row tiles swept column by column
+    const int nb = sh ? nb_s : nb_r, T = (pl.tiles + tall - 1) / tall, q = (pl.tiles + T - 1) / T;
+    const int grp = pl.at / (8 * nb), gsz = min(8, T - 8 * grp), in = pl.at - grp * 8 * nb;
+    const int rt = 8 * grp + in % gsz, n0 = in / gsz * kCols;
+    const int t0 = pl.first + rt * q;
+    const int rows64 = min(q, pl.tiles - rt * q);  // list tiles of this row tile: 1..4, or none (T q > tiles + q)
+    if (rows64 <= 0) continue;
+
+    const int Fe = sh ? p.Fs : p.F;
+    const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
+    const int nk = K >> 6;
+    const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
+    const int ldx = MODE == 1 ? p.ldh : p.W;
+    auto weights = [&](const void* routed_w, const void* shared_w) {
+      return reinterpret_cast<const bf16*>(sh ? shared_w : routed_w) + (sh ? 0 : (int64_t)e * p.F * p.W);
+    };
+    // the wave's weight DMA is of one kind: column tiles alternate gate / up, and wave w stages tiles of parity w & 1
+    const bf16* Wp = MODE == 1 ? weights(p.down, p.sdown)
+                               : (MODE == 0 && !(w & 1) ? weights(p.gate, p.sgate) : weights(p.up, p.sup));
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, (uint32_t)((size_t)(MODE == 1 ? p.M * p.S : p.M) * ldx * 2));
+    const __amdgpu_buffer_rsrc_t wr = make_rsrc(Wp, (uint32_t)((size_t)N * K * 2));
+
+    int* s_id = reinterpret_cast<int*>(smem + kIds);
+    float* s_w = reinterpret_cast<float*>(smem + kIds + 256 * 4);
+    __syncthreads();  // a second tile: every wave is past the first one's epilogue
+    if ((int)threadIdx.x < rows64 * 64) {
+      const int id = ld_global<int>(p.sorted + t0 * 64 + threadIdx.x);
+      const int row = id >= 0 ? id / p.S : 0;
+      s_id[threadIdx.x] = id;
+      s_w[threadIdx.x] = id < 0 ? 0.0f : (MODE == 1 ? out_weight(p, row, id - row * p.S) : in_weight(p, id));
+    }
+    __syncthreads();
+
+    const int QI = rows64, QR = 16 * QI;  // MFMA row tiles and rows per quadrant
+    uint32_t a_vo[2][2], b_vo[2][2];
+    int a_lo[2][2], b_lo[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int j = 2 * w + i;                                          // instruction j of this half's 16
+        const int rb = (j >> 3) * 128 + h * 64 + (j & 7) * 8;             // first of its 8 LDS rows
+        const int row = rb + (lane >> 3), sr = (j & 7) * 8 + (lane >> 3);  // LDS row, row inside the quadrant
+        int id = -1;
+        if (sr < QR) id = s_id[((j >> 3) * 2 + h) * QR + sr];
+        a_lo[h][i] = rb * 128;
+        a_vo[h][i] = id >= 0 ? (uint32_t)(((size_t)(MODE == 1 ? id : id / p.S) * ldx + 8 * ((lane & 7) ^ swizzle(row))) * 2)
+                             : kOOB;
+        const int tb = (j >> 2) * 4 + h * 2 + ((j >> 1) & 1);             // column tile
+        const int br = (j & 1) * 8 + (lane >> 3);                         // row inside it
+        const int n = MODE == 0 ? n0 + (tb >> 1) * 16 + br : n0 + tb * 16 + br;
+        b_lo[h][i] = kA + (tb * 16 + (j & 1) * 8) * 128;
+        b_vo[h][i] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ swizzle(br))) * 2) : kOOB;
+      }
+    auto issue_a = [&](int h, int t) {
+      char* base = smem + (t & 1) * kBuf;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dma(xr, base + a_lo[h][i], a_vo[h][i], (uint32_t)t * 128);
+    };
+    auto issue_b = [&](int h, int t) {
+      char* base = smem + (t & 1) * kBuf;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dma(wr, base + b_lo[h][i], b_vo[h][i], (uint32_t)t * 128);
+    };
+    int a_rd[2], b_rd[2];
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) {
+      const int piece = ((2 * g + sp) ^ swizzle(r)) << 4;
+      a_rd[sp] = (wm * 128 + r) * 128 + piece;
+      b_rd[sp] = kA + (wn * 64 + r) * 128 + piece;
+    }
+    f32x4 acc[8][4];
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 a[4][2], b[4][2];
+    auto read_a = [&](const char* buf, int qm) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < QI)  // uniform
+#pragma unroll
+          for (int sp = 0; sp < 2; ++sp)
+            a[i][sp] = *reinterpret_cast<const bf16x8*>(buf + a_rd[sp] + (64 * qm + 16 * i) * 128);
+    };
+    auto read_b = [&](const char* buf, int qn) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int sp = 0; sp < 2; ++sp)
+          b[2 * qn + i][sp] = *reinterpret_cast<const bf16x8*>(buf + b_rd[sp] + (2 * qn + i) * 2048);
+    };
+    auto mma = [&](int qm, int qn) {
+      asm volatile("s_barrier\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i >= QI) continue;  // uniform (one copy of the loop per height keeps no accumulators in registers)
+#pragma unroll
+        for (int sp = 0; sp < 2; ++sp)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[4 * qm + i][2 * qn + j] = mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j]);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      asm volatile("s_barrier" ::: "memory");
+    };
+    // half-tile order, counted waits and their reasons: gemm_pipe.hip
+    issue_a(0, 0);
+    issue_b(0, 0);
+    issue_b(1, 0);
+    issue_a(1, 0);
+    issue_a(0, 1);
+    issue_b(0, 1);
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    if (wm == 1) asm volatile("s_barrier" ::: "memory");
+    auto step = [&](int t, auto tail_tag) {  // TAIL 0: steady; 1: no step t + 2; 2: the last step
+      constexpr int TAIL = decltype(tail_tag)::value;
+      const char* buf = smem + (t & 1) * kBuf;
+      read_a(buf, 0);
+      read_b(buf, 0);
+      if constexpr (TAIL < 2) {
+        issue_b(1, t + 1);
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // B-half 1 of step t
+      } else {
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      }
+      mma(0, 0);
+      read_b(buf, 1);
+      if constexpr (TAIL < 2) {
+        issue_a(1, t + 1);
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // A-half 1 of step t
+      } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      mma(0, 1);
+      read_a(buf, 1);
+      if constexpr (TAIL == 0) issue_a(0, t + 2);
+      mma(1, 1);
+      if constexpr (TAIL == 0) {
+        issue_b(0, t + 2);
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // A0 / B0 of step t + 1
+      } else if constexpr (TAIL == 1) {
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      }
+      mma(1, 0);
+    };
+    int t = 0;
+    for (; t < nk - 2; ++t) step(t, std::integral_constant<int, 0>{});
+    step(t++, std::integral_constant<int, 1>{});  // nk >= 2 (moe_pipe_ok)
+    step(t, std::integral_constant<int, 2>{});
+    if (wm == 0) asm volatile("s_barrier" ::: "memory");  // the two rows' barrier counts meet
+
+#pragma unroll
+    for (int qm = 0; qm < 2; ++qm)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (i >= QI) continue;  // uniform
+          const int at = (wm * 2 + qm) * QR + 16 * i + 4 * g + j;
+          const int id = s_id[at];
+          if (id < 0) continue;
+          const float wt = s_w[at];
+          const f32x4(&c)[4] = acc[4 * qm + i];
+          if (MODE == 0) {
+#pragma unroll
+            for (int qn = 0; qn < 2; ++qn) {
+              const int f = n0 + (wn * 2 + qn) * 16 + r;
+              const float gv = c[2 * qn][j] * wt;
+              if (f < N)
+                reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] =
+                    (bf16)(gv / (1.0f + expf(-gv)) * (c[2 * qn + 1][j] * wt));
+            }
+          } else {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+              const int f = n0 + (wn * 4 + n) * 16 + r;
+              if (f >= N) continue;
+              const float v = c[n][j] * wt;
+              if (MODE == 1) p.o[(int64_t)id * p.W + f] = v;
+              else reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(v > 0.0f ? v * v : 0.0f);
+            }
+          }
+        }
+  }
+}
+
+// Most workgroup tiles that the routed experts (the shared expert) can make: sum of ceil(rows / (64 tall)) over experts
+int64_t col_blocks(const MoeGroupedParams& p, int mode, int F) {
+  const int cols = mode == 0 ? 128 : 256;
+  return ((mode == 1 ? p.W : F) + cols - 1) / cols;
+}
+int64_t routed_tiles(const MoeGroupedParams& p, int mode, int tall) {
+  const int64_t rows = 64 * tall, ids = (int64_t)p.M * p.top;
+  return std::min((ids + (rows - 1) * p.E) / rows, ids) * col_blocks(p, mode, p.F);
+}
+int64_t shared_tiles(const MoeGroupedParams& p, int mode, int tall) {
+  return p.S > p.top ? (p.M + 64 * (int64_t)tall - 1) / (64 * tall) * col_blocks(p, mode, p.Fs) : 0;
+}
+// The row tiles' greatest height: the one whose tiles finish first by a simple model, rounds of 256 workgroups (one per CU)
+// times the tiles' mean time.  A tile of 1 / 2 / 3 / 4 list tiles takes 0.5 / 0.7 / 0.85 / 1 of the tallest one's time
+// (0.75 to 1.7 us per K step, measured at 2048 x 1024, 8 experts); choices spread evenly over the experts but for one
+// standard deviation, which is what decides whether a round is full.
+int moe_pipe_height(const MoeGroupedParams& p, int mode) {
+  static const double kTime[5] = {0.0, 0.5, 0.7, 0.85, 1.0};
+  const double each = (double)p.M * p.top / p.E;
+  const int64_t nb_r = col_blocks(p, mode, p.F), nb_s = p.S > p.top ? col_blocks(p, mode, p.Fs) : 0;
+  const int64_t k_r = std::max<int64_t>(1, (int64_t)((each + std::sqrt(each) + 63.0) / 64.0)), k_s = (p.M + 63) / 64;
+  int best = 4;
+  double least = 0.0;
+  for (int tall = 4; tall >= 1; tall /= 2) {
+    const int64_t t_r = (k_r + tall - 1) / tall, t_s = (k_s + tall - 1) / tall;
+    const int64_t q_r = (k_r + t_r - 1) / t_r, q_s = (k_s + t_s - 1) / t_s;
+    const int64_t n_r = t_r * p.E * nb_r, n_s = t_s * nb_s;
+    const double mean = (n_r * kTime[q_r] + n_s * kTime[q_s]) / (double)(n_r + n_s);
+    const double time = (double)((n_r + n_s + 255) / 256) * mean;
+    if (tall == 4 || time < least) best = tall, least = time;
+  }
+  return best;
+}
+
+template <int MODE>
+hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
+  constexpr int kCols = MODE == 0 ? 128 : 256;
+  static bool attr_set = false;
+  if (!attr_set) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_pipe_kernel<MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)mp::kLDS);
+    attr_set = true;
+  }
+  const int tall = moe_pipe_height(p, MODE);
+  const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8);
+  hipLaunchKernelGGL(moe_pipe_kernel<MODE>, dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
+  return hipGetLastError();
+}
+
+bool pieces(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+bool moe_pipe_ok(const MoeGroupedParams& p) {
+  constexpr int64_t kRange = (int64_t)1 << 31;
+  const int64_t ids = (int64_t)p.M * p.S, widest = p.F > p.Fs ? p.F : p.Fs;
+  const bool shared = p.S > p.top;
+  if (p.f32 || p.W % 64 || p.W < 128 || p.F % 64 || p.F < 128 || (shared && (p.Fs % 64 || p.Fs < 128)) || p.ldh % 8)
+    return false;
+  if ((int64_t)p.M * p.W * 2 >= kRange || ids * p.ldh * 2 >= kRange || widest * p.W * 2 >= kRange) return false;
+  // fewer than 256 ids (no row of every expert's first list tile is sure to be there): the register-direct kernels are as
+  // fast up to 32 rows (two sub-tiles); above, the pipeline wins where the down product alone makes 96 tiles (64 rows:
+  // 146 -> 101 us at 2048 x 1408 of 16 experts + shared 2816, 518 -> 343 us at 4096 x 3584 + 7168; 64 tiles: equal)
+  if (ids < 256 && (p.M <= 32 || p.E * col_blocks(p, 1, p.F) < 96)) return false;
+  if (!pieces(p.x) || !pieces(p.h) || !pieces(p.up) || !pieces(p.down) || (p.gate && !pieces(p.gate))) return false;
+  return !shared || (pieces(p.sgate) && pieces(p.sup) && pieces(p.sdown));
+}
+
+}  // namespace dsse
+
+extern "C" hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st) {
+  const hipError_t e = p->gate ? dsse::launch_moe_pipe<0>(*p, st) : dsse::launch_moe_pipe<2>(*p, st);
+  return e != hipSuccess ? e : dsse::launch_moe_pipe<1>(*p, st);
+}

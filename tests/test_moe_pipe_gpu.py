@@ -1,0 +1,54 @@
+"""The pipelined expert GEMMs (moe_pipe.hip) against the PyTorch reference, at the sizes where their tiling changes."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    ops.load_library(required=True)
+    return torch.device("cuda", 0)
+
+
+# rows of expert 0 sit on both sides of a 64-row list tile and of the 128-, 192- and 256-row tiles; two K steps and odd
+# counts of them; output widths that end inside a column block; no shared expert, one expert, and a work list of more than
+# 256 tiles (the list's chunks beyond those held in registers)
+@pytest.mark.parametrize("M,W,F,Fs,E,top,first,gated", [
+    (128, 128, 128, 128, 2, 2, 64, True), (130, 320, 192, 448, 3, 2, 65, True), (257, 128, 448, 128, 2, 1, 129, True),
+    (400, 192, 128, 0, 4, 2, 193, True), (513, 576, 320, 192, 3, 1, 257, True), (300, 128, 128, 0, 1, 1, 300, True),
+    (300, 128, 128, 128, 300, 1, 0, True), (700, 256, 192, 0, 3, 1, 256, False), (1100, 512, 128, 0, 2, 1, 1025, False)])
+@pytest.mark.parametrize("weight_input", [False, True])
+def test_pipelined_experts(gpu, M, W, F, Fs, E, top, first, gated, weight_input):
+    g = torch.Generator().manual_seed(M + W + F)
+
+    def rnd(*s):
+        return (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16()
+
+    x = torch.randn(M, W, generator=g).bfloat16()
+    gate, up, down = rnd(E, F, W) if gated else None, rnd(E, F, W), rnd(E, W, F)
+    sh = (rnd(Fs, W), rnd(Fs, W), rnd(W, Fs)) if Fs else (None, None, None)
+    S = top + (1 if Fs else 0)
+    # `first` rows choose expert 0 first, the others begin elsewhere; further choices are the next experts
+    start = torch.randint(0, max(1, E - 1), (M,), generator=g) + 1
+    start[torch.randperm(M, generator=g)[:first]] = 0
+    idx = ((start[:, None] + torch.arange(top)) % E).int()
+    w = torch.rand(M, S, generator=g) + 0.25
+    ref = torch.zeros(M * S, W)
+    lref.moe_grouped(x, idx, w, gate, up, down, *sh, ref, weight_input)
+    tiles = -(-M * S // 64) + E + 2
+    c = lambda t: None if t is None else t.to(gpu)  # noqa: E731
+    o = torch.full((M * S, W), float("nan"), device=gpu)
+    ops.moe_grouped(c(x), c(idx), c(w), c(gate), c(up), c(down), *(c(t) for t in sh),
+                    torch.zeros(tiles * 64, dtype=torch.int32, device=gpu), torch.zeros(tiles, dtype=torch.int32, device=gpu),
+                    torch.zeros(1, dtype=torch.int32, device=gpu),
+                    torch.zeros(M * S, max(F, Fs), dtype=torch.bfloat16, device=gpu), o, weight_input)
+    # every hidden value is rounded to bf16 once, by at most 2^-8 of itself; the sums are fp32
+    err = (o.cpu().double() - ref.double()).norm() / ref.double().norm()
+    assert float(err) <= 2.0 ** -8
+    assert float((o.cpu() - ref).abs().max()) <= 2.0 ** -5 * float(ref.abs().max())
