@@ -195,6 +195,7 @@ hipError_t dsse_latent_attention(int num_work, const dsse::LatentAttnParams* p, 
 // (bf16, rk in {64, 128, 256, 512}, dr % 32 == 0; 16 columns = rt rows x hp heads per work item)
 hipError_t dsse_latent_flash(int num_work, const dsse::LatentAttnParams* p, const void* vt, int rt, int hp,
                              hipStream_t st);
+hipError_t dsse_latent_tile(int num_work, const dsse::LatentAttnParams* p, const void* vt, int rt, int hp, hipStream_t st);
 hipError_t dsse_conv_state(const dsse::ConvStateParams* p, hipStream_t st);
 hipError_t dsse_lru_scan(const dsse::LruScanParams* p, hipStream_t st);
 hipError_t dsse_moe_router(const dsse::MoeRouterParams* p, hipStream_t st);

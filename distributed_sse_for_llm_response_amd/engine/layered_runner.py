@@ -137,8 +137,6 @@ SINK_DECODE_GROUPS = 512  # workgroups a decode launch of the sink attention aim
 SINK_TILE_GROUPS = 256    # workgroups from which prompt portions take the shared-page form: below, one-tile items fill more
 SINK_DECODE_PAGES = 32    # fewest pages of a full cache that a workgroup's stretch of a split walk is worth
 SINK_ROWS_TILE = 16   # query rows per work item of the sink attention's MFMA form (one head per wave)
-FLASH_ROWS_TILE = 4   # query rows per work item of the MFMA attention form, x 4 heads = 16 columns: a page of keys is
-                      # read once for four heads (16 rows x 1 head re-read it per head: 2-3x the time at 16 heads)
 
 
 LDS_BYTES = 64 * 1024  # what an attention launch may ask for
@@ -160,7 +158,7 @@ class LayeredRunner(RunnerBase):
         self.use_graphs = (self.device.type == "cuda") if use_graphs is None else use_graphs
         cfg, dev = self.cfg, self.device
         self._init_slots(max_batch, self.max_blocks, cfg.vocab_size, dev, self.comm)
-        self._tile_rows = []   # row counts of the shared-page attention's work items that this design's layers use
+        self._tile_rows = []   # row counts of the shared-page attention forms' work items that this design's layers use
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
         self.multistream = getattr(cfg, "family", "") == "dironex"  # pre-norm blocks on several residual streams
@@ -196,6 +194,7 @@ class LayeredRunner(RunnerBase):
             key = (m.rot, m.rot_dim)
             if key not in self._rope:
                 self._rope[key] = m.rot.table(self.max_model_len + 1, m.rot_dim, dev)
+        self._tile_rows = sorted({ops.latent_tile_rows(att[i].heads, att[i].kv_rank, att[i].rot_dim) for i in flash})
         words = max((ops.latent_flash_part_floats(max_batch, m.heads, 16, 16, m.kv_rank) for i, m in att.items()
                      if i in flash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -306,8 +305,9 @@ class LayeredRunner(RunnerBase):
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope,
                                          lat, m.window, m.scale, 1, vt, 16, self._flash_part if np_ > 1 else None, np_)
                 else:
-                    ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["fs"], g["ft"], rope,
-                                         lat, m.window, m.scale, FLASH_ROWS_TILE, vt, 16 // FLASH_ROWS_TILE)
+                    rows = ops.latent_tile_rows(H, rk, dr)
+                    ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], *g["tiles"][rows], rope,
+                                         lat, m.window, m.scale, rows, vt, 16 // rows)
             else:
                 ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope, lat,
                                      m.window, m.scale, g["qt"])
@@ -603,6 +603,7 @@ class LayeredRunner(RunnerBase):
         self.kv = MixedKVCache({r: m.kv_rank + m.rot_dim for r, m in lat.items()}, kv, self.num_blocks, dev, self.dtype,
                                latent_transposed=lflash, kv_transposed=kflash)
         self.state = ConvTailCache(tails, self.max_batch, dev)
+        self._tile_rows = sorted({ops.latent_tile_rows(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash})
         words = max((ops.latent_flash_part_floats(self.max_batch, m.heads, 16, 16, m.kv_rank) for r, m in lat.items()
                      if r in lflash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -727,8 +728,9 @@ class LayeredRunner(RunnerBase):
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope,
                                          lat, m.window, m.scale, 1, vt, 16, self._flash_part if np_ > 1 else None, np_)
                 else:
-                    ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["fs"], g["ft"], rope,
-                                         lat, m.window, m.scale, FLASH_ROWS_TILE, vt, 16 // FLASH_ROWS_TILE)
+                    rows = ops.latent_tile_rows(H, rk, dr)
+                    ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], *g["tiles"][rows], rope,
+                                         lat, m.window, m.scale, rows, vt, 16 // rows)
             else:
                 ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope, lat,
                                      m.window, m.scale, g["qt"])
@@ -1369,7 +1371,7 @@ class LayeredRunner(RunnerBase):
         list, device dict: ids / pos / slots per row, qs / ql / ctx / ss per sequence, ws / wt work items, bt)."""
         n = len(seqs)
         ids_l, pos_l, slots_l, qs, ql, ctx, ss = [], [], [], [], [], [], []
-        ws, wt, fs, ft, hs, ht = [], [], [], [], [], []
+        ws, wt, hs, ht = [], [], [], []
         prev_l, last = [], []
         bt = torch.zeros(n, self.max_blocks, dtype=torch.int32)
         row = 0
@@ -1397,20 +1399,17 @@ class LayeredRunner(RunnerBase):
             nt = math.ceil(m / ATTN_ROWS_TILE)
             ws += [i] * nt
             wt += list(range(nt))
-            nf = math.ceil(m / FLASH_ROWS_TILE)
-            fs += [i] * nf
-            ft += list(range(nf))
             nh = math.ceil(m / SINK_ROWS_TILE)
             hs += [i] * nh
             ht += list(range(nh))
             row += m
         T = row
-        shared = []  # shared-page attention: the longest walks first
+        shared = []  # work items of the shared-page attention forms: the longest walks first
         for R in self._tile_rows:
             items = [(i, t) for i, s in enumerate(seqs) for t in range(math.ceil(len(s.tokens) / R))]
             items.sort(key=lambda it: -(seqs[it[0]].start_pos + it[1] * R))
             shared += [("tile_seq", R, [i for i, _ in items]), ("tile_no", R, [t for _, t in items])]
-        lists = np.asarray(qs + ql + ctx + ss + ws + wt + fs + ft + hs + ht + last + [x for _, _, xs in shared for x in xs],
+        lists = np.asarray(qs + ql + ctx + ss + ws + wt + hs + ht + last + [x for _, _, xs in shared for x in xs],
                            dtype=np.int64)
         meta = torch.from_numpy(np.concatenate(ids_l + pos_l + slots_l + prev_l + [lists]).astype(np.int32))
         if self.device.type == "cuda":
@@ -1418,8 +1417,8 @@ class LayeredRunner(RunnerBase):
             bt = bt.pin_memory().to(self.device, non_blocking=True)
         d, o = {}, 0
         for name, k in (("ids", T), ("pos", T), ("slots", T), ("prev", T if self.pair else 0), ("qs", n), ("ql", n),
-                        ("ctx", n), ("ss", n), ("ws", len(ws)), ("wt", len(ws)), ("fs", len(fs)), ("ft", len(fs)),
-                        ("hs", len(hs)), ("ht", len(hs)), ("last", len(last))):
+                        ("ctx", n), ("ss", n), ("ws", len(ws)), ("wt", len(ws)), ("hs", len(hs)),
+                        ("ht", len(hs)), ("last", len(last))):
             d[name], o = meta[o:o + k], o + k
         for name, R, xs in shared:
             d.setdefault(name, {})[R], o = meta[o:o + len(xs)], o + len(xs)

@@ -56,6 +56,17 @@ def latent_kv_write(ckr, norm_w, positions, slots, rope, cache, eps: float, vt=N
         lref.latent_kv_write(ckr, norm_w, positions, slots, rope, cache, eps, vt)
 
 
+def latent_tile_rows(heads: int, rk: int, dr: int) -> int:
+    """Query rows per work item of latent_attention's MFMA form in prompt portions, with 16 // rows heads in an item's 16
+    columns: the fewest rows whose items fill at least half of the eight column tiles that share a page (latent_tile.hip), or
+    four where that form does not apply."""
+    if dr == 64 and rk in (128, 256, 512):
+        for rows in (4, 8, 16):
+            if -(-heads // (16 // rows)) >= (6 if rows < 16 else 4):
+                return rows
+    return 4
+
+
 def latent_flash_ok(dtype, rk: int, dr: int) -> bool:
     """Shapes the MFMA form of latent_attention covers (everything else takes the row kernel)."""
     return dtype == torch.bfloat16 and rk in (64, 128, 256, 512) and dr % 32 == 0
