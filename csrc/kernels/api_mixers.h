@@ -114,6 +114,12 @@ struct MatrixScanParams {
   float* a_out;          // [nseq, H, D] product of the chunk's per-channel decays (decay_kind 3) or null
 };
 
+// Workspace floats of the chunked form (matrix_chunk.hip) for `rows` rows, of them `longest` in the longest sequence (0 = not
+// known); 0 where the walk by tokens is taken: by its time, and for shapes that the chunks do not take.  They take key widths
+// 32, 64 and 128, whole 16-column tiles of values, decays that do not differ between key channels, 16-byte-aligned rows.
+// Sequences share no rows.
+int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest);
+
 // The carry between the two passes of the two-level walk: per sequence, the incoming state of each of its chunks.
 struct ScanCarryParams {
   float* scratch;        // [chunks, H, D, V]: in: a chunk's end state from zeros; out: the chunk's incoming state
@@ -239,6 +245,7 @@ hipError_t dsse_sink_decode(int num_work, const dsse::SinkAttnParams* p, const v
 // p1 / p2 hold N / rep1 and N / rep2 numbers: entry j serves columns [j rep, (j + 1) rep)
 hipError_t dsse_gate_math(float* x, int ld, int M, int N, int kind, const float* p1, int rep1, const float* p2, int rep2,
                           float c, hipStream_t st);
+hipError_t dsse_scan_chunks(const dsse::MatrixScanParams* p, float* ws, int rows, int64_t longest, hipStream_t st);
 hipError_t dsse_matrix_scan(const dsse::MatrixScanParams* p, hipStream_t st);
 hipError_t dsse_scan_carry(const dsse::ScanCarryParams* p, hipStream_t st);
 // gate_kind 0: silu(gate), 1: sigmoid(gate)

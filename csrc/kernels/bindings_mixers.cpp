@@ -301,7 +301,7 @@ void gate_math(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2
 
 void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
                  Tensor& state, const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
-                 const Tensor& state_slot, Tensor& out, double q_scale) {
+                 const Tensor& state_slot, Tensor& out, double q_scale, int64_t longest) {
   head_view(q, "q");
   head_view(k, "k");
   head_view(v, "v");
@@ -354,6 +354,12 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   p.out = out.data_ptr<float>();
   p.q_scale = (float)q_scale;
   p.portions = T > 2 * p.nseq;  // more than a row or two per sequence: prompt portions, not a decode step
+  TORCH_CHECK(longest >= 0 && longest <= T, "longest must be 0 (not known) .. T rows");
+  if (const int64_t floats = dsse::scan_chunk_floats(p, T, longest)) {
+    Tensor ws = at::empty({floats}, v.options());
+    DSSE_CHECK_HIP(dsse_scan_chunks(&p, ws.data_ptr<float>(), T, longest, cur_stream()));
+    return;
+  }
   DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
 }
 
@@ -807,7 +813,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor? rel=None, int keep_first=0, float out_scale=1.0, Tensor(b!)? part=None, int nparts=1) -> ()");
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
-        "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0) -> ()");
+        "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
   m.def("matrix_scan_chunked(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor(a!) state, Tensor q_len, Tensor ctx_len, "
         "Tensor state_slot, Tensor s_first, Tensor s_count, Tensor cmeta, Tensor(b!) scratch, Tensor(c!)? a_scratch, "
         "Tensor(d!) out, float q_scale=1.0) -> ()");

@@ -38,7 +38,8 @@ same weights and its own pages and state slots per pass:
     feed-forward            fused [gate | up] GEMM -> gated_act (gelu) -> down GEMM
     head                    stream_step (last add + final norm) -> head GEMM -> logit_cap (scale, tanh cap)
 
-Long prompt groups walk the recurrences without the delta rule in two levels (matrix_scan_chunked).
+Long prompt groups take the recurrences by chunks of 64 tokens: on the matrix cores in matrix_scan, as a two-level walk
+(matrix_scan_chunked) where the decay differs between key channels.
 
 The multi-stream walk (`_stream_layers`) also goes over layer runs; a row carries S residual copies:
 
@@ -492,17 +493,16 @@ class LayeredRunner(RunnerBase):
         """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection."""
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
-            if beta is None and "ck" in g:
+            D, chan = k.shape[2], decay is not None and decay.dim() == 3
+            if beta is None and "ck" in g and not ops.scan_chunks_form(D, V, chan):
                 s_first, s_count, cm = g["ck"]
-                D = k.shape[2]
                 scr = self._scratch(d, "scan_s", cm.shape[1] * H * D * V)
-                chan = decay is not None and decay.dim() == 3
                 ascr = self._scratch(d, "scan_a", cm.shape[1] * H * D) if chan else None
                 ops.matrix_scan_chunked(q, k, v, decay, self.state.state[ri], g["qs"], g["ql"], g["ctx"], g["ss"],
                                         s_first, s_count, cm, scr, ascr, o, q_scale)
             else:
                 ops.matrix_scan(q, k, v, decay, beta, self.state.state[ri], g["qs"], g["ql"], g["ctx"], g["ss"], o,
-                                q_scale)
+                                q_scale, g.get("longest", 0))
         ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw_norm, gate, self.cfg.eps, ao)
         self._lin(ao, o_w, o_t, y)
@@ -1426,6 +1426,7 @@ class LayeredRunner(RunnerBase):
         d["bt"] = bt
         d["qt"] = ATTN_ROWS_TILE
         d["rows"] = (row0, T)   # the packed rows of these portions
+        d["longest"] = max(ql)
         if self.prenorm and T >= ops.layers.SCAN_CHUNKED_FROM:  # long portions: the recurrences' two-level walk
             s_first, s_count, rows = ops.layers.scan_chunks(qs, ql, ss)
             ck = torch.tensor([s_first, s_count], dtype=torch.int32)

@@ -272,12 +272,15 @@ def gate_math(x, kind: int, p1=None, p2=None, c: float = 1.0):
         lref.gate_math(x, kind, p1, p2, c)
 
 
-def matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale: float = 1.0):
+def matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale: float = 1.0,
+                longest: int = 0):
     """Matrix-state recurrence per (sequence, head) continued from the slot state [slots, H, D, V] (fp32; zeros at
     position 0): S = a S; u = beta (v - S^T k) with beta (the delta rule), else u = v; S += k u^T; o = S^T (q_scale q).
-    decay: None, [H], [T, H] or [T, H, D]; q, k [T, G, D], v [T, H, V] are fp32 (column slices are fine)."""
+    decay: None, [H], [T, H] or [T, H, D]; q, k [T, G, D], v [T, H, V] are fp32 (column slices are fine).  `longest`:
+    rows of the longest sequence where the caller knows them; long sequences then go by chunks of tokens."""
     if _hip(v):
-        torch.ops.dsse.matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale)
+        torch.ops.dsse.matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale,
+                                   longest)
     else:
         lref.matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale)
 
@@ -301,6 +304,12 @@ def scan_state_from_plain(plain):
 
 SCAN_CHUNK = 64        # tokens per chunk of the two-level walk
 SCAN_CHUNKED_FROM = 256  # rows of a prompt group from which matrix_scan_chunked pays
+
+
+def scan_chunks_form(dim: int, vdim: int, per_channel: bool) -> bool:
+    """Whether matrix_scan takes long sequences of this state by chunks: it does for decays that do not differ between
+    key channels (matrix_scan_chunked walks the others in two levels)."""
+    return not per_channel and dim in (32, 64, 128) and vdim % 16 == 0
 
 
 def scan_chunks(q_start: list, q_len: list, slots: list):

@@ -1,0 +1,57 @@
+"""Long sequences of the matrix-state recurrence by chunks of 64 tokens on the matrix cores (csrc/kernels/matrix_chunk.hip),
+against the op's reference walk."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+from distributed_sse_for_llm_response_amd.ops.layers import scan_state_from_plain, scan_state_plain
+
+pytestmark = pytest.mark.gpu
+
+
+def i32(x):
+    return torch.tensor(x, dtype=torch.int32)
+
+
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 32, 16), (3, 3, 64, 48), (2, 1, 128, 32)])
+@pytest.mark.parametrize("mode", ["delta", "delta_fixed", "tokens", "fixed", "plain"])
+@pytest.mark.parametrize("ql,cont", [([1, 64, 65, 130, 0, 3], True), ([96], False), ([193, 2], True)])
+def test_chunks_match_the_walk(H, G, D, V, mode, ql, cont):
+    """Lengths around the chunk's 64 tokens, an empty and a one-row sequence, continued and fresh slots in reversed order,
+    rows outside every sequence, column slices of wider rows, decays of exactly zero.  Error: sums of D products and of 64
+    tokens in fp32, (D + 64) 2^-24 < 1.2e-5 of the largest result, on either side."""
+    g = torch.Generator().manual_seed(3 + D + len(ql))
+    n, pad = len(ql), 2
+    T = sum(ql) + 2 * pad
+    qs = [pad + sum(ql[:i]) for i in range(n)]
+    ctx = [m + (7 if cont and i % 2 == 0 else 0) for i, m in enumerate(ql)]
+    slot = list(range(n, 0, -1))
+    wide = torch.randn(T, 2 * G * D + H * V + 3 + 5, generator=g)   # rows of q | k | 3 odd columns | v, to a multiple of 4
+    wide = torch.nn.functional.pad(wide, (0, -wide.shape[1] % 4))
+    wide[:, G * D:2 * G * D] = torch.nn.functional.normalize(wide[:, G * D:2 * G * D].unflatten(1, (G, D)), dim=-1).flatten(1)
+    if "delta" not in mode:
+        wide[:, :G * D] *= D ** -0.5
+
+    def views(t):
+        return (t[:, :G * D].unflatten(1, (G, D)), t[:, G * D:2 * G * D].unflatten(1, (G, D)),
+                t[:, 2 * G * D + 3:2 * G * D + 3 + H * V].unflatten(1, (H, V)))
+
+    decay = None
+    if mode in ("delta", "tokens"):
+        decay = torch.rand(T, H, generator=g) ** 0.2
+        decay[pad + 5::17] = 0.0
+    elif mode != "plain":
+        decay = torch.linspace(0.5, 0.999, H)
+    beta = torch.rand(T, H, generator=g) if "delta" in mode else None
+    state0 = torch.randn(n + 1, H, D, V, generator=g)
+    st_ref, o_ref = state0.clone(), torch.zeros(T, H, V)
+    lref.matrix_scan(*views(wide), decay, beta, st_ref, i32(qs), i32(ql), i32(ctx), i32(slot), o_ref, 0.5)
+    c = lambda t: None if t is None else t.cuda()  # noqa: E731
+    st, o = scan_state_from_plain(c(state0)), torch.zeros(T, H, V, device="cuda")
+    ops.matrix_scan(*views(c(wide)), c(decay), c(beta), st, c(i32(qs)), c(i32(ql)), c(i32(ctx)), c(i32(slot)), o, 0.5, max(ql))
+    tol = 2 * (D + 64) * 2.0 ** -24
+    assert (o.cpu() - o_ref).abs().max() <= tol * o_ref.abs().max()
+    got = scan_state_plain(st).cpu()
+    assert (got - st_ref).abs().max() <= tol * st_ref.abs().max()
+    assert torch.equal(got[0], state0[0]) and not o[:pad].any() and not o[T - pad:].any()   # other slots and rows
