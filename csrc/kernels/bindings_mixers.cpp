@@ -271,8 +271,8 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
     TORCH_CHECK(p.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 8 == 0, "the MFMA form stores 8-byte pieces of out");
     if (qt > 16) {  // pages shared by 128 / qt heads of a group
       TORCH_CHECK((qt == 32 || qt == 64 || qt == 128) && (p.H / p.G) % (128 / qt) == 0 && p.D % 32 == 0 && p.V % 16 == 0 &&
-                      p.D <= 128 && p.V <= 128 && !p.rel && !p.out_rope && !split && work_seq.numel() <= 65535,
-                  "the shared-page form: qt 32 / 64 / 128 for groups of 4 / 2 / 1 heads, widths up to 128, no bias, no rotation");
+                      p.D <= 128 && p.V <= 128 && !p.out_rope && !split && work_seq.numel() <= 65535,
+                  "the shared-page form: qt 32 / 64 / 128 for groups of 4 / 2 / 1 heads, widths up to 128, no rotation");
       DSSE_CHECK_HIP(dsse_sink_tile((int)work_seq.numel(), &p, vt->data_ptr(), (int)qt / 16, cur_stream()));
       return;
     }

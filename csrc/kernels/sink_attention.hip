@@ -488,19 +488,38 @@ __global__ __launch_bounds__(256) void sink_flash_kernel(SinkAttnParams p, const
 
 // ---------------------------------------------------------------------------------------------------------------------
 // Shared-page form for prompt portions (bf16, head widths up to 128): a workgroup takes hb heads of ONE key/value group times
-// rt tiles of 16 query rows, hb rt = 8 column tiles, two per wave.  Each page's keys and transposed values are staged in LDS
-// once for all eight tiles, and a fragment read from LDS feeds both tiles of a wave; the next two pages are on their way
-// (in registers) while the current one is in the MFMAs, one barrier per page.  The query operands stay in registers.  Masks and
-// the rescaling of the sums are branches here: pages that every row sees whole and maxima that stay skip them.  The head
-// group is the fast grid dimension, so workgroups of one XCD keep to the same keys when the groups are a multiple of eight.
+// rt tiles of 16 query rows, hb rt = 8 column tiles, CT per wave.  Each page's keys and transposed values are staged in LDS
+// once for all eight tiles, and a fragment read from LDS feeds all tiles of a wave; the next two pages are on their way
+// (in registers) while the current one is in the MFMAs, one barrier per page.  The query operands stay in registers.  Masks,
+// the cap and the rescaling of the sums are branches here: pages that every row sees whole and maxima that stay skip them.
+// The head group is the fast grid dimension, so workgroups of one XCD keep to the same keys when the groups are a multiple
+// of eight.
+//
+// What bounds it: a page's chain of products, maximum, exponentials and products, about 1700 cycles a CU of which 512 are
+// MFMA.  2048 rows of 32 heads over 8 key/value heads: 277 us (a wave per 16 rows and head), 99 with a branch per k-step and
+// score, 85 without them, 70 with maxima that lag.  16 heads over 8, window 1024 and bias: 500 + 500 + 500 rows 51 -> 23 us.
 constexpr int kTileWidth = 128;   // widest query and value heads
 constexpr int kTileLdv = kBS + 8;
 
-template <int NT>
-__global__ __launch_bounds__(256, 2) void sink_tile_kernel(SinkAttnParams p, const bf16* __restrict__ vt, int hb, int rt) {
+// The sums are scaled by a maximum that may lag behind the scores by this much (log2 units): weights stay below 2^8, which
+// fp32 sums and bf16 weights hold as exactly as weights below one, and pages that raise no row's maximum by more need no
+// rescaling and no exchange between lanes.
+constexpr float kLazyMax = 8.0f;
+
+DEV bf16x8 ld_buffer(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+// BIAS: the distance bias, the first rel_lds entries of the group's heads in LDS behind the pages.
+// KD: the key width over 32 where it equals the value width (every load, product and LDS store of a page is then free of
+// branches), 0: read from the parameters.
+template <int NT, int KD, bool BIAS, int CT>
+__global__ __launch_bounds__(512 / CT, 2) void sink_tile_kernel(SinkAttnParams p, const bf16* __restrict__ vt, int hb, int rt,
+                                                           int rel_lds) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int V = 16 * NT, KS = kTileWidth / 32, KC = kTileWidth * kBS / 8 / 256, VC = (V * kBS / 8 + 255) / 256;
-  const int D = p.D, nks = D / 32, ldk = D + 8;
+  constexpr int V = 16 * NT, KS = KD ? KD : kTileWidth / 32, TH = 512 / CT,
+                KC = (32 * KS * kBS / 8 + TH - 1) / TH, VC = (V * kBS / 8 + TH - 1) / TH;
+  const int D = KD ? 32 * KD : p.D, nks = D / 32, ldk = D + 8;
   const int buf_elems = kBS * ldk + V * kTileLdv;
   bf16* smem = reinterpret_cast<bf16*>(smem_raw);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
@@ -526,14 +545,14 @@ __global__ __launch_bounds__(256, 2) void sink_tile_kernel(SinkAttnParams p, con
     const int b = it0 + lane < walk ? bt[page_at(it0 + lane)] : 0;
     return (unsigned)b < (unsigned)p.num_blocks ? b : 0;
   };
-  // this wave's two column tiles
-  int head[2], pos[2], tile_lo[2], tile_hi[2];
-  bool on[2];
-  int64_t row[2];
-  bf16x8 qf[2][KS];
+  // this wave's column tiles
+  int head[CT], pos[CT], tile_lo[CT], tile_hi[CT];
+  bool on[CT];
+  int64_t row[CT];
+  bf16x8 qf[CT][KS];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int ct = 2 * wave + c, off = row_first + 16 * (ct % rt) + r;
+  for (int c = 0; c < CT; ++c) {
+    const int ct = CT * wave + c, off = row_first + 16 * (ct % rt) + r;
     head[c] = h_first + ct / rt;
     on[c] = off < ql;
     row[c] = q0 + (on[c] ? off : 0);
@@ -551,106 +570,167 @@ __global__ __launch_bounds__(256, 2) void sink_tile_kernel(SinkAttnParams p, con
       }
     }
   }
+  // the heads' bias entries behind the two page buffers
+  float* rels = reinterpret_cast<float*>(smem + 2 * buf_elems);
+  float rel_far[CT];
+  if constexpr (BIAS) {
+    for (int hd = 0; hd < hb; ++hd)
+      for (int i = tid; i < rel_lds; i += TH) rels[hd * rel_lds + i] = p.rel[(int64_t)(h_first + hd) * p.rel_len + i];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) rel_far[c] = p.rel[(int64_t)head[c] * p.rel_len + p.rel_len - 1] * kLog2e;
+  }
   int blks = ids_from(0);
   // staging: 16-byte pieces of the page's keys (rows G D apart) and of its transposed values (contiguous)
   const bf16* kc = reinterpret_cast<const bf16*>(p.k);
   const int k16 = D / 8;
   bf16x8 nk[2][KC], nv[2][VC];  // two pages on their way
-  int koff[KC], kdst[KC], vdst[VC];
+  uint32_t koff[KC];  // bytes into the page
+  int kdst[KC], vdst[VC];
 #pragma unroll
   for (int i = 0; i < KC; ++i) {
-    const int idx = tid + 256 * i, kr = idx / k16, c = idx - kr * k16;
+    const int idx = tid + TH * i, kr = idx / k16, c = idx - kr * k16;
     const bool in = kr < kBS;
-    koff[i] = in ? kr * p.G * D + 8 * c : 0;
+    koff[i] = in ? (uint32_t)(kr * p.G * D + 8 * c) * 2 : 0;
     kdst[i] = in ? kr * ldk + 8 * c : -1;
   }
 #pragma unroll
   for (int i = 0; i < VC; ++i) {
-    const int idx = tid + 256 * i;
+    const int idx = tid + TH * i;
     vdst[i] = idx < V * kBS / 8 ? kBS * ldk + (idx / (kBS / 8)) * kTileLdv + 8 * (idx % (kBS / 8)) : -1;
   }
   auto request = [&](int it, bf16x8(&rk)[KC], bf16x8(&rv)[VC]) {  // pages past the walk read its last one again
     if (it < walk && (it & 63) == 0 && it > 0) blks = ids_from(it);
     const int blk = __builtin_amdgcn_readlane(blks, it < walk ? it & 63 : (walk - 1) & 63);
-    const bf16* kp = kc + ((int64_t)blk * kBS * p.G + kvh) * D;
-    const bf16* vp = vt + ((int64_t)blk * p.G + kvh) * V * kBS;
+    // buffer loads: the page's base is uniform and the lanes' offsets never change.  (Global loads took an address
+    // register pair that overlapped the destination, and with it a wait for the page before.)
+    const __amdgpu_buffer_rsrc_t kr = make_rsrc(kc + ((int64_t)blk * kBS * p.G + kvh) * D, (uint32_t)(((kBS - 1) * p.G + 1) * D * 2));
+    const __amdgpu_buffer_rsrc_t vr = make_rsrc(vt + ((int64_t)blk * p.G + kvh) * V * kBS, (uint32_t)(V * kBS * 2));
 #pragma unroll
-    for (int i = 0; i < KC; ++i) rk[i] = ld_global<bf16x8>(kp + koff[i]);
+    for (int i = 0; i < KC; ++i) rk[i] = ld_buffer(kr, koff[i]);
 #pragma unroll
-    for (int i = 0; i < VC; ++i) rv[i] = ld_global<bf16x8>(vp + (vdst[i] >= 0 ? 8 * (tid + 256 * i) : 0));
+    for (int i = 0; i < VC; ++i) rv[i] = ld_buffer(vr, vdst[i] >= 0 ? 16u * (tid + TH * i) : 0u);
   };
   auto stash = [&](int buf, const bf16x8(&rk)[KC], const bf16x8(&rv)[VC]) {
     bf16* b = smem + buf * buf_elems;
 #pragma unroll
     for (int i = 0; i < KC; ++i)
-      if (kdst[i] >= 0) *reinterpret_cast<bf16x8*>(b + kdst[i]) = rk[i];
+      if ((KD && 32 * KS * kBS / 8 % TH == 0) || kdst[i] >= 0) *reinterpret_cast<bf16x8*>(b + kdst[i]) = rk[i];
 #pragma unroll
     for (int i = 0; i < VC; ++i)
-      if (vdst[i] >= 0) *reinterpret_cast<bf16x8*>(b + vdst[i]) = rv[i];
+      if (V * kBS / 8 % TH == 0 || vdst[i] >= 0) *reinterpret_cast<bf16x8*>(b + vdst[i]) = rv[i];
   };
-  f32x4 O[2][NT];
+  f32x4 O[CT][NT];
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
     for (int n = 0; n < NT; ++n) O[c][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+  // m: the maximum that the sums are scaled by (at: the same, 0 before the first key); l: this lane's part of the sum
+  float m[CT], at[CT], l[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) m[c] = -INFINITY, at[c] = 0.f, l[c] = 0.f;
   const float cap_inv = p.softcap > 0.f ? 1.0f / p.softcap : 0.f, cap2 = p.softcap * kLog2e;
   const float scale2 = p.softcap > 0.f ? p.scale : p.scale * kLog2e;
-  const int wave_lo = tile_lo[0] < tile_lo[1] ? tile_lo[0] : tile_lo[1], wave_hi = tile_hi[0] > tile_hi[1] ? tile_hi[0] : tile_hi[1];
+  const int wave_lo = min(tile_lo[0], tile_lo[CT - 1]), wave_hi = max(tile_hi[0], tile_hi[CT - 1]);
   auto page_step = [&](int it, bf16x8(&rk)[KC], bf16x8(&rv)[VC], const bf16x8(&tk)[KC], const bf16x8(&tv)[VC]) {
     const int pg = page_at(it);
     request(it + 2, rk, rv);
     if (pg * kBS <= wave_hi) {  // uniform for the wave: some row of it may see this page
       const bf16* kb = smem + (it & 1) * buf_elems;
       const bf16* vb = kb + kBS * ldk;
-      f32x4 s0[2], s1[2];
+      f32x4 s0[CT], s1[CT];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) s0[c] = s1[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < CT; ++c) s0[c] = s1[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < KS; ++u)
-        if (u < nks) {
+        if (KD || u < nks) {
           const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kb + r * ldk + 32 * u + 8 * g);
           const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kb + (16 + r) * ldk + 32 * u + 8 * g);
 #pragma unroll
-          for (int c = 0; c < 2; ++c) {
+          for (int c = 0; c < CT; ++c) {
             s0[c] = mfma16x16x32(k0, qf[c][u], s0[c]);
             s1[c] = mfma16x16x32(k1, qf[c][u], s1[c]);
           }
         }
+      // x: scores in log2 units; mx: a lane's largest
+      float x[CT][8], mx[CT];
       // uniform: every key of the page is at or before the wave's first row and inside the window of its last one
       const bool full = pg * kBS + kBS - 1 <= wave_lo && wave_hi - pg * kBS < p.window;
-      bf16x8 pf[2];
-      float corr[2];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float sv[8];
+      for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float sc = (i < 4 ? s0[c][i] : s1[c][i - 4]) * scale2;
-          if (p.softcap > 0.f) sc = cap2 * tanh_fast(sc * cap_inv);
-          sv[i] = sc;
+        for (int i = 0; i < 8; ++i) x[c][i] = (i < 4 ? s0[c][i] : s1[c][i - 4]) * scale2;
+      if (p.softcap > 0.f) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[c][i] = cap2 * tanh_fast(x[c][i] * cap_inv);
+      }
+      if constexpr (BIAS) {
+        // uniform: every (row, key) pair of the wave's tiles and the page is at least rel_len - 1 apart
+        if (wave_lo - (pg * kBS + kBS - 1) >= p.rel_len - 1) {
+#pragma unroll
+          for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[c][i] += rel_far[c];
+        } else {
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            float bv[8];
+            bias_entries(bv, false, 0.f, rels + (head[c] - h_first) * rel_lds, p.rel + (int64_t)head[c] * p.rel_len, rel_lds,
+                         p.rel_len, pos[c] - pg * kBS - 4 * g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[c][i] += bv[i] * kLog2e;
+          }
         }
-        if (!full) {
+      }
+      if (!full) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const int key = pg * kBS + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4));
-            const bool seen = key <= pos[c] && (pos[c] - key < p.window || key < p.keep_first);
-            sv[i] = seen ? sv[i] : -INFINITY;
+            const bool seen = (key <= pos[c]) & ((pos[c] - key < p.window) | (key < p.keep_first));
+            x[c][i] = seen ? x[c][i] : -INFINITY;
           }
-        }
-        corr[c] = softmax_step(sv, m[c], l[c], pf[c]);
       }
-      if (!__all(corr[0] == 1.0f && corr[1] == 1.0f)) {
+      bool grown = false;
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
+      for (int c = 0; c < CT; ++c) {
+        mx[c] = x[c][0];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) O[0][n][i] *= corr[0], O[1][n][i] *= corr[1];
+        for (int i = 1; i < 8; ++i) mx[c] = fmaxf(mx[c], x[c][i]);
+        grown |= mx[c] > m[c] + kLazyMax;
+      }
+      if (__any(grown)) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          const float mn = fmaxf(m[c], rows4_max(mx[c]));
+          at[c] = mn == -INFINITY ? 0.0f : mn;  // nothing seen yet: exp2(-inf - 0) is 0
+          const float corr = exp2_hw(m[c] - at[c]);
+          m[c] = mn;
+          l[c] *= corr;
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) O[c][n][i] *= corr;
+        }
+      }
+      bf16x8 pf[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          e[i] = exp2_hw(x[c][i] - at[c]);
+          pf[c][i] = (bf16)e[i];
+        }
+        l[c] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
       }
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const bf16x8 v = *reinterpret_cast<const bf16x8*>(vb + (16 * n + r) * kTileLdv + 8 * g);
 #pragma unroll
-        for (int c = 0; c < 2; ++c) O[c][n] = mfma16x16x32(v, pf[c], O[c][n]);
+        for (int c = 0; c < CT; ++c) O[c][n] = mfma16x16x32(v, pf[c], O[c][n]);
       }
     }
     stash((it + 1) & 1, tk, tv);  // page it + 1; that buffer was last read before the previous barrier
@@ -665,7 +745,8 @@ __global__ __launch_bounds__(256, 2) void sink_tile_kernel(SinkAttnParams p, con
     if (it + 1 < walk) page_step(it + 1, nk[1], nv[1], nk[0], nv[0]);  // uniform for the workgroup
   }
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < CT; ++c) {
+    l[c] = rows4_sum(l[c]);
     if (!on[c]) continue;
     const int h = head[c];
     float den = l[c], f = 1.0f;
@@ -1001,6 +1082,29 @@ void launch_flash(int num_work, const SinkAttnParams& p, const bf16* vt, int spl
   else launch_flash_ext<NT, false>(num_work, p, vt, split, st);
 }
 
+// Two column tiles per wave read half as much of LDS, one per wave has twice the waves to hide a page's chain behind: one where
+// the grid leaves CUs empty.  One against two, 16 heads of 128 over 8 key/value heads, window 1024 with a bias: 100 rows 10.4 /
+// 12.1 us, 1024 rows (128 workgroups) 36.5 / 38.8; causal over 4 key/value heads: 1024 rows (128) 33.9 / 33.4, 4096 rows (512)
+// 139 / 126.
+constexpr int64_t kTileFill = 256;
+
+template <int NT>
+void launch_tile(dim3 grid, size_t lds, const SinkAttnParams& p, const bf16* vt, int hb, int rt, int rel_lds, hipStream_t st) {
+  auto go = [&](auto kd, auto ct) {
+    constexpr int KD = decltype(kd)::value, CT = decltype(ct)::value;
+    if (p.rel) hipLaunchKernelGGL((sink_tile_kernel<NT, KD, true, CT>), grid, dim3(512 / CT), lds, st, p, vt, hb, rt, rel_lds);
+    else hipLaunchKernelGGL((sink_tile_kernel<NT, KD, false, CT>), grid, dim3(512 / CT), lds, st, p, vt, hb, rt, 0);
+  };
+  const bool fills = (int64_t)grid.x * grid.y >= kTileFill;
+  if constexpr (NT % 2 == 0) {
+    if (p.D == p.V) {
+      using Kd = std::integral_constant<int, NT / 2>;
+      return fills ? go(Kd{}, std::integral_constant<int, 2>{}) : go(Kd{}, std::integral_constant<int, 1>{});
+    }
+  }
+  go(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
+}
+
 }  // namespace
 }  // namespace dsse
 
@@ -1023,20 +1127,25 @@ extern "C" hipError_t dsse_sink_flash(int num_work, const dsse::SinkAttnParams* 
   return hipGetLastError();
 }
 
-// shared-page form: work_tile counts tiles of 16 rt rows, hb rt = 8; D and V up to 128, no bias and no output rotation
+// shared-page form: work_tile counts tiles of 16 rt rows, hb rt = 8; D and V up to 128, no output rotation
 extern "C" hipError_t dsse_sink_tile(int num_work, const dsse::SinkAttnParams* p, const void* vt, int rt, hipStream_t st) {
   if (num_work <= 0 || p->H <= 0) return hipSuccess;
   if ((rt != 2 && rt != 4 && rt != 8) || p->H % p->G || (p->H / p->G) % (8 / rt)) return hipErrorInvalidValue;
-  if (p->f32 || p->D % 32 || p->V % 16 || p->D > dsse::kTileWidth || p->V > dsse::kTileWidth || p->rel || p->out_rope ||
+  if (p->f32 || p->D % 32 || p->V % 16 || p->D > dsse::kTileWidth || p->V > dsse::kTileWidth || p->out_rope ||
       num_work > 65535)
     return hipErrorInvalidValue;
   const int hb = 8 / rt;
   const dim3 grid(p->H / hb, num_work);
-  const size_t lds = 2 * sizeof(bf16) * (dsse::kBS * (size_t)(p->D + 8) + (size_t)p->V * dsse::kTileLdv);
+  size_t lds = 2 * sizeof(bf16) * (dsse::kBS * (size_t)(p->D + 8) + (size_t)p->V * dsse::kTileLdv);
+  int rel_lds = 0;
+  if (p->rel) {  // bias entries per head: all of them, at most 1024 (38 KB of pages + 16 KB)
+    rel_lds = p->rel_len < 1024 ? p->rel_len : 1024;
+    lds += (size_t)hb * rel_lds * sizeof(float);
+  }
   const bf16* v = reinterpret_cast<const bf16*>(vt);
   switch (p->V / 16) {
 #define DSSE_TILE_CASE(n) \
-  case n: hipLaunchKernelGGL(dsse::sink_tile_kernel<n>, grid, dim3(256), lds, st, *p, v, hb, rt); break;
+  case n: dsse::launch_tile<n>(grid, lds, *p, v, hb, rt, rel_lds, st); break;
     DSSE_TILE_CASE(1) DSSE_TILE_CASE(2) DSSE_TILE_CASE(3) DSSE_TILE_CASE(4) DSSE_TILE_CASE(5) DSSE_TILE_CASE(6)
     DSSE_TILE_CASE(7) DSSE_TILE_CASE(8)
 #undef DSSE_TILE_CASE

@@ -135,7 +135,6 @@ from .weights import LayeredWeights
 ATTN_ROWS_TILE = 4    # query rows per work item of the row-wise attention kernel (prompt portions)
 FLASH_DECODE_WAVES = 512  # waves a decode attention launch aims for (two per CU)
 SINK_DECODE_GROUPS = 512  # workgroups a decode launch of the sink attention aims for (two per CU)
-SINK_TILE_GROUPS = 256    # workgroups from which prompt portions take the shared-page form: below, one-tile items fill more
 SINK_DECODE_PAGES = 32    # fewest pages of a full cache that a workgroup's stretch of a split walk is worth
 SINK_ROWS_TILE = 16   # query rows per work item of the sink attention's MFMA form (one head per wave)
 
@@ -219,8 +218,20 @@ class LayeredRunner(RunnerBase):
             if rot is not None and rot.dims > 0 and rot not in self._rope:
                 self._rope[rot] = rot.table(self.max_model_len + 1, dev)
         flash = [r for r, (_, d, v) in kv.items() if ops.sink_flash_ok(self.dtype, d, v)]
+        self._tile_rows = self._sink_tile_rows([cfg.layers[r.layer].mixer.left for r in self.runs if r.index in flash])
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MatrixStateCache(st, self.max_batch, dev)
+
+    def _sink_tile_rows(self, mixers) -> list:
+        """Rows per work item of the shared-page form of the given sink attention layers, each once."""
+        return sorted({ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim) for a in mixers} - {0})
+
+    def _prompt_items(self, g: dict, a):
+        """Work items of a prompt group and the query rows of one: the shared-page form, the one-tile form for wide heads."""
+        rows = ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim)
+        if rows and g["tiles"][rows][0].numel() <= 65535:
+            return g["tiles"][rows], rows
+        return (g["hs"], g["ht"]), SINK_ROWS_TILE
 
     # ------------------------------------------------------------------ buffers
     def _buffers(self, M: int) -> dict:
@@ -544,9 +555,10 @@ class LayeredRunner(RunnerBase):
         ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, None, self.kv.v[ri], slots, 0, 0.0, 1.0, vt)
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
-            if vt is not None and g["qt"] > 1:  # prompt portions on the MFMA form: tiles of 16 rows
-                ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["hs"],
-                                   g["ht"], Lw.sink, small[:, :H], ao, a.window, a.scale, SINK_ROWS_TILE, vt)
+            if vt is not None and g["qt"] > 1:  # prompt portions on the MFMA forms
+                work, rows = self._prompt_items(g, a)
+                ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], *work,
+                                   Lw.sink, small[:, :H], ao, a.window, a.scale, rows, vt)
             elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:  # decode rows: tile 0, keys split over the waves
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
                                    g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, SINK_ROWS_TILE, vt, True)
@@ -603,7 +615,9 @@ class LayeredRunner(RunnerBase):
         self.kv = MixedKVCache({r: m.kv_rank + m.rot_dim for r, m in lat.items()}, kv, self.num_blocks, dev, self.dtype,
                                latent_transposed=lflash, kv_transposed=kflash)
         self.state = ConvTailCache(tails, self.max_batch, dev)
-        self._tile_rows = sorted({ops.latent_tile_rows(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash})
+        tiles = {ops.latent_tile_rows(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash}
+        self._tile_rows = sorted(tiles | set(self._sink_tile_rows(
+            [cfg.layers[r.layer].mixer for r in self.runs if r.index in kflash])))
         words = max((ops.latent_flash_part_floats(self.max_batch, m.heads, 16, 16, m.kv_rank) for r, m in lat.items()
                      if r in lflash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -754,8 +768,9 @@ class LayeredRunner(RunnerBase):
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
             if vt is not None and g["qt"] > 1:
-                ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], g["hs"], g["ht"], None, None, ao,
-                                   m.window, m.scale, SINK_ROWS_TILE, vt)
+                work, rows = self._prompt_items(g, m)
+                ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], *work, None, None, ao,
+                                   m.window, m.scale, rows, vt)
             elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:
                 ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], None, None, ao,
                                    m.window, m.scale, SINK_ROWS_TILE, vt, True)
@@ -1037,7 +1052,7 @@ class LayeredRunner(RunnerBase):
                  ops.sink_flash_lds(dm) <= LDS_BYTES]
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MemoryStateCache(mem, convs, self.max_batch, dev)
-        self._tile_rows = sorted({ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim) for a in atts} - {0})
+        self._tile_rows = self._sink_tile_rows(atts)
         words = max((B * a.heads * self._walk_parts(B, a) * (a.vdim + 2) for B in range(1, self.max_batch + 1) for a in atts),
                     default=0)
         self._walk_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -1111,11 +1126,9 @@ class LayeredRunner(RunnerBase):
         kc, vc, vt = self.kv.k[ri], self.kv.v[ri], self.kv.vt.get(ri)
         for g in groups:
             nparts = 1
-            rows = ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim)
-            if vt is not None and g["qt"] > 1 and rows and g["tiles"][rows][0].numel() * a.heads * rows >= 128 * SINK_TILE_GROUPS:
-                work, form = g["tiles"][rows], (rows, vt, False)
-            elif vt is not None and g["qt"] > 1:
-                work, form = (g["hs"], g["ht"]), (SINK_ROWS_TILE, vt, False)
+            if vt is not None and g["qt"] > 1:
+                work, rows = self._prompt_items(g, a)
+                form = (rows, vt, False)
             elif vt is not None and ops.sink_decode_ok(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim):
                 work, form = (g["ws"], g["wt"]), (1, vt, False)
                 nparts = self._walk_parts(g["ws"].numel(), a)
@@ -1186,6 +1199,7 @@ class LayeredRunner(RunnerBase):
         kv = {i: (L.mixer.kv_heads, L.mixer.dim, L.mixer.vdim) for i, L in enumerate(cfg.layers) if cfg.kv_layer(i) == i}
         flash = [i for i, (_, dm, v) in kv.items() if ops.sink_flash_ok(self.dtype, dm, v) and
                  ops.sink_flash_lds(dm) <= LDS_BYTES]
+        self._tile_rows = self._sink_tile_rows([L.mixer for i, L in enumerate(cfg.layers) if cfg.kv_layer(i) in flash])
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MatrixStateCache({}, self.max_batch, dev)  # no layer keeps state beside its pages
         self._pos_table = position_table(self.max_model_len + 1, cfg.width, dev)
@@ -1266,7 +1280,8 @@ class LayeredRunner(RunnerBase):
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
             if vt is not None and g["qt"] > 1:
-                work, form = (g["hs"], g["ht"]), (SINK_ROWS_TILE, vt, False)
+                work, rows = self._prompt_items(g, m)
+                form = (rows, vt, False)
             elif vt is not None and ops.sink_decode_ok(self.dtype, H, G, D, V):
                 work, form = (g["ws"], g["wt"]), (1, vt, False)
             else:

@@ -242,7 +242,7 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, wor
     head's output by its sigmoid.  `qt` query rows per work item (work_seq, work_tile).  With vt (transposed value
     pages [pages, G, V, 32], sink_flash_ok shapes, qt = 16): the MFMA form; split (V <= 128) lets the four waves of a
     workgroup share one (tile, head) and split its pages, for decode steps.  With vt and qt = sink_tile_rows: the shared-page
-    form (no rel, no out_rope), a page staged once for all rows and heads of an item.  With vt and qt = 1: the decode form
+    form (no out_rope), a page staged once for all rows and heads of an item.  With vt and qt = 1: the decode form
     (sink_decode_ok shapes), one row per item, the heads of a key/value group side by side, pages split over the waves of
     a workgroup.  softcap > 0: scores
     softcap * tanh(scale q.k / softcap).  out_rope ([positions, V / 2, 2] (cos, sin), rotate-half pairs over the whole
