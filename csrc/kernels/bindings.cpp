@@ -293,7 +293,7 @@ double pipe_est_us(int M, int N, int K, int bm, int S, bool fix, int out_bytes =
                    kFixSync = 12.0, kNext = 5.68, kHbm = 4.458e6, kCUs = 256;
   const int nbm = (M + bm - 1) / bm, rows = std::min(bm, M);
   const double Kr = (double)K / S;
-  const long wgs = (long)nbm * (N / 256) * S;
+  const long wgs = (long)nbm * ((N + 255) / 256) * S;
   const long full = wgs / (long)kCUs, rem = wgs - full * (long)kCUs;
   const double t_wg = kT0 + std::max((double)(rows + 256) * Kr * 2 / kFill, 2.0 * bm * 256 * Kr / kMfma);
   double t = full * t_wg + (rem ? t_wg * (kPartial + (1 - kPartial) * rem / kCUs) : 0.0);
@@ -312,7 +312,7 @@ TCfg pipe_plan(int M, int N, int K, bool slab_consumer) {
   best.ok = false;
   const bool no_fix = env_int("t_fix", -1) == 0;  // t_fix=0 (DSSE_KERNEL_CFG): slabs only, for A/Bs
   for (int bm : {256, 192, 128}) {
-    const long tiles = (long)((M + bm - 1) / bm) * (N / 256);
+    const long tiles = (long)((M + bm - 1) / bm) * ((N + 255) / 256);
     for (int S = 1; S <= 16; S *= 2) {
       if (K % (128 * S) != 0) break;
       for (int fix = 0; fix < 2; ++fix) {
@@ -335,11 +335,22 @@ TCfg pipe_plan(int M, int N, int K, bool slab_consumer) {
 
 constexpr int kModelMinM = 256;  // above this many rows every N % 256 == 0 projection is planned by pipe_plan
 
+// N % 256 == 128 on gemm_pipe: its last column block is half empty, and short or narrow products are better cut into the
+// 128-column tiles of gemm_tiled.  Measured, gemm_tiled against gemm_pipe in us (rows x N x K): 320 x 5248 x 2048 21 / 25,
+// 800 x 3200 x 2048 26 / 28, 512 x 1664 x 4096 26 / 26; 1500 x 1152 x 2048 34 / 27, 800 x 5248 x 2048 37 / 31, 257 x 8320 x
+// 2048 44 / 25, 257 x 2176 x 4096 33 / 24, 800 x 1152 x 4096 44 / 27, 2048 x 26752 x 4096 509 / 386.
+bool half_block_pays(int M, int N, int K) {
+  const int64_t weight = (int64_t)N * K;
+  if (K >= 4096) return M > 512 || N >= 2048;
+  return M > 1024 || weight >= (1 << 24) || (M > 512 && weight >= (1 << 23));
+}
+
 TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
   TCfg c{};
   int cfg = env_int("t_cfg", -1);
   const bool forced = cfg == 0 || cfg == 1 || cfg == 5 || cfg == 8 || cfg == 9 || cfg == 10;
-  if (!forced && env_int("t_model", 1) && N % 256 == 0 && K % 128 == 0 && M > kModelMinM) {
+  if (!forced && env_int("t_model", 1) && N % 128 == 0 && K % 128 == 0 && M > kModelMinM &&
+      (N % 256 == 0 || half_block_pays(M, N, K))) {
     c = pipe_plan(M, N, K, slab_consumer);
     if (c.ok) return c;
   }

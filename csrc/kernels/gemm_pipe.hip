@@ -99,7 +99,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
   // ---- tile order: bijective XCD remap, then groups of 8 row blocks swept column by column (L2 panel reuse)
   constexpr int QR = BM / 4, QI = QR / 16;  // X rows per quadrant, MFMA row tiles per quadrant
   static_assert(BM == 256 || BM == 192 || BM == 128, "row tile");
-  const int nbm = (M + BM - 1) / BM, nbn = N / 256, ntile = nbm * nbn;
+  const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256, ntile = nbm * nbn;
   const int nwg = gridDim.x;
   const int bid = blockIdx.x, xcd = bid % 8, q8 = nwg / 8, rem = nwg % 8;
   const int lid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + bid / 8;
@@ -134,7 +134,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       a_vo[q][i] = sr < QR && xrow < M ? (uint32_t)(((size_t)xrow * ldx + 32 * (pc >> 1) + 8 * (pc & 1)) * 2) : kOOB;
       const int tb = (j >> 2) * 4 + q * 2 + ((j >> 1) & 1), sub = j & 1;  // column tile of the block, k sub-step
       b_lo[q][i] = kA + tb * 2048 + sub * 1024;
-      b_vo[q][i] = (uint32_t)((((size_t)(n0 / 16 + tb) * KC) * kTileChunk + sub * 512 + lane * 8) * 2);
+      b_vo[q][i] = n0 + 16 * tb < N ? (uint32_t)((((size_t)(n0 / 16 + tb) * KC) * kTileChunk + sub * 512 + lane * 8) * 2) : kOOB;
     }
   // K step t: X columns 128c + 16h + (piece offsets), W chunk c, k sub-steps 2h, 2h+1
   auto a_so = [&](int t) {
@@ -343,11 +343,13 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
 
   // acc[4 qm + i] holds X rows row0 + QR qm + 16 i (i < QI)
   const int row0 = m0 + wm * (BM / 2), tile0 = n0 / 16 + wn * 4;
+  const bool cols = tile0 * 16 < N;  // uniform; N % 128 == 0: a wave's 64 columns are all there or none is
   auto mrow = [&](int mt) { return row0 + QR * (mt >> 2) + 16 * (mt & 3); };
   if constexpr (MODE == kStoreBf16) {
     // stage the wave's 128 x 64 bf16 tile in LDS (all DMA retired, everyone past its last fragment read), then
     // 16-byte row stores: 8 lanes per 128-byte row, 8 rows per instruction
     __syncthreads();
+    if (!cols) return;
     bf16* st = reinterpret_cast<bf16*>(smem + w * (128 * 64 * 2));
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt)
@@ -372,6 +374,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     if constexpr (FIX) stamp(ep, 5, now());
     return;
   }
+  if (!cols) return;
   if constexpr (MODE == kSiluMul) {
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt)
@@ -405,7 +408,7 @@ static hipError_t launch_pipe_bm(const bf16* X, int ldx, int M, const bf16* W, i
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)gp::kLDS);
     attr_set = true;
   }
-  const int nbm = (M + BM - 1) / BM, nbn = N / 256;
+  const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256;
   hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(nbm * nbn * S), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
                      N, K / S, ep, part);
   return hipGetLastError();
@@ -420,14 +423,14 @@ static hipError_t launch_pipe(int bm, const bf16* X, int ldx, int M, const bf16*
 
 }  // namespace dsse
 
-// Shape contract (checked here): N % 256 == 0, K % (128 S) == 0 (>= 2 K steps of 64 per slice), the tiled weight
+// Shape contract (checked here): N % 128 == 0 (the last column block may be half empty: zeros loaded, nothing stored), K % (128 S) == 0 (>= 2 K steps of 64 per slice), the tiled weight
 // layout (api.h), X rows of ldx >= K elements.  S > 1: partial_only 0 = fp32 slabs [S, M, N] into `part` reduced by
 // launch_splitk_reduce, 1 = the slabs only (the consumer reduces them), 2 = in-launch fix-up (FIX above): `part`
 // holds dsse_gemm_pipe_fix_floats() floats and ep->fix_cnt the counters (api.h), tiles <= kFixTiles.
 extern "C" hipError_t dsse_gemm_pipe(int mode, int bm, int S, int partial_only, const void* X, int ldx, int M,
                                      const void* W, int K, int N, const dsse::GemmEpi* ep, float* part, hipStream_t st) {
   using namespace dsse;
-  if (M < 1 || N % 256 != 0 || S < 1 || K % (128 * S) != 0 || ldx < K || (bm != 256 && bm != 192 && bm != 128))
+  if (M < 1 || N % 128 != 0 || S < 1 || K % (128 * S) != 0 || ldx < K || (bm != 256 && bm != 192 && bm != 128))
     return hipErrorInvalidValue;
   const bf16* x = reinterpret_cast<const bf16*>(X);
   const bf16* w = reinterpret_cast<const bf16*>(W);
@@ -442,7 +445,7 @@ extern "C" hipError_t dsse_gemm_pipe(int mode, int bm, int S, int partial_only, 
     return hipErrorInvalidValue;
   }
   if (partial_only == 2) {
-    if (ep->fix_cnt == nullptr || (size_t)((M + bm - 1) / bm) * (N / 256) > (size_t)kFixTiles) return hipErrorInvalidValue;
+    if (ep->fix_cnt == nullptr || (size_t)((M + bm - 1) / bm) * ((N + 255) / 256) > (size_t)kFixTiles) return hipErrorInvalidValue;
     switch (mode) {
       case kStoreBf16: return launch_pipe<kStoreBf16, true>(bm, x, ldx, M, w, K, N, S, *ep, part, st);
       case kStoreF32: return launch_pipe<kStoreF32, true>(bm, x, ldx, M, w, K, N, S, *ep, part, st);
@@ -460,5 +463,5 @@ extern "C" hipError_t dsse_gemm_pipe(int mode, int bm, int S, int partial_only, 
 // Workspace floats of the in-launch fix-up (partial_only = 2): S - 1 register-order slots per tile.
 extern "C" size_t dsse_gemm_pipe_fix_floats(int bm, int S, int M, int N) {
   const int nbm = (M + bm - 1) / bm, qi = bm / 64;
-  return (size_t)nbm * (N / 256) * (S - 1) * (8 * 8 * qi * 64) * 4;
+  return (size_t)nbm * ((N + 255) / 256) * (S - 1) * (8 * 8 * qi * 64) * 4;
 }
