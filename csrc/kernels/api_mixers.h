@@ -73,6 +73,10 @@ struct SinkAttnParams {
   float* part;           // [work items, H, nparts, V + 2] when split
 };
 
+// Whether the exact mode's shared-page form (sink_exact.hip) takes a launch of num_work items of p.qt rows: fp32, head widths up
+// to 128 in multiples of 16, 16 / 32 / 64 rows per item with groups of 4 / 2 / 1 heads, no output rotation, 16-byte-aligned rows.
+bool sink_exact_ok(const SinkAttnParams& p, int64_t num_work);
+
 // The fused projection's q | k | v columns into the attention's operands.
 struct QkvRowsParams {
   const float* x;        // rows ldx apart: [q (H D) | k (G D) | v (G V) | ..] (only q when k is null)
@@ -239,6 +243,7 @@ hipError_t dsse_sink_attention(int num_work, const dsse::SinkAttnParams* p, hipS
 // split (V <= 128): the four waves of a workgroup share one (tile, head) and split its pages -- decode steps
 hipError_t dsse_sink_flash(int num_work, const dsse::SinkAttnParams* p, const void* vt, int split, hipStream_t st);
 // prompt portions with every page staged once for 8 / rt heads of a key/value group and rt tiles of 16 rows (rt 2, 4, 8)
+hipError_t dsse_sink_exact(int num_work, const dsse::SinkAttnParams* p, hipStream_t st);
 hipError_t dsse_sink_tile(int num_work, const dsse::SinkAttnParams* p, const void* vt, int rt, hipStream_t st);
 // decode form over the same pages: one row per item, the heads of a key/value group side by side, pages split over waves
 hipError_t dsse_sink_decode(int num_work, const dsse::SinkAttnParams* p, const void* vt, hipStream_t st);

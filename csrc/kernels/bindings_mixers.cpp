@@ -281,6 +281,10 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
     DSSE_CHECK_HIP(dsse_sink_flash((int)work_seq.numel(), &p, vt->data_ptr(), split ? 1 : 0, cur_stream()));
     return;
   }
+  if (dsse::sink_exact_ok(p, work_seq.numel())) {
+    DSSE_CHECK_HIP(dsse_sink_exact((int)work_seq.numel(), &p, cur_stream()));
+    return;
+  }
   DSSE_CHECK_HIP(dsse_sink_attention((int)work_seq.numel(), &p, cur_stream()));
 }
 

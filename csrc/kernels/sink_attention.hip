@@ -18,10 +18,10 @@
 // "nothing".  Scores, the running maximum, the weights and the output sums are fp32 in both element types; queries
 // arrive in fp32 (normed and rotated), keys and values are read from their pages in the cache's element type.
 //
-// Row kernel (any sizes, both element types; every decode step): a workgroup serves `qt` query rows of one head; for each row its four waves split the keys in chunks of
+// Row kernel (any sizes, both element types): a workgroup serves `qt` query rows of one head; for each row its four waves split the keys in chunks of
 // 64 (one key per lane for the scores, then one output coordinate per lane and 64 broadcast weights for the values),
-// keep their own running (max, sum, output) and are merged through LDS.  A decode row and a prompt row take the same
-// path, so a position's result does not depend on how the prompt was cut.
+// keep their own running (max, sum, output) and are merged through LDS.  Exact-mode prompt portions whose widths fit take
+// sink_exact.hip instead.
 #include "api_mixers.h"
 
 namespace dsse {

@@ -218,7 +218,7 @@ class LayeredRunner(RunnerBase):
             if rot is not None and rot.dims > 0 and rot not in self._rope:
                 self._rope[rot] = rot.table(self.max_model_len + 1, dev)
         flash = [r for r, (_, d, v) in kv.items() if ops.sink_flash_ok(self.dtype, d, v)]
-        self._tile_rows = self._sink_tile_rows([cfg.layers[r.layer].mixer.left for r in self.runs if r.index in flash])
+        self._tile_rows = self._sink_tile_rows([cfg.layers[r.layer].mixer.left for r in self.runs if r.index in kv])
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MatrixStateCache(st, self.max_batch, dev)
 
@@ -226,12 +226,13 @@ class LayeredRunner(RunnerBase):
         """Rows per work item of the shared-page form of the given sink attention layers, each once."""
         return sorted({ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim) for a in mixers} - {0})
 
-    def _prompt_items(self, g: dict, a):
-        """Work items of a prompt group and the query rows of one: the shared-page form, the one-tile form for wide heads."""
+    def _prompt_items(self, g: dict, a, vt):
+        """Work items of a prompt group and the query rows of one: the shared-page forms, the one-tile MFMA form for wide heads
+        (transposed value pages vt), the row form for head widths that none covers."""
         rows = ops.sink_tile_rows(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim)
         if rows and g["tiles"][rows][0].numel() <= 65535:
             return g["tiles"][rows], rows
-        return (g["hs"], g["ht"]), SINK_ROWS_TILE
+        return ((g["hs"], g["ht"]), SINK_ROWS_TILE) if vt is not None else ((g["ws"], g["wt"]), g["qt"])
 
     # ------------------------------------------------------------------ buffers
     def _buffers(self, M: int) -> dict:
@@ -555,8 +556,8 @@ class LayeredRunner(RunnerBase):
         ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, None, self.kv.v[ri], slots, 0, 0.0, 1.0, vt)
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
-            if vt is not None and g["qt"] > 1:  # prompt portions on the MFMA forms
-                work, rows = self._prompt_items(g, a)
+            if g["qt"] > 1:  # prompt portions
+                work, rows = self._prompt_items(g, a, vt)
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], *work,
                                    Lw.sink, small[:, :H], ao, a.window, a.scale, rows, vt)
             elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:  # decode rows: tile 0, keys split over the waves
@@ -617,7 +618,7 @@ class LayeredRunner(RunnerBase):
         self.state = ConvTailCache(tails, self.max_batch, dev)
         tiles = {ops.latent_tile_rows(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash}
         self._tile_rows = sorted(tiles | set(self._sink_tile_rows(
-            [cfg.layers[r.layer].mixer for r in self.runs if r.index in kflash])))
+            [cfg.layers[r.layer].mixer for r in self.runs if r.index in kv])))
         words = max((ops.latent_flash_part_floats(self.max_batch, m.heads, 16, 16, m.kv_rank) for r, m in lat.items()
                      if r in lflash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -767,8 +768,8 @@ class LayeredRunner(RunnerBase):
         ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, None, vc, slots, 0, 0.0, 1.0, vt)
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
-            if vt is not None and g["qt"] > 1:
-                work, rows = self._prompt_items(g, m)
+            if g["qt"] > 1:
+                work, rows = self._prompt_items(g, m, vt)
                 ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], *work, None, None, ao,
                                    m.window, m.scale, rows, vt)
             elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:
@@ -1126,8 +1127,8 @@ class LayeredRunner(RunnerBase):
         kc, vc, vt = self.kv.k[ri], self.kv.v[ri], self.kv.vt.get(ri)
         for g in groups:
             nparts = 1
-            if vt is not None and g["qt"] > 1:
-                work, rows = self._prompt_items(g, a)
+            if g["qt"] > 1:
+                work, rows = self._prompt_items(g, a, vt)
                 form = (rows, vt, False)
             elif vt is not None and ops.sink_decode_ok(self.dtype, a.heads, a.kv_heads, a.dim, a.vdim):
                 work, form = (g["ws"], g["wt"]), (1, vt, False)
@@ -1199,7 +1200,7 @@ class LayeredRunner(RunnerBase):
         kv = {i: (L.mixer.kv_heads, L.mixer.dim, L.mixer.vdim) for i, L in enumerate(cfg.layers) if cfg.kv_layer(i) == i}
         flash = [i for i, (_, dm, v) in kv.items() if ops.sink_flash_ok(self.dtype, dm, v) and
                  ops.sink_flash_lds(dm) <= LDS_BYTES]
-        self._tile_rows = self._sink_tile_rows([L.mixer for i, L in enumerate(cfg.layers) if cfg.kv_layer(i) in flash])
+        self._tile_rows = self._sink_tile_rows([L.mixer for L in cfg.layers])
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MatrixStateCache({}, self.max_batch, dev)  # no layer keeps state beside its pages
         self._pos_table = position_table(self.max_model_len + 1, cfg.width, dev)
@@ -1279,8 +1280,8 @@ class LayeredRunner(RunnerBase):
         gate = big[:, c0:c0 + H * V]
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
-            if vt is not None and g["qt"] > 1:
-                work, rows = self._prompt_items(g, m)
+            if g["qt"] > 1:
+                work, rows = self._prompt_items(g, m, vt)
                 form = (rows, vt, False)
             elif vt is not None and ops.sink_decode_ok(self.dtype, H, G, D, V):
                 work, form = (g["ws"], g["wt"]), (1, vt, False)

@@ -222,7 +222,12 @@ def sink_decode_ok(dtype, heads: int, kv_heads: int, dim: int, vdim: int) -> boo
 
 def sink_tile_rows(dtype, heads: int, kv_heads: int, dim: int, vdim: int) -> int:
     """Query rows per work item of the shared-page form of sink_attention (32, 64 or 128: the heads of a key/value group
-    that fill the rest of eight 16-column tiles), 0 for shapes it does not cover."""
+    that fill the rest of eight 16-column tiles; in fp32 16, 32 or 64, four tiles), 0 for shapes it does not cover."""
+    if dtype == torch.float32:
+        if dim % 16 or vdim % 16 or dim > 128 or vdim > 128:
+            return 0
+        rep = heads // kv_heads
+        return 16 if rep % 4 == 0 else (32 if rep % 2 == 0 else 64)
     if not sink_flash_ok(dtype, dim, vdim) or dim > 128 or vdim > 128:
         return 0
     rep = heads // kv_heads
@@ -242,7 +247,7 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, wor
     head's output by its sigmoid.  `qt` query rows per work item (work_seq, work_tile).  With vt (transposed value
     pages [pages, G, V, 32], sink_flash_ok shapes, qt = 16): the MFMA form; split (V <= 128) lets the four waves of a
     workgroup share one (tile, head) and split its pages, for decode steps.  With vt and qt = sink_tile_rows: the shared-page
-    form (no out_rope), a page staged once for all rows and heads of an item.  With vt and qt = 1: the decode form
+    form (no out_rope), a page staged once for all rows and heads of an item (fp32 caches: the same without vt).  With vt and qt = 1: the decode form
     (sink_decode_ok shapes), one row per item, the heads of a key/value group side by side, pages split over the waves of
     a workgroup.  softcap > 0: scores
     softcap * tanh(scale q.k / softcap).  out_rope ([positions, V / 2, 2] (cos, sin), rotate-half pairs over the whole
