@@ -9,6 +9,7 @@
 //   * Every kernel takes an explicit hipStream_t from the caller (torch's current stream),
 //     so the whole decode step can be captured into one hipGraph.
 #pragma once
+#include <initializer_list>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -107,6 +108,29 @@ DEV float rows4_sum(float v) {
   v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
   const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+
+// four consecutive elements as fp32 (16-byte-aligned fp32, 8-byte-aligned bf16)
+DEV f32x4 ld4(const float* p) { return ld_global<f32x4>(p); }
+DEV f32x4 ld4(const bf16* p) {
+  const bf16x4 v = ld_global<bf16x4>(p);
+  return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+DEV void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+DEV void st4(bf16* p, f32x4 v) { *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]}; }
+// host: pointers that ld4 / st4 may take, null ones included
+inline bool fours(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+  return true;
+}
+// host: threads of a workgroup that keeps a row of W <= 16384 floats (W % 4 == 0) in registers, at most four groups of four per
+// thread: as many as the row has groups while the rows leave CUs empty, 256 where they do not
+inline int row_threads(int M, int W) {
+  const int groups = (W / 4 + 63) / 64 * 64;
+  const int least = (groups / 4 + 63) / 64 * 64, most = groups < 1024 ? groups : 1024;
+  const int want = M <= 512 ? most : (256 < most ? 256 : most);
+  return want < least ? least : want;
 }
 
 DEV float silu(float x) { return x / (1.0f + __expf(-x)); }
