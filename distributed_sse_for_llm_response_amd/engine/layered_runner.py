@@ -560,7 +560,10 @@ class LayeredRunner(RunnerBase):
                 work, rows = self._prompt_items(g, a, vt)
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], *work,
                                    Lw.sink, small[:, :H], ao, a.window, a.scale, rows, vt)
-            elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:  # decode rows: tile 0, keys split over the waves
+            elif vt is not None and ops.sink_decode_ok(self.dtype, H, G, D, V):  # decode rows: a group's heads side by side
+                ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
+                                   g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, 1, vt)
+            elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:  # tile 0, keys split over the waves
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
                                    g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, SINK_ROWS_TILE, vt, True)
             else:
