@@ -413,6 +413,90 @@ hipError_t launch(const MatrixScanParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// Decode rows of tile-major states (V % 16 == 0, D = 16 NR): one wave per (sequence, head, 16 columns), a lane the rows
+// 16 i + lane / 4 of four columns in 16-byte pieces, no LDS and no barrier.  Sums over D are NR products in a lane, two row
+// rotations and two row swaps.
+//
+// What bounds it: the state, read and written once -- 67 MB at 16 sequences of 32 heads of 128 x 128 -- behind one chain of
+// loads (lengths, then everything else).  matrix_scan_kernel, which stages blocks of tokens for eight waves, took 37 us with
+// the delta rule there, this 11; 128 sequences 258 and 82; one sequence 5.7 and 4.2.  A sequence with several rows walks them, the next row's operands in flight.
+template <int NR, bool DELTA>
+__global__ __launch_bounds__(256) void matrix_scan_step_kernel(MatrixScanParams p) {
+  const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (tile * kScanCols >= p.V) return;  // uniform for the wave
+  const int ql = p.q_len[seq], row0 = p.q_start[seq], ctx = p.ctx_len[seq], slot = p.state_slot[seq];
+  if (ql <= 0) return;
+  const int dr = lane >> 2, cq = lane & 3, D = 16 * NR;
+  const int g = h / (p.H / p.G), j = tile * kScanCols + 4 * cq;
+  const bool chan = p.decay_kind == 3;
+  float* st = p.state + ((int64_t)slot * p.H + h) * D * p.V + ((int64_t)tile * D + dr) * kScanCols + 4 * cq;
+  const float fixed = p.decay_kind == 1 ? p.decay[h] : 1.0f;
+  float nk[NR], nq[NR], na[NR], nb = 0.f, ns = fixed;
+  f32x4 nv;
+  auto request = [&](int t) {  // rows past the last one read it again
+    const int64_t row = row0 + (t < ql ? t : ql - 1);
+    const float* k = p.k + row * p.ldk + g * D + dr;
+    const float* q = p.q + row * p.ldq + g * D + dr;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) nk[i] = k[16 * i], nq[i] = q[16 * i];
+    if (chan) {
+      const float* a = p.decay + row * p.ldd + h * D + dr;
+#pragma unroll
+      for (int i = 0; i < NR; ++i) na[i] = a[16 * i];
+    } else if (p.decay_kind == 2) {
+      ns = p.decay[row * p.ldd + h];
+    }
+    if (DELTA) nb = p.beta[row * p.ldb + h];
+    nv = ld4(p.v + row * p.ldv + h * p.V + j);
+  };
+  request(0);
+  f32x4 S[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (ctx - ql != 0)  // a sequence's first step starts from zeros
+#pragma unroll
+    for (int i = 0; i < NR; ++i) S[i] = ld4(st + 16 * i * kScanCols);
+  for (int t = 0; t < ql; ++t) {
+    float k[NR], q[NR];
+    f32x4 u = nv;
+    const float b = nb;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      k[i] = nk[i], q[i] = nq[i] * p.q_scale;
+      S[i] = S[i] * (chan ? na[i] : ns);
+    }
+    if (t + 1 < ql) request(t + 1);
+    if (DELTA) {
+      f32x4 part = S[0] * k[0];
+#pragma unroll
+      for (int i = 1; i < NR; ++i) part += S[i] * k[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) u[e] = b * (u[e] - groups16_sum(part[e]));
+    }
+    f32x4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      S[i] += k[i] * u;
+      o += S[i] * q[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = groups16_sum(o[e]);
+    if (dr == 0) st4(p.out + ((int64_t)(row0 + t) * p.H + h) * p.V + j, o);
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) st4(st + 16 * i * kScanCols, S[i]);
+}
+
+template <int NR>
+hipError_t launch_step(const MatrixScanParams& p, hipStream_t st) {
+  const dim3 grid((p.V + 4 * kScanCols - 1) / (4 * kScanCols), p.H, p.nseq);
+  if (p.beta) hipLaunchKernelGGL((matrix_scan_step_kernel<NR, true>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((matrix_scan_step_kernel<NR, false>), grid, dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
 }  // namespace
 }  // namespace dsse
 
@@ -427,8 +511,14 @@ extern "C" hipError_t dsse_matrix_scan(const dsse::MatrixScanParams* p, hipStrea
     if (p->D <= 256) return dsse::launch_wave<16, 8>(*p, st);
     return dsse::launch_wave<32, 4>(*p, st);
   }
-  // rows of S per lane (a wave holds 4 DPT rows of 16 columns, a workgroup up to 16 waves) and tokens per block (as
-  // long as 64 KB of LDS allow)
+  if (p->V % dsse::kScanCols == 0 && p->ldv % 4 == 0 && dsse::fours({p->state, p->v, p->out})) {
+    if (p->D == 16) return dsse::launch_step<1>(*p, st);
+    if (p->D == 32) return dsse::launch_step<2>(*p, st);
+    if (p->D == 64) return dsse::launch_step<4>(*p, st);
+    if (p->D == 128) return dsse::launch_step<8>(*p, st);
+  }
+  // other widths.  Rows of S per lane (a wave holds 4 DPT rows of 16 columns, a workgroup up to 16 waves) and tokens per block
+  // (as long as 64 KB of LDS allow)
   if (p->D <= 64) return dsse::launch<2, 16>(*p, st);
   if (p->D <= 128) return dsse::launch<4, 16>(*p, st);
   if (p->D <= 256) return dsse::launch<4, 8>(*p, st);
