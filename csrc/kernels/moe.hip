@@ -162,16 +162,17 @@ DEV void align_ids(int M, int S, int top, int E, Choice choice, int* sorted, int
   int* cnt = sm;            // [NE]
   int* off = sm + NE;       // [NE + 1] first sorted position of each expert (multiples of kMoeRows)
   int* fill = off + NE + 1; // [NE]
-  const int n = M * S;
-  auto expert_of = [&](int id) {
-    const int row = id / S, k = id % S;
-    const int e = k < top ? choice(row, k) : E;
+  // choices only: every row goes to a shared expert, whose list is the rows in order (counting those with the others put M
+  // atomics on one address)
+  const int n = M * top;
+  auto expert_of = [&](int i) {
+    const int e = choice(i / top, i % top);
     return (unsigned)e < (unsigned)NE ? e : 0;
   };
-  const int mine = (int)threadIdx.x < n ? expert_of(threadIdx.x) : 0;  // a thread's first id: read once
-  for (int e = threadIdx.x; e < NE; e += blockDim.x) cnt[e] = 0, fill[e] = 0;
+  const int mine = (int)threadIdx.x < n ? expert_of(threadIdx.x) : 0;  // a thread's first choice: read once
+  for (int e = threadIdx.x; e < NE; e += blockDim.x) cnt[e] = e == E ? M : 0, fill[e] = e == E ? M : 0;
   __syncthreads();
-  for (int id = threadIdx.x; id < n; id += blockDim.x) atomicAdd(&cnt[id == (int)threadIdx.x ? mine : expert_of(id)], 1);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) atomicAdd(&cnt[i == (int)threadIdx.x ? mine : expert_of(i)], 1);
   __syncthreads();
   if (threadIdx.x < 64) {  // offsets: a wave's prefix sums over the padded counts, 64 experts at a time
     const int lane = threadIdx.x;
@@ -199,13 +200,15 @@ DEV void align_ids(int M, int S, int top, int E, Choice choice, int* sorted, int
     for (int t = off[e] / kMoeRows; t < off[e + 1] / kMoeRows; ++t) tile_expert[t] = e;
   for (int t = total / kMoeRows + threadIdx.x; t < max_tiles; t += blockDim.x) tile_expert[t] = -1;
   __syncthreads();
-  for (int id = threadIdx.x; id < n; id += blockDim.x) {
-    const int e = id == (int)threadIdx.x ? mine : expert_of(id);
-    sorted[off[e] + atomicAdd(&fill[e], 1)] = id;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const int e = i == (int)threadIdx.x ? mine : expert_of(i);
+    sorted[off[e] + atomicAdd(&fill[e], 1)] = i / top * S + i % top;
   }
+  if (NE > E)
+    for (int row = threadIdx.x; row < M; row += blockDim.x) sorted[off[E] + row] = row * S + top;
 }
 
-__global__ __launch_bounds__(256) void moe_align_kernel(MoeGroupedParams p) {
+__global__ __launch_bounds__(1024) void moe_align_kernel(MoeGroupedParams p) {
   extern __shared__ int sm[];
   align_ids(p.M, p.S, p.top, p.E, [&](int row, int k) { return p.topk_idx[row * p.top + k]; }, p.sorted, p.tile_expert,
             p.num_tiles, p.max_tiles, sm);
@@ -675,7 +678,8 @@ extern "C" hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStrea
   if (p->M <= 0) return hipSuccess;
   const int NE = p->E + (p->S > p->top ? 1 : 0);
   if (!p->aligned)
-    hipLaunchKernelGGL(dsse::moe_align_kernel, dim3(1), dim3(256), sizeof(int) * (3 * NE + 1), st, *p);
+    hipLaunchKernelGGL(dsse::moe_align_kernel, dim3(1), dim3((int64_t)p->M * p->top > 256 ? 1024 : 256),
+                       sizeof(int) * (3 * NE + 1), st, *p);
   const int fmax = p->F > p->Fs ? p->F : p->Fs;
   dim3 g1((fmax + 15) / 16, p->max_tiles), g2((p->W + 15) / 16, p->max_tiles);
   if (dsse::moe_pipe_ok(*p)) return dsse_moe_pipe(p, st);
