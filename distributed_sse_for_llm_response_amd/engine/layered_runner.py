@@ -235,54 +235,57 @@ class LayeredRunner(RunnerBase):
         return ((g["hs"], g["ht"]), SINK_ROWS_TILE) if vt is not None else ((g["ws"], g["wt"]), g["qt"])
 
     # ------------------------------------------------------------------ buffers
-    def _buffers(self, M: int) -> dict:
+    def _buffers(self, M: int, clear: bool = True) -> dict:
+        """Activations of a step of M rows.  clear=False (a prompt pass: every row belongs to a portion): what each step writes
+        whole before it reads it is not zeroed first -- a dozen fills and launches per pass."""
         cfg, dev = self.cfg, self.device
+        new = torch.zeros if clear else torch.empty
         f32 = dict(device=dev, dtype=torch.float32)
         el = dict(device=dev, dtype=self.dtype)
         W = cfg.width
-        d = {"resid": torch.zeros(M, W, **f32), "xb": torch.zeros(M, W, **el), "y": torch.zeros(M, W, **f32)}
+        d = {"resid": new(M, W, **f32), "xb": new(M, W, **el), "y": new(M, W, **f32)}
         if self.joint:
-            d.update(self._joint_buffers(M))
+            d.update(self._joint_buffers(M, new))
             return d
         if self.bracket:
-            d.update(self._memory_buffers(M) if self.memory else self._bracket_buffers(M))
+            d.update(self._memory_buffers(M, new) if self.memory else self._bracket_buffers(M))
             return d
         if self.multistream:
             d.update(self._stream_buffers(M))
             return d
         if self.prenorm:
-            d.update(self._prenorm_buffers(M))
+            d.update(self._prenorm_buffers(M, new))
             return d
         att = [L.mixer for L in cfg.layers if L.kind == "latent_attention"]
         rec = [L.mixer for L in cfg.layers if L.kind == "rglru"]
         moe = [L.mlp for L in cfg.layers if L.mlp is not None]
         if att:
-            d["q"] = torch.zeros(M * max(m.heads * (m.dim + m.rot_dim) for m in att), **el)
-            d["ckr"] = torch.zeros(M * max(m.kv_rank + m.rot_dim for m in att), **f32)
-            d["qabs"] = torch.zeros(M * max(m.heads * m.kv_rank for m in att), **f32)
-            d["lat"] = torch.zeros(M * max(m.heads * m.kv_rank for m in att), **el)
-            d["attn"] = torch.zeros(M * max(m.heads * m.vdim for m in att), **el)
+            d["q"] = new(M * max(m.heads * (m.dim + m.rot_dim) for m in att), **el)
+            d["ckr"] = new(M * max(m.kv_rank + m.rot_dim for m in att), **f32)
+            d["qabs"] = new(M * max(m.heads * m.kv_rank for m in att), **f32)
+            d["lat"] = new(M * max(m.heads * m.kv_rank for m in att), **el)
+            d["attn"] = new(M * max(m.heads * m.vdim for m in att), **el)
         if rec:
             C = max(m.width for m in rec)
-            d["ub"], d["hs"] = (torch.zeros(M * C, **el) for _ in range(2))
-            d["yr"], d["ux"], d["u"] = (torch.zeros(M * C, **f32) for _ in range(3))
-            d["gates"] = torch.zeros(M * 2 * C, **f32)
+            d["ub"], d["hs"] = (new(M * C, **el) for _ in range(2))
+            d["yr"], d["ux"], d["u"] = (new(M * C, **f32) for _ in range(3))
+            d["gates"] = new(M * 2 * C, **f32)
             # chunked walk of the recurrence over prompt portions: (A, B) per 32-row chunk
-            d["scan"] = torch.zeros(2 * (M // 32 + max(M, self.max_batch) + 2) * C, **f32) if M >= 128 else None
+            d["scan"] = new(2 * (M // 32 + max(M, self.max_batch) + 2) * C, **f32) if M >= 128 else None
         if moe:
             top = max(f.top for f in moe)
             d["tki"] = torch.zeros(M * top, device=dev, dtype=torch.int32)
-            d["tkw"] = torch.zeros(M * top, **f32)
+            d["tkw"] = new(M * top, **f32)
             # grouped experts: ids = (row, slot), slots = top (+ 1: the shared expert)
             slots = max(f.top + (1 if f.shared_ff else 0) for f in moe)
             tiles = -(-M * slots // 64) + max(f.experts for f in moe) + 2
-            d["mo_z"] = torch.zeros(M * max(f.experts for f in moe), **f32)
+            d["mo_z"] = new(M * max(f.experts for f in moe), **f32)
             ldh = -(-max(max(f.ff, f.shared_ff) for f in moe) // 8) * 8
             d["mo_sorted"] = torch.zeros(tiles * 64, device=dev, dtype=torch.int32)
             d["mo_tile"] = torch.zeros(tiles, device=dev, dtype=torch.int32)
             d["mo_n"] = torch.zeros(1, device=dev, dtype=torch.int32)
             d["mo_h"] = torch.zeros(M * slots, ldh, **el)
-            d["mo_o"] = torch.zeros(M * slots * W, **f32)
+            d["mo_o"] = new(M * slots * W, **f32)
         return d
 
     # ------------------------------------------------------------------ layers
@@ -427,7 +430,7 @@ class LayeredRunner(RunnerBase):
             self._lin(xn, self.w.head, self.w.head_t, logits)
 
     # ------------------------------------------------------------------ pre-norm designs, matrix-state mixers
-    def _prenorm_buffers(self, M: int) -> dict:
+    def _prenorm_buffers(self, M: int, new) -> dict:
         """Scratch of a step of M rows, each sized for the widest layer: `big` takes the fused projection's fp32 output
         (its column ranges are the mixer's q, k, v and gates), `cv` the convolution's, `z` the per-channel
         decays, `qa` the attention's normed and rotated queries, `o` the recurrences' outputs, `ao` a mixer's gated
@@ -450,10 +453,10 @@ class LayeredRunner(RunnerBase):
                 big, o = max(big, 2 * m.heads * (m.dim + m.vdim)), max(o, m.heads * m.vdim)
             if L.mlp is not None:
                 ff = max(ff, L.mlp.ff)
-        return {"y2": torch.zeros(M, cfg.width, **f32), "big": torch.zeros(M * big, **f32),
-                "cv": torch.zeros(M * cv, **f32), "z": torch.zeros(M * z, **f32),
-                "qa": torch.zeros(M * qa, **f32), "o": torch.zeros(M * o, **f32), "ao": torch.zeros(M * o, **el),
-                "gu": torch.zeros(M * 2 * ff, **f32), "h": torch.zeros(M * ff, **el)}
+        return {"y2": new(M, cfg.width, **f32), "big": new(M * big, **f32),
+                "cv": new(M * cv, **f32), "z": new(M * z, **f32),
+                "qa": new(M * qa, **f32), "o": new(M * o, **f32), "ao": new(M * o, **el),
+                "gu": new(M * 2 * ff, **f32), "h": new(M * ff, **el)}
 
     def _prenorm_layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None) -> None:
         """Every layer run over M packed rows.  Between sublayers ONE stream_step adds the finished sublayer's output
@@ -1062,7 +1065,7 @@ class LayeredRunner(RunnerBase):
         self._walk_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
         self._moe_layers = [i for i, L in enumerate(cfg.layers) if hasattr(L.mlp, "experts") and L.weights_of == i]
 
-    def _memory_buffers(self, M: int) -> dict:
+    def _memory_buffers(self, M: int, new) -> dict:
         """Scratch of a step of M rows, each sized for the widest layer: `big` the fused projection's fp32 output, `qa`
         the attention's queries, `ao` a mixer's gated heads in the element type (both halves of a twin layer side by
         side), `mm` the matrix memory's work area (prompt-sized steps), `up` / `h` the dense feed-forward's hidden row,
@@ -1211,7 +1214,7 @@ class LayeredRunner(RunnerBase):
         # its own between the norm and the next add (a fork and a join in the captured graph)
         self._side_stream = torch.cuda.Stream(dev) if dev.type == "cuda" else None
 
-    def _joint_buffers(self, M: int) -> dict:
+    def _joint_buffers(self, M: int, new) -> dict:
         """Scratch of a step of M rows, each sized for the widest layer: `big` the fused projection's fp32 output, `qa`
         the normed queries, `ao` the gated heads in the element type, `hn` the fp32 normed row the router reads, and the
         experts' lists (slots = top + 1 with a shared expert)."""
@@ -1224,17 +1227,17 @@ class LayeredRunner(RunnerBase):
         qa = max(L.mixer.heads * L.mixer.dim for L in cfg.layers)
         ao = max(L.mixer.heads * L.mixer.vdim for L in cfg.layers)
         moe = [L.mlp for L in cfg.layers if L.mlp is not None]
-        d = {"big": torch.zeros(M * big, **f32), "qa": torch.zeros(M * qa, **f32), "ao": torch.zeros(M * ao, **el),
-             "hn": torch.zeros(M, W, **f32) if moe else None}
+        d = {"big": new(M * big, **f32), "qa": new(M * qa, **f32), "ao": new(M * ao, **el),
+             "hn": new(M, W, **f32) if moe else None}
         if moe:
             slots = max(f.top + (1 if f.shared_ff else 0) for f in moe)
             experts = max(f.experts for f in moe)
             tiles = -(-M * slots // 64) + experts + 2
             ldh = -(-max(max(f.ff, f.shared_ff) for f in moe) // 8) * 8
             d.update({"tki": torch.zeros(M * slots, **i32), "tkw": torch.zeros(M * slots, **f32),
-                      "mo_z": torch.zeros(M * (experts + 1), **f32), "mo_sorted": torch.zeros(tiles * 64, **i32),
+                      "mo_z": new(M * (experts + 1), **f32), "mo_sorted": torch.zeros(tiles * 64, **i32),
                       "mo_tile": torch.zeros(tiles, **i32), "mo_n": torch.zeros(2, **i32),
-                      "mo_h": torch.zeros(M * slots, ldh, **el), "mo_o": torch.zeros(M * slots * W, **f32)})
+                      "mo_h": torch.zeros(M * slots, ldh, **el), "mo_o": new(M * slots * W, **f32)})
         return d
 
     def _joint_layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None) -> None:
@@ -1462,7 +1465,7 @@ class LayeredRunner(RunnerBase):
         if not seqs:
             return
         T, qs, ql, g = self._pack(seqs)
-        d = self._buffers(T)
+        d = self._buffers(T, clear=False)
         self._layers(T, d, g["ids"], g["pos"], g["slots"], [g], trace, prev=(g["prev"], None, None))
         self._remember_last(seqs, g)
         self._prefill_sample(seqs, d["resid"], qs, ql, ring_row)
