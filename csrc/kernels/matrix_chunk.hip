@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
   const int own = 16 * w + r;
   const uint32_t q_vo = (uint32_t)(own * p.ldq + 4 * g) * 4, k_vo = (uint32_t)(own * p.ldk + 4 * g) * 4,
                  m_vo = (uint32_t)(own * kC + 4 * g) * 4,
-                 v_vo = (uint32_t)((16 * w + 4 * g) * p.ldv + r) * 4;
+                 v_vo = (uint32_t)((16 * w + 4 * g) * p.ldv + r) * 4, v_row = (uint32_t)p.ldv * 4;
   auto request = [&](int c, Ch& x) {  // chunks past the last one read it again
     c = c < n ? c : n - 1;
     const int left = ql - c * kC < kC ? ql - c * kC : kC;
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
     }
     x.a = buf4(ur, (kUnitA + 16 * w + 4 * g) * 4, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x.v[i] = buf1(vr, v_vo, (uint32_t)(i * p.ldv) * 4);
+    for (int i = 0; i < 4; ++i) x.v[i] = buf1(vr, v_vo + i * v_row, 0);  // the scalar offset is not range-checked
 #pragma unroll
     for (int t = 0; t < 4; ++t)
       if constexpr (DELTA) x.t[t] = buf4(ur, kUnitT * 4 + m_vo + 64 * t, 0);
