@@ -194,7 +194,7 @@ struct Chunk {
 };
 
 template <int NT, bool DELTA>
-__global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, const float* __restrict__ ws) {
+__global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, const float* __restrict__ ws, int chunks) {
   using Ch = Chunk<NT, DELTA>;
   constexpr int kOwn = Ch::kOwn;
   constexpr int kKeyRow = 16 * NT + 4;  // floats of a key row in LDS: rows four apart start 16 banks apart
@@ -208,6 +208,11 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
   if (ql <= 0) return;  // uniform
   const int first = chunks_before(p.q_len, seq, lane), n = (ql + kC - 1) / kC;
   const int64_t row0 = p.q_start[seq];
+  if (first + n > chunks) {  // uniform.  Only where sequences share rows: no unit was made for this one
+    for (int i = threadIdx.x; i < ql * kScanCols; i += 256)
+      p.out[((row0 + i / kScanCols) * p.H + h) * p.V + cb * kScanCols + i % kScanCols] = __builtin_nanf("");
+    return;
+  }
   constexpr int units = DELTA ? kUnitT + kC * kC : kUnitT;
   const int col = cb * kScanCols + r;
   const bool owner = w * kOwn < NT;  // narrow states have fewer row tiles than waves
@@ -349,7 +354,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
 template <int NT, bool DELTA>
 hipError_t launch_chunks(const MatrixScanParams& p, float* ws, int chunks, hipStream_t st) {
   hipLaunchKernelGGL((chunk_prepare_kernel<NT, DELTA>), dim3(chunks, p.H), dim3(256), 0, st, p, ws);
-  hipLaunchKernelGGL((chunk_walk_kernel<NT, DELTA>), dim3(p.H, p.V / kScanCols, p.nseq), dim3(256), 0, st, p, ws);
+  hipLaunchKernelGGL((chunk_walk_kernel<NT, DELTA>), dim3(p.H, p.V / kScanCols, p.nseq), dim3(256), 0, st, p, ws, chunks);
   return hipGetLastError();
 }
 
@@ -365,10 +370,8 @@ static bool chunks_pay(const MatrixScanParams& p, int64_t rows, int64_t chunks, 
   return walk > (p.beta ? 30 + std::max(6.4 * n, 1.26 * chunks * work) : 18 + std::max(4.4 * n, 0.82 * chunks * work));
 }
 
-// chunks of `rows` rows at most: the launch's workgroups find theirs by the lengths
-static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows, int64_t longest) {
-  return std::min(rows / kC + p.nseq, p.nseq * ((longest + kC - 1) / kC));
-}
+// chunks of `rows` rows at most, whatever their sequences' lengths: the launch's workgroups find theirs by the lengths
+static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows) { return rows / kC + p.nseq; }
 
 int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) {
   auto aligned = [](const float* x, int ld) { return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ld % 4 == 0; };
@@ -377,9 +380,9 @@ int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) 
     return 0;
   // rows of a chunk lie within 31-bit offsets of its first one
   const int64_t ld = std::max(std::max((int64_t)p.ldq, (int64_t)p.ldk), (int64_t)p.ldv);
-  const int64_t chunks = chunk_bound(p, rows, longest);
+  const int64_t chunks = chunk_bound(p, rows);
   if (chunks > 65535 || p.nseq > 65535 || p.H > 65535 || ld * kC * 4 > INT32_MAX ||
-      !chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunks, longest))
+      !chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), std::min(chunks, p.nseq * ((longest + kC - 1) / kC)), longest))
     return 0;
   const int64_t floats = chunks * p.H * (p.beta ? kUnitT + kC * kC : kUnitT);
   return floats <= (int64_t{1} << 28) ? floats : 0;  // a gigabyte: 128k rows of 16 heads; the token walk needs no workspace
@@ -390,7 +393,7 @@ int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) 
 extern "C" hipError_t dsse_scan_chunks(const dsse::MatrixScanParams* p, float* ws, int rows, int64_t longest, hipStream_t st) {
   if (p->nseq <= 0 || p->H <= 0 || rows <= 0) return hipSuccess;
   if (p->H % p->G || !dsse::scan_chunk_floats(*p, rows, longest)) return hipErrorInvalidValue;
-  const int chunks = (int)dsse::chunk_bound(*p, rows, longest);
+  const int chunks = (int)dsse::chunk_bound(*p, rows);
 #define DSSE_CHUNK_CASE(n)                                                            \
   case 16 * n:                                                                        \
     return p->beta ? dsse::launch_chunks<n, true>(*p, ws, chunks, st) : dsse::launch_chunks<n, false>(*p, ws, chunks, st);

@@ -63,3 +63,24 @@ def test_chunks_match_the_walk(H, G, D, V, mode, ql, cont):
     got = scan_state_plain(st).cpu()
     assert (got - st_ref).abs().max() <= tol * st_ref.abs().max()
     assert torch.equal(got[0], state0[0]) and not o[outside.cuda()].any()   # other slots and rows
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_the_longest_length_only_chooses_the_form(delta):
+    """Sequences that are longer than the caller says: the workspace has room for all their chunks."""
+    g = torch.Generator().manual_seed(11)
+    ql, H, D, V = [300, 7, 449], 2, 64, 32
+    T, qs = sum(ql), [0, 300, 307]
+    q, k, v = (torch.randn(T, H, w, generator=g) * D ** -0.5 for w in (D, D, V))
+    decay, beta = torch.rand(T, H, generator=g) ** 0.2, torch.rand(T, H, generator=g) if delta else None
+    state0 = torch.randn(3, H, D, V, generator=g)
+    st_ref, o_ref = state0.clone(), torch.zeros(T, H, V)
+    meta = (i32(qs), i32(ql), i32([m + 1 for m in ql]), i32([2, 0, 1]))
+    lref.matrix_scan(q, k, v, decay, beta, st_ref, *meta, o_ref)
+    c = lambda t: None if t is None else t.cuda()  # noqa: E731
+    for longest in (200, 449, T):
+        st, o = scan_state_from_plain(c(state0)), torch.zeros(T, H, V, device="cuda")
+        ops.matrix_scan(c(q), c(k), c(v), c(decay), c(beta), st, *map(c, meta), o, 1.0, longest)
+        tol = 2 * (D + 64) * 2.0 ** -24   # as above
+        assert (o.cpu() - o_ref).abs().max() <= tol * o_ref.abs().max()
+        assert (scan_state_plain(st).cpu() - st_ref).abs().max() <= tol * st_ref.abs().max()
