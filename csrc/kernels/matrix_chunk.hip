@@ -20,8 +20,9 @@
 // written values and their scaled copy go from one product to the next without a change of layout; they meet between the four
 // waves (16 tokens and D / 4 state rows each) in LDS.  The next chunk's operands are in registers a whole chunk ahead.
 //
-// A chunk's products run over its later tokens with weights of zero, so a token that is not finite makes the outputs of its
-// whole chunk NaN, where the walk leaves the tokens before it; neither reaches another sequence.
+// A chunk's products run over its later tokens with weights of zero, so a token that is not finite would make the outputs of its
+// whole chunk NaN.  Where an output is not finite, the sequence's columns are walked once more token by token (walk_tokens): such
+// a token reaches the tokens after it and none before it.  The same walk serves sequences that the launch has no chunks for.
 #include <algorithm>
 #include <climits>
 
@@ -193,12 +194,52 @@ struct Chunk {
   float last;  // the product of the chunk's decays
 };
 
+// One wave's walk of a sequence, token by token: 16 value columns of a head, state rows 16 t + 4 g + i of column r in a lane
+template <int NT, bool DELTA>
+DEV void walk_tokens(const MatrixScanParams& p, int h, int64_t row0, int ql, bool fresh, int col, int r, int g, float* to) {
+  const int grp = h / (p.H / p.G);
+  f32x4 S[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[t][i] = fresh ? 0.0f : to[(16 * t + 4 * g + i) * kScanCols];
+  for (int64_t row = row0; row < row0 + ql; ++row) {
+    const float* k = p.k + row * p.ldk + grp * p.D + 4 * g;
+    const float* q = p.q + row * p.ldq + grp * p.D + 4 * g;
+    const float a = p.decay_kind == 1 ? p.decay[h] : (p.decay_kind == 2 ? p.decay[row * p.ldd + h] : 1.0f);
+    float u = p.v[row * p.ldv + h * p.V + col], part = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      S[t] = S[t] * a;
+      const f32x4 k4 = ld_global<f32x4>(k + 16 * t);
+      if (DELTA)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part += S[t][i] * k4[i];
+    }
+    if (DELTA) u = p.beta[row * p.ldb + h] * (u - rows4_sum(part));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const f32x4 k4 = ld_global<f32x4>(k + 16 * t), q4 = ld_global<f32x4>(q + 16 * t);
+      S[t] += k4 * u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o += S[t][i] * (q4[i] * p.q_scale);
+    }
+    o = rows4_sum(o);
+    if (g == 0) p.out[(row * p.H + h) * p.V + col] = o;
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) to[(16 * t + 4 * g + i) * kScanCols] = S[t][i];
+}
+
 template <int NT, bool DELTA>
 __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, const float* __restrict__ ws, int chunks) {
   using Ch = Chunk<NT, DELTA>;
   constexpr int kOwn = Ch::kOwn;
   constexpr int kKeyRow = 16 * NT + 4;  // floats of a key row in LDS: rows four apart start 16 banks apart
   __shared__ f32x4 bB[4][64], bU[4][64], bE[4][64], bS[NT][64];
+  __shared__ int votes[4];
   __shared__ __align__(16) float keys[kC * kKeyRow];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   // heads fastest: the column blocks of a head read the same keys, queries and T, M, and land on one XCD's L2 when the heads
@@ -208,11 +249,6 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
   if (ql <= 0) return;  // uniform
   const int first = chunks_before(p.q_len, seq, lane), n = (ql + kC - 1) / kC;
   const int64_t row0 = p.q_start[seq];
-  if (first + n > chunks) {  // uniform.  Only where sequences share rows: no unit was made for this one
-    for (int i = threadIdx.x; i < ql * kScanCols; i += 256)
-      p.out[((row0 + i / kScanCols) * p.H + h) * p.V + cb * kScanCols + i % kScanCols] = __builtin_nanf("");
-    return;
-  }
   constexpr int units = DELTA ? kUnitT + kC * kC : kUnitT;
   const int col = cb * kScanCols + r;
   const bool owner = w * kOwn < NT;  // narrow states have fewer row tiles than waves
@@ -251,12 +287,17 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
   float* to = p.state + p.state_slot[seq] * ((int64_t)p.H * p.D * p.V) + (int64_t)h * p.D * p.V +
               (int64_t)cb * p.D * kScanCols + r;
   const bool fresh = p.ctx_len[seq] - ql == 0;
+  if (first + n > chunks) {  // uniform: sequences longer than the caller said, or sharing rows; no units were made for this one
+    if (w == 0) walk_tokens<NT, DELTA>(p, h, row0, ql, fresh, col, r, g, to);
+    return;
+  }
   f32x4 S[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) S[t][i] = fresh ? 0.0f : to[(16 * t + 4 * g + i) * kScanCols];
 
+  float odd = 0.0f;  // NaN once an output is not finite
   auto walk = [&](int c, const Ch& x, Ch& next) {
     request(c + 1, next);  // in flight across this chunk
     // the chunk's key rows: the state's update reads them by columns
@@ -308,7 +349,10 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
       for (int t = 0; t < 4; ++t) o[t] = mfma_f32(x.m[t][i], bU[t][lane][i], o[t]);
     f32x4 res = total(o);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) res[i] += x.a[i] * (ps[i] * p.q_scale);
+    for (int i = 0; i < 4; ++i) {
+      res[i] += x.a[i] * (ps[i] * p.q_scale);
+      odd += res[i] * 0.0f;
+    }
     if (owner) {
       f32x4 s[kOwn];
 #pragma unroll
@@ -344,6 +388,14 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
     walk(c, x, y);
     if (c + 1 < n) walk(c + 1, y, x);  // uniform
   }
+  const bool mine = __any(odd != 0.0f);
+  if (lane == 0) votes[w] = mine;
+  lds_barrier();
+  if (votes[0] | votes[1] | votes[2] | votes[3]) {  // uniform for the workgroup
+    __syncthreads();                                // every wave's outputs are written
+    if (w == 0) walk_tokens<NT, DELTA>(p, h, row0, ql, fresh, col, r, g, to);
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     if (t / kOwn == w)  // uniform
@@ -370,8 +422,10 @@ static bool chunks_pay(const MatrixScanParams& p, int64_t rows, int64_t chunks, 
   return walk > (p.beta ? 30 + std::max(6.4 * n, 1.26 * chunks * work) : 18 + std::max(4.4 * n, 0.82 * chunks * work));
 }
 
-// chunks of `rows` rows at most, whatever their sequences' lengths: the launch's workgroups find theirs by the lengths
-static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows) { return rows / kC + p.nseq; }
+// chunks of `rows` rows at most: the launch's workgroups find theirs by the lengths
+static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows, int64_t longest) {
+  return std::min(rows / kC + p.nseq, p.nseq * ((longest + kC - 1) / kC));
+}
 
 int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) {
   auto aligned = [](const float* x, int ld) { return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ld % 4 == 0; };
@@ -380,9 +434,9 @@ int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) 
     return 0;
   // rows of a chunk lie within 31-bit offsets of its first one
   const int64_t ld = std::max(std::max((int64_t)p.ldq, (int64_t)p.ldk), (int64_t)p.ldv);
-  const int64_t chunks = chunk_bound(p, rows);
+  const int64_t chunks = chunk_bound(p, rows, longest);
   if (chunks > 65535 || p.nseq > 65535 || p.H > 65535 || ld * kC * 4 > INT32_MAX ||
-      !chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), std::min(chunks, p.nseq * ((longest + kC - 1) / kC)), longest))
+      !chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunks, longest))
     return 0;
   const int64_t floats = chunks * p.H * (p.beta ? kUnitT + kC * kC : kUnitT);
   return floats <= (int64_t{1} << 28) ? floats : 0;  // a gigabyte: 128k rows of 16 heads; the token walk needs no workspace
@@ -393,7 +447,7 @@ int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) 
 extern "C" hipError_t dsse_scan_chunks(const dsse::MatrixScanParams* p, float* ws, int rows, int64_t longest, hipStream_t st) {
   if (p->nseq <= 0 || p->H <= 0 || rows <= 0) return hipSuccess;
   if (p->H % p->G || !dsse::scan_chunk_floats(*p, rows, longest)) return hipErrorInvalidValue;
-  const int chunks = (int)dsse::chunk_bound(*p, rows);
+  const int chunks = (int)dsse::chunk_bound(*p, rows, longest);
 #define DSSE_CHUNK_CASE(n)                                                            \
   case 16 * n:                                                                        \
     return p->beta ? dsse::launch_chunks<n, true>(*p, ws, chunks, st) : dsse::launch_chunks<n, false>(*p, ws, chunks, st);

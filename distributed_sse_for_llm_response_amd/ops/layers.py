@@ -282,8 +282,8 @@ def matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot
     """Matrix-state recurrence per (sequence, head) continued from the slot state [slots, H, D, V] (fp32; zeros at
     position 0): S = a S; u = beta (v - S^T k) with beta (the delta rule), else u = v; S += k u^T; o = S^T (q_scale q).
     decay: None, [H], [T, H] or [T, H, D]; q, k [T, G, D], v [T, H, V] are fp32 (column slices are fine).  `longest`:
-    rows of the longest sequence where the caller knows them (it chooses the form and nothing else); long sequences then
-    go by chunks of tokens.  Sequences share no rows."""
+    rows of the longest sequence where the caller knows them (it chooses the form, results do not depend on it);
+    long sequences then go by chunks of tokens."""
     if _hip(v):
         torch.ops.dsse.matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale,
                                    longest)

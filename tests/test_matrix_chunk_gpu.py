@@ -67,7 +67,7 @@ def test_chunks_match_the_walk(H, G, D, V, mode, ql, cont):
 
 @pytest.mark.parametrize("delta", [False, True])
 def test_the_longest_length_only_chooses_the_form(delta):
-    """Sequences that are longer than the caller says: the workspace has room for all their chunks."""
+    """Sequences that are longer than the caller says: those that the workspace has no room for are walked."""
     g = torch.Generator().manual_seed(11)
     ql, H, D, V = [300, 7, 449], 2, 64, 32
     T, qs = sum(ql), [0, 300, 307]
@@ -78,9 +78,42 @@ def test_the_longest_length_only_chooses_the_form(delta):
     meta = (i32(qs), i32(ql), i32([m + 1 for m in ql]), i32([2, 0, 1]))
     lref.matrix_scan(q, k, v, decay, beta, st_ref, *meta, o_ref)
     c = lambda t: None if t is None else t.cuda()  # noqa: E731
-    for longest in (200, 449, T):
+    for longest in (200, 300, 449, T):
         st, o = scan_state_from_plain(c(state0)), torch.zeros(T, H, V, device="cuda")
         ops.matrix_scan(c(q), c(k), c(v), c(decay), c(beta), st, *map(c, meta), o, 1.0, longest)
         tol = 2 * (D + 64) * 2.0 ** -24   # as above
         assert (o.cpu() - o_ref).abs().max() <= tol * o_ref.abs().max()
         assert (scan_state_plain(st).cpu() - st_ref).abs().max() <= tol * st_ref.abs().max()
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("what", ["q", "k", "v", "inf", "decay", "beta"])
+@pytest.mark.parametrize("at", [0, 5, 17, 63, 64, 100])
+def test_tokens_before_one_that_is_not_finite(delta, what, at):
+    """What a token that is not finite reaches is what the walk lets it reach: later tokens (of one value column, of a head
+    group, or its own output alone), never an earlier one."""
+    if what == "beta" and not delta:
+        return
+    g = torch.Generator().manual_seed(at)
+    ql, H, G, D, V = [130, 70], 4, 2, 64, 32
+    T, qs = sum(ql), [0, 130]
+    q, k, v = (torch.randn(T, h, w, generator=g) * D ** -0.5 for h, w in ((G, D), (G, D), (H, V)))
+    decay, beta = 0.5 + 0.5 * torch.rand(T, H, generator=g), torch.rand(T, H, generator=g) if delta else None
+    if what in ("q", "k"):
+        {"q": q, "k": k}[what][at, 1, 3] = float("nan")
+    elif what in ("v", "inf"):
+        v[at, 1, 9] = float("nan" if what == "v" else "inf")
+    else:
+        {"decay": decay, "beta": beta}[what][at, 2] = float("nan")
+    state0 = torch.randn(2, H, D, V, generator=g)
+    st_ref, o_ref = state0.clone(), torch.zeros(T, H, V)
+    meta = (i32(qs), i32(ql), i32([m + 1 for m in ql]), i32([1, 0]))
+    lref.matrix_scan(q, k, v, decay, beta, st_ref, *meta, o_ref)
+    c = lambda t: None if t is None else t.cuda()  # noqa: E731
+    st, o = scan_state_from_plain(c(state0)), torch.zeros(T, H, V, device="cuda")
+    ops.matrix_scan(c(q), c(k), c(v), c(decay), c(beta), st, *map(c, meta), o, 1.0, T)
+    tol = 2 * (D + 64) * 2.0 ** -24   # as above
+    for got, ref in ((o.cpu(), o_ref), (scan_state_plain(st).cpu(), st_ref)):
+        fine = torch.isfinite(ref)
+        assert torch.equal(torch.isfinite(got), fine)
+        assert (got - ref)[fine].abs().max() <= tol * ref[fine].abs().max()
