@@ -412,14 +412,27 @@ hipError_t launch_chunks(const MatrixScanParams& p, float* ws, int chunks, hipSt
 
 }  // namespace
 
-// Time in us of the walk by tokens and of the chunks, fitted over 1..128 sequences of 16..4096 rows, 16 heads, key and value
-// width 128 (128 column blocks a sequence): each is a start, then its longest chain or the work of all, whichever is more.  One
-// sequence, walk against chunks: delta rule 64 rows 31 / 38, 128 rows 57 / 43, 2048 rows 946 / 221; without 32 rows 17 / 20,
-// 64 rows 28 / 25, 2048 rows 919 / 150.  128 sequences of 32 rows: 108 / 177 and 104 / 118.
+// Time in us of the walk by tokens and of the chunks: each is a start, then its longest chain or the work of all its column blocks,
+// whichever is more.  Fitted per key width over 1..128 sequences of 16..4096 rows of 2..1024 column blocks (both within 11 % rms);
+// of 864 timings the slower of the two is taken by more than 6 % in seven, by 9 % at most.  Walk against
+// chunks, H x D x V: delta rule, 16 x 128 x 128, one sequence of 64 rows 31 / 38, 128 rows 56 / 44, 2048 rows 995 / 217, 128 of 32
+// rows 388 / 531; 32 x 64 x 64, 64 of 64 rows 223 / 290 (one chunk each: the delta rule's start is not made up for); without it,
+// 16 x 128 x 128, 64 rows 28 / 22, 2048 rows 913 / 146, 128 of 32 rows 360 / 491; 16 x 32 x 64, 64 of 64 rows 76 / 62.
+struct ScanCost {
+  double walk0, row, row_block, chunk0, chunk, chunk_block, seq_block;
+};
 static bool chunks_pay(const MatrixScanParams& p, int64_t rows, int64_t chunks, int64_t longest) {
-  const double work = p.H * (p.V / kScanCols) / 128.0, n = (double)((longest + kC - 1) / kC);
-  const double walk = 4 + std::max(0.46 * longest, 0.026 * rows * work);
-  return walk > (p.beta ? 30 + std::max(6.4 * n, 1.26 * chunks * work) : 18 + std::max(4.4 * n, 0.82 * chunks * work));
+  static const ScanCost kDelta[3] = {{5.3, 0.269, 0.044, 24.2, 2.53, 1.93, 0.42},   // widths 32, 64, 128
+                                     {5.5, 0.301, 0.061, 25.8, 3.33, 2.22, 1.17},
+                                     {5.5, 0.425, 0.118, 29.9, 5.24, 3.54, 1.17}};
+  static const ScanCost kPlain[3] = {{5.4, 0.233, 0.039, 12.1, 1.84, 1.11, 0.46},
+                                     {5.4, 0.270, 0.051, 13.7, 2.38, 1.34, 0.44},
+                                     {5.2, 0.380, 0.107, 17.0, 4.03, 2.23, 1.18}};
+  if (p.beta && longest <= kC) return false;
+  const ScanCost& c = (p.beta ? kDelta : kPlain)[p.D == 32 ? 0 : (p.D == 64 ? 1 : 2)];
+  const double blocks = (double)p.H * (p.V / kScanCols) / 128.0, n = (double)((longest + kC - 1) / kC);
+  const double walk = c.walk0 + std::max(c.row * longest, c.row_block * rows * blocks);
+  return walk > c.chunk0 + std::max(c.chunk * n, (c.chunk_block * chunks + c.seq_block * p.nseq) * blocks);
 }
 
 // chunks of `rows` rows at most: the launch's workgroups find theirs by the lengths
