@@ -124,6 +124,10 @@ struct MatrixScanParams {
 // `longest` only chooses the form and the room: sequences that it leaves no room for are walked.
 int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest);
 
+// Whether such rows are better walked in two levels (matrix_scan_chunked) than by either form of matrix_scan: the one decision
+// between the three.  Reads the shapes, strides and alignment of q, k and v.
+bool scan_two_levels(const MatrixScanParams& p, int rows, int64_t longest);
+
 // The carry between the two passes of the two-level walk: per sequence, the incoming state of each of its chunks.
 struct ScanCarryParams {
   float* scratch;        // [chunks, H, D, V]: in: a chunk's end state from zeros; out: the chunk's incoming state

@@ -367,6 +367,16 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
 }
 
+bool matrix_scan_two_levels(const Tensor& q, const Tensor& k, const Tensor& v, bool channels, int64_t rows, int64_t nseq,
+                            int64_t longest) {
+  dsse::MatrixScanParams p{};
+  p.H = (int)v.size(1), p.V = (int)v.size(2), p.G = (int)k.size(1), p.D = (int)k.size(2), p.nseq = (int)nseq;
+  p.q = q.data_ptr<float>(), p.k = k.data_ptr<float>(), p.v = v.data_ptr<float>();
+  p.ldq = (int)q.stride(0), p.ldk = (int)k.stride(0), p.ldv = (int)v.stride(0);
+  p.decay_kind = channels ? 3 : 1;
+  return dsse::scan_two_levels(p, (int)rows, longest);
+}
+
 // Two-level walk of long prompt portions without the delta rule: (1) every chunk but a sequence's last is walked from
 // zeros and leaves its end state in `scratch`; (2) the carry turns those into each chunk's incoming state; (3) every
 // chunk is walked from its incoming state and writes its outputs, the last chunk of a sequence also the slot's state.
@@ -818,12 +828,17 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
         "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
+  m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest) -> bool");
   m.def("matrix_scan_chunked(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor(a!) state, Tensor q_len, Tensor ctx_len, "
         "Tensor state_slot, Tensor s_first, Tensor s_count, Tensor cmeta, Tensor(b!) scratch, Tensor(c!)? a_scratch, "
         "Tensor(d!) out, float q_scale=1.0) -> ()");
   m.def("gated_head_norm(Tensor o, Tensor? w, Tensor gate, float eps, Tensor(a!) out, int kind=0) -> ()");
   m.def("rms_mix(Tensor ya, Tensor wa, Tensor yb, Tensor wb, float eps, float coef, Tensor(a!) out) -> ()");
   m.def("logit_cap(Tensor(a!) logits, float scale, float cap) -> ()");
+}
+
+TORCH_LIBRARY_IMPL(dsse, CompositeExplicitAutograd, m) {
+  m.impl("matrix_scan_two_levels", &matrix_scan_two_levels);  // looks at shapes and addresses only
 }
 
 TORCH_LIBRARY_IMPL(dsse, CUDA, m) {

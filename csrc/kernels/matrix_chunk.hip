@@ -32,6 +32,7 @@ namespace dsse {
 namespace {
 
 constexpr int kC = 64;         // tokens per chunk
+constexpr int kTwoLevelRows = 256;  // rows of a launch from which the two-level walk pays
 constexpr int kScanCols = 16;  // value columns per workgroup: a tile of the state entry (matrix_scan.hip)
 
 DEV f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -440,7 +441,8 @@ static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows, int64_t long
   return std::min(rows / kC + p.nseq, p.nseq * ((longest + kC - 1) / kC));
 }
 
-int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) {
+// Whether the chunks take the shape, and their workspace floats
+static int64_t chunk_room(const MatrixScanParams& p, int rows, int64_t longest) {
   auto aligned = [](const float* x, int ld) { return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ld % 4 == 0; };
   if (longest <= 0 || p.nseq <= 0 || p.src_idx || p.decay_kind > 2 || (p.D != 32 && p.D != 64 && p.D != 128) ||
       p.V % kScanCols || !aligned(p.q, p.ldq) || !aligned(p.k, p.ldk))
@@ -448,11 +450,26 @@ int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) 
   // rows of a chunk lie within 31-bit offsets of its first one
   const int64_t ld = std::max(std::max((int64_t)p.ldq, (int64_t)p.ldk), (int64_t)p.ldv);
   const int64_t chunks = chunk_bound(p, rows, longest);
-  if (chunks > 65535 || p.nseq > 65535 || p.H > 65535 || ld * kC * 4 > INT32_MAX ||
-      !chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunks, longest))
-    return 0;
+  if (chunks > 65535 || p.nseq > 65535 || p.H > 65535 || ld * kC * 4 > INT32_MAX) return 0;
   const int64_t floats = chunks * p.H * (p.beta ? kUnitT + kC * kC : kUnitT);
   return floats <= (int64_t{1} << 28) ? floats : 0;  // a gigabyte: 128k rows of 16 heads; the token walk needs no workspace
+}
+
+int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) {
+  const int64_t floats = chunk_room(p, rows, longest);
+  if (!floats) return 0;
+  return chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunk_bound(p, rows, longest), longest) ? floats : 0;
+}
+
+// Without the delta rule.  Where the chunks are out of the question (decays per key channel, other widths, unaligned rows) two
+// levels beat one long chain; where they are not, only for a long sequence of a few column blocks, whose chunks follow one
+// another on a mostly empty chip.  Chunks against two levels: 2 heads of 128 x 128, 700 rows 59 / 66, 1000 rows 77 / 72; 2 heads of
+// 64 x 64, 1000 rows 49 / 57, 2048 rows 84 / 74; 2 of 32 x 16, 2048 rows 66 / 68, 4096 rows 120 / 98; 16 x 64 x 64, 4096 rows 170 / 257.
+bool scan_two_levels(const MatrixScanParams& p, int rows, int64_t longest) {
+  if (p.beta || rows < kTwoLevelRows) return false;
+  if (!chunk_room(p, rows, longest)) return true;
+  const int64_t from = p.D == 128 ? 900 : (p.D == 64 ? 1500 : 2500);
+  return longest >= from && (int64_t)p.nseq * p.H * (p.V / kScanCols) <= 16;
 }
 
 }  // namespace dsse

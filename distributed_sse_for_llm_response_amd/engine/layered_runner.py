@@ -508,9 +508,9 @@ class LayeredRunner(RunnerBase):
         """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection."""
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
-            D, chan = k.shape[2], decay is not None and decay.dim() == 3
-            if beta is None and "ck" in g and not ops.scan_chunks_form(D, V, chan):
-                s_first, s_count, cm = g["ck"]
+            D, chan, seqs = k.shape[2], decay is not None and decay.dim() == 3, g.get("seqs")  # seqs: prompt portions
+            if beta is None and seqs and ops.matrix_scan_two_levels(q, k, v, chan, g["rows"][1], len(seqs[0]), g["longest"]):
+                s_first, s_count, cm = self._scan_lists(g)
                 scr = self._scratch(d, "scan_s", cm.shape[1] * H * D * V)
                 ascr = self._scratch(d, "scan_a", cm.shape[1] * H * D) if chan else None
                 ops.matrix_scan_chunked(q, k, v, decay, self.state.state[ri], g["qs"], g["ql"], g["ctx"], g["ss"],
@@ -521,6 +521,18 @@ class LayeredRunner(RunnerBase):
         ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw_norm, gate, self.cfg.eps, ao)
         self._lin(ao, o_w, o_t, y)
+
+    def _scan_lists(self, g: dict):
+        """Chunk lists of the two-level walk over a group's portions, made by the first layer that takes it."""
+        if "ck" not in g:
+            s_first, s_count, rows = ops.layers.scan_chunks(*g["seqs"])
+            ck = torch.tensor([s_first, s_count], dtype=torch.int32)
+            cm = torch.tensor(rows, dtype=torch.int32)
+            if self.device.type == "cuda":
+                ck = ck.pin_memory().to(self.device, non_blocking=True)
+                cm = cm.pin_memory().to(self.device, non_blocking=True)
+            g["ck"] = (ck[0], ck[1], cm)
+        return g["ck"]
 
     def _delta(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
         H, G, D, V = m.heads, m.kv_heads, m.dim, m.vdim
@@ -1449,14 +1461,7 @@ class LayeredRunner(RunnerBase):
         d["qt"] = ATTN_ROWS_TILE
         d["rows"] = (row0, T)   # the packed rows of these portions
         d["longest"] = max(ql)
-        if self.prenorm and T >= ops.layers.SCAN_CHUNKED_FROM:  # long portions: the recurrences' two-level walk
-            s_first, s_count, rows = ops.layers.scan_chunks(qs, ql, ss)
-            ck = torch.tensor([s_first, s_count], dtype=torch.int32)
-            cm = torch.tensor(rows, dtype=torch.int32)
-            if self.device.type == "cuda":
-                ck = ck.pin_memory().to(self.device, non_blocking=True)
-                cm = cm.pin_memory().to(self.device, non_blocking=True)
-            d["ck"] = (ck[0], ck[1], cm)
+        d["seqs"] = (qs, ql, ss)
         return T, qs, ql, d
 
     def prefill(self, seqs: list, ring_row: int, trace: list | None = None) -> None:

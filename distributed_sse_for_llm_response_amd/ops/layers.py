@@ -309,13 +309,12 @@ def scan_state_from_plain(plain):
 
 
 SCAN_CHUNK = 64        # tokens per chunk of the two-level walk
-SCAN_CHUNKED_FROM = 256  # rows of a prompt group from which matrix_scan_chunked pays
 
 
-def scan_chunks_form(dim: int, vdim: int, per_channel: bool) -> bool:
-    """Whether matrix_scan takes long sequences of this state by chunks: it does for decays that do not differ between
-    key channels (matrix_scan_chunked walks the others in two levels)."""
-    return not per_channel and dim in (32, 64, 128) and vdim % 16 == 0
+def matrix_scan_two_levels(q, k, v, per_channel: bool, rows: int, nseq: int, longest: int) -> bool:
+    """Whether nseq sequences of `rows` rows together, `longest` in the longest, without the delta rule are better walked in
+    two levels (matrix_scan_chunked) than by matrix_scan: the kernels' own answer, by shapes, row pitches and alignment."""
+    return _hip(v) and torch.ops.dsse.matrix_scan_two_levels(q, k, v, per_channel, rows, nseq, longest)
 
 
 def scan_chunks(q_start: list, q_len: list, slots: list):
