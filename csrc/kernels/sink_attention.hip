@@ -22,7 +22,7 @@
 // 64 (one key per lane for the scores, then one output coordinate per lane and 64 broadcast weights for the values),
 // keep their own running (max, sum, output) and are merged through LDS.  Exact-mode prompt portions whose widths fit take
 // sink_exact.hip instead.
-#include "api_mixers.h"
+#include "sink_rows.h"
 
 namespace dsse {
 namespace {
@@ -30,34 +30,6 @@ namespace {
 constexpr int kMaxV = 512;
 constexpr int kMaxParts = 16;  // stretches a decode walk may be split into
 constexpr int kAccs = kMaxV / 64;
-
-// q (LDS, fp32) . key row (global): 16-byte loads when the row width allows
-DEV float dot_row(const float* q, const bf16* k, int D) {
-  float s = 0.f;
-  int d = 0;
-  if (D % 8 == 0) {
-    for (; d < D; d += 8) {
-      const bf16x8 kv = *reinterpret_cast<const bf16x8*>(k + d);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += q[d + e] * (float)kv[e];
-    }
-  }
-  for (; d < D; ++d) s += q[d] * (float)k[d];
-  return s;
-}
-DEV float dot_row(const float* q, const float* k, int D) {
-  float s = 0.f;
-  int d = 0;
-  if (D % 4 == 0) {
-    for (; d < D; d += 4) {
-      const f32x4 kv = *reinterpret_cast<const f32x4*>(k + d);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s += q[d + e] * kv[e];
-    }
-  }
-  for (; d < D; ++d) s += q[d] * k[d];
-  return s;
-}
 
 template <typename T>
 __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnParams p) {
@@ -68,22 +40,13 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnParams p) {
   const int seq = p.work_seq[work], tile = p.work_tile[work];
   const int ql = p.q_len[seq];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = h / (p.H / p.G);
   const int D = p.D, V = p.V;
-  const int* bt = p.block_tables + (int64_t)seq * p.max_blocks;
-  const T* kc = reinterpret_cast<const T*>(p.k);
-  const T* vc = reinterpret_cast<const T*>(p.v);
   const float sink = p.sink ? p.sink[h] : -INFINITY;
   for (int i = 0; i < p.qt; ++i) {
     const int off = tile * p.qt + i;
     if (off >= ql) break;  // uniform for the workgroup
     const int row = p.q_start[seq] + off;
     const int pos = p.ctx_len[seq] - ql + off;
-    const int lo = pos - p.window + 1 > 0 ? pos - p.window + 1 : 0;
-    const int kept = p.keep_first < lo ? p.keep_first : lo;  // keys 0 .. kept - 1 are walked ahead of the window's
-    const int nkeys = kept + pos - lo + 1;
-    const int last_rel = p.rel_len - 1;
-    const float* rel = p.rel ? p.rel + (int64_t)h * p.rel_len : nullptr;
     __syncthreads();  // the previous row's merge has read qs / acc_s
     for (int d = threadIdx.x; d < D; d += blockDim.x) qs[d] = p.q[((int64_t)row * p.H + h) * D + d];
     __syncthreads();
@@ -91,36 +54,7 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnParams p) {
     float acc[kAccs];
 #pragma unroll
     for (int a = 0; a < kAccs; ++a) acc[a] = 0.f;
-    for (int c = wave; c * 64 < nkeys; c += 4) {
-      const int jj = c * 64 + lane;
-      const bool on = jj < nkeys;
-      const int j0 = on ? jj : 0;
-      const int j = j0 < kept ? j0 : lo + j0 - kept;
-      int page = bt[j / kBS];
-      page = (unsigned)page < (unsigned)p.num_blocks ? page : 0;
-      const int krow = (page * kBS + j % kBS) * p.G + g;
-      const float s_dot = dot_row(qs, kc + (int64_t)krow * D, D);
-      float s = s_dot * p.scale;
-      if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
-      if (rel) s += rel[pos - j < last_rel ? pos - j : last_rel];
-      s = on ? s : -INFINITY;
-      const float m_new = fmaxf(m, wave_max(s));  // finite: the chunk holds at least one key
-      const float w = on ? expf(s - m_new) : 0.f;
-      const float f = expf(m - m_new);            // 0 when m was -inf
-      l = l * f + wave_sum(w);
-      m = m_new;
-#pragma unroll
-      for (int a = 0; a < kAccs; ++a) acc[a] *= f;
-      const int cnt = nkeys - c * 64 < 64 ? nkeys - c * 64 : 64;
-      for (int t = 0; t < cnt; ++t) {
-        const float wt = __shfl(w, t);
-        const int vrow = __shfl(krow, t);
-        const T* vp = vc + (int64_t)vrow * V;
-#pragma unroll
-        for (int a = 0; a < kAccs; ++a)
-          if (a * 64 + lane < V) acc[a] += wt * (float)vp[a * 64 + lane];
-      }
-    }
+    walk_row<T>(p, seq, h, pos, qs, wave, 4, m, l, acc);
     if (lane == 0) {
       m_s[wave] = m;
       l_s[wave] = l;

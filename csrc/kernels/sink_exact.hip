@@ -11,10 +11,14 @@
 // so an output's error against 64 bits is no larger: 400 rows of 16 heads of 128 2.0e-7 (row kernel 3.3e-7), 64 rows
 // behind 2000 keys 3.1e-7 (5.7e-7).
 //
+// A page's values meet all 16 rows of a tile, with weights of zero for keys that a row does not see: later tokens, keys behind
+// the window, places of the page that hold nothing yet (or what an earlier sequence left).  Where such a value is not finite the
+// row would be NaN, so a wave whose outputs are not all finite makes its rows once more one by one, from the keys they see.
+//
 // What bounds it: a page costs a wave 2 x 64 v_mfma_f32_16x16x4_f32 at widths of 128, 4096 cycles.  The row kernel (four waves
 // walk one row's keys, a load per key and value) took 371 us for 400 rows of 16 heads of 128; here 56; 1000 rows 1460
 // us and 130; 8 rows of each of 16 sequences behind 50 keys 97 and 14.
-#include "api_mixers.h"
+#include "sink_rows.h"
 
 namespace dsse {
 namespace {
@@ -22,6 +26,29 @@ namespace {
 constexpr int kExactTiles = 4;  // column tiles (waves) of a workgroup
 
 DEV f32x4 mma_exact(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// One row by one wave
+DEV void exact_row(const SinkAttnParams& p, int seq, int h, int64_t row, int pos) {
+  const int lane = threadIdx.x & 63;
+  float m = -INFINITY, l = 0.f, acc[2] = {0.f, 0.f};  // V <= 128
+  walk_row<float>(p, seq, h, pos, p.q + (row * p.H + h) * p.D, 0, 1, m, l, acc);
+  float f = 1.0f;
+  if (p.sink) {
+    const float sk = p.sink[h], mm = fmaxf(m, sk);
+    f = expf(m - mm);
+    l = l * f + expf(sk - mm);
+  }
+  float gate = 1.0f;
+  if (p.gate && !p.gate_wide) gate = 1.0f / (1.0f + expf(-p.gate[row * p.ldg + h]));
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int d = 64 * a + lane;
+    if (d >= p.V) continue;
+    float o = acc[a] * f / l * gate;
+    if (p.gate_wide) o *= 1.0f / (1.0f + expf(-p.gate[row * p.ldg + h * p.V + d]));
+    reinterpret_cast<float*>(p.out)[row * p.ldo + h * p.V + d] = o * p.out_scale;
+  }
+}
 
 // NT = V / 16; KT = D / 16 when it equals NT, else 0: read from the parameters
 template <int NT, int KT>
@@ -166,25 +193,30 @@ __global__ __launch_bounds__(64 * kExactTiles) void sink_exact_kernel(SinkAttnPa
         for (int n = 0; n < NT; ++n)
           O[n] = mma_exact(vals[(16 * h + 4 * g + i) * ldv + 16 * n + r], w[4 * h + i], O[n]);
   }
-  if (!on) return;
-  float den = l, f = 1.0f;
-  if (p.sink) {
-    const float sk = p.sink[head], mm = fmaxf(m, sk);
-    f = expf(m - mm);
-    den = l * f + expf(sk - mm);
-  }
-  float gate = 1.0f;
-  if (p.gate && !p.gate_wide) gate = 1.0f / (1.0f + expf(-p.gate[row * p.ldg + head]));
-  const float* gw = p.gate_wide ? p.gate + row * p.ldg + head * V + 4 * g : nullptr;
-  float* out = reinterpret_cast<float*>(p.out) + row * p.ldo + head * V + 4 * g;
-#pragma unroll
-  for (int n = 0; n < NT; ++n)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float o = (all[n][i] + O[n][i]) * f / den * gate;
-      if (gw) o *= 1.0f / (1.0f + expf(-gw[16 * n + i]));
-      out[16 * n + i] = o * p.out_scale;
+  float odd = 0.0f;  // NaN once an output is not finite
+  if (on) {
+    float den = l, f = 1.0f;
+    if (p.sink) {
+      const float sk = p.sink[head], mm = fmaxf(m, sk);
+      f = expf(m - mm);
+      den = l * f + expf(sk - mm);
     }
+    float gate = 1.0f;
+    if (p.gate && !p.gate_wide) gate = 1.0f / (1.0f + expf(-p.gate[row * p.ldg + head]));
+    const float* gw = p.gate_wide ? p.gate + row * p.ldg + head * V + 4 * g : nullptr;
+    float* out = reinterpret_cast<float*>(p.out) + row * p.ldo + head * V + 4 * g;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float o = (all[n][i] + O[n][i]) * f / den * gate;
+        if (gw) o *= 1.0f / (1.0f + expf(-gw[16 * n + i]));
+        out[16 * n + i] = o * p.out_scale;
+        odd += o * 0.0f;
+      }
+  }
+  if (!__any(odd != 0.0f)) return;
+  for (int i = 0; i < 16 && tile_first + i < ql; ++i) exact_row(p, seq, head, q0 + tile_first + i, pos0 + tile_first + i);
 }
 
 template <int NT>

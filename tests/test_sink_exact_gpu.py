@@ -48,3 +48,41 @@ def test_prompt_portions(H, G, D, V, window, keep, rel_len, cap, gates):
     # scores: sums of D products, D 2^-24 of |q||k| scale < 10 each, times a factor e^s; outputs: 600 weights.  Both sides round.
     assert (got.cpu() - want).abs().max() <= 2 * (10 * D + 600) * 2.0 ** -24 * vc.abs().max()
     assert (wide[:, :2] == 9.0).all() and (wide[:, 2 + H * V:] == 9.0).all()
+
+
+@pytest.mark.parametrize("H,G,D,V,window,keep", [(4, 2, 64, 64, 1 << 30, 0), (4, 1, 128, 96, 40, 3), (2, 2, 16, 128, 20, 0)])
+@pytest.mark.parametrize("bad", ["nan", "inf"])
+def test_values_that_a_row_does_not_see(H, G, D, V, window, keep, bad):
+    """Values that are not finite where a row sees nothing -- later tokens, keys behind the window, places past the context that
+    an earlier owner of the page left -- do not reach it; where it sees them they do."""
+    ql, start = [50, 9, 33], [0, 31, 100]
+    g = torch.Generator().manual_seed(D + V)
+    n, T = len(ql), sum(ql)
+    need = [-(-(a + b) // PAGE) for a, b in zip(ql, start)]
+    bt, k = torch.zeros(n, max(need), dtype=torch.int32), 0
+    for s, m in enumerate(need):
+        bt[s, :m], k = torch.arange(k, k + m, dtype=torch.int32), k + m
+    q = torch.randn(T, H, D, generator=g)
+    kc, vc = (torch.randn(sum(need), PAGE, G, w, generator=g) for w in (D, V))
+
+    def place(s, j):
+        return int(bt[s, j // PAGE]), j % PAGE
+
+    vc[place(0, 20) + (0, 5)] = float(bad)       # rows 20 .. of the first sequence see it, until the window has passed
+    vc[place(2, 10) + (G - 1, V - 1)] = float(bad)  # behind the window of some cases
+    for s in range(n):                            # the rest of the last pages
+        for j in range(ql[s] + start[s], need[s] * PAGE):
+            kc[place(s, j)] = vc[place(s, j)] = float(bad)
+    meta = (i32([sum(ql[:s]) for s in range(n)]), i32(ql), i32([a + b for a, b in zip(ql, start)]))
+    rows = ops.sink_tile_rows(torch.float32, H, G, D, V)
+    items = [(s, t) for s in range(n) for t in range(-(-ql[s] // rows))]
+    sink, gate = torch.randn(H, generator=g), torch.randn(T, H, generator=g)
+    want = torch.zeros(T, H, V)
+    lref.sink_attention(q, kc, vc, bt, *meta, sink, gate, want, window, D ** -0.5, keep_first=keep)
+    c = lambda t: t.cuda()  # noqa: E731
+    got = torch.zeros(T, H, V, device="cuda")
+    ops.sink_attention(c(q), c(kc), c(vc), c(bt), *map(c, meta), c(i32([s for s, _ in items])), c(i32([t for _, t in items])),
+                       c(sink), c(gate), got, window, D ** -0.5, rows, keep_first=keep)
+    fine = torch.isfinite(want)
+    assert fine.any() and not fine.all() and torch.equal(torch.isfinite(got.cpu()), fine)
+    assert (got.cpu() - want)[fine].abs().max() <= 2 * (10 * D + 600) * 2.0 ** -24 * 5   # as above; |v| < 5
