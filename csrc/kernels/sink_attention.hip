@@ -21,7 +21,8 @@
 // Row kernel (any sizes, both element types): a workgroup serves `qt` query rows of one head; for each row its four waves split the keys in chunks of
 // 64 (one key per lane for the scores, then one output coordinate per lane and 64 broadcast weights for the values),
 // keep their own running (max, sum, output) and are merged through LDS.  Exact-mode prompt portions whose widths fit take
-// sink_exact.hip instead.
+// sink_exact.hip instead: a position's result does not depend on how the prompt was cut there either, but a decode row's sums are
+// ordered differently (equal within fp32 rounding).
 #include "sink_rows.h"
 
 namespace dsse {

@@ -122,8 +122,10 @@ __global__ __launch_bounds__(64 * kExactTiles) void sink_exact_kernel(SinkAttnPa
     }
   };
   // outputs: sums over kSumPages pages, joined in `all`: one chain over a long walk would round more than the row kernel's
-  // four waves with a part of the keys each
+  // four waves with a part of the keys each.  The groups are pages of the sequence, not of the walk, and a page that a row does
+  // not see adds exactly nothing to it: a row's result is the same however its prompt was cut into portions.
   constexpr int kSumPages = 4;
+  int group = -1;
   f32x4 O[NT], all[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) O[n] = all[n] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -181,7 +183,8 @@ __global__ __launch_bounds__(64 * kExactTiles) void sink_exact_kernel(SinkAttnPa
 #pragma unroll
       for (int n = 0; n < NT; ++n) O[n] = O[n] * corr, all[n] = all[n] * corr;
     }
-    if (it % kSumPages == 0) {  // uniform
+    if (pg / kSumPages != group) {  // uniform
+      group = pg / kSumPages;
 #pragma unroll
       for (int n = 0; n < NT; ++n) all[n] += O[n], O[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }

@@ -86,3 +86,28 @@ def test_values_that_a_row_does_not_see(H, G, D, V, window, keep, bad):
     fine = torch.isfinite(want)
     assert fine.any() and not fine.all() and torch.equal(torch.isfinite(got.cpu()), fine)
     assert (got.cpu() - want)[fine].abs().max() <= 2 * (10 * D + 600) * 2.0 ** -24 * 5   # as above; |v| < 5
+
+
+@pytest.mark.parametrize("H,G,D,V,window,keep,rel_len", [(4, 2, 128, 128, 1 << 30, 0, 0), (4, 1, 64, 64, 70, 40, 9), (2, 2, 32, 48, 200, 0, 0)])
+def test_rows_do_not_depend_on_the_cut(H, G, D, V, window, keep, rel_len):
+    """The same rows bit for bit, whatever portions their prompt comes in: sums are grouped by pages of the sequence."""
+    T = 420
+    g = torch.Generator().manual_seed(D)
+    pages = -(-T // PAGE)
+    bt = torch.randperm(pages, generator=g).to(torch.int32)[None].cuda()
+    q = torch.randn(T, H, D, generator=g).cuda()
+    kc, vc = (torch.randn(pages, PAGE, G, w, generator=g).cuda() for w in (D, V))
+    sink = torch.randn(H, generator=g).cuda()
+    rel = torch.randn(H, rel_len, generator=g).cuda() if rel_len else None
+    rows = ops.sink_tile_rows(torch.float32, H, G, D, V)
+    outs = []
+    for cut in ([T], [1, 37, 130, 2, 64, 186], [33] * 12 + [24]):
+        out, at = torch.zeros(T, H, V, device="cuda"), 0
+        for n in cut:
+            items = range(-(-n // rows))
+            meta = (i32([0]), i32([n]), i32([at + n]), i32([0] * len(items)), i32(list(items)))
+            ops.sink_attention(q[at:at + n], kc, vc, bt, *(t.cuda() for t in meta), sink, None, out[at:at + n], window,
+                               D ** -0.5, rows, keep_first=keep, rel=rel)
+            at += n
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
