@@ -151,10 +151,11 @@ __global__ __launch_bounds__(64 * WS * WS * KG) void gemm_rm_lds_kernel(GemmRmPa
 #pragma unroll
   for (int t = 0; t < kStages - 1; ++t) issue(t);
   for (int t = 0; t < steps; ++t) {
-    // this wave's part of step t has landed (those of the two younger steps may be in flight), then everybody's
+    // this wave's part of step t has landed (those of the two younger steps may be in flight) and its fragments of step t - 1
+    // are in registers, then everybody's
     static_assert(kStages == 4 && (kPer == 4 || kPer == 8), "the waits below");
-    if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+    if constexpr (kPer == 4) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     issue(t + kStages - 1);
     const char* buf = smem + ((t % kStages) * KG + kg) * kSlot;
     typename Frag<T>::V a[2][2], b[2][2];
