@@ -307,10 +307,13 @@ hipError_t dispatch(const GemmRmParams& p, hipStream_t st) {
   if (lds_ok<T>(p)) {
     // 64 x 64 tiles while they fill the CUs; two wave groups per tile when there is one tile per CU at most (nothing else
     // would run while a wave waits for its fragments: 400 rows of 2048 x 2048 in fp32 45.4 -> 42.2 us); 32 x 32 tiles, four
-    // groups each, while those make at most two (fp32, bound by the matrix rate) or one (bf16, bound by LDS traffic)
-    // rounds: 64 rows of 2048 x 8192 in fp32 157 -> 50 us, 400 rows of 576 x 4096 in bf16 19 -> 11 us
+    // groups each, while those make one round (64 rows of 2048 x 8192 in fp32 157 -> 50 us, 400 rows of 576 x 4096 in bf16
+    // 19 -> 11 us).  A second round of them pays in fp32 (bound by the matrix rate) where the groups have four chunks each;
+    // with fewer, filling and joining them is most of the time: mean of 256..512 tiles against the kernel above, 64 x 64 / 32 x
+    // 32 tiles, 1 chunk 0.84 / 1.39, 4 chunks 0.70 / 0.92, 8 chunks 0.60 / 0.69, 16 chunks 0.52 / 0.52.
     const int chunks = (int)(p.K * sizeof(T) / 128);
-    if (lds_tiles(p, 32) * p.batch <= (sizeof(T) == 4 ? 512 : 256)) return launch_lds<T, 1, 4>(p, st);
+    const int64_t small = lds_tiles(p, 32) * p.batch;
+    if (chunks >= 2 && small <= (sizeof(T) == 4 && chunks >= 16 ? 512 : 256)) return launch_lds<T, 1, 4>(p, st);
     if (lds_tiles(p, 64) * p.batch <= 256 && chunks >= 8) return launch_lds<T, 2, 2>(p, st);
     // one or two chunks and many rows: the store is all there is to wait for (3000 rows of 512 x 128, 32 slices: 68 us here,
     // 76 us through LDS)
