@@ -56,7 +56,7 @@ def test_stream_rows(M, W, dtype):
         near(out, want, 2 * steps)
 
 
-@pytest.mark.parametrize("T,nh,D", [(1, 1, 6), (5, 3, 64), (2, 16, 128), (3, 37, 32), (513, 5, 128)])
+@pytest.mark.parametrize("T,nh,D", [(1, 1, 6), (5, 3, 64), (2, 16, 128), (3, 37, 32), (513, 5, 128), (700, 37, 32), (1500, 19, 6), (3001, 41, 6)])
 @pytest.mark.parametrize("kind", [0, 1, 2, 3])
 def test_heads_over_workgroups_and_waves(T, nh, D, kind):
     g = torch.Generator().manual_seed(nh + D)
