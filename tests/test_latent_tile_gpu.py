@@ -19,6 +19,14 @@ def gpu():
     return torch.device("cuda", 0)
 
 
+def near(out, ref):
+    """Every (row, head) by itself: a wrong column, key or window edge is one of them.  Query vectors, weights and results are
+    rounded to bf16 (2^-9 each at most); a rounded query moves a score by some 2^-9 |q||k| / sqrt(D) of it, which the softmax
+    passes on: 2^-6 bounds the three together.  One wrong key of n changes a row by some n^-1/2: 2 % of 2100 keys."""
+    diff, size = (out.cpu().double() - ref.double()).norm(dim=-1), ref.double().norm(dim=-1)
+    assert float((diff / size).max()) <= 2.0 ** -6
+
+
 # heads that fill eight column tiles exactly, leave some empty, need a second workgroup and are single columns; portions that
 # start inside a page, of one row, and behind more than 64 pages; windows of one key, of a page and its neighbours
 @pytest.mark.parametrize("H,rk,window", [(32, 512, 10 ** 6), (16, 512, 33), (9, 512, 1), (5, 256, 10 ** 6), (40, 256, 32),
@@ -54,7 +62,4 @@ def test_prompt_portions(gpu, H, rk, window):
     out = torch.full((T, H, rk), float("nan"), dtype=torch.bfloat16, device=gpu)
     ops.latent_attention(q.to(gpu), q_abs.to(gpu), cache.to(gpu), bt.to(gpu), *(m.to(gpu) for m in meta), rope.to(gpu), out,
                          window, scale, rows, vt.to(gpu), 16 // rows)
-    # query vectors, weights and results are rounded to bf16 (2^-9 each at most); a rounded query moves a score by some
-    # 2^-9 |q||k| / sqrt(D) of it, which the softmax passes on: 2^-6 bounds the three together
-    err = (out.cpu().double() - ref.double()).norm() / ref.double().norm()
-    assert float(err) <= 2.0 ** -6
+    near(out, ref)
