@@ -158,7 +158,8 @@ class LayeredRunner(RunnerBase):
         self.use_graphs = (self.device.type == "cuda") if use_graphs is None else use_graphs
         cfg, dev = self.cfg, self.device
         self._init_slots(max_batch, self.max_blocks, cfg.vocab_size, dev, self.comm)
-        self._tile_rows = []   # row counts of the shared-page attention forms' work items that this design's layers use
+        self._tile_rows = []   # row counts of the shared-page sink attention's work items that this design's layers use
+        self._latents = set()  # (heads, rank, rotated width) of the latent attentions on the MFMA form
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
         self.multistream = getattr(cfg, "family", "") == "dironex"  # pre-norm blocks on several residual streams
@@ -194,7 +195,7 @@ class LayeredRunner(RunnerBase):
             key = (m.rot, m.rot_dim)
             if key not in self._rope:
                 self._rope[key] = m.rot.table(self.max_model_len + 1, m.rot_dim, dev)
-        self._tile_rows = sorted({ops.latent_tile_rows(att[i].heads, att[i].kv_rank, att[i].rot_dim) for i in flash})
+        self._latents = {(att[i].heads, att[i].kv_rank, att[i].rot_dim) for i in flash}
         words = max((ops.latent_flash_part_floats(max_batch, m.heads, 16, 16, m.kv_rank) for i, m in att.items()
                      if i in flash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -321,7 +322,7 @@ class LayeredRunner(RunnerBase):
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope,
                                          lat, m.window, m.scale, 1, vt, 16, self._flash_part if np_ > 1 else None, np_)
                 else:
-                    rows = ops.latent_tile_rows(H, rk, dr)
+                    rows = ops.latent_tile_rows(H, rk, dr, g["keys"], g["rows"][1])
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], *g["tiles"][rows], rope,
                                          lat, m.window, m.scale, rows, vt, 16 // rows)
             else:
@@ -634,9 +635,8 @@ class LayeredRunner(RunnerBase):
         self.kv = MixedKVCache({r: m.kv_rank + m.rot_dim for r, m in lat.items()}, kv, self.num_blocks, dev, self.dtype,
                                latent_transposed=lflash, kv_transposed=kflash)
         self.state = ConvTailCache(tails, self.max_batch, dev)
-        tiles = {ops.latent_tile_rows(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash}
-        self._tile_rows = sorted(tiles | set(self._sink_tile_rows(
-            [cfg.layers[r.layer].mixer for r in self.runs if r.index in kv])))
+        self._latents = {(lat[r].heads, lat[r].kv_rank, lat[r].rot_dim) for r in lflash}
+        self._tile_rows = self._sink_tile_rows([cfg.layers[r.layer].mixer for r in self.runs if r.index in kv])
         words = max((ops.latent_flash_part_floats(self.max_batch, m.heads, 16, 16, m.kv_rank) for r, m in lat.items()
                      if r in lflash), default=0)
         self._flash_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
@@ -761,7 +761,7 @@ class LayeredRunner(RunnerBase):
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope,
                                          lat, m.window, m.scale, 1, vt, 16, self._flash_part if np_ > 1 else None, np_)
                 else:
-                    rows = ops.latent_tile_rows(H, rk, dr)
+                    rows = ops.latent_tile_rows(H, rk, dr, g["keys"], g["rows"][1])
                     ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], *g["tiles"][rows], rope,
                                          lat, m.window, m.scale, rows, vt, 16 // rows)
             else:
@@ -1439,7 +1439,8 @@ class LayeredRunner(RunnerBase):
             row += m
         T = row
         shared = []  # work items of the shared-page attention forms: the longest walks first
-        for R in self._tile_rows:
+        tile_rows = sorted(set(self._tile_rows) | {ops.latent_tile_rows(*a, max(ctx), T) for a in self._latents})
+        for R in tile_rows:
             items = [(i, t) for i, s in enumerate(seqs) for t in range(math.ceil(len(s.tokens) / R))]
             items.sort(key=lambda it: -(seqs[it[0]].start_pos + it[1] * R))
             shared += [("tile_seq", R, [i for i, _ in items]), ("tile_no", R, [t for _, t in items])]
@@ -1456,11 +1457,11 @@ class LayeredRunner(RunnerBase):
             d[name], o = meta[o:o + k], o + k
         for name, R, xs in shared:
             d.setdefault(name, {})[R], o = meta[o:o + len(xs)], o + len(xs)
-        d["tiles"] = {R: (d["tile_seq"][R], d["tile_no"][R]) for R in self._tile_rows}
+        d["tiles"] = {R: (d["tile_seq"][R], d["tile_no"][R]) for R in tile_rows}
         d["bt"] = bt
         d["qt"] = ATTN_ROWS_TILE
         d["rows"] = (row0, T)   # the packed rows of these portions
-        d["longest"] = max(ql)
+        d["longest"], d["keys"] = max(ql), max(ctx)
         d["seqs"] = (qs, ql, ss)
         return T, qs, ql, d
 

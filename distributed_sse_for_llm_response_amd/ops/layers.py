@@ -56,14 +56,19 @@ def latent_kv_write(ckr, norm_w, positions, slots, rope, cache, eps: float, vt=N
         lref.latent_kv_write(ckr, norm_w, positions, slots, rope, cache, eps, vt)
 
 
-def latent_tile_rows(heads: int, rk: int, dr: int) -> int:
-    """Query rows per work item of latent_attention's MFMA form in prompt portions, with 16 // rows heads in an item's 16
+def latent_tile_rows(heads: int, rk: int, dr: int, longest: int = 1 << 30, rows: int = 1 << 30) -> int:
+    """Query rows per work item of latent_attention's MFMA form in prompt portions, with 16 // result heads in an item's 16
     columns: the fewest rows whose items fill at least half of the eight column tiles that share a page (latent_tile.hip), or
-    four where that form does not apply."""
+    four where that form does not apply.  Where no key is further than the second page (`longest`: the longest context) and the
+    step's `rows` leave CUs empty, the one-wave form with as many heads side by side as there are: filling eight column tiles
+    takes longer than the walk (one prompt of 16 tokens, 32 heads of rank 512: 25 us, 15 here; 64 tokens 28 and 20; 16 heads
+    27.8 and 16.6; 16 prompts of 33 tokens, 16896 pairs of a row and a head: 31 and 40)."""
     if dr == 64 and rk in (128, 256, 512):
-        for rows in (4, 8, 16):
-            if -(-heads // (16 // rows)) >= (6 if rows < 16 else 4):
-                return rows
+        if longest <= 64 and rows * heads <= 16384:
+            return 1 if heads > 8 else (2 if heads > 4 else 4)
+        for tile in (4, 8, 16):
+            if -(-heads // (16 // tile)) >= (6 if tile < 16 else 4):
+                return tile
     return 4
 
 

@@ -32,9 +32,21 @@ def near(out, ref):
 @pytest.mark.parametrize("H,rk,window", [(32, 512, 10 ** 6), (16, 512, 33), (9, 512, 1), (5, 256, 10 ** 6), (40, 256, 32),
                                          (24, 128, 31), (64, 128, 10 ** 6), (16, 128, 2050)])
 def test_prompt_portions(gpu, H, rk, window):
+    portions(gpu, H, rk, window, [(0, 70), (31, 1), (64, 33), (2100, 19), (5, 3)], ops.latent_tile_rows(H, rk, 64))
+
+
+@pytest.mark.parametrize("H,rk,rows", [(33, 512, 1), (16, 128, 1), (9, 256, 1), (8, 256, 2), (5, 128, 2), (4, 128, 4), (1, 512, 4)])
+def test_short_prompts(gpu, H, rk, rows):
+    """No key further than the second page and few rows: the one-wave form, as many heads side by side as there are."""
+    seqs = [(0, 64), (31, 1), (32, 32), (5, 3), (0, 9)]
+    assert ops.latent_tile_rows(H, rk, 64, 64, 109) == rows
+    assert ops.latent_tile_rows(H, rk, 64, 65, 109) == ops.latent_tile_rows(H, rk, 64, 64, 16384 // H + 1) \
+        == ops.latent_tile_rows(H, rk, 64)
+    portions(gpu, H, rk, 10 ** 6, seqs, rows)
+
+
+def portions(gpu, H, rk, window, seqs, rows):
     dn, dr = 24, 64
-    seqs = [(0, 70), (31, 1), (64, 33), (2100, 19), (5, 3)]
-    rows = ops.latent_tile_rows(H, rk, dr)
     g = torch.Generator().manual_seed(H + rk)
     pages = [-(-(s + n) // 32) for s, n in seqs]
     bt = torch.zeros(len(seqs), max(pages), dtype=torch.int32)
