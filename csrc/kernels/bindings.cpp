@@ -335,24 +335,35 @@ TCfg pipe_plan(int M, int N, int K, bool slab_consumer) {
 
 constexpr int kModelMinM = 256;  // above this many rows every N % 256 == 0 projection is planned by pipe_plan
 
-// N % 256 == 128 on gemm_pipe: its last column block is half empty, and short or narrow products are better cut into the
-// 128-column tiles of gemm_tiled.  Measured, gemm_tiled against gemm_pipe in us (rows x N x K): 320 x 5248 x 2048 21 / 25,
-// 800 x 3200 x 2048 26 / 28, 512 x 1664 x 4096 26 / 26; 1500 x 1152 x 2048 34 / 27, 800 x 5248 x 2048 37 / 31, 257 x 8320 x
-// 2048 44 / 25, 257 x 2176 x 4096 33 / 24, 800 x 1152 x 4096 44 / 27, 2048 x 26752 x 4096 509 / 386.
-bool half_block_pays(int M, int N, int K) {
+// N % 256 == 128 on gemm_pipe, planned as `c`: its last column block is half empty, and short or narrow products are better cut
+// into the 128-column tiles of gemm_tiled.  Measured, gemm_tiled against gemm_pipe in us (rows x N x K): 320 x 5248 x 2048
+// 21 / 25, 800 x 3200 x 2048 26 / 28, 512 x 1664 x 4096 26 / 26; 1500 x 1152 x 2048 34 / 27, 800 x 5248 x 2048 37 / 31, 257 x
+// 8320 x 2048 44 / 25, 257 x 2176 x 4096 33 / 24, 800 x 1152 x 4096 44 / 27, 2048 x 26752 x 4096 509 / 386.  Two kinds of larger
+// products stay there as well: reductions of up to 512 that fill one round of 256 x 128 tiles (1800 x 3200 x 512 17.0 / 18.3), and
+// those that the plan cuts into slices of up to 2048 combined in the launch, which take some 1.17 of their estimate where the
+// rounds of gemm_tiled's tiles fit (1500 x 26752 x 4096 361 / 380, 700 x 26752 x 8192 389 / 427, 6000 x 3200 x 8192 371 / 432; its
+// time over 572 such shapes to 5 % rms: rounds of 256 tiles, a partial one at 0.82 + 0.18 x its fill, 15.2 ns per element of K).
+bool half_block_pays(int M, int N, int K, const TCfg& c) {
   const int64_t weight = (int64_t)N * K;
-  if (K >= 4096) return M > 512 || N >= 2048;
-  return M > 1024 || weight >= (1 << 24) || (M > 512 && weight >= (1 << 23));
+  if (!(K >= 4096 ? M > 512 || N >= 2048 : M > 1024 || weight >= (1 << 24) || (M > 512 && weight >= (1 << 23)))) return false;
+  const int64_t tiles = (int64_t)((M + 255) / 256) * (N / 128), rem = tiles % 256;
+  if (K <= 512 && tiles > 192 && tiles <= 256) return false;
+  if (c.fix && c.cfg == 8 && K / c.S <= 2048) {
+    const double round = 4.5 + 0.01523 * K;
+    const double tiled = 3.9 + round * (double)(tiles / 256) + (rem ? round * (0.823 + 0.177 * rem / 256.0) : 0.0);
+    return 1.17 * c.est_us <= tiled;
+  }
+  return true;
 }
 
 TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
   TCfg c{};
   int cfg = env_int("t_cfg", -1);
   const bool forced = cfg == 0 || cfg == 1 || cfg == 5 || cfg == 8 || cfg == 9 || cfg == 10;
-  if (!forced && env_int("t_model", 1) && N % 128 == 0 && K % 128 == 0 && M > kModelMinM &&
-      (N % 256 == 0 || half_block_pays(M, N, K))) {
+  if (!forced && env_int("t_model", 1) && N % 128 == 0 && K % 128 == 0 && M > kModelMinM) {
     c = pipe_plan(M, N, K, slab_consumer);
-    if (c.ok) return c;
+    if (c.ok && (N % 256 == 0 || half_block_pays(M, N, K, c))) return c;
+    c = TCfg{};
   }
   if (!forced) {
     // up to kModelMinM rows (and N % 256 != 0): the decode buckets' measured table
