@@ -249,7 +249,7 @@ class LayeredRunner(RunnerBase):
             d.update(self._joint_buffers(M, new))
             return d
         if self.bracket:
-            d.update(self._memory_buffers(M, new) if self.memory else self._bracket_buffers(M))
+            d.update(self._memory_buffers(M) if self.memory else self._bracket_buffers(M))
             return d
         if self.multistream:
             d.update(self._stream_buffers(M))
@@ -1077,7 +1077,7 @@ class LayeredRunner(RunnerBase):
         self._walk_part = torch.zeros(max(1, words), device=dev, dtype=torch.float32)
         self._moe_layers = [i for i, L in enumerate(cfg.layers) if hasattr(L.mlp, "experts") and L.weights_of == i]
 
-    def _memory_buffers(self, M: int, new) -> dict:
+    def _memory_buffers(self, M: int) -> dict:
         """Scratch of a step of M rows, each sized for the widest layer: `big` the fused projection's fp32 output, `qa`
         the attention's queries, `ao` a mixer's gated heads in the element type (both halves of a twin layer side by
         side), `mm` the matrix memory's work area (prompt-sized steps), `up` / `h` the dense feed-forward's hidden row,
