@@ -159,6 +159,7 @@ class LayeredRunner(RunnerBase):
         cfg, dev = self.cfg, self.device
         self._init_slots(max_batch, self.max_blocks, cfg.vocab_size, dev, self.comm)
         self._tile_rows = []   # row counts of the shared-page sink attention's work items that this design's layers use
+        self._channel_decays = False  # some layer's recurrence decays per key channel
         self._latents = set()  # (heads, rank, rotated width) of the latent attentions on the MFMA form
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
@@ -205,6 +206,7 @@ class LayeredRunner(RunnerBase):
         with the same weights and has its own pages and state slots each time."""
         cfg, dev = self.cfg, self.device
         self.runs = cfg.runs()
+        self._channel_decays = any(L.kind == "parallel" for L in cfg.layers)
         kv, st, self._rope = {}, {}, {}
         for r in self.runs:
             L, m = cfg.layers[r.layer], cfg.layers[r.layer].mixer
@@ -1463,6 +1465,8 @@ class LayeredRunner(RunnerBase):
         d["rows"] = (row0, T)   # the packed rows of these portions
         d["longest"], d["keys"] = max(ql), max(ctx)
         d["seqs"] = (qs, ql, ss)
+        if self._channel_decays and T >= 4 * ops.layers.SCAN_CHUNK:
+            self._scan_lists(d)  # surely asked for: with the other lists, before the step's first launch
         return T, qs, ql, d
 
     def prefill(self, seqs: list, ring_row: int, trace: list | None = None) -> None:
