@@ -14,6 +14,9 @@
 //     o    = A (Q S) + M u,    M[t][i] = R[t][i] q_t . k_i  for i <= t
 //     S'   = A_C S + K^T (E u),  E_i = R[C - 1][i]
 //
+// (the chunkwise form of the delta rule: Yang et al., "Parallelizing Linear Transformers with the Delta Rule over Sequence
+// Length", 2024)
+//
 // Two launches: T, M, A and E depend on the inputs alone and are made for all chunks at once; the second walks the chunks of
 // a (sequence, head, 16 value columns).  All products are v_mfma_f32_16x16x4_f32, 32-bit like the walk.  The accumulator
 // layout (rows 4 g + i of column r) IS the B operand of a product whose k index runs 4 g + i over i, so the state, the

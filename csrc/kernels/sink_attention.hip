@@ -438,7 +438,7 @@ constexpr int kTileLdv = kBS + 8;
 
 // The sums are scaled by a maximum that may lag behind the scores by this much (log2 units): weights stay below 2^8, which
 // fp32 sums and bf16 weights hold as exactly as weights below one, and pages that raise no row's maximum by more need no
-// rescaling and no exchange between lanes.
+// rescaling and no exchange between lanes (the conditional rescaling published with FlashAttention-4).
 constexpr float kLazyMax = 8.0f;
 
 DEV bf16x8 ld_buffer(__amdgpu_buffer_rsrc_t r, uint32_t off) {
