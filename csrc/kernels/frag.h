@@ -35,7 +35,7 @@ DEV typename Frag<T>::V load_frag(const T* row, int k, int K, bool valid, bool v
 DEV f32x4 mma(const bf16x8& a, const bf16x8& b, f32x4 c) { return mfma16x16x32(a, b, c); }
 DEV f32x4 mma(const f32x4& a, const f32x4& b, f32x4 c) {
 #pragma unroll
-  for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
+  for (int s = 0; s < 4; ++s) c = mfma16x16x4(a[s], b[s], c);
   return c;
 }
 

@@ -36,6 +36,7 @@
 //   * epilogues: bf16 store staged through LDS (16-byte row stores), SiLU·mul, fp32 / residual / QKV+RoPE /
 //     split-K partial slabs through gemm_epilogue.h.
 #include "gemm_epilogue.h"
+#include "lds_dma.h"
 
 #ifndef DSSE_PIPE_STAMPS
 #define DSSE_PIPE_STAMPS 0
@@ -58,17 +59,6 @@ constexpr int kA = 256 * 128;     // A image of one K step: 256 rows x 64 bf16, 
 constexpr int kB = 16 * 2048;     // B image: 16 column tiles x two 1 KiB k-step blocks
 constexpr int kBuf = kA + kB;     // 64 KiB per K step
 constexpr size_t kLDS = 2 * (size_t)kBuf;
-constexpr uint32_t kOOB = 0x80000000u;  // buffer offset past every range: the load returns zeros, no traffic
-
-typedef __attribute__((address_space(3))) void* lds_t;
-
-DEV void dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, 0);
-}
-
-// A-image swizzle (as gemm_tiled.hip a_swz): piece q of LDS row `row` holds piece q ^ swz(row) of the X row;
-// conflict-free ds_read_b128 for the A-fragment pattern (lane (r, g) reads row r, piece 2g + s).
-DEV int a_swz(int row) { return (row >> 1) & 5; }
 
 }  // namespace gp
 
@@ -129,7 +119,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       const int rb = (j >> 3) * 128 + q * 64 + (j & 7) * 8;        // first of its 8 rows
       const int row = rb + (lane >> 3), sr = (j & 7) * 8 + (lane >> 3);  // LDS slot row, slot row in the quadrant
       const int xrow = m0 + (j >> 3) * (BM / 2) + q * QR + sr;          // the X row it holds
-      const int pc = (lane & 7) ^ a_swz(row);
+      const int pc = (lane & 7) ^ piece_swizzle(row);
       a_lo[q][i] = rb * 128;
       a_vo[q][i] = sr < QR && xrow < M ? (uint32_t)(((size_t)xrow * ldx + 32 * (pc >> 1) + 8 * (pc & 1)) * 2) : kOOB;
       const int tb = (j >> 2) * 4 + q * 2 + ((j >> 1) & 1), sub = j & 1;  // column tile of the block, k sub-step
@@ -149,13 +139,13 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     char* base = smem + (t & 1) * kBuf;
     const uint32_t so = __builtin_amdgcn_readfirstlane(a_so(t));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma(xr, base + a_lo[q][i], a_vo[q][i], so);
+    for (int i = 0; i < 2; ++i) lds_dma(xr, base + a_lo[q][i], a_vo[q][i], so);
   };
   auto issue_b = [&](int q, int t) {
     char* base = smem + (t & 1) * kBuf;
     const uint32_t so = __builtin_amdgcn_readfirstlane(b_so(t));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma(wr, base + b_lo[q][i], b_vo[q][i], so);
+    for (int i = 0; i < 2; ++i) lds_dma(wr, base + b_lo[q][i], b_vo[q][i], so);
   };
 
   // ---- fragment reads: A rows wm*128 + 64 qm + 16 i + r (the swizzle is the same for every i), B column tiles
@@ -164,7 +154,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
 #pragma unroll
   for (int sp = 0; sp < 2; ++sp) {
     const int row = wm * 128 + r;
-    a_rd[sp] = row * 128 + (((2 * g + sp) ^ a_swz(row)) << 4);
+    a_rd[sp] = row * 128 + (((2 * g + sp) ^ piece_swizzle(row)) << 4);
   }
   f32x4 acc[8][4];
 #pragma unroll

@@ -11,6 +11,7 @@
 // (lane group, element) pair stands for only has to agree between the A and the B fragment, so both use k0 + PER g + j.
 #include "api_layers.h"
 #include "frag.h"
+#include "lds_dma.h"
 
 namespace dsse {
 namespace {
@@ -91,13 +92,6 @@ __global__ __launch_bounds__(256) void gemm_rm_kernel(GemmRmParams p) {
 // Measured (one MI355X): 400 rows in fp32, 2048 x 2048 205 -> 42 us, 16384 x 2048 330 -> 250 us (108 TFLOP/s), 2048 x 8192
 // 788 -> 148 us; 1000 rows in bf16, 576 x 4096 119 -> 17 us; 3000 rows of 32 slices of 128 x 512 91 -> 39 us.
 constexpr int kStages = 4;
-constexpr uint32_t kOOB = 0x80000000u;
-typedef __attribute__((address_space(3))) void* lds_t;
-
-DEV void rm_dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, 0);
-}
-DEV int rm_swizzle(int row) { return (row >> 1) & 5; }
 
 // WS x WS waves of 32 x 32 outputs make the tile; KG such groups work on alternate chunks of K and meet in LDS.
 template <typename T, int WS, int KG>
@@ -129,19 +123,19 @@ __global__ __launch_bounds__(64 * WS * WS * KG) void gemm_rm_lds_kernel(GemmRmPa
     const int global = (is_x ? m0 : n0) + row;
     if (i % (WS == 1 ? 4 : kPer) == 0)
       src[WS == 1 ? i / 4 : 0] = make_rsrc(is_x ? X : W, (uint32_t)(((size_t)(rows - 1) * ld + p.K) * sizeof(T)));
-    vo[i] = global < rows ? (uint32_t)((size_t)global * ld * sizeof(T)) + 16 * ((lane & 7) ^ rm_swizzle(row)) : kOOB;
+    vo[i] = global < rows ? (uint32_t)((size_t)global * ld * sizeof(T)) + 16 * ((lane & 7) ^ piece_swizzle(row)) : kOOB;
   }
   auto issue = [&](int t) {
     const int c = t * KG + kg;
     char* base = smem + ((t % kStages) * KG + kg) * kSlot + w * kPer * 1024;
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
-      rm_dma(src[WS == 1 ? i / 4 : 0], base + i * 1024, c < nk ? vo[i] : kOOB, (uint32_t)c * 128);
+      lds_dma(src[WS == 1 ? i / 4 : 0], base + i * 1024, c < nk ? vo[i] : kOOB, (uint32_t)c * 128);
   };
   int a_rd[2], b_rd[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    const int piece = ((2 * g + s) ^ rm_swizzle(r)) << 4;
+    const int piece = ((2 * g + s) ^ piece_swizzle(r)) << 4;
     a_rd[s] = (wm * 32 + r) * 128 + piece;
     b_rd[s] = (kTile + wn * 32 + r) * 128 + piece;
   }

@@ -25,6 +25,7 @@
 // Replaces the library GEMMs of round 1's prefill and wide decode path, which needed a second, standard
 // layout copy of every weight (engine/weights.py).
 #include "gemm_epilogue.h"
+#include "lds_dma.h"
 
 namespace dsse {
 
@@ -47,13 +48,6 @@ DEV void glds16(const void* src, char* lds_base) {
                                    16, 0, 0);
 }
 
-
-// A-image swizzle: 16-byte piece q of LDS row `row` holds piece q ^ a_swz(row) of the X row.  Rows r and r+1
-// sit in the two halves of a 256-byte bank row.  A fragment read = lane (r, g) -> row r, piece 2g + s; gfx950
-// serves ds_read_b128 in the lane groups {0-3,12-15,20-27}, {4-11,16-19,28-31} (+32): with (r >> 1) & 5 the
-// 16 lanes of each group hit 16 distinct slots.  (The earlier (r >> 1) & 7 -- conflict-free for groups of 16
-// consecutive lanes -- was 2-way conflicted in every group: SQ_LDS_BANK_CONFLICT 40 % of the LDS cycles.)
-DEV int a_swz(int row) { return (row >> 1) & 5; }
 
 // NS: LDS stages (3: one stage's DMA stays in flight across the publishing barrier; 2: the next stage is issued
 // after the barrier and waited for at the next one).  FB: 2 = both k sub-steps' fragments are read before the
@@ -94,7 +88,7 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
 #pragma unroll
   for (int i = 0; i < G::A_INS; ++i) {
     const int row = (w * G::A_INS + i) * 8 + (lane >> 3);
-    const int p = (lane & 7) ^ a_swz(row);  // X piece p = 2g' + s' -> K offset 32g' + 8s' (+16h per half chunk)
+    const int p = (lane & 7) ^ piece_swizzle(row);  // X piece p = 2g' + s' -> K offset 32g' + 8s' (+16h per half chunk)
     a_src[i] = X + (size_t)min(m0 + row, M - 1) * ldx;
     a_koff[i] = 32 * (p >> 1) + 8 * (p & 1);
   }
@@ -137,7 +131,7 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
   for (int mt = 0; mt < MT; ++mt) {
     const int row = wm * MT * 16 + 16 * mt + r;
 #pragma unroll
-    for (int sp = 0; sp < 2; ++sp) a_off[mt][sp] = row * 128 + (((2 * g + sp) ^ a_swz(row)) << 4);
+    for (int sp = 0; sp < 2; ++sp) a_off[mt][sp] = row * 128 + (((2 * g + sp) ^ piece_swizzle(row)) << 4);
   }
 
   constexpr int INS = G::A_INS + G::B_INS;

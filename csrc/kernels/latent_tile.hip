@@ -20,17 +20,12 @@
 // TFLOP/s), 4096 tokens 4178 -> 756 us (773 TFLOP/s); 16 heads, 1024 tokens 267 -> 101 us; rank 128, 2000 tokens 243 -> 94 us.
 // Filling the page's 69 KB takes a CU longer than its products (about 1.5 us against 1), which is what is left.
 #include "api_layers.h"
+#include "lds_dma.h"
 
 namespace dsse {
 namespace {
 namespace lt {
 
-typedef __attribute__((address_space(3))) void* lds_t;
-
-DEV void dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(reinterpret_cast<uintptr_t>(lds)), 16, voff, 0, 0, 0);
-}
-DEV int key_swizzle(int row) { return (row >> 1) & 5; }
 DEV int value_swizzle(int row) { return -(row >> 2) & 3; }
 
 constexpr int kWaves = 8;
@@ -84,7 +79,7 @@ latent_tile_kernel(LatentAttnParams p, const bf16* __restrict__ vt, int rt, int 
 #pragma unroll
   for (int i = 0; i < KI; ++i) {
     const int piece = (i * kWaves + w) * 64 + lane, row = piece / (D / 8), slot = piece - row * (D / 8);
-    k_vo[i] = (uint32_t)(row * D * 2 + (((slot & ~7) | ((slot & 7) ^ key_swizzle(row))) << 4));
+    k_vo[i] = (uint32_t)(row * D * 2 + (((slot & ~7) | ((slot & 7) ^ piece_swizzle(row))) << 4));
   }
 #pragma unroll
   for (int i = 0; i < VI; ++i) {
@@ -99,7 +94,7 @@ latent_tile_kernel(LatentAttnParams p, const bf16* __restrict__ vt, int rt, int 
 #pragma unroll
     for (int j = 0; j < KI; ++j)
       if ((j + 1) * kWaves * 1024 <= kKey || (j * kWaves + w) * 1024 < kKey)  // uniform
-        dma(src, dst + (j * kWaves + w) * 1024, k_vo[j]);
+        lds_dma(src, dst + (j * kWaves + w) * 1024, k_vo[j]);
   };
   auto issue_vals = [&](int i) {
     if ((i & 63) == 0 && i > 0) vid = ids_from(i);
@@ -107,7 +102,7 @@ latent_tile_kernel(LatentAttnParams p, const bf16* __restrict__ vt, int rt, int 
     const __amdgpu_buffer_rsrc_t src = make_rsrc(vt + (int64_t)blk * rk * kBS, (uint32_t)kVal);
     char* dst = vals + (i & 1) * kVal;
 #pragma unroll
-    for (int j = 0; j < VI; ++j) dma(src, dst + (j * kWaves + w) * 1024, v_vo[j]);
+    for (int j = 0; j < VI; ++j) lds_dma(src, dst + (j * kWaves + w) * 1024, v_vo[j]);
   };
   issue_keys(0);
 
@@ -141,7 +136,7 @@ latent_tile_kernel(LatentAttnParams p, const bf16* __restrict__ vt, int rt, int 
   }
   int k_rd[2];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) k_rd[s] = r * D * 2 + (((2 * g + s) ^ key_swizzle(r)) << 4);
+  for (int s = 0; s < 2; ++s) k_rd[s] = r * D * 2 + (((2 * g + s) ^ piece_swizzle(r)) << 4);
   const int v_rd = (w * NW * 16 + r) * kBS * 2 + ((g ^ value_swizzle(r)) << 4);
 
   f32x4 O[NW][kWaves];  // [value tile][column tile]

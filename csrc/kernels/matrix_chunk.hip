@@ -38,8 +38,6 @@ constexpr int kC = 64;         // tokens per chunk
 constexpr int kTwoLevelRows = 256;  // rows of a launch from which the two-level walk pays
 constexpr int kScanCols = 16;  // value columns per workgroup: a tile of the state entry (matrix_scan.hip)
 
-DEV f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 // floats of one (chunk, head): M | A | E | T
 constexpr int kUnitA = kC * kC, kUnitE = kUnitA + kC, kUnitT = kUnitE + kC;
 DEV int64_t unit_floats(bool delta) { return delta ? kUnitT + kC * kC : kUnitT; }
@@ -142,8 +140,8 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(MatrixScanParams p, 
       if (j <= w)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (DELTA) kk[j][t % kSums] = mfma_f32(ka[i], kb[j][i], kk[j][t % kSums]);
-          qk[j][t % kSums] = mfma_f32(qa[i], kb[j][i], qk[j][t % kSums]);
+          if (DELTA) kk[j][t % kSums] = mfma16x16x4(ka[i], kb[j][i], kk[j][t % kSums]);
+          qk[j][t % kSums] = mfma16x16x4(qa[i], kb[j][i], qk[j][t % kSums]);
         }
   }
   __syncthreads();
@@ -318,7 +316,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          W[t % kSums] = mfma_f32(x.k[t][i], S[t][i], W[t % kSums]), P[t % kSums] = mfma_f32(x.q[t][i], S[t][i], P[t % kSums]);
+          W[t % kSums] = mfma16x16x4(x.k[t][i], S[t][i], W[t % kSums]), P[t % kSums] = mfma16x16x4(x.q[t][i], S[t][i], P[t % kSums]);
       const f32x4 ws4 = total(W);
 #pragma unroll
       for (int i = 0; i < 4; ++i) u[i] = x.v[i] - x.a[i] * ws4[i];
@@ -330,7 +328,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
         const f32x4 b = bB[t][lane];
         ut[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ut[t] = mfma_f32(x.t[t][i], b[i], ut[t]);
+        for (int i = 0; i < 4; ++i) ut[t] = mfma16x16x4(x.t[t][i], b[i], ut[t]);
       }
       u = total(ut);
     }
@@ -340,7 +338,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) P[t % kSums] = mfma_f32(x.q[t][i], S[t][i], P[t % kSums]);
+        for (int t = 0; t < NT; ++t) P[t % kSums] = mfma16x16x4(x.q[t][i], S[t][i], P[t % kSums]);
     }
     lds_barrier();
     const f32x4 ps = total(P);
@@ -350,7 +348,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) o[t] = mfma_f32(x.m[t][i], bU[t][lane][i], o[t]);
+      for (int t = 0; t < 4; ++t) o[t] = mfma16x16x4(x.m[t][i], bU[t][lane][i], o[t]);
     f32x4 res = total(o);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -372,7 +370,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, 
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int o = 0; o < kOwn; ++o) s[o] = mfma_f32(keys[(16 * t + 4 * g + i) * kKeyRow + 16 * (w * kOwn + o) + r], b[i], s[o]);
+          for (int o = 0; o < kOwn; ++o) s[o] = mfma16x16x4(keys[(16 * t + 4 * g + i) * kKeyRow + 16 * (w * kOwn + o) + r], b[i], s[o]);
       }
 #pragma unroll
       for (int o = 0; o < kOwn; ++o) bS[w * kOwn + o][lane] = s[o];

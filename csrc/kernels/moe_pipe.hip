@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "lds_dma.h"
 #include "moe_rows.h"
 
 namespace dsse {
@@ -38,14 +39,6 @@ constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 
 constexpr int kBuf = kA + kB;
 constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), then their weights (256 floats)
 constexpr size_t kLDS = kIds + 2 * 256 * 4;
-constexpr uint32_t kOOB = 0x80000000u;  // buffer offset past every range: zeros, no traffic
-
-typedef __attribute__((address_space(3))) void* lds_t;
-
-DEV void dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t)(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, 0);
-}
-DEV int swizzle(int row) { return (row >> 1) & 5; }
 
 struct Place {
   int first;  // the expert's first list tile
@@ -185,28 +178,28 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         int id = -1;
         if (sr < QR) id = s_id[((j >> 3) * 2 + h) * QR + sr];
         a_lo[h][i] = rb * 128;
-        a_vo[h][i] = id >= 0 ? (uint32_t)(((size_t)(MODE == 1 ? id : id / p.S) * ldx + 8 * ((lane & 7) ^ swizzle(row))) * 2)
+        a_vo[h][i] = id >= 0 ? (uint32_t)(((size_t)(MODE == 1 ? id : id / p.S) * ldx + 8 * ((lane & 7) ^ piece_swizzle(row))) * 2)
                              : kOOB;
         const int tb = (j >> 2) * 4 + h * 2 + ((j >> 1) & 1);             // column tile
         const int br = (j & 1) * 8 + (lane >> 3);                         // row inside it
         const int n = MODE == 0 ? n0 + (tb >> 1) * 16 + br : n0 + tb * 16 + br;
         b_lo[h][i] = kA + (tb * 16 + (j & 1) * 8) * 128;
-        b_vo[h][i] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ swizzle(br))) * 2) : kOOB;
+        b_vo[h][i] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ piece_swizzle(br))) * 2) : kOOB;
       }
     auto issue_a = [&](int h, int t) {
       char* base = smem + (t & 1) * kBuf;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma(xr, base + a_lo[h][i], a_vo[h][i], (uint32_t)t * 128);
+      for (int i = 0; i < 2; ++i) lds_dma(xr, base + a_lo[h][i], a_vo[h][i], (uint32_t)t * 128);
     };
     auto issue_b = [&](int h, int t) {
       char* base = smem + (t & 1) * kBuf;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) dma(wr, base + b_lo[h][i], b_vo[h][i], (uint32_t)t * 128);
+      for (int i = 0; i < 2; ++i) lds_dma(wr, base + b_lo[h][i], b_vo[h][i], (uint32_t)t * 128);
     };
     int a_rd[2], b_rd[2];
 #pragma unroll
     for (int sp = 0; sp < 2; ++sp) {
-      const int piece = ((2 * g + sp) ^ swizzle(r)) << 4;
+      const int piece = ((2 * g + sp) ^ piece_swizzle(r)) << 4;
       a_rd[sp] = (wm * 128 + r) * 128 + piece;
       b_rd[sp] = kA + (wn * 64 + r) * 128 + piece;
     }
@@ -246,7 +239,9 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
       __builtin_amdgcn_s_setprio(0);
       asm volatile("s_barrier" ::: "memory");
     };
-    // half-tile order, counted waits and their reasons: gemm_pipe.hip
+    // Half-tiles of two instructions, in the order A0 B0 B1 A1 of a step.  A wait for 8 leaves the four youngest in flight and
+    // has the half-tile that the next phase reads: B1 of step t in phase 0, A1 in phase 1, A0 and B0 of step t + 1 in phase 3,
+    // each followed by the barrier that opens the reading phase.  A slot is refilled two phases or more after its last read.
     issue_a(0, 0);
     issue_b(0, 0);
     issue_b(1, 0);

@@ -25,8 +25,6 @@ namespace {
 
 constexpr int kExactTiles = 4;  // column tiles (waves) of a workgroup
 
-DEV f32x4 mma_exact(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 // One row by one wave
 DEV void exact_row(const SinkAttnParams& p, int seq, int h, int64_t row, int pos) {
   const int lane = threadIdx.x & 63;
@@ -150,7 +148,7 @@ __global__ __launch_bounds__(64 * kExactTiles) void sink_exact_kernel(SinkAttnPa
         if (KT || t < kt) {
           const f32x4 k4 = *reinterpret_cast<const f32x4*>(&keys[(16 * h + r) * ldk + 16 * t + 4 * g]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[i] = mma_exact(k4[i], qf[t][i], s[i]);
+          for (int i = 0; i < 4; ++i) s[i] = mfma16x16x4(k4[i], qf[t][i], s[i]);
         }
       const f32x4 sum = (s[0] + s[1]) + (s[2] + s[3]);
 #pragma unroll
@@ -194,7 +192,7 @@ __global__ __launch_bounds__(64 * kExactTiles) void sink_exact_kernel(SinkAttnPa
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
-          O[n] = mma_exact(vals[(16 * h + 4 * g + i) * ldv + 16 * n + r], w[4 * h + i], O[n]);
+          O[n] = mfma16x16x4(vals[(16 * h + 4 * g + i) * ldv + 16 * n + r], w[4 * h + i], O[n]);
   }
   float odd = 0.0f;  // NaN once an output is not finite
   if (on) {
