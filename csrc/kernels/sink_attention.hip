@@ -566,10 +566,14 @@ __global__ __launch_bounds__(512 / CT, 2) void sink_tile_kernel(SinkAttnParams p
   const float cap_inv = p.softcap > 0.f ? 1.0f / p.softcap : 0.f, cap2 = p.softcap * kLog2e;
   const float scale2 = p.softcap > 0.f ? p.scale : p.scale * kLog2e;
   const int wave_lo = min(tile_lo[0], tile_lo[CT - 1]), wave_hi = max(tile_hi[0], tile_hi[CT - 1]);
+  // the pages that some row of the wave may see.  The workgroup's walk has others, later and behind their window: their values
+  // would be multiplied by zero weights, and one that is not finite would reach rows that do not see it.
+  const int seen_to = __builtin_amdgcn_readfirstlane(wave_hi / kBS), kept_to = (p.keep_first + kBS - 1) / kBS,
+            seen_from = __builtin_amdgcn_readfirstlane(max(wave_lo - p.window + 1, 0) / kBS);
   auto page_step = [&](int it, bf16x8(&rk)[KC], bf16x8(&rv)[VC], const bf16x8(&tk)[KC], const bf16x8(&tv)[VC]) {
     const int pg = page_at(it);
     request(it + 2, rk, rv);
-    if (pg * kBS <= wave_hi) {  // uniform for the wave: some row of it may see this page
+    if (pg <= seen_to && (pg >= seen_from || pg < kept_to)) {  // uniform for the wave
       const bf16* kb = smem + (it & 1) * buf_elems;
       const bf16* vb = kb + kBS * ldk;
       f32x4 s0[CT], s1[CT];

@@ -55,3 +55,35 @@ def test_prompt_portions(H, G, D, V, window, keep, rel_len, many, growth):
                        c(sink), None, got, window, scale, rows, c(vt), keep_first=keep, rel=c(rel))
     # weights and outputs are rounded to bf16 (2^-9 each); scores below 100, so weights differ by exp(100 2^-22) besides
     assert (got.cpu().float() - want).abs().max() <= (2.0 ** -8 + 5e-5) * vc.float().abs().max()
+
+
+# one and two column tiles per wave, with kept first keys and a bias
+@pytest.mark.parametrize("D,V,keep,rel_len", [(128, 128, 0, 0), (64, 48, 0, 0), (64, 64, 40, 9)])
+def test_pages_behind_a_window(D, V, keep, rel_len):
+    """A value that is not finite reaches rows whose 32-row stretch has its page in the window, and no others: the walk of an
+    item of 128 rows starts up to 127 keys ahead of a row's window."""
+    T, H, window, bad = 400, 2, 64, 80
+    g = torch.Generator().manual_seed(D + V)
+    pages = -(-T // PAGE)
+    kc = torch.randn(pages, PAGE, H, D, generator=g).bfloat16().cuda()
+    vt = torch.randn(pages, H, V, PAGE, generator=g).bfloat16().cuda()
+    bt = torch.arange(pages, dtype=torch.int32)[None].cuda()
+    q, sink = torch.randn(T, H, D, generator=g).cuda(), torch.randn(H, generator=g).cuda()
+    rel = torch.randn(H, rel_len, generator=g).cuda() if rel_len else None
+    rows = ops.sink_tile_rows(torch.bfloat16, H, H, D, V)
+    assert rows == 128
+    items = list(range(-(-T // rows)))
+    meta = [t.cuda() for t in (i32([0]), i32([T]), i32([T]), i32([0] * len(items)), i32(items))]
+    outs = []
+    for x in (0.0, float("nan")):
+        vt[bad // PAGE, :, :, lref.vt_position(bad % PAGE)] = x
+        out = torch.zeros(T, H, V, dtype=torch.bfloat16, device="cuda")
+        # the kernel reads values from the transposed pages alone
+        ops.sink_attention(q, kc, torch.zeros(pages, PAGE, H, V, dtype=torch.bfloat16, device="cuda"), bt, *meta, sink, None, out,
+                           window, D ** -0.5, rows, vt, keep_first=keep, rel=rel)
+        outs.append(out.cpu())
+    clean, got = outs
+    far = torch.ones(T, dtype=torch.bool)
+    far[bad // PAGE * PAGE:(bad // PAGE + 1) * PAGE + window] = False   # rows 64 .. 159
+    assert torch.isfinite(clean).all() and torch.equal(got[far], clean[far])
+    assert torch.isnan(got[bad:bad + window].float()).all()
