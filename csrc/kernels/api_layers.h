@@ -162,9 +162,11 @@ struct MoeGroupedParams {
   int f32;
 };
 
-// Shapes that the pipelined expert GEMMs take (moe_pipe.hip): reduction lengths of whole 64-element steps, two at least;
-// 16-byte-aligned operands; every operand inside a 2 GiB buffer range; and enough rows to be worth it.
-bool moe_pipe_ok(const MoeGroupedParams& p);
+// Shapes that the expert GEMMs on LDS-DMA take (moe_pipe.hip, moe_stream.hip): reduction lengths of whole 64-element steps,
+// two at least; 16-byte-aligned operands; every operand inside a 2 GiB buffer range.
+bool moe_lines_ok(const MoeGroupedParams& p);
+// Of those, the ones that read the weights as one stream (moe_stream.hip)
+bool moe_stream_pays(const MoeGroupedParams& p);
 
 // Router, choice and work list of a decode-sized step in one launch.
 struct MoeRouteRowsParams {
@@ -184,6 +186,7 @@ struct MoeRouteRowsParams {
 
 extern "C" {
 hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st);  // the GEMMs alone: the work list is ready
+hipError_t dsse_moe_stream(const dsse::MoeGroupedParams* p, hipStream_t st);  // likewise
 hipError_t dsse_gemm_rm(const dsse::GemmRmParams* p, hipStream_t st);
 hipError_t dsse_scalar_norm(const dsse::ScalarNormParams* p, hipStream_t st);
 // resid = embed[ids] * scale + table[positions] (table fp32 [table_len, W] or null); xb (or null) the same rounded

@@ -9,9 +9,10 @@ namespace {
 // may leave the buffer belongs into it and not into the scalar one.
 constexpr uint32_t kOOB = 0x80000000u;
 
+template <int AUX = 0>
 DEV void lds_dma(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff = 0) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      r, reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, 0);
+      r, reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(lds)), 16, voff, soff, 0, AUX);
 }
 
 // Swizzle of an LDS image of 128-byte rows: piece q of row `row` holds piece q ^ piece_swizzle(row) of the source row.  Rows r

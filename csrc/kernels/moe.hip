@@ -514,7 +514,7 @@ void launch_expert_gemms(const MoeGroupedParams& p, dim3 g1, dim3 g2, hipStream_
   hipLaunchKernelGGL((moe_down_kernel<T, SUBS>), g2, dim3(256), 0, st, p);
 }
 
-// Prompt-sized row counts (bf16, widths multiples of 8) whose shapes the pipelined form (moe_pipe.hip) does not take: the
+// Prompt-sized row counts (bf16, widths multiples of 8) whose shapes the LDS-DMA forms (moe_pipe.hip, moe_stream.hip) do not take: the
 // same two GEMMs with both operands staged through LDS.
 // A workgroup owns a 64-row tile of one expert times 128 weight rows (MODE 0: 64 hidden units' gate rows and the same
 // units' up rows; MODE 1: 128 output columns of the down projection) and walks K in chunks of 64: 256 threads copy the
@@ -682,7 +682,7 @@ extern "C" hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStrea
                        sizeof(int) * (3 * NE + 1), st, *p);
   const int fmax = p->F > p->Fs ? p->F : p->Fs;
   dim3 g1((fmax + 15) / 16, p->max_tiles), g2((p->W + 15) / 16, p->max_tiles);
-  if (dsse::moe_pipe_ok(*p)) return dsse_moe_pipe(p, st);
+  if (dsse::moe_lines_ok(*p)) return dsse::moe_stream_pays(*p) ? dsse_moe_stream(p, st) : dsse_moe_pipe(p, st);
   // other prompt-sized steps in bf16 with rows of whole 16-byte pieces: operands staged through registers and LDS
   if (!p->f32 && p->lds_tiles && p->W % 8 == 0 && p->F % 8 == 0 && p->Fs % 8 == 0 && p->ldh % 8 == 0) {
     dim3 l1((fmax + 63) / 64, p->max_tiles), l2((p->W + 127) / 128, p->max_tiles), l3((fmax + 127) / 128, p->max_tiles);

@@ -23,7 +23,7 @@
 //
 // Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
 // experts, top 2, shared 7168: 2369 -> 1014 us (1042 TFLOP/s); 2048 rows: 1695 -> 775; 1024 rows of 2048 x 1408, shared
-// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Never slower from 256 ids on.
+// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Below 193 rows moe_stream.hip is faster.
 #include <algorithm>
 #include <cmath>
 
@@ -66,7 +66,9 @@ struct List {
 }  // namespace mp
 
 // MODE 0: h = silu(gate x) * (up x); 1: o = weight * down h; 2: h = relu(up x)^2
-template <int MODE>
+// ONCE: most weight panels have one row tile: they are non-temporal, and a column block starts at a K step of its own and wraps
+// around, since rows a power of two apart ask a few memory channels at a time when every workgroup walks K in step
+template <int MODE, bool ONCE>
 __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int tall) {
   using namespace mp;  // tall: most list tiles in a row tile, 1, 2 or 4
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -142,7 +144,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
 
     const int Fe = sh ? p.Fs : p.F;
     const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
-    const int nk = K >> 6;
+    const int nk = K >> 6, off = ONCE ? n0 / kCols % nk : 0;
     const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
     const int ldx = MODE == 1 ? p.ldh : p.W;
     auto weights = [&](const void* routed_w, const void* shared_w) {
@@ -186,15 +188,16 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         b_lo[h][i] = kA + (tb * 16 + (j & 1) * 8) * 128;
         b_vo[h][i] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ piece_swizzle(br))) * 2) : kOOB;
       }
+    auto place = [&](int t) { return (uint32_t)(t + off < nk ? t + off : t + off - nk) * 128; };
     auto issue_a = [&](int h, int t) {
       char* base = smem + (t & 1) * kBuf;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) lds_dma(xr, base + a_lo[h][i], a_vo[h][i], (uint32_t)t * 128);
+      for (int i = 0; i < 2; ++i) lds_dma(xr, base + a_lo[h][i], a_vo[h][i], place(t));
     };
     auto issue_b = [&](int h, int t) {
       char* base = smem + (t & 1) * kBuf;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) lds_dma(wr, base + b_lo[h][i], b_vo[h][i], (uint32_t)t * 128);
+      for (int i = 0; i < 2; ++i) lds_dma<ONCE ? kAuxNT : 0>(wr, base + b_lo[h][i], b_vo[h][i], place(t));
     };
     int a_rd[2], b_rd[2];
 #pragma unroll
@@ -356,43 +359,46 @@ int moe_pipe_height(const MoeGroupedParams& p, int mode) {
   return best;
 }
 
-template <int MODE>
+template <int MODE, bool ONCE>
 hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
-  constexpr int kCols = MODE == 0 ? 128 : 256;
   static bool attr_set = false;
   if (!attr_set) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_pipe_kernel<MODE>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_pipe_kernel<MODE, ONCE>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)mp::kLDS);
     attr_set = true;
   }
   const int tall = moe_pipe_height(p, MODE);
   const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8);
-  hipLaunchKernelGGL(moe_pipe_kernel<MODE>, dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
+  hipLaunchKernelGGL((moe_pipe_kernel<MODE, ONCE>), dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
   return hipGetLastError();
+}
+
+template <bool ONCE>
+hipError_t launch_moe_pipes(const MoeGroupedParams& p, hipStream_t st) {
+  const hipError_t e = p.gate ? launch_moe_pipe<0, ONCE>(p, st) : launch_moe_pipe<2, ONCE>(p, st);
+  return e != hipSuccess ? e : launch_moe_pipe<1, ONCE>(p, st);
 }
 
 bool pieces(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
 
-bool moe_pipe_ok(const MoeGroupedParams& p) {
+bool moe_lines_ok(const MoeGroupedParams& p) {
   constexpr int64_t kRange = (int64_t)1 << 31;
   const int64_t ids = (int64_t)p.M * p.S, widest = p.F > p.Fs ? p.F : p.Fs;
   const bool shared = p.S > p.top;
   if (p.f32 || p.W % 64 || p.W < 128 || p.F % 64 || p.F < 128 || (shared && (p.Fs % 64 || p.Fs < 128)) || p.ldh % 8)
     return false;
   if ((int64_t)p.M * p.W * 2 >= kRange || ids * p.ldh * 2 >= kRange || widest * p.W * 2 >= kRange) return false;
-  // fewer than 256 ids (no row of every expert's first list tile is sure to be there): the register-direct kernels are as
-  // fast up to 32 rows (two sub-tiles); above, the pipeline wins where the down product alone makes 96 tiles (64 rows:
-  // 146 -> 101 us at 2048 x 1408 of 16 experts + shared 2816, 518 -> 343 us at 4096 x 3584 + 7168; 64 tiles: equal)
-  if (ids < 256 && (p.M <= 32 || p.E * col_blocks(p, 1, p.F) < 96)) return false;
   if (!pieces(p.x) || !pieces(p.h) || !pieces(p.up) || !pieces(p.down) || (p.gate && !pieces(p.gate))) return false;
   return !shared || (pieces(p.sgate) && pieces(p.sup) && pieces(p.sdown));
 }
 
 }  // namespace dsse
 
+// The line lies at a mean of 128 rows per expert.  Plain / ONCE at 16 experts, top 2 and a shared one: 2048 x 1408 + 2816: 400 rows
+// 116 / 110 us, 1000 173 / 166, 1500 185 / 182 (but a whole prompt of 1649 rows in four 2708 / 2748), 3000 259 / 261; 4096 x 3584 +
+// 7168: 256 rows 333 / 314, 700 407 / 404, 1000 471 / 465, 3000 1038 / 1068.
 extern "C" hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st) {
-  const hipError_t e = p->gate ? dsse::launch_moe_pipe<0>(*p, st) : dsse::launch_moe_pipe<2>(*p, st);
-  return e != hipSuccess ? e : dsse::launch_moe_pipe<1>(*p, st);
+  return (int64_t)p->M * p->top <= 128 * (int64_t)p->E ? dsse::launch_moe_pipes<true>(*p, st) : dsse::launch_moe_pipes<false>(*p, st);
 }

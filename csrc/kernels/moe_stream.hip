@@ -1,0 +1,233 @@
+// Expert GEMMs of decode steps and short prompts (bf16): the weights as one stream through per-wave LDS rings.
+//
+// What bounds it: a few rows per expert, so nearly every weight of the layer is read once for them (311 MB at 2048 x 1408 of
+// 16 experts and a shared one of 2816, 1.59 GB at 4096 x 3584 and 7168), and what counts is how many bytes of weights are in
+// flight.  256-row tiles (moe_pipe.hip) hold 32 KiB per CU for a step and a quarter and fill 136 to 198 of the 256 CUs at the
+// smaller size; loads straight into MFMA operands touch 16 lines per quarter wave.  Here
+//
+//   * every wave streams its own 32 (gate / up) or 16 (down) weight rows through its own LDS ring, three to six 64-element
+//     steps deep, whole 128-byte lines per eight lanes, two workgroups per CU: some 96 KiB of weights in flight;
+//   * X comes through a ring that the four waves share, one barrier per step; its requests are spread over the waves, so a
+//     counted vmcnt covers both rings;
+//   * weights are non-temporal, and a column block starts at a K step of its own and wraps around: rows lie a power of two
+//     apart, and workgroups that walk K in step ask a few memory channels at a time;
+//   * sub-tiles of 16 rows: a workgroup takes the body for 16, 32 or 64 rows that its list tile needs, deeper for fewer;
+//   * narrow tiles for the down product (64 columns): its K axis is the hidden width, twice that for a shared expert, and it
+//     is the longest tile that ends last.
+//
+// Measured (one MI355X, work list and both products; weights of 700 MB and more read in turn; before: register-direct to 32
+// rows, moe_pipe.hip above).  2048 x 1408, 16 experts, top 2, shared 2816: 1 row 33 -> 27 us, 8 68 -> 56, 32 84 -> 65,
+// 64 105 -> 74, 160 106 -> 81.  4096 x 3584, shared 7168: 1 row 94 -> 67 us, 8 241 -> 202, 32 308 -> 237 (6.7 TB/s),
+// 64 320 -> 259, 160 323 -> 314.  On the way (32 rows, the two sizes): without its own first step and the non-temporal
+// hint 79 / 288, with the hint 73 / 261, with both 69 / 250, narrow down tiles 65 / 237; narrow gate / up tiles 64 / 251.
+#include <algorithm>
+
+#include "lds_dma.h"
+#include "moe_rows.h"
+
+namespace dsse {
+namespace {
+namespace ms {
+
+constexpr int kWaves = 4;
+constexpr int kStep = 64;         // K elements per step: 128 bytes of every row
+constexpr int kTile = 16 * 128;   // 16 weight rows of one step
+// By kind: weight tiles per wave, hidden units or output columns of a workgroup
+constexpr int wave_tiles(int mode) { return mode == 1 ? 1 : 2; }
+constexpr int columns(int mode) { return mode == 2 ? 128 : 64; }
+// By kind and sub-tiles of 16 rows: ring depth, X's DMA instructions (8 rows each) per wave and step
+constexpr int depth(int mode, int subs) { return mode == 1 ? (subs == 4 ? 5 : 6) : (subs == 4 ? 3 : 4); }
+constexpr int x_dma(int subs) { return subs == 4 ? 2 : 1; }
+constexpr int x_slot(int subs) { return x_dma(subs) * kWaves * 1024; }
+constexpr int lds_bytes(int mode, int subs) { return depth(mode, subs) * (kWaves * wave_tiles(mode) * kTile + x_slot(subs)); }
+constexpr int kLDS = 80 * 1024;   // two workgroups per CU
+
+}  // namespace ms
+
+// MODE 0: h = silu(gate x) * (up x); 1: o = weight * down h; 2: h = relu(up x)^2.  The column block cb of the list tile whose
+// ids the lanes hold in `mine`, the first `rows` of them real.
+template <int MODE, int SUBS>
+DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int mine, int rows) {
+  using namespace ms;
+  constexpr int CT = wave_tiles(MODE), D = depth(MODE, SUBS), NX = x_dma(SUBS), NW = 2 * CT;
+  static_assert(lds_bytes(MODE, SUBS) <= kLDS);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const bool sh = e >= p.E;
+  const int Fe = sh ? p.Fs : p.F;
+  const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
+  const int nk = K / kStep, first = cb % nk;
+  const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
+  const int ldx = MODE == 1 ? p.ldh : p.W;
+
+  auto weights = [&](const void* routed_w, const void* shared_w) {
+    return reinterpret_cast<const bf16*>(sh ? shared_w : routed_w) + (sh ? 0 : (int64_t)e * p.F * p.W);
+  };
+  const bf16* w0 = MODE == 1 ? weights(p.down, p.sdown) : (MODE == 0 ? weights(p.gate, p.sgate) : weights(p.up, p.sup));
+  const bf16* w1 = MODE == 0 ? weights(p.up, p.sup) : w0;
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, (uint32_t)((size_t)(MODE == 1 ? p.M * p.S : p.M) * ldx * 2));
+  const __amdgpu_buffer_rsrc_t wr0 = make_rsrc(w0, (uint32_t)((size_t)N * K * 2));
+  const __amdgpu_buffer_rsrc_t wr1 = make_rsrc(w1, (uint32_t)((size_t)N * K * 2));
+  const int n0 = cb * columns(MODE) + w * (columns(MODE) / kWaves);  // the wave's first hidden unit or column
+
+  uint32_t xo[NX], wo[NW];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) {
+    const int row = (w * NX + i) * 8 + (lane >> 3);
+    const int id = __shfl(mine, row);
+    xo[i] = row < rows && row < 16 * SUBS
+                ? (uint32_t)(((size_t)(MODE == 1 ? id : id / p.S) * ldx + 8 * ((lane & 7) ^ piece_swizzle(row))) * 2)
+                : kOOB;
+  }
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {  // instruction j: 8 rows of weight tile j / 2 (gate and up are tiles of the same units)
+    const int br = (j & 1) * 8 + (lane >> 3);
+    const int n = n0 + br + (MODE == 0 ? 0 : 16 * (j >> 1));
+    wo[j] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ piece_swizzle(br))) * 2) : kOOB;
+  }
+  char* wring = smem + w * D * CT * kTile;
+  char* xring = smem + kWaves * D * CT * kTile;
+  // byte offset of step c in every row; a step past the last lands as zeros, without traffic
+  auto place = [&](int c) {
+    const int k = c + first < nk ? c + first : c + first - nk;
+    return c < nk ? (uint32_t)k * 128 : kOOB;
+  };
+  auto issue_w = [&](int c, int slot) {
+    const uint32_t at = place(c);
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+      lds_dma<kAuxNT>(MODE == 0 && j >= 2 ? wr1 : wr0, wring + slot * CT * kTile + j * 1024, wo[j] | (at & kOOB), at & ~kOOB);
+  };
+  auto issue_x = [&](int c, int slot) {
+    const uint32_t at = place(c);
+#pragma unroll
+    for (int i = 0; i < NX; ++i)
+      lds_dma(xr, xring + slot * x_slot(SUBS) + (w * NX + i) * 1024, xo[i] | (at & kOOB), at & ~kOOB);
+  };
+  f32x4 acc[SUBS][CT];
+#pragma unroll
+  for (int i = 0; i < SUBS; ++i)
+#pragma unroll
+    for (int n = 0; n < CT; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int rd[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) rd[s] = r * 128 + (((2 * g + s) ^ piece_swizzle(r)) << 4);
+
+  // Step c's X is requested D - 1 steps ahead, into the slot of step c - 1 once the barrier of step c says that every wave
+  // has read it; its weights D steps ahead, into the wave's own ring once this wave has read them.  Younger than step c's X
+  // when step c opens: the weights of step c + 1 and D - 2 whole steps.
+  issue_w(0, 0);
+#pragma unroll
+  for (int c = 1; c < D; ++c) issue_x(c - 1, c - 1), issue_w(c, c);
+  int slot = 0;
+  for (int c = 0; c < nk; ++c) {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(NW + (D - 2) * (NX + NW)) : "memory");
+    const char* wb = wring + slot * CT * kTile;
+    const char* xb = xring + slot * x_slot(SUBS);
+    bf16x8 b[CT][2], a[SUBS][2];
+#pragma unroll
+    for (int n = 0; n < CT; ++n)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) b[n][s] = *reinterpret_cast<const bf16x8*>(wb + n * kTile + rd[s]);
+#pragma unroll
+    for (int i = 0; i < SUBS; ++i)
+      if (16 * i < rows)  // uniform
+#pragma unroll
+        for (int s = 0; s < 2; ++s) a[i][s] = *reinterpret_cast<const bf16x8*>(xb + i * 2048 + rd[s]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    issue_x(c + D - 1, slot == 0 ? D - 1 : slot - 1);
+    issue_w(c + D, slot);
+#pragma unroll
+    for (int i = 0; i < SUBS; ++i) {
+      if (16 * i >= rows) continue;  // uniform
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int n = 0; n < CT; ++n) acc[i][n] = mfma16x16x32(a[i][s], b[n][s], acc[i][n]);
+    }
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no piece lands in LDS that this workgroup has given back
+
+#pragma unroll
+  for (int i = 0; i < SUBS; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int id = __shfl(mine, 16 * i + 4 * g + j);
+      if (id < 0) continue;
+      const int row = id / p.S;
+      const float wt = MODE == 1 ? out_weight(p, row, id - row * p.S) : in_weight(p, id);
+      if (MODE == 0) {
+        const int f = n0 + r;
+        const float gv = acc[i][0][j] * wt;
+        if (f < N)
+          reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(gv / (1.0f + expf(-gv)) * (acc[i][CT - 1][j] * wt));
+      } else {
+#pragma unroll
+        for (int n = 0; n < CT; ++n) {
+          const int f = n0 + 16 * n + r;
+          if (f >= N) continue;
+          const float v = acc[i][n][j] * wt;
+          if (MODE == 1) p.o[(int64_t)id * p.W + f] = v;
+          else reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(v > 0.0f ? v * v : 0.0f);
+        }
+      }
+    }
+}
+
+// A workgroup per (list tile, column block): the shared expert's tiles, the last of the list, come first
+template <int MODE>
+__global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeGroupedParams p, int shared_tiles, int cols_s, int cols_r) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int v = blockIdx.x, head = shared_tiles * cols_s;
+  const int tiles = __builtin_amdgcn_readfirstlane(ld_global<int>(p.num_tiles));
+  int t, cb;
+  if (v < head) t = max(tiles - shared_tiles, 0) + v / cols_s, cb = v % cols_s;
+  else t = (v - head) / cols_r, cb = (v - head) % cols_r;
+  // a routed tile's expert and ids are requested together with the tile count: the list has room for every t of the grid
+  const int e = __builtin_amdgcn_readfirstlane(ld_global<int>(p.tile_expert + t));
+  const int mine = ld_global<int>(p.sorted + t * kMoeRows + (threadIdx.x & 63));
+  if (e < 0 || (v >= head && t >= tiles - shared_tiles)) return;
+  if (cb * ms::columns(MODE) >= (MODE == 1 ? p.W : (e >= p.E ? p.Fs : p.F))) return;
+  const int rows = __popcll(__ballot(mine >= 0));  // an expert's ids fill its tiles from the front
+  if (rows <= 16) stream_tile<MODE, 1>(p, smem, e, cb, mine, rows);
+  else if (rows <= 32) stream_tile<MODE, 2>(p, smem, e, cb, mine, rows);
+  else stream_tile<MODE, 4>(p, smem, e, cb, mine, rows);
+}
+
+template <int MODE>
+hipError_t launch_moe_stream(const MoeGroupedParams& p, hipStream_t st) {
+  static bool attr_set = false;
+  if (!attr_set) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_stream_kernel<MODE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, ms::kLDS);
+    attr_set = true;
+  }
+  // a multiple of 8 column blocks: the row tiles of a weight panel meet on one XCD
+  auto blocks = [&](int F) {
+    constexpr int cols = ms::columns(MODE);
+    return (((MODE == 1 ? p.W : F) + cols - 1) / cols + 7) / 8 * 8;
+  };
+  const int shared = p.S > p.top ? (p.M + kMoeRows - 1) / kMoeRows : 0;
+  const int64_t ids = (int64_t)p.M * p.top;
+  // most list tiles that the routed experts can make
+  const int64_t routed = std::min((ids + (int64_t)(kMoeRows - 1) * p.E) / kMoeRows, ids);
+  const int cols_s = shared ? blocks(p.Fs) : 1, cols_r = blocks(p.F);
+  const int64_t grid = (int64_t)shared * cols_s + routed * cols_r;
+  hipLaunchKernelGGL(moe_stream_kernel<MODE>, dim3((unsigned)grid), dim3(256), ms::kLDS, st, p, shared, cols_s, cols_r);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// Above three list tiles of a shared expert the stream's 64-row tiles read its weights once too often.  Stream / pipeline, the two
+// sizes above: 160 rows 81 / 95 us and 312 / 300, 192 rows 80 / 96 and 311 / 305, 224 rows 91 / 98 and 355 / 310, 256 rows 92 / 99
+// and 357 / 314; below, the stream is ahead at both (128 rows 74 / 96 and 282 / 298).
+bool moe_stream_pays(const MoeGroupedParams& p) { return p.M <= 192; }
+
+}  // namespace dsse
+
+extern "C" hipError_t dsse_moe_stream(const dsse::MoeGroupedParams* p, hipStream_t st) {
+  const hipError_t e = p->gate ? dsse::launch_moe_stream<0>(*p, st) : dsse::launch_moe_stream<2>(*p, st);
+  return e != hipSuccess ? e : dsse::launch_moe_stream<1>(*p, st);
+}

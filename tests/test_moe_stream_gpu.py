@@ -1,0 +1,55 @@
+"""The streamed expert GEMMs (moe_stream.hip) against the PyTorch reference, at the sizes where their tiling changes."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    ops.load_library(required=True)
+    return torch.device("cuda", 0)
+
+
+# rows of expert 0 on both sides of the 16-, 32- and 64-row bodies; two K steps (fewer than any ring is deep), odd counts of
+# them, and K walks that wrap at every column block; widths that end inside a column block; rows that choose one expert only;
+# no shared expert; the largest step (three list tiles of the shared expert)
+@pytest.mark.parametrize("M,W,F,Fs,E,top,first,gated", [
+    (1, 128, 128, 128, 2, 2, 1, True), (1, 192, 320, 0, 3, 1, 1, False), (16, 320, 192, 448, 3, 2, 16, True),
+    (17, 576, 448, 192, 4, 2, 17, True), (33, 128, 1088, 128, 2, 1, 32, True), (64, 192, 192, 320, 5, 2, 33, True),
+    (65, 448, 128, 128, 2, 1, 65, True), (100, 256, 576, 0, 3, 2, 64, False), (192, 320, 192, 128, 8, 2, 129, True),
+    (40, 128, 128, 128, 300, 1, 0, True)])
+@pytest.mark.parametrize("weight_input", [False, True])
+def test_streamed_experts(gpu, M, W, F, Fs, E, top, first, gated, weight_input):
+    g = torch.Generator().manual_seed(M + W + F)
+
+    def rnd(*s):
+        return (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16()
+
+    x = torch.randn(M, W, generator=g).bfloat16()
+    gate, up, down = rnd(E, F, W) if gated else None, rnd(E, F, W), rnd(E, W, F)
+    sh = (rnd(Fs, W), rnd(Fs, W), rnd(W, Fs)) if Fs else (None, None, None)
+    S = top + (1 if Fs else 0)
+    # `first` rows choose expert 0 first, the others begin elsewhere; further choices are the next experts
+    start = torch.randint(0, max(1, E - 1), (M,), generator=g) + 1
+    start[torch.randperm(M, generator=g)[:first]] = 0
+    idx = ((start[:, None] + torch.arange(top)) % E).int()
+    w = torch.rand(M, S, generator=g) + 0.25
+    ref = torch.zeros(M * S, W)
+    lref.moe_grouped(x, idx, w, gate, up, down, *sh, ref, weight_input)
+    tiles = -(-M * S // 64) + E + 2
+    c = lambda t: None if t is None else t.to(gpu)  # noqa: E731
+    o = torch.full((M * S, W), float("nan"), device=gpu)
+    ops.moe_grouped(c(x), c(idx), c(w), c(gate), c(up), c(down), *(c(t) for t in sh),
+                    torch.zeros(tiles * 64, dtype=torch.int32, device=gpu), torch.zeros(tiles, dtype=torch.int32, device=gpu),
+                    torch.zeros(1, dtype=torch.int32, device=gpu),
+                    torch.zeros(M * S, max(F, Fs), dtype=torch.bfloat16, device=gpu), o, weight_input)
+    # every hidden value is rounded to bf16 once, by at most 2^-8 of itself; the sums are fp32
+    err = (o.cpu().double() - ref.double()).norm() / ref.double().norm()
+    assert float(err) <= 2.0 ** -8
+    assert float((o.cpu() - ref).abs().max()) <= 2.0 ** -5 * float(ref.abs().max())
