@@ -234,7 +234,7 @@ WCfg pick_wide(int M, int N, int K) {
   return c;
 }
 
-// cfg 8 / 9 / 10 = the pipelined 256 / 192 / 128 x 256 kernel of gemm_pipe.hip; 0, 1, 5 = gemm_tiled.hip's
+// cfg 8 / 9 / 10 = the pipelined 256 / 192 / 128 x 256 kernel of gemm_pipe.hip; 0, 1, 2, 5 = gemm_tiled.hip's
 // configurations.  partial_only 2 (gemm_pipe only) = split-K slices combined inside the launch (run_pipe_fix).
 hipError_t tiled_call(int mode, int cfg, int S, int partial_only, const void* X, int ldx, int M, const void* W, int K,
                       int N, const dsse::GemmEpi* ep, float* part) {
@@ -266,7 +266,7 @@ int* fix_counters(const at::Device& dev) { return fix_state(dev).data_ptr<int>()
 constexpr int kMaxDecodeM = 512;  // gemm_stream: one workgroup per tile group up to 256 rows, row blocks above
 
 // Tiled LDS-DMA GEMMs (gemm_tiled.hip, gemm_pipe.hip; prefill and wide batches).  DSSE_KERNEL_CFG overrides: t_cfg
-// (0 = 256x128, 1 = 128x128, 5 = 128x256, 8 / 9 / 10 = the 256 / 192 / 128 x 256 gemm_pipe tile), t_split, t_fix
+// (0 = 256x128, 1 = 128x128, 2 = up to 256 rows x 128, 5 = 128x256, 8 / 9 / 10 = the 256 / 192 / 128 x 256 gemm_pipe tile), t_split, t_fix
 // (1 = split-K slices combined inside the launch, gemm_pipe only), t_model (0 = the round-5 row-range table).
 struct TCfg {
   int cfg, S;
@@ -356,10 +356,51 @@ bool half_block_pays(int M, int N, int K, const TCfg& c) {
   return true;
 }
 
+// 65 to 256 rows on one tile that holds them all (gemm_tiled cfg 2), in one round of at most 256 workgroups.  Two row blocks
+// of 128 fetch every weight twice and compute dead rows.  Measured with X rewritten and 4 GB of weights read in turn, this tile /
+// what the other rules give, in us:
+//   129 to 192 rows, wide products: 28672 x 4096 SiLU 160 rows 58 / 70, fp32 180 rows 68 / 76; 32768 x 4096 75 / 85; 26752 x 4096 64 /
+//   89; 14336 x 4096 47 / 49; 32768 x 2048 42 / 44; 8320 x 2048 160 rows 25 / 42; 10240 x 4096 43 / 43.  To 8192 columns it is behind
+//   (8192 x 4096 160 rows 32 / 30, 6144 x 2048 22 / 21) unless the slabs are the next kernel's: 6144 x 4096 in 4 slices 160 rows 20 / 22,
+//   4096 x 14336 in 8 32 / 36 (200 rows 37 / 38); 4096 x 4096 15 / 17, but in 8 slices instead of 4, which the norm reads;
+//   193 rows and more: only without a 256-column tile (26752 x 4096 224 rows 72 / 91) or where two slices or one fill half a round
+//   to a whole one (16384 x 4096 54 / 58, 14336 x 4096 51 / 53) or the weights fill the chip (28672 x 4096 200 rows 75 / 79, 224 78 / 80,
+//   but 256 83 / 82, and 32768 x 2048 49 / 46);
+//   65 to 128 rows: the widest (28672 x 4096 72 rows 51 / 58, 128 56 / 56; 32768 x 2048 35 / 40, 38 / 43; but 26752 x 4096 55 / 52), and
+//   where the ring's slices end above one round (8320 x 2048 72 rows 21 / 23, 10240 x 4096 31 / 35, 128 rows 37 / 40).
+// Two slices where half the K walk is longer than their slabs and the reduction: 10240 x 4096 160 rows 38 / 49, 8320 x 2048 25 / 26,
+// 14464 x 2048 29 / 27, 16384 x 2048 31 / 28.
+TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
+  TCfg c{};
+  c.ok = false;
+  c.cfg = 2;
+  c.S = 1;
+  const int blocks = N / 128;
+  if (M <= 64 || M > 256 || N % 128 || K % 128 || blocks > 256 || (int64_t)M * K * 2 >= ((int64_t)1 << 31)) return c;
+  if (N > 8192) {
+    if (M > 192) c.ok = N % 256 || (blocks >= 112 && blocks <= 128) || (M <= 224 && K >= 4096 && blocks >= 224);
+    else if (M > 128) c.ok = true;
+    else {
+      const SCfg r = pick_stream(M, N, K);
+      c.ok = blocks >= 224 || (r.ok && r.nw == 4 && N / 64 * r.S > 256);
+    }
+    c.S = blocks <= 128 && K >= 1024 && (double)K * (M + 128) > 61e3 * (4.0 + 3.2e-6 * M * N) ? 2 : 1;
+  } else if (M > 128 && M <= 192 && slab_consumer && K >= 4096 && (N > 4096 || K > 4096)) {
+    while (blocks * c.S * 2 <= 256 && K % (128 * c.S) == 0 && K / (c.S * 2) >= 512) c.S *= 2;
+    c.ok = blocks * c.S >= 160;
+  }
+  return c;
+}
+
 TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
   TCfg c{};
   int cfg = env_int("t_cfg", -1);
-  const bool forced = cfg == 0 || cfg == 1 || cfg == 5 || cfg == 8 || cfg == 9 || cfg == 10;
+  const bool forced = cfg == 0 || cfg == 1 || cfg == 2 || cfg == 5 || cfg == 8 || cfg == 9 || cfg == 10;
+  if (!forced) {
+    c = rows_plan(M, N, K, slab_consumer);
+    if (c.ok) return c;
+    c = TCfg{};
+  }
   if (!forced && env_int("t_model", 1) && N % 128 == 0 && K % 128 == 0 && M > kModelMinM) {
     c = pipe_plan(M, N, K, slab_consumer);
     if (c.ok && (N % 256 == 0 || half_block_pays(M, N, K, c))) return c;
@@ -397,11 +438,11 @@ TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
   }
   constexpr int min_wgs = 160;  // split K until this many workgroups (table choices, M <= 512)
   // tile shapes by cfg (gemm_tiled.hip launch_t_mode: 0, 1, 5; gemm_pipe.hip: 8, 9, 10)
-  const int BM = cfg == 1 || cfg == 5 || cfg == 10 ? 128 : cfg == 9 ? 192 : 256, BN = cfg == 0 || cfg == 1 ? 128 : 256;
+  const int BM = cfg == 1 || cfg == 5 || cfg == 10 ? 128 : cfg == 9 ? 192 : 256, BN = cfg <= 2 ? 128 : 256;
   c.cfg = cfg;
   c.S = 1;
   const bool pipe = cfg >= 8;
-  c.ok = N % BN == 0 && K % (pipe ? 128 : 64) == 0;
+  c.ok = N % BN == 0 && K % (pipe ? 128 : 64) == 0 && (cfg != 2 || (M > 64 && M <= 256));
   if (!c.ok) return c;
   const int tiles = ((M + BM - 1) / BM) * (N / BN);
   int S = env_int("t_split", 0);
@@ -444,6 +485,7 @@ int gemm_impl(int M, int N, int K) {
     // 65-128 rows, narrow N (4-wave stream shapes: qkv / o / down): the ring kernel with 8 row tiles, 3 slots;
     // 128-stream step 6.19 / 6.23 vs 6.36 / 6.37 ms on gemm_wide (profiles/r2/ring128_ab.log)
     if (impl < 0 && M <= 128) {
+      if (env_int("t_cfg", -1) < 0 && rows_plan(M, N, K, false).ok) return 4;
       const SCfg sc = pick_stream(M, N, K);
       if (sc.ok && sc.mt == 8 && sc.nt == 1 && sc.nw == 4) return 2;
     }

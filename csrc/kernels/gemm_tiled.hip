@@ -32,7 +32,7 @@ namespace dsse {
 template <int WM, int WN, int MT, int NT, int NS>
 struct TiledGeom {
   static constexpr int BM = WM * MT * 16, BN = WN * NT * 16, NTHR = 64 * WM * WN;
-  static constexpr int A_BYTES = BM * 128;            // 64 bf16 per row
+  static constexpr int A_BYTES = (BM + 8 * WM * WN - 1) / (8 * WM * WN) * (8 * WM * WN) * 128;  // 64 bf16 per row
   static constexpr int B_BYTES = (BN / 16) * 2048;    // two 1 KiB k-step blocks per 16-column tile
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int A_INS = A_BYTES / 1024 / (WM * WN);  // 1 KiB DMA instructions per wave per stage
@@ -57,7 +57,14 @@ DEV void glds16(const void* src, char* lds_base) {
 #endif
 constexpr bool kBurst = DSSE_TILED_BURST;  // A/B build only: every tile issues its stage in one burst
 
-template <int WM, int WN, int MT, int NT, int NS, int FB, int MODE>
+// ROWS: one tile holds all rows (65 to 256, MT of 3 to 8 sub-tiles per wave row) and 128 columns, so that every weight is fetched
+// once, non-temporal, and no row that is not there is fetched; four stages where they fit.  What bounds it is the LDS fill, 45
+// GB/s per CU: (rows + 128) x 128 bytes per K step.  Mistral's gate_up at 160 rows: 57 us (0.86 us per step, 0.82 by the fill) against
+// 69 with two row blocks of 128 x 256; with 192 rows computed for 160 the same, with 256 66.  A column
+// block begins at a K step of its own and wraps around: X has just been written on other XCDs, and workgroups that ask for different
+// parts of it bring it into their XCD's L2 for each other (160-stream decode step 6201 -> 6075 us, 200-row prompt 6277 -> 6108).
+
+template <int WM, int WN, int MT, int NT, int NS, int FB, int MODE, bool ROWS = false>
 __global__ void __launch_bounds__(64 * WM * WN)
 gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restrict__ W, int K, int N, int Kr,
                   GemmEpi ep, float* __restrict__ part) {
@@ -100,16 +107,44 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
     b_src[i] = W + ((size_t)(n0 / 16 + (j >> 1)) * KC) * kTileChunk + (j & 1) * 512 + lane * 8;
   }
 
+  // ROWS: the same places as offsets into buffers, where rows that do not exist land as zeros without traffic
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, (uint32_t)((size_t)M * ldx * 2));
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(W + (size_t)(n0 / 16) * KC * kTileChunk, (uint32_t)(G::BN / 16) * KC * kTileChunk * 2);
+  uint32_t a_vo[G::A_INS], b_vo[G::B_INS];
+#pragma unroll
+  for (int i = 0; i < G::A_INS; ++i) {
+    const int row = m0 + (w * G::A_INS + i) * 8 + (lane >> 3);
+    a_vo[i] = row < M ? (uint32_t)(row * ldx + a_koff[i]) * 2 : kOOB;
+  }
+#pragma unroll
+  for (int i = 0; i < G::B_INS; ++i) {
+    const int j = w * G::B_INS + i;
+    b_vo[i] = (uint32_t)((j >> 1) * KC * kTileChunk + (j & 1) * 512 + lane * 8) * 2;
+  }
+  const int turn = ROWS ? bn % nk : 0;  // the K step this workgroup begins at; it wraps around
   auto issue_a = [&](int stage, int t) {
+    t = t + turn < nk ? t + turn : t + turn - nk;
     const int kk = k0 + 64 * t, c = kk >> 7, h = (kk >> 6) & 1;
     char* base = smem + stage * G::STAGE;
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int i = 0; i < G::A_INS; ++i) lds_dma(xr, base + (w * G::A_INS + i) * 1024, a_vo[i], (uint32_t)(c * 128 + 16 * h) * 2);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < G::A_INS; ++i)
       glds16(a_src[i] + c * 128 + 16 * h + a_koff[i], base + (w * G::A_INS + i) * 1024);
   };
   auto issue_b = [&](int stage, int t) {
+    t = t + turn < nk ? t + turn : t + turn - nk;
     const int kk = k0 + 64 * t, c = kk >> 7, h = (kk >> 6) & 1;
     char* base = smem + stage * G::STAGE;
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int i = 0; i < G::B_INS; ++i)
+        lds_dma<kAuxNT>(wr, base + G::A_BYTES + (w * G::B_INS + i) * 1024, b_vo[i], (uint32_t)(c * kTileChunk + h * 1024) * 2);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < G::B_INS; ++i)
       glds16(b_src[i] + (size_t)c * kTileChunk + h * 1024, base + G::A_BYTES + (w * G::B_INS + i) * 1024);
@@ -212,18 +247,18 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
       }
 }
 
-template <int WM, int WN, int MT, int NT, int NS, int FB, int MODE>
+template <int WM, int WN, int MT, int NT, int NS, int FB, int MODE, bool ROWS = false>
 static hipError_t launch_t(const bf16* X, int ldx, int M, const bf16* W, int K, int N, int S, const GemmEpi& ep,
                            float* part, hipStream_t st) {
   using G = TiledGeom<WM, WN, MT, NT, NS>;
   static bool attr_set = false;
   if (!attr_set) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WM, WN, MT, NT, NS, FB, MODE>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tiled_kernel<WM, WN, MT, NT, NS, FB, MODE, ROWS>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS);
     attr_set = true;
   }
   const int nbm = (M + G::BM - 1) / G::BM, nbn = N / G::BN;
-  hipLaunchKernelGGL((gemm_tiled_kernel<WM, WN, MT, NT, NS, FB, MODE>), dim3(nbm * nbn * S), dim3(G::NTHR), G::LDS, st,
+  hipLaunchKernelGGL((gemm_tiled_kernel<WM, WN, MT, NT, NS, FB, MODE, ROWS>), dim3(nbm * nbn * S), dim3(G::NTHR), G::LDS, st,
                      X, ldx, M, W, K, N, K / S, ep, part);
   return hipGetLastError();
 }
@@ -236,6 +271,16 @@ static hipError_t launch_t_mode(int cfg, const bf16* X, int ldx, int M, const bf
     // in profiles/experiments_r2.md; the 256 x 256 configurations moved to gemm_pipe.hip (cfg 8, round 5)
     case 0: return launch_t<4, 2, 4, 4, 3, 2, MODE>(X, ldx, M, W, K, N, S, ep, part, st);  // 256 x 128, 8 waves
     case 1: return launch_t<2, 2, 4, 4, 3, 2, MODE>(X, ldx, M, W, K, N, S, ep, part, st);  // 128 x 128, 4 waves
+    case 2:  // 65-256 rows, all in one tile x 128 columns, 8 waves
+      switch ((M + 31) / 32) {
+        case 3: return launch_t<2, 4, 3, 2, 4, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+        case 4: return launch_t<2, 4, 4, 2, 4, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+        case 5: return launch_t<2, 4, 5, 2, 4, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+        case 6: return launch_t<2, 4, 6, 2, 4, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+        case 7: return launch_t<2, 4, 7, 2, 3, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+        case 8: return launch_t<2, 4, 8, 2, 3, 2, MODE, true>(X, ldx, M, W, K, N, S, ep, part, st);
+      }
+      return hipErrorInvalidValue;
     case 5: return launch_t<2, 4, 4, 4, 3, 2, MODE>(X, ldx, M, W, K, N, S, ep, part, st);  // 128 x 256, 8 waves
   }
   return hipErrorInvalidValue;
@@ -243,7 +288,7 @@ static hipError_t launch_t_mode(int cfg, const bf16* X, int ldx, int M, const bf
 
 }  // namespace dsse
 
-// cfg: 0 = 256 x 128 tile (8 waves, 3 LDS stages), 1 = 128 x 128 (4 waves), 5 = 128 x 256 (8 waves, 3 stages of 16
+// cfg: 0 = 256 x 128 tile (8 waves, 3 LDS stages), 1 = 128 x 128 (4 waves), 2 = 65-256 rows x 128 (8 waves, 4 or 3 stages), 5 = 128 x 256 (8 waves, 3 stages of 16
 // KiB X + 32 KiB W: twice the weight bytes in flight per CU of cfg 0, for the weight-streaming 129-256-row decode
 // GEMMs; the two row blocks of a column block share an XCD and its L2).  (Round 4's 256 x 256 configurations 2, 3, 4,
 // 6 and 7 are gone: gemm_pipe.hip, cfg 8, replaces them.)
