@@ -107,6 +107,7 @@ struct LruScanParams {
   void* out;             // [T, C] element type: state * y
   int nseq, C, bw, rows; // rows = T
   int coeff;             // 1: compute (a, b) for all rows first; 0: gates already hold them (a later sequence group)
+  int alone;             // 1 (with coeff): the sequences hold all T rows, and nobody reads the coefficients afterwards
   float* chunk_a;        // [rows / 32 + nseq + 1, C] scratch of the chunked walk (prompt portions), or null
   float* chunk_b;
   float c;               // 8: log a = -c r softplus(lam)
@@ -182,9 +183,22 @@ struct MoeRouteRowsParams {
   float scale;
 };
 
+// Choice (the `top` largest logits, softmax over them) and work list of a decode-sized step in one launch, by one workgroup.
+struct MoeTopkListsParams {
+  const float* z;        // [M, E] logits
+  int* topk_idx;         // [M, top]
+  float* topk_w;         // [M, top]
+  int* sorted;           // as in MoeGroupedParams
+  int* tile_expert;
+  int* num_tiles;
+  int M, E, top, S, max_tiles;
+};
+bool moe_topk_lists_ok(int M, int E, int top);
+
 }  // namespace dsse
 
 extern "C" {
+hipError_t dsse_moe_topk_lists(const dsse::MoeTopkListsParams* p, hipStream_t st);
 hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st);  // the GEMMs alone: the work list is ready
 hipError_t dsse_moe_stream(const dsse::MoeGroupedParams* p, hipStream_t st);  // likewise
 hipError_t dsse_gemm_rm(const dsse::GemmRmParams* p, hipStream_t st);

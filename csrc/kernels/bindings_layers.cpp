@@ -328,7 +328,7 @@ void conv_state(const Tensor& in, const Tensor& taps, const OptTensor& bias, con
 
 void lru_scan(const Tensor& u, Tensor& gates, const Tensor& y, const Tensor& lam, Tensor& state,
               const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len, const Tensor& state_slot, Tensor& out,
-              double c, const OptTensor& y_bias, bool coeff, const OptTensor& scratch) {
+              double c, const OptTensor& y_bias, bool coeff, const OptTensor& scratch, bool alone) {
   f32t(u, "u");
   f32t(gates, "gates");
   f32t(y, "y");
@@ -354,6 +354,7 @@ void lru_scan(const Tensor& u, Tensor& gates, const Tensor& y, const Tensor& lam
   }
   p.rows = (int)u.size(0);
   p.coeff = coeff ? 1 : 0;
+  p.alone = alone ? 1 : 0;
   if (scratch.has_value()) {  // [2, slots, C] with slots >= rows / 32 + sequences + 1: the chunked walk's scratch
     f32t(*scratch, "scratch");
     const int64_t slots = p.rows / 32 + p.nseq + 1;
@@ -577,6 +578,35 @@ void moe_topk(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w) {
                                cur_stream()));
 }
 
+// moe_topk and the work list of moe_grouped (aligned) in one launch, for decode-sized steps; false: nothing done, the step is larger.
+bool moe_topk_lists(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w, Tensor& sorted, Tensor& tile_expert,
+                    Tensor& num_tiles, bool shared) {
+  f32t(logits, "logits");
+  i32(topk_idx, "topk_idx");
+  f32t(topk_w, "topk_w");
+  i32(sorted, "sorted");
+  i32(tile_expert, "tile_expert");
+  i32(num_tiles, "num_tiles");
+  const int M = (int)logits.size(0), E = (int)logits.size(1), top = (int)topk_idx.size(1), S = top + (shared ? 1 : 0);
+  TORCH_CHECK(logits.dim() == 2 && topk_idx.dim() == 2 && topk_idx.size(0) == M && topk_w.sizes() == topk_idx.sizes() &&
+                  top >= 1 && top <= E,
+              "moe_topk_lists shapes");
+  if (!dsse::moe_topk_lists_ok(M, E, top)) return false;
+  dsse::MoeTopkListsParams p{};
+  p.z = logits.data_ptr<float>();
+  p.topk_idx = topk_idx.data_ptr<int>();
+  p.topk_w = topk_w.data_ptr<float>();
+  p.sorted = sorted.data_ptr<int>();
+  p.tile_expert = tile_expert.data_ptr<int>();
+  p.num_tiles = num_tiles.data_ptr<int>();
+  p.M = M, p.E = E, p.top = top, p.S = S;
+  p.max_tiles = (int)tile_expert.numel();
+  TORCH_CHECK(p.max_tiles >= ((int64_t)M * S + 63) / 64 + E + 1 && sorted.numel() >= (int64_t)p.max_tiles * 64 && num_tiles.numel() >= 1,
+              "moe_topk_lists: scratch too small");
+  DSSE_CHECK_HIP(dsse_moe_topk_lists(&p, cur_stream()));
+  return true;
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(dsse, m) {
@@ -599,9 +629,11 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "bool single=False) -> ()");
   m.def("lru_scan(Tensor u, Tensor(c!) gates, Tensor y, Tensor lam, Tensor(a!) state, Tensor q_start, Tensor q_len, "
         "Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float c, Tensor? y_bias=None, bool coeff=True, "
-        "Tensor(d!)? scratch=None) -> ()");
+        "Tensor(d!)? scratch=None, bool alone=False) -> ()");
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
+  m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "
+        "Tensor(e!) num_tiles, bool shared) -> bool");
   m.def("moe_ffn(Tensor x, Tensor topk_idx, Tensor topk_w, Tensor gate, Tensor up, Tensor down, Tensor? sgate, "
         "Tensor? sup, Tensor? sdown, Tensor(a!) out) -> ()");
 }
@@ -616,6 +648,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("lru_scan", &lru_scan);
   m.impl("moe_router", &moe_router);
   m.impl("moe_topk", &moe_topk);
+  m.impl("moe_topk_lists", &moe_topk_lists);
   m.impl("moe_ffn", &moe_ffn);
   m.impl("moe_grouped", &moe_grouped);
   m.impl("moe_route_rows", &moe_route_rows);

@@ -61,8 +61,9 @@ __global__ __launch_bounds__(256) void conv_state_kernel(ConvStateParams p) {
     }
 }
 
-// The same for prompt portions with four taps, four channels per thread and the last three inputs in registers: an input is
-// read once instead of four times (3000 rows of 4096: 74 -> 26 us)
+// The same with four taps, four channels per thread and the last three inputs in registers: an input is read once instead of
+// four times (3000 rows of 4096: 74 -> 26 us).  Only a sequence's first rows read the old tail, so their thread writes the new
+// one as well: no second launch (4.5 us in a decode step).
 template <typename T>
 __global__ __launch_bounds__(256) void conv_state4_kernel(ConvStateParams p) {
   constexpr int K = 4, Kt = K - 1;
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(256) void conv_state4_kernel(ConvStateParams p) {
   const int t1 = t0 + kConvRows < ql ? t0 + kConvRows : ql;
   const int row0 = p.q_start[seq];
   const bool fresh = p.ctx_len[seq] - ql == 0;
-  const float* tail = p.tail + (int64_t)p.state_slot[seq] * Kt * p.C + c;
+  float* tail = p.tail + (int64_t)p.state_slot[seq] * Kt * p.C + c;
   const f32x4 zero{0.f, 0.f, 0.f, 0.f};
   f32x4 taps[4];  // of channel c + e
 #pragma unroll
@@ -88,6 +89,16 @@ __global__ __launch_bounds__(256) void conv_state4_kernel(ConvStateParams p) {
   }
 #pragma unroll
   for (int t = 0; t < kConvRows; ++t) next[t] = t0 + t < t1 ? ld4(in + (int64_t)(t0 + t) * p.ld_in) : zero;
+  if (t0 == 0) {
+    f32x4 last[Kt];  // the input at offset ql - Kt + j, for a shorter step an entry of the old tail (ql + j)
+#pragma unroll
+    for (int j = 0; j < Kt; ++j) {
+      const int i = ql - Kt + j;
+      last[j] = i >= 0 ? ld4(in + (int64_t)i * p.ld_in) + ib : (ql + j == 1 ? x[1] : x[2]);
+    }
+#pragma unroll
+    for (int j = 0; j < Kt; ++j) st4(tail + (int64_t)j * p.C, last[j]);
+  }
 #pragma unroll
   for (int t = 0; t < kConvRows; ++t) {
     if (t0 + t >= t1) break;
@@ -129,9 +140,15 @@ __global__ __launch_bounds__(256) void conv_tail_kernel(ConvStateParams p) {
   }
 }
 
+// (a, b) of S = a S + b: a = exp(-c sigmoid(g_r) softplus(lam)), b = sqrt(1 - a^2) sigmoid(g_i) u
+DEV void lru_coeff(float gr, float gi, float u, float c, float sp, float& a, float& b) {
+  const float log_a = -c * sigmoidf(gr) * sp;
+  a = expf(log_a);
+  b = sqrtf(-expm1f(2.0f * log_a)) * sigmoidf(gi) * u;  // sqrt(1 - a^2) without cancellation near a = 1
+}
+
 // Everything of the recurrence that does not depend on the state, for every row at once: the gates' pre-activations
-// [recurrence gate | input gate] of each block are overwritten with (a, b) of S = a S + b:
-// a = exp(-c sigmoid(g_r) softplus(lam)), b = sqrt(1 - a^2) sigmoid(g_i) u.
+// [recurrence gate | input gate] of each block are overwritten with (a, b) of S = a S + b.
 // R rows per thread: their loads are in flight together and the channel's softplus is made once (3000 rows of 4096: 80 ->
 // 53 us, some 100 vector instructions per element)
 template <typename T, int R>
@@ -155,10 +172,10 @@ __global__ __launch_bounds__(256) void lru_coeff_kernel(LruScanParams p, int row
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     if (i >= n) break;
-    const float log_a = -p.c * sigmoidf(gr[i]) * sp;
-    g[(int64_t)i * 2 * p.C] = expf(log_a);
-    // sqrt(1 - a^2) without cancellation near a = 1
-    g[(int64_t)i * 2 * p.C + p.bw] = sqrtf(-expm1f(2.0f * log_a)) * sigmoidf(gi[i]) * ui[i];
+    float a, bb;
+    lru_coeff(gr[i], gi[i], ui[i], p.c, sp, a, bb);
+    g[(int64_t)i * 2 * p.C] = a;
+    g[(int64_t)i * 2 * p.C + p.bw] = bb;
   }
 }
 
@@ -198,32 +215,91 @@ __global__ __launch_bounds__(256) void lru_scan_kernel(LruScanParams p) {
   *st = S;
 }
 
+// A step that is all of u's rows and few per sequence (decode): coefficients and walk in one launch, the gates stay as they are
+// (one row each of 160 sequences x 2560 channels: 20.1 us in four launches, 6.4 in this one; 16 sequences 9.0 in two, 4.7)
+template <typename T>
+__global__ __launch_bounds__(256) void lru_step_kernel(LruScanParams p) {
+  const int seq = blockIdx.y;
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ql = p.q_len[seq];
+  if (c >= p.C || ql <= 0) return;
+  const int row0 = p.q_start[seq];
+  float* st = p.state + (int64_t)p.state_slot[seq] * p.C + c;
+  const int b = c / p.bw, o = c % p.bw;
+  const float* g = p.gates + (int64_t)row0 * 2 * p.C + (int64_t)b * 2 * p.bw + o;
+  const float* u = p.u + (int64_t)row0 * p.C + c;
+  const float* y = p.y + (int64_t)row0 * p.C + c;
+  T* out = reinterpret_cast<T*>(p.out) + (int64_t)row0 * p.C + c;
+  float S = p.ctx_len[seq] - ql == 0 ? 0.0f : *st;
+  const float yb = p.y_bias ? (float)reinterpret_cast<const T*>(p.y_bias)[c] : 0.0f;
+  const float sp = softplusf((float)reinterpret_cast<const T*>(p.lam)[c]);
+  for (int t = 0; t < ql; ++t) {
+    float a, bb;
+    lru_coeff(g[(int64_t)t * 2 * p.C], g[(int64_t)t * 2 * p.C + p.bw], u[(int64_t)t * p.C], p.c, sp, a, bb);
+    S = a * S + bb;
+    out[(int64_t)t * p.C] = (T)(S * gelu_tanh_f(y[(int64_t)t * p.C] + yb));
+  }
+  *st = S;
+}
+
 // Prompt portions: the walk in three phases so that no thread takes more than ~3 x 32 dependent steps.  A chunk is
 // kScanRows rows of one sequence; its scratch slot is (first row) / kScanRows + (sequence index), which is unique because
 // sequences are packed in row order.
-//   1. per chunk, in parallel: A = prod a_t and B = the chunk's walk from S = 0          (S_end = A S_in + B)
+//   1. per chunk, in parallel: A = prod a_t and B = the chunk's walk from S = 0          (S_end = A S_in + B); a call that holds
+//      all rows makes the coefficients here, for one reading of the gates
 //   2. per sequence: the chunks in order -- each chunk's incoming state replaces its B, the last one is the slot's state
 //   3. per chunk, in parallel: the walk from the incoming state, times gelu(branch + bias)
+// A few chunks (kFoldChunks) take no second phase: the first leaves (S_in, S_end) of a sequence's first chunk, and every thread of
+// the third folds the chunks before its own.  Rows go in batches whose loads are in flight together.  Per layer (coefficients
+// and walk), four launches before / now: 200 rows of 2560 35 / 24 us, 700 42 / 30, 3000 rows of 4096 127 / 105.
 constexpr int kScanRows = 32;
 constexpr int kChunkedFrom = 128;  // rows of a step from which the walk is chunked (below: one thread per sequence)
 
 DEV int scan_slot(int row0, int t0, int seq) { return (row0 + t0) / kScanRows + seq; }
 
-__global__ __launch_bounds__(256) void lru_chunk_reduce_kernel(LruScanParams p) {
+constexpr int kScanBatch = 8;    // rows whose loads are in flight together
+constexpr int kFoldChunks = 32;  // chunks of a step up to which the third phase folds
+
+template <typename T, bool COEFF>
+__global__ __launch_bounds__(256) void lru_chunk_reduce_kernel(LruScanParams p, int fold) {
   const int seq = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
   const int ql = p.q_len[seq], t0 = blockIdx.z * kScanRows;
   if (c >= p.C || t0 >= ql) return;
   const int t1 = t0 + kScanRows < ql ? t0 + kScanRows : ql;
   const int row0 = p.q_start[seq];
   const int b = c / p.bw, o = c % p.bw;
-  const float* ab = p.gates + (int64_t)row0 * 2 * p.C + (int64_t)b * 2 * p.bw + o;
+  float* ab = const_cast<float*>(p.gates) + (int64_t)row0 * 2 * p.C + (int64_t)b * 2 * p.bw + o;
+  const float* u = p.u + (int64_t)row0 * p.C + c;
+  const float sp = COEFF ? softplusf((float)reinterpret_cast<const T*>(p.lam)[c]) : 0.0f;
   float A = 1.0f, B = 0.0f;
-  for (int t = t0; t < t1; ++t) {
-    const float a = ab[(int64_t)t * 2 * p.C];
-    B = a * B + ab[(int64_t)t * 2 * p.C + p.bw];
-    A *= a;
+  for (int t = t0; t < t1; t += kScanBatch) {
+    float ga[kScanBatch], gb[kScanBatch], ui[kScanBatch];
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      const int64_t at = t + i < t1 ? t + i : t;
+      ga[i] = ab[at * 2 * p.C];
+      gb[i] = ab[at * 2 * p.C + p.bw];
+      if (COEFF) ui[i] = u[at * p.C];
+    }
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      if (t + i >= t1) break;
+      float a = ga[i], bb = gb[i];
+      if (COEFF) {
+        lru_coeff(ga[i], gb[i], ui[i], p.c, sp, a, bb);
+        ab[(int64_t)(t + i) * 2 * p.C] = a;
+        ab[(int64_t)(t + i) * 2 * p.C + p.bw] = bb;
+      }
+      B = a * B + bb;
+      A *= a;
+    }
   }
   const int64_t s = (int64_t)scan_slot(row0, t0, seq) * p.C + c;
+  if (fold && t0 == 0) {
+    const float S = p.ctx_len[seq] - ql == 0 ? 0.0f : p.state[(int64_t)p.state_slot[seq] * p.C + c];
+    B = A * S + B;
+    A = S;
+  }
   p.chunk_a[s] = A;
   p.chunk_b[s] = B;
 }
@@ -232,20 +308,30 @@ __global__ __launch_bounds__(256) void lru_chunk_carry_kernel(LruScanParams p) {
   const int seq = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
   const int ql = p.q_len[seq];
   if (c >= p.C || ql <= 0) return;
-  const int row0 = p.q_start[seq];
+  const int row0 = p.q_start[seq], chunks = (ql + kScanRows - 1) / kScanRows;
   float* st = p.state + (int64_t)p.state_slot[seq] * p.C + c;
   float S = p.ctx_len[seq] - ql == 0 ? 0.0f : *st;
-  for (int t0 = 0; t0 < ql; t0 += kScanRows) {
-    const int64_t s = (int64_t)scan_slot(row0, t0, seq) * p.C + c;
-    const float next = p.chunk_a[s] * S + p.chunk_b[s];
-    p.chunk_b[s] = S;  // the chunk's incoming state
-    S = next;
+  const int64_t s0 = (int64_t)scan_slot(row0, 0, seq) * p.C + c;  // a sequence's slots follow each other
+  for (int k = 0; k < chunks; k += kScanBatch) {
+    float a[kScanBatch], bb[kScanBatch];
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      const int64_t s = s0 + (int64_t)(k + i < chunks ? k + i : k) * p.C;
+      a[i] = p.chunk_a[s];
+      bb[i] = p.chunk_b[s];
+    }
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      if (k + i >= chunks) break;
+      p.chunk_b[s0 + (int64_t)(k + i) * p.C] = S;  // the chunk's incoming state
+      S = a[i] * S + bb[i];
+    }
   }
   *st = S;
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void lru_chunk_apply_kernel(LruScanParams p) {
+__global__ __launch_bounds__(256) void lru_chunk_apply_kernel(LruScanParams p, int fold) {
   const int seq = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
   const int ql = p.q_len[seq], t0 = blockIdx.z * kScanRows;
   if (c >= p.C || t0 >= ql) return;
@@ -256,11 +342,35 @@ __global__ __launch_bounds__(256) void lru_chunk_apply_kernel(LruScanParams p) {
   const float* ab = p.gates + (int64_t)row0 * 2 * p.C + (int64_t)b * 2 * p.bw + o;
   const float* y = p.y + (int64_t)row0 * p.C + c;
   T* out = reinterpret_cast<T*>(p.out) + (int64_t)row0 * p.C + c;
-  float S = p.chunk_b[(int64_t)scan_slot(row0, t0, seq) * p.C + c];
-  for (int t = t0; t < t1; ++t) {
-    S = ab[(int64_t)t * 2 * p.C] * S + ab[(int64_t)t * 2 * p.C + p.bw];
-    out[(int64_t)t * p.C] = (T)(S * gelu_tanh_f(y[(int64_t)t * p.C] + yb));
+  const int64_t s0 = (int64_t)scan_slot(row0, 0, seq) * p.C + c;
+  const int chunk = blockIdx.z;
+  float S;
+  if (!fold) {
+    S = p.chunk_b[s0 + (int64_t)chunk * p.C];
+  } else if (chunk == 0) {
+    S = p.chunk_a[s0];
+  } else {
+    S = p.chunk_b[s0];
+#pragma unroll 8
+    for (int k = 1; k < chunk; ++k) S = p.chunk_a[s0 + (int64_t)k * p.C] * S + p.chunk_b[s0 + (int64_t)k * p.C];
   }
+  for (int t = t0; t < t1; t += kScanBatch) {
+    float a[kScanBatch], bb[kScanBatch], yy[kScanBatch];
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      const int64_t at = t + i < t1 ? t + i : t;
+      a[i] = ab[at * 2 * p.C];
+      bb[i] = ab[at * 2 * p.C + p.bw];
+      yy[i] = y[at * p.C];
+    }
+#pragma unroll
+    for (int i = 0; i < kScanBatch; ++i) {
+      if (t + i >= t1) break;
+      S = a[i] * S + bb[i];
+      out[(int64_t)(t + i) * p.C] = (T)(S * gelu_tanh_f(yy[i] + yb));
+    }
+  }
+  if (fold && t1 == ql) p.state[(int64_t)p.state_slot[seq] * p.C + c] = S;
 }
 
 }  // namespace
@@ -277,8 +387,6 @@ extern "C" hipError_t dsse_conv_state(const dsse::ConvStateParams* p, hipStream_
   if (four) {
     if (p->f32) hipLaunchKernelGGL(dsse::conv_state4_kernel<float>, fgrid, dim3(256), 0, st, *p);
     else hipLaunchKernelGGL(dsse::conv_state4_kernel<bf16>, fgrid, dim3(256), 0, st, *p);
-    if (p->f32) hipLaunchKernelGGL(dsse::conv_tail_kernel<float>, tgrid, dim3(256), 0, st, *p);
-    else hipLaunchKernelGGL(dsse::conv_tail_kernel<bf16>, tgrid, dim3(256), 0, st, *p);
   } else if (p->f32) {
     hipLaunchKernelGGL(dsse::conv_state_kernel<float>, grid, dim3(256), 0, st, *p);
     if (tails) hipLaunchKernelGGL(dsse::conv_tail_kernel<float>, tgrid, dim3(256), 0, st, *p);
@@ -290,25 +398,36 @@ extern "C" hipError_t dsse_conv_state(const dsse::ConvStateParams* p, hipStream_
 }
 
 extern "C" hipError_t dsse_lru_scan(const dsse::LruScanParams* p, hipStream_t st) {
+  using namespace dsse;
   if (p->nseq <= 0 || p->rows <= 0) return hipSuccess;
   dim3 grid((p->C + 255) / 256, p->nseq);
-  if (p->coeff) {
-    const int per = p->rows >= 256 ? 4 : 1;  // few rows: a thread per element fills more of the chip
-    dim3 cgrid((p->rows + per - 1) / per, (p->C + 255) / 256);
-    if (p->f32 && per == 4) hipLaunchKernelGGL((dsse::lru_coeff_kernel<float, 4>), cgrid, dim3(256), 0, st, *p, p->rows);
-    else if (p->f32) hipLaunchKernelGGL((dsse::lru_coeff_kernel<float, 1>), cgrid, dim3(256), 0, st, *p, p->rows);
-    else if (per == 4) hipLaunchKernelGGL((dsse::lru_coeff_kernel<bf16, 4>), cgrid, dim3(256), 0, st, *p, p->rows);
-    else hipLaunchKernelGGL((dsse::lru_coeff_kernel<bf16, 1>), cgrid, dim3(256), 0, st, *p, p->rows);
-  }
-  if (p->chunk_a && p->chunk_b && p->rows >= dsse::kChunkedFrom) {  // prompt portions: the three-phase walk
-    dim3 zgrid((p->C + 255) / 256, p->nseq, (p->rows + dsse::kScanRows - 1) / dsse::kScanRows);
-    hipLaunchKernelGGL(dsse::lru_chunk_reduce_kernel, zgrid, dim3(256), 0, st, *p);
-    hipLaunchKernelGGL(dsse::lru_chunk_carry_kernel, grid, dim3(256), 0, st, *p);
-    if (p->f32) hipLaunchKernelGGL(dsse::lru_chunk_apply_kernel<float>, zgrid, dim3(256), 0, st, *p);
-    else hipLaunchKernelGGL(dsse::lru_chunk_apply_kernel<bf16>, zgrid, dim3(256), 0, st, *p);
+  const bool alone = p->coeff && p->alone;
+  if (alone && p->rows <= 4 * p->nseq) {
+    if (p->f32) hipLaunchKernelGGL(lru_step_kernel<float>, grid, dim3(256), 0, st, *p);
+    else hipLaunchKernelGGL(lru_step_kernel<bf16>, grid, dim3(256), 0, st, *p);
     return hipGetLastError();
   }
-  if (p->f32) hipLaunchKernelGGL(dsse::lru_scan_kernel<float>, grid, dim3(256), 0, st, *p);
-  else hipLaunchKernelGGL(dsse::lru_scan_kernel<bf16>, grid, dim3(256), 0, st, *p);
+  const bool chunked = p->chunk_a && p->chunk_b && p->rows >= kChunkedFrom;  // prompt portions
+  if (p->coeff && !(alone && chunked)) {
+    const int per = p->rows >= 256 ? 4 : 1;  // few rows: a thread per element fills more of the chip
+    dim3 cgrid((p->rows + per - 1) / per, (p->C + 255) / 256);
+    if (p->f32 && per == 4) hipLaunchKernelGGL((lru_coeff_kernel<float, 4>), cgrid, dim3(256), 0, st, *p, p->rows);
+    else if (p->f32) hipLaunchKernelGGL((lru_coeff_kernel<float, 1>), cgrid, dim3(256), 0, st, *p, p->rows);
+    else if (per == 4) hipLaunchKernelGGL((lru_coeff_kernel<bf16, 4>), cgrid, dim3(256), 0, st, *p, p->rows);
+    else hipLaunchKernelGGL((lru_coeff_kernel<bf16, 1>), cgrid, dim3(256), 0, st, *p, p->rows);
+  }
+  if (chunked) {
+    dim3 zgrid((p->C + 255) / 256, p->nseq, (p->rows + kScanRows - 1) / kScanRows);
+    const int fold = (int)zgrid.z <= kFoldChunks;
+    if (!alone) hipLaunchKernelGGL((lru_chunk_reduce_kernel<float, false>), zgrid, dim3(256), 0, st, *p, fold);
+    else if (p->f32) hipLaunchKernelGGL((lru_chunk_reduce_kernel<float, true>), zgrid, dim3(256), 0, st, *p, fold);
+    else hipLaunchKernelGGL((lru_chunk_reduce_kernel<bf16, true>), zgrid, dim3(256), 0, st, *p, fold);
+    if (!fold) hipLaunchKernelGGL(lru_chunk_carry_kernel, grid, dim3(256), 0, st, *p);
+    if (p->f32) hipLaunchKernelGGL(lru_chunk_apply_kernel<float>, zgrid, dim3(256), 0, st, *p, fold);
+    else hipLaunchKernelGGL(lru_chunk_apply_kernel<bf16>, zgrid, dim3(256), 0, st, *p, fold);
+    return hipGetLastError();
+  }
+  if (p->f32) hipLaunchKernelGGL(lru_scan_kernel<float>, grid, dim3(256), 0, st, *p);
+  else hipLaunchKernelGGL(lru_scan_kernel<bf16>, grid, dim3(256), 0, st, *p);
   return hipGetLastError();
 }

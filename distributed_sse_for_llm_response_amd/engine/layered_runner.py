@@ -360,7 +360,7 @@ class LayeredRunner(RunnerBase):
                 slots = M // 32 + g["ql"].numel() + 1
                 scr = scr[:2 * slots * C].view(2, slots, C)
             ops.lru_scan(u, gates, yr, Lw.lam, self.state.state[li], g["qs"], g["ql"], g["ctx"], g["ss"], hs,
-                         LRU_DECAY_SCALE, Lw.y_b, i == 0, scr)
+                         LRU_DECAY_SCALE, Lw.y_b, i == 0, scr, len(groups) == 1)
         self._lin(hs, Lw.o, Lw.o_t, d["y"])
 
     def _moe(self, f, Fw, M: int, d: dict):
@@ -371,9 +371,9 @@ class LayeredRunner(RunnerBase):
         o = d["mo_o"][:M * S * self.cfg.width].view(M * S, self.cfg.width)
         z = d["mo_z"][:M * f.experts].view(M, f.experts)
         ops.gemm_rm(d["xb"], Fw.router, z, bias=Fw.router_b)  # fp32 logits
-        ops.moe_topk(z, tki, tkw)
+        aligned = ops.moe_topk_lists(z, tki, tkw, d["mo_sorted"], d["mo_tile"], d["mo_n"], bool(f.shared_ff))
         ops.moe_grouped(d["xb"], tki, tkw, Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown, d["mo_sorted"],
-                        d["mo_tile"], d["mo_n"], d["mo_h"], o)
+                        d["mo_tile"], d["mo_n"], d["mo_h"], o, aligned=aligned)
         return o, S
 
     def _layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None = None, prev=None) -> None:

@@ -111,14 +111,15 @@ def conv_state(inp, taps, bias, tail, q_start, q_len, ctx_len, state_slot, out, 
 
 
 def lru_scan(u, gates, y, lam, state, q_start, q_len, ctx_len, state_slot, out, c: float, y_bias=None,
-             coeff: bool = True, scratch=None):
+             coeff: bool = True, scratch=None, alone: bool = False):
     """Real-gated linear recurrence continued from each sequence's slot state; out = state · gelu(y + y_bias).
     coeff: turn the gate pre-activations of ALL rows into the recurrence's coefficients first (in place); pass False
     for a further sequence group of the same step.  scratch (fp32 [2, rows / 32 + sequences + 1, C]): steps of 128 rows
-    or more walk in three phases over 32-row chunks instead of one thread per sequence and channel."""
+    or more walk in three phases over 32-row chunks instead of one thread per sequence and channel.  alone (with coeff):
+    the sequences hold all rows of u, so the coefficients are made where they are used and gates may keep either."""
     if _hip(u):
         torch.ops.dsse.lru_scan(u, gates, y, lam, state, q_start, q_len, ctx_len, state_slot, out, c, y_bias, coeff,
-                                scratch)
+                                scratch, alone)
     else:
         lref.lru_scan(u, gates, y, lam, state, q_start, q_len, ctx_len, state_slot, out, c, y_bias, coeff)
 
@@ -129,6 +130,14 @@ def moe_topk(logits, topk_idx, topk_w):
         torch.ops.dsse.moe_topk(logits, topk_idx, topk_w)
     else:
         lref.moe_topk(logits, topk_idx, topk_w)
+
+
+def moe_topk_lists(logits, topk_idx, topk_w, sorted_ids, tile_expert, num_tiles, shared: bool) -> bool:
+    """moe_topk, and in a decode-sized step the work list of moe_grouped in the same launch: returns moe_grouped's aligned."""
+    if _hip(logits) and torch.ops.dsse.moe_topk_lists(logits, topk_idx, topk_w, sorted_ids, tile_expert, num_tiles, shared):
+        return True
+    moe_topk(logits, topk_idx, topk_w)
+    return False
 
 
 def moe_router(x, w, b, topk_idx, topk_w):
