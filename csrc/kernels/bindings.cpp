@@ -98,11 +98,30 @@ void refresh_env() { g_env_gen.fetch_add(1, std::memory_order_acq_rel); }
 
 // Tile selection for the skinny GEMM.  NT = output tiles per wave, KW = waves splitting K.
 // Defaults come from the gfx950 sweep in tools/tune_gemm.py; DSSE_KERNEL_CFG gemm_nt / gemm_kw override.
+//
+// 8 to 16 rows take two column tiles per wave -- every X fragment, a request of 64 lines, feeds two products -- where N / 32
+// workgroups end in a full or well filled round.  One tile / two, 16 rows, us: 6144 x 4096 16.2 / 13.9, 8192 x 4096 18.1 / 15.9, 5248 x
+// 4096 16.1 / 13.9, 14464 x 4096 28.4 / 25.3, 16384 x 2048 16.6 / 15.2, 16384 x 4096 (gemm_stream 29.2) 25.3, 32768 x 2048 28.2 / 24.9,
+// 32768 x 4096 (gemm_stream 47.9) 44.8; 8 rows, 6144 x 4096 13.7 / 12.6; but 10240 x 4096 (320 workgroups) 21.6 / 22.6, 8320 x 2048 (260)
+// 13.1 / 13.6, 26752 x 4096 (836) 41.6 / 42.6.
+bool skinny_pairs(int M, int N) {
+  if (M < 8 || M > 16 || N % 32) return false;
+  const int wgs = N / 32, rem = wgs % 256;
+  return wgs >= 160 && (rem == 0 || rem >= 160);
+}
+// 17 to 64 rows in one launch of the skinny kernel, where a sliced product and its reduction are two latency-sized ones: up to 256
+// workgroups and K walks of at most two rounds.  Sliced / skinny, us: 2048 x 2048 17 rows 9.8 / 7.7, 32 rows 10.7 / 9.3, 48 rows 10.6 /
+// 11.9; 4096 x 2048 17 rows 10.8 / 8.1, 32 11.4 / 9.7; 2048 x 2560 32 rows 10.8 / 10.7; 2048 x 4096 24 rows 11.8 / 12.3; 2048 x 1024 64
+// rows 10.1 / 9.3; 6144 x 2048 24 rows 12.3 / 12.6.  K % 512 != 0 (a tensor-parallel shard's) stays with the ring kernel.
+bool skinny_whole(int M, int N, int K) {
+  return M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
+}
+
 void pick_tiles(int M, int N, int K, int mode, int& mt, int& nt, int& kw) {
   mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  nt = 1;
+  nt = skinny_pairs(M, N) ? 2 : 1;
   const int chunks = K / 128;
-  kw = chunks >= 32 ? 8 : 4;
+  kw = nt == 2 ? 4 : (chunks >= 32 || (mt == 2 && chunks >= 8) ? 8 : 4);
   const int e_nt = env_int("gemm_nt", 0), e_kw = env_int("gemm_kw", 0);
   if (e_nt) nt = e_nt;
   if (e_kw) kw = e_kw;
@@ -510,7 +529,8 @@ int gemm_impl(int M, int N, int K) {
     return impl == 1 ? fallback : impl;
   }
   if (M <= 8) return 0;
-  if (M <= 16 && N < 16384) return 0;
+  if (M <= 16 && (N < 16384 || skinny_pairs(M, N))) return 0;
+  if (skinny_whole(M, N, K)) return 0;
   return pick_stream(M, N, K).ok ? 2 : fallback;
 }
 
