@@ -120,12 +120,12 @@ struct MatrixScanParams {
 
 // Workspace floats of the chunked form (matrix_chunk.hip) for `rows` rows, of them `longest` in the longest sequence (0 = not
 // known); 0 where the walk by tokens is taken: by its time, and for shapes that the chunks do not take.  They take key widths
-// 32, 64 and 128, whole 16-column tiles of values, decays that do not differ between key channels, 16-byte-aligned rows.
+// 32, 64 and 128, whole 16-column tiles of values, 16-byte-aligned rows.
 // `longest` only chooses the form and the room: sequences that it leaves no room for are walked.
 int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest);
 
 // Whether such rows are better walked in two levels (matrix_scan_chunked) than by either form of matrix_scan: the one decision
-// between the three.  Reads the shapes, strides and alignment of q, k and v.
+// between the three.  Reads the shapes, strides and alignment of q, k, v and the decays per key channel.
 bool scan_two_levels(const MatrixScanParams& p, int rows, int64_t longest);
 
 // The carry between the two passes of the two-level walk: per sequence, the incoming state of each of its chunks.

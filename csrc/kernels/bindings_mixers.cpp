@@ -367,13 +367,19 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
 }
 
+// decay: the decays where the caller has them, [T, H, D] when channels; without them decays per channel count as unaligned
 bool matrix_scan_two_levels(const Tensor& q, const Tensor& k, const Tensor& v, bool channels, int64_t rows, int64_t nseq,
-                            int64_t longest) {
+                            int64_t longest, const OptTensor& decay) {
   dsse::MatrixScanParams p{};
   p.H = (int)v.size(1), p.V = (int)v.size(2), p.G = (int)k.size(1), p.D = (int)k.size(2), p.nseq = (int)nseq;
   p.q = q.data_ptr<float>(), p.k = k.data_ptr<float>(), p.v = v.data_ptr<float>();
   p.ldq = (int)q.stride(0), p.ldk = (int)k.stride(0), p.ldv = (int)v.stride(0);
   p.decay_kind = channels ? 3 : 1;
+  p.ldd = 1;
+  if (channels && decay.has_value()) {
+    TORCH_CHECK(decay->dim() == 3 && decay->scalar_type() == at::kFloat, "decay [T, H, D], float32");
+    p.decay = decay->data_ptr<float>(), p.ldd = (int)decay->stride(0);
+  }
   return dsse::scan_two_levels(p, (int)rows, longest);
 }
 
@@ -828,7 +834,8 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
         "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
-  m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest) -> bool");
+  m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest, "
+        "Tensor? decay=None) -> bool");
   m.def("matrix_scan_chunked(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor(a!) state, Tensor q_len, Tensor ctx_len, "
         "Tensor state_slot, Tensor s_first, Tensor s_count, Tensor cmeta, Tensor(b!) scratch, Tensor(c!)? a_scratch, "
         "Tensor(d!) out, float q_scale=1.0) -> ()");

@@ -1,31 +1,39 @@
-// Matrix-state recurrences of prompt portions in chunks of 64 tokens on the fp32 matrix cores: decays that are one number per
-// head (or per token and head, or none), with or without the delta rule.
+// Matrix-state recurrences of prompt portions in chunks of 16 tokens on the fp32 matrix cores: with or without the delta rule, under
+// decays that are one number per head, per token and head, or per token, head and key channel (or none).
 //
-// What bounds it: the chain from chunk to chunk.  The token walk (matrix_scan.hip) spends some 75 vector instructions per
-// token and wave, 0.46 us per token of a sequence; a chunk of 64 tokens is five small products here, 6.4 us with the delta
-// rule and 4.4 us without.  2048 tokens, 16 heads, 128 x 128: 946 -> 221 us and 919 -> 150 us; prompts of 582, 352 and 566
-// tokens 281 -> 140 us and 268 -> 87 us (two-level walk of matrix_scan_chunked: some 220 us).  With A_t the
-// product of the decays up to token t of the chunk, R[t][i] = A_t / A_i (formed as the product of the decays between them, so
-// a decay of zero is no division), S the incoming state and u_i the written values,
+// What bounds it: the chain from chunk to chunk.  The token walk (matrix_scan.hip) spends some 75 vector instructions per token and
+// wave, 0.46 us per token of a sequence.  A chunk of 16 is 29 products of 16 x 16 x 4 per wave with the delta rule and 17 without,
+// 0.42 and 0.25 us of matrix time, and takes 1.1 and 0.63 us (key width 128): the rest is LDS, the barrier and dependent products.
+// With P[t][i] the product of the decays after token i up to token t (P[t][-1]: from the chunk's start), per key channel, S the
+// incoming state and u_i the written values, all products with P elementwise along the key width,
 //
-//     S_t  = A_t S + sum_{i <= t} R[t][i] k_i u_i^T
-//     u    = T (v - A (K S)),  T = (1 + L)^-1 diag(beta),  L[t][i] = beta_t R[t][i] k_t . k_i  for i < t   (delta rule)
-//     u    = v                                                                                              (without)
-//     o    = A (Q S) + M u,    M[t][i] = R[t][i] q_t . k_i  for i <= t
-//     S'   = A_C S + K^T (E u),  E_i = R[C - 1][i]
+//     W    = (K P[.][-1]) S,   u = T (v - W),   T = (1 + L)^-1 diag(beta),  L[t][i] = beta_t k_t . (P[t][i] k_i) for i < t   (delta rule)
+//     u    = v                                                                                                         (without)
+//     o    = (Q P[.][-1]) S + M u,   M[t][i] = q_t . (P[t][i] k_i)  for i <= t
+//     S'   = P[15][-1] S + (K P[15][.])^T u
 //
-// (the chunkwise form of the delta rule: Yang et al., "Parallelizing Linear Transformers with the Delta Rule over Sequence
-// Length", 2024)
+// (the chunkwise form of the delta rule: Yang et al., "Parallelizing Linear Transformers with the Delta Rule over Sequence Length",
+// 2024).  Every P is formed as the product of the decays between the two tokens, so a decay of zero is no division; a chunk no longer
+// than a tile of the matrix cores is what makes that affordable per key channel.
 //
-// Two launches: T, M, A and E depend on the inputs alone and are made for all chunks at once; the second walks the chunks of
-// a (sequence, head, 16 value columns).  All products are v_mfma_f32_16x16x4_f32, 32-bit like the walk.  The accumulator
-// layout (rows 4 g + i of column r) IS the B operand of a product whose k index runs 4 g + i over i, so the state, the
-// written values and their scaled copy go from one product to the next without a change of layout; they meet between the four
-// waves (16 tokens and D / 4 state rows each) in LDS.  The next chunk's operands are in registers a whole chunk ahead.
+// Two launches: the scaled rows, T, M and the chunk's decay depend on the inputs alone and are made for all chunks at once, laid out
+// as operands; the second walks the chunks of a (sequence, head, 16 or 32 value columns), each of its waves holding D / 4 state rows.
+// All products are v_mfma_f32_16x16x4_f32, 32-bit like the walk.  The accumulator layout (rows 4 g + i of column r) IS the B operand
+// of a product whose k index runs 4 g + i over i, so the state and the written values go from one product to the next without a
+// change of layout; only the waves' shares of W and o meet in LDS, those of o behind the next chunk's products.
+//
+// Measured, us, key and value width 128 (before: chunks of 64 tokens for decays per head, two parallel token walks per key channel):
+// delta rule, 16 heads: prompts of 582, 352 and 566 tokens 140 -> 81, one of 2048 217 -> 147, of 200 58 -> 25; retention 87 -> 54,
+// 146 -> 89, 30 -> 16; decays per channel, 8 heads: 146 -> 39, 210 -> 88, one of 200 (token walk) 74 -> 19.  Error of the outputs
+// against 64 bits, root mean square: 1.1e-7 with the delta rule (walk 1.0e-7, chunks of 64 1.2e-7 .. 1.4e-7), 2.7e-7 under decays near
+// one (walk 3.2e-7, chunks of 64 2.3e-7 .. 3.2e-7), 1.3e-7 per channel (walk and two walks 1.3e-7).
 //
 // A chunk's products run over its later tokens with weights of zero, so a token that is not finite would make the outputs of its
 // whole chunk NaN.  Where an output is not finite, the sequence's columns are walked once more token by token (walk_tokens): such
 // a token reaches the tokens after it and none before it.  The same walk serves sequences that the launch has no chunks for.
+//
+// The workspace is 17 (25) KB per chunk and head at width 128; past kRoom the launch goes by segments of every sequence, which meet in
+// the state entries.
 #include <algorithm>
 #include <climits>
 
@@ -34,20 +42,30 @@
 namespace dsse {
 namespace {
 
-constexpr int kC = 64;         // tokens per chunk
+constexpr int kC = 16;         // tokens per chunk: a tile of the matrix cores
 constexpr int kTwoLevelRows = 256;  // rows of a launch from which the two-level walk pays
-constexpr int kScanCols = 16;  // value columns per workgroup: a tile of the state entry (matrix_scan.hip)
+constexpr int kScanCols = 16;  // value columns of a tile of the state entry (matrix_scan.hip)
+constexpr int64_t kRoom = int64_t{1} << 26;   // workspace floats of a segment: 268 MB
+constexpr int64_t kMostRows = int64_t{1} << 22;  // rows x heads
 
-// floats of one (chunk, head): M | A | E | T
-constexpr int kUnitA = kC * kC, kUnitE = kUnitA + kC, kUnitT = kUnitE + kC;
-DEV int64_t unit_floats(bool delta) { return delta ? kUnitT + kC * kC : kUnitT; }
+// floats of one (chunk, head): Q' | K^ | (K') | M | (T) | A; the first three as tiles of 16 key channels
+__host__ __device__ constexpr int unit_floats(int D, bool delta) {
+  return (delta ? 3 : 2) * kC * D + (delta ? 2 : 1) * kC * kC + D;
+}
 
+// The launch's part of each sequence: its chunks [c0, c0 + span)
+struct Segment {
+  int c0, span;
+};
+DEV int chunks_of(int ql, Segment sg) {
+  const int n = ql > 0 ? (ql + kC - 1) / kC - sg.c0 : 0;
+  return n < 0 ? 0 : (n < sg.span ? n : sg.span);
+}
 // chunks of the sequences before `seq` (wave-uniform; every lane calls it)
-DEV int chunks_before(const int* q_len, int seq, int lane) {
+DEV int chunks_before(const int* q_len, int seq, int lane, Segment sg) {
   int sum = 0;
   for (int s0 = 0; s0 < seq; s0 += 64) {
-    const int n = s0 + lane < seq ? q_len[s0 + lane] : 0;
-    int c = n > 0 ? (n + kC - 1) / kC : 0;
+    int c = s0 + lane < seq ? chunks_of(q_len[s0 + lane], sg) : 0;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o);
     sum += c;
@@ -55,30 +73,39 @@ DEV int chunks_before(const int* q_len, int seq, int lane) {
   return __builtin_amdgcn_readfirstlane(sum);
 }
 
-// rows of four consecutive floats at p + row * ld, zero past the end
-DEV f32x4 row4(const float* p, int64_t ld, int row, int rows) {
-  const f32x4 v = ld_global<f32x4>(p + (int64_t)(row < rows ? row : 0) * ld);
-  return row < rows ? v : f32x4{0.f, 0.f, 0.f, 0.f};
+template <int CTRL>
+DEV float row_rotated(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+DEV float row16_sum(float v) {
+  v += row_rotated<0x128>(v);
+  v += row_rotated<0x124>(v);
+  v += row_rotated<0x122>(v);
+  v += row_rotated<0x121>(v);
+  return v;
 }
 
-// Sums over the key width in kSums parts, added pairwise: a chain of 32 dependent products would round more than the token
-// walk's tree over the lanes does.  Error of a layer's outputs against 64 bits, root mean square: 1.2e-7..1.4e-7 here and
-// 1.0e-7..1.4e-7 in the walk; 2.3e-7 and 3.2e-7 where decays stay near one; of whole fp32 models 1.2e-6 and 1.3e-6.
-constexpr int kSums = 8;
-DEV f32x4 total(const f32x4 (&s)[4]) { return (s[0] + s[1]) + (s[2] + s[3]); }
-DEV f32x4 total(const f32x4 (&s)[kSums]) { return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])); }
+template <int N, typename T>
+DEV T pairwise(const T* x) {
+  if constexpr (N == 1) return x[0];
+  else return pairwise<N / 2>(x) + pairwise<N / 2>(x + N / 2);
+}
 
-template <int NT, bool DELTA>
-__global__ __launch_bounds__(256) void chunk_prepare_kernel(MatrixScanParams p, float* __restrict__ ws) {
-  __shared__ float a_s[kC], b_s[kC], R[kC][kC + 1];
-  __shared__ __align__(16) float Ls[DELTA ? kC : 1][kC + 4];
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+// One (chunk, head): everything that does not depend on the state.  CHAN: the decays differ between key channels.
+template <int NT, bool DELTA, bool CHAN>
+__global__ __launch_bounds__(256) void chunk_prepare_kernel(MatrixScanParams p, float* __restrict__ ws, Segment sg) {
+  constexpr int D = 16 * NT, kPer = NT, kVec = kPer < 4 ? kPer : 4;  // channels per lane of a row of 16 lanes, in vectors
+  using vec = float __attribute__((ext_vector_type(kVec)));
+  constexpr int kRow = D + 4;  // rows start four banks apart
+  __shared__ __align__(16) float qs[kC][kRow], ks[kC][kRow], as[kC][CHAN ? kRow : 1];
+  __shared__ __align__(16) float Ls[DELTA ? kC : 1][kC];
+  __shared__ float bs[kC];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.y;
   // the sequence and the place in it of chunk blockIdx.x
   int seq = -1, c = 0, before = 0;
   for (int s0 = 0; s0 < p.nseq && seq < 0; s0 += 64) {
-    const int n = s0 + lane < p.nseq ? p.q_len[s0 + lane] : 0;
-    const int own = n > 0 ? (n + kC - 1) / kC : 0;
+    const int own = s0 + lane < p.nseq ? chunks_of(p.q_len[s0 + lane], sg) : 0;
     int upto = own;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -95,79 +122,145 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(MatrixScanParams p, 
     before += __builtin_amdgcn_readlane(upto, 63);
   }
   if (seq < 0) return;  // uniform for the workgroup: past the last chunk
-  const int ql = p.q_len[seq], cnt = ql - c * kC < kC ? ql - c * kC : kC;
-  const int64_t row0 = p.q_start[seq] + c * kC;
+  const int first = (sg.c0 + c) * kC, left = p.q_len[seq] - first, cnt = left < kC ? left : kC;
+  const int64_t row0 = p.q_start[seq] + first;
   const int grp = h / (p.H / p.G);
-  float* unit = ws + ((int64_t)blockIdx.x * p.H + h) * unit_floats(DELTA);
-  if (tid < kC) {
-    float a = 1.0f, b = 0.0f;
-    if (tid < cnt) {
-      a = p.decay_kind == 1 ? p.decay[h] : (p.decay_kind == 2 ? p.decay[(row0 + tid) * p.ldd + h] : 1.0f);
-      if (DELTA) b = p.beta[(row0 + tid) * p.ldb + h];
+  float* unit = ws + ((int64_t)blockIdx.x * p.H + h) * unit_floats(D, DELTA);
+  float* uk = unit + kC * D;
+  float* ub = uk + kC * D;
+  float* um = ub + (DELTA ? kC * D : 0);
+  float* ut = um + kC * kC;
+  float* ua = um + (DELTA ? 2 : 1) * kC * kC;
+  // tokens past the sequence's end: no key, no query, no decay
+  for (int i = tid; i < kC * D / 4; i += 256) {
+    const int t = i / (D / 4), d = 4 * (i % (D / 4));
+    const bool on = t < cnt;
+    const int64_t row = row0 + (on ? t : 0);
+    f32x4 q = ld_global<f32x4>(p.q + row * p.ldq + grp * D + d), k = ld_global<f32x4>(p.k + row * p.ldk + grp * D + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = on ? q[e] * p.q_scale : 0.0f, k[e] = on ? k[e] : 0.0f;
+    *reinterpret_cast<f32x4*>(&qs[t][d]) = q;
+    *reinterpret_cast<f32x4*>(&ks[t][d]) = k;
+    if constexpr (CHAN) {
+      f32x4 a = ld_global<f32x4>(p.decay + row * p.ldd + h * D + d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = on ? a[e] : 1.0f;
+      *reinterpret_cast<f32x4*>(&as[t][d]) = a;
     }
-    a_s[tid] = a;
-    b_s[tid] = b;
   }
+  if (!CHAN && tid < kC)
+    as[tid][0] = tid >= cnt || p.decay_kind == 0 ? 1.0f : (p.decay_kind == 1 ? p.decay[h] : p.decay[(row0 + tid) * p.ldd + h]);
+  if (DELTA && tid < kC) bs[tid] = tid < cnt ? p.beta[(row0 + tid) * p.ldb + h] : 0.0f;
   __syncthreads();
-  if (w == 3) {  // the wave with the most products makes them; this wave's column of R first (its products are independent)
-    const float mine = a_s[lane];
-    float v = 0.f;
-#pragma unroll 8
+  auto decay = [&](int t, int d) {
+    if constexpr (CHAN) return *reinterpret_cast<const f32x4*>(&as[t][d]);
+    else return f32x4{as[t][0], as[t][0], as[t][0], as[t][0]};
+  };
+  // the state's view of the tokens: rows times the decays up to them, keys times the decays after them
+  if (w >= 2 && lane < D / 4) {  // the waves with the fewest pairs, or none
+    const int d = 4 * lane, at = d / 16 * (16 * kC) + d % 16;
+    f32x4 a{1.f, 1.f, 1.f, 1.f};
+    if (w == 2) {
+#pragma unroll
+      for (int t = 0; t < kC; ++t) {
+        a *= decay(t, d);
+        *reinterpret_cast<f32x4*>(unit + at + 16 * t) = *reinterpret_cast<const f32x4*>(&qs[t][d]) * a;
+        if (DELTA) *reinterpret_cast<f32x4*>(ub + at + 16 * t) = *reinterpret_cast<const f32x4*>(&ks[t][d]) * a;
+      }
+      *reinterpret_cast<f32x4*>(ua + d) = a;
+    } else {
+      f32x4 x[kC];
+#pragma unroll
+      for (int t = kC - 1; t >= 0; --t) {
+        x[t] = *reinterpret_cast<const f32x4*>(&ks[t][d]) * a;
+        a *= decay(t, d);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < kC; t += 4)
+          *reinterpret_cast<f32x4*>(uk + (d + e) * kC + t) = f32x4{x[t][e], x[t + 1][e], x[t + 2][e], x[t + 3][e]};
+    }
+  }
+  if constexpr (!CHAN) {
+    // pairs of tokens: the rows' products on the matrix cores, times the decays between the two
+    if (w < (DELTA ? 2 : 1)) {  // uniform: queries against keys, keys against keys
+      const int r = lane & 15, g = lane >> 4;
+      const float(&rows)[kC][kRow] = w ? ks : qs;
+      f32x4 s[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(&rows[r][16 * t + 4 * g]), b = *reinterpret_cast<const f32x4*>(&ks[r][16 * t + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[t] = mfma16x16x4(a[i], b[i], s[t]);
+      }
+      f32x4 R{0.f, 0.f, 0.f, 0.f};
+      float v = 0.f;
+#pragma unroll
+      for (int t = 0; t < kC; ++t) {
+        v = t == r ? 1.0f : v * as[t][0];
+        if (g == t / 4) R[t % 4] = v;
+      }
+      const f32x4 x = R * pairwise<NT>(s);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 4 * g + i;
+        if (w == 0) um[t * kC + r] = r <= t ? x[i] : 0.0f;
+        else if (DELTA) Ls[t][r] = r < t ? bs[t] * x[i] : 0.0f;
+      }
+    }
+  } else {
+  // pairs of tokens: key i, decayed from token to token, against the queries (and keys) of the tokens from it on
+  {
+    const int dg = lane & 15, i = 4 * (lane >> 4) + w;
+    vec kr[kPer / kVec];
+#pragma unroll
+    for (int e = 0; e < kPer / kVec; ++e) kr[e] = *reinterpret_cast<const vec*>(&ks[i][kVec * (dg + 16 * e)]);
+    float m = 0.f, l = 0.f;
+#pragma unroll
     for (int t = 0; t < kC; ++t) {
-      const float at = __shfl(mine, t);  // by every lane, also by the one that starts its column here
-      v = t == lane ? 1.0f : v * at;
-      R[t][lane] = v;
-    }
-  }
-  // rows 16 w .. of K K^T and Q K^T, the tiles at and left of the diagonal
-  const float* K = p.k + row0 * p.ldk + grp * p.D + 4 * g;
-  const float* Q = p.q + row0 * p.ldq + grp * p.D + 4 * g;
-  f32x4 kk[4][kSums], qk[4][kSums];
+      if (t < w) continue;  // uniform: none of the wave's keys is at or before t
+      float sq[kVec], sk[kVec];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < kVec; ++j) sq[j] = sk[j] = 0.f;
 #pragma unroll
-    for (int s = 0; s < kSums; ++s) kk[j][s] = qk[j][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int e = 0; e < kPer / kVec; ++e) {
+        const int d = kVec * (dg + 16 * e);
+        const vec a = *reinterpret_cast<const vec*>(&as[t][d]), q = *reinterpret_cast<const vec*>(&qs[t][d]);
+        if (t > i) kr[e] *= a;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const f32x4 qa = row4(Q + 16 * t, p.ldq, 16 * w + r, cnt);
-    f32x4 kb[4];
+        for (int j = 0; j < kVec; ++j) sq[j] += q[j] * kr[e][j];
+        if (DELTA) {
+          const vec k = *reinterpret_cast<const vec*>(&ks[t][d]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= w) kb[j] = row4(K + 16 * t, p.ldk, 16 * j + r, cnt);  // uniform
-    const f32x4 ka = row4(K + 16 * t, p.ldk, 16 * w + r, cnt);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= w)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (DELTA) kk[j][t % kSums] = mfma16x16x4(ka[i], kb[j][i], kk[j][t % kSums]);
-          qk[j][t % kSums] = mfma16x16x4(qa[i], kb[j][i], qk[j][t % kSums]);
+          for (int j = 0; j < kVec; ++j) sk[j] += k[j] * kr[e][j];
         }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const f32x4 qs = total(qk[j]), ks = total(kk[j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * w + 4 * g + i, col = 16 * j + r;
-      const float rt = R[t][col];
-      unit[t * kC + col] = col <= t ? rt * qs[i] * p.q_scale : 0.0f;
-      if (DELTA) Ls[t][col] = col < t ? b_s[t] * rt * ks[i] : 0.0f;
+      }
+      auto sum = [](const float (&s)[kVec]) {
+        if constexpr (kVec == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+        else return s[0] + s[1];
+      };
+      const float mt = row16_sum(sum(sq));
+      if (dg == t) m = mt;
+      if (DELTA) {
+        const float lt = row16_sum(sum(sk));
+        if (dg == t) l = lt;
+      }
     }
+    um[dg * kC + i] = i <= dg ? m : 0.0f;
+    if (DELTA) Ls[dg][i] = i < dg ? bs[dg] * l : 0.0f;
   }
-  if (tid < kC) {
-    unit[kUnitA + tid] = a_s[0] * R[tid][0];
-    unit[kUnitE + tid] = R[kC - 1][tid];
   }
   if constexpr (DELTA) {
     __syncthreads();
-    if (w != 0) return;
-    // column `lane` of (1 + L)^-1 by forward substitution: a row of L is the same for all lanes
+    if (tid >= kC) return;
+    // column `tid` of (1 + L)^-1 by forward substitution: a row of L is the same for all lanes
     float x[kC];
 #pragma unroll
     for (int t = 0; t < kC; ++t) {
-      float s[4] = {t == lane ? 1.0f : 0.0f, 0.f, 0.f, 0.f};
+      float s[4] = {t == tid ? 1.0f : 0.0f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < t; i += 4) {
         const f32x4 l4 = *reinterpret_cast<const f32x4*>(&Ls[t][i]);
@@ -176,7 +269,7 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(MatrixScanParams p, 
           if (i + e < t) s[e] -= l4[e] * x[i + e];
       }
       x[t] = (s[0] + s[1]) + (s[2] + s[3]);
-      unit[kUnitT + t * kC + lane] = x[t] * b_s[lane];
+      ut[t * kC + tid] = x[t] * bs[tid];
     }
   }
 }
@@ -188,17 +281,9 @@ DEV float buf1(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
-// Operands of one chunk in a wave's registers (16 tokens 16 w .. of it)
-template <int NT, bool DELTA>
-struct Chunk {
-  static constexpr int kOwn = NT >= 4 ? NT / 4 : 1;  // state row tiles of a wave
-  f32x4 k[NT], q[NT], t[DELTA ? 4 : 1], m[4], v, a, e;
-  float last;  // the product of the chunk's decays
-};
-
 // One wave's walk of a sequence, token by token: 16 value columns of a head, state rows 16 t + 4 g + i of column r in a lane
 template <int NT, bool DELTA>
-DEV void walk_tokens(const MatrixScanParams& p, int h, int64_t row0, int ql, bool fresh, int col, int r, int g, float* to) {
+DEV void walk_tokens(const MatrixScanParams& p, int h, int64_t row0, int ql, bool fresh, int col, int g, float* to) {
   const int grp = h / (p.H / p.G);
   f32x4 S[NT];
 #pragma unroll
@@ -208,11 +293,14 @@ DEV void walk_tokens(const MatrixScanParams& p, int h, int64_t row0, int ql, boo
   for (int64_t row = row0; row < row0 + ql; ++row) {
     const float* k = p.k + row * p.ldk + grp * p.D + 4 * g;
     const float* q = p.q + row * p.ldq + grp * p.D + 4 * g;
+    const bool chan = p.decay_kind == 3;
+    const float* ac = p.decay + row * p.ldd + h * p.D + 4 * g;
     const float a = p.decay_kind == 1 ? p.decay[h] : (p.decay_kind == 2 ? p.decay[row * p.ldd + h] : 1.0f);
     float u = p.v[row * p.ldv + h * p.V + col], part = 0.0f, o = 0.0f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      S[t] = S[t] * a;
+      if (chan) S[t] *= ld_global<f32x4>(ac + 16 * t);  // uniform
+      else S[t] = S[t] * a;
       const f32x4 k4 = ld_global<f32x4>(k + 16 * t);
       if (DELTA)
 #pragma unroll
@@ -235,241 +323,313 @@ DEV void walk_tokens(const MatrixScanParams& p, int h, int64_t row0, int ql, boo
     for (int i = 0; i < 4; ++i) to[(16 * t + 4 * g + i) * kScanCols] = S[t][i];
 }
 
-template <int NT, bool DELTA>
-__global__ __launch_bounds__(256, 1) void chunk_walk_kernel(MatrixScanParams p, const float* __restrict__ ws, int chunks) {
-  using Ch = Chunk<NT, DELTA>;
-  constexpr int kOwn = Ch::kOwn;
-  constexpr int kKeyRow = 16 * NT + 4;  // floats of a key row in LDS: rows four apart start 16 banks apart
-  __shared__ f32x4 bB[4][64], bU[4][64], bE[4][64], bS[NT][64];
-  __shared__ int votes[4];
-  __shared__ __align__(16) float keys[kC * kKeyRow];
+// CT tiles of 16 value columns per workgroup
+template <int NT, bool DELTA, int CT>
+__global__ __launch_bounds__(64 * (NT < 4 ? NT : 4), 2) void chunk_walk_kernel(MatrixScanParams p, const float* __restrict__ ws,
+                                                                              int chunks, Segment sg) {
+  constexpr int NW = NT < 4 ? NT : 4, OWN = NT / NW, MI = 4 / NW;  // waves, state row tiles and products with M of each
+  constexpr int D = 16 * NT, kUnit = unit_floats(D, DELTA);
+  constexpr int kAhead = DELTA ? 2 : (CT == 1 ? 4 : 3);  // chunks whose operands are in registers or on their way
+  constexpr int kB = 2 * kC * D, kM = kB + (DELTA ? kC * D : 0), kT = kM + kC * kC, kA = kM + (DELTA ? 2 : 1) * kC * kC;
+  __shared__ f32x4 bO[2][NW][CT][64], bW[DELTA ? 2 : 1][NW][CT][64];
+  __shared__ int votes[NW];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
-  // heads fastest: the column blocks of a head read the same keys, queries and T, M, and land on one XCD's L2 when the heads
-  // are a multiple of eight
-  const int seq = blockIdx.z, h = blockIdx.x, cb = blockIdx.y, grp = h / (p.H / p.G);
-  const int ql = p.q_len[seq];
-  if (ql <= 0) return;  // uniform
-  const int first = chunks_before(p.q_len, seq, lane), n = (ql + kC - 1) / kC;
-  const int64_t row0 = p.q_start[seq];
-  constexpr int units = DELTA ? kUnitT + kC * kC : kUnitT;
-  const int col = cb * kScanCols + r;
-  const bool owner = w * kOwn < NT;  // narrow states have fewer row tiles than waves
-  // Buffer loads: the lane's offsets never change, a chunk's place is in the descriptor's base and its rows past the
-  // sequence's end are past the descriptor's range, so they read as zeros
-  const int own = 16 * w + r;
-  const uint32_t q_vo = (uint32_t)(own * p.ldq + 4 * g) * 4, k_vo = (uint32_t)(own * p.ldk + 4 * g) * 4,
-                 m_vo = (uint32_t)(own * kC + 4 * g) * 4,
-                 v_vo = (uint32_t)((16 * w + 4 * g) * p.ldv + r) * 4, v_row = (uint32_t)p.ldv * 4;
-  auto request = [&](int c, Ch& x) {  // chunks past the last one read it again
-    c = c < n ? c : n - 1;
-    const int left = ql - c * kC < kC ? ql - c * kC : kC;
-    const int64_t at = row0 + (int64_t)c * kC;
-    const __amdgpu_buffer_rsrc_t qr = make_rsrc(p.q + at * p.ldq + grp * p.D, (uint32_t)((left - 1) * p.ldq + p.D) * 4);
-    const __amdgpu_buffer_rsrc_t kr = make_rsrc(p.k + at * p.ldk + grp * p.D, (uint32_t)((left - 1) * p.ldk + p.D) * 4);
-    const __amdgpu_buffer_rsrc_t vr =
-        make_rsrc(p.v + at * p.ldv + h * p.V + cb * kScanCols, (uint32_t)((left - 1) * p.ldv + kScanCols) * 4);
-    const __amdgpu_buffer_rsrc_t ur = make_rsrc(ws + ((int64_t)(first + c) * p.H + h) * units, (uint32_t)units * 4);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      x.k[t] = buf4(kr, k_vo + 64 * t, 0);
-      x.q[t] = buf4(qr, q_vo + 64 * t, 0);
-    }
-    x.a = buf4(ur, (kUnitA + 16 * w + 4 * g) * 4, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x.v[i] = buf1(vr, v_vo + i * v_row, 0);  // the scalar offset is not range-checked
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if constexpr (DELTA) x.t[t] = buf4(ur, kUnitT * 4 + m_vo + 64 * t, 0);
-    x.e = buf4(ur, (kUnitE + 16 * w + 4 * g) * 4, 0);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x.m[t] = buf4(ur, m_vo + 64 * t, 0);
-    x.last = buf1(ur, (kUnitA + kC - 1) * 4, 0);
-  };
+  // heads fastest: the column blocks of a head read the same units and land on one XCD's L2 when the heads are a multiple of eight
+  const int seq = blockIdx.z, h = blockIdx.x, cb = blockIdx.y;
+  const int n = chunks_of(p.q_len[seq], sg);
+  if (n <= 0) return;  // uniform
+  const int first = chunks_before(p.q_len, seq, lane, sg);
+  const int64_t row0 = (int64_t)p.q_start[seq] + (int64_t)sg.c0 * kC;
+  const int all = p.q_len[seq] - sg.c0 * kC, ql = all < sg.span * kC ? all : sg.span * kC;
+  const bool fresh = sg.c0 == 0 && p.ctx_len[seq] - p.q_len[seq] == 0;
   // the state entry is tile-major [H][V / 16][D][16] (V % 16 == 0)
-  float* to = p.state + p.state_slot[seq] * ((int64_t)p.H * p.D * p.V) + (int64_t)h * p.D * p.V +
-              (int64_t)cb * p.D * kScanCols + r;
-  const bool fresh = p.ctx_len[seq] - ql == 0;
+  float* to = p.state + p.state_slot[seq] * ((int64_t)p.H * D * p.V) + (int64_t)h * D * p.V + (int64_t)cb * CT * D * kScanCols + r;
+  const int col = cb * CT * kScanCols + r;
+  auto by_tokens = [&]() {
+#pragma unroll
+    for (int x = 0; x < CT; ++x)
+      walk_tokens<NT, DELTA>(p, h, row0, ql, fresh, col + 16 * x, g, to + x * D * kScanCols);
+  };
   if (first + n > chunks) {  // uniform: sequences longer than the caller said, or sharing rows; no units were made for this one
-    if (w == 0) walk_tokens<NT, DELTA>(p, h, row0, ql, fresh, col, r, g, to);
+    if (w == 0) by_tokens();
     return;
   }
-  f32x4 S[NT];
+  struct Operands {
+    f32x4 q[OWN], k[OWN], b[DELTA ? OWN : 1], a[OWN], t, v[CT];
+    float m[MI];
+  };
+  // Chunks are requested one after another: what is left of the sequence, and where its next unit and value rows lie.  The
+  // value rows past its end, and every operand of a chunk past the last one, are past their descriptor's range: zeros, no traffic.
+  const float* next_unit = ws + ((int64_t)first * p.H + h) * kUnit;
+  const float* next_v = p.v + row0 * p.ldv + h * p.V + cb * CT * kScanCols;
+  int ahead = ql;
+  const int64_t unit_step = (int64_t)p.H * kUnit, v_step = (int64_t)kC * p.ldv;
+  const uint32_t u_vo = (uint32_t)(16 * r + 4 * g) * 4, v_vo = (uint32_t)(4 * g * p.ldv + r) * 4, v_row = (uint32_t)p.ldv * 4;
+  auto range = [&](int rows, uint32_t row) {  // bytes of CT tiles of the last of up to 16 rows, and of the rows before it
+    rows = rows < kC ? rows : kC;
+    return rows > 0 ? (uint32_t)(rows - 1) * row + CT * kScanCols * 4 : 0u;
+  };
+  auto request = [&](Operands& x) {
+    const __amdgpu_buffer_rsrc_t ur = make_rsrc(next_unit, ahead > 0 ? kUnit * 4 : 0);
+    const __amdgpu_buffer_rsrc_t vr = make_rsrc(next_v, range(ahead, v_row));
+    next_unit += unit_step, next_v += v_step, ahead -= kC;
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S[t][i] = fresh ? 0.0f : to[(16 * t + 4 * g + i) * kScanCols];
-
-  float odd = 0.0f;  // NaN once an output is not finite
-  auto walk = [&](int c, const Ch& x, Ch& next) {
-    request(c + 1, next);  // in flight across this chunk
-    // the chunk's key rows: the state's update reads them by columns
-#pragma unroll
-    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(&keys[own * kKeyRow + 16 * t + 4 * g]) = x.k[t];
-    f32x4 P[kSums], u = x.v;
-#pragma unroll
-    for (int q = 0; q < kSums; ++q) P[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (DELTA) {
-      f32x4 W[kSums];
-#pragma unroll
-      for (int q = 0; q < kSums; ++q) W[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          W[t % kSums] = mfma16x16x4(x.k[t][i], S[t][i], W[t % kSums]), P[t % kSums] = mfma16x16x4(x.q[t][i], S[t][i], P[t % kSums]);
-      const f32x4 ws4 = total(W);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) u[i] = x.v[i] - x.a[i] * ws4[i];
-      bB[w][lane] = u;
-      lds_barrier();
-      f32x4 ut[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const f32x4 b = bB[t][lane];
-        ut[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ut[t] = mfma16x16x4(x.t[t][i], b[i], ut[t]);
-      }
-      u = total(ut);
+    for (int o = 0; o < OWN; ++o) {
+      const int t = w * OWN + o;
+      if constexpr (DELTA) x.b[o] = buf4(ur, u_vo, (kB + 256 * t) * 4);
+      x.q[o] = buf4(ur, u_vo, 256 * t * 4);
+      x.k[o] = buf4(ur, u_vo, (kC * D + 256 * t) * 4);
+      x.a[o] = buf4(ur, 16 * g, (kA + 16 * t) * 4);
     }
-    bU[w][lane] = u;
-    bE[w][lane] = x.e * u;
-    if constexpr (!DELTA) {
+    if constexpr (DELTA) x.t = buf4(ur, u_vo, kT * 4);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) x.m[i] = buf1(ur, u_vo, (kM + w + NW * i) * 4);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x.v[ct][i] = buf1(vr, v_vo + i * v_row + 64 * ct, 0);  // the scalar offset is not range-checked
+  };
+  f32x4 S[OWN][CT];
+#pragma unroll
+  for (int o = 0; o < OWN; ++o)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        S[o][ct][i] = fresh ? 0.0f : to[(ct * D + 16 * (w * OWN + o) + 4 * g + i) * kScanCols];
+  float odd = 0.0f;  // NaN once an output is not finite
+  const uint32_t o_row = (uint32_t)(p.H * p.V) * 4;
+  float part[CT][MI][NW];
+  auto collect = [&](int c) {  // every wave's share of chunk c's rows 4 g + w (+ NW)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int o = 0; o < NW; ++o) part[ct][i][o] = reinterpret_cast<const float*>(&bO[c & 1][o][ct][lane])[w + NW * i];
+  };
+  float* next_out = p.out + (row0 * p.H + h) * p.V + cb * CT * kScanCols;
+  int behind = ql;
+  auto write = [&]() {  // chunk after chunk; rows past the sequence's end are out of the descriptor's range
+    const __amdgpu_buffer_rsrc_t to_out = make_rsrc(next_out, range(behind, o_row));
+    next_out += (int64_t)kC * p.H * p.V, behind -= kC;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        float s = part[ct][i][0] + part[ct][i][1];
+        if constexpr (NW == 4) s += part[ct][i][2] + part[ct][i][3];
+        odd += s * 0.0f;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), to_out, (4 * g + w + NW * i) * o_row + r * 4 + 64 * ct, 0, 0);
+      }
+  };
+  const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+  // One chunk: the outputs of the chunk before leave LDS meanwhile, behind the barrier that the delta rule needs anyway
+  auto step = [&](int c, Operands& x) {
+    f32x4 u[CT], O[OWN][CT];
+    auto read_out = [&](int i0, int i1) {
+#pragma unroll
+      for (int i = i0; i < i1; ++i)
+#pragma unroll
+        for (int o = 0; o < OWN; ++o)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) O[o][ct] = mfma16x16x4(x.q[o][i], S[o][ct][i], i ? O[o][ct] : zero);
+    };
+    if constexpr (DELTA) {
+      f32x4 W[OWN][CT];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) P[t % kSums] = mfma16x16x4(x.q[t][i], S[t][i], P[t % kSums]);
-    }
-    lds_barrier();
-    const f32x4 ps = total(P);
-    f32x4 o[4];
+        for (int o = 0; o < OWN; ++o)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int ct = 0; ct < CT; ++ct) W[o][ct] = mfma16x16x4(x.b[o][i], S[o][ct][i], i ? W[o][ct] : zero);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        f32x4 s = W[0][ct];
+#pragma unroll
+        for (int o = 1; o < OWN; ++o) s += W[o][ct];
+        bW[c & 1][w][ct][lane] = s;
+      }
+      read_out(0, 2);
+      lds_barrier();
+      f32x4 ws4[CT][NW];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int o = 0; o < NW; ++o) ws4[ct][o] = bW[c & 1][o][ct][lane];
+      collect(c > 0 ? c - 1 : 0);
+      __builtin_amdgcn_sched_barrier(0);
+      read_out(2, 4);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        f32x4 s = ws4[ct][0] + ws4[ct][1];
+        if constexpr (NW == 4) s += ws4[ct][2] + ws4[ct][3];
+        const f32x4 d = x.v[ct] - s;
+        f32x4 t0 = mfma16x16x4(x.t[0], d[0], zero), t1 = mfma16x16x4(x.t[1], d[1], zero);
+        t0 = mfma16x16x4(x.t[2], d[2], t0);
+        t1 = mfma16x16x4(x.t[3], d[3], t1);
+        u[ct] = t0 + t1;
+      }
+    } else {
+      read_out(0, 4);
+      lds_barrier();
+      collect(c > 0 ? c - 1 : 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) u[ct] = x.v[ct];
+    }
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) S[o][ct] *= x.a[o];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) o[t] = mfma16x16x4(x.m[t][i], bU[t][lane][i], o[t]);
-    f32x4 res = total(o);
+      for (int o = 0; o < OWN; ++o)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      res[i] += x.a[i] * (ps[i] * p.q_scale);
-      odd += res[i] * 0.0f;
-    }
-    if (owner) {
-      f32x4 s[kOwn];
+        for (int ct = 0; ct < CT; ++ct) S[o][ct] = mfma16x16x4(x.k[o][i], u[ct][i], S[o][ct]);
 #pragma unroll
-      for (int o = 0; o < kOwn; ++o) s[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < CT; ++ct) {
+      f32x4 s = O[0][ct];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)  // this wave's tiles, picked without indexing registers at run time
+      for (int o = 1; o < OWN; ++o) s += O[o][ct];
 #pragma unroll
-        for (int o = 0; o < kOwn; ++o)
-          if (t == w * kOwn + o) s[o] = S[t] * x.last;  // uniform
+      for (int i = 0; i < MI; ++i) {
+        float uw = u[ct][NW * i];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const f32x4 b = bE[t][lane];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int o = 0; o < kOwn; ++o) s[o] = mfma16x16x4(keys[(16 * t + 4 * g + i) * kKeyRow + 16 * (w * kOwn + o) + r], b[i], s[o]);
+        for (int k = 1; k < NW; ++k) uw = w == k ? u[ct][NW * i + k] : uw;
+        s = mfma16x16x4(x.m[i], uw, s);
       }
-#pragma unroll
-      for (int o = 0; o < kOwn; ++o) bS[w * kOwn + o][lane] = s[o];
+      bO[c & 1][w][ct][lane] = s;
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = c * kC + 16 * w + 4 * g + i;
-      if (tok < ql) p.out[((row0 + tok) * p.H + h) * p.V + col] = res[i];
-    }
-    lds_barrier();
-#pragma unroll
-    for (int t = 0; t < NT; ++t) S[t] = bS[t][lane];
+    if (c > 0) write();  // uniform
+    __builtin_amdgcn_sched_barrier(0);  // requests stay in the order of their use
+    request(x);
+    __builtin_amdgcn_sched_barrier(0);
   };
-  Ch x, y;
-  request(0, x);
-  for (int c = 0; c < n; c += 2) {
-    walk(c, x, y);
-    if (c + 1 < n) walk(c + 1, y, x);  // uniform
+  Operands x[kAhead];
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) {
+    request(x[i]);
+    __builtin_amdgcn_sched_barrier(0);
   }
+  int c = 0;
+  for (; c + kAhead <= n; c += kAhead)  // no branch between the steps: each waits for its own operands alone
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) step(c + i, x[i]);
+#pragma unroll
+  for (int i = 0; i + 1 < kAhead; ++i)
+    if (c + i < n) step(c + i, x[i]);  // uniform
+  lds_barrier();
+  collect(n - 1);
+  write();
   const bool mine = __any(odd != 0.0f);
   if (lane == 0) votes[w] = mine;
   lds_barrier();
-  if (votes[0] | votes[1] | votes[2] | votes[3]) {  // uniform for the workgroup
-    __syncthreads();                                // every wave's outputs are written
-    if (w == 0) walk_tokens<NT, DELTA>(p, h, row0, ql, fresh, col, r, g, to);
+  int any = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) any |= votes[i];
+  if (any) {          // uniform for the workgroup
+    __syncthreads();  // every wave's outputs are written
+    if (w == 0) by_tokens();
     return;
   }
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-    if (t / kOwn == w)  // uniform
+  for (int o = 0; o < OWN; ++o)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) to[(16 * t + 4 * g + i) * kScanCols] = S[t][i];
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[(ct * D + 16 * (w * OWN + o) + 4 * g + i) * kScanCols] = S[o][ct][i];
+}
+
+// two column tiles per workgroup once single ones are more than the CUs
+bool scan_pairs(const MatrixScanParams& p) {
+  return p.V % (2 * kScanCols) == 0 && (int64_t)p.H * (p.V / kScanCols) * p.nseq > 256;
+}
+
+// chunks of `rows` rows at most, `longest` in the longest sequence, in segments of `span` chunks of each
+int64_t chunk_bound(const MatrixScanParams& p, int64_t rows, int64_t longest, int64_t span) {
+  return std::min(rows / kC + p.nseq, p.nseq * std::min(span, (longest + kC - 1) / kC));
+}
+// the segment's chunks per sequence: all of them where the workspace has the room
+int64_t segment_span(const MatrixScanParams& p, int64_t rows, int64_t longest) {
+  const int64_t n = (longest + kC - 1) / kC, unit = (int64_t)p.H * unit_floats(p.D, p.beta);
+  if (chunk_bound(p, rows, longest, n) * unit <= kRoom) return n;
+  return std::max<int64_t>(1, kRoom / unit / p.nseq);
 }
 
 template <int NT, bool DELTA>
-hipError_t launch_chunks(const MatrixScanParams& p, float* ws, int chunks, hipStream_t st) {
-  hipLaunchKernelGGL((chunk_prepare_kernel<NT, DELTA>), dim3(chunks, p.H), dim3(256), 0, st, p, ws);
-  hipLaunchKernelGGL((chunk_walk_kernel<NT, DELTA>), dim3(p.H, p.V / kScanCols, p.nseq), dim3(256), 0, st, p, ws, chunks);
+hipError_t launch_chunks(const MatrixScanParams& p, float* ws, int64_t rows, int64_t longest, hipStream_t st) {
+  const int64_t n = (longest + kC - 1) / kC, span = segment_span(p, rows, longest);
+  const int chunks = (int)chunk_bound(p, rows, longest, span);
+  const bool pairs = scan_pairs(p);
+  // a sequence may be longer than the caller said: the last segment takes what is left of it
+  for (int64_t c0 = 0; c0 < n; c0 += span) {
+    const Segment sg{(int)c0, c0 + span < n ? (int)span : INT_MAX / kC - (int)c0};
+    if (p.decay_kind == 3)
+      hipLaunchKernelGGL((chunk_prepare_kernel<NT, DELTA, true>), dim3(chunks, p.H), dim3(256), 0, st, p, ws, sg);
+    else
+      hipLaunchKernelGGL((chunk_prepare_kernel<NT, DELTA, false>), dim3(chunks, p.H), dim3(256), 0, st, p, ws, sg);
+    const dim3 block(64 * (NT < 4 ? NT : 4));
+    if (pairs)
+      hipLaunchKernelGGL((chunk_walk_kernel<NT, DELTA, 2>), dim3(p.H, p.V / (2 * kScanCols), p.nseq), block, 0, st, p, ws, chunks, sg);
+    else
+      hipLaunchKernelGGL((chunk_walk_kernel<NT, DELTA, 1>), dim3(p.H, p.V / kScanCols, p.nseq), block, 0, st, p, ws, chunks, sg);
+  }
   return hipGetLastError();
 }
 
 }  // namespace
 
 // Time in us of the walk by tokens and of the chunks: each is a start, then its longest chain or the work of all its column blocks,
-// whichever is more.  Fitted per key width over 1..128 sequences of 16..4096 rows of 2..1024 column blocks (both within 11 % rms);
-// of 864 timings the slower of the two is taken by more than 6 % in seven, by 9 % at most.  Walk against
-// chunks, H x D x V: delta rule, 16 x 128 x 128, one sequence of 64 rows 31 / 38, 128 rows 56 / 44, 2048 rows 995 / 217, 128 of 32
-// rows 388 / 531; 32 x 64 x 64, 64 of 64 rows 223 / 290 (one chunk each: the delta rule's start is not made up for); without it,
-// 16 x 128 x 128, 64 rows 28 / 22, 2048 rows 913 / 146, 128 of 32 rows 360 / 491; 16 x 32 x 64, 64 of 64 rows 76 / 62.
+// whichever is more.  Fitted per key width over 1..128 sequences of 4..2048 rows of 2..256 column blocks (both within 12 % rms); of 831
+// timings the slower of the two is taken by more than 6 % in 14.  Walk against chunks, H x D x V: delta rule, 16 x 128 x 128, one
+// sequence of 17 rows 12.6 / 11.9, 64 rows 30 / 14, 2048 rows 962 / 147, 16 of 8 rows 24 / 26, 64 of 64 rows 372 / 165; without it, 17
+// rows 11.6 / 9.9, 64 rows 27 / 11, 64 of 64 rows 328 / 105; 2 x 128 x 128, 16 rows, decays per channel 10 / 12.
 struct ScanCost {
-  double walk0, row, row_block, chunk0, chunk, chunk_block, seq_block;
+  double walk0, row, row_block, walk_seq, chunk0, chunk, chunk_block, seq_block, channels;
 };
 static bool chunks_pay(const MatrixScanParams& p, int64_t rows, int64_t chunks, int64_t longest) {
-  static const ScanCost kDelta[3] = {{5.3, 0.269, 0.044, 24.2, 2.53, 1.93, 0.42},   // widths 32, 64, 128
-                                     {5.5, 0.301, 0.061, 25.8, 3.33, 2.22, 1.17},
-                                     {5.5, 0.425, 0.118, 29.9, 5.24, 3.54, 1.17}};
-  static const ScanCost kPlain[3] = {{5.4, 0.233, 0.039, 12.1, 1.84, 1.11, 0.46},
-                                     {5.4, 0.270, 0.051, 13.7, 2.38, 1.34, 0.44},
-                                     {5.2, 0.380, 0.107, 17.0, 4.03, 2.23, 1.18}};
-  if (p.beta && longest <= kC) return false;
+  static const ScanCost kDelta[3] = {{4.3, 0.266, 0.034, 0.229, 8.7, 0.615, 0.340, 0.095, 1.0},   // widths 32, 64, 128
+                                     {4.4, 0.303, 0.048, 0.319, 8.8, 0.754, 0.377, 0.291, 1.2},
+                                     {5.2, 0.421, 0.092, 0.486, 9.3, 1.123, 0.464, 0.439, 2.1}};
+  static const ScanCost kPlain[3] = {{4.2, 0.228, 0.030, 0.248, 7.8, 0.334, 0.232, 0.129, 1.0},
+                                     {4.2, 0.272, 0.040, 0.327, 8.0, 0.418, 0.249, 0.228, 1.2},
+                                     {4.8, 0.382, 0.086, 0.484, 8.6, 0.631, 0.333, 0.437, 2.1}};
   const ScanCost& c = (p.beta ? kDelta : kPlain)[p.D == 32 ? 0 : (p.D == 64 ? 1 : 2)];
   const double blocks = (double)p.H * (p.V / kScanCols) / 128.0, n = (double)((longest + kC - 1) / kC);
-  const double walk = c.walk0 + std::max(c.row * longest, c.row_block * rows * blocks);
-  return walk > c.chunk0 + std::max(c.chunk * n, (c.chunk_block * chunks + c.seq_block * p.nseq) * blocks);
+  const double walk = c.walk0 + std::max(c.row * longest, (c.row_block * rows + c.walk_seq * p.nseq) * blocks);
+  const double start = c.chunk0 + (p.decay_kind == 3 ? c.channels : 0.0);
+  return walk > start + std::max(c.chunk * n, (c.chunk_block * chunks + c.seq_block * p.nseq) * blocks);
 }
 
-// chunks of `rows` rows at most: the launch's workgroups find theirs by the lengths
-static int64_t chunk_bound(const MatrixScanParams& p, int64_t rows, int64_t longest) {
-  return std::min(rows / kC + p.nseq, p.nseq * ((longest + kC - 1) / kC));
-}
-
-// Whether the chunks take the shape, and their workspace floats
-static int64_t chunk_room(const MatrixScanParams& p, int rows, int64_t longest) {
+// Whether the chunks take the shape
+static bool chunk_room(const MatrixScanParams& p, int64_t rows, int64_t longest) {
   auto aligned = [](const float* x, int ld) { return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ld % 4 == 0; };
-  if (longest <= 0 || p.nseq <= 0 || p.src_idx || p.decay_kind > 2 || (p.D != 32 && p.D != 64 && p.D != 128) ||
-      p.V % kScanCols || !aligned(p.q, p.ldq) || !aligned(p.k, p.ldk))
-    return 0;
-  // rows of a chunk lie within 31-bit offsets of its first one
-  const int64_t ld = std::max(std::max((int64_t)p.ldq, (int64_t)p.ldk), (int64_t)p.ldv);
-  const int64_t chunks = chunk_bound(p, rows, longest);
-  if (chunks > 65535 || p.nseq > 65535 || p.H > 65535 || ld * kC * 4 > INT32_MAX) return 0;
-  const int64_t floats = chunks * p.H * (p.beta ? kUnitT + kC * kC : kUnitT);
-  return floats <= (int64_t{1} << 28) ? floats : 0;  // a gigabyte: 128k rows of 16 heads; the token walk needs no workspace
+  if (longest <= 0 || p.nseq <= 0 || p.src_idx || p.decay_kind > 3 || (p.D != 32 && p.D != 64 && p.D != 128) ||
+      p.V % kScanCols || !aligned(p.q, p.ldq) || !aligned(p.k, p.ldk) || (p.decay_kind == 3 && !aligned(p.decay, p.ldd)))
+    return false;
+  // value rows of a chunk lie within 31-bit offsets of its first one
+  if (p.nseq > 65535 || p.H > 65535 || std::max<int64_t>(p.ldv, (int64_t)p.H * p.V) * kC * 4 > INT32_MAX || rows * p.H > kMostRows) return false;
+  return (int64_t)p.nseq * p.H * unit_floats(p.D, p.beta) <= (int64_t{1} << 29);  // a chunk of each sequence: 2 GB
 }
 
 int64_t scan_chunk_floats(const MatrixScanParams& p, int rows, int64_t longest) {
-  const int64_t floats = chunk_room(p, rows, longest);
-  if (!floats) return 0;
-  return chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunk_bound(p, rows, longest), longest) ? floats : 0;
+  if (!chunk_room(p, rows, longest)) return 0;
+  const int64_t all = (longest + kC - 1) / kC;
+  if (!chunks_pay(p, std::min<int64_t>(rows, p.nseq * longest), chunk_bound(p, rows, longest, all), longest)) return 0;
+  return chunk_bound(p, rows, longest, segment_span(p, rows, longest)) * p.H * unit_floats(p.D, p.beta);
 }
 
-// Without the delta rule.  Where the chunks are out of the question (decays per key channel, other widths, unaligned rows) two
-// levels beat one long chain; where they are not, only for a long sequence of a few column blocks, whose chunks follow one
-// another on a mostly empty chip.  Chunks against two levels: 2 heads of 128 x 128, 700 rows 59 / 66, 1000 rows 77 / 72; 2 heads of
-// 64 x 64, 1000 rows 49 / 57, 2048 rows 84 / 74; 2 of 32 x 16, 2048 rows 66 / 68, 4096 rows 120 / 98; 16 x 64 x 64, 4096 rows 170 / 257.
+// Without the delta rule.  Where the chunks are out of the question (other widths, unaligned rows) two levels beat one long chain;
+// where they are not, only for a very long sequence of a few column blocks, whose chunks follow one another on a mostly empty chip.
+// Chunks against two levels, decays per channel: 2 heads of 128 x 128, 2048 rows 84 / 84, 8192 rows 290 / 237; 4 of 64 x 64, 2048 rows
+// 57 / 60, 4096 104 / 82; 4 of 32 x 32, 4096 rows 85 / 61.  One line for all decays: those per head take 81 / 101, 287 / 315; 55 / 75,
+// 102 / 120; 83 / 100 (chunks of 64 took 138 and 509, 86 and 167, 121).
 bool scan_two_levels(const MatrixScanParams& p, int rows, int64_t longest) {
   if (p.beta || rows < kTwoLevelRows) return false;
   if (!chunk_room(p, rows, longest)) return true;
-  const int64_t from = p.D == 128 ? 900 : (p.D == 64 ? 1500 : 2500);
+  const int64_t from = p.D == 32 ? 4096 : 2048;
   return longest >= from && (int64_t)p.nseq * p.H * (p.V / kScanCols) <= 16;
 }
 
@@ -478,10 +638,9 @@ bool scan_two_levels(const MatrixScanParams& p, int rows, int64_t longest) {
 extern "C" hipError_t dsse_scan_chunks(const dsse::MatrixScanParams* p, float* ws, int rows, int64_t longest, hipStream_t st) {
   if (p->nseq <= 0 || p->H <= 0 || rows <= 0) return hipSuccess;
   if (p->H % p->G || !dsse::scan_chunk_floats(*p, rows, longest)) return hipErrorInvalidValue;
-  const int chunks = (int)dsse::chunk_bound(*p, rows, longest);
 #define DSSE_CHUNK_CASE(n)                                                            \
   case 16 * n:                                                                        \
-    return p->beta ? dsse::launch_chunks<n, true>(*p, ws, chunks, st) : dsse::launch_chunks<n, false>(*p, ws, chunks, st);
+    return p->beta ? dsse::launch_chunks<n, true>(*p, ws, rows, longest, st) : dsse::launch_chunks<n, false>(*p, ws, rows, longest, st);
   switch (p->D) {
     DSSE_CHUNK_CASE(2)
     DSSE_CHUNK_CASE(4)

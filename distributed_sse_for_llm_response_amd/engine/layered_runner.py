@@ -38,8 +38,8 @@ same weights and its own pages and state slots per pass:
     feed-forward            fused [gate | up] GEMM -> gated_act (gelu) -> down GEMM
     head                    stream_step (last add + final norm) -> head GEMM -> logit_cap (scale, tanh cap)
 
-Long prompt groups take the recurrences by chunks of 64 tokens: on the matrix cores in matrix_scan, as a two-level walk
-(matrix_scan_chunked) where the decay differs between key channels.
+Prompt groups take the recurrences by chunks of 16 tokens on the matrix cores in matrix_scan, as a two-level walk
+(matrix_scan_chunked) where a long group's shapes are not the chunks'.
 
 The multi-stream walk (`_stream_layers`) also goes over layer runs; a row carries S residual copies:
 
@@ -159,7 +159,6 @@ class LayeredRunner(RunnerBase):
         cfg, dev = self.cfg, self.device
         self._init_slots(max_batch, self.max_blocks, cfg.vocab_size, dev, self.comm)
         self._tile_rows = []   # row counts of the shared-page sink attention's work items that this design's layers use
-        self._channel_decays = False  # some layer's recurrence decays per key channel
         self._latents = set()  # (heads, rank, rotated width) of the latent attentions on the MFMA form
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
@@ -206,7 +205,6 @@ class LayeredRunner(RunnerBase):
         with the same weights and has its own pages and state slots each time."""
         cfg, dev = self.cfg, self.device
         self.runs = cfg.runs()
-        self._channel_decays = any(L.kind == "parallel" for L in cfg.layers)
         kv, st, self._rope = {}, {}, {}
         for r in self.runs:
             L, m = cfg.layers[r.layer], cfg.layers[r.layer].mixer
@@ -512,7 +510,8 @@ class LayeredRunner(RunnerBase):
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
             D, chan, seqs = k.shape[2], decay is not None and decay.dim() == 3, g.get("seqs")  # seqs: prompt portions
-            if beta is None and seqs and ops.matrix_scan_two_levels(q, k, v, chan, g["rows"][1], len(seqs[0]), g["longest"]):
+            if beta is None and seqs and ops.matrix_scan_two_levels(q, k, v, chan, g["rows"][1], len(seqs[0]), g["longest"],
+                                                                       decay if chan else None):
                 s_first, s_count, cm = self._scan_lists(g)
                 scr = self._scratch(d, "scan_s", cm.shape[1] * H * D * V)
                 ascr = self._scratch(d, "scan_a", cm.shape[1] * H * D) if chan else None
@@ -1020,7 +1019,7 @@ class LayeredRunner(RunnerBase):
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
             ops.matrix_scan(q, k, v, z.unflatten(1, (H, D)), beta, self.state.state[ri], g["qs"], g["ql"], g["ctx"],
-                            g["ss"], o, D ** -0.5)
+                            g["ss"], o, D ** -0.5, g.get("longest", 0))
         ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw.norm, gz, self.cfg.eps, ao, 1)
         self._lin(ao, Lw.o, Lw.o_t, d["y"])
@@ -1465,8 +1464,6 @@ class LayeredRunner(RunnerBase):
         d["rows"] = (row0, T)   # the packed rows of these portions
         d["longest"], d["keys"] = max(ql), max(ctx)
         d["seqs"] = (qs, ql, ss)
-        if self._channel_decays and T >= 4 * ops.layers.SCAN_CHUNK:
-            self._scan_lists(d)  # surely asked for: with the other lists, before the step's first launch
         return T, qs, ql, d
 
     def prefill(self, seqs: list, ring_row: int, trace: list | None = None) -> None:

@@ -325,10 +325,11 @@ def scan_state_from_plain(plain):
 SCAN_CHUNK = 64        # tokens per chunk of the two-level walk
 
 
-def matrix_scan_two_levels(q, k, v, per_channel: bool, rows: int, nseq: int, longest: int) -> bool:
+def matrix_scan_two_levels(q, k, v, per_channel: bool, rows: int, nseq: int, longest: int, decay=None) -> bool:
     """Whether nseq sequences of `rows` rows together, `longest` in the longest, without the delta rule are better walked in
-    two levels (matrix_scan_chunked) than by matrix_scan: the kernels' own answer, by shapes, row pitches and alignment."""
-    return _hip(v) and torch.ops.dsse.matrix_scan_two_levels(q, k, v, per_channel, rows, nseq, longest)
+    two levels (matrix_scan_chunked) than by matrix_scan: the kernels' own answer, by shapes, row pitches and alignment
+    (decay: those per key channel, whose rows count too)."""
+    return _hip(v) and torch.ops.dsse.matrix_scan_two_levels(q, k, v, per_channel, rows, nseq, longest, decay)
 
 
 def scan_chunks(q_start: list, q_len: list, slots: list):
