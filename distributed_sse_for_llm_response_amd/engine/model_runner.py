@@ -137,11 +137,12 @@ PREFILL_SLAB_ROWS = 512
 
 # Prompt-chunk sizes of the captured mixed steps: one graph per (decode bucket, C).  The engine sizes each step's
 # chunk from the measured step costs (engine.PassCost.mixed_chunk); a prompt longer than the chunk is split evenly.
-# B + C stays within MIXED_MAX_ROWS.  Round 5 set 512 because of a GEMM cliff at 576 rows; the round-6 cost-model
-# dispatch removed that cliff (profiles/r6/gemm_model_r6.md), and 768 was re-measured with the serving bench at
-# 40 req/s: TTFT p50 29.5 vs 29.8 ms, ITL p99 13.4 vs 10.7 ms (profiles/r6/serving_r6.md).  The bigger chunks buy no
-# TTFT and cost ITL, so 512 stays.
-MIXED_CHUNKS = (128, 256, 384, 512)
+# Every whole number of 64-row flash-prefill tiles: a step pays for its captured rows, 9 to 14 us each (Mistral-7B, 64
+# streams, C = 64 .. 448: 6.26, 7.18, 8.09, 8.81, 9.33, 10.04, 10.48 ms), so a chunk should not be padded by more than
+# a tile; with every second size alone a prompt of 300 rows ran as 384.  B + C stays within MIXED_MAX_ROWS: 768 was
+# measured with the serving bench at 40 req/s, TTFT p50 29.5 vs 29.8 ms, ITL p99 13.4 vs 10.7 ms
+# (profiles/r6/serving_r6.md).  The bigger chunks buy no TTFT and cost ITL, so 512 stays.
+MIXED_CHUNKS = tuple(range(64, 513, 64))
 MIXED_MAX_ROWS = 512
 
 
@@ -625,8 +626,7 @@ class ModelRunner(RunnerBase):
         if fixed > 0:
             return [c for c in [self.mixed_chunk(B)] if B + c <= tmax]
         top = (MIXED_MAX_ROWS - B) // PREFILL_TILE * PREFILL_TILE
-        sizes = sorted({c for c in MIXED_CHUNKS if c <= top} | ({top} if top >= MIXED_CHUNKS[0] else set()))
-        return [c for c in sizes if B + c <= tmax]
+        return [c for c in MIXED_CHUNKS if c <= top and B + c <= tmax]
 
     def _capture_mixed(self, decode_buckets) -> None:
         """One graph per (decode bucket B, chunk size C in mixed_chunks(B)) for the mixed step (ModelRunner.mixed;
