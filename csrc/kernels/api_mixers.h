@@ -43,6 +43,14 @@ struct NormRopeParams {
   int out_f32;
 };
 
+// Up to three sets of heads of the same rows in one launch: their inputs and outputs do not overlap (each may work in place)
+struct NormRopeList {
+  static constexpr int kMost = 3;
+  NormRopeParams p[kMost];
+  int gy[kMost];         // workgroups per row (set by the launch)
+  int n;
+};
+
 struct SinkAttnParams {
   const float* q;        // [T, H, D] fp32 (normed, rotated)
   const void* k;         // [pages * kBS, G, D] element type
@@ -240,7 +248,7 @@ hipError_t dsse_moe_route(const float* z, int ldz, const float* corr, int M, int
                           float scale, int kind, int* topk_idx, float* topk_w, int ldw, hipStream_t st);
 hipError_t dsse_stream_step(const dsse::StreamStepParams* p, hipStream_t st);
 hipError_t dsse_gated_act(const float* gu, int ldg, void* h, int M, int F, int kind, int f32, hipStream_t st);
-hipError_t dsse_norm_rope_rows(const dsse::NormRopeParams* p, hipStream_t st);
+hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st);
 hipError_t dsse_sink_attention(int num_work, const dsse::SinkAttnParams* p, hipStream_t st);
 // MFMA form for prompt portions (bf16, D % 32 == 0, V / 16 in {1..8, 10, 12, 16, 20, 24, 32}): 16-row tiles, values from the
 // transposed pages vt [pages, G, V, kBS] (keys permuted inside a page as the MFMA's k axis wants them)

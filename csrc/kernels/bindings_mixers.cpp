@@ -121,8 +121,9 @@ void gated_act(const Tensor& gu, Tensor& h, int64_t kind) {
                                 (int)kind, elem(h, "h"), cur_stream()));
 }
 
-void norm_rope_rows(const Tensor& x, const OptTensor& norm_w, const Tensor& positions, const OptTensor& rope, Tensor& out,
-                    const OptTensor& out_rows, int64_t kind, double eps, double scale, const OptTensor& out_t) {
+dsse::NormRopeParams norm_rope_params(const Tensor& x, const OptTensor& norm_w, const Tensor& positions, const OptTensor& rope,
+                                      const Tensor& out, const OptTensor& out_rows, int64_t kind, double eps, double scale,
+                                      const OptTensor& out_t) {
   head_view(x, "x");
   dsse::NormRopeParams p{};
   p.T = (int)x.size(0), p.nh = (int)x.size(1), p.D = (int)x.size(2);
@@ -170,7 +171,33 @@ void norm_rope_rows(const Tensor& x, const OptTensor& norm_w, const Tensor& posi
     p.num_out_rows = p.T;
   }
   p.eps = (float)eps, p.scale = (float)scale;
-  DSSE_CHECK_HIP(dsse_norm_rope_rows(&p, cur_stream()));
+  return p;
+}
+
+void norm_rope_rows(const Tensor& x, const OptTensor& norm_w, const Tensor& positions, const OptTensor& rope, Tensor& out,
+                    const OptTensor& out_rows, int64_t kind, double eps, double scale, const OptTensor& out_t) {
+  dsse::NormRopeList l{};
+  l.p[0] = norm_rope_params(x, norm_w, positions, rope, out, out_rows, kind, eps, scale, out_t);
+  l.n = 1;
+  DSSE_CHECK_HIP(dsse_norm_rope_rows(l, cur_stream()));
+}
+
+// norm_rope_rows of up to three sets of heads of the same rows in one launch
+void norm_rope_list(at::TensorList x, const c10::List<OptTensor>& norm_w, const Tensor& positions, const c10::List<OptTensor>& rope,
+                    at::TensorList out, const c10::List<OptTensor>& out_rows, at::IntArrayRef kind, at::ArrayRef<double> eps,
+                    at::ArrayRef<double> scale, const c10::List<OptTensor>& out_t) {
+  const size_t n = x.size();
+  TORCH_CHECK(n >= 1 && n <= dsse::NormRopeList::kMost && norm_w.size() == n && rope.size() == n && out.size() == n &&
+                  out_rows.size() == n && kind.size() == n && eps.size() == n && scale.size() == n && out_t.size() == n,
+              "one to three sets of heads, an entry of every list each");
+  dsse::NormRopeList l{};
+  for (size_t i = 0; i < n; ++i) {
+    TORCH_CHECK(x[i].size(0) == x[0].size(0), "every set of heads has the same rows");
+    l.p[i] = norm_rope_params(x[i], norm_w.get(i), positions, rope.get(i), out[i], out_rows.get(i), kind[i], eps[i], scale[i],
+                              out_t.get(i));
+  }
+  l.n = (int)n;
+  DSSE_CHECK_HIP(dsse_norm_rope_rows(l, cur_stream()));
 }
 
 void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache, const Tensor& block_tables,
@@ -291,15 +318,16 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
 void gate_math(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2, double c) {
   col_view(x, "x");
   const int M = (int)x.size(0), N = (int)x.size(1);
-  TORCH_CHECK(kind >= 0 && kind <= 2, "kind 0..2");
-  // p1 / p2 hold one number per column, or one per run of neighbouring columns
-  const int64_t n1 = p1.has_value() ? p1->numel() : N, n2 = p2.has_value() ? p2->numel() : N;
-  TORCH_CHECK(n1 >= 1 && n2 >= 1 && N % n1 == 0 && N % n2 == 0, "p1 and p2 must divide the row into equal runs");
+  TORCH_CHECK(kind >= 0 && kind <= 3 && (kind != 3 || N % 2 == 0), "kind 0..3, two halves");
+  // p1 / p2 hold one number per column (of the left half with kind 3), or one per run of neighbouring columns
+  const int64_t cols = kind == 3 ? N / 2 : N;
+  const int64_t n1 = p1.has_value() ? p1->numel() : cols, n2 = p2.has_value() ? p2->numel() : cols;
+  TORCH_CHECK(n1 >= 1 && n2 >= 1 && cols % n1 == 0 && cols % n2 == 0, "p1 and p2 must divide the row into equal runs");
   const float* a = opt_f32(p1, "p1", n1);
   const float* b = opt_f32(p2, "p2", n2);
-  TORCH_CHECK(kind != 0 || (a && b), "kind 0 needs p1 and p2");
+  TORCH_CHECK((kind != 0 && kind != 3) || (a && b), "kinds 0 and 3 need p1 and p2");
   TORCH_CHECK(kind != 2 || c > 0, "kind 2 needs c > 0");
-  DSSE_CHECK_HIP(dsse_gate_math(x.data_ptr<float>(), (int)x.stride(0), M, N, (int)kind, a, (int)(N / n1), b, (int)(N / n2),
+  DSSE_CHECK_HIP(dsse_gate_math(x.data_ptr<float>(), (int)x.stride(0), M, N, (int)kind, a, (int)(cols / n1), b, (int)(cols / n2),
                                 (float)c, cur_stream()));
 }
 
@@ -825,6 +853,8 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("stream_step(Tensor? y, float mult, Tensor(a!) resid, Tensor? ids, Tensor? embed, Tensor? vec, Tensor? alpha, "
         "Tensor? w, Tensor? b, Tensor(b!)? xb) -> ()");
   m.def("gated_act(Tensor gu, Tensor(a!) h, int kind=1) -> ()");
+  m.def("norm_rope_list(Tensor[] x, Tensor?[] norm_w, Tensor positions, Tensor?[] rope, Tensor(a!)[] out, Tensor?[] out_rows, "
+        "int[] kind, float[] eps, float[] scale, Tensor?[] out_t) -> ()");
   m.def("norm_rope_rows(Tensor x, Tensor? norm_w, Tensor positions, Tensor? rope, Tensor(a!) out, Tensor? out_rows, "
         "int kind, float eps, float scale=1.0, Tensor(b!)? out_t=None) -> ()");
   m.def("sink_attention(Tensor q, Tensor kcache, Tensor vcache, Tensor block_tables, Tensor q_start, Tensor q_len, "
@@ -860,6 +890,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("stream_step", &stream_step);
   m.impl("gated_act", &gated_act);
   m.impl("norm_rope_rows", &norm_rope_rows);
+  m.impl("norm_rope_list", &norm_rope_list);
   m.impl("sink_attention", &sink_attention);
   m.impl("gate_math", &gate_math);
   m.impl("matrix_scan", &matrix_scan);

@@ -7,12 +7,15 @@
 //                    head with one gain vector for all heads (or without a gain), or nothing;
 //                    rotate-half rotation of each head's leading coordinates; a scale; written to a chosen output row
 //                    (a cache row: keys and values go straight into their pages) in fp32 or bf16
-//   gate_math        decays and gates in place: exp(-exp(A) softplus(x + dt)), sigmoid(x), sigmoid(x)^(1/tau)
+//   gate_math        decays and gates in place: exp(-exp(A) softplus(x + dt)), sigmoid(x), sigmoid(x)^(1/tau), or the first of
+//                    these on a row's left half and the second on its right half
 //   gated_head_norm  out = o / rms(o) * w * silu(gate) per (row, head), or * sigmoid(gate)
 //   rms_mix          out = c * (rms-norm(ya) * wa + rms-norm(yb) * wb)
 //   logit_cap        logits * scale, then cap * tanh(. / cap)
 //
 // Everything is computed in fp32; only xb / h / out of the element type and bf16 cache rows are rounded.
+#include <algorithm>
+
 #include "api_mixers.h"
 
 namespace dsse {
@@ -91,9 +94,7 @@ constexpr int kMaxHeadDim = 512;
 
 // WAVES: most waves of a workgroup
 template <typename OutT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopeParams p) {
-  extern __shared__ float strips[];  // [waves][D]
-  __shared__ float red[16];
+DEV void norm_rope_row(const NormRopeParams& p, int gy, float* strips, float* red) {
   const int row = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = WAVES == 4 ? 4 : blockDim.x >> 6;
   const float* x = p.x + (int64_t)row * p.ldx;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopePara
   const float2* cs = p.rope ? p.rope + (int64_t)pos * p.half : nullptr;
   const int dims = p.rope ? 2 * p.half : 0;
   float* s = strips + wave * p.D;
-  for (int h0 = nw * blockIdx.y; h0 < p.nh; h0 += nw * gridDim.y) {  // uniform trip count: the barriers below are reached by every wave
+  for (int h0 = nw * blockIdx.y; h0 < p.nh; h0 += nw * gy) {  // uniform trip count: the barriers below are reached by every wave
     const int h = h0 + wave;
     const bool on = h < p.nh;
     const float* xh = x + (on ? h : 0) * p.D;
@@ -148,6 +149,19 @@ __global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopePara
   }
 }
 
+// A layer's queries, keys and values (blockIdx.z) in one launch.  What bounds it in a decode step: the launch, 4 to 5 us whatever it
+// moves.  Surodra-wide, 16 rows, ten launches fewer (two of them gates): 703 -> 678 us; 1500 prompt rows of surodra-mid 1813 -> 1792.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopeList l) {
+  extern __shared__ float strips[];  // [waves][D]
+  __shared__ float red[16];
+  const NormRopeParams& p = l.p[blockIdx.z];
+  const int gy = l.gy[blockIdx.z];
+  if ((int)blockIdx.y >= gy) return;  // uniform: another set's share of the grid
+  if (p.out_f32) norm_rope_row<float, WAVES>(p, gy, strips, red);
+  else norm_rope_row<bf16, WAVES>(p, gy, strips, red);
+}
+
 __global__ __launch_bounds__(256) void gate_math_kernel(float* x, int ld, int M, int N, int kind, const float* p1,
                                                         int rep1, const float* p2, int rep2, float c) {
   const int64_t n = (int64_t)M * N;
@@ -157,9 +171,9 @@ __global__ __launch_bounds__(256) void gate_math_kernel(float* x, int ld, int M,
     float* px = x + r * ld + col;
     const float v = *px;
     float o;
-    if (kind == 0) {
+    if (kind == 0 || (kind == 3 && 2 * col < N)) {
       o = expf(-expf(p1[col / rep1]) * softplus_f(v + p2[col / rep2]));
-    } else if (kind == 1) {
+    } else if (kind == 1 || kind == 3) {
       o = sigmoid_f(v);
     } else {
       const float ls = fminf(v, 0.0f) - log1pf(expf(-fabsf(v)));  // log sigmoid(v)
@@ -277,26 +291,33 @@ extern "C" hipError_t dsse_gated_act(const float* gu, int ldg, void* h, int M, i
   return hipGetLastError();
 }
 
-extern "C" hipError_t dsse_norm_rope_rows(const dsse::NormRopeParams* p, hipStream_t st) {
-  if (p->T <= 0 || p->nh <= 0) return hipSuccess;
-  if (p->D > dsse::kMaxHeadDim) return hipErrorInvalidValue;
-  const int groups = (p->nh + 3) / 4;
-  const int waves = p->kind != 1 || p->T > 512 ? 4 : (p->nh < 16 ? (p->nh < 4 ? 4 : p->nh) : 16);
+extern "C" hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st) {
+  if (l.n < 1 || l.n > dsse::NormRopeList::kMost) return hipErrorInvalidValue;
+  int waves = 4, width = 0, most = 0;
+  for (int i = 0; i < l.n; ++i) {
+    const dsse::NormRopeParams& p = l.p[i];
+    if (p.T != l.p[0].T || p.D > dsse::kMaxHeadDim) return hipErrorInvalidValue;
+    if (p.kind == 1 && p.T <= 512 && p.nh > 4) waves = std::max(waves, std::min(p.nh, 16));
+    width = std::max(width, p.D);
+  }
+  const int T = l.p[0].T;
+  if (T <= 0) return hipSuccess;
   // four heads to a workgroup while the rows alone leave the chip idle, then more of them: a workgroup's start (lengths, places,
   // position) costs as much as a group of narrow heads.  One group / all groups per workgroup / this rule, rows x heads x width:
   // 512 x 32 x 64 normed in place 8.4 / 11.4 / 8.2 us, 1000 x 32 x 128 15.3 / 17.5 / 14.7; rotated into bf16, 4096 x 16 x 64
   // 16.8 / 11.2 / 11.4, 4096 x 64 x 64 54.1 / 33.7 / 35.5, 1500 x 32 x 128 16.7 / 15.6 / 16.1.
-  const int each = p->T <= 512 ? 1 : (p->T < 1500 ? 2 : (p->T < 3000 ? 4 : 8));
-  const int gy = (groups + each - 1) / each;
-  const dim3 grid(p->T, p->kind == 1 ? 1 : (gy < 65535 ? gy : 65535));
-  const size_t lds = (size_t)waves * p->D * sizeof(float);
-  if (waves == 4) {
-    if (p->out_f32) hipLaunchKernelGGL((dsse::norm_rope_rows_kernel<float, 4>), grid, dim3(256), lds, st, *p);
-    else hipLaunchKernelGGL((dsse::norm_rope_rows_kernel<bf16, 4>), grid, dim3(256), lds, st, *p);
-  } else {
-    if (p->out_f32) hipLaunchKernelGGL((dsse::norm_rope_rows_kernel<float, 16>), grid, dim3(64 * waves), lds, st, *p);
-    else hipLaunchKernelGGL((dsse::norm_rope_rows_kernel<bf16, 16>), grid, dim3(64 * waves), lds, st, *p);
+  const int each = T <= 512 ? 1 : (T < 1500 ? 2 : (T < 3000 ? 4 : 8));
+  for (int i = 0; i < l.n; ++i) {
+    const dsse::NormRopeParams& p = l.p[i];
+    const int groups = (p.nh + waves - 1) / waves;
+    l.gy[i] = p.nh <= 0 ? 0 : (p.kind == 1 ? 1 : std::min((groups + each - 1) / each, 65535));
+    most = std::max(most, l.gy[i]);
   }
+  if (most <= 0) return hipSuccess;
+  const dim3 grid(T, most, l.n);
+  const size_t lds = (size_t)waves * width * sizeof(float);
+  if (waves == 4) hipLaunchKernelGGL(dsse::norm_rope_rows_kernel<4>, grid, dim3(256), lds, st, l);
+  else hipLaunchKernelGGL(dsse::norm_rope_rows_kernel<16>, grid, dim3(64 * waves), lds, st, l);
   return hipGetLastError();
 }
 

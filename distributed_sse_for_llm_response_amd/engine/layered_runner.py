@@ -547,10 +547,8 @@ class LayeredRunner(RunnerBase):
             ops.conv_state(big[:, :C], Lw.conv, None, self.state.tail.get(ri), g["qs"], g["ql"], g["ctx"], g["ss"], cv,
                            None, None, 1)
         q, k, v = self._cols(cv, 0, G, D), self._cols(cv, G * D, G, D), self._cols(cv, 2 * G * D, H, V)
-        ops.norm_rope_rows(q, None, pos, None, q, None, 2, UNIT_EPS, D ** -0.5)
-        ops.norm_rope_rows(k, None, pos, None, k, None, 2, UNIT_EPS, 1.0)
-        ops.gate_math(small[:, :H], 0, Lw.a_log, Lw.dt_bias)
-        ops.gate_math(small[:, H:], 1)
+        ops.norm_rope_list(pos, (q, None, None, q, None, 2, UNIT_EPS, D ** -0.5, None), (k, None, None, k, None, 2, UNIT_EPS, 1.0, None))
+        ops.gate_math(small, 3, Lw.a_log, Lw.dt_bias)
         self._scan_out(ri, Lw.norm, big[:, C:C + H * V], H, V, M, d, q, k, v, small[:, :H], small[:, H:], groups, 1.0,
                        Lw.o, Lw.o_t, d["y"])
 
@@ -566,11 +564,10 @@ class LayeredRunner(RunnerBase):
         # left: softmax attention with a sink over this run's pages
         rope = self._rope.get(a.rot)
         qa = d["qa"][:M * H * D].view(M, H, D)
-        ops.norm_rope_rows(self._cols(big, 0, H, D), Lw.q_norm, pos, rope, qa, None, 1, self.cfg.eps, 1.0)
-        ops.norm_rope_rows(self._cols(big, H * D, G, D), Lw.k_norm, pos, rope, self.kv.k[ri], slots, 1, self.cfg.eps,
-                           1.0)
         vt = self.kv.vt.get(ri)
-        ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, None, self.kv.v[ri], slots, 0, 0.0, 1.0, vt)
+        ops.norm_rope_list(pos, (self._cols(big, 0, H, D), Lw.q_norm, rope, qa, None, 1, self.cfg.eps, 1.0, None),
+                           (self._cols(big, H * D, G, D), Lw.k_norm, rope, self.kv.k[ri], slots, 1, self.cfg.eps, 1.0, None),
+                           (self._cols(big, (H + G) * D, G, V), None, None, self.kv.v[ri], slots, 0, 0.0, 1.0, vt))
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
             if g["qt"] > 1:  # prompt portions
@@ -606,8 +603,7 @@ class LayeredRunner(RunnerBase):
         self._lin(d["xb"], Lw.big, Lw.big_t, big)
         rope = self._rope.get(m.rot)
         q, k, v = self._cols(big, 0, H, D), self._cols(big, H * D, H, D), self._cols(big, 2 * H * D, H, V)
-        ops.norm_rope_rows(q, None, pos, rope, q, None, 0, 0.0, 1.0)
-        ops.norm_rope_rows(k, None, pos, rope, k, None, 0, 0.0, D ** -0.5)
+        ops.norm_rope_list(pos, (q, None, rope, q, None, 0, 0.0, 1.0, None), (k, None, rope, k, None, 0, 0.0, D ** -0.5, None))
         self._scan_out(ri, None, big[:, 2 * H * D + H * V:], H, V, M, d, q, k, v, Lw.decay, None, groups, 1.0, Lw.o,
                        Lw.o_t, d["y"])
 
@@ -782,9 +778,9 @@ class LayeredRunner(RunnerBase):
         kc, vc, vt = self.kv.paged.k[ri], self.kv.paged.v[ri], self.kv.paged.vt.get(ri)
         qa = d["qa"][:M * H * D].view(M, H, D)
         eps = self.cfg.eps
-        ops.norm_rope_rows(self._cols(big, 0, H, D), Lw.q_norm, pos, None, qa, None, 3, eps, 1.0)
-        ops.norm_rope_rows(self._cols(big, H * D, G, D), Lw.k_norm, pos, None, kc, slots, 3, eps, 1.0)
-        ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, None, vc, slots, 0, 0.0, 1.0, vt)
+        ops.norm_rope_list(pos, (self._cols(big, 0, H, D), Lw.q_norm, None, qa, None, 3, eps, 1.0, None),
+                           (self._cols(big, H * D, G, D), Lw.k_norm, None, kc, slots, 3, eps, 1.0, None),
+                           (self._cols(big, (H + G) * D, G, V), None, None, vc, slots, 0, 0.0, 1.0, vt))
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:
             if g["qt"] > 1:
@@ -976,9 +972,9 @@ class LayeredRunner(RunnerBase):
         vrope = self._rope[HalfRotarySpec(dims=V, base=m.rot_base)]
         qa = d["qa"][:M * H * D].view(M, H, D)
         eps = self.cfg.eps
-        ops.norm_rope_rows(self._cols(big, 0, H, D), Lw.q_norm, pos, rope, qa, None, 1, eps, 1.0)
-        ops.norm_rope_rows(self._cols(big, H * D, G, D), Lw.k_norm, pos, rope, kc, slots, 1, eps, 1.0)
-        ops.norm_rope_rows(self._cols(big, (H + G) * D, G, V), None, pos, vrope, vc, slots, 3, eps, 1.0, vt)
+        ops.norm_rope_list(pos, (self._cols(big, 0, H, D), Lw.q_norm, rope, qa, None, 1, eps, 1.0, None),
+                           (self._cols(big, H * D, G, D), Lw.k_norm, rope, kc, slots, 1, eps, 1.0, None),
+                           (self._cols(big, (H + G) * D, G, V), None, vrope, vc, slots, 3, eps, 1.0, vt))
         gate = big[:, (H + G) * D + G * V:(H + G) * D + G * V + H]
         ao = d["ao"][:M * H * V].view(M, H, V)
         for g in groups:

@@ -217,6 +217,17 @@ def norm_rope_rows(x, norm_w, positions, rope, out, out_rows, norm_kind: int, ep
         lref.norm_rope_rows(x, norm_w, positions, rope, out, out_rows, norm_kind, eps, scale, out_t)
 
 
+def norm_rope_list(positions, *sets):
+    """norm_rope_rows of up to three sets of heads of the same rows in one launch: each set (x, norm_w, rope, out, out_rows,
+    norm_kind, eps, scale, out_t), with inputs and outputs that do not overlap between sets."""
+    if _hip(sets[0][0]):
+        x, norm_w, rope, out, out_rows, kind, eps, scale, out_t = map(list, zip(*sets))
+        torch.ops.dsse.norm_rope_list(x, norm_w, positions, rope, out, out_rows, kind, eps, scale, out_t)
+    else:
+        for x, norm_w, rope, out, out_rows, kind, eps, scale, out_t in sets:
+            lref.norm_rope_rows(x, norm_w, positions, rope, out, out_rows, kind, eps, scale, out_t)
+
+
 SINK_FLASH_TILES = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 20, 24, 32)  # value widths / 16 the MFMA form is built for
 
 
@@ -283,7 +294,7 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, wor
 
 def gate_math(x, kind: int, p1=None, p2=None, c: float = 1.0):
     """In place on fp32 x [T, N] (a column slice is fine): 0: exp(-exp(p1) * softplus(x + p2)); 1: sigmoid(x);
-    2: sigmoid(x)^(1 / c).  p1 and p2 hold N numbers, or N / k of them: each then serves k neighbouring columns (one
+    2: sigmoid(x)^(1 / c); 3: kind 0 on the left half of a row, kind 1 on the right.  p1 and p2 hold N numbers, or N / k of them: each then serves k neighbouring columns (one
     rate per head beside one bias per head and channel)."""
     if _hip(x):
         torch.ops.dsse.gate_math(x, kind, p1, p2, c)

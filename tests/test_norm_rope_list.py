@@ -1,0 +1,75 @@
+"""Several sets of heads normed, rotated and written in one launch (csrc/kernels/stream_ops.hip) against one launch each, and the two
+kinds of gates on the halves of a row."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+
+UNIT, ROW, HEAD, NONE = 2, 1, 3, 0
+
+
+def gates(T, H, dev):
+    g = torch.Generator().manual_seed(H)
+    x = torch.randn(T, 2 * H + 3, generator=g)
+    p1, p2 = torch.randn(H, generator=g), torch.randn(H, generator=g)
+    want = x.clone()
+    lref.gate_math(want[:, 1:1 + H], 0, p1, p2, 1.0)
+    lref.gate_math(want[:, 1 + H:1 + 2 * H], 1, None, None, 1.0)
+    got = x.to(dev)
+    ops.gate_math(got[:, 1:1 + 2 * H], 3, p1.to(dev), p2.to(dev))
+    assert torch.allclose(got.cpu(), want, rtol=4e-6, atol=1e-6)   # three exponentials of 2 ulp each
+
+
+def test_gate_halves_cpu():
+    gates(5, 3, "cpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H", [(1, 1), (7, 16), (300, 33)])
+def test_gate_halves(T, H):
+    gates(T, H, "cuda")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,G,D,V", [(1, 32, 8, 128, 128), (16, 20, 4, 64, 96), (513, 3, 3, 32, 48), (1600, 16, 8, 128, 64)])
+@pytest.mark.parametrize("kinds", [(ROW, ROW, NONE), (HEAD, HEAD, NONE), (UNIT, UNIT, HEAD)])
+def test_list_equals_single_launches(T, H, G, D, V, kinds):
+    """Queries in place or to a buffer of their own, keys and values to cache rows (some skipped), values to transposed pages too.
+    A row norm's sum goes over more waves beside wider rows: its rounding, 2^-22 of a value, is the only difference."""
+    g = torch.Generator().manual_seed(T)
+    wide = torch.randn(T, H * D + G * D + G * V, generator=g).cuda()
+    pages = T // 32 + 2
+    slots = torch.randperm(pages * 32, generator=g)[:T].to(torch.int32)
+    slots[1::5] = -1
+    slots, pos = slots.cuda(), torch.randint(0, 64, (T,), generator=g).to(torch.int32).cuda()
+    rope = torch.randn(64, D // 2, 2, generator=g).cuda()
+    gain = [torch.randn(n, generator=g).cuda() for n in (H * D if kinds[0] == ROW else D, G * D if kinds[1] == ROW else D, V)]
+
+    def sets(x):
+        q, k, v = x[:, :H * D].unflatten(1, (H, D)), x[:, H * D:(H + G) * D].unflatten(1, (G, D)), x[:, (H + G) * D:].unflatten(1, (G, V))
+        kc = torch.zeros(pages, 32, G, D, device="cuda", dtype=torch.bfloat16)
+        vc, vt = torch.zeros(pages, 32, G, V, device="cuda", dtype=torch.bfloat16), torch.zeros(pages, G, V, 32, device="cuda", dtype=torch.bfloat16)
+        w = [a if n in (ROW, HEAD) else None for a, n in zip(gain, kinds)]
+        return [(q, w[0], rope, q, None, kinds[0], 1e-5, 0.25, None), (k, w[1], rope, kc, slots, kinds[1], 1e-5, 1.0, None),
+                (v, w[2], None, vc, slots, kinds[2], 1e-5, 1.0, vt)]
+
+    one, each = wide.clone(), wide.clone()
+    a, b = sets(one), sets(each)
+    ops.norm_rope_list(pos, *a)
+    for x, w, r, out, rows, kind, eps, scale, out_t in b:
+        ops.norm_rope_rows(x, w, pos, r, out, rows, kind, eps, scale, out_t)
+    assert torch.allclose(one, each, rtol=2.0 ** -21, atol=2.0 ** -20)
+    for (_, _, _, oa, *_, ta), (_, _, _, ob, *_, tb) in zip(a[1:], b[1:]):
+        assert torch.allclose(oa.float(), ob.float(), rtol=2.0 ** -7, atol=2.0 ** -20) and oa.any()   # a value may round to the other side
+        assert ta is None or torch.allclose(ta.float(), tb.float(), rtol=2.0 ** -7, atol=2.0 ** -20)
+    two = sets(wide.clone())[:2]   # fewer sets
+    ops.norm_rope_list(pos, *two)
+    assert torch.equal(two[1][3], a[1][3])
+
+
+def test_list_cpu():
+    x, w = torch.randn(4, 2, 8), torch.randn(16)
+    pos, outs = torch.zeros(4, dtype=torch.int32), [torch.zeros(4, 2, 8) for _ in range(2)]
+    ops.norm_rope_list(pos, (x, w, None, outs[0], None, 1, 1e-5, 1.0, None), (x, None, None, outs[1], None, 2, 1e-6, 2.0, None))
+    assert torch.allclose(outs[1].norm(dim=-1), torch.full((4, 2), 2.0), atol=1e-4) and outs[0].any()
