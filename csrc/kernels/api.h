@@ -33,6 +33,7 @@ struct GemmEpi {
   // timed-out waits, then the per-tile ticket and done counters (zero between launches: each tile's last arriver
   // resets its pair); null when unused
   int* fix_cnt;
+  int gelu;               // mode 3: the gate's activation is GELU (tanh form) instead of SiLU
 };
 constexpr int kFixTiles = 8192;  // tiles of one fix-up launch at most
 // the per-device counter block (bindings.cpp fix_state): [4 words][2 kFixTiles GEMM fix-up counters]

@@ -700,7 +700,7 @@ int64_t gemm_out_split(const Tensor& x, const Tensor& w, Tensor& out, Tensor& pa
   return 0;
 }
 
-void gemm_silu(const Tensor& x, const Tensor& w, Tensor& out) {
+void gated_gemm(const Tensor& x, const Tensor& w, Tensor& out, bool gelu) {
   check_gpu(out, "out");
   check_dtype(out, at::kBFloat16, "out");
   TORCH_CHECK(out.dim() == 2 && out.size(0) == x.size(0) && out.size(1) * 2 == w.size(0),
@@ -708,8 +708,11 @@ void gemm_silu(const Tensor& x, const Tensor& w, Tensor& out) {
   dsse::GemmEpi ep{};
   ep.out = out.data_ptr();
   ep.ldo = (int)out.size(1);
+  ep.gelu = gelu;
   run_gemm(dsse::kSiluMul, x, w, ep);
 }
+void gemm_silu(const Tensor& x, const Tensor& w, Tensor& out) { gated_gemm(x, w, out, false); }
+void gemm_gelu(const Tensor& x, const Tensor& w, Tensor& out) { gated_gemm(x, w, out, true); }
 
 void gemm_qkv_rope(const Tensor& x, const Tensor& w, const Tensor& positions, const Tensor& slots,
                    const Tensor& rope, Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh,
@@ -1342,6 +1345,7 @@ TORCH_LIBRARY(dsse, m) {
   m.def("gemm_out(Tensor x, Tensor w, Tensor(a!) out) -> ()");
   m.def("gemm_resid(Tensor x, Tensor w, Tensor(a!) resid) -> ()");
   m.def("gemm_silu(Tensor x, Tensor w, Tensor(a!) out) -> ()");
+  m.def("gemm_gelu(Tensor x, Tensor w, Tensor(a!) out) -> ()");
   m.def("gemm_qkv_rope(Tensor x, Tensor w, Tensor positions, Tensor slots, Tensor rope, Tensor(a!) q_out, "
         "Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv) -> ()");
   m.def("rmsnorm(Tensor(a!) resid, Tensor w, Tensor(b!) y, float eps, Tensor? delta=None, Tensor? embed=None, "
@@ -1395,6 +1399,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("gemm_resid_split", &gemm_resid_split);
   m.impl("gemm_out_split", &gemm_out_split);
   m.impl("gemm_silu", &gemm_silu);
+  m.impl("gemm_gelu", &gemm_gelu);
   m.impl("gemm_qkv_rope", &gemm_qkv_rope);
   m.impl("rmsnorm", &rmsnorm);
   m.impl("rope_kv_write", &rope_kv_write);

@@ -20,7 +20,7 @@
 //     (QKV).  The paired epilogues rely on the engine's weight-row permutation: inside each
 //     16-row tile, rows 0..7 and 8..15 are partners (gate/up, or rotary dims d and d+64), so
 //     the partner value is one __shfl_xor(·, 8) away.
-#include "api.h"
+#include "gemm_epilogue.h"
 
 namespace dsse {
 
@@ -134,7 +134,7 @@ skinny_gemm_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __res
           const float partner = __shfl_xor(v, 8);
           if (r < 8 && m < M)
             reinterpret_cast<bf16*>(ep.out)[(size_t)m * ep.ldo + tile * 8 + r] =
-                f2bf(silu(v) * partner);
+                f2bf(gate_act(ep, v) * partner);
         } else if constexpr (MODE == kQkvRope) {
           const float partner = __shfl_xor(v, 8);
           const int unit = tile >> 3, j = tile & 7;

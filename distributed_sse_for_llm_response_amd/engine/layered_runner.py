@@ -35,7 +35,7 @@ same weights and its own pages and state slots per pass:
                             GEMM (fp32) -> gate_math -> matrix_scan (per-channel decay) -> gated_head_norm -> output
                             GEMM; rms_mix of the two
     retention layer         fused GEMM -> rotation of q, k -> matrix_scan (fixed decay) -> gated_head_norm -> output GEMM
-    feed-forward            fused [gate | up] GEMM -> gated_act (gelu) -> down GEMM
+    feed-forward            fused gate, up GEMM with gelu(gate) * up as its epilogue (exact mode and small shapes: gated_act) -> down GEMM
     head                    stream_step (last add + final norm) -> head GEMM -> logit_cap (scale, tanh cap)
 
 Prompt groups take the recurrences by chunks of 16 tokens on the matrix cores in matrix_scan, as a two-level walk
@@ -439,7 +439,7 @@ class LayeredRunner(RunnerBase):
         cfg, dev = self.cfg, self.device
         f32 = dict(device=dev, dtype=torch.float32)
         el = dict(device=dev, dtype=self.dtype)
-        big = cv = z = qa = o = ff = 1
+        big = cv = z = qa = o = ff = gu = 1
         for i, L in enumerate(cfg.layers):
             m = L.mixer
             if L.kind == "delta":
@@ -454,10 +454,11 @@ class LayeredRunner(RunnerBase):
                 big, o = max(big, 2 * m.heads * (m.dim + m.vdim)), max(o, m.heads * m.vdim)
             if L.mlp is not None:
                 ff = max(ff, L.mlp.ff)
+                gu = max(gu, 0 if self.w.layers[i].mlp.gu is None else 2 * L.mlp.ff)
         return {"y2": new(M, cfg.width, **f32), "big": new(M * big, **f32),
                 "cv": new(M * cv, **f32), "z": new(M * z, **f32),
                 "qa": new(M * qa, **f32), "o": new(M * o, **f32), "ao": new(M * o, **el),
-                "gu": new(M * 2 * ff, **f32), "h": new(M * ff, **el)}
+                "gu": new(M * gu, **f32), "h": new(M * ff, **el)}
 
     def _prenorm_layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None) -> None:
         """Every layer run over M packed rows.  Between sublayers ONE stream_step adds the finished sublayer's output
@@ -486,10 +487,13 @@ class LayeredRunner(RunnerBase):
             ops.stream_step(pending, mult, d["resid"], None, None, None, None, None, None, None)
 
     def _dense_ff(self, f, Fw, M: int, d: dict) -> None:
-        gu = d["gu"][:M * 2 * f.ff].view(M, 2 * f.ff)
         h = d["h"][:M * f.ff].view(M, f.ff)
-        self._lin(d["xb"], Fw.gu, Fw.gu_t, gu)
-        ops.gated_act(gu, h, 1)
+        if Fw.gu_t is not None:
+            ops.gemm_gelu(d["xb"], Fw.gu_t, h)
+        else:
+            gu = d["gu"][:M * 2 * f.ff].view(M, 2 * f.ff)
+            ops.gemm_rm(d["xb"], Fw.gu, gu)
+            ops.gated_act(gu, h, 1)
         self._lin(h, Fw.down, Fw.down_t, d["y"])
 
     def _scratch(self, d: dict, name: str, numel: int):

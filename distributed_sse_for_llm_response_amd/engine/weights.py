@@ -430,7 +430,7 @@ class RetentionWeights:
 class DenseFfWeights:
     gu: torch.Tensor         # rows [gate (F) | up (F)] x W
     down: torch.Tensor       # [W, F]
-    gu_t: torch.Tensor = None
+    gu_t: torch.Tensor = None  # tiled, gate and up rows interleaved by eight (ops.gemm_gelu)
     down_t: torch.Tensor = None
 
 
@@ -496,6 +496,8 @@ def convert_surodra(cfg, tensors: dict, device="cpu", dtype=torch.bfloat16) -> L
         if L.mlp is not None:
             layer.norm2 = norm(f"l{i}.norm2")
             layer.mlp = DenseFfWeights(gu=cat(f"l{i}.mlp.gate", f"l{i}.mlp.up"), down=t(f"l{i}.mlp.down"))
+            if fits_tiled(layer.mlp.gu):
+                layer.mlp.gu = layer.mlp.gu[gate_up_perm(L.mlp.ff).to(device)]
             _tile_fields(layer.mlp, ("gu", "down"))
         layers.append(layer)
     out = LayeredWeights(cfg=cfg, embed=t("embed"), layers=layers, final_norm=norm("final.norm"), head=t("head"),

@@ -85,6 +85,14 @@ def gemm_silu(x, w, out):
         ref.gemm_silu(x, w, out)
 
 
+def gemm_gelu(x, w, out):
+    """out[M, N/2] = gelu(gate) * up (tanh form) with the interleaved gate/up weight rows."""
+    if _hip(x):
+        torch.ops.dsse.gemm_gelu(x, w, out)
+    else:
+        ref.gemm_gelu(x, w, out)
+
+
 def gemm_qkv_rope(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv):
     """Fused QKV projection + RoPE + paged KV write (decode)."""
     if _hip(x):

@@ -113,6 +113,12 @@ def gemm_silu(x, w, out):
     out.copy_((torch.nn.functional.silu(g) * u).reshape(x.shape[0], -1).to(out.dtype))
 
 
+def gemm_gelu(x, w, out):
+    y = (x.float() @ untile_weight(w).float().t()).view(x.shape[0], -1, 2, 8)
+    g, u = y[:, :, 0, :], y[:, :, 1, :]
+    out.copy_((torch.nn.functional.gelu(g, approximate="tanh") * u).reshape(x.shape[0], -1).to(out.dtype))
+
+
 def gemm_qkv_rope(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv):
     M = x.shape[0]
     y = x.float() @ untile_weight(w).float().t()
