@@ -315,10 +315,9 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
   DSSE_CHECK_HIP(dsse_sink_attention((int)work_seq.numel(), &p, cur_stream()));
 }
 
-void gate_math(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2, double c) {
+void gate_rows(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2, double c) {
   col_view(x, "x");
   const int M = (int)x.size(0), N = (int)x.size(1);
-  TORCH_CHECK(kind >= 0 && kind <= 3 && (kind != 3 || N % 2 == 0), "kind 0..3, two halves");
   // p1 / p2 hold one number per column (of the left half with kind 3), or one per run of neighbouring columns
   const int64_t cols = kind == 3 ? N / 2 : N;
   const int64_t n1 = p1.has_value() ? p1->numel() : cols, n2 = p2.has_value() ? p2->numel() : cols;
@@ -329,6 +328,17 @@ void gate_math(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2
   TORCH_CHECK(kind != 2 || c > 0, "kind 2 needs c > 0");
   DSSE_CHECK_HIP(dsse_gate_math(x.data_ptr<float>(), (int)x.stride(0), M, N, (int)kind, a, (int)(cols / n1), b, (int)(cols / n2),
                                 (float)c, cur_stream()));
+}
+
+void gate_math(Tensor& x, int64_t kind, const OptTensor& p1, const OptTensor& p2, double c) {
+  TORCH_CHECK(kind >= 0 && kind <= 2, "kind 0..2");
+  gate_rows(x, kind, p1, p2, c);
+}
+
+// gate_math kind 0 on a row's left half, kind 1 on its right half
+void gate_pair(Tensor& x, const Tensor& p1, const Tensor& p2) {
+  TORCH_CHECK(x.dim() == 2 && x.size(1) % 2 == 0, "x must be [T, 2 N]");
+  gate_rows(x, 3, p1, p2, 1.0);
 }
 
 void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
@@ -862,6 +872,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "float scale, int qt, Tensor? vt=None, bool split=False, float softcap=0.0, Tensor? out_rope=None, "
         "Tensor? rel=None, int keep_first=0, float out_scale=1.0, Tensor(b!)? part=None, int nparts=1) -> ()");
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
+  m.def("gate_pair(Tensor(a!) x, Tensor p1, Tensor p2) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
         "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
   m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest, "
@@ -893,6 +904,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("norm_rope_list", &norm_rope_list);
   m.impl("sink_attention", &sink_attention);
   m.impl("gate_math", &gate_math);
+  m.impl("gate_pair", &gate_pair);
   m.impl("matrix_scan", &matrix_scan);
   m.impl("matrix_scan_chunked", &matrix_scan_chunked);
   m.impl("gated_head_norm", &gated_head_norm);

@@ -27,7 +27,7 @@ same weights and its own pages and state slots per pass:
     stream_step             resid += m * (finished sublayer) (+ embedding again + the pass's vector at a pass's start);
                             xb = tanh(alpha resid) w + b -- the add, the pass additions and the next norm in one kernel
     delta layer             ONE fused GEMM [q | k | v | g | a | b] (fp32 out) -> conv_state over q | k | v (SiLU; slot
-                            tail) -> unit q, k per head -> gate_math (decay, write strength) -> matrix_scan (delta rule;
+                            tail) -> unit q, k per head -> gate_pair (decay, write strength) -> matrix_scan (delta rule;
                             slot state) -> gated_head_norm -> output GEMM
     parallel layer          ONE fused GEMM for both halves -> left: norm_rope_rows (whole-row RMS norm + rotation: q to
                             a buffer, k and v into this run's pages) -> sink_attention (MFMA form over transposed value
@@ -552,7 +552,7 @@ class LayeredRunner(RunnerBase):
                            None, None, 1)
         q, k, v = self._cols(cv, 0, G, D), self._cols(cv, G * D, G, D), self._cols(cv, 2 * G * D, H, V)
         ops.norm_rope_list(pos, (q, None, None, q, None, 2, UNIT_EPS, D ** -0.5, None), (k, None, None, k, None, 2, UNIT_EPS, 1.0, None))
-        ops.gate_math(small, 3, Lw.a_log, Lw.dt_bias)
+        ops.gate_pair(small, Lw.a_log, Lw.dt_bias)
         self._scan_out(ri, Lw.norm, big[:, C:C + H * V], H, V, M, d, q, k, v, small[:, :H], small[:, H:], groups, 1.0,
                        Lw.o, Lw.o_t, d["y"])
 

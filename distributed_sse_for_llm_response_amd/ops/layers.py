@@ -294,12 +294,22 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, wor
 
 def gate_math(x, kind: int, p1=None, p2=None, c: float = 1.0):
     """In place on fp32 x [T, N] (a column slice is fine): 0: exp(-exp(p1) * softplus(x + p2)); 1: sigmoid(x);
-    2: sigmoid(x)^(1 / c); 3: kind 0 on the left half of a row, kind 1 on the right.  p1 and p2 hold N numbers, or N / k of them: each then serves k neighbouring columns (one
+    2: sigmoid(x)^(1 / c).  p1 and p2 hold N numbers, or N / k of them: each then serves k neighbouring columns (one
     rate per head beside one bias per head and channel)."""
     if _hip(x):
         torch.ops.dsse.gate_math(x, kind, p1, p2, c)
     else:
         lref.gate_math(x, kind, p1, p2, c)
+
+
+def gate_pair(x, p1, p2):
+    """gate_math of kind 0 on the left half of fp32 rows x [T, 2 N] and of kind 1 on the right half, in one launch."""
+    if _hip(x):
+        torch.ops.dsse.gate_pair(x, p1, p2)
+    else:
+        N = x.shape[1] // 2
+        lref.gate_math(x[:, :N], 0, p1, p2, 1.0)
+        lref.gate_math(x[:, N:], 1, None, None, 1.0)
 
 
 def matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale: float = 1.0,

@@ -343,12 +343,7 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, sin
 
 def gate_math(x, kind, p1, p2, c):
     """In place on fp32 x [T, N]: kind 0: exp(-exp(p1) * softplus(x + p2)) (p1, p2 [N]); 1: sigmoid(x);
-    2: sigmoid(x)^(1 / c) as exp(logsigmoid(x) / c); 3: kind 0 on a row's left half, kind 1 on its right half."""
-    if kind == 3:
-        H = x.shape[1] // 2
-        gate_math(x[:, :H], 0, p1, p2, c)
-        gate_math(x[:, H:], 1, None, None, c)
-        return
+    2: sigmoid(x)^(1 / c) as exp(logsigmoid(x) / c)."""
     if kind == 0:  # p1, p2 may be shorter than a row: each entry then serves a run of neighbouring columns
         N = x.shape[1]
         a = p1.float().repeat_interleave(N // p1.numel())

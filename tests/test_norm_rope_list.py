@@ -17,7 +17,7 @@ def gates(T, H, dev):
     lref.gate_math(want[:, 1:1 + H], 0, p1, p2, 1.0)
     lref.gate_math(want[:, 1 + H:1 + 2 * H], 1, None, None, 1.0)
     got = x.to(dev)
-    ops.gate_math(got[:, 1:1 + 2 * H], 3, p1.to(dev), p2.to(dev))
+    ops.gate_pair(got[:, 1:1 + 2 * H], p1.to(dev), p2.to(dev))
     assert torch.allclose(got.cpu(), want, rtol=4e-6, atol=1e-6)   # three exponentials of 2 ulp each
 
 
