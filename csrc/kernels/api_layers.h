@@ -108,6 +108,7 @@ struct LruScanParams {
   int nseq, C, bw, rows; // rows = T
   int coeff;             // 1: compute (a, b) for all rows first; 0: gates already hold them (a later sequence group)
   int alone;             // 1 (with coeff): the sequences hold all T rows, and nobody reads the coefficients afterwards
+  int longest;           // rows of the longest sequence, as far as the caller knows (rows otherwise): only chooses the form
   float* chunk_a;        // [rows / 32 + nseq + 1, C] scratch of the chunked walk (prompt portions), or null
   float* chunk_b;
   float c;               // 8: log a = -c r softplus(lam)

@@ -328,7 +328,7 @@ void conv_state(const Tensor& in, const Tensor& taps, const OptTensor& bias, con
 
 void lru_scan(const Tensor& u, Tensor& gates, const Tensor& y, const Tensor& lam, Tensor& state,
               const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len, const Tensor& state_slot, Tensor& out,
-              double c, const OptTensor& y_bias, bool coeff, const OptTensor& scratch, bool alone) {
+              double c, const OptTensor& y_bias, bool coeff, const OptTensor& scratch, bool alone, int64_t longest) {
   f32t(u, "u");
   f32t(gates, "gates");
   f32t(y, "y");
@@ -355,6 +355,7 @@ void lru_scan(const Tensor& u, Tensor& gates, const Tensor& y, const Tensor& lam
   p.rows = (int)u.size(0);
   p.coeff = coeff ? 1 : 0;
   p.alone = alone ? 1 : 0;
+  p.longest = longest > 0 && longest < p.rows ? (int)longest : p.rows;
   if (scratch.has_value()) {  // [2, slots, C] with slots >= rows / 32 + sequences + 1: the chunked walk's scratch
     f32t(*scratch, "scratch");
     const int64_t slots = p.rows / 32 + p.nseq + 1;
@@ -629,7 +630,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "bool single=False) -> ()");
   m.def("lru_scan(Tensor u, Tensor(c!) gates, Tensor y, Tensor lam, Tensor(a!) state, Tensor q_start, Tensor q_len, "
         "Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float c, Tensor? y_bias=None, bool coeff=True, "
-        "Tensor(d!)? scratch=None, bool alone=False) -> ()");
+        "Tensor(d!)? scratch=None, bool alone=False, int longest=0) -> ()");
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "

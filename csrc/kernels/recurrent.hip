@@ -14,6 +14,8 @@
 // thread per (sequence, channel) -- a decode step is one iteration.  The biases of the two input projections and the
 // gelu of the branch are applied here, so those projections are plain GEMMs with fp32 output.  Everything here is fp32
 // whatever the element type of the projections around it.
+#include <algorithm>
+
 #include "api_layers.h"
 
 namespace dsse {
@@ -215,8 +217,9 @@ __global__ __launch_bounds__(256) void lru_scan_kernel(LruScanParams p) {
   *st = S;
 }
 
-// A step that is all of u's rows and few per sequence (decode): coefficients and walk in one launch, the gates stay as they are
-// (one row each of 160 sequences x 2560 channels: 20.1 us in four launches, 6.4 in this one; 16 sequences 9.0 in two, 4.7)
+// A step that is all of u's rows and few of every sequence (decode): coefficients and walk in one launch, the gates stay as they are
+// (one row each of 160 sequences x 2560 channels: 20.1 us in four launches, 6.4 in this one; 16 sequences 9.0 in two, 4.7).  Its
+// chain is the longest sequence's, 0.46 us a row (lru_takes_step).
 template <typename T>
 __global__ __launch_bounds__(256) void lru_step_kernel(LruScanParams p) {
   const int seq = blockIdx.y;
@@ -373,6 +376,14 @@ __global__ __launch_bounds__(256) void lru_chunk_apply_kernel(LruScanParams p, i
   if (fold && t1 == ql) p.state[(int64_t)p.state_slot[seq] * p.C + c] = S;
 }
 
+// One launch or the other forms, by the longest sequence: coefficients in parallel and a walk of 0.19 us a row below kChunkedFrom
+// rows, chunks (a workgroup for every 32 rows of the step per sequence) from there on.  One launch / the others, 2560 channels:
+// 8 rows 6.2 / 6.4, 12 8.0 / 7.1; 63 of 1 row and one of 8 6.9 / 7.5, of 12 8.7 / 8.3, of 32 18 / 12; chunks: 8 of 16 rows 10.0 / 12.6,
+// of 24 13.7 / 16.4, 63 of 1 row and one of 190 89 / 33; 159 of 1 row and one of 24 16 / 23, of 48 27 / 27, 255 and one of 48 28 / 33.
+bool lru_takes_step(const LruScanParams& p, bool chunked) {
+  return p.longest <= (chunked ? std::max(24, std::min(48, p.nseq / 4)) : 8);
+}
+
 }  // namespace
 }  // namespace dsse
 
@@ -402,12 +413,12 @@ extern "C" hipError_t dsse_lru_scan(const dsse::LruScanParams* p, hipStream_t st
   if (p->nseq <= 0 || p->rows <= 0) return hipSuccess;
   dim3 grid((p->C + 255) / 256, p->nseq);
   const bool alone = p->coeff && p->alone;
-  if (alone && p->rows <= 4 * p->nseq) {
+  const bool chunked = p->chunk_a && p->chunk_b && p->rows >= kChunkedFrom;  // prompt portions
+  if (alone && lru_takes_step(*p, chunked)) {
     if (p->f32) hipLaunchKernelGGL(lru_step_kernel<float>, grid, dim3(256), 0, st, *p);
     else hipLaunchKernelGGL(lru_step_kernel<bf16>, grid, dim3(256), 0, st, *p);
     return hipGetLastError();
   }
-  const bool chunked = p->chunk_a && p->chunk_b && p->rows >= kChunkedFrom;  // prompt portions
   if (p->coeff && !(alone && chunked)) {
     const int per = p->rows >= 256 ? 4 : 1;  // few rows: a thread per element fills more of the chip
     dim3 cgrid((p->rows + per - 1) / per, (p->C + 255) / 256);

@@ -358,7 +358,8 @@ class LayeredRunner(RunnerBase):
                 slots = M // 32 + g["ql"].numel() + 1
                 scr = scr[:2 * slots * C].view(2, slots, C)
             ops.lru_scan(u, gates, yr, Lw.lam, self.state.state[li], g["qs"], g["ql"], g["ctx"], g["ss"], hs,
-                         LRU_DECAY_SCALE, Lw.y_b, i == 0, scr, len(groups) == 1)
+                         LRU_DECAY_SCALE, Lw.y_b, i == 0, scr, len(groups) == 1,
+                         1 if g["qt"] == 1 else g["longest"])
         self._lin(hs, Lw.o, Lw.o_t, d["y"])
 
     def _moe(self, f, Fw, M: int, d: dict):
