@@ -579,6 +579,19 @@ void moe_topk(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w) {
                                cur_stream()));
 }
 
+// Which form the expert GEMMs of moe_grouped take for bf16 operands on LDS-DMA: 1 the stream (moe_stream.hip), 0 the pipeline
+// (moe_pipe.hip), -1 shapes that neither takes
+int64_t moe_plan(int64_t M, int64_t W, int64_t F, int64_t Fs, int64_t E, int64_t top, bool gated) {
+  dsse::MoeGroupedParams p{};
+  p.M = (int)M, p.W = (int)W, p.F = (int)F, p.Fs = (int)Fs, p.E = (int)E, p.top = (int)top, p.S = (int)top + (Fs > 0 ? 1 : 0);
+  p.ldh = (int)std::max(F, Fs);
+  alignas(16) static const char aligned[16] = {};
+  p.x = p.up = p.down = p.sgate = p.sup = p.sdown = aligned;
+  p.h = const_cast<char*>(aligned);
+  if (gated) p.gate = aligned;
+  return dsse::moe_lines_ok(p) ? (dsse::moe_stream_pays(p) ? 1 : 0) : -1;
+}
+
 // moe_topk and the work list of moe_grouped (aligned) in one launch, for decode-sized steps; false: nothing done, the step is larger.
 bool moe_topk_lists(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w, Tensor& sorted, Tensor& tile_expert,
                     Tensor& num_tiles, bool shared) {
@@ -633,6 +646,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor(d!)? scratch=None, bool alone=False, int longest=0) -> ()");
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
+  m.def("moe_plan(int M, int W, int F, int Fs, int E, int top, bool gated) -> int", &moe_plan);
   m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "
         "Tensor(e!) num_tiles, bool shared) -> bool");
   m.def("moe_ffn(Tensor x, Tensor topk_idx, Tensor topk_w, Tensor gate, Tensor up, Tensor down, Tensor? sgate, "

@@ -23,7 +23,8 @@
 //
 // Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
 // experts, top 2, shared 7168: 2369 -> 1014 us (1042 TFLOP/s); 2048 rows: 1695 -> 775; 1024 rows of 2048 x 1408, shared
-// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Below 193 rows moe_stream.hip is faster.
+// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Up to 192 rows moe_stream.hip takes
+// the sizes whose weights it need not read twice (moe_stream_pays).
 #include <algorithm>
 #include <cmath>
 

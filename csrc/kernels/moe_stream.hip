@@ -21,6 +21,7 @@
 // 64 320 -> 259, 160 323 -> 314.  On the way (32 rows, the two sizes): without its own first step and the non-temporal
 // hint 79 / 288, with the hint 73 / 261, with both 69 / 250, narrow down tiles 65 / 237; narrow gate / up tiles 64 / 251.
 #include <algorithm>
+#include <cmath>
 
 #include "lds_dma.h"
 #include "moe_rows.h"
@@ -220,10 +221,32 @@ hipError_t launch_moe_stream(const MoeGroupedParams& p, hipStream_t st) {
 
 }  // namespace
 
-// Above three list tiles of a shared expert the stream's 64-row tiles read its weights once too often.  Stream / pipeline, the two
-// sizes above: 160 rows 81 / 95 us and 312 / 300, 192 rows 80 / 96 and 311 / 305, 224 rows 91 / 98 and 355 / 310, 256 rows 92 / 99
-// and 357 / 314; below, the stream is ahead at both (128 rows 74 / 96 and 282 / 298).
-bool moe_stream_pays(const MoeGroupedParams& p) { return p.M <= 192; }
+// To one list tile of every expert the stream reads each weight once and is ahead; from there on it is a matter of cost, in us: the stream
+// 24 and 155 per GB that it reads, a list tile's weights at a time; the pipeline 25, 84 per GB of the weights and 0.63 per K step of its
+// rounds of 256 workgroups.  Fitted over 27 sizes of 64 to 192 rows (rms 7 and 4 %); of 191 pairs four are decided for the slower one by
+// more than 2 %, by 7.5 % at most.  Stream / pipeline at 96, 129, 160, 192 rows, top 2: 16 experts of 4096 x 3584 and a shared one of 7168
+// 285 / 296, 302 / 301, 315 / 303, 313 / 308; 2048 x 1408 and 2816 73 / 95, 78 / 95, 81 / 95, 80 / 96; 5120 x 3584 and 7168 367 / 353, 391 / 364,
+// 406 / 370, 411 / 376; 4 of 4096 x 14336 251 / 363, 398 / 375, 470 / 372, 479 / 374; 8 of them 442 / 539 .. 481 / 566; 4 of 4096 x 3584 and 7168
+// 147 / 170, 217 / 173, 231 / 175, 232 / 176; top 8 of 16 of 4096 x 3584 258 / 240, 387 / 252, 485 / 260, 485 / 264.
+bool moe_stream_pays(const MoeGroupedParams& p) {
+  if (p.M > 3 * kMoeRows) return false;
+  if (p.M <= kMoeRows) return true;
+  const bool shared = p.S > p.top;
+  // list tiles of a routed expert: one, and a second and third as far as its rows' spread reaches over 64 and 128
+  const double rows = std::max(1.0, (double)p.M * p.top / p.E), spread = 3 * std::sqrt(rows);
+  double tiles_r = 1;
+  for (int i = 1; i <= 2; ++i) tiles_r += std::min(1.0, std::max(0.0, 0.5 + (rows - i * kMoeRows) / spread));
+  const int tiles_s = shared ? (p.M + kMoeRows - 1) / kMoeRows : 0;
+  const double unit = (p.gate ? 6e-9 : 4e-9) * p.W;  // GB per hidden unit
+  const double gb_r = unit * p.F * p.E, gb_s = shared ? unit * p.Fs : 0;
+  // the pipeline's K steps: tiles of 256 weight rows, the down product's of a shared expert counted by their length
+  auto blocks = [](int rows_w) { return (rows_w + 255) / 256; };
+  const int per = p.gate ? 2 : 1;
+  const int64_t up = (int64_t)p.E * blocks(per * p.F) + (shared ? blocks(per * p.Fs) : 0);
+  const double down = (double)blocks(p.W) * (p.E + (shared ? (double)p.Fs / p.F : 0));
+  const double steps = (double)((up + 255) / 256) * p.W / 64 + std::max(std::ceil(down / 256) * p.F, shared ? (double)p.Fs : 0.0) / 64;
+  return 24 + 155 * (tiles_r * gb_r + tiles_s * gb_s) <= 25 + 84 * (gb_r + gb_s) + 0.63 * steps;
+}
 
 }  // namespace dsse
 

@@ -1,0 +1,22 @@
+"""Which form the expert GEMMs of up to 192 rows take (csrc/kernels/moe_stream.hip): host code."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+
+STREAM, PIPE = 1, 0
+
+
+# one list tile of every expert; a shared expert's second and third; routed experts whose rows pass 64; both sides of the lines,
+# experts without a gate, the first row count of the pipeline alone, shapes that neither takes
+@pytest.mark.parametrize("M,W,F,Fs,E,top,gated,want", [
+    (1, 4096, 3584, 7168, 16, 2, True, STREAM), (64, 4096, 14336, 0, 4, 4, True, STREAM), (128, 4096, 3584, 7168, 16, 2, True, STREAM),
+    (160, 4096, 3584, 7168, 16, 2, True, PIPE), (192, 4096, 3584, 7168, 16, 2, True, PIPE), (192, 2048, 1408, 2816, 16, 2, True, STREAM),
+    (160, 5120, 3584, 7168, 16, 2, True, PIPE), (160, 3072, 2560, 5120, 16, 2, True, STREAM), (192, 4096, 4096, 0, 16, 2, False, STREAM),
+    (96, 4096, 14336, 0, 4, 2, True, STREAM), (160, 4096, 14336, 0, 4, 2, True, PIPE), (192, 4096, 14336, 0, 8, 2, True, STREAM),
+    (96, 4096, 3584, 7168, 4, 2, True, STREAM), (160, 4096, 3584, 7168, 4, 2, True, PIPE), (160, 4096, 3584, 0, 16, 8, True, PIPE),
+    (192, 2048, 1408, 2816, 64, 6, True, STREAM), (193, 2048, 1408, 2816, 16, 2, True, PIPE), (192, 4096, 3584, 7168, 16, 2, False, STREAM),
+    (64, 2048, 1400, 0, 16, 2, True, -1), (64, 64, 128, 0, 16, 2, True, -1)])
+def test_plan(M, W, F, Fs, E, top, gated, want):
+    ops.load_library(required=True)
+    assert torch.ops.dsse.moe_plan(M, W, F, Fs, E, top, gated) == want
