@@ -387,8 +387,8 @@ gemm_ring_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
 #pragma unroll
     for (int u = 0; u < D; ++u) {
       if (u > 0 && c0 + u >= nch) break;
-      // chunk c0 + u landed for every wave, chunks up to c0 + u + D - 2 still in flight
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 2) * PER) : "memory");
+      // chunk c0 + u landed for every wave, chunks up to c0 + u + D - 2 still in flight; the chunk before has been read
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * PER) : "memory");
       if (DSSE_PIPE_STAMPS && c0 + u == 0) st1 = stamps::now();
       const char* xb = smem + u * G::SLOT;
       const char* wb = xb + G::SLOTX + w * 4096 + lane * 16;
@@ -641,8 +641,8 @@ gemm_ring2_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       if (u > 0 && c0 + u >= nch) break;
-      // own W(c) landed (W(c+1) .. W(c+DW-2) may stay in flight), then X(c) published by the loaders
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((DW - 2) * 4) : "memory");
+      // own W(c) landed (W(c+1) .. W(c+DW-2) may stay in flight) and chunk c-1 read, then X(c) published by the loaders
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((DW - 2) * 4) : "memory");
       const char* xb = smem + G::XOFF + (u % DX) * G::SLOTX;
       const char* wb = wring + (u % DW) * 4096 + lane * 16;
 #pragma unroll

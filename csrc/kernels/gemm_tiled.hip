@@ -175,11 +175,12 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
   if (NS >= 3 && nk > 1) issue(1, 1);
   if (NS == 4 && nk > 2) issue(2, 2);
   for (int t = 0; t < nk; ++t) {
-    // step t's DMA done on this wave (steps t+1 .. t+NS-2 may stay in flight), then everyone's: publish step t
+    // step t's DMA done on this wave (steps t+1 .. t+NS-2 may stay in flight) and its fragments of step t-1 in registers, then
+    // everyone's: publish step t
     const int younger = min(NS - 2, nk - 1 - t);
-    if (NS == 4 && younger == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * INS) : "memory");
-    else if (NS >= 3 && younger >= 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(INS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (NS == 4 && younger == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * INS) : "memory");
+    else if (NS >= 3 && younger >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(INS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // the stage step t+NS-1 overwrites was last read in step t-1, which every wave finished before this barrier.
     // 128x256 tile (the weight-heavy 129-256-row decode buckets): its X half goes out now, its weight half between
     // the two MFMA clusters, so the DMA issue is spread over the step (the order gemm_pipe.hip measured faster):
