@@ -43,7 +43,7 @@ struct NormRopeParams {
   int out_f32;
 };
 
-// Up to three sets of heads of the same rows in one launch: their inputs and outputs do not overlap (each may work in place)
+// Up to three sets of heads of the same rows in one launch: none reads or writes what another writes (each may work in place)
 struct NormRopeList {
   static constexpr int kMost = 3;
   NormRopeParams p[kMost];

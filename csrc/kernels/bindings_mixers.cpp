@@ -182,7 +182,27 @@ void norm_rope_rows(const Tensor& x, const OptTensor& norm_w, const Tensor& posi
   DSSE_CHECK_HIP(dsse_norm_rope_rows(l, cur_stream()));
 }
 
-// norm_rope_rows of up to three sets of heads of the same rows in one launch
+// Bytes of a tensor: `rows` runs of `width`, a pitch apart
+struct Extent {
+  uintptr_t at;
+  int64_t rows, pitch, width;
+  uintptr_t end() const { return at + (rows - 1) * pitch + width; }
+};
+Extent rows_extent(const Tensor& t) {
+  const int64_t e = t.element_size();
+  return {(uintptr_t)t.data_ptr(), t.size(0), t.stride(0) * e, t.size(1) * t.size(2) * e};
+}
+Extent whole_extent(const Tensor& t) { return {(uintptr_t)t.data_ptr(), 1, 0, t.numel() * t.element_size()}; }
+bool apart(const Extent& a, const Extent& b) {
+  if (a.end() <= b.at || b.end() <= a.at) return true;
+  if (a.rows < 2 || b.rows < 2 || a.pitch != b.pitch) return false;
+  int64_t off = (int64_t)(b.at - a.at) % a.pitch;  // columns of the same rows
+  if (off < 0) off += a.pitch;
+  return off >= a.width && off + b.width <= a.pitch;
+}
+
+// norm_rope_rows of up to three sets of heads of the same rows in one launch: the sets run side by side, so sets that meet in memory
+// (one reads or writes what another writes) go one after another instead, a launch each
 void norm_rope_list(at::TensorList x, const c10::List<OptTensor>& norm_w, const Tensor& positions, const c10::List<OptTensor>& rope,
                     at::TensorList out, const c10::List<OptTensor>& out_rows, at::IntArrayRef kind, at::ArrayRef<double> eps,
                     at::ArrayRef<double> scale, const c10::List<OptTensor>& out_t) {
@@ -191,10 +211,31 @@ void norm_rope_list(at::TensorList x, const c10::List<OptTensor>& norm_w, const 
                   out_rows.size() == n && kind.size() == n && eps.size() == n && scale.size() == n && out_t.size() == n,
               "one to three sets of heads, an entry of every list each");
   dsse::NormRopeList l{};
+  Extent writes[dsse::NormRopeList::kMost][2];
+  int nw[dsse::NormRopeList::kMost];
   for (size_t i = 0; i < n; ++i) {
-    TORCH_CHECK(x[i].size(0) == x[0].size(0), "every set of heads has the same rows");
     l.p[i] = norm_rope_params(x[i], norm_w.get(i), positions, rope.get(i), out[i], out_rows.get(i), kind[i], eps[i], scale[i],
                               out_t.get(i));
+    TORCH_CHECK(l.p[i].T == l.p[0].T, "every set of heads has the same rows");
+    nw[i] = 0;
+    writes[i][nw[i]++] = out_rows.get(i).has_value() ? whole_extent(out[i]) : rows_extent(out[i]);
+    if (const OptTensor t = out_t.get(i); t.has_value()) writes[i][nw[i]++] = whole_extent(*t);
+  }
+  bool meet = false;
+  for (size_t i = 0; i < n; ++i)
+    for (size_t j = 0; j < n; ++j)
+      for (int a = 0; a < nw[i] && j != i; ++a) {
+        meet |= !apart(writes[i][a], rows_extent(x[j]));
+        for (int b = 0; b < nw[j]; ++b) meet |= !apart(writes[i][a], writes[j][b]);
+      }
+  if (meet && l.p[0].T > 0) {
+    for (size_t i = 0; i < n; ++i) {
+      dsse::NormRopeList one{};
+      one.p[0] = l.p[i];
+      one.n = 1;
+      DSSE_CHECK_HIP(dsse_norm_rope_rows(one, cur_stream()));
+    }
+    return;
   }
   l.n = (int)n;
   DSSE_CHECK_HIP(dsse_norm_rope_rows(l, cur_stream()));
@@ -864,7 +905,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor? w, Tensor? b, Tensor(b!)? xb) -> ()");
   m.def("gated_act(Tensor gu, Tensor(a!) h, int kind=1) -> ()");
   m.def("norm_rope_list(Tensor[] x, Tensor?[] norm_w, Tensor positions, Tensor?[] rope, Tensor(a!)[] out, Tensor?[] out_rows, "
-        "int[] kind, float[] eps, float[] scale, Tensor?[] out_t) -> ()");
+        "int[] kind, float[] eps, float[] scale, Tensor(b!)?[] out_t) -> ()");
   m.def("norm_rope_rows(Tensor x, Tensor? norm_w, Tensor positions, Tensor? rope, Tensor(a!) out, Tensor? out_rows, "
         "int kind, float eps, float scale=1.0, Tensor(b!)? out_t=None) -> ()");
   m.def("sink_attention(Tensor q, Tensor kcache, Tensor vcache, Tensor block_tables, Tensor q_start, Tensor q_len, "

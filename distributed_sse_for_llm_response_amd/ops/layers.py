@@ -220,7 +220,7 @@ def norm_rope_rows(x, norm_w, positions, rope, out, out_rows, norm_kind: int, ep
 
 def norm_rope_list(positions, *sets):
     """norm_rope_rows of up to three sets of heads of the same rows in one launch: each set (x, norm_w, rope, out, out_rows,
-    norm_kind, eps, scale, out_t), with inputs and outputs that do not overlap between sets."""
+    norm_kind, eps, scale, out_t).  Sets that overlap, one in what another writes, run one after another."""
     if _hip(sets[0][0]):
         x, norm_w, rope, out, out_rows, kind, eps, scale, out_t = map(list, zip(*sets))
         torch.ops.dsse.norm_rope_list(x, norm_w, positions, rope, out, out_rows, kind, eps, scale, out_t)

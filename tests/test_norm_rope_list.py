@@ -68,6 +68,41 @@ def test_list_equals_single_launches(T, H, G, D, V, kinds):
     assert torch.equal(two[1][3], a[1][3])
 
 
+# a chain over one buffer, sets whose columns overlap by one head, an output row that is another set's input at a different pitch
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 2, 300])
+def test_sets_that_meet_in_memory_run_in_order(T):
+    g = torch.Generator().manual_seed(T)
+    pos = torch.randint(0, 64, (T,), generator=g).to(torch.int32).cuda()
+    rope = torch.randn(64, 16, 2, generator=g).cuda()
+    start, w = torch.randn(T, 8 * 32, generator=g).cuda(), torch.randn(32, generator=g).cuda()
+
+    def run(call):
+        x, y, z = start.clone(), torch.zeros(T, 4, 32, device="cuda"), torch.zeros(T * 4 * 32 + 128, device="cuda")
+        q, mid = x[:, :128].unflatten(1, (4, 32)), x[:, 96:224].unflatten(1, (4, 32))
+        late = z[32:32 + T * 128].view(T, 4, 32)
+        chain = [(q, w, rope, y, None, HEAD, 1e-5, 0.5, None), (y, None, rope, y, None, NONE, 0.0, 2.0, None), (y, w, None, late, None, HEAD, 1e-5, 1.0, None)]
+        columns = [(q, None, rope, q, None, NONE, 0.0, 1.0, None), (mid, None, rope, mid, None, UNIT, 1e-6, 1.0, None)]
+        pitch = [(late, None, rope, x[:, 128:].unflatten(1, (4, 32)), None, NONE, 0.0, 1.0, None),
+                 (x.view(-1)[64:64 + T * 128].view(T, 4, 32), None, None, y, None, UNIT, 1e-6, 1.0, None)]
+        for sets in (chain, columns, pitch):
+            call(sets)
+        return x, y, z
+
+    def each(sets):
+        for xs, wt, r, out, rows, kind, eps, scale, out_t in sets:
+            ops.norm_rope_rows(xs, wt, pos, r, out, rows, kind, eps, scale, out_t)
+
+    for a, b in zip(run(lambda sets: ops.norm_rope_list(pos, *sets)), run(each)):
+        assert torch.equal(a, b)
+
+
+def test_schema_names_every_write():
+    ops.load_library(required=True)
+    args = torch.ops.dsse.norm_rope_list.default._schema.arguments
+    assert [a.name for a in args if a.alias_info is not None and a.alias_info.is_write] == ["out", "out_t"]
+
+
 def test_list_cpu():
     x, w = torch.randn(4, 2, 8), torch.randn(16)
     pos, outs = torch.zeros(4, dtype=torch.int32), [torch.zeros(4, 2, 8) for _ in range(2)]
