@@ -159,6 +159,7 @@ class LayeredRunner(RunnerBase):
         cfg, dev = self.cfg, self.device
         self._init_slots(max_batch, self.max_blocks, cfg.vocab_size, dev, self.comm)
         self._tile_rows = []   # row counts of the shared-page sink attention's work items that this design's layers use
+        self._plain_scans = []  # one row of the operands (q, k, v, channel decays or None) of each recurrence without the delta rule
         self._latents = set()  # (heads, rank, rotated width) of the latent attentions on the MFMA form
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
@@ -222,6 +223,17 @@ class LayeredRunner(RunnerBase):
         self._tile_rows = self._sink_tile_rows([cfg.layers[r.layer].mixer.left for r in self.runs if r.index in kv])
         self.kv = PagedKVCache(kv, self.num_blocks, dev, self.dtype, transposed=flash)
         self.state = MatrixStateCache(st, self.max_batch, dev)
+        plain = set()  # (heads, width, value width, row pitch, first column, decays per channel)
+        for i, L in enumerate(cfg.layers):
+            m = L.mixer
+            if L.kind == "parallel":
+                a, r = m.left, m.right
+                plain.add((r.heads, r.dim, r.vdim, self.w.layers[i].mix.n_big, (a.heads + a.kv_heads) * a.dim + a.kv_heads * a.vdim, True))
+            elif L.kind == "retention":
+                plain.add((m.heads, m.dim, m.vdim, 2 * m.heads * (m.dim + m.vdim), 0, False))
+        for H, D, V, pitch, c0, chan in sorted(plain):
+            row = torch.empty(1, pitch, device=dev, dtype=torch.float32)
+            self._plain_scans.append((*self._scan_rows(row, c0, H, D, V), torch.empty(1, H, D, device=dev, dtype=torch.float32) if chan else None))
 
     def _sink_tile_rows(self, mixers) -> list:
         """Rows per work item of the shared-page form of the given sink attention layers, each once."""
@@ -509,14 +521,17 @@ class LayeredRunner(RunnerBase):
         """Columns [c0, c0 + heads * width) of a row-major fp32 buffer as [rows, heads, width] (a view)."""
         return buf[:, c0:c0 + heads * width].unflatten(1, (heads, width))
 
+    def _scan_rows(self, buf, c0: int, H: int, D: int, V: int):
+        """Queries, keys and values that lie side by side from column c0 on."""
+        return self._cols(buf, c0, H, D), self._cols(buf, c0 + H * D, H, D), self._cols(buf, c0 + 2 * H * D, H, V)
+
     def _scan_out(self, ri: int, Lw_norm, gate, H: int, V: int, M: int, d: dict, q, k, v, decay, beta, groups, q_scale,
                   o_w, o_t, y) -> None:
         """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection."""
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
-            D, chan, seqs = k.shape[2], decay is not None and decay.dim() == 3, g.get("seqs")  # seqs: prompt portions
-            if beta is None and seqs and ops.matrix_scan_two_levels(q, k, v, chan, g["rows"][1], len(seqs[0]), g["longest"],
-                                                                       decay if chan else None):
+            D, chan = k.shape[2], decay is not None and decay.dim() == 3
+            if beta is None and self._two_levels(g, q, k, v, decay if chan else None):
                 s_first, s_count, cm = self._scan_lists(g)
                 scr = self._scratch(d, "scan_s", cm.shape[1] * H * D * V)
                 ascr = self._scratch(d, "scan_a", cm.shape[1] * H * D) if chan else None
@@ -529,8 +544,14 @@ class LayeredRunner(RunnerBase):
         ops.gated_head_norm(o, Lw_norm, gate, self.cfg.eps, ao)
         self._lin(ao, o_w, o_t, y)
 
+    @staticmethod
+    def _two_levels(g: dict, q, k, v, channels) -> bool:
+        """Whether the two-level walk takes a recurrence without the delta rule over a group: of prompt portions (seqs) only."""
+        seqs = g.get("seqs")
+        return bool(seqs) and ops.matrix_scan_two_levels(q, k, v, channels is not None, g["rows"][1], len(seqs[0]), g["longest"], channels)
+
     def _scan_lists(self, g: dict):
-        """Chunk lists of the two-level walk over a group's portions, made by the first layer that takes it."""
+        """Chunk lists of the two-level walk over a group's portions: made with the step's other lists when a layer will ask for them."""
         if "ck" not in g:
             s_first, s_count, rows = ops.layers.scan_chunks(*g["seqs"])
             ck = torch.tensor([s_first, s_count], dtype=torch.int32)
@@ -594,8 +615,7 @@ class LayeredRunner(RunnerBase):
         ops.gemm_rm(small[:, H:], Lw.a2, z, bias=Lw.a2_b)
         ops.gate_math(z, 2, None, None, r.tau)
         c0 = NL
-        q, k = self._cols(big, c0, Hr, Dr), self._cols(big, c0 + Hr * Dr, Hr, Dr)
-        v = self._cols(big, c0 + 2 * Hr * Dr, Hr, Vr)
+        q, k, v = self._scan_rows(big, c0, Hr, Dr, Vr)
         gate = big[:, c0 + 2 * Hr * Dr + Hr * Vr:NL + NR]
         self._scan_out(ri, Lw.rnorm, gate, Hr, Vr, M, d, q, k, v, z.view(M, Hr, Dr), None, groups, Dr ** -0.5, Lw.ro,
                        Lw.ro_t, d["y2"])
@@ -607,7 +627,7 @@ class LayeredRunner(RunnerBase):
         big = d["big"][:M * N].view(M, N)
         self._lin(d["xb"], Lw.big, Lw.big_t, big)
         rope = self._rope.get(m.rot)
-        q, k, v = self._cols(big, 0, H, D), self._cols(big, H * D, H, D), self._cols(big, 2 * H * D, H, V)
+        q, k, v = self._scan_rows(big, 0, H, D, V)
         ops.norm_rope_list(pos, (q, None, rope, q, None, 0, 0.0, 1.0, None), (k, None, rope, k, None, 0, 0.0, D ** -0.5, None))
         self._scan_out(ri, None, big[:, 2 * H * D + H * V:], H, V, M, d, q, k, v, Lw.decay, None, groups, 1.0, Lw.o,
                        Lw.o_t, d["y"])
@@ -1465,6 +1485,8 @@ class LayeredRunner(RunnerBase):
         d["rows"] = (row0, T)   # the packed rows of these portions
         d["longest"], d["keys"] = max(ql), max(ctx)
         d["seqs"] = (qs, ql, ss)
+        if T >= 4 * ops.layers.SCAN_CHUNK and any(self._two_levels(d, *operands) for operands in self._plain_scans):
+            self._scan_lists(d)  # before the step's first launch: inside it the upload costs some 80 us
         return T, qs, ql, d
 
     def prefill(self, seqs: list, ring_row: int, trace: list | None = None) -> None:

@@ -37,3 +37,23 @@ def test_two_levels_for_one_long_sequence_of_few_columns():
     assert two_levels(2048, 2, 2, 128, 128) and two_levels(2048, 4, 4, 64, 64) and two_levels(4096, 4, 2, 32, 32)
     assert not two_levels(800, 2, 2, 128, 128) and not two_levels(1000, 4, 4, 64, 64) and not two_levels(2048, 4, 2, 32, 32)
     assert not two_levels(2048, 4, 4, 128, 128)
+
+
+# widths that the chunks refuse (the lists will be asked for), widths that they take, and a group too short for two levels
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,vdim,rows,made", [(10, 7, 256, True), (32, 16, 256, False), (10, 7, 255, False)])
+def test_chunk_lists_are_ready_before_the_first_launch(dim, vdim, rows, made, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    import test_surodra as S
+    from distributed_sse_for_llm_response_amd.engine.model_runner import PrefillSeq
+
+    r = S.Model(S.config([S.ff(S.par(rdim=dim, rvdim=vdim)), S.ret(dim=dim, vdim=vdim)]), "cuda", max_tokens=512).runner
+    assert len(r._plain_scans) == 2
+    asked = []
+    real = type(r)._scan_lists
+    monkeypatch.setattr(type(r), "_scan_lists", lambda self, g: asked.append("ck" in g) or real(self, g))
+    monkeypatch.setattr(type(r), "_layers", lambda self, *a, layers=type(r)._layers, **k: asked.append("layers") or layers(self, *a, **k))
+    r.prefill([PrefillSeq(slot=0, tokens=S.toks(rows), start_pos=0, block_table=list(range(8)), last_chunk=True)], ring_row=0)
+    # made once, before the layers; found by both of them
+    assert asked == ([False, "layers", True, True] if made else ["layers"])
