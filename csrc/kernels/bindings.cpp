@@ -66,17 +66,32 @@ std::unordered_map<std::string, int> parse_kernel_cfg() {
   }
   return m;
 }
-int env_int(const char* key, int dflt) {
-  thread_local std::unordered_map<std::string, int> cfg;
-  thread_local uint64_t gen = 0;
+struct KernelCfg {
+  std::unordered_map<std::string, int> keys;
+  bool gemm = false;  // some key of a GEMM kernel's shape is set
+  uint64_t gen = 0;
+};
+const KernelCfg& kernel_cfg() {
+  thread_local KernelCfg cfg;
   const uint64_t g = g_env_gen.load(std::memory_order_acquire);
-  if (gen != g) {
-    cfg = parse_kernel_cfg();
-    gen = g;
+  if (cfg.gen != g) {
+    cfg.keys = parse_kernel_cfg();
+    cfg.gemm = false;
+    for (const char* k : {"t_split", "t_small", "t_model", "t_fix", "s_nw", "s_nt", "s_rd", "s_split", "s_ring", "s_fix", "ring2", "resid_nw",
+                          "resid_split", "qkv_split", "w_split", "w_rd", "gemm_nt", "gemm_kw"})
+      cfg.gemm |= cfg.keys.count(k) > 0;
+    cfg.gen = g;
   }
-  auto it = cfg.find(key);
-  return it == cfg.end() ? dflt : it->second;
+  return cfg;
 }
+int env_int(const char* key, int dflt) {
+  const auto& keys = kernel_cfg().keys;
+  const auto it = keys.find(key);
+  return it == keys.end() ? dflt : it->second;
+}
+// The rules that put one GEMM kernel in another's place by size alone (skinny_pairs, skinny_whole, rows_plan) step aside where a key
+// shapes a kernel that they would pass over: a run that sets s_split means the sliced kernel
+bool gemm_rules_free() { return !kernel_cfg().gemm; }
 // trap_fpe=1: print the native stack of a host SIGFPE (integer division by zero) before dying.
 void fpe_handler(int sig) {
   void* frames[64];
@@ -105,7 +120,7 @@ void refresh_env() { g_env_gen.fetch_add(1, std::memory_order_acq_rel); }
 // 32768 x 4096 (gemm_stream 47.9) 44.8; 8 rows, 6144 x 4096 13.7 / 12.6; but 10240 x 4096 (320 workgroups) 21.6 / 22.6, 8320 x 2048 (260)
 // 13.1 / 13.6, 26752 x 4096 (836) 41.6 / 42.6.
 bool skinny_pairs(int M, int N) {
-  if (M < 8 || M > 16 || N % 32) return false;
+  if (M < 8 || M > 16 || N % 32 || !gemm_rules_free()) return false;
   const int wgs = N / 32, rem = wgs % 256;
   return wgs >= 160 && (rem == 0 || rem >= 160);
 }
@@ -114,7 +129,7 @@ bool skinny_pairs(int M, int N) {
 // 11.9; 4096 x 2048 17 rows 10.8 / 8.1, 32 11.4 / 9.7; 2048 x 2560 32 rows 10.8 / 10.7; 2048 x 4096 24 rows 11.8 / 12.3; 2048 x 1024 64
 // rows 10.1 / 9.3; 6144 x 2048 24 rows 12.3 / 12.6.  K % 512 != 0 (a tensor-parallel shard's) stays with the ring kernel.
 bool skinny_whole(int M, int N, int K) {
-  return M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
+  return gemm_rules_free() && M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
 }
 
 void pick_tiles(int M, int N, int K, int mode, int& mt, int& nt, int& kw) {
@@ -395,7 +410,7 @@ TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
   c.cfg = 2;
   c.S = 1;
   const int blocks = N / 128;
-  if (M <= 64 || M > 256 || N % 128 || K % 128 || blocks > 256 || (int64_t)M * K * 2 >= ((int64_t)1 << 31)) return c;
+  if (!gemm_rules_free() || M <= 64 || M > 256 || N % 128 || K % 128 || blocks > 256 || (int64_t)M * K * 2 >= ((int64_t)1 << 31)) return c;
   if (N > 8192) {
     if (M > 192) c.ok = N % 256 || (blocks >= 112 && blocks <= 128) || (M <= 224 && K >= 4096 && blocks >= 224);
     else if (M > 128) c.ok = true;

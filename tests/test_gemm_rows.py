@@ -23,6 +23,25 @@ def test_plan(M, N, K, slabs, want):
         assert (split, fix) == (want, False)
 
 
+# a key that shapes another kernel means that kernel: the size rules step aside, here and in the rules of fewer rows
+@pytest.mark.parametrize("M,N,K,key,value,want", [
+    (160, 14464, 4096, "t_split", 1, (3, -1, 0)), (72, 32768, 4096, "w_split", 1, (3, -1, 0)), (72, 32768, 4096, "w_rd", 2, (3, -1, 0)),
+    (72, 8320, 2048, "s_split", 2, (2, -1, 0)), (200, 16384, 4096, "t_fix", 1, (4, 5, 2)), (200, 16384, 4096, "t_small", 0, (4, 5, 2)),
+    (16, 16384, 4096, "s_split", 1, (2, -1, 0)), (32, 2048, 2048, "s_ring", 1, (2, -1, 0)), (32, 2048, 2048, "resid_split", 4, (2, -1, 0)),
+    (160, 16384, 4096, "t_split", 1, (4, 5, 1)), (160, 14464, 4096, "attn_pd", 1, (4, 2, 2))])
+def test_plan_under_keys(monkeypatch, M, N, K, key, value, want):
+    ops.load_library(required=True)
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(**{key: value}))
+    ops.refresh_env()
+    try:
+        got = torch.ops.dsse.gemm_plan(M, N, K)[:3]
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
+    assert got == want
+    assert torch.ops.dsse.gemm_plan(M, N, K)[:3] != want or key == "attn_pd"
+
+
 @pytest.fixture
 def forced(monkeypatch):
     if not torch.cuda.is_available():
