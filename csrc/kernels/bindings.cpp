@@ -128,6 +128,8 @@ bool skinny_pairs(int M, int N) {
 // workgroups and K walks of at most two rounds.  Sliced / skinny, us: 2048 x 2048 17 rows 9.8 / 7.7, 32 rows 10.7 / 9.3, 48 rows 10.6 /
 // 11.9; 4096 x 2048 17 rows 10.8 / 8.1, 32 11.4 / 9.7; 2048 x 2560 32 rows 10.8 / 10.7; 2048 x 4096 24 rows 11.8 / 12.3; 2048 x 1024 64
 // rows 10.1 / 9.3; 6144 x 2048 24 rows 12.3 / 12.6.  K % 512 != 0 (a tensor-parallel shard's) stays with the ring kernel.
+// Not where the next kernel sums the slices (gemm_impl's slab_consumer): product and RMSNorm, sliced / skinny, 4096 x 2048 24 rows 12.0 /
+// 13.6, 2048 x 2048 32 rows 10.6 / 13.3, 4096 x 1024 64 rows 11.9 / 17.0, 4096 x 512 32 rows 10.3 / 11.1.
 bool skinny_whole(int M, int N, int K) {
   return gemm_rules_free() && M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
 }
@@ -511,7 +513,8 @@ void run_tiled(int mode, const TCfg& c, const Tensor& x, const Tensor& w, int M,
 // 0 = register-streaming (gemm_skinny.hip; tiny batches, X re-reads are cheap), 2 = X streamed through LDS
 // slices (gemm_stream.hip), 3 = gemm_wide.hip (32x32 MFMAs), 4 = gemm_tiled.hip (register-blocked, LDS-DMA).
 // gemm_impl (DSSE_KERNEL_CFG) forces one (1, the removed whole-slice X-in-LDS kernel, maps to the fallback).
-int gemm_impl(int M, int N, int K) {
+// slab_consumer: the next kernel sums split-K slabs, so a sliced product has no reduction launch to save.
+int gemm_impl(int M, int N, int K, bool slab_consumer = false) {
   const int impl = env_int("gemm_impl", -1);
   if (M > 64) {
     // every branch returns a kernel whose shape contract holds (or -1): prefill calls arrive with any M and
@@ -545,7 +548,7 @@ int gemm_impl(int M, int N, int K) {
   }
   if (M <= 8) return 0;
   if (M <= 16 && (N < 16384 || skinny_pairs(M, N))) return 0;
-  if (skinny_whole(M, N, K)) return 0;
+  if (!slab_consumer && skinny_whole(M, N, K)) return 0;
   return pick_stream(M, N, K).ok ? 2 : fallback;
 }
 
@@ -638,7 +641,7 @@ int64_t gemm_resid_split(const Tensor& x, const Tensor& w, Tensor& resid, Tensor
   check_dtype(part, at::kFloat, "part");
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = M >= 1 && K % 128 == 0 && N % 16 == 0 && w.size(1) == K;
-  const int impl = shape_ok ? gemm_impl(M, N, K) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
   if (impl == 4) {
     const TCfg c = pick_tiled(M, N, K, true);
     if (c.S > 1 && !c.fix && part.numel() >= (int64_t)c.S * M * N) {
@@ -690,7 +693,7 @@ int64_t gemm_out_split(const Tensor& x, const Tensor& w, Tensor& out, Tensor& pa
   check_dtype(part, at::kFloat, "part");
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = M >= 1 && K % 128 == 0 && N % 16 == 0 && w.size(1) == K;
-  const int impl = shape_ok ? gemm_impl(M, N, K) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
   dsse::GemmEpi ep{};
   if (impl == 2) {
     const SCfg c = pick_stream(M, N, K);
@@ -1006,7 +1009,7 @@ int64_t qkv_attention_decode(const Tensor& x, const Tensor& w, const Tensor& pos
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = x.dim() == 2 && w.dim() == 2 && M >= 1 && K % 128 == 0 && w.size(1) == K &&
                         N == (nh + 2 * nkv) * 128;
-  const int impl = shape_ok ? gemm_impl(M, N, K) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
   int S = 0;
   if (impl == 4) {
     const TCfg c = pick_tiled(M, N, K, true);
@@ -1264,7 +1267,7 @@ int64_t kernels_abi_version() { return 16; }
 // The dispatch's choice for an (M, N, K) projection: (impl, tiled cfg, split, fix, model estimate in us) -- impl as
 // gemm_impl (4 = tiled / pipe); cfg / split / fix / estimate only for impl 4 (tools/bench_decode_gemm.py --plan).
 std::tuple<int64_t, int64_t, int64_t, bool, double> gemm_plan(int64_t M, int64_t N, int64_t K, bool slab_consumer) {
-  const int impl = gemm_impl((int)M, (int)N, (int)K);
+  const int impl = gemm_impl((int)M, (int)N, (int)K, slab_consumer);
   if (impl != 4) return {impl, -1, 0, false, 0.0};
   const TCfg c = pick_tiled((int)M, (int)N, (int)K, slab_consumer);
   return {impl, c.cfg, c.S, c.fix, c.est_us};

@@ -18,6 +18,32 @@ def test_plan(M, N, K, skinny):
     assert (torch.ops.dsse.gemm_plan(M, N, K)[0] == 0) == skinny
 
 
+# the same products where the next kernel sums the slices (a tensor-parallel shard's o projection before its norm): sliced
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 2048), (32, 2048, 2560), (64, 2048, 1024), (32, 4096, 512)])
+def test_plan_before_a_slab_consumer(M, N, K):
+    ops.load_library(required=True)
+    assert torch.ops.dsse.gemm_plan(M, N, K)[0] == 0
+    assert torch.ops.dsse.gemm_plan(M, N, K, True)[0] == 2
+
+
+# and those calls leave slabs: their sum is the product
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 2048), (64, 2048, 1024)])
+def test_slabs(M, N, K):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    ops.load_library(required=True)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = R.tile_weight((torch.randn(N, K, device="cuda", generator=g) / math.sqrt(K)).bfloat16())
+    ref = x.double() @ R.untile_weight(w).double().t()
+    for call, out in ((ops.gemm_out_split, torch.zeros(M, N, device="cuda", dtype=torch.bfloat16)), (ops.gemm_resid_split, torch.zeros(M, N, device="cuda"))):
+        part = torch.full((16 * M * N,), float("nan"), device="cuda")
+        S = call(x, w, out, part)
+        assert S > 1
+        assert float((part[:S * M * N].view(S, M, N).sum(0) - ref).abs().max()) <= K * 2.0 ** -23 * float(ref.abs().max())  # K fp32 additions
+
+
 # both sides of two column tiles per wave (8 and 16 rows, full and nearly empty last rounds), the first and last row of a 16-row
 # tile in the 32- and 64-row forms, K walks shorter than the waves that share them
 @pytest.mark.gpu
