@@ -118,10 +118,12 @@ void refresh_env() { g_env_gen.fetch_add(1, std::memory_order_acq_rel); }
 // workgroups end in a full or well filled round.  One tile / two, 16 rows, us: 6144 x 4096 16.2 / 13.9, 8192 x 4096 18.1 / 15.9, 5248 x
 // 4096 16.1 / 13.9, 14464 x 4096 28.4 / 25.3, 16384 x 2048 16.6 / 15.2, 16384 x 4096 (gemm_stream 29.2) 25.3, 32768 x 2048 28.2 / 24.9,
 // 32768 x 4096 (gemm_stream 47.9) 44.8; 8 rows, 6144 x 4096 13.7 / 12.6; but 10240 x 4096 (320 workgroups) 21.6 / 22.6, 8320 x 2048 (260)
-// 13.1 / 13.6, 26752 x 4096 (836) 41.6 / 42.6.
+// 13.1 / 13.6, 26752 x 4096 (836) 41.6 / 42.6.  At one full round of pairs, which is two of single tiles, from 12 rows: 8192 x 2048 SiLU
+// 8 rows 10.1 / 10.6, 12 rows the same.
 bool skinny_pairs(int M, int N) {
   if (M < 8 || M > 16 || N % 32 || !gemm_rules_free()) return false;
   const int wgs = N / 32, rem = wgs % 256;
+  if (M < 12 && wgs == 256) return false;
   return wgs >= 160 && (rem == 0 || rem >= 160);
 }
 // 17 to 64 rows in one launch of the skinny kernel, where a sliced product and its reduction are two latency-sized ones: up to 256
@@ -394,16 +396,19 @@ bool half_block_pays(int M, int N, int K, const TCfg& c) {
 
 // 65 to 256 rows on one tile that holds them all (gemm_tiled cfg 2), in one round of at most 256 workgroups.  Two row blocks
 // of 128 fetch every weight twice and compute dead rows.  Measured with X rewritten and 4 GB of weights read in turn, this tile /
-// what the other rules give, in us:
-//   129 to 192 rows, wide products: 28672 x 4096 SiLU 160 rows 58 / 70, fp32 180 rows 68 / 76; 32768 x 4096 75 / 85; 26752 x 4096 64 /
-//   89; 14336 x 4096 47 / 49; 32768 x 2048 42 / 44; 8320 x 2048 160 rows 25 / 42; 10240 x 4096 43 / 43.  To 8192 columns it is behind
-//   (8192 x 4096 160 rows 32 / 30, 6144 x 2048 22 / 21) unless the slabs are the next kernel's: 6144 x 4096 in 4 slices 160 rows 20 / 22,
-//   4096 x 14336 in 8 32 / 36 (200 rows 37 / 38); 4096 x 4096 15 / 17, but in 8 slices instead of 4, which the norm reads;
-//   193 rows and more: only without a 256-column tile (26752 x 4096 224 rows 72 / 91) or where two slices or one fill half a round
-//   to a whole one (16384 x 4096 54 / 58, 14336 x 4096 51 / 53) or the weights fill the chip (28672 x 4096 200 rows 75 / 79, 224 78 / 80,
-//   but 256 83 / 82, and 32768 x 2048 49 / 46);
-//   65 to 128 rows: the widest (28672 x 4096 72 rows 51 / 58, 128 56 / 56; 32768 x 2048 35 / 40, 38 / 43; but 26752 x 4096 55 / 52), and
-//   where the ring's slices end above one round (8320 x 2048 72 rows 21 / 23, 10240 x 4096 31 / 35, 128 rows 37 / 40).
+// what the other rules give, in us; over 1000 products of 45 widths and lengths the geometric mean is 1.17, the worst 0.98:
+//   129 to 192 rows, wide products: 28672 x 4096 SiLU 160 rows 58 / 70; 32768 x 4096 75 / 85; 26752 x 4096 64 / 89; 15360 x 4096 1.08 times,
+//   x 5120 1.10; 14336 x 4096 47 / 49; 32768 x 2048 42 / 44; 8320 x 2048 25 / 42; but short products to 14336 columns where the 256-column
+//   tile fits 10240 x 2048 160 rows 30 / 28, 192 32 / 29, 12288 x 2048 31 / 29, 11008 x 3584 SiLU 40 / 38.
+//   To 8192 columns it is behind (8192 x 4096 160 rows 32 / 30, 6144 x 2048 22 / 21) unless its slabs are the next kernel's and there are
+//   enough of them; product and RMSNorm, 4096 x 14336 in 8 slices 1.12 times, x 8192 1.04, 5120 x 13824 1.03, 8192 x 4096 1.04, x 8192 1.13, but
+//   6144 x 4096 31 / 30 (Mistral's step of 160 streams 6105 -> 5790 us without it), 5120 x 5120 34 / 33, 3072 x 8192 32 / 31, 2048 x 8192 in
+//   16 slices 27 / 25;
+//   193 rows and more: only without a 256-column tile (26752 x 4096 224 rows 72 / 91) or where two slices fill half a round
+//   to a whole one (16384 x 4096 54 / 58, 14336 x 4096 51 / 53; but 14336 x 2048 37 / 34) or the weights fill the chip (28672 x 4096 200
+//   rows 75 / 79, 224 78 / 80, but 256 83 / 82, and 32768 x 2048 49 / 46);
+//   65 to 128 rows: the widest (28672 x 4096 72 rows 51 / 58, but 128 56 / 56 and 31104 x 4608 65 / 63; 32768 x 2048 35 / 40, 128 rows 38 / 43;
+//   26752 x 4096 55 / 52), and where the ring's slices end above one round (8320 x 2048 72 rows 21 / 23, 10240 x 4096 31 / 35, 128 rows 37 / 40).
 // Two slices where half the K walk is longer than their slabs and the reduction: 10240 x 4096 160 rows 38 / 49, 8320 x 2048 25 / 26,
 // 14464 x 2048 29 / 27, 16384 x 2048 31 / 28.
 TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
@@ -414,14 +419,14 @@ TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
   const int blocks = N / 128;
   if (!gemm_rules_free() || M <= 64 || M > 256 || N % 128 || K % 128 || blocks > 256 || (int64_t)M * K * 2 >= ((int64_t)1 << 31)) return c;
   if (N > 8192) {
-    if (M > 192) c.ok = N % 256 || (blocks >= 112 && blocks <= 128) || (M <= 224 && K >= 4096 && blocks >= 224);
-    else if (M > 128) c.ok = true;
+    if (M > 192) c.ok = N % 256 || (blocks >= 112 && blocks <= 128 && K >= 4096) || (M <= 224 && K >= 4096 && blocks >= 224);
+    else if (M > 128) c.ok = N % 256 || N > 14336 || K >= 4096;
     else {
       const SCfg r = pick_stream(M, N, K);
-      c.ok = blocks >= 224 || (r.ok && r.nw == 4 && N / 64 * r.S > 256);
+      c.ok = (blocks >= 224 && (M <= 96 || K < 4096)) || (r.ok && r.nw == 4 && N / 64 * r.S > 256);
     }
     c.S = blocks <= 128 && K >= 1024 && (double)K * (M + 128) > 61e3 * (4.0 + 3.2e-6 * M * N) ? 2 : 1;
-  } else if (M > 128 && M <= 192 && slab_consumer && K >= 4096 && (N > 4096 || K > 4096)) {
+  } else if (M > 128 && M <= 192 && slab_consumer && N >= 4096 && K >= 4096 && (N > 7168 || K > 6144)) {
     while (blocks * c.S * 2 <= 256 && K % (128 * c.S) == 0 && K / (c.S * 2) >= 512) c.S *= 2;
     c.ok = blocks * c.S >= 160;
   }

@@ -13,8 +13,9 @@ from distributed_sse_for_llm_response_amd.ops import reference as R
     (64, 28672, 4096, False, None), (65, 28672, 4096, False, 1), (192, 28672, 4096, False, 1), (224, 28672, 4096, False, 1), (225, 28672, 4096, False, None),
     (160, 32768, 4096, False, 1), (160, 32896, 4096, False, None), (128, 26752, 4096, False, None), (129, 14464, 4096, False, 2),
     (256, 26752, 4096, False, 1), (257, 26752, 4096, False, None), (160, 14464, 2048, False, 1), (72, 8320, 2048, False, 2),
-    (72, 10368, 4096, False, None), (200, 10240, 4096, False, None), (200, 16384, 4096, False, 2), (160, 8192, 4096, False, None),
-    (160, 6144, 4096, True, 4), (160, 4096, 14336, True, 8), (160, 4096, 4096, True, None), (200, 4096, 14336, True, None)])
+    (72, 10368, 4096, False, None), (160, 12288, 2048, False, None), (160, 14464, 1536, False, 1), (208, 14336, 2048, False, None), (128, 28672, 4096, False, None),
+    (96, 28672, 4096, False, 1), (128, 32768, 2048, False, 1), (200, 10240, 4096, False, None), (200, 16384, 4096, False, 2), (160, 8192, 4096, False, None),
+    (160, 6144, 4096, True, None), (160, 8192, 4096, True, 4), (160, 4096, 14336, True, 8), (160, 2048, 8192, True, None), (160, 4096, 4096, True, None), (200, 4096, 14336, True, None)])
 def test_plan(M, N, K, slabs, want):
     ops.load_library(required=True)
     impl, cfg, split, fix, _ = torch.ops.dsse.gemm_plan(M, N, K, slabs)
