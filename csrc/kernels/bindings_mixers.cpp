@@ -446,9 +446,9 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
 }
 
-// decay: the decays where the caller has them, [T, H, D] when channels; without them decays per channel count as unaligned
-bool matrix_scan_two_levels(const Tensor& q, const Tensor& k, const Tensor& v, bool channels, int64_t rows, int64_t nseq,
-                            int64_t longest, const OptTensor& decay) {
+// What the choice of a form looks at: shapes, row pitches and addresses.  decay: the decays where the caller has them, [T, H, D] when
+// channels; without them decays per channel count as unaligned.
+dsse::MatrixScanParams scan_shape(const Tensor& q, const Tensor& k, const Tensor& v, bool channels, int64_t nseq, const OptTensor& decay) {
   dsse::MatrixScanParams p{};
   p.H = (int)v.size(1), p.V = (int)v.size(2), p.G = (int)k.size(1), p.D = (int)k.size(2), p.nseq = (int)nseq;
   p.q = q.data_ptr<float>(), p.k = k.data_ptr<float>(), p.v = v.data_ptr<float>();
@@ -459,7 +459,19 @@ bool matrix_scan_two_levels(const Tensor& q, const Tensor& k, const Tensor& v, b
     TORCH_CHECK(decay->dim() == 3 && decay->scalar_type() == at::kFloat, "decay [T, H, D], float32");
     p.decay = decay->data_ptr<float>(), p.ldd = (int)decay->stride(0);
   }
-  return dsse::scan_two_levels(p, (int)rows, longest);
+  return p;
+}
+bool matrix_scan_two_levels(const Tensor& q, const Tensor& k, const Tensor& v, bool channels, int64_t rows, int64_t nseq,
+                            int64_t longest, const OptTensor& decay) {
+  return dsse::scan_two_levels(scan_shape(q, k, v, channels, nseq, decay), (int)rows, longest);
+}
+// Whether matrix_scan of such rows goes by chunks (else by tokens)
+bool matrix_scan_by_chunks(const Tensor& q, const Tensor& k, const Tensor& v, bool delta, bool channels, int64_t rows, int64_t nseq,
+                           int64_t longest, const OptTensor& decay) {
+  dsse::MatrixScanParams p = scan_shape(q, k, v, channels, nseq, decay);
+  if (delta) p.beta = p.v;
+  p.portions = rows > 2 * nseq;
+  return dsse::scan_chunk_floats(p, (int)rows, longest) > 0;
 }
 
 // Two-level walk of long prompt portions without the delta rule: (1) every chunk but a sequence's last is walked from
@@ -918,6 +930,8 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
   m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest, "
         "Tensor? decay=None) -> bool");
+  m.def("matrix_scan_by_chunks(Tensor q, Tensor k, Tensor v, bool delta, bool channels, int rows, int nseq, int longest, "
+        "Tensor? decay=None) -> bool");
   m.def("matrix_scan_chunked(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor(a!) state, Tensor q_len, Tensor ctx_len, "
         "Tensor state_slot, Tensor s_first, Tensor s_count, Tensor cmeta, Tensor(b!) scratch, Tensor(c!)? a_scratch, "
         "Tensor(d!) out, float q_scale=1.0) -> ()");
@@ -927,6 +941,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
 }
 
 TORCH_LIBRARY_IMPL(dsse, CompositeExplicitAutograd, m) {
+  m.impl("matrix_scan_by_chunks", &matrix_scan_by_chunks);
   m.impl("matrix_scan_two_levels", &matrix_scan_two_levels);  // looks at shapes and addresses only
 }
 

@@ -581,26 +581,30 @@ hipError_t launch_chunks(const MatrixScanParams& p, float* ws, int64_t rows, int
 
 }  // namespace
 
-// Time in us of the walk by tokens and of the chunks: each is a start, then its longest chain or the work of all its column blocks,
-// whichever is more.  Fitted per key width over 1..128 sequences of 4..2048 rows of 2..256 column blocks (both within 12 % rms); of 831
-// timings the slower of the two is taken by more than 6 % in 14.  Walk against chunks, H x D x V: delta rule, 16 x 128 x 128, one
-// sequence of 17 rows 12.6 / 11.9, 64 rows 30 / 14, 2048 rows 962 / 147, 16 of 8 rows 24 / 26, 64 of 64 rows 372 / 165; without it, 17
-// rows 11.6 / 9.9, 64 rows 27 / 11, 64 of 64 rows 328 / 105; 2 x 128 x 128, 16 rows, decays per channel 10 / 12.
+// Time in us of the walk by tokens and of the chunks.  The walk: a start, then its longest chain or the work of all its column blocks, whichever
+// is more (decode-sized launches, up to two rows a sequence on average, walk another kernel's chain).  The chunks: a start, the
+// preparation of every (chunk, head), which costs the same however few its column blocks, and the longest chain or all column blocks.
+// Fitted per key width over 1..180 sequences of 3..8192 rows of 1..1024 column blocks (each within 12 % rms); of 2784 timings the slower of
+// the two is taken by more than 6 % in 58, by 10 % in 32; on average 0.4 % is lost.  Walk against chunks, H x D x V: delta rule, 16 x
+// 128 x 128, one sequence of 17 rows 12.6 / 11.9, 64 rows 30 / 14, 2048 rows 962 / 147, 16 of 8 rows 27 / 24, 64 of 64 rows 372 / 165; without
+// it, 17 rows 11.6 / 9.9, 64 rows 27 / 11, 64 of 64 rows 328 / 105; 2 x 128 x 128, 16 rows, decays per channel 10 / 12; few column blocks,
+// 16 x 64 x 16, 64 of 32 rows 21 / 29, 128 of 24 rows, decays per channel 32 / 53; 2 x 128 x 32, 64 of 17 13 / 17; 8 x 128 x 16, 64 of 16 13 / 20.
 struct ScanCost {
-  double walk0, row, row_block, walk_seq, chunk0, chunk, chunk_block, seq_block, channels;
+  double walk0, row, row_block, walk_seq, chunk0, channels, unit, chunk, chunk_block, seq_block;
 };
 static bool chunks_pay(const MatrixScanParams& p, int64_t rows, int64_t chunks, int64_t longest) {
-  static const ScanCost kDelta[3] = {{4.3, 0.266, 0.034, 0.229, 8.7, 0.615, 0.340, 0.095, 1.0},   // widths 32, 64, 128
-                                     {4.4, 0.303, 0.048, 0.319, 8.8, 0.754, 0.377, 0.291, 1.2},
-                                     {5.2, 0.421, 0.092, 0.486, 9.3, 1.123, 0.464, 0.439, 2.1}};
-  static const ScanCost kPlain[3] = {{4.2, 0.228, 0.030, 0.248, 7.8, 0.334, 0.232, 0.129, 1.0},
-                                     {4.2, 0.272, 0.040, 0.327, 8.0, 0.418, 0.249, 0.228, 1.2},
-                                     {4.8, 0.382, 0.086, 0.484, 8.6, 0.631, 0.333, 0.437, 2.1}};
+  static const ScanCost kDelta[3] = {{4.7, 0.264, 0.041, 0.205, 8.7, 2.2, 0.083, 0.580, 0.120, 0.087},   // widths 32, 64, 128
+                                     {4.4, 0.326, 0.058, 0.311, 9.2, 2.5, 0.109, 0.575, 0.286, 0.222},
+                                     {4.9, 0.441, 0.106, 0.500, 9.6, 3.5, 0.207, 1.130, 0.300, 0.417}};
+  static const ScanCost kPlain[3] = {{4.6, 0.224, 0.038, 0.229, 7.9, 1.4, 0.056, 0.260, 0.113, 0.091},
+                                     {4.2, 0.288, 0.047, 0.338, 8.0, 1.9, 0.077, 0.343, 0.161, 0.205},
+                                     {4.8, 0.390, 0.093, 0.513, 8.8, 2.7, 0.155, 0.707, 0.163, 0.466}};
   const ScanCost& c = (p.beta ? kDelta : kPlain)[p.D == 32 ? 0 : (p.D == 64 ? 1 : 2)];
   const double blocks = (double)p.H * (p.V / kScanCols) / 128.0, n = (double)((longest + kC - 1) / kC);
-  const double walk = c.walk0 + std::max(c.row * longest, (c.row_block * rows + c.walk_seq * p.nseq) * blocks);
-  const double start = c.chunk0 + (p.decay_kind == 3 ? c.channels : 0.0);
-  return walk > start + std::max(c.chunk * n, (c.chunk_block * chunks + c.seq_block * p.nseq) * blocks);
+  const double walk = c.walk0 + std::max(c.row * (p.portions ? 1.0 : 1.8) * longest, (c.row_block * rows + c.walk_seq * p.nseq) * blocks);
+  const bool chan = p.decay_kind == 3;
+  const double prepare = c.chunk0 + (chan ? c.channels : 0.0) + c.unit * (chan ? 1.25 : 1.0) * chunks * p.H / 16;
+  return walk > prepare + std::max(c.chunk * n, (c.chunk_block * chunks + c.seq_block * p.nseq) * blocks);
 }
 
 // Whether the chunks take the shape

@@ -57,3 +57,19 @@ def test_chunk_lists_are_ready_before_the_first_launch(dim, vdim, rows, made, mo
     r.prefill([PrefillSeq(slot=0, tokens=S.toks(rows), start_pos=0, block_table=list(range(8)), last_chunk=True)], ring_row=0)
     # made once, before the layers; found by both of them
     assert asked == ([False, "layers", True, True] if made else ["layers"])
+
+
+# the costs of both forms (csrc/kernels/matrix_chunk.hip): one and many sequences, few column blocks and many, where the two were measured
+# 10 % and more apart; a decode step, and one long portion among portions of one row
+@pytest.mark.parametrize("H,D,V,lens,delta,channels,chunks", [
+    (16, 128, 128, [64], True, False, True), (16, 128, 128, [2048], False, False, True), (16, 128, 128, [8], True, False, False),
+    (8, 128, 128, [200], False, True, True), (16, 64, 16, [32] * 64, True, False, False), (16, 64, 16, [24] * 128, True, True, False),
+    (2, 128, 32, [17] * 64, True, False, False), (8, 128, 16, [16] * 64, True, False, False), (16, 128, 32, [64] * 32, True, False, True),
+    (4, 64, 16, [128] * 64, True, False, True), (16, 64, 16, [300] * 8, False, False, True), (16, 32, 16, [24] * 128, False, False, False),
+    (16, 64, 16, [1] * 60 + [40], True, False, True), (16, 128, 128, [1] * 64, True, False, False)])
+def test_walk_or_chunks(H, D, V, lens, delta, channels, chunks):
+    ops.load_library(required=True)
+    T = sum(lens)
+    q, k, v = torch.empty(T, H, D), torch.empty(T, H, D), torch.empty(T, H, V)
+    decay = torch.empty(T, H, D) if channels else None
+    assert torch.ops.dsse.matrix_scan_by_chunks(q, k, v, delta, channels, T, len(lens), max(lens), decay) is chunks
