@@ -5,6 +5,9 @@
 
 namespace dsse {
 
+// DSSE_KERNEL_CFG's value of `key` (bindings.cpp)
+int kernel_cfg_int(const char* key, int dflt);
+
 constexpr int kBS = 32;  // KV-cache page size in tokens (fixed for every kernel)
 
 enum GemmMode { kStoreBf16 = 0, kStoreF32 = 1, kResidAdd = 2, kSiluMul = 3, kQkvRope = 4 };

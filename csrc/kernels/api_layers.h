@@ -162,13 +162,16 @@ struct MoeGroupedParams {
   int aligned;           // 1: sorted / tile_expert / num_tiles are already made (moe_route_rows)
   int lds_tiles;         // 1: enough rows for the LDS-staged tiles (prompt portions); 0: the register-direct kernels
   int f32;
+  int form, once;        // 0: by cost; else (moe_form, moe_once of DSSE_KERNEL_CFG) form 1 stream, 2 pipeline, 3 register-direct where that
+                         // one takes the step; once 1 / 2: the pipeline's non-temporal weights on / off
 };
 
 // Shapes that the expert GEMMs on LDS-DMA take (moe_pipe.hip, moe_stream.hip): reduction lengths of whole 64-element steps,
 // two at least; 16-byte-aligned operands; every operand inside a 2 GiB buffer range.
 bool moe_lines_ok(const MoeGroupedParams& p);
-// Of those, the ones that read the weights as one stream (moe_stream.hip)
-bool moe_stream_pays(const MoeGroupedParams& p);
+// Which form those take: the register-direct kernels of moe.hip (few rows of small experts), the stream, the pipeline
+enum class MoeForm { kDirect, kStream, kPipe };
+MoeForm moe_form(const MoeGroupedParams& p);
 
 // Router, choice and work list of a decode-sized step in one launch.
 struct MoeRouteRowsParams {

@@ -46,7 +46,7 @@ void check_dtype(const Tensor& t, at::ScalarType st, const char* name) {
 // Kernel-configuration overrides: ONE environment variable, DSSE_KERNEL_CFG = "key=value,key=value" (diagnostics and
 // the tests that force a kernel path; e.g. "gemm_impl=4,t_cfg=8,t_split=2").  Keys name the selector inputs below
 // (gemm_impl, t_cfg, t_split, t_small, s_nw, s_nt, s_rd, s_split, s_ring, ring2, resid_nw, resid_split, qkv_split, w_split, w_rd,
-// gemm_nt, gemm_kw, attn_kwv, attn_pd, fused_qkv_attn, trap_fpe); docs/operations.md lists them.  Parsed once per
+// gemm_nt, gemm_kw, attn_kwv, attn_pd, fused_qkv_attn, moe_form, moe_once, trap_fpe); docs/operations.md lists them.  Parsed once per
 // thread into a thread-local map: no getenv and no lock on the launch path.  refresh_env() (op dsse::refresh_env, for
 // the tools that change it in-process) bumps a generation that makes every thread re-parse on its next lookup.
 std::atomic<uint64_t> g_env_gen{1};
@@ -108,6 +108,10 @@ const bool g_fpe_trap = [] {
 }();
 
 void refresh_env() { g_env_gen.fetch_add(1, std::memory_order_acq_rel); }
+
+}  // namespace
+int dsse::kernel_cfg_int(const char* key, int dflt) { return env_int(key, dflt); }
+namespace {
 
 
 

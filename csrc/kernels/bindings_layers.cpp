@@ -529,6 +529,7 @@ void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, 
   p.vec_w = p.W % per == 0;
   p.vec_h = p.ldh % per == 0 && p.F % per == 0;
   p.lds_tiles = ids >= 256;  // prompt-sized: most 64-row tiles are full
+  p.form = dsse::kernel_cfg_int("moe_form", 0), p.once = dsse::kernel_cfg_int("moe_once", 0);
   DSSE_CHECK_HIP(dsse_moe_grouped(&p, cur_stream()));
 }
 
@@ -580,7 +581,7 @@ void moe_topk(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w) {
 }
 
 // Which form the expert GEMMs of moe_grouped take for bf16 operands on LDS-DMA: 1 the stream (moe_stream.hip), 0 the pipeline
-// (moe_pipe.hip), -1 shapes that neither takes
+// (moe_pipe.hip), 2 the register-direct kernels (moe.hip), -1 shapes that neither of the first two takes
 int64_t moe_plan(int64_t M, int64_t W, int64_t F, int64_t Fs, int64_t E, int64_t top, bool gated) {
   dsse::MoeGroupedParams p{};
   p.M = (int)M, p.W = (int)W, p.F = (int)F, p.Fs = (int)Fs, p.E = (int)E, p.top = (int)top, p.S = (int)top + (Fs > 0 ? 1 : 0);
@@ -589,7 +590,10 @@ int64_t moe_plan(int64_t M, int64_t W, int64_t F, int64_t Fs, int64_t E, int64_t
   p.x = p.up = p.down = p.sgate = p.sup = p.sdown = aligned;
   p.h = const_cast<char*>(aligned);
   if (gated) p.gate = aligned;
-  return dsse::moe_lines_ok(p) ? (dsse::moe_stream_pays(p) ? 1 : 0) : -1;
+  p.lds_tiles = M * p.S >= 256;
+  if (!dsse::moe_lines_ok(p)) return -1;
+  const dsse::MoeForm form = dsse::moe_form(p);
+  return form == dsse::MoeForm::kPipe ? 0 : (form == dsse::MoeForm::kStream ? 1 : 2);
 }
 
 // moe_topk and the work list of moe_grouped (aligned) in one launch, for decode-sized steps; false: nothing done, the step is larger.

@@ -721,7 +721,10 @@ extern "C" hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStrea
                        sizeof(int) * (3 * NE + 1), st, *p);
   const int fmax = p->F > p->Fs ? p->F : p->Fs;
   dim3 g1((fmax + 15) / 16, p->max_tiles), g2((p->W + 15) / 16, p->max_tiles);
-  if (dsse::moe_lines_ok(*p)) return dsse::moe_stream_pays(*p) ? dsse_moe_stream(p, st) : dsse_moe_pipe(p, st);
+  if (dsse::moe_lines_ok(*p)) {
+    const dsse::MoeForm form = dsse::moe_form(*p);
+    if (form != dsse::MoeForm::kDirect) return form == dsse::MoeForm::kStream ? dsse_moe_stream(p, st) : dsse_moe_pipe(p, st);
+  }
   // other prompt-sized steps in bf16 with rows of whole 16-byte pieces: operands staged through registers and LDS
   if (!p->f32 && p->lds_tiles && p->W % 8 == 0 && p->F % 8 == 0 && p->Fs % 8 == 0 && p->ldh % 8 == 0) {
     dim3 l1((fmax + 63) / 64, p->max_tiles), l2((p->W + 127) / 128, p->max_tiles), l3((fmax + 127) / 128, p->max_tiles);

@@ -24,7 +24,7 @@
 // Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
 // experts, top 2, shared 7168: 2369 -> 1014 us (1042 TFLOP/s); 2048 rows: 1695 -> 775; 1024 rows of 2048 x 1408, shared
 // 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Up to 192 rows moe_stream.hip takes
-// the sizes whose weights it need not read twice (moe_stream_pays).
+// the sizes whose weights it need not read twice, or the kernels of moe.hip a few rows of small experts (moe_form).
 #include <algorithm>
 #include <cmath>
 
@@ -399,7 +399,11 @@ bool moe_lines_ok(const MoeGroupedParams& p) {
 
 // The line lies at a mean of 128 rows per expert.  Plain / ONCE at 16 experts, top 2 and a shared one: 2048 x 1408 + 2816: 400 rows
 // 116 / 110 us, 1000 173 / 166, 1500 185 / 182 (but a whole prompt of 1649 rows in four 2708 / 2748), 3000 259 / 261; 4096 x 3584 +
-// 7168: 256 rows 333 / 314, 700 407 / 404, 1000 471 / 465, 3000 1038 / 1068.
+// 7168: 256 rows 333 / 314, 700 407 / 404, 1000 471 / 465, 3000 1038 / 1068.  And where the weights are 40 MB and more: 300 rows, 8 of 512 x 2048
+// (50 MB) 1.05 times, 16 of 1024 x 1024 (100 MB) 1.02, 16 of 2048 x 2048 1.07; 8 of 1024 x 512 (25 MB) 0.98, 16 of 768 x 384 and 768 (32 MB)
+// 0.97, 4 of 512 x 256 (3 MB) 0.92.
 extern "C" hipError_t dsse_moe_pipe(const dsse::MoeGroupedParams* p, hipStream_t st) {
-  return (int64_t)p->M * p->top <= 128 * (int64_t)p->E ? dsse::launch_moe_pipes<true>(*p, st) : dsse::launch_moe_pipes<false>(*p, st);
+  const int64_t weights = (int64_t)(p->gate ? 6 : 4) * p->W * ((int64_t)p->F * p->E + (p->S > p->top ? p->Fs : 0));
+  const bool once = p->once ? p->once == 1 : (int64_t)p->M * p->top <= 128 * (int64_t)p->E && weights >= 40000000;
+  return once ? dsse::launch_moe_pipes<true>(*p, st) : dsse::launch_moe_pipes<false>(*p, st);
 }

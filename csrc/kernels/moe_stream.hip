@@ -221,31 +221,59 @@ hipError_t launch_moe_stream(const MoeGroupedParams& p, hipStream_t st) {
 
 }  // namespace
 
-// To one list tile of every expert the stream reads each weight once and is ahead; from there on it is a matter of cost, in us: the stream
-// 24 and 155 per GB that it reads, a list tile's weights at a time; the pipeline 25, 84 per GB of the weights and 0.63 per K step of its
-// rounds of 256 workgroups.  Fitted over 27 sizes of 64 to 192 rows (rms 7 and 4 %); of 191 pairs four are decided for the slower one by
-// more than 2 %, by 7.5 % at most.  Stream / pipeline at 96, 129, 160, 192 rows, top 2: 16 experts of 4096 x 3584 and a shared one of 7168
-// 285 / 296, 302 / 301, 315 / 303, 313 / 308; 2048 x 1408 and 2816 73 / 95, 78 / 95, 81 / 95, 80 / 96; 5120 x 3584 and 7168 367 / 353, 391 / 364,
-// 406 / 370, 411 / 376; 4 of 4096 x 14336 251 / 363, 398 / 375, 470 / 372, 479 / 374; 8 of them 442 / 539 .. 481 / 566; 4 of 4096 x 3584 and 7168
-// 147 / 170, 217 / 173, 231 / 175, 232 / 176; top 8 of 16 of 4096 x 3584 258 / 240, 387 / 252, 485 / 260, 485 / 264.
-bool moe_stream_pays(const MoeGroupedParams& p) {
-  if (p.M > 3 * kMoeRows) return false;
-  if (p.M <= kMoeRows) return true;
+// The form of the expert GEMMs by cost, in us.  Up to 32 rows: the stream takes 8.3, 0.32 a list tile (to 16), and for each product the longer of
+// its K steps, 0.19 each, and its bytes, 166 per GB where 134 workgroups and more ask for them; the register-direct kernels 8, 0.23 a
+// list tile, and 0.094 a K step and 181 per GB that partly overlap.  Above, with S a form's K steps and G the GB it reads, a list tile's
+// weights at a time: the stream 17.6 + max(0.067 S, 148 G) + 2.05 min(..), the direct kernels 10.6 + max(0.315 S, 237 G) + 1.16 min(..), the
+// pipeline 20.4, 81 per GB of the weights and 0.683 per K step of its rounds of 256 workgroups.  Fitted over 49 sizes of 1 to 255 rows: of 589
+// choices 15 are for a form that is slower by more than 3 %, by 13 % at most.
+// Direct / stream, top 2 unless said: 1 row of 16 experts of 2048 x 2048 21 / 26, 2 rows 32 / 30; 4096 x 512 22 / 30, 4 rows 34 / 35, 8 50 / 43; 8 of
+// 1024 x 512 4 rows 14 / 17, 32 18 / 18; 4 of 512 x 256, top 1, 16 rows 12 / 15, 192 19 / 22 (pipeline 28); 16 of 2048 x 1408 and a shared one of
+// 2816 1 row 33 / 27, 32 rows 84 / 65.
+// Stream / pipeline at 96, 129, 160, 192 rows: 16 of 4096 x 3584 and 7168 285 / 296, 302 / 301, 315 / 303, 313 / 308; 2048 x 1408 and 2816 73 / 95,
+// 78 / 95, 81 / 95, 80 / 96; 5120 x 3584 and 7168 367 / 353, 391 / 364, 406 / 370, 411 / 376; 4 of 4096 x 14336 251 / 363, 398 / 375, 470 / 372, 479 / 374;
+// 8 of them 442 / 539 .. 481 / 566; 4 of 4096 x 3584 and 7168 147 / 170, 217 / 173, 231 / 175, 232 / 176; top 8 of 16 of 4096 x 3584 258 / 240,
+// 387 / 252, 485 / 260, 485 / 264.  Above 192 rows the stream is not asked (255 rows of 2048 x 1408 and 2816 101 / 99).
+MoeForm moe_form(const MoeGroupedParams& p) {
   const bool shared = p.S > p.top;
-  // list tiles of a routed expert: one, and a second and third as far as its rows' spread reaches over 64 and 128
-  const double rows = std::max(1.0, (double)p.M * p.top / p.E), spread = 3 * std::sqrt(rows);
-  double tiles_r = 1;
-  for (int i = 1; i <= 2; ++i) tiles_r += std::min(1.0, std::max(0.0, 0.5 + (rows - i * kMoeRows) / spread));
-  const int tiles_s = shared ? (p.M + kMoeRows - 1) / kMoeRows : 0;
-  const double unit = (p.gate ? 6e-9 : 4e-9) * p.W;  // GB per hidden unit
-  const double gb_r = unit * p.F * p.E, gb_s = shared ? unit * p.Fs : 0;
-  // the pipeline's K steps: tiles of 256 weight rows, the down product's of a shared expert counted by their length
-  auto blocks = [](int rows_w) { return (rows_w + 255) / 256; };
-  const int per = p.gate ? 2 : 1;
-  const int64_t up = (int64_t)p.E * blocks(per * p.F) + (shared ? blocks(per * p.Fs) : 0);
-  const double down = (double)blocks(p.W) * (p.E + (shared ? (double)p.Fs / p.F : 0));
-  const double steps = (double)((up + 255) / 256) * p.W / 64 + std::max(std::ceil(down / 256) * p.F, shared ? (double)p.Fs : 0.0) / 64;
-  return 24 + 155 * (tiles_r * gb_r + tiles_s * gb_s) <= 25 + 84 * (gb_r + gb_s) + 0.63 * steps;
+  const bool direct_ok = !p.lds_tiles, stream_ok = p.M <= 3 * kMoeRows, pipe_ok = p.M > 32;
+  if (p.form == 1 && stream_ok) return MoeForm::kStream;
+  if (p.form == 2) return MoeForm::kPipe;
+  if (p.form == 3 && direct_ok) return MoeForm::kDirect;
+  const int Fs = shared ? p.Fs : 0, long_f = std::max(p.F, Fs);
+  const int mats = p.gate ? 3 : 2;
+  const double unit = 2e-9 * mats * p.W;  // GB per hidden unit
+  const double hit = p.E * (1.0 - std::pow(1.0 - (double)p.top / p.E, p.M));  // experts that some row chooses
+  const double near = std::min(hit, 16.0), steps = (p.W + long_f) / 64.0;
+  double direct, stream, pipe = 0;
+  if (!pipe_ok) {
+    const double gb = unit * (p.F * hit + Fs), down = gb / mats, up = gb - down;
+    auto product = [](double gbs, int K, double wgs) { return std::max(0.19 * K / 64, 166 * gbs * std::max(1.0, 134 / wgs)); };
+    stream = 8.3 + 0.32 * near + product(up, p.W, (hit * p.F + Fs) / 64) + product(down, long_f, (hit + shared) * p.W / 64);
+    direct = 8.0 + 0.23 * near + std::pow(std::pow(0.094 * steps, 0.85) + std::pow(181 * gb, 0.85), 1 / 0.85);
+  } else {
+    // list tiles of a routed expert: one, and a second and third as far as its rows' spread reaches over 64 and 128
+    const double rows = std::max(1.0, (double)p.M * p.top / p.E), spread = 3 * std::sqrt(rows);
+    double tiles_r = 1;
+    for (int i = 1; i <= 2; ++i) tiles_r += std::min(1.0, std::max(0.0, 0.5 + (rows - i * kMoeRows) / spread));
+    const int tiles_s = (p.M + kMoeRows - 1) / kMoeRows;
+    const double gb = unit * (p.F * hit * tiles_r + Fs * (double)tiles_s);
+    auto both = [](double a, double b, double part) { return std::max(a, b) + part * std::min(a, b); };
+    stream = 17.6 + both(0.067 * steps, 148 * gb, 2.05);
+    direct = 10.6 + both(0.315 * steps, 237 * gb, 1.16);
+    // the pipeline's K steps: tiles of 256 weight rows, the down product's of a shared expert counted by their length
+    auto blocks = [](int rows_w) { return (rows_w + 255) / 256; };
+    const int per = p.gate ? 2 : 1;
+    const int64_t up = (int64_t)p.E * blocks(per * p.F) + blocks(per * Fs);
+    const double down = (double)blocks(p.W) * (p.E + (double)Fs / p.F);
+    const double rounds = (double)((up + 255) / 256) * p.W / 64 + std::max(std::ceil(down / 256) * p.F, (double)Fs) / 64;
+    pipe = 20.4 + 81 * unit * (p.F * hit + Fs) + 0.683 * rounds;
+  }
+  MoeForm best = stream_ok ? MoeForm::kStream : MoeForm::kPipe;
+  double least = stream_ok ? stream : pipe;
+  if (pipe_ok && pipe < least) best = MoeForm::kPipe, least = pipe;
+  if (direct_ok && direct < least) best = MoeForm::kDirect;
+  return best;
 }
 
 }  // namespace dsse

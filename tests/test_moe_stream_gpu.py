@@ -16,6 +16,15 @@ def gpu():
     return torch.device("cuda", 0)
 
 
+@pytest.fixture
+def stream(monkeypatch):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=1))  # experts this small would take the direct kernels
+    ops.refresh_env()
+    yield
+    monkeypatch.undo()
+    ops.refresh_env()
+
+
 # rows of expert 0 on both sides of the 16-, 32- and 64-row bodies; two K steps (fewer than any ring is deep), odd counts of
 # them, and K walks that wrap at every column block; widths that end inside a column block; rows that choose one expert only;
 # no shared expert; the largest step (three list tiles of the shared expert)
@@ -25,7 +34,7 @@ def gpu():
     (65, 448, 128, 128, 2, 1, 65, True), (100, 256, 576, 0, 3, 2, 64, False), (192, 320, 192, 128, 8, 2, 129, True),
     (40, 128, 128, 128, 300, 1, 0, True)])
 @pytest.mark.parametrize("weight_input", [False, True])
-def test_streamed_experts(gpu, M, W, F, Fs, E, top, first, gated, weight_input):
+def test_streamed_experts(gpu, stream, M, W, F, Fs, E, top, first, gated, weight_input):
     g = torch.Generator().manual_seed(M + W + F)
 
     def rnd(*s):
