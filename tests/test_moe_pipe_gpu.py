@@ -16,15 +16,26 @@ def gpu():
     return torch.device("cuda", 0)
 
 
+@pytest.fixture(params=[1, 2], ids=["once", "plain"])
+def pipe(request, monkeypatch):
+    # steps and experts this small would take other forms
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2, moe_once=request.param))
+    ops.refresh_env()
+    yield
+    monkeypatch.undo()
+    ops.refresh_env()
+
+
 # rows of expert 0 sit on both sides of a 64-row list tile and of the 128-, 192- and 256-row tiles; two K steps and odd
-# counts of them; output widths that end inside a column block; no shared expert, one expert, and a work list of more than
+# counts of them, fewer and more than the column blocks whose first steps differ; output widths that end inside a column block; no shared expert, one expert, and a work list of more than
 # 256 tiles (the list's chunks beyond those held in registers)
 @pytest.mark.parametrize("M,W,F,Fs,E,top,first,gated", [
     (128, 128, 128, 128, 2, 2, 64, True), (130, 320, 192, 448, 3, 2, 65, True), (257, 128, 448, 128, 2, 1, 129, True),
     (400, 192, 128, 0, 4, 2, 193, True), (513, 576, 320, 192, 3, 1, 257, True), (300, 128, 128, 0, 1, 1, 300, True),
-    (300, 128, 128, 128, 300, 1, 0, True), (700, 256, 192, 0, 3, 1, 256, False), (1100, 512, 128, 0, 2, 1, 1025, False)])
+    (300, 128, 128, 128, 300, 1, 0, True), (700, 256, 192, 0, 3, 1, 256, False), (1100, 512, 128, 0, 2, 1, 1025, False),
+    (200, 576, 448, 320, 8, 2, 40, True), (193, 1088, 192, 0, 4, 1, 65, True), (210, 192, 1088, 0, 5, 2, 64, False), (194, 2112, 128, 0, 2, 1, 130, True)])
 @pytest.mark.parametrize("weight_input", [False, True])
-def test_pipelined_experts(gpu, M, W, F, Fs, E, top, first, gated, weight_input):
+def test_pipelined_experts(gpu, pipe, M, W, F, Fs, E, top, first, gated, weight_input):
     g = torch.Generator().manual_seed(M + W + F)
 
     def rnd(*s):
