@@ -32,3 +32,20 @@ def test_gelu_cpu():
 @pytest.mark.parametrize("M", [1, 8, 9, 17, 48, 64, 65, 128, 150, 256, 257, 400, 1100])
 def test_gelu(M, F, K):
     check(M, F, K, "cuda")
+
+
+# gates far outside exp's range, whose squares overflow: z for the positive ones, zero for the negative ones, in both activations
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 17, 64, 100, 160, 300])
+@pytest.mark.parametrize("act", [ops.gemm_silu, ops.gemm_gelu])
+def test_large_gates(M, act):
+    F, K = 1024, 1024
+    x = torch.zeros(M, K)
+    x[:, 0] = 1
+    w = torch.zeros(2 * F, K)
+    gate = torch.tensor([2.0 ** 10, -2.0 ** 10, 2.0 ** 70, -2.0 ** 70, 2.0 ** 120, -2.0 ** 120, 0.0, float("inf")]).repeat(F // 8)
+    w[:F, 0], w[F:, 0] = gate, 0.5
+    out = torch.full((M, F), float("nan"), dtype=torch.bfloat16, device="cuda")
+    act(x.bfloat16().cuda(), tile_weight(w.bfloat16()[gate_up_perm(F)].contiguous()).cuda(), out)
+    want = (gate.clamp_min(0) * 0.5).expand(M, F)
+    assert torch.equal(out.float().cpu(), want)
