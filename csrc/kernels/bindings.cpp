@@ -482,7 +482,7 @@ TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
     if (cfg == 8 && M > 256 && M <= 384) cfg = 9;
   }
   constexpr int min_wgs = 160;  // split K until this many workgroups (table choices, M <= 512)
-  // tile shapes by cfg (gemm_tiled.hip launch_t_mode: 0, 1, 5; gemm_pipe.hip: 8, 9, 10)
+  // tile shapes by cfg (gemm_tiled.hip launch_t_mode: 0, 1, 2, 5; gemm_pipe.hip: 8, 9, 10); kind 2 is as tall as the rows, one row tile
   const int BM = cfg == 1 || cfg == 5 || cfg == 10 ? 128 : cfg == 9 ? 192 : 256, BN = cfg <= 2 ? 128 : 256;
   c.cfg = cfg;
   c.S = 1;

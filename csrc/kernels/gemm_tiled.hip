@@ -291,8 +291,8 @@ static hipError_t launch_t_mode(int cfg, const bf16* X, int ldx, int M, const bf
 
 // cfg: 0 = 256 x 128 tile (8 waves, 3 LDS stages), 1 = 128 x 128 (4 waves), 2 = 65-256 rows x 128 (8 waves, 4 or 3 stages), 5 = 128 x 256 (8 waves, 3 stages of 16
 // KiB X + 32 KiB W: twice the weight bytes in flight per CU of cfg 0, for the weight-streaming 129-256-row decode
-// GEMMs; the two row blocks of a column block share an XCD and its L2).  (Round 4's 256 x 256 configurations 2, 3, 4,
-// 6 and 7 are gone: gemm_pipe.hip, cfg 8, replaces them.)
+// GEMMs; the two row blocks of a column block share an XCD and its L2).  (256 x 256 configurations are
+// gone: gemm_pipe.hip, cfg 8, replaces them.)
 // (Round 3 also tried 4-stage rings and separate X / W loader rings for the 129-512-row decode buckets: all
 // slower in the 256-stream step, removed; profiles/r3/experiments_r3.md.)
 // Shape contract (checked by the caller): N % BN == 0, K % (64 S) == 0, the tiled weight layout (api.h).

@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     };
     int t = 0;
     for (; t < nk - 2; ++t) step(t, std::integral_constant<int, 0>{});
-    step(t++, std::integral_constant<int, 1>{});  // nk >= 2 (moe_pipe_ok)
+    step(t++, std::integral_constant<int, 1>{});  // nk >= 2 (moe_lines_ok)
     step(t, std::integral_constant<int, 2>{});
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // the two rows' barrier counts meet
 

@@ -137,9 +137,10 @@ PREFILL_SLAB_ROWS = 512
 
 # Prompt-chunk sizes of the captured mixed steps: one graph per (decode bucket, C).  The engine sizes each step's
 # chunk from the measured step costs (engine.PassCost.mixed_chunk); a prompt longer than the chunk is split evenly.
-# Every whole number of 64-row flash-prefill tiles: a step pays for its captured rows, 9 to 14 us each (Mistral-7B, 64
+# Every whole number of 64-row flash-prefill tiles: a step pays for its captured rows, 7 to 14 us each (Mistral-7B, 64
 # streams, C = 64 .. 448: 6.26, 7.18, 8.09, 8.81, 9.33, 10.04, 10.48 ms), so a chunk should not be padded by more than
-# a tile; with every second size alone a prompt of 300 rows ran as 384.  B + C stays within MIXED_MAX_ROWS: 768 was
+# a tile; with every second size alone a prompt of 300 rows ran as 384.  Its price is paid once: capture of decode and mixed
+# graphs of the buckets 1, 4, 16, 64, 128 and 256 takes 1.36 s and 67 MB, with every second size 1.12 s and 63 MB.  B + C stays within MIXED_MAX_ROWS: 768 was
 # measured with the serving bench at 40 req/s, TTFT p50 29.5 vs 29.8 ms, ITL p99 13.4 vs 10.7 ms
 # (profiles/r6/serving_r6.md).  The bigger chunks buy no TTFT and cost ITL, so 512 stays.
 MIXED_CHUNKS = tuple(range(64, 513, 64))

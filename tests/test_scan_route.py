@@ -25,7 +25,8 @@ def test_chunks_where_they_take_the_shape(D):
 @pytest.mark.parametrize("kw", [dict(channels=True), dict(pitch=1), dict(pitch=2), dict(shift=1), dict(D=48), dict(V=24),
                                 dict(T=200000, H=32, seqs=8)])
 def test_two_levels_where_chunks_are_refused(kw):
-    """Decays per key channel, rows that do not keep 16-byte alignment, other widths, a workspace of more than a gigabyte."""
+    """Decays per key channel that the question comes without, rows that do not keep 16-byte alignment, other widths, more rows times
+    heads than the chunks take."""
     a = dict(T=512, H=16, G=8, D=64, V=64)
     a.update(kw)
     assert two_levels(**a)
