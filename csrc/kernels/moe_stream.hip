@@ -221,15 +221,17 @@ hipError_t launch_moe_stream(const MoeGroupedParams& p, hipStream_t st) {
 
 }  // namespace
 
-// The form of the expert GEMMs by cost, in us.  Up to 32 rows: the stream takes 8.3, 0.32 a list tile (to 16), and for each product the longer of
-// its K steps, 0.19 each, and its bytes, 166 per GB where 134 workgroups and more ask for them; the register-direct kernels 8, 0.23 a
-// list tile, and 0.094 a K step and 181 per GB that partly overlap.  Above, with S a form's K steps and G the GB it reads, a list tile's
-// weights at a time: the stream 17.6 + max(0.067 S, 148 G) + 2.05 min(..), the direct kernels 10.6 + max(0.315 S, 237 G) + 1.16 min(..), the
-// pipeline 20.4, 81 per GB of the weights and 0.683 per K step of its rounds of 256 workgroups.  Fitted over 49 sizes of 1 to 255 rows: of 589
-// choices 15 are for a form that is slower by more than 3 %, by 13 % at most.
-// Direct / stream, top 2 unless said: 1 row of 16 experts of 2048 x 2048 21 / 26, 2 rows 32 / 30; 4096 x 512 22 / 30, 4 rows 34 / 35, 8 50 / 43; 8 of
-// 1024 x 512 4 rows 14 / 17, 32 18 / 18; 4 of 512 x 256, top 1, 16 rows 12 / 15, 192 19 / 22 (pipeline 28); 16 of 2048 x 1408 and a shared one of
-// 2816 1 row 33 / 27, 32 rows 84 / 65.
+// The form of the expert GEMMs by cost, in us.  Up to 32 rows: the stream takes 7.7, 0.36 a list tile (to 16), and for each product the longer of
+// its K steps, 0.19 each, and its bytes, 170 per GB where 119 workgroups and more ask for them; the register-direct kernels 8.6, 0.25 a
+// list tile, and the root of the sum of 0.17 a K step and 200 per GB, each to the power of 1.34, a tenth less without gates.  Above,
+// with S a form's K steps and G the GB it reads, a list tile's weights at a time: the stream 17.6 + max(0.067 S, 148 G) + 2.05 min(..), the
+// direct kernels 10.6 + max(0.315 S, 237 G) + 1.16 min(..), the pipeline 20.4, 81 per GB of the weights and 0.683 per K step of its rounds
+// of 256 workgroups.  Fitted over 57 sizes of 1 to 255 rows whose weights were last read 700 MB and more ago (choices of few experts are
+// otherwise timed from the last-level cache); of 711 choices 8 are for a form that is slower by more than 3 %, by 8 % at most.
+// Direct / stream, top 2 unless said: 1 row of 16 experts of 2048 x 2048 25 / 25, 2 rows 34 / 28, without gates 21 / 24, 26 / 26; of 4096 x
+// 4096 59 / 45, without gates 41 / 42 (Dironex-wide's step 943 / 888); 4096 x 512 1 row 26 / 30, 4 rows 34 / 35; 8 of 1024 x 512 4 rows
+// 16 / 16, 32 18 / 18; 4 of 512 x 256, top 1, 16 rows 13 / 14, 192 19 / 22 (pipeline 28); 16 of 2048 x 1408 and a shared one of 2816 1 row
+// 36 / 28, 32 rows 89 / 67.
 // Stream / pipeline at 96, 129, 160, 192 rows: 16 of 4096 x 3584 and 7168 285 / 296, 302 / 301, 315 / 303, 313 / 308; 2048 x 1408 and 2816 73 / 95,
 // 78 / 95, 81 / 95, 80 / 96; 5120 x 3584 and 7168 367 / 353, 391 / 364, 406 / 370, 411 / 376; 4 of 4096 x 14336 251 / 363, 398 / 375, 470 / 372, 479 / 374;
 // 8 of them 442 / 539 .. 481 / 566; 4 of 4096 x 3584 and 7168 147 / 170, 217 / 173, 231 / 175, 232 / 176; top 8 of 16 of 4096 x 3584 258 / 240,
@@ -248,9 +250,9 @@ MoeForm moe_form(const MoeGroupedParams& p) {
   double direct, stream, pipe = 0;
   if (!pipe_ok) {
     const double gb = unit * (p.F * hit + Fs), down = gb / mats, up = gb - down;
-    auto product = [](double gbs, int K, double wgs) { return std::max(0.19 * K / 64, 166 * gbs * std::max(1.0, 134 / wgs)); };
-    stream = 8.3 + 0.32 * near + product(up, p.W, (hit * p.F + Fs) / 64) + product(down, long_f, (hit + shared) * p.W / 64);
-    direct = 8.0 + 0.23 * near + std::pow(std::pow(0.094 * steps, 0.85) + std::pow(181 * gb, 0.85), 1 / 0.85);
+    auto product = [](double gbs, int K, double wgs) { return std::max(0.193 * K / 64, 170 * gbs * std::max(1.0, 119 / wgs)); };
+    stream = 7.7 + 0.36 * near + product(up, p.W, (hit * p.F + Fs) / (p.gate ? 64 : 128)) + product(down, long_f, (hit + shared) * p.W / 64);
+    direct = 8.6 + 0.25 * near + (p.gate ? 1.0 : 0.89) * std::pow(std::pow(0.17 * steps, 1.34) + std::pow(200 * gb, 1.34), 1 / 1.34);
   } else {
     // list tiles of a routed expert: one, and a second and third as far as its rows' spread reaches over 64 and 128
     const double rows = std::max(1.0, (double)p.M * p.top / p.E), spread = 3 * std::sqrt(rows);

@@ -16,8 +16,10 @@ STREAM, PIPE, DIRECT = 1, 0, 2
     (96, 4096, 14336, 0, 4, 2, True, STREAM), (160, 4096, 14336, 0, 4, 2, True, PIPE), (192, 4096, 14336, 0, 8, 2, True, STREAM),
     (96, 4096, 3584, 7168, 4, 2, True, STREAM), (160, 4096, 3584, 7168, 4, 2, True, PIPE), (160, 4096, 3584, 0, 16, 8, True, PIPE),
     (192, 2048, 1408, 2816, 64, 6, True, STREAM), (193, 2048, 1408, 2816, 16, 2, True, PIPE), (300, 256, 128, 0, 4, 1, True, PIPE),
-    (1, 2048, 2048, 0, 16, 2, True, DIRECT), (4, 2048, 2048, 0, 16, 2, True, STREAM), (1, 4096, 512, 0, 16, 2, True, DIRECT), (8, 4096, 512, 0, 16, 2, True, STREAM),
+    (1, 2048, 2048, 0, 16, 2, True, STREAM), (4, 2048, 2048, 0, 16, 2, True, STREAM), (1, 4096, 512, 0, 16, 2, True, DIRECT), (8, 4096, 512, 0, 16, 2, True, STREAM),
     (16, 512, 256, 0, 4, 1, True, DIRECT), (255, 512, 256, 0, 4, 1, True, DIRECT), (256, 512, 256, 0, 4, 1, True, PIPE), (1, 2048, 1408, 2816, 16, 2, True, STREAM),
+    (1, 2048, 2048, 0, 16, 2, False, DIRECT), (4, 2048, 2048, 0, 16, 2, False, STREAM), (1, 4096, 4096, 0, 16, 2, False, STREAM), (1, 1536, 768, 0, 16, 1, True, DIRECT), (2, 4096, 4096, 0, 16, 2, False, STREAM),
+    (1, 4096, 4096, 0, 16, 2, True, STREAM),
     (64, 2048, 1400, 0, 16, 2, True, -1), (64, 64, 128, 0, 16, 2, True, -1)])
 def test_plan(M, W, F, Fs, E, top, gated, want):
     ops.load_library(required=True)
