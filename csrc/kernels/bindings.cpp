@@ -134,8 +134,8 @@ bool skinny_pairs(int M, int N) {
 // workgroups and K walks of at most two rounds.  Sliced / skinny, us: 2048 x 2048 17 rows 9.8 / 7.7, 32 rows 10.7 / 9.3, 48 rows 10.6 /
 // 11.9; 4096 x 2048 17 rows 10.8 / 8.1, 32 11.4 / 9.7; 2048 x 2560 32 rows 10.8 / 10.7; 2048 x 4096 24 rows 11.8 / 12.3; 2048 x 1024 64
 // rows 10.1 / 9.3; 6144 x 2048 24 rows 12.3 / 12.6.  K % 512 != 0 (a tensor-parallel shard's) stays with the ring kernel.
-// Not where the next kernel sums the slices (gemm_impl's slab_consumer): product and RMSNorm, sliced / skinny, 4096 x 2048 24 rows 12.0 /
-// 13.6, 2048 x 2048 32 rows 10.6 / 13.3, 4096 x 1024 64 rows 11.9 / 17.0, 4096 x 512 32 rows 10.3 / 11.1.
+// Not where the next kernel sums the slices (gemm_impl's slab_consumer): product and RMSNorm, sliced / skinny, 4096 x 2048 32 rows 11.9 /
+// 13.9, 2048 x 2048 9.8 / 12.8, 4096 x 1024 64 rows 11.5 / 16.4, 4096 x 512 32 rows 10.4 / 10.5; but 4096 x 2560 17 rows 14.6 / 13.1.
 bool skinny_whole(int M, int N, int K) {
   return gemm_rules_free() && M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
 }
