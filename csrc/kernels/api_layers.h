@@ -156,8 +156,9 @@ struct MoeGroupedParams {
   int* tile_expert;      // [max_tiles]
   int* num_tiles;        // [1]
   void* h;               // [M * S, ldh] element type
-  float* o;              // [M * S, W]
+  float* o;              // [M * parts, W]: a row's parts are its slots, and the further slices of the shared expert's
   int M, W, F, Fs, E, top, S, ldh, max_tiles;
+  int parts;             // S, or S + n: the shared expert's down product in n + 1 slices of its hidden units (moe_parts)
   int vec_w, vec_h;      // 16-byte fragment loads allowed on rows W wide / on rows of h
   int aligned;           // 1: sorted / tile_expert / num_tiles are already made (moe_route_rows)
   int lds_tiles;         // 1: enough rows for the LDS-staged tiles (prompt portions); 0: the register-direct kernels
@@ -172,6 +173,9 @@ bool moe_lines_ok(const MoeGroupedParams& p);
 // Which form those take: the register-direct kernels of moe.hip (few rows of small experts), the stream, the pipeline
 enum class MoeForm { kDirect, kStream, kPipe };
 MoeForm moe_form(const MoeGroupedParams& p);
+// Parts of a row of o that the step is best computed in: S, or S + 1 where the shared expert's hidden units are worth two slices (moe_pipe.hip)
+constexpr int kMoeSlices = 2;
+int moe_parts(const MoeGroupedParams& p);
 
 // Router, choice and work list of a decode-sized step in one launch.
 struct MoeRouteRowsParams {

@@ -450,12 +450,13 @@ void moe_ffn(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, cons
 }
 
 // Grouped form of the routed experts: o [M * S, W] (fp32) = per-(row, slot) expert outputs times their weights, S = top
-// (+ 1 with a shared expert); the caller sums a row's S parts (scalar_norm nsum).  Scratch: sorted [tiles * 64],
+// (+ 1 with a shared expert; + 1 more, as moe_parts says, for the second slice of the shared one's hidden units); the caller sums a row's
+// parts (scalar_norm nsum).  Scratch: sorted [tiles * 64],
 // tile_expert [tiles], num_tiles [1] (int32), h [M * S, ldh] (element type), tiles >= ceil(M S / 64) + experts + 1.
 void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, const OptTensor& gate, const Tensor& up,
                  const Tensor& down, const OptTensor& sgate, const OptTensor& sup, const OptTensor& sdown, Tensor& sorted,
                  Tensor& tile_expert, Tensor& num_tiles, Tensor& h, Tensor& o, bool weight_input,
-                 bool aligned) {
+                 bool aligned, int64_t parts) {
   gpu(x, "x");
   i32(topk_idx, "topk_idx");
   f32t(topk_w, "topk_w");
@@ -509,9 +510,12 @@ void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, 
   p.max_tiles = (int)tile_expert.numel();
   TORCH_CHECK(p.max_tiles >= (ids + 63) / 64 + p.E + 1 && sorted.numel() >= (int64_t)p.max_tiles * 64 && p.max_tiles <= 65535,
               "moe_grouped: scratch too small for ", ids, " ids");
-  TORCH_CHECK(h.dim() == 2 && h.size(0) >= ids && h.size(1) >= std::max(p.F, p.Fs) && o.dim() == 2 && o.size(0) == ids &&
-                  o.size(1) == p.W && p.E + 1 <= 4096,
+  TORCH_CHECK(h.dim() == 2 && h.size(0) >= ids && h.size(1) >= std::max(p.F, p.Fs) && o.dim() == 2 && o.size(1) == p.W &&
+                  p.E + 1 <= 4096,
               "moe_grouped: h / o shapes");
+  p.parts = parts ? (int)parts : p.S;
+  TORCH_CHECK(parts == 0 || parts == p.S || (sgate.has_value() && parts > p.S && parts < p.S + dsse::kMoeSlices), "moe_grouped: parts as moe_parts says");
+  TORCH_CHECK(o.size(0) == (int64_t)p.M * p.parts, "moe_grouped: o must hold ", p.parts, " parts of every row");
   p.ldh = (int)h.size(1);
   p.x = x.data_ptr();
   p.topk_idx = topk_idx.data_ptr<int>();
@@ -530,6 +534,8 @@ void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, 
   p.vec_h = p.ldh % per == 0 && p.F % per == 0;
   p.lds_tiles = ids >= 256;  // prompt-sized: most 64-row tiles are full
   p.form = dsse::kernel_cfg_int("moe_form", 0), p.once = dsse::kernel_cfg_int("moe_once", 0);
+  TORCH_CHECK(p.parts == p.S || (dsse::moe_lines_ok(p) && dsse::moe_form(p) != dsse::MoeForm::kDirect && p.Fs / 64 >= 2 * (p.parts - p.S + 1)),
+              "moe_grouped: this step's shared expert cannot be computed in ", p.parts - p.S + 1, " slices (moe_parts)");
   DSSE_CHECK_HIP(dsse_moe_grouped(&p, cur_stream()));
 }
 
@@ -578,6 +584,26 @@ void moe_topk(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w) {
               "moe_topk shapes");
   DSSE_CHECK_HIP(dsse_moe_topk(logits.data_ptr<float>(), M, E, top, topk_idx.data_ptr<int>(), topk_w.data_ptr<float>(),
                                cur_stream()));
+}
+
+// Rows of moe_grouped's o per row of x: its slots, and one more where the shared expert is better computed in two slices (h: the
+// scratch that moe_grouped will get)
+int64_t moe_parts(const Tensor& x, int64_t top, const OptTensor& gate, const Tensor& up, const Tensor& down, const OptTensor& sgate,
+                  const OptTensor& sup, const OptTensor& sdown, const Tensor& h) {
+  TORCH_CHECK(x.dim() == 2 && up.dim() == 3 && h.dim() == 2 && (!sgate.has_value() || (sgate->dim() == 2 && sup.has_value() && sdown.has_value())),
+              "moe_parts shapes");
+  dsse::MoeGroupedParams p{};
+  p.M = (int)x.size(0), p.W = (int)x.size(1), p.E = (int)up.size(0), p.F = (int)up.size(1), p.top = (int)top;
+  p.Fs = sgate.has_value() ? (int)sgate->size(0) : 0;
+  p.S = p.parts = p.top + (sgate.has_value() ? 1 : 0);
+  p.ldh = (int)h.size(1);
+  p.x = x.data_ptr(), p.up = up.data_ptr(), p.down = down.data_ptr(), p.h = h.data_ptr();
+  p.gate = gate.has_value() ? gate->data_ptr() : nullptr;
+  if (sgate.has_value()) p.sgate = sgate->data_ptr(), p.sup = sup->data_ptr(), p.sdown = sdown->data_ptr();
+  p.f32 = elem(x, "x");
+  p.lds_tiles = (int64_t)p.M * p.S >= 256;
+  p.form = dsse::kernel_cfg_int("moe_form", 0);
+  return p.M ? dsse::moe_parts(p) : p.S;
 }
 
 // Which form the expert GEMMs of moe_grouped take for bf16 operands on LDS-DMA: 1 the stream (moe_stream.hip), 0 the pipeline
@@ -632,7 +658,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("scalar_norm(Tensor? y, Tensor g, Tensor(a!) resid, Tensor(b!) xb, float eps, int nsum=1) -> ()");
   m.def("moe_grouped(Tensor x, Tensor topk_idx, Tensor topk_w, Tensor? gate, Tensor up, Tensor down, Tensor? sgate, "
         "Tensor? sup, Tensor? sdown, Tensor(a!) sorted, Tensor(b!) tile_expert, Tensor(c!) num_tiles, Tensor(d!) h, "
-        "Tensor(e!) o, bool weight_input=False, bool aligned=False) -> ()");
+        "Tensor(e!) o, bool weight_input=False, bool aligned=False, int parts=0) -> ()");
   m.def("moe_route_rows(Tensor x, Tensor w, Tensor(a!) topk_idx, Tensor(b!) topk_w, float scale, Tensor(c!) sorted, "
         "Tensor(d!) tile_expert, Tensor(e!) num_tiles) -> ()");
   m.def("embed_rows(Tensor ids, Tensor embed, Tensor(a!) resid, Tensor(b!)? xb, float scale=1.0, Tensor? positions=None, "
@@ -651,6 +677,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_plan(int M, int W, int F, int Fs, int E, int top, bool gated) -> int", &moe_plan);
+  m.def("moe_parts(Tensor x, int top, Tensor? gate, Tensor up, Tensor down, Tensor? sgate, Tensor? sup, Tensor? sdown, Tensor h) -> int");
   m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "
         "Tensor(e!) num_tiles, bool shared) -> bool");
   m.def("moe_ffn(Tensor x, Tensor topk_idx, Tensor topk_w, Tensor gate, Tensor up, Tensor down, Tensor? sgate, "
@@ -670,5 +697,6 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("moe_topk_lists", &moe_topk_lists);
   m.impl("moe_ffn", &moe_ffn);
   m.impl("moe_grouped", &moe_grouped);
+  m.impl("moe_parts", &moe_parts);
   m.impl("moe_route_rows", &moe_route_rows);
 }

@@ -38,8 +38,8 @@ namespace mp {
 constexpr int kA = 256 * 128;   // row image of one K step: 256 rows x 64 bf16
 constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 bf16
 constexpr int kBuf = kA + kB;
-constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), then their weights (256 floats)
-constexpr size_t kLDS = kIds + 2 * 256 * 4;
+constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), their weights (256 floats), their rows of the result (256 ints)
+constexpr size_t kLDS = kIds + 3 * 256 * 4;
 
 struct Place {
   int first;  // the expert's first list tile
@@ -104,7 +104,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
   row_tiles = walk([&](int, int v, int, bool, int) { routed += __popcll(__ballot(v < p.E)); });
   const int shared = list.n - routed;
   const int nb_r = blocks(p.F), nb_s = blocks(p.Fs);
-  const int total_s = (shared + tall - 1) / tall * nb_s, total_r = row_tiles * nb_r;
+  const int slices = MODE == 1 ? p.parts - p.S + 1 : 1;  // of the shared expert's hidden units
+  const int tiles_s = (shared + tall - 1) / tall * nb_s, total_s = tiles_s * slices, total_r = row_tiles * nb_r;
 
   for (int v = blockIdx.x; ; v += gridDim.x) {  // one tile; a second round only if a choice list is not what it should be
     const int x = v & 7, u = v >> 3;
@@ -116,7 +117,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     Place pl;
     int e;
     if (sh) {
-      pl = Place{routed, shared, s0 + u};
+      pl = Place{routed, shared, (s0 + u) % tiles_s};
       e = p.E;
     } else {
       const int at = r0 + u - ns, want = at / nb_r;
@@ -145,7 +146,9 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
 
     const int Fe = sh ? p.Fs : p.F;
     const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
-    const int nk = K >> 6, off = ONCE ? n0 / kCols % nk : 0;
+    const int slice = sh ? (s0 + u) / tiles_s : 0, cut = sh ? slices : 1;
+    const int first = (K >> 6) * slice / cut, nk = (K >> 6) * (slice + 1) / cut - first;  // its K steps
+    const int off = ONCE ? n0 / kCols % nk : 0;
     const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
     const int ldx = MODE == 1 ? p.ldh : p.W;
     auto weights = [&](const void* routed_w, const void* shared_w) {
@@ -159,11 +162,13 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
 
     int* s_id = reinterpret_cast<int*>(smem + kIds);
     float* s_w = reinterpret_cast<float*>(smem + kIds + 256 * 4);
+    int* s_o = reinterpret_cast<int*>(smem + kIds + 2 * 256 * 4);
     __syncthreads();  // a second tile: every wave is past the first one's epilogue
     if ((int)threadIdx.x < rows64 * 64) {
       const int id = ld_global<int>(p.sorted + t0 * 64 + threadIdx.x);
       const int row = id >= 0 ? id / p.S : 0;
       s_id[threadIdx.x] = id;
+      s_o[threadIdx.x] = row * (p.parts - p.S) + id + slice;
       s_w[threadIdx.x] = id < 0 ? 0.0f : (MODE == 1 ? out_weight(p, row, id - row * p.S) : in_weight(p, id));
     }
     __syncthreads();
@@ -189,7 +194,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         b_lo[h][i] = kA + (tb * 16 + (j & 1) * 8) * 128;
         b_vo[h][i] = n < N ? (uint32_t)(((size_t)n * K + 8 * ((lane & 7) ^ piece_swizzle(br))) * 2) : kOOB;
       }
-    auto place = [&](int t) { return (uint32_t)(t + off < nk ? t + off : t + off - nk) * 128; };
+    auto place = [&](int t) { return (uint32_t)(first + (t + off < nk ? t + off : t + off - nk)) * 128; };
     auto issue_a = [&](int h, int t) {
       char* base = smem + (t & 1) * kBuf;
 #pragma unroll
@@ -318,7 +323,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
               const int f = n0 + (wn * 4 + n) * 16 + r;
               if (f >= N) continue;
               const float v = c[n][j] * wt;
-              if (MODE == 1) p.o[(int64_t)id * p.W + f] = v;
+              if (MODE == 1) p.o[(int64_t)s_o[at] * p.W + f] = v;
               else reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(v > 0.0f ? v * v : 0.0f);
             }
           }
@@ -336,11 +341,12 @@ int64_t routed_tiles(const MoeGroupedParams& p, int mode, int tall) {
   return std::min((ids + (rows - 1) * p.E) / rows, ids) * col_blocks(p, mode, p.F);
 }
 int64_t shared_tiles(const MoeGroupedParams& p, int mode, int tall) {
-  return p.S > p.top ? (p.M + 64 * (int64_t)tall - 1) / (64 * tall) * col_blocks(p, mode, p.Fs) : 0;
+  const int64_t slices = mode == 1 ? p.parts - p.S + 1 : 1;
+  return p.S > p.top ? (p.M + 64 * (int64_t)tall - 1) / (64 * tall) * col_blocks(p, mode, p.Fs) * slices : 0;
 }
-// The row tiles' greatest height: the one whose tiles finish first by a simple model, rounds of 256 workgroups (one per CU)
-// times the tiles' mean time.  A tile of 1 / 2 / 3 / 4 list tiles takes 0.5 / 0.7 / 0.85 / 1 of the tallest one's time
-// (0.75 to 1.7 us per K step, measured at 2048 x 1024, 8 experts); choices spread evenly over the experts but for one
+// The row tiles' greatest height in the gate / up product: the one whose tiles finish first by a simple model, rounds of 256
+// workgroups (one per CU) times the tiles' mean time.  A tile of 1 / 2 / 3 / 4 list tiles takes 0.5 / 0.7 / 0.85 / 1 of the tallest one's
+// time (0.75 to 1.7 us per K step, measured at 2048 x 1024, 8 experts); choices spread evenly over the experts but for one
 // standard deviation, which is what decides whether a round is full.
 int moe_pipe_height(const MoeGroupedParams& p, int mode) {
   static const double kTime[5] = {0.0, 0.5, 0.7, 0.85, 1.0};
@@ -360,6 +366,74 @@ int moe_pipe_height(const MoeGroupedParams& p, int mode) {
   return best;
 }
 
+// The down product's row tiles and what it takes with them.  Here tiles differ in length: a shared expert's K axis is its hidden
+// width, most often twice a routed one's, and with its tiles first the rest may wait for the last of them: 700 rows of 2048 x 1408, 16
+// experts, took 52 us with a shared expert of 2816 and 34 without.  So its hidden units may be cut into slices, each a part of its own
+// in o, which the norm that follows adds.
+struct Height {
+  int tall;
+  double us;
+};
+
+// What is asked: when the last of 256 CUs is done if every tile goes to the one that is free first, tiles in the order of the kernel (6 us each
+// and 1.3 per K step of the tallest, 0.54 / 0.72 / 0.86 of it for 1 / 2 / 3 list tiles); the weights at 160 us per GB, three tenths of that where another
+// row tile reads them again; 0.3 of the shorter one of the two; 400 us per GB of further parts, written and read.  Rows per expert: normal about
+// their mean.
+Height down_height(const MoeGroupedParams& p, int slices) {
+  static const double kTime[5] = {0.0, 0.54, 0.72, 0.86, 1.0};
+  const bool shared = p.S > p.top;
+  const int cols = (p.W + 255) / 256;
+  const double each = (double)p.M * p.top / p.E, sd = std::sqrt(each);
+  const double hit = p.E * (1.0 - std::pow(1.0 - (double)p.top / p.E, p.M));
+  auto below = [&](int k) { return 0.5 * std::erfc((each - 64.0 * k) / (1.4142135623730951 * sd)); };  // share of experts of k list tiles at most
+  const int lo = std::max(1, (int)std::ceil((each - 2 * sd) / 64)), hi = std::max(lo, (int)std::ceil((each + 2 * sd) / 64));
+  Height best{4, 0.0};
+  for (int tall = 4; tall >= 1; tall /= 2) {
+    struct {
+      double until, cus;
+    } g[32] = {{0.0, 256.0}};
+    int n = 1;
+    double last = 0.0, again = 0.0;
+    auto tiles = [&](double count, double steps, int q) {
+      const double t = 6.0 + 1.3 * steps * kTime[q];
+      while (count > 1e-6) {
+        int first = 0;
+        for (int i = 1; i < n; ++i)
+          if (g[i].until < g[first].until) first = i;
+        const double take = std::min(count, g[first].cus), until = g[first].until + t;
+        g[first].cus -= take;
+        count -= take;
+        int at = first;
+        if (g[first].cus > 1e-6) {
+          for (at = 0; at < n && std::abs(g[at].until - until) > 1e-6; ++at) {}
+          if (at == n) {
+            if (n < 32) g[n++] = {until, 0.0};
+            else at = first;  // (never seen) the classes are few
+          }
+        }
+        g[at].until = until;
+        g[at].cus += take;
+        last = std::max(last, until);
+      }
+    };
+    auto expert = [&](double count, int k, double steps) {  // `count` times the tiles of an expert of k list tiles
+      const int T = (k + tall - 1) / tall, q = (k + T - 1) / T;
+      tiles(count * (k / q), steps, q);
+      if (k % q) tiles(count, steps, k % q);
+      return T - 1;
+    };
+    if (shared) again += (double)p.Fs * expert((double)cols * slices, (p.M + 63) / 64, p.Fs / 64.0 / slices);
+    for (int k = lo; k <= hi; ++k) {
+      const double share = (k < hi ? below(k) : 1.0) - (k > lo ? below(k - 1) : 0.0);
+      if (share * hit > 0.05) again += share * hit * p.F * expert(share * hit * cols, k, p.F / 64.0);
+    }
+    const double gb = 2e-9 * p.W * (p.F * hit + (shared ? p.Fs : 0) + 0.3 * again);
+    const double us = std::max(last, 160.0 * gb) + 0.3 * std::min(last, 160.0 * gb) + 400 * 8e-9 * p.M * p.W * (slices - 1);
+    if (tall == 4 || us < best.us) best = Height{tall, us};
+  }
+  return best;
+}
+
 template <int MODE, bool ONCE>
 hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
   static bool attr_set = false;
@@ -368,7 +442,7 @@ hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)mp::kLDS);
     attr_set = true;
   }
-  const int tall = moe_pipe_height(p, MODE);
+  const int tall = MODE == 1 ? down_height(p, p.parts - p.S + 1).tall : moe_pipe_height(p, MODE);
   const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8);
   hipLaunchKernelGGL((moe_pipe_kernel<MODE, ONCE>), dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
   return hipGetLastError();
@@ -393,6 +467,22 @@ bool moe_lines_ok(const MoeGroupedParams& p) {
   if ((int64_t)p.M * p.W * 2 >= kRange || ids * p.ldh * 2 >= kRange || widest * p.W * 2 >= kRange) return false;
   if (!pieces(p.x) || !pieces(p.h) || !pieces(p.up) || !pieces(p.down) || (p.gate && !pieces(p.gate))) return false;
   return !shared || (pieces(p.sgate) && pieces(p.sup) && pieces(p.sdown));
+}
+
+// Two slices where they end sooner.  One / two, work list, both products and the norm that adds the parts, in us: 2048 x 1408, 16 experts,
+// top 2, shared 2816: 200 rows 103 / 90, 700 125 / 111, 1500 203 / 182, 2048 222 / 238; 1024 x 2048, 8 of them, 4096: 256 rows 94 / 71, 2500
+// 221 / 189; 4096 x 3584, 4 of them, 7168: 300 rows 218 / 183, 1300 490 / 488; 16 of them, bound by their bytes: 200 rows 317 / 321, 3000
+// 1083 / 1104.  Three and four are behind two.  Over 200 sizes of 12 widths the geometric mean is 1.045, one of them 5 % behind (1000 rows of the
+// third: 384 / 403).  The stream up to 192 rows (moe_form): two where the shared expert's K steps, 0.45 us each, outlast the bytes, 170 us per GB:
+// 1 row of the first 31 / 28, 64 77 / 72, 192 85 / 89; 96 rows of the third 150 / 137, 128 153 / 158; 64 rows of the second 56 / 48.
+int moe_parts(const MoeGroupedParams& p) {
+  if (p.S == p.top || p.Fs < 4 * 64 || !moe_lines_ok(p)) return p.S;
+  const MoeForm form = moe_form(p);
+  if (form == MoeForm::kDirect) return p.S;
+  if (form == MoeForm::kPipe) return down_height(p, 2).us < down_height(p, 1).us ? p.S + 1 : p.S;
+  const double rows = (double)p.M * p.top / p.E, hit = p.E * (1.0 - std::pow(1.0 - (double)p.top / p.E, p.M));
+  const double tiles = std::max(1.0, 0.5 + rows / 64), gb = 2e-9 * p.W * (p.F * hit * tiles + (double)p.Fs * ((p.M + 63) / 64));
+  return 0.45 * p.Fs / 64 > 170 * gb ? p.S + 1 : p.S;
 }
 
 }  // namespace dsse

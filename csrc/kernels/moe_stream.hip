@@ -48,7 +48,7 @@ constexpr int kLDS = 80 * 1024;   // two workgroups per CU
 // MODE 0: h = silu(gate x) * (up x); 1: o = weight * down h; 2: h = relu(up x)^2.  The column block cb of the list tile whose
 // ids the lanes hold in `mine`, the first `rows` of them real.
 template <int MODE, int SUBS>
-DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int mine, int rows) {
+DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int mine, int rows, int slice) {
   using namespace ms;
   constexpr int CT = wave_tiles(MODE), D = depth(MODE, SUBS), NX = x_dma(SUBS), NW = 2 * CT;
   static_assert(lds_bytes(MODE, SUBS) <= kLDS);
@@ -57,7 +57,8 @@ DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int m
   const bool sh = e >= p.E;
   const int Fe = sh ? p.Fs : p.F;
   const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
-  const int nk = K / kStep, first = cb % nk;
+  const int cut = MODE == 1 && sh ? p.parts - p.S + 1 : 1;  // the shared expert's hidden units in slices
+  const int begin = K / kStep * slice / cut, nk = K / kStep * (slice + 1) / cut - begin, first = cb % nk;
   const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
   const int ldx = MODE == 1 ? p.ldh : p.W;
 
@@ -91,7 +92,7 @@ DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int m
   // byte offset of step c in every row; a step past the last lands as zeros, without traffic
   auto place = [&](int c) {
     const int k = c + first < nk ? c + first : c + first - nk;
-    return c < nk ? (uint32_t)k * 128 : kOOB;
+    return c < nk ? (uint32_t)(begin + k) * 128 : kOOB;
   };
   auto issue_w = [&](int c, int slot) {
     const uint32_t at = place(c);
@@ -169,7 +170,7 @@ DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int m
           const int f = n0 + 16 * n + r;
           if (f >= N) continue;
           const float v = acc[i][n][j] * wt;
-          if (MODE == 1) p.o[(int64_t)id * p.W + f] = v;
+          if (MODE == 1) p.o[((int64_t)row * (p.parts - p.S) + id + slice) * p.W + f] = v;
           else reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(v > 0.0f ? v * v : 0.0f);
         }
       }
@@ -180,10 +181,10 @@ DEV void stream_tile(const MoeGroupedParams& p, char* smem, int e, int cb, int m
 template <int MODE>
 __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeGroupedParams p, int shared_tiles, int cols_s, int cols_r) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int v = blockIdx.x, head = shared_tiles * cols_s;
+  const int v = blockIdx.x, each = shared_tiles * cols_s, head = MODE == 1 ? each * (p.parts - p.S + 1) : each;
   const int tiles = __builtin_amdgcn_readfirstlane(ld_global<int>(p.num_tiles));
-  int t, cb;
-  if (v < head) t = max(tiles - shared_tiles, 0) + v / cols_s, cb = v % cols_s;
+  int t, cb, slice = 0;
+  if (v < head) slice = v / each, t = max(tiles - shared_tiles, 0) + v % each / cols_s, cb = v % cols_s;
   else t = (v - head) / cols_r, cb = (v - head) % cols_r;
   // a routed tile's expert and ids are requested together with the tile count: the list has room for every t of the grid
   const int e = __builtin_amdgcn_readfirstlane(ld_global<int>(p.tile_expert + t));
@@ -191,9 +192,9 @@ __global__ void __launch_bounds__(256, 2) moe_stream_kernel(MoeGroupedParams p, 
   if (e < 0 || (v >= head && t >= tiles - shared_tiles)) return;
   if (cb * ms::columns(MODE) >= (MODE == 1 ? p.W : (e >= p.E ? p.Fs : p.F))) return;
   const int rows = __popcll(__ballot(mine >= 0));  // an expert's ids fill its tiles from the front
-  if (rows <= 16) stream_tile<MODE, 1>(p, smem, e, cb, mine, rows);
-  else if (rows <= 32) stream_tile<MODE, 2>(p, smem, e, cb, mine, rows);
-  else stream_tile<MODE, 4>(p, smem, e, cb, mine, rows);
+  if (rows <= 16) stream_tile<MODE, 1>(p, smem, e, cb, mine, rows, slice);
+  else if (rows <= 32) stream_tile<MODE, 2>(p, smem, e, cb, mine, rows, slice);
+  else stream_tile<MODE, 4>(p, smem, e, cb, mine, rows, slice);
 }
 
 template <int MODE>
@@ -214,7 +215,7 @@ hipError_t launch_moe_stream(const MoeGroupedParams& p, hipStream_t st) {
   // most list tiles that the routed experts can make
   const int64_t routed = std::min((ids + (int64_t)(kMoeRows - 1) * p.E) / kMoeRows, ids);
   const int cols_s = shared ? blocks(p.Fs) : 1, cols_r = blocks(p.F);
-  const int64_t grid = (int64_t)shared * cols_s + routed * cols_r;
+  const int64_t grid = (int64_t)shared * cols_s * (MODE == 1 ? p.parts - p.S + 1 : 1) + routed * cols_r;
   hipLaunchKernelGGL(moe_stream_kernel<MODE>, dim3((unsigned)grid), dim3(256), ms::kLDS, st, p, shared, cols_s, cols_r);
   return hipGetLastError();
 }

@@ -298,7 +298,7 @@ class LayeredRunner(RunnerBase):
             d["mo_tile"] = torch.zeros(tiles, device=dev, dtype=torch.int32)
             d["mo_n"] = torch.zeros(1, device=dev, dtype=torch.int32)
             d["mo_h"] = torch.zeros(M * slots, ldh, **el)
-            d["mo_o"] = new(M * slots * W, **f32)
+            d["mo_o"] = new(M * (slots + any(f.shared_ff for f in moe)) * W, **f32)  # a shared expert may come in two parts
         return d
 
     # ------------------------------------------------------------------ layers
@@ -375,17 +375,17 @@ class LayeredRunner(RunnerBase):
         self._lin(hs, Lw.o, Lw.o_t, d["y"])
 
     def _moe(self, f, Fw, M: int, d: dict):
-        """Router + grouped experts; returns (per-slot outputs [M * S, W] fp32, S): the norm that follows sums them."""
+        """Router + grouped experts; returns (outputs [M * P, W] fp32, P parts per row): the norm that follows sums them."""
         tki = d["tki"][:M * f.top].view(M, f.top)
         tkw = d["tkw"][:M * f.top].view(M, f.top)
-        S = f.top + (1 if f.shared_ff else 0)
-        o = d["mo_o"][:M * S * self.cfg.width].view(M * S, self.cfg.width)
+        w = (Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown)
+        P = ops.moe_parts(d["xb"], f.top, *w, d["mo_h"])
+        o = d["mo_o"][:M * P * self.cfg.width].view(M * P, self.cfg.width)
         z = d["mo_z"][:M * f.experts].view(M, f.experts)
         ops.gemm_rm(d["xb"], Fw.router, z, bias=Fw.router_b)  # fp32 logits
         aligned = ops.moe_topk_lists(z, tki, tkw, d["mo_sorted"], d["mo_tile"], d["mo_n"], bool(f.shared_ff))
-        ops.moe_grouped(d["xb"], tki, tkw, Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown, d["mo_sorted"],
-                        d["mo_tile"], d["mo_n"], d["mo_h"], o, aligned=aligned)
-        return o, S
+        ops.moe_grouped(d["xb"], tki, tkw, *w, d["mo_sorted"], d["mo_tile"], d["mo_n"], d["mo_h"], o, aligned=aligned, parts=P)
+        return o, P
 
     def _layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None = None, prev=None) -> None:
         """Embedding + every layer over M packed rows.  `groups`: sequence groups of the step (decode slots, prompt
@@ -1132,7 +1132,7 @@ class LayeredRunner(RunnerBase):
                       "tkw": {f.top: torch.full((M * f.top,), 1.0 / f.top, **f32) for f in moe},
                       "mo_sorted": [torch.zeros(t * 64, **i32) for t in tiles],
                       "mo_tile": [torch.zeros(t, **i32) for t in tiles], "mo_n": [torch.zeros(1, **i32) for _ in moe],
-                      "mo_h": torch.empty(M * max(slots), ldh, **el), "mo_o": torch.empty(M * max(slots) * W, **f32)})
+                      "mo_h": torch.empty(M * max(slots), ldh, **el), "mo_o": torch.empty(M * (max(slots) + any(f.shared_ff for f in moe)) * W, **f32)})
         return d
 
     def _expert_lists(self, ids, M: int, d: dict) -> None:
@@ -1154,12 +1154,12 @@ class LayeredRunner(RunnerBase):
             self._lin(h, Fw.down, Fw.down_t, d["y"])
             return d["y"], 1
         n = self._moe_layers.index(layer)
-        S, W = f.top + (f.shared_ff > 0), self.cfg.width
+        W, w = self.cfg.width, (Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown)
+        P = ops.moe_parts(d["xb"], f.top, *w, d["mo_h"])
         tki, tkw = d["tki"][n][:M * f.top].view(M, f.top), d["tkw"][f.top][:M * f.top].view(M, f.top)
-        o = d["mo_o"][:M * S * W].view(M * S, W)
-        ops.moe_grouped(d["xb"], tki, tkw, Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown, d["mo_sorted"][n],
-                        d["mo_tile"][n], d["mo_n"][n], d["mo_h"], o, False, True)
-        return o, S
+        o = d["mo_o"][:M * P * W].view(M * P, W)
+        ops.moe_grouped(d["xb"], tki, tkw, *w, d["mo_sorted"][n], d["mo_tile"][n], d["mo_n"][n], d["mo_h"], o, False, True, P)
+        return o, P
 
     def _sink_rows(self, ri: int, a, qa, sink, gate, out, groups: list, out_scale: float = 1.0) -> None:
         """Causal sink attention of every sequence group over this run's pages: the shared-page MFMA form (wide heads: the
@@ -1271,7 +1271,7 @@ class LayeredRunner(RunnerBase):
             d.update({"tki": torch.zeros(M * slots, **i32), "tkw": torch.zeros(M * slots, **f32),
                       "mo_z": new(M * (experts + 1), **f32), "mo_sorted": torch.zeros(tiles * 64, **i32),
                       "mo_tile": torch.zeros(tiles, **i32), "mo_n": torch.zeros(2, **i32),
-                      "mo_h": torch.zeros(M * slots, ldh, **el), "mo_o": new(M * slots * W, **f32)})
+                      "mo_h": torch.zeros(M * slots, ldh, **el), "mo_o": new(M * (slots + any(f.shared_ff for f in moe)) * W, **f32)})
         return d
 
     def _joint_layers(self, M: int, d: dict, ids, pos, slots, groups: list, trace: list | None) -> None:
@@ -1334,12 +1334,14 @@ class LayeredRunner(RunnerBase):
     def _input_weighted_ff(self, f, Fw, M: int, d: dict):
         """Router GEMM in true fp32 on the fp32 normed row (the shared expert's gate is its last column) -> the largest
         sigmoid scores, used as they are (decode-sized steps: one launch that also lists the work) -> grouped gated-SiLU experts with the weights on their inputs, the shared expert
-        as one more slot with its gate on the output; returns (per-slot outputs [M * S, W] fp32, S)."""
+        as one more slot with its gate on the output; returns (outputs [M * P, W] fp32, P parts per row)."""
         shared = f.shared_ff > 0
         S, W, E = f.top + shared, self.cfg.width, f.experts + shared
         tki = d["tki"][:M * f.top].view(M, f.top)
         tkw = d["tkw"][:M * S].view(M, S)
-        o = d["mo_o"][:M * S * W].view(M * S, W)
+        w = (Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown)
+        P = ops.moe_parts(d["xb"], f.top, *w, d["mo_h"])
+        o = d["mo_o"][:M * P * W].view(M * P, W)
         lists = (d["mo_sorted"], d["mo_tile"], d["mo_n"])
         one_launch = M <= ops.layers.ROUTE_ROWS_MAX
         if one_launch:
@@ -1348,9 +1350,8 @@ class LayeredRunner(RunnerBase):
             z = d["mo_z"][:M * E].view(M, E)
             ops.gemm_rm(d["hn"], Fw.router, z)
             ops.moe_route(z, None, tki, tkw, 1, 1, 1.0, 2)
-        ops.moe_grouped(d["xb"], tki, tkw, Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown, *lists, d["mo_h"], o, True,
-                        one_launch)
-        return o, S
+        ops.moe_grouped(d["xb"], tki, tkw, *w, *lists, d["mo_h"], o, True, one_launch, P)
+        return o, P
 
     def _remember_last(self, seqs: list, g: dict) -> None:
         """After prompt portions: every portion's last token becomes its slot's previous token."""

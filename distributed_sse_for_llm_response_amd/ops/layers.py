@@ -158,18 +158,28 @@ def moe_ffn(x, topk_idx, topk_w, gate, up, down, sgate, sup, sdown, out):
 
 
 def moe_grouped(x, topk_idx, topk_w, gate, up, down, sgate, sup, sdown, sorted_ids, tile_expert, num_tiles, h, o,
-                weight_input: bool = False, aligned: bool = False):
+                weight_input: bool = False, aligned: bool = False, parts: int = 0):
     """Grouped form of the routed experts: rows sorted by expert, 16-row MFMA tiles of one expert each.  o [M · S, W]
     (fp32) = weight · expert output per (row, slot), S = top (+ 1: the shared expert's slot); the norm or stream step
     that follows sums them (nsum=S).  gate None: experts without a gate, down(relu(up x)^2).  topk_w may have a
     column more than topk_idx: the shared expert's weight per row (1 without it).  weight_input: a routed expert's weight
     multiplies its input instead of its output (the shared expert's always its output).  A row's chosen experts are
-    distinct.  sorted_ids / tile_expert / num_tiles / h are scratch; aligned: the first three are moe_route_rows'."""
+    distinct.  sorted_ids / tile_expert / num_tiles / h are scratch; aligned: the first three are moe_route_rows'.
+    parts (moe_parts; 0: S): the rows of o per row of x, S and one for every further slice of the shared expert's hidden
+    units, whose products add up to its output."""
     if _hip(x):
         torch.ops.dsse.moe_grouped(x, topk_idx, topk_w, gate, up, down, sgate, sup, sdown, sorted_ids, tile_expert,
-                                   num_tiles, h, o, weight_input, aligned)
+                                   num_tiles, h, o, weight_input, aligned, parts)
     else:
         lref.moe_grouped(x, topk_idx, topk_w, gate, up, down, sgate, sup, sdown, o, weight_input)
+
+
+def moe_parts(x, top: int, gate, up, down, sgate, sup, sdown, h) -> int:
+    """The parts per row that moe_grouped's output has in a step on these rows, weights and scratch: the slots, and one more
+    where the shared expert's down product is sooner done in two slices."""
+    if _hip(x):
+        return torch.ops.dsse.moe_parts(x, top, gate, up, down, sgate, sup, sdown, h)
+    return top + (sgate is not None)
 
 
 ROUTE_ROWS_MAX = 64  # steps of up to this many rows make router, choice and work list in one launch
