@@ -37,6 +37,7 @@ struct GemmEpi {
   // resets its pair); null when unused
   int* fix_cnt;
   int gelu;               // mode 3: the gate's activation is GELU (tanh form) instead of SiLU
+  int parts;              // S slices left for a consumer as the S parts of every row, [M, S, N] (0: as slabs [S, M, N])
 };
 constexpr int kFixTiles = 8192;  // tiles of one fix-up launch at most
 // the per-device counter block (bindings.cpp fix_state): [4 words][2 kFixTiles GEMM fix-up counters]

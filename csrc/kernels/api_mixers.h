@@ -13,7 +13,8 @@
 namespace dsse {
 
 struct StreamStepParams {
-  const float* y;        // [M, W] sublayer output or null
+  const float* y;        // [M * nsum, W] sublayer output or null
+  int nsum;              // a row's parts, summed first
   float mult;            // resid += mult * y
   float* resid;          // [M, W] fp32 stream
   const int* ids;        // [M] token ids (with embed)
@@ -196,7 +197,8 @@ struct AddNormParams {
   const float* y;        // [M * nsum, W] or null: resid += rms-norm(sum of the row's parts) * g_add
   int nsum;
   const float* g_add;    // [W] or null: the parts' sum is added as it is
-  const float* y2;       // [M, W] or null: added too (with g_add null)
+  const float* y2;       // [M * nsum2, W] or null: added too (with g_add null)
+  int nsum2;
   float* resid;          // [M, W] fp32
   const float* g_out;    // [W] or null: out = resid itself
   void* out;             // rows ldo apart (fp32 when out_f32, else bf16) or null
@@ -268,7 +270,8 @@ hipError_t dsse_scan_carry(const dsse::ScanCarryParams* p, hipStream_t st);
 // gate_kind 0: silu(gate), 1: sigmoid(gate)
 hipError_t dsse_gated_head_norm(const float* o, const float* w, const float* gate, int ldg, void* out, int M, int H,
                                 int V, float eps, int gate_kind, int f32, hipStream_t st);
-hipError_t dsse_rms_mix(const float* ya, const float* wa, const float* yb, const float* wb, float* out, int M, int W,
+// ya [M * na, W] and yb [M * nb, W]: a row's parts are summed first; out is ya itself only where na is 1
+hipError_t dsse_rms_mix(const float* ya, int na, const float* wa, const float* yb, int nb, const float* wb, float* out, int M, int W,
                         float eps, float coef, hipStream_t st);
 hipError_t dsse_logit_cap(float* logits, long long n, float scale, float cap, hipStream_t st);
 }

@@ -134,7 +134,7 @@ bool skinny_pairs(int M, int N) {
 // workgroups and K walks of at most two rounds.  Sliced / skinny, us: 2048 x 2048 17 rows 9.8 / 7.7, 32 rows 10.7 / 9.3, 48 rows 10.6 /
 // 11.9; 4096 x 2048 17 rows 10.8 / 8.1, 32 11.4 / 9.7; 2048 x 2560 32 rows 10.8 / 10.7; 2048 x 4096 24 rows 11.8 / 12.3; 2048 x 1024 64
 // rows 10.1 / 9.3; 6144 x 2048 24 rows 12.3 / 12.6.  K % 512 != 0 (a tensor-parallel shard's) stays with the ring kernel.
-// Not where the next kernel sums the slices (gemm_impl's slab_consumer): product and RMSNorm, sliced / skinny, 4096 x 2048 32 rows 11.9 /
+// Not where the next kernel sums the slices (gemm_impl's kSlabs): product and RMSNorm, sliced / skinny, 4096 x 2048 32 rows 11.9 /
 // 13.9, 2048 x 2048 9.8 / 12.8, 4096 x 1024 64 rows 11.5 / 16.4, 4096 x 512 32 rows 10.4 / 10.5; but 4096 x 2560 17 rows 14.6 / 13.1.
 bool skinny_whole(int M, int N, int K) {
   return gemm_rules_free() && M > 16 && N <= 4096 && K % 512 == 0 && (M <= 32 ? K <= 2560 : M <= 64 && K <= 1024);
@@ -326,7 +326,7 @@ struct TCfg {
 // reading S - 1 slots at ~26 GB/s (the stamps of profiles/r6/pipe_fix_stamps_r6.log), or left as slabs for the
 // next kernel (the norm or attention consumer, else splitk_reduce) that reads S x M x N x 4 bytes at ~4.5 TB/s
 // after ~5.7 us.  Constants least-squares fitted to 238 measured launches at 192-1024 rows (12 % rms error).
-double pipe_est_us(int M, int N, int K, int bm, int S, bool fix, int out_bytes = 0) {
+double pipe_est_us(int M, int N, int K, int bm, int S, bool fix, int out_bytes = 0, bool parts = false) {
   // kFixSync: the fit gave 7.06 us over isolated launches; 12 after the TP = 8 rank's prefill, where the fix-up GEMMs
   // (gate_up at 2048-row chunks, qkv at 8192 rows, model ties with slab forms) run beside the side stream's
   // collectives and lost 2 ms per 8k prompt to the slab forms (25.2 vs 23.3 ms, profiles/r6/tp8_fix_ab_r6.log); 12
@@ -341,15 +341,21 @@ double pipe_est_us(int M, int N, int K, int bm, int S, bool fix, int out_bytes =
   double t = full * t_wg + (rem ? t_wg * (kPartial + (1 - kPartial) * rem / kCUs) : 0.0);
   if (S > 1) {
     const double slot = (double)bm * 256 * 4;
-    t += fix ? kFixSync + (S - 1) * slot / kSlotRead : kNext + ((double)S * M * N * 4 + (double)M * N * out_bytes) / kHbm;
+    t += fix ? kFixSync + (S - 1) * slot / kSlotRead : parts ? 2.0 + (S - 1) * (double)M * N * 4 / 3.5e6 : kNext + ((double)S * M * N * 4 + (double)M * N * out_bytes) / kHbm;
   }
   return t;
 }
 
+// What becomes of a split product's fp32 slices: a reduction launch, slabs that the next kernel sums (Mistral's norms and attention), or
+// the parts of a row that a norm adds.  A norm that adds S parts takes 2 us and (S - 1) parts' bytes at 3.5 TB/s longer than with one (the
+// plan is within 0.1 % of the best of nine over 55 products of 300 to 4096 rows; at the slabs' price 2 %: 1500 x 2048 x 2048
+// 38.7 / 34.5 us, 2048 x 2048 x 2048 47.2 / 40.4).
+enum Slices { kReduced, kSlabs, kParts };
+
 // Best gemm_pipe configuration by the model: tile 256 / 192 / 128 rows x split 1-16, slices combined in the launch
-// (fix) or left as fp32 slabs -- for the caller's next kernel when `slab_consumer` (norm, attention), else for
+// (fix) or left as fp32 slabs -- for the caller's next kernel (kSlabs, kParts), else for
 // splitk_reduce (which also writes the bf16 output: counted).
-TCfg pipe_plan(int M, int N, int K, bool slab_consumer) {
+TCfg pipe_plan(int M, int N, int K, Slices to) {
   TCfg best{};
   best.ok = false;
   const bool no_fix = env_int("t_fix", -1) == 0;  // t_fix=0 (DSSE_KERNEL_CFG): slabs only, for A/Bs
@@ -361,7 +367,7 @@ TCfg pipe_plan(int M, int N, int K, bool slab_consumer) {
         if (S == 1 && fix) continue;
         if (fix && no_fix) continue;
         if (fix && (tiles > dsse::kFixTiles || (double)tiles * (S - 1) * bm * 256 * 4 > (1u << 30))) continue;
-        const double t = pipe_est_us(M, N, K, bm, S, fix, slab_consumer ? 0 : 2);
+        const double t = pipe_est_us(M, N, K, bm, S, fix, to == kReduced ? 2 : 0, to == kParts);
         if (!best.ok || t < best.est_us * 0.98) {  // ties: the simpler (earlier) form
           best.ok = true;
           best.est_us = t;
@@ -415,7 +421,7 @@ bool half_block_pays(int M, int N, int K, const TCfg& c) {
 //   26752 x 4096 55 / 52), and where the ring's slices end above one round (8320 x 2048 72 rows 21 / 23, 10240 x 4096 31 / 35, 128 rows 37 / 40).
 // Two slices where half the K walk is longer than their slabs and the reduction: 10240 x 4096 160 rows 38 / 49, 8320 x 2048 25 / 26,
 // 14464 x 2048 29 / 27, 16384 x 2048 31 / 28.
-TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
+TCfg rows_plan(int M, int N, int K, Slices to) {
   TCfg c{};
   c.ok = false;
   c.cfg = 2;
@@ -430,24 +436,24 @@ TCfg rows_plan(int M, int N, int K, bool slab_consumer) {
       c.ok = (blocks >= 224 && (M <= 96 || K < 4096)) || (r.ok && r.nw == 4 && N / 64 * r.S > 256);
     }
     c.S = blocks <= 128 && K >= 1024 && (double)K * (M + 128) > 61e3 * (4.0 + 3.2e-6 * M * N) ? 2 : 1;
-  } else if (M > 128 && M <= 192 && slab_consumer && N >= 4096 && K >= 4096 && (N > 7168 || K > 6144)) {
+  } else if (M > 128 && M <= 192 && to != kReduced && N >= 4096 && K >= 4096 && (N > 7168 || K > 6144)) {
     while (blocks * c.S * 2 <= 256 && K % (128 * c.S) == 0 && K / (c.S * 2) >= 512) c.S *= 2;
     c.ok = blocks * c.S >= 160;
   }
   return c;
 }
 
-TCfg pick_tiled(int M, int N, int K, bool slab_consumer = false) {
+TCfg pick_tiled(int M, int N, int K, Slices to = kReduced) {
   TCfg c{};
   int cfg = env_int("t_cfg", -1);
   const bool forced = cfg == 0 || cfg == 1 || cfg == 2 || cfg == 5 || cfg == 8 || cfg == 9 || cfg == 10;
   if (!forced) {
-    c = rows_plan(M, N, K, slab_consumer);
+    c = rows_plan(M, N, K, to);
     if (c.ok) return c;
     c = TCfg{};
   }
   if (!forced && env_int("t_model", 1) && N % 128 == 0 && K % 128 == 0 && M > kModelMinM) {
-    c = pipe_plan(M, N, K, slab_consumer);
+    c = pipe_plan(M, N, K, to);
     if (c.ok && (N % 256 == 0 || half_block_pays(M, N, K, c))) return c;
     c = TCfg{};
   }
@@ -522,8 +528,8 @@ void run_tiled(int mode, const TCfg& c, const Tensor& x, const Tensor& w, int M,
 // 0 = register-streaming (gemm_skinny.hip; tiny batches, X re-reads are cheap), 2 = X streamed through LDS
 // slices (gemm_stream.hip), 3 = gemm_wide.hip (32x32 MFMAs), 4 = gemm_tiled.hip (register-blocked, LDS-DMA).
 // gemm_impl (DSSE_KERNEL_CFG) forces one (1, the removed whole-slice X-in-LDS kernel, maps to the fallback).
-// slab_consumer: the next kernel sums split-K slabs, so a sliced product has no reduction launch to save.
-int gemm_impl(int M, int N, int K, bool slab_consumer = false) {
+// to: where the next kernel sums split-K slices, a sliced product has no reduction launch to save.
+int gemm_impl(int M, int N, int K, Slices to = kReduced) {
   const int impl = env_int("gemm_impl", -1);
   if (M > 64) {
     // every branch returns a kernel whose shape contract holds (or -1): prefill calls arrive with any M and
@@ -531,7 +537,7 @@ int gemm_impl(int M, int N, int K, bool slab_consumer = false) {
     // 65-128 rows, narrow N (4-wave stream shapes: qkv / o / down): the ring kernel with 8 row tiles, 3 slots;
     // 128-stream step 6.19 / 6.23 vs 6.36 / 6.37 ms on gemm_wide (profiles/r2/ring128_ab.log)
     if (impl < 0 && M <= 128) {
-      if (env_int("t_cfg", -1) < 0 && rows_plan(M, N, K, false).ok) return 4;
+      if (env_int("t_cfg", -1) < 0 && rows_plan(M, N, K, kReduced).ok) return 4;
       const SCfg sc = pick_stream(M, N, K);
       if (sc.ok && sc.mt == 8 && sc.nt == 1 && sc.nw == 4) return 2;
     }
@@ -557,7 +563,8 @@ int gemm_impl(int M, int N, int K, bool slab_consumer = false) {
   }
   if (M <= 8) return 0;
   if (M <= 16 && (N < 16384 || skinny_pairs(M, N))) return 0;
-  if (!slab_consumer && skinny_whole(M, N, K)) return 0;
+  // (17 rows of 2048 x 2048 and the norm that adds its parts: 10.8 us in one launch, 11.6 in slices, 32 rows 12.5 / 12.2)
+  if ((to == kReduced || (to == kParts && M < 32)) && skinny_whole(M, N, K)) return 0;
   return pick_stream(M, N, K).ok ? 2 : fallback;
 }
 
@@ -650,9 +657,9 @@ int64_t gemm_resid_split(const Tensor& x, const Tensor& w, Tensor& resid, Tensor
   check_dtype(part, at::kFloat, "part");
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = M >= 1 && K % 128 == 0 && N % 16 == 0 && w.size(1) == K;
-  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, kSlabs) : 0;
   if (impl == 4) {
-    const TCfg c = pick_tiled(M, N, K, true);
+    const TCfg c = pick_tiled(M, N, K, kSlabs);
     if (c.S > 1 && !c.fix && part.numel() >= (int64_t)c.S * M * N) {
       check_dtype(x, at::kBFloat16, "x");
       check_dtype(w, at::kBFloat16, "w");
@@ -702,7 +709,7 @@ int64_t gemm_out_split(const Tensor& x, const Tensor& w, Tensor& out, Tensor& pa
   check_dtype(part, at::kFloat, "part");
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = M >= 1 && K % 128 == 0 && N % 16 == 0 && w.size(1) == K;
-  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, kSlabs) : 0;
   dsse::GemmEpi ep{};
   if (impl == 2) {
     const SCfg c = pick_stream(M, N, K);
@@ -714,7 +721,7 @@ int64_t gemm_out_split(const Tensor& x, const Tensor& w, Tensor& out, Tensor& pa
       return c.S;
     }
   } else if (impl == 4) {
-    const TCfg c = pick_tiled(M, N, K, true);
+    const TCfg c = pick_tiled(M, N, K, kSlabs);
     if (c.S > 1 && !c.fix && part.numel() >= (int64_t)c.S * M * N) {
       check_dtype(x, at::kBFloat16, "x");
       check_dtype(w, at::kBFloat16, "w");
@@ -725,6 +732,49 @@ int64_t gemm_out_split(const Tensor& x, const Tensor& w, Tensor& out, Tensor& pa
   }
   gemm_out(x, w, out);
   return 0;
+}
+
+// fp32 projection for a consumer that adds the consecutive parts of a row (the grouped experts' norms, nsum): returns S and leaves the row's S
+// K slices, or the whole product (1), as [M, S, N] in `part`.
+int64_t gemm_out_parts(const Tensor& x, const Tensor& w, Tensor& part) {
+  check_gpu(x, "x");
+  check_gpu(w, "w");
+  check_gpu(part, "part");
+  check_dtype(x, at::kBFloat16, "x");
+  check_dtype(w, at::kBFloat16, "w");
+  check_dtype(part, at::kFloat, "part");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(0) >= 1, "x [M, K] and w [N, K]");
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  TORCH_CHECK(part.numel() >= (int64_t)M * N, "part must hold [M, N]");
+  dsse::GemmEpi ep{};
+  const bool shape_ok = K % 128 == 0 && N % 16 == 0 && w.size(1) == K && (int64_t)N * K * 2 < (1LL << 31);
+  const int impl = shape_ok ? gemm_impl(M, N, K, kParts) : 0;
+  auto fits = [&](int S) { ep.parts = S; return S > 1 && part.numel() >= (int64_t)S * M * N; };
+  if (impl == 4) {
+    const TCfg c = pick_tiled(M, N, K, kParts);
+    if (!c.fix && fits(c.S)) {
+      DSSE_CHECK_HIP(tiled_call(dsse::kStoreF32, c.cfg, c.S, 1, x.data_ptr(), K, M, w.data_ptr(), K, N, &ep, part.data_ptr<float>()));
+      return c.S;
+    }
+  } else if (impl == 3) {
+    const WCfg c = pick_wide(M, N, K);
+    if (fits(c.S)) {
+      DSSE_CHECK_HIP(dsse_gemm_wide(dsse::kStoreF32, c.mb, c.rd, c.S, 1, x.data_ptr(), K, M, w.data_ptr(), K, N, &ep, part.data_ptr<float>(),
+                                    cur_stream()));
+      return c.S;
+    }
+  } else if (impl == 2) {
+    const SCfg c = pick_stream(M, N, K);
+    if (fits(c.S)) {
+      DSSE_CHECK_HIP(stream_launch(dsse::kStoreF32, c, c.S, 1, x.data_ptr(), M, w.data_ptr(), K, N, &ep, part.data_ptr<float>()));
+      return c.S;
+    }
+  }
+  ep.parts = 0;
+  ep.out = part.data_ptr();
+  ep.ldo = N;
+  run_gemm(dsse::kStoreF32, x, w, ep);
+  return 1;
 }
 
 void gated_gemm(const Tensor& x, const Tensor& w, Tensor& out, bool gelu) {
@@ -1018,10 +1068,10 @@ int64_t qkv_attention_decode(const Tensor& x, const Tensor& w, const Tensor& pos
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const bool shape_ok = x.dim() == 2 && w.dim() == 2 && M >= 1 && K % 128 == 0 && w.size(1) == K &&
                         N == (nh + 2 * nkv) * 128;
-  const int impl = shape_ok ? gemm_impl(M, N, K, true) : 0;
+  const int impl = shape_ok ? gemm_impl(M, N, K, kSlabs) : 0;
   int S = 0;
   if (impl == 4) {
-    const TCfg c = pick_tiled(M, N, K, true);
+    const TCfg c = pick_tiled(M, N, K, kSlabs);
     S = c.fix ? 0 : c.S;  // combined in the launch: the unfused path (gemm_qkv_rope's FIX launch + attention)
   }
   else if (impl == 3) S = pick_wide(M, N, K).S;
@@ -1059,7 +1109,7 @@ int64_t qkv_attention_decode(const Tensor& x, const Tensor& w, const Tensor& pos
   const void* X = x.data_ptr();
   float* sl = slabs.data_ptr<float>();
   if (impl == 4) {
-    const TCfg c = pick_tiled(M, N, K, true);
+    const TCfg c = pick_tiled(M, N, K, kSlabs);
     DSSE_CHECK_HIP(tiled_call(dsse::kQkvRope, c.cfg, S, 1, X, K, M, w.data_ptr(), K, N, &ep, sl));
   } else if (impl == 3) {
     const WCfg c = pick_wide(M, N, K);
@@ -1276,9 +1326,9 @@ int64_t kernels_abi_version() { return 16; }
 // The dispatch's choice for an (M, N, K) projection: (impl, tiled cfg, split, fix, model estimate in us) -- impl as
 // gemm_impl (4 = tiled / pipe); cfg / split / fix / estimate only for impl 4 (tools/bench_decode_gemm.py --plan).
 std::tuple<int64_t, int64_t, int64_t, bool, double> gemm_plan(int64_t M, int64_t N, int64_t K, bool slab_consumer) {
-  const int impl = gemm_impl((int)M, (int)N, (int)K, slab_consumer);
+  const int impl = gemm_impl((int)M, (int)N, (int)K, slab_consumer ? kSlabs : kReduced);
   if (impl != 4) return {impl, -1, 0, false, 0.0};
-  const TCfg c = pick_tiled((int)M, (int)N, (int)K, slab_consumer);
+  const TCfg c = pick_tiled((int)M, (int)N, (int)K, slab_consumer ? kSlabs : kReduced);
   return {impl, c.cfg, c.S, c.fix, c.est_us};
 }
 
@@ -1378,6 +1428,7 @@ TORCH_LIBRARY(dsse, m) {
   m.def("rmsnorm(Tensor(a!) resid, Tensor w, Tensor(b!) y, float eps, Tensor? delta=None, Tensor? embed=None, "
         "Tensor? ids=None, Tensor? part=None, int nsplit=0) -> ()");
   m.def("gemm_resid_split(Tensor x, Tensor w, Tensor(a!) resid, Tensor(b!) part) -> int");
+  m.def("gemm_out_parts(Tensor x, Tensor w, Tensor(a!) part) -> int");
   m.def("gemm_out_split(Tensor x, Tensor w, Tensor(a!) out, Tensor(b!) part) -> int");
   m.def("refresh_env() -> ()", &refresh_env);
   m.def("rope_kv_write(Tensor qkv, Tensor positions, Tensor slots, Tensor rope, Tensor(a!) q_out, "
@@ -1424,6 +1475,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("gemm_out", &gemm_out);
   m.impl("gemm_resid", &gemm_resid);
   m.impl("gemm_resid_split", &gemm_resid_split);
+  m.impl("gemm_out_parts", &gemm_out_parts);
   m.impl("gemm_out_split", &gemm_out_split);
   m.impl("gemm_silu", &gemm_silu);
   m.impl("gemm_gelu", &gemm_gelu);

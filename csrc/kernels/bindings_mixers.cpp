@@ -73,7 +73,7 @@ void seq_meta(const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
 
 void stream_step(const OptTensor& y, double mult, Tensor& resid, const OptTensor& ids, const OptTensor& embed,
                  const OptTensor& vec, const OptTensor& alpha, const OptTensor& w, const OptTensor& b,
-                 const OptTensor& xb) {
+                 const OptTensor& xb, int64_t nsum) {
   f32t(resid, "resid");
   TORCH_CHECK(resid.dim() == 2, "resid must be [M, W]");
   dsse::StreamStepParams p{};
@@ -83,8 +83,9 @@ void stream_step(const OptTensor& y, double mult, Tensor& resid, const OptTensor
   p.f32 = 1;
   if (y.has_value()) {
     f32t(*y, "y");
-    TORCH_CHECK(y->sizes() == resid.sizes(), "y must match resid");
+    TORCH_CHECK(nsum >= 1 && y->dim() == 2 && y->size(0) == resid.size(0) * nsum && y->size(1) == resid.size(1), "y must be [M * nsum, W] like resid");
     p.y = y->data_ptr<float>();
+    p.nsum = (int)nsum;
   }
   if (embed.has_value()) {
     TORCH_CHECK(ids.has_value(), "embed needs ids");
@@ -577,16 +578,24 @@ void gated_head_norm(const Tensor& o, const OptTensor& w, const Tensor& gate, do
                                       cur_stream()));
 }
 
-void rms_mix(const Tensor& ya, const Tensor& wa, const Tensor& yb, const Tensor& wb, double eps, double coef, Tensor& out) {
+void rms_mix(const Tensor& ya, const Tensor& wa, const Tensor& yb, const Tensor& wb, double eps, double coef, Tensor& out, int64_t na,
+             int64_t nb) {
   f32t(ya, "ya");
   f32t(yb, "yb");
   f32t(out, "out");
-  TORCH_CHECK(ya.dim() == 2 && yb.sizes() == ya.sizes() && out.sizes() == ya.sizes(), "ya, yb, out must be [M, W]");
-  const int M = (int)ya.size(0), W = (int)ya.size(1);
+  TORCH_CHECK(out.dim() == 2 && na >= 1 && nb >= 1, "out must be [M, W]");
+  const int M = (int)out.size(0), W = (int)out.size(1);
+  TORCH_CHECK(ya.dim() == 2 && yb.dim() == 2 && ya.size(0) == M * na && yb.size(0) == M * nb && ya.size(1) == W && yb.size(1) == W,
+              "ya must be [M * na, W], yb [M * nb, W]");
+  auto apart = [&](const Tensor& y) {  // a row's sum is written where other rows' parts lie
+    const char *a = (const char*)y.data_ptr(), *b = (const char*)out.data_ptr();
+    return a + y.nbytes() <= b || b + out.nbytes() <= a;
+  };
+  TORCH_CHECK((na == 1 || apart(ya)) && (nb == 1 || apart(yb)), "rms_mix: out shares memory with rows of several parts");
   f32t(wa, "wa");
   f32t(wb, "wb");
   TORCH_CHECK(wa.numel() == W && wb.numel() == W, "gains must be [W]");
-  DSSE_CHECK_HIP(dsse_rms_mix(ya.data_ptr<float>(), wa.data_ptr<float>(), yb.data_ptr<float>(), wb.data_ptr<float>(),
+  DSSE_CHECK_HIP(dsse_rms_mix(ya.data_ptr<float>(), (int)na, wa.data_ptr<float>(), yb.data_ptr<float>(), (int)nb, wb.data_ptr<float>(),
                               out.data_ptr<float>(), M, W, (float)eps, (float)coef, cur_stream()));
 }
 
@@ -748,7 +757,7 @@ void embed_pair_rows(const Tensor& ids, const OptTensor& prev, const Tensor& pos
 }
 
 void add_norm_rows(const OptTensor& y, int64_t nsum, const OptTensor& g_add, Tensor& resid, const OptTensor& g_out,
-                   double eps, const OptTensor& out, const OptTensor& out32, const OptTensor& y2) {
+                   double eps, const OptTensor& out, const OptTensor& out32, const OptTensor& y2, int64_t nsum2) {
   f32t(resid, "resid");
   TORCH_CHECK(resid.dim() == 2 && nsum >= 1, "resid [M, W], nsum >= 1");
   dsse::AddNormParams p{};
@@ -763,7 +772,9 @@ void add_norm_rows(const OptTensor& y, int64_t nsum, const OptTensor& g_add, Ten
   }
   if (y2.has_value()) {
     TORCH_CHECK(p.y && !p.g_add, "y2 is added beside a y that has no norm");
-    p.y2 = opt_f32(y2, "y2", (int64_t)p.M * p.W);
+    TORCH_CHECK(nsum2 >= 1, "nsum2 >= 1");
+    p.nsum2 = (int)nsum2;
+    p.y2 = opt_f32(y2, "y2", (int64_t)p.M * nsum2 * p.W);
   }
   p.g_out = opt_f32(g_out, "g_out", p.W);
   if (out.has_value()) {
@@ -911,10 +922,10 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("embed_pair_rows(Tensor ids, Tensor? prev, Tensor positions, Tensor embed, Tensor? pair, int mul_prev, "
         "int mul_cur, int buckets, Tensor(a!) resid, Tensor(b!)? x0, Tensor(c!)? prev_out, Tensor? keep) -> ()");
   m.def("add_norm_rows(Tensor? y, int nsum, Tensor? g_add, Tensor(a!) resid, Tensor? g_out, float eps, "
-        "Tensor(b!)? out, Tensor(c!)? out32, Tensor? y2=None) -> ()");
+        "Tensor(b!)? out, Tensor(c!)? out32, Tensor? y2=None, int nsum2=1) -> ()");
   m.def("token_gate_rows(Tensor x, Tensor ids, Tensor table, int col0, Tensor(a!) out) -> ()");
   m.def("stream_step(Tensor? y, float mult, Tensor(a!) resid, Tensor? ids, Tensor? embed, Tensor? vec, Tensor? alpha, "
-        "Tensor? w, Tensor? b, Tensor(b!)? xb) -> ()");
+        "Tensor? w, Tensor? b, Tensor(b!)? xb, int nsum=1) -> ()");
   m.def("gated_act(Tensor gu, Tensor(a!) h, int kind=1) -> ()");
   m.def("norm_rope_list(Tensor[] x, Tensor?[] norm_w, Tensor positions, Tensor?[] rope, Tensor(a!)[] out, Tensor?[] out_rows, "
         "int[] kind, float[] eps, float[] scale, Tensor(b!)?[] out_t) -> ()");
@@ -936,7 +947,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor state_slot, Tensor s_first, Tensor s_count, Tensor cmeta, Tensor(b!) scratch, Tensor(c!)? a_scratch, "
         "Tensor(d!) out, float q_scale=1.0) -> ()");
   m.def("gated_head_norm(Tensor o, Tensor? w, Tensor gate, float eps, Tensor(a!) out, int kind=0) -> ()");
-  m.def("rms_mix(Tensor ya, Tensor wa, Tensor yb, Tensor wb, float eps, float coef, Tensor(a!) out) -> ()");
+  m.def("rms_mix(Tensor ya, Tensor wa, Tensor yb, Tensor wb, float eps, float coef, Tensor(a!) out, int na=1, int nb=1) -> ()");
   m.def("logit_cap(Tensor(a!) logits, float scale, float cap) -> ()");
 }
 

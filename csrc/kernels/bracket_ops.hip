@@ -64,6 +64,10 @@ constexpr int kNormRegs = 8;  // vectors of VEC floats a thread keeps of its row
 template <int VEC>
 struct FVec {
   float v[VEC];
+  DEV void operator+=(const FVec& o) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) v[e] += o.v[e];
+  }
 };
 template <int VEC>
 DEV FVec<VEC> ld_f(const float* p) {
@@ -110,24 +114,14 @@ __global__ __launch_bounds__(256) void add_norm_rows_kernel(AddNormParams p) {
     }
   };
   auto parts = [&](int d) {  // the row's parts of y summed
-    FVec<VEC> v = ld_f<VEC>(y + d);
-    for (int s = 1; s < p.nsum; ++s) {
-      const FVec<VEC> t = ld_f<VEC>(y + (int64_t)s * W + d);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) v.v[e] += t.v[e];
-    }
-    return v;
+    return add_parts<FVec<VEC>>(p.nsum, [&](int s) { return ld_f<VEC>(y + (int64_t)s * W + d); });
   };
   float ss = 0.f;
   if (y && !p.g_add) {  // sublayers whose outputs are added as they are
-    const float* y2 = p.y2 ? p.y2 + row * W : nullptr;
+    const float* y2 = p.y2 ? p.y2 + row * p.nsum2 * W : nullptr;
     each([&](int i, int d) {
       FVec<VEC> v = parts(d);
-      if (y2) {
-        const FVec<VEC> t = ld_f<VEC>(y2 + d);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) v.v[e] += t.v[e];
-      }
+      if (y2) v += add_parts<FVec<VEC>>(p.nsum2, [&](int s) { return ld_f<VEC>(y2 + (int64_t)s * W + d); });
       FVec<VEC> r = ld_f<VEC>(resid + d);
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
@@ -371,7 +365,7 @@ extern "C" hipError_t dsse_embed_pair_rows(const dsse::EmbedPairParams* p, hipSt
 
 extern "C" hipError_t dsse_add_norm_rows(const dsse::AddNormParams* p, hipStream_t st) {
   if (p->M <= 0) return hipSuccess;
-  if (p->nsum < 1 || (p->y2 && (!p->y || p->g_add))) return hipErrorInvalidValue;
+  if (p->nsum < 1 || (p->y2 && (!p->y || p->g_add || p->nsum2 < 1))) return hipErrorInvalidValue;
   if (p->out_f32) dsse::launch_add_norm<float>(*p, st);
   else dsse::launch_add_norm<bf16>(*p, st);
   return hipGetLastError();

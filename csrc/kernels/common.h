@@ -127,6 +127,22 @@ inline bool fours(std::initializer_list<const void*> ps) {
     if (reinterpret_cast<uintptr_t>(p) % 16) return false;
   return true;
 }
+// The n parts of a value added in order, up to four of them requested together (one after another they are a chain of
+// memory latencies: 64 rows of 2048 in 8 parts)
+template <typename V, typename L>
+DEV V add_parts(int n, L load) {
+  V v = load(0);
+  for (int s = 1; s < n; s += 4) {
+    V t[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (s + k < n) t[k] = load(s + k);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (s + k < n) v += t[k];
+  }
+  return v;
+}
 // host: threads of a workgroup that keeps a row of W <= 16384 floats (W % 4 == 0) in registers, at most four groups of four per
 // thread: as many as the row has groups while the rows leave CUs empty, 256 where they do not
 inline int row_threads(int M, int W) {

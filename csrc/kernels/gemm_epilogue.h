@@ -6,7 +6,10 @@
 
 namespace dsse {
 
-constexpr int kPartial = 5;  // internal mode: write fp32 split-K partial slabs part[ks, m, n]
+constexpr int kPartial = 5;  // internal mode: write fp32 split-K partial slabs part[ks, m, n], or part[m, ks, n] (GemmEpi::parts)
+DEV float* partial_of(const GemmEpi& ep, float* part, int ks, int M, int N) {
+  return part ? part + (size_t)ks * (ep.parts ? 1 : M) * N : nullptr;
+}
 
 DEV int vperm_tok(int off) { return ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4 + (off & 3); }
 
@@ -55,7 +58,7 @@ DEV void epilogue(const GemmEpi& ep, float* part, int M, int N, int m, int tile,
       }
     }
   } else {  // kPartial
-    part[(size_t)m * N + n] = v;
+    part[(size_t)m * (ep.parts ? ep.parts * N : N) + n] = v;
   }
 }
 

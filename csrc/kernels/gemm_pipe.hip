@@ -374,7 +374,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     if constexpr (FIX) stamp(ep, 5, now());
     return;
   }
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt) {
     if ((mt & 3) >= QI) continue;

@@ -214,7 +214,7 @@ gemm_stream_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __res
 
   if (TOUCH && M < 0) part[touch & 1] = (float)touch;  // never runs: keeps the warm-up loads
 
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
   if constexpr (MODE == kSiluMul) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -464,7 +464,7 @@ gemm_ring_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     }
   }
 
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
   if constexpr (MODE == kSiluMul) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) silu_epilogue4(ep, M, 16 * mt + 4 * g, tgi, r, acc[mt]);
@@ -660,7 +660,7 @@ gemm_ring2_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
   if constexpr (MODE == kSiluMul) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) silu_epilogue4(ep, M, 16 * mt + 4 * g, tgi, r, acc[mt]);

@@ -227,7 +227,7 @@ gemm_tiled_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __rest
     }
   }
 
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
   const int row0 = m0 + wm * MT * 16, tile0 = n0 / 16 + wn * NT;
   if constexpr (MODE == kSiluMul) {
 #pragma unroll

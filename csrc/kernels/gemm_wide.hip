@@ -144,7 +144,7 @@ gemm_wide_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     }
   }
 
-  float* part_ks = part ? part + (size_t)ks * M * N : nullptr;
+  float* part_ks = partial_of(ep, part, ks, M, N);
   const int tile = 2 * strip + (n32 >> 4), r = n32 & 15;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)

@@ -63,15 +63,9 @@ __global__ __launch_bounds__(1024) void scalar_norm_vec_kernel(ScalarNormParams 
     const int d = 4 * (threadIdx.x + n * blockDim.x);
     y[n] = u[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (d >= p.W) continue;
-    y[n] = ld4(src + d);
     if (p.mode == 0) u[n] = ld4(resid + d);
+    y[n] = add_parts<f32x4>(ns, [&](int s) { return ld4(src + (int64_t)s * p.W + d); });
   }
-  for (int s = 1; s < ns; ++s)
-#pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const int d = 4 * (threadIdx.x + n * blockDim.x);
-      if (d < p.W) y[n] += ld4(src + (int64_t)s * p.W + d);
-    }
   float ss = 0.f;
 #pragma unroll
   for (int n = 0; n < NV; ++n)

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void stream_step_kernel(StreamStepParams p) {
   const int row = blockIdx.x, d = (blockIdx.y * 256 + threadIdx.x) * VEC;
   if (d >= p.W) return;
   float* resid = p.resid + (int64_t)row * p.W + d;
-  const float* y = p.y ? p.y + (int64_t)row * p.W + d : nullptr;
+  const float* y = p.y ? p.y + (int64_t)row * p.nsum * p.W + d : nullptr;
   const T* e = nullptr;
   if (p.embed) {
     int id = p.ids[row];
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void stream_step_kernel(StreamStepParams p) {
   }
   if constexpr (VEC == 4) {
     f32x4 v = ld4(resid);
-    if (y) v += p.mult * ld4(y);
+    if (y) v += p.mult * add_parts<f32x4>(p.nsum, [&](int s) { return ld4(y + (int64_t)s * p.W); });
     if (e) v += ld4(e);
     if (p.vec) v += ld4(p.vec + d);
     if (y || e || p.vec) st4(resid, v);
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void stream_step_kernel(StreamStepParams p) {
     }
   } else {
     float v = *resid;
-    if (y) v += p.mult * *y;
+    if (y) v += p.mult * add_parts<float>(p.nsum, [&](int s) { return y[(int64_t)s * p.W]; });
     if (e) v += (float)*e;
     if (p.vec) v += p.vec[d];
     if (y || e || p.vec) *resid = v;
@@ -200,27 +200,28 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* o, co
   for (int i = lane; i < V; i += 64) dst[i] = (T)(oh[i] * inv * (w ? w[i] : 1.0f) * (gate_kind == 1 ? sigmoid_f(g[i]) : silu_f(g[i])));
 }
 
-__global__ __launch_bounds__(256) void rms_mix_kernel(const float* ya, const float* wa, const float* yb, const float* wb,
+__global__ __launch_bounds__(256) void rms_mix_kernel(const float* ya, int na, const float* wa, const float* yb, int nb, const float* wb,
                                                       float* out, int W, float eps, float coef) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
-  const float* a = ya + row * W;
-  const float* b = yb + row * W;
+  auto a = [&](int d) { return add_parts<float>(na, [&](int s) { return ya[(row * na + s) * W + d]; }); };
+  auto b = [&](int d) { return add_parts<float>(nb, [&](int s) { return yb[(row * nb + s) * W + d]; }); };
   float sa = 0.f, sb = 0.f;
   for (int d = threadIdx.x; d < W; d += blockDim.x) {
-    sa += a[d] * a[d];
-    sb += b[d] * b[d];
+    const float u = a(d), v = b(d);
+    sa += u * u;
+    sb += v * v;
   }
   sa = block_sum256(sa, red);
   sb = block_sum256(sb, red);
   const float ia = 1.0f / sqrtf(sa / (float)W + eps), ib = 1.0f / sqrtf(sb / (float)W + eps);
-  for (int d = threadIdx.x; d < W; d += blockDim.x) out[row * W + d] = coef * (a[d] * ia * wa[d] + b[d] * ib * wb[d]);
+  for (int d = threadIdx.x; d < W; d += blockDim.x) out[row * W + d] = coef * (a(d) * ia * wa[d] + b(d) * ib * wb[d]);
 }
 
 // The same with a row's values in registers, NV groups of four per thread: one read of each row, a decode step's row on up to
 // 1024 threads (16 rows of 4096: 6.9 -> 3.2 us, 3000 rows 39 -> 23)
 template <int NV>
-__global__ __launch_bounds__(1024) void rms_mix_vec_kernel(const float* ya, const float* wa, const float* yb, const float* wb,
+__global__ __launch_bounds__(1024) void rms_mix_vec_kernel(const float* ya, int na, const float* wa, const float* yb, int nb, const float* wb,
                                                            float* out, int W, float eps, float coef) {
   __shared__ float red[2][16];
   const int64_t row = blockIdx.x;
@@ -230,7 +231,10 @@ __global__ __launch_bounds__(1024) void rms_mix_vec_kernel(const float* ya, cons
   for (int n = 0; n < NV; ++n) {
     const int d = 4 * (threadIdx.x + n * blockDim.x);
     a[n] = b[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (d < W) a[n] = ld4(ya + row * W + d), b[n] = ld4(yb + row * W + d);
+    if (d < W) {
+      a[n] = add_parts<f32x4>(na, [&](int s) { return ld4(ya + (row * na + s) * W + d); });
+      b[n] = add_parts<f32x4>(nb, [&](int s) { return ld4(yb + (row * nb + s) * W + d); });
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) sa += a[n][i] * a[n][i], sb += b[n][i] * b[n][i];
   }
@@ -270,6 +274,7 @@ inline int flat_blocks(int64_t n) {
 
 extern "C" hipError_t dsse_stream_step(const dsse::StreamStepParams* p, hipStream_t st) {
   if (p->M <= 0) return hipSuccess;
+  if (p->y && p->nsum < 1) return hipErrorInvalidValue;
   const bool vec = p->W % 4 == 0 && dsse::fours({p->resid, p->y, p->embed, p->vec, p->w, p->b, p->xb});
   const dim3 grid(p->M, (p->W + (vec ? 1023 : 255)) / (vec ? 1024 : 256));
   if (p->f32 && vec) hipLaunchKernelGGL((dsse::stream_step_kernel<float, 4>), grid, dim3(256), 0, st, *p);
@@ -343,19 +348,20 @@ extern "C" hipError_t dsse_gated_head_norm(const float* o, const float* w, const
   return hipGetLastError();
 }
 
-extern "C" hipError_t dsse_rms_mix(const float* ya, const float* wa, const float* yb, const float* wb, float* out, int M,
+extern "C" hipError_t dsse_rms_mix(const float* ya, int na, const float* wa, const float* yb, int nb, const float* wb, float* out, int M,
                                    int W, float eps, float coef, hipStream_t st) {
   if (M <= 0) return hipSuccess;
+  if (na < 1 || nb < 1) return hipErrorInvalidValue;
   if (W % 4 == 0 && W <= 16384 && dsse::fours({ya, wa, yb, wb, out})) {
     const int threads = dsse::row_threads(M, W), nv = (W / 4 + threads - 1) / threads;
-#define DSSE_MIX(n) hipLaunchKernelGGL(dsse::rms_mix_vec_kernel<n>, dim3(M), dim3(threads), 0, st, ya, wa, yb, wb, out, W, eps, coef)
+#define DSSE_MIX(n) hipLaunchKernelGGL(dsse::rms_mix_vec_kernel<n>, dim3(M), dim3(threads), 0, st, ya, na, wa, yb, nb, wb, out, W, eps, coef)
     if (nv <= 1) DSSE_MIX(1);
     else if (nv <= 2) DSSE_MIX(2);
     else DSSE_MIX(4);
 #undef DSSE_MIX
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(dsse::rms_mix_kernel, dim3(M), dim3(256), 0, st, ya, wa, yb, wb, out, W, eps, coef);
+  hipLaunchKernelGGL(dsse::rms_mix_kernel, dim3(M), dim3(256), 0, st, ya, na, wa, yb, nb, wb, out, W, eps, coef);
   return hipGetLastError();
 }
 

@@ -256,7 +256,7 @@ class LayeredRunner(RunnerBase):
         f32 = dict(device=dev, dtype=torch.float32)
         el = dict(device=dev, dtype=self.dtype)
         W = cfg.width
-        d = {"resid": new(M, W, **f32), "xb": new(M, W, **el), "y": new(M, W, **f32)}
+        d = {"resid": new(M, W, **f32), "xb": new(M, W, **el), "y": new(self._part_rows(M) * W, **f32)}
         if self.joint:
             d.update(self._joint_buffers(M, new))
             return d
@@ -301,7 +301,23 @@ class LayeredRunner(RunnerBase):
             d["mo_o"] = new(M * (slots + any(f.shared_ff for f in moe)) * W, **f32)  # a shared expert may come in two parts
         return d
 
+    @staticmethod
+    def _part_rows(M: int) -> int:
+        """Rows of a sublayer's output that the norm after it sums: K slices of its product are parts of every row (up to 16
+        in a step of a few hundred rows, two where the row tiles fill the chip by themselves)."""
+        return M * max(2, min(16, -(-8192 // M)))
+
     # ------------------------------------------------------------------ layers
+    def _out(self, x, w, wt, y):
+        """A sublayer's output projection into the flat buffer y, for a norm that sums a row's parts: (rows, parts)."""
+        M, N = x.shape[0], w.shape[0] if wt is None else wt.shape[0]
+        S = 1
+        if wt is not None:
+            S = ops.gemm_out_parts(x, wt, y)
+        else:
+            ops.gemm_rm(x, w, y[:M * N].view(M, N))
+        return y[:M * S * N].view(M * S, N), S
+
     @staticmethod
     def _lin(x, w, wt, out) -> None:
         """out = x · Wᵀ: the engine's tiled-layout GEMMs when the projection was tiled at load (model-sized, aligned
@@ -311,7 +327,7 @@ class LayeredRunner(RunnerBase):
         else:
             ops.gemm_rm(x, w, out)
 
-    def _attention(self, li: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _attention(self, li: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         H, dn, dr, rk, dv = m.heads, m.dim, m.rot_dim, m.kv_rank, m.vdim
         rope = self._rope[(m.rot, m.rot_dim)]
         cache = self.kv[li]
@@ -341,7 +357,7 @@ class LayeredRunner(RunnerBase):
                 ops.latent_attention(q, qabs, cache, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], rope, lat,
                                      m.window, m.scale, g["qt"])
         ops.gemm_rm(lat.permute(1, 0, 2), Lw.uv, attn.permute(1, 0, 2))
-        self._lin(attn.view(M, H * dv), Lw.o, Lw.o_t, d["y"])
+        return self._out(attn.view(M, H * dv), Lw.o, Lw.o_t, d["y"])
 
     def _decode_parts(self, B: int, heads: int, window: int) -> int:
         """Key partitions of the decode attention: enough (item, head tile, partition) waves for the chip, at most one
@@ -350,7 +366,7 @@ class LayeredRunner(RunnerBase):
         want = -(-FLASH_DECODE_WAVES // max(1, B * (-(-heads // 16))))
         return max(1, min(16, pages, want))
 
-    def _recurrent(self, li: int, m, Lw, M: int, d: dict, groups: list) -> None:
+    def _recurrent(self, li: int, m, Lw, M: int, d: dict, groups: list):
         C, nb = m.width, m.blocks
         bw = C // nb
         ub, hs = (d[k][:M * C].view(M, C) for k in ("ub", "hs"))
@@ -372,7 +388,7 @@ class LayeredRunner(RunnerBase):
             ops.lru_scan(u, gates, yr, Lw.lam, self.state.state[li], g["qs"], g["ql"], g["ctx"], g["ss"], hs,
                          LRU_DECAY_SCALE, Lw.y_b, i == 0, scr, len(groups) == 1,
                          1 if g["qt"] == 1 else g["longest"])
-        self._lin(hs, Lw.o, Lw.o_t, d["y"])
+        return self._out(hs, Lw.o, Lw.o_t, d["y"])
 
     def _moe(self, f, Fw, M: int, d: dict):
         """Router + grouped experts; returns (outputs [M * P, W] fp32, P parts per row): the norm that follows sums them."""
@@ -409,10 +425,10 @@ class LayeredRunner(RunnerBase):
             return
         for li, (L, Lw) in enumerate(zip(cfg.layers, self.w.layers)):
             if L.kind == "latent_attention":
-                self._attention(li, L.mixer, Lw.mix, M, d, pos, slots, groups)
+                y, S = self._attention(li, L.mixer, Lw.mix, M, d, pos, slots, groups)
             else:
-                self._recurrent(li, L.mixer, Lw.mix, M, d, groups)
-            ops.scalar_norm(d["y"], Lw.norm1, d["resid"], d["xb"], eps)
+                y, S = self._recurrent(li, L.mixer, Lw.mix, M, d, groups)
+            ops.scalar_norm(y, Lw.norm1, d["resid"], d["xb"], eps, S)
             if L.mlp is not None:
                 o, S = self._moe(L.mlp, Lw.mlp, M, d)
                 ops.scalar_norm(o, Lw.norm2, d["resid"], d["xb"], eps, S)
@@ -468,7 +484,8 @@ class LayeredRunner(RunnerBase):
             if L.mlp is not None:
                 ff = max(ff, L.mlp.ff)
                 gu = max(gu, 0 if self.w.layers[i].mlp.gu is None else 2 * L.mlp.ff)
-        return {"y2": new(M, cfg.width, **f32), "big": new(M * big, **f32),
+        y2 = {"y2": new(self._part_rows(M) * cfg.width, **f32), "ym": new(M, cfg.width, **f32)} if any(L.kind == "parallel" for L in cfg.layers) else {}
+        return {**y2, "big": new(M * big, **f32),
                 "cv": new(M * cv, **f32), "z": new(M * z, **f32),
                 "qa": new(M * qa, **f32), "o": new(M * o, **f32), "ao": new(M * o, **el),
                 "gu": new(M * gu, **f32), "h": new(M * ff, **el)}
@@ -479,27 +496,26 @@ class LayeredRunner(RunnerBase):
         vector) and applies the next sublayer's norm; the last output is added before the head's norm."""
         cfg, w = self.cfg, self.w
         mult = cfg.residual_mult
-        pending = None
+        y, S = None, 1  # the sublayer output that is not in the stream yet and its parts per row
         for run in self.runs:
             L, Lw = cfg.layers[run.layer], w.layers[run.layer]
             t = run.pass_no
             n = Lw.norm1
-            ops.stream_step(pending, mult, d["resid"], ids if t > 0 else None, w.embed if t > 0 else None,
-                            w.step[t] if t >= 0 else None, n.alpha, n.w, n.b, d["xb"])
-            getattr(self, "_" + L.kind)(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups)
+            ops.stream_step(y, mult, d["resid"], ids if t > 0 else None, w.embed if t > 0 else None,
+                            w.step[t] if t >= 0 else None, n.alpha, n.w, n.b, d["xb"], S)
+            y, S = getattr(self, "_" + L.kind)(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups)
             if L.mlp is not None:
                 n = Lw.norm2
-                ops.stream_step(d["y"], mult, d["resid"], None, None, None, n.alpha, n.w, n.b, d["xb"])
-                self._dense_ff(L.mlp, Lw.mlp, M, d)
-            pending = d["y"]
+                ops.stream_step(y, mult, d["resid"], None, None, None, n.alpha, n.w, n.b, d["xb"], S)
+                y, S = self._dense_ff(L.mlp, Lw.mlp, M, d)
             if trace is not None:
-                ops.stream_step(pending, mult, d["resid"], None, None, None, None, None, None, None)
-                pending = None
+                ops.stream_step(y, mult, d["resid"], None, None, None, None, None, None, None, S)
+                y, S = None, 1
                 trace.append(d["resid"].clone())
-        if pending is not None:
-            ops.stream_step(pending, mult, d["resid"], None, None, None, None, None, None, None)
+        if y is not None:
+            ops.stream_step(y, mult, d["resid"], None, None, None, None, None, None, None, S)
 
-    def _dense_ff(self, f, Fw, M: int, d: dict) -> None:
+    def _dense_ff(self, f, Fw, M: int, d: dict):
         h = d["h"][:M * f.ff].view(M, f.ff)
         if Fw.gu_t is not None:
             ops.gemm_gelu(d["xb"], Fw.gu_t, h)
@@ -507,7 +523,7 @@ class LayeredRunner(RunnerBase):
             gu = d["gu"][:M * 2 * f.ff].view(M, 2 * f.ff)
             ops.gemm_rm(d["xb"], Fw.gu, gu)
             ops.gated_act(gu, h, 1)
-        self._lin(h, Fw.down, Fw.down_t, d["y"])
+        return self._out(h, Fw.down, Fw.down_t, d["y"])
 
     def _scratch(self, d: dict, name: str, numel: int):
         """An fp32 work area of the step, grown on demand and shared by its layers."""
@@ -526,8 +542,8 @@ class LayeredRunner(RunnerBase):
         return self._cols(buf, c0, H, D), self._cols(buf, c0 + H * D, H, D), self._cols(buf, c0 + 2 * H * D, H, V)
 
     def _scan_out(self, ri: int, Lw_norm, gate, H: int, V: int, M: int, d: dict, q, k, v, decay, beta, groups, q_scale,
-                  o_w, o_t, y) -> None:
-        """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection."""
+                  o_w, o_t, y):
+        """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection (_out)."""
         o = d["o"][:M * H * V].view(M, H, V)
         for g in groups:
             D, chan = k.shape[2], decay is not None and decay.dim() == 3
@@ -542,7 +558,7 @@ class LayeredRunner(RunnerBase):
                                 q_scale, g.get("longest", 0))
         ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw_norm, gate, self.cfg.eps, ao)
-        self._lin(ao, o_w, o_t, y)
+        return self._out(ao, o_w, o_t, y)
 
     @staticmethod
     def _two_levels(g: dict, q, k, v, channels) -> bool:
@@ -562,7 +578,7 @@ class LayeredRunner(RunnerBase):
             g["ck"] = (ck[0], ck[1], cm)
         return g["ck"]
 
-    def _delta(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _delta(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         H, G, D, V = m.heads, m.kv_heads, m.dim, m.vdim
         C = 2 * G * D + H * V
         big = d["big"][:M * Lw.n_big].view(M, Lw.n_big)
@@ -575,10 +591,10 @@ class LayeredRunner(RunnerBase):
         q, k, v = self._cols(cv, 0, G, D), self._cols(cv, G * D, G, D), self._cols(cv, 2 * G * D, H, V)
         ops.norm_rope_list(pos, (q, None, None, q, None, 2, UNIT_EPS, D ** -0.5, None), (k, None, None, k, None, 2, UNIT_EPS, 1.0, None))
         ops.gate_pair(small, Lw.a_log, Lw.dt_bias)
-        self._scan_out(ri, Lw.norm, big[:, C:C + H * V], H, V, M, d, q, k, v, small[:, :H], small[:, H:], groups, 1.0,
-                       Lw.o, Lw.o_t, d["y"])
+        return self._scan_out(ri, Lw.norm, big[:, C:C + H * V], H, V, M, d, q, k, v, small[:, :H], small[:, H:], groups, 1.0,
+                              Lw.o, Lw.o_t, d["y"])
 
-    def _parallel(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _parallel(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         a, r = m.left, m.right
         H, G, D, V = a.heads, a.kv_heads, a.dim, a.vdim
         Hr, Dr, Vr = r.heads, r.dim, r.vdim
@@ -609,7 +625,7 @@ class LayeredRunner(RunnerBase):
             else:
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
                                    g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, g["qt"])
-        self._lin(ao.view(M, H * V), Lw.lo, Lw.lo_t, d["y"])
+        left, na = self._out(ao.view(M, H * V), Lw.lo, Lw.lo_t, d["y"])
         # right: gated linear attention, decay per key channel from the low-rank projection (fp32 throughout)
         z = d["z"][:M * Hr * Dr].view(M, Hr * Dr)
         ops.gemm_rm(small[:, H:], Lw.a2, z, bias=Lw.a2_b)
@@ -617,11 +633,12 @@ class LayeredRunner(RunnerBase):
         c0 = NL
         q, k, v = self._scan_rows(big, c0, Hr, Dr, Vr)
         gate = big[:, c0 + 2 * Hr * Dr + Hr * Vr:NL + NR]
-        self._scan_out(ri, Lw.rnorm, gate, Hr, Vr, M, d, q, k, v, z.view(M, Hr, Dr), None, groups, Dr ** -0.5, Lw.ro,
-                       Lw.ro_t, d["y2"])
-        ops.rms_mix(d["y"], Lw.left_out, d["y2"], Lw.right_out, self.cfg.eps, 0.5, d["y"])
+        right, nb = self._scan_out(ri, Lw.rnorm, gate, Hr, Vr, M, d, q, k, v, z.view(M, Hr, Dr), None, groups, Dr ** -0.5, Lw.ro,
+                                   Lw.ro_t, d["y2"])
+        ops.rms_mix(left, Lw.left_out, right, Lw.right_out, self.cfg.eps, 0.5, d["ym"], na, nb)
+        return d["ym"], 1
 
-    def _retention(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _retention(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         H, D, V = m.heads, m.dim, m.vdim
         N = 2 * H * (D + V)
         big = d["big"][:M * N].view(M, N)
@@ -629,8 +646,8 @@ class LayeredRunner(RunnerBase):
         rope = self._rope.get(m.rot)
         q, k, v = self._scan_rows(big, 0, H, D, V)
         ops.norm_rope_list(pos, (q, None, rope, q, None, 0, 0.0, 1.0, None), (k, None, rope, k, None, 0, 0.0, D ** -0.5, None))
-        self._scan_out(ri, None, big[:, 2 * H * D + H * V:], H, V, M, d, q, k, v, Lw.decay, None, groups, 1.0, Lw.o,
-                       Lw.o_t, d["y"])
+        return self._scan_out(ri, None, big[:, 2 * H * D + H * V:], H, V, M, d, q, k, v, Lw.decay, None, groups, 1.0, Lw.o,
+                              Lw.o_t, d["y"])
 
     # ------------------------------------------------------------------ pre-norm designs on several residual streams
     def _setup_streams(self) -> None:
@@ -735,13 +752,11 @@ class LayeredRunner(RunnerBase):
                 elif routed:
                     ops.act_rows(d["hn"], d["xb"], 0)
                 if sub == 1:
-                    getattr(self, "_" + L.kind + "_streams")(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups)
-                    prev = (d["y"], 1, hc)
+                    prev = getattr(self, "_" + L.kind + "_streams")(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups) + (hc,)
                 elif routed:
                     prev = self._routed_ff(L.mlp, Lw.mlp, M, d, d["hc"] if conv else d["hn"]) + (hc,)
                 else:
-                    self._act_ff(L.mlp, Lw.mlp, M, d)
-                    prev = (d["y"], 1, hc)
+                    prev = self._act_ff(L.mlp, Lw.mlp, M, d) + (hc,)
             if trace is not None:
                 y, nsum, pw = prev
                 ops.stream_mix(y, nsum, mult, x, out_w=pw.outw, mix=pw.mix, total=d["resid"])
@@ -751,7 +766,7 @@ class LayeredRunner(RunnerBase):
         ops.stream_mix(y, nsum, mult, x, ids if first else None, w.embed if first else None, cfg.embed_scale,
                        pw.outw if pw else None, pw.mix if pw else None, total=d["resid"])
 
-    def _latent_attention_streams(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _latent_attention_streams(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Latent attention with a query latent and a sigmoid output gate: ONE fused GEMM [dq | dkv | g] (fp32 out) ->
         RMS norm of the query latent -> query up-projection; latent_kv_write (norm + rotation + cache row) from the
         dkv columns; folded attention over this run's latent pages; per-head value up-projection (fp32) times
@@ -791,9 +806,9 @@ class LayeredRunner(RunnerBase):
                                      m.window, m.scale, g["qt"])
         ops.gemm_rm(lat.permute(1, 0, 2), Lw.uv, o.permute(1, 0, 2))
         ops.act_rows(o.view(M, H * dv), ao, 0, None, big[:, qr + rk + dr:qr + rk + dr + H * dv])
-        self._lin(ao, Lw.o, Lw.o_t, d["y"])
+        return self._out(ao, Lw.o, Lw.o_t, d["y"])
 
-    def _attention_streams(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _attention_streams(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Sliding-window attention with grouped key/value heads and per-head RMS norms on q and k, no rotation: ONE
         fused GEMM [q | k | v] -> norm rows (q to a buffer, k and v straight into this run's pages) -> attention over
         the window (MFMA form where the head widths allow it) -> output GEMM."""
@@ -818,15 +833,15 @@ class LayeredRunner(RunnerBase):
             else:
                 ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], None, None, ao,
                                    m.window, m.scale, g["qt"])
-        self._lin(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
+        return self._out(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
 
-    def _act_ff(self, f, Fw, M: int, d: dict) -> None:
+    def _act_ff(self, f, Fw, M: int, d: dict):
         """Dense feed-forward: up GEMM (fp32) -> xIELU -> down GEMM."""
         up = d["up"][:M * f.ff].view(M, f.ff)
         h = d["h"][:M * f.ff].view(M, f.ff)
         self._lin(d["xb"], Fw.up, Fw.up_t, up)
         ops.act_rows(up, h, 1, Fw.act)
-        self._lin(h, Fw.down, Fw.down_t, d["y"])
+        return self._out(h, Fw.down, Fw.down_t, d["y"])
 
     def _routed_ff(self, f, Fw, M: int, d: dict, h32):
         """Router GEMM in true fp32 on the sublayer's fp32 input `h32` (a close call is decided by the row itself, not by
@@ -946,8 +961,7 @@ class LayeredRunner(RunnerBase):
             if not ready:
                 ops.add_norm_rows(*pending, d["resid"], Lw.norm1, eps, d["xb"])
             ready = False
-            getattr(self, "_" + L.kind + "_bracket")(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups)
-            pending = (d["y"], 1, Lw.norm1b)
+            pending = getattr(self, "_" + L.kind + "_bracket")(run.index, L.mixer, Lw.mix, M, d, pos, slots, groups) + (Lw.norm1b,)
             if L.mlp is not None:
                 routed = isinstance(L.mlp, SoftmaxRoutedSpec)
                 ops.add_norm_rows(*pending, d["resid"], Lw.norm2, eps, d["xb"], d["hn"] if routed else None)
@@ -956,8 +970,7 @@ class LayeredRunner(RunnerBase):
                 elif self.memory:
                     pending = self._memory_ff(run.layer, L.mlp, Lw.mlp, M, d) + (Lw.norm2b,)
                 else:
-                    self._relu2_ff(L.mlp, Lw.mlp, M, d)
-                    pending = (d["y"], 1, Lw.norm2b)
+                    pending = self._relu2_ff(L.mlp, Lw.mlp, M, d) + (Lw.norm2b,)
             if Lw.side is not None:  # the layer's token input reads the stream after the feed-forward
                 sd = Lw.side
                 if fused_side:  # decode-sized steps: one launch, which also makes the next sublayer's input
@@ -974,8 +987,7 @@ class LayeredRunner(RunnerBase):
                     ops.add_norm_rows(*pending, d["resid"], None, eps, d["xb"])
                     ops.gemm_rm(d["xb"], sd.gate, sg)
                     ops.token_gate_rows(sg, ids, w.side_embed, sd.col0, sh)
-                    ops.gemm_rm(sh, sd.proj, d["y"])
-                    pending = (d["y"], 1, sd.norm)
+                    pending = self._out(sh, sd.proj, None, d["y"]) + (sd.norm,)
             if trace is not None:
                 if pending[0] is not None:
                     ops.add_norm_rows(*pending, d["resid"], None, eps)
@@ -984,7 +996,7 @@ class LayeredRunner(RunnerBase):
         if pending[0] is not None:
             ops.add_norm_rows(*pending, d["resid"], None, eps)
 
-    def _attention_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _attention_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Softmax attention whose values are rotated by their positions: ONE fused GEMM [q | k | v | g] (fp32 out) ->
         norm rows (q: whole-row RMS norm + rotation into a buffer; k the same into this run's pages; v: RMS norm per
         head + rotation over the whole value width into the pages, also transposed) -> attention over the window with
@@ -1012,9 +1024,9 @@ class LayeredRunner(RunnerBase):
             else:
                 ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"], g["wt"], None, gate, ao,
                                    m.window, m.scale, g["qt"], None, False, m.softcap, vrope)
-        self._lin(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
+        return self._out(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
 
-    def _channel_delta_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _channel_delta_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Gated delta rule with a decay per head and key channel: ONE fused GEMM [q | k | v | b | a1 | g1] (fp32 out)
         -> conv_state over q | k | v (SiLU; slot tail) -> unit q, k per head in one launch (the query's dim^-1/2
         rides in the scan) -> the decay's and the gate's second projections in fp32 as one block-diagonal product
@@ -1043,15 +1055,15 @@ class LayeredRunner(RunnerBase):
                             g["ss"], o, D ** -0.5, g.get("longest", 0))
         ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw.norm, gz, self.cfg.eps, ao, 1)
-        self._lin(ao, Lw.o, Lw.o_t, d["y"])
+        return self._out(ao, Lw.o, Lw.o_t, d["y"])
 
-    def _relu2_ff(self, f, Fw, M: int, d: dict) -> None:
+    def _relu2_ff(self, f, Fw, M: int, d: dict):
         """Dense feed-forward: up GEMM (fp32) -> squared ReLU -> down GEMM."""
         up = d["up"][:M * f.ff].view(M, f.ff)
         h = d["h"][:M * f.ff].view(M, f.ff)
         self._lin(d["xb"], Fw.up, Fw.up_t, up)
         ops.act_rows(up, h, 2)
-        self._lin(h, Fw.down, Fw.down_t, d["y"])
+        return self._out(h, Fw.down, Fw.down_t, d["y"])
 
     def _softmax_routed_ff(self, f, Fw, M: int, d: dict):
         """Router GEMM in true fp32 on the fp32 normed row -> softmax scores, group-limited choice, unnormalised weights
@@ -1151,8 +1163,7 @@ class LayeredRunner(RunnerBase):
             up, h = d["up"][:M * f.ff].view(M, f.ff), d["h"][:M * f.ff].view(M, f.ff)
             self._lin(d["xb"], Fw.up, Fw.up_t, up)
             ops.act_rows(up, h, 3)
-            self._lin(h, Fw.down, Fw.down_t, d["y"])
-            return d["y"], 1
+            return self._out(h, Fw.down, Fw.down_t, d["y"])
         n = self._moe_layers.index(layer)
         W, w = self.cfg.width, (Fw.gate, Fw.up, Fw.down, Fw.sgate, Fw.sup, Fw.sdown)
         P = ops.moe_parts(d["xb"], f.top, *w, d["mo_h"])
@@ -1191,7 +1202,7 @@ class LayeredRunner(RunnerBase):
                               a.heads, a.kv_heads, a.dim, vdim, rope, temp, slots, qa, self.kv.k[ri], self.kv.v[ri],
                               self.kv.vt.get(ri))
 
-    def _conv_attention_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _conv_attention_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Attention whose q and k pass a convolution over time and whose values are the keys before their rotation."""
         H, G, D = m.heads, m.kv_heads, m.dim
         big = d["big"][:M * Lw.n_big].view(M, Lw.n_big)
@@ -1200,9 +1211,9 @@ class LayeredRunner(RunnerBase):
         self._qkv_rows(ri, m, big, Lw.conv, 0, self._rope.get(m.rot), None, slots, qa, groups)
         ao = d["ao"][:M * H * D].view(M, H, D)
         self._sink_rows(ri, m, qa, Lw.sink, big[:, (H + G) * D:(H + G) * D + H], ao, groups)
-        self._lin(ao.view(M, H * D), Lw.o, Lw.o_t, d["y"])
+        return self._out(ao.view(M, H * D), Lw.o, Lw.o_t, d["y"])
 
-    def _twin_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list) -> None:
+    def _twin_bracket(self, ri: int, m, Lw, M: int, d: dict, pos, slots, groups: list):
         """Attention and matrix memory on the same rows; their gated heads, times the layer's two scales, are the two
         column ranges of one row, and one output projection sums both halves."""
         a, r = m.left, m.right
@@ -1228,7 +1239,7 @@ class LayeredRunner(RunnerBase):
                               g["qs"], g["ql"], g["ctx"], g["ss"], gate, Lw.norm, self.cfg.eps, MEMORY_EPS, Dr ** -0.5,
                               m.right_scale, ao[:, H * V:H * V + Hr * Vr], d["mm"] if chunked else None,
                               *(g["rows"] if chunked else ()))
-        self._lin(ao, Lw.o, Lw.o_t, d["y"])
+        return self._out(ao, Lw.o, Lw.o_t, d["y"])
 
     # ------------------------------------------------------------------ mixer and feed-forward side by side
     def _setup_joint(self) -> None:
@@ -1280,31 +1291,31 @@ class LayeredRunner(RunnerBase):
         the same time: the mixer's launches are latency-sized, the experts' stream weights."""
         cfg, w, eps = self.cfg, self.w, self.cfg.eps
         ops.embed_rows(ids, w.embed, d["resid"], None, cfg.embed_scale, pos, self._pos_table)
-        pending = (None, 1, None)  # sublayer outputs that are not in the stream yet: (rows, parts per row, second rows)
+        none = (None, 1, None, 1)
+        pending = none  # sublayer outputs that are not in the stream yet: (rows, parts per row) of both
         for i, (L, Lw) in enumerate(zip(cfg.layers, w.layers)):
-            y, nsum, y2 = pending
-            ops.add_norm_rows(y, nsum, None, d["resid"], Lw.norm1, eps, d["xb"], d["hn"] if L.mlp is not None else None, y2)
-            pending = (d["y"], 1, None)
+            y, nsum, y2, nsum2 = pending
+            ops.add_norm_rows(y, nsum, None, d["resid"], Lw.norm1, eps, d["xb"], d["hn"] if L.mlp is not None else None, y2, nsum2)
             if L.mlp is None:
-                self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
+                pending = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups) + (None, 1)
             elif self._side_stream is None:
-                self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
-                pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d) + (d["y"],)
+                mixed = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
+                pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d) + mixed
             else:
                 main = torch.cuda.current_stream(self.device)
                 self._side_stream.wait_stream(main)
                 with torch.cuda.stream(self._side_stream):
-                    pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d) + (d["y"],)
-                self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
+                    pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d)
+                pending += self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
                 main.wait_stream(self._side_stream)
             if trace is not None:
-                ops.add_norm_rows(pending[0], pending[1], None, d["resid"], None, eps, y2=pending[2])
-                pending = (None, 1, None)
+                ops.add_norm_rows(pending[0], pending[1], None, d["resid"], None, eps, None, None, *pending[2:])
+                pending = none
                 trace.append(d["resid"].clone())
         if pending[0] is not None:
-            ops.add_norm_rows(pending[0], pending[1], None, d["resid"], None, eps, y2=pending[2])
+            ops.add_norm_rows(pending[0], pending[1], None, d["resid"], None, eps, None, None, *pending[2:])
 
-    def _attention_joint(self, li: int, m, Lw, M: int, d: dict, slots, groups: list) -> None:
+    def _attention_joint(self, li: int, m, Lw, M: int, d: dict, slots, groups: list):
         """Windowed attention with a distance bias over this layer's pages, or over those of the layer it takes keys and
         values from (that layer has written this step's rows before)."""
         H, G, D, V = m.heads, m.kv_heads, m.dim, m.vdim
@@ -1329,7 +1340,7 @@ class LayeredRunner(RunnerBase):
                 work, form = (g["ws"], g["wt"]), (g["qt"], None, False)
             ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], *work, None, gate, ao, m.window, m.scale,
                                *form, rel=Lw.rel, keep_first=m.keep_first)
-        self._lin(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
+        return self._out(ao.view(M, H * V), Lw.o, Lw.o_t, d["y"])
 
     def _input_weighted_ff(self, f, Fw, M: int, d: dict):
         """Router GEMM in true fp32 on the fp32 normed row (the shared expert's gate is its last column) -> the largest
@@ -1373,7 +1384,7 @@ class LayeredRunner(RunnerBase):
         r = slice(0, B)
         ops.decode_prep(self.active[r], self.positions[r], self.block_tables[r], self.slots[r], self.ctx_len[r],
                         self.q_len[r], self.kv.num_blocks)
-        rows = ("resid", "xb", "y", "y2", "streams", "hn", "hc", "cat")
+        rows = ("resid", "xb", "ym", "streams", "hn", "hc", "cat")
         d = {k: (v[:B] if k in rows and v is not None else v) for k, v in self._dec.items()}
         prev = (self.prev_ids[r], self.prev_ids[r], self.q_len[r]) if self.pair else None
         self._layers(B, d, self.ids[r], self.positions[r], self.slots[r], [self._decode_group(B)], prev=prev)

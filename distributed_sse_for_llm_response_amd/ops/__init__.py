@@ -110,6 +110,15 @@ def gemm_resid_split(x, w, resid, part) -> int:
     return 0
 
 
+def gemm_out_parts(x, w, part) -> int:
+    """The fp32 product x · wᵀ for a consumer that adds the consecutive parts of a row (the norms' nsum): writes [M, S, N]
+    to the front of `part` and returns S -- the kernel's K slices where it splits K and `part` holds them, else 1."""
+    if _hip(x):
+        return int(torch.ops.dsse.gemm_out_parts(x, w, part))
+    ref.gemm_out(x, w, part.view(-1)[:x.shape[0] * w.shape[0]].view(x.shape[0], w.shape[0]))
+    return 1
+
+
 def gemm_out_split(x, w, out, part) -> int:
     """out = x · wᵀ (bf16), or (when the chosen kernel splits K) fp32 slabs [S, M, N] into `part` and return S for a
     consumer that sums them (the TP decode step's IPC all-reduce, comm.all_reduce_rmsnorm(part=..., nsplit=S))."""

@@ -198,13 +198,14 @@ def moe_route_rows(x, w, topk_idx, topk_w, scale: float, sorted_ids, tile_expert
 # ---------------------------------------------------------------------------------------------------------------------
 # Pre-norm designs with matrix-state mixers.  Small parameter vectors (norm gains, sinks, decay parameters) are fp32
 # in both element types.
-def stream_step(y, mult: float, resid, ids, embed, vec, alpha, w, b, xb):
-    """The residual stream's step between sublayers: resid (fp32) += mult * y (y given) + embed[ids] (embed given) +
+def stream_step(y, mult: float, resid, ids, embed, vec, alpha, w, b, xb, nsum: int = 1):
+    """The residual stream's step between sublayers: resid (fp32) += mult * y (y given, [M * nsum, W]; a row's nsum
+    consecutive parts are summed first) + embed[ids] (embed given) +
     vec (vec [W] given); then, when a norm follows (w given), xb = tanh(alpha * resid) * w + b in the element type."""
     if _hip(resid):
-        torch.ops.dsse.stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb)
+        torch.ops.dsse.stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb, nsum)
     else:
-        lref.stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb)
+        lref.stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb, nsum)
 
 
 def gated_act(gu, h, kind: int = 1):
@@ -403,12 +404,13 @@ def gated_head_norm(o, w, gate, eps: float, out, kind: int = 0):
         lref.gated_head_norm(o, w, gate, eps, out, kind)
 
 
-def rms_mix(ya, wa, yb, wb, eps: float, coef: float, out):
-    """out (fp32) = coef * (rms-norm(ya) * wa + rms-norm(yb) * wb)."""
+def rms_mix(ya, wa, yb, wb, eps: float, coef: float, out, na: int = 1, nb: int = 1):
+    """out (fp32) = coef * (rms-norm(ya) * wa + rms-norm(yb) * wb); ya [M * na, W] and yb [M * nb, W]: a row's parts are
+    summed first.  out may be ya or yb where that has one part per row."""
     if _hip(ya):
-        torch.ops.dsse.rms_mix(ya, wa, yb, wb, eps, coef, out)
+        torch.ops.dsse.rms_mix(ya, wa, yb, wb, eps, coef, out, na, nb)
     else:
-        lref.rms_mix(ya, wa, yb, wb, eps, coef, out)
+        lref.rms_mix(ya, wa, yb, wb, eps, coef, out, na, nb)
 
 
 def logit_cap(logits, scale: float, cap: float):
@@ -473,17 +475,17 @@ def embed_pair_rows(ids, prev, positions, embed, pair, mul_prev: int, mul_cur: i
         lref.embed_pair_rows(ids, prev, positions, embed, pair, mul_prev, mul_cur, buckets, resid, x0, prev_out, keep)
 
 
-def add_norm_rows(y, nsum: int, g_add, resid, g_out, eps: float, out=None, out32=None, y2=None):
+def add_norm_rows(y, nsum: int, g_add, resid, g_out, eps: float, out=None, out32=None, y2=None, nsum2: int = 1):
     """The stream's step between sublayers of a design that norms a sublayer's input AND its output, in one pass over
     the row: y given ([M * nsum, W] fp32; a row's nsum consecutive parts are summed first, the grouped experts' slots):
     resid += y / rms(y) * g_add; out given (element type or fp32; a column slice of a wider buffer is fine):
     out = resid / rms(resid) * g_out, or the stream itself when g_out is None; out32 (fp32) receives that row unrounded
-    (what a router reads).  Gains are fp32 [W].  g_add None with y given: y is added as it is (no norm), and y2 [M, W] (a
+    (what a router reads).  Gains are fp32 [W].  g_add None with y given: y is added as it is (no norm), and y2 [M * nsum2, W] (a
     second sublayer that read the same norm) with it."""
     if _hip(resid):
-        torch.ops.dsse.add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2)
+        torch.ops.dsse.add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2, nsum2)
     else:
-        lref.add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2)
+        lref.add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2, nsum2)
 
 
 def token_gate_rows(x, ids, table, col0: int, out):

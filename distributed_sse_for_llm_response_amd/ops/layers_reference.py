@@ -223,12 +223,12 @@ def moe_grouped(x, topk_idx, topk_w, gate, up, down, sgate, sup, sdown, o, weigh
 
 # ---------------------------------------------------------------------------------------------------------------------
 # Pre-norm designs with matrix-state mixers (models/surodra.py)
-def stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb):
-    """resid += mult * y (y given) + embed[ids] (embed given) + vec (vec given); then, with a norm (w given),
+def stream_step(y, mult, resid, ids, embed, vec, alpha, w, b, xb, nsum=1):
+    """resid += mult * y (y given, a row's nsum parts summed first) + embed[ids] (embed given) + vec (vec given); then, with a norm (w given),
     xb = tanh(alpha * resid) * w + b."""
     M = resid.shape[0]
     if y is not None:
-        resid.add_(y.float() * mult)
+        resid.add_(y.float().view(M, nsum, -1).sum(1) * mult)
     if embed is not None:
         idx = ids[:M].long()
         idx = torch.where((idx >= 0) & (idx < embed.shape[0]), idx, torch.zeros_like(idx))
@@ -391,12 +391,13 @@ def gated_head_norm(o, w, gate, eps, out, kind=0):
     out.copy_((n.reshape(T, H * V) * g).to(out.dtype))
 
 
-def rms_mix(ya, wa, yb, wb, eps, coef, out):
-    """out (fp32) = coef * (ya / rms(ya) * wa + yb / rms(yb) * wb), rows of the model width."""
-    def n(y, w):
-        return y.float() / torch.sqrt(y.float().pow(2).mean(-1, keepdim=True) + eps) * w.float()
+def rms_mix(ya, wa, yb, wb, eps, coef, out, na=1, nb=1):
+    """out (fp32) = coef * (ya / rms(ya) * wa + yb / rms(yb) * wb), rows of the model width, their na / nb parts summed first."""
+    def n(y, w, parts):
+        y = y.float().view(out.shape[0], parts, -1).sum(1)
+        return y / torch.sqrt(y.pow(2).mean(-1, keepdim=True) + eps) * w.float()
 
-    out.copy_(coef * (n(ya, wa) + n(yb, wb)))
+    out.copy_(coef * (n(ya, wa, na) + n(yb, wb, nb)))
 
 
 def logit_cap(logits, scale, cap):
@@ -495,14 +496,14 @@ def embed_pair_rows(ids, prev, positions, embed, pair, mul_prev, mul_cur, bucket
         x0.copy_(rows.to(x0.dtype))
 
 
-def add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2=None):
+def add_norm_rows(y, nsum, g_add, resid, g_out, eps, out, out32, y2=None, nsum2=1):
     """The residual stream's step of a design with a norm before AND after each sublayer.  y given ([M * nsum, W] fp32,
     a row's nsum consecutive parts are summed first): resid += y / rms(y) * g_add.  out given (element type or fp32, may
     be a column slice): out = resid / rms(resid) * g_out, or resid itself without g_out; out32 (optional, fp32) receives
     the same row unrounded.  g_add None: y is added as it is, and so is y2 (a second sublayer's output) when given."""
     if y is not None and g_add is None:
         v = y.float().view(resid.shape[0], nsum, -1).sum(1)
-        resid.add_(v if y2 is None else v + y2.float())
+        resid.add_(v if y2 is None else v + y2.float().view(resid.shape[0], nsum2, -1).sum(1))
     elif y is not None:
         v = y.float().view(resid.shape[0], nsum, -1).sum(1)
         resid.add_(v / torch.sqrt(v.pow(2).mean(-1, keepdim=True) + eps) * g_add.float())

@@ -1,0 +1,74 @@
+"""K slices of a product as the parts of its rows (gemm_out_parts), and the norms that add them, against fp32 references."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    ops.load_library(required=True)
+    return torch.device("cuda", 0)
+
+
+# register streaming; one launch before a norm of few rows; the ring to 64 and to 128 rows; the tile of all rows and the one of 128; the pipeline
+# with rows past its tiles and a half-empty column block; shapes that are not split
+@pytest.mark.parametrize("M,N,K,parts", [
+    (1, 2048, 2048, 1), (20, 2048, 2048, 1), (33, 2048, 2048, 4), (100, 2048, 2048, 8), (160, 4096, 14336, 8), (200, 2048, 2048, 4),
+    (301, 2048, 2048, 0), (400, 1152, 4096, 0), (2500, 2048, 512, 1), (40, 2064, 384, 0)])
+def test_parts(gpu, M, N, K, parts):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.empty(M, K, device=gpu, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(N, K, device=gpu, dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g)
+    wt = ops.ref.tile_weight(w.cpu()).to(gpu).view(N, K)
+    want = x.float() @ w.float().t()
+    part = torch.full((16 * M * N,), float("nan"), device=gpu)
+    S = ops.gemm_out_parts(x, wt, part)
+    assert S == parts or (parts == 0 and S >= 1)
+    # fp32 sums of exact products: an error of K / 2 roundings of 2^-24 at the most, a few in fact
+    got = part[:S * M * N].view(M, S, N).sum(1)
+    assert float((got - want).norm() / want.norm()) <= 1e-5
+    assert bool(torch.isnan(part[S * M * N:]).all())  # nothing behind its parts
+    # a buffer that does not hold the slices gets the whole product
+    whole = torch.full((M * N,), float("nan"), device=gpu)
+    assert ops.gemm_out_parts(x, wt, whole) == 1
+    assert float((whole.view(M, N) - want).norm() / want.norm()) <= 1e-5
+    with pytest.raises(RuntimeError):
+        ops.gemm_out_parts(x, wt, whole[:-1])
+
+
+# vector and scalar rows; parts up to and past a group of four
+@pytest.mark.parametrize("W", [64, 130, 2048])
+@pytest.mark.parametrize("na,nb", [(1, 1), (2, 5), (8, 4), (9, 1)])
+def test_norms_add_parts(gpu, W, na, nb):
+    M, g = 5, torch.Generator().manual_seed(W + na)
+    r = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    ya, yb, resid, w, b, alpha = r(M * na, W), r(M * nb, W), r(M, W), r(W), r(W), r(1)
+    c = lambda t: t.to(gpu)  # noqa: E731
+    close = lambda a, b: torch.testing.assert_close(a.cpu(), b, rtol=2e-5, atol=2e-5)  # noqa: E731
+
+    want, wx, got, gx = resid.clone(), torch.zeros(M, W), c(resid.clone()), torch.zeros(M, W, device=gpu)
+    lref.stream_step(ya, 0.5, want, None, None, None, alpha, w, b, wx, na)
+    ops.stream_step(c(ya), 0.5, got, None, None, None, c(alpha), c(w), c(b), gx, na)
+    close(got, want), close(gx, wx)
+
+    want, got = torch.zeros(M, W), torch.zeros(M, W, device=gpu)
+    lref.rms_mix(ya, w, yb, b, 1e-5, 0.5, want, na, nb)
+    ops.rms_mix(c(ya), c(w), c(yb), c(b), 1e-5, 0.5, got, na, nb)
+    close(got, want)
+    if na > 1:
+        both = c(ya)
+        with pytest.raises(RuntimeError):
+            ops.rms_mix(both, c(w), c(yb), c(b), 1e-5, 0.5, both[:M], na, nb)
+
+    want, wx, got, gx = resid.clone(), torch.zeros(M, W), c(resid.clone()), torch.zeros(M, W, device=gpu)
+    lref.add_norm_rows(ya, na, None, want, w, 1e-5, wx, None, yb, nb)
+    ops.add_norm_rows(c(ya), na, None, got, c(w), 1e-5, gx, None, c(yb), nb)
+    close(got, want), close(gx, wx)
+    with pytest.raises(RuntimeError):
+        ops.add_norm_rows(c(ya), na, None, got, c(w), 1e-5, gx, None, c(yb), nb + 1)
