@@ -145,7 +145,7 @@ hipError_t dsse_rope_kv_write(int T, const void* qkv, int hq, int hkv, const int
                               void* v_cache, int num_slots, int rope_len, hipStream_t st);
 hipError_t dsse_silu_mul(int T, int F, const void* gu, void* h, hipStream_t st);
 hipError_t dsse_decode_prep(int B, const int* active, const int* positions, const int* block_tables,
-                            int max_blocks, int num_blocks, int* slots, int* ctx_len, int* q_len, hipStream_t st);
+                            int max_blocks, int num_blocks, int* slots, int* ctx_len, int* q_len, int* walked, hipStream_t st);
 hipError_t dsse_ring_advance(int* counter, hipStream_t st);
 // TP all-reduce + residual + RMSNorm over IPC peer buffers (allreduce.hip)
 size_t dsse_ar_buffer_bytes(int rows, int H);

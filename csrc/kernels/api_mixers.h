@@ -80,6 +80,8 @@ struct SinkAttnParams {
   float out_scale;       // multiplies the output before it is rounded (1: nothing)
   int nparts;            // decode form: stretches the walk of a row is split into (<= 1: none, at most 16)
   float* part;           // [work items, H, nparts, V + 2] when split
+  const int* walked;     // decode form: tokens of all rows together, or null
+  float once;            // ... pages of more bytes than this in one launch are read non-temporally
 };
 
 // Whether the exact mode's shared-page form (sink_exact.hip) takes a launch of num_work items of p.qt rows: fp32, head widths up

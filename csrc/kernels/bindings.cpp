@@ -895,7 +895,7 @@ void silu_mul(const Tensor& gu, Tensor& h) {
 }
 
 void decode_prep(const Tensor& active, const Tensor& positions, const Tensor& block_tables,
-                 Tensor& slots, Tensor& ctx_len, Tensor& q_len, int64_t num_blocks) {
+                 Tensor& slots, Tensor& ctx_len, Tensor& q_len, int64_t num_blocks, const std::optional<Tensor>& walked) {
   for (const Tensor* t : {&active, &positions, &block_tables, (const Tensor*)&slots, (const Tensor*)&ctx_len, (const Tensor*)&q_len}) {
     check_gpu(*t, "decode metadata");
     check_dtype(*t, at::kInt, "decode metadata");
@@ -903,10 +903,15 @@ void decode_prep(const Tensor& active, const Tensor& positions, const Tensor& bl
   const int B = (int)active.numel();
   TORCH_CHECK(positions.numel() >= B && slots.numel() >= B && ctx_len.numel() >= B &&
                   q_len.numel() >= B && block_tables.size(0) >= B, "decode metadata too short");
+  if (walked.has_value()) {
+    check_gpu(*walked, "walked");
+    check_dtype(*walked, at::kInt, "walked");
+    TORCH_CHECK(walked->numel() >= 1, "walked must hold one number");
+  }
   DSSE_CHECK_HIP(dsse_decode_prep(B, active.data_ptr<int>(), positions.data_ptr<int>(),
                                   block_tables.data_ptr<int>(), (int)block_tables.size(1),
                                   (int)std::min<int64_t>(num_blocks, INT32_MAX), slots.data_ptr<int>(), ctx_len.data_ptr<int>(), q_len.data_ptr<int>(),
-                                  cur_stream()));
+                                  walked.has_value() ? walked->data_ptr<int>() : nullptr, cur_stream()));
 }
 
 // Warm the Infinity Cache with the first `bytes` of `t` (all of it when bytes < 0) on `wgs` workgroups; `sink`:
@@ -1435,7 +1440,7 @@ TORCH_LIBRARY(dsse, m) {
         "Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv) -> ()");
   m.def("silu_mul(Tensor gu, Tensor(a!) h) -> ()");
   m.def("decode_prep(Tensor active, Tensor positions, Tensor block_tables, Tensor(a!) slots, "
-        "Tensor(b!) ctx_len, Tensor(c!) q_len, int num_blocks=2147483647) -> ()");
+        "Tensor(b!) ctx_len, Tensor(c!) q_len, int num_blocks=2147483647, Tensor(d!)? walked=None) -> ()");
   m.def("ring_advance(Tensor(a!) counter) -> ()");
   m.def("paged_attention(int mode, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor q_start, Tensor q_len, Tensor ctx_len, Tensor work_seq, Tensor work_tile, Tensor(a!) out, "

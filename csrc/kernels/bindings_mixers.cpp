@@ -246,7 +246,8 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
                     const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len, const Tensor& work_seq,
                     const Tensor& work_tile, const OptTensor& sink, const OptTensor& gate, Tensor& out, int64_t window,
                     double scale, int64_t qt, const OptTensor& vt, bool split, double softcap, const OptTensor& out_rope,
-                    const OptTensor& rel, int64_t keep_first, double out_scale, const OptTensor& part, int64_t nparts) {
+                    const OptTensor& rel, int64_t keep_first, double out_scale, const OptTensor& part, int64_t nparts,
+                    const OptTensor& walked, double once) {
   f32t(q, "q");
   gpu(kcache, "kcache");
   gpu(vcache, "vcache");
@@ -270,6 +271,11 @@ void sink_attention(const Tensor& q, const Tensor& kcache, const Tensor& vcache,
               "out rows must hold adjacent heads");
   p.ldo = (int)out.stride(0);
   p.out_scale = (float)out_scale;
+  if (walked.has_value()) {
+    i32(*walked, "walked");
+    TORCH_CHECK(walked->numel() >= 1, "walked must hold one number");
+    p.walked = walked->data_ptr<int>(), p.once = (float)once;
+  }
   TORCH_CHECK(block_tables.dim() == 2, "block_tables must be [seqs, max_blocks]");
   const int ns = (int)block_tables.size(0);
   seq_meta(q_start, q_len, ctx_len, ns);
@@ -934,7 +940,8 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("sink_attention(Tensor q, Tensor kcache, Tensor vcache, Tensor block_tables, Tensor q_start, Tensor q_len, "
         "Tensor ctx_len, Tensor work_seq, Tensor work_tile, Tensor? sink, Tensor? gate, Tensor(a!) out, int window, "
         "float scale, int qt, Tensor? vt=None, bool split=False, float softcap=0.0, Tensor? out_rope=None, "
-        "Tensor? rel=None, int keep_first=0, float out_scale=1.0, Tensor(b!)? part=None, int nparts=1) -> ()");
+        "Tensor? rel=None, int keep_first=0, float out_scale=1.0, Tensor(b!)? part=None, int nparts=1, "
+        "Tensor? walked=None, float once=0.0) -> ()");
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
   m.def("gate_pair(Tensor(a!) x, Tensor p1, Tensor p2) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "

@@ -47,6 +47,11 @@ template <typename V>
 DEV V ld_global(const void* p) {
   return *(const DSSE_GLOBAL V*)(p);
 }
+// data that one wave reads once: non-temporal
+template <typename V>
+DEV V ld_once(const void* p) {
+  return __builtin_nontemporal_load((const DSSE_GLOBAL V*)(p));
+}
 
 DEV bf16x8 zero_bf16x8() {
   bf16x8 z;

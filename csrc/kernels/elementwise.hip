@@ -227,25 +227,36 @@ silu_mul_kernel(const bf16* __restrict__ gu, bf16* __restrict__ h, int F, int T)
 }
 
 // ---- decode-step metadata (runs first inside the captured graph) -----------------------------
-// For slot b: live sequences process the token at positions[b]; dead slots write nothing.
-__global__ void decode_prep_kernel(int B, const int* __restrict__ active, const int* __restrict__ positions,
-                                   const int* __restrict__ block_tables, int max_blocks, int num_blocks,
-                                   int* __restrict__ slots, int* __restrict__ ctx_len,
-                                   int* __restrict__ q_len) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  if (active[b]) {
-    const int pos = positions[b];
-    const int page = DSSE_IDX(block_tables[(size_t)b * max_blocks + DSSE_IDX(pos / kPageTok, max_blocks, 0)],
-                              num_blocks, 0);
-    slots[b] = page * kPageTok + pos % kPageTok;
-    ctx_len[b] = pos + 1;
-    q_len[b] = 1;
-  } else {
-    slots[b] = -1;
-    ctx_len[b] = 0;
-    q_len[b] = 0;
+// For slot b: live sequences process the token at positions[b]; dead slots write nothing.  One workgroup; `walked` (or null)
+// receives the tokens of all live sequences.
+__global__ void __launch_bounds__(1024)
+decode_prep_kernel(int B, const int* __restrict__ active, const int* __restrict__ positions,
+                   const int* __restrict__ block_tables, int max_blocks, int num_blocks, int* __restrict__ slots,
+                   int* __restrict__ ctx_len, int* __restrict__ q_len, int* __restrict__ walked) {
+  __shared__ int sums[16];
+  int tokens = 0;
+  for (int b = threadIdx.x; b < B; b += blockDim.x) {
+    if (active[b]) {
+      const int pos = positions[b];
+      const int page = DSSE_IDX(block_tables[(size_t)b * max_blocks + DSSE_IDX(pos / kPageTok, max_blocks, 0)],
+                                num_blocks, 0);
+      slots[b] = page * kPageTok + pos % kPageTok;
+      ctx_len[b] = pos + 1;
+      q_len[b] = 1;
+      tokens += pos + 1;
+    } else {
+      slots[b] = -1;
+      ctx_len[b] = 0;
+      q_len[b] = 0;
+    }
   }
+  if (!walked) return;  // uniform
+  tokens = wave_sum(tokens);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = tokens;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) tokens += sums[w];
+  *walked = tokens;
 }
 
 // Token-ring head advance (one thread), the last node of a step.
@@ -298,9 +309,10 @@ extern "C" hipError_t dsse_silu_mul(int T, int F, const void* gu, void* h, hipSt
 
 extern "C" hipError_t dsse_decode_prep(int B, const int* active, const int* positions,
                                        const int* block_tables, int max_blocks, int num_blocks, int* slots,
-                                       int* ctx_len, int* q_len, hipStream_t st) {
-  hipLaunchKernelGGL(decode_prep_kernel, dim3((B + 255) / 256), dim3(256), 0, st, B, active,
-                     positions, block_tables, max_blocks, num_blocks, slots, ctx_len, q_len);
+                                       int* ctx_len, int* q_len, int* walked, hipStream_t st) {
+  const int threads = std::min(1024, (std::max(B, 1) + 63) / 64 * 64);
+  hipLaunchKernelGGL(decode_prep_kernel, dim3(1), dim3(threads), 0, st, B, active, positions, block_tables, max_blocks,
+                     num_blocks, slots, ctx_len, q_len, walked);
   return hipGetLastError();
 }
 

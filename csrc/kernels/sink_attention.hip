@@ -721,10 +721,20 @@ __global__ __launch_bounds__(512 / CT, 2) void sink_tile_kernel(SinkAttnParams p
 // values of a page while its scores are being made.  Same key order, masks, bias and epilogue as above.  Few sequences
 // with long walks: nparts workgroups per (item, group) take a stretch of the walk each, leave sum, maximum and weights in
 // `part`, and a second kernel joins the stretches.
-template <int NT, int KB, int NW, bool EXT>
+//
+// A page is read once in a step.  Loads that allocate find it in the 256 MB behind the L2s again one step later if all layers'
+// pages fit there; if they don't, these loads only wash it through, and non-temporal ones are the faster: the caller says from
+// how many bytes of a launch on (p.once), the step's tokens stand in memory (p.walked).  Measured, non-temporal against
+// allocating, the decode step: 64 sequences of 500 over six layers 923 / 965 us, 32 of 500 738 / 770,
+// 16 of 2000 790 / 822, but 16 of 500 673 / 647; 16 of 1000 over two layers beside 200 MB of state 646 / 667, 4 of 3000 632 /
+// 594.  Beside the expert products of a joint layer (distance bias) allocating loads were hardly ever the slower ones.  KD: the
+// k-steps of keys as wide as the values, at compile time; counted at run time (KD = 0) every k-step is a branch in the page's
+// chain of loads: 8 sequences of 1500 719 us, now 695.
+template <int NT, int KD, int NW, bool EXT>
 __global__ __launch_bounds__(NW * 64) void sink_decode_kernel(SinkAttnParams p, const bf16* __restrict__ vt, int rel_lds) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int D = p.D, V = p.V;
+  constexpr int KB = KD > 0 ? KD : 4;
+  const int D = KD > 0 ? 32 * KD : p.D, V = KD > 0 ? 16 * NT : p.V;
   const int ldq = D + 8;
   const int rep = p.H / p.G;
   const int kvh = blockIdx.y;
@@ -759,6 +769,9 @@ __global__ __launch_bounds__(NW * 64) void sink_decode_kernel(SinkAttnParams p, 
     return (unsigned)b < (unsigned)p.num_blocks ? b : 0;
   };
   int blks = ids_from(0);
+  // all rows decide alike; one column tile only: a second one reads the pages again
+  const bool past = !EXT && rep <= 16 && p.walked &&
+                    fminf((float)*p.walked, (float)gridDim.x * (float)p.window) * (float)(p.G * 2 * (D + V)) > p.once;
   bf16* qs = reinterpret_cast<bf16*>(smem_raw);
   float* rels = reinterpret_cast<float*>(smem_raw + 16 * ldq * sizeof(bf16));   // [cols][rel_lds]
   float* mg = rels + cols * rel_lds;                                            // [NW][cols][V + 2]
@@ -787,14 +800,14 @@ __global__ __launch_bounds__(NW * 64) void sink_decode_kernel(SinkAttnParams p, 
   const int nks = D / 32;
   auto key_row = [&](int blk) { return kc + (((int64_t)blk * kBS + r) * p.G + kvh) * D + 8 * g; };
   bf16x8 ka[KB], kb[KB];  // the current page's keys (k-steps 0 .. KB - 1)
-  auto load_keys = [&](int blk) {
+  auto load_keys = [&](int blk, auto ld) {
     const bf16* k0 = key_row(blk);
     const bf16* k1 = k0 + (int64_t)16 * p.G * D;
 #pragma unroll
     for (int u = 0; u < KB; ++u)
-      if (u < nks) {
-        ka[u] = ld_global<bf16x8>(k0 + 32 * u);
-        kb[u] = ld_global<bf16x8>(k1 + 32 * u);
+      if (KD > 0 || u < nks) {
+        ka[u] = ld(k0 + 32 * u);
+        kb[u] = ld(k1 + 32 * u);
       }
   };
   f32x4 O[NT];
@@ -803,60 +816,66 @@ __global__ __launch_bounds__(NW * 64) void sink_decode_kernel(SinkAttnParams p, 
   float m = -INFINITY, l = 0.f;
   // scores in log2 units; a cap acts on the plain ones
   const float cap_inv = p.softcap > 0.f ? 1.0f / p.softcap : 0.f, cap2 = p.softcap * kLog2e;
-  const float scale2 = p.softcap > 0.f ? p.scale : p.scale * kLog2e;
-  if (mine > 0) load_keys(__builtin_amdgcn_readlane(blks, 0));
-  __syncthreads();
-  for (int it = 0; it < mine; ++it) {
-    const int pg = page_at(it);
-    const int blk = __builtin_amdgcn_readlane(blks, it & 63);
-    const bf16* vrow = vt + (((int64_t)blk * p.G + kvh) * V + r) * kBS + 8 * g;
-    bf16x8 vf[NT];
+  const float scale2 = EXT && p.softcap > 0.f ? p.scale : p.scale * kLog2e;
+  auto walk_pages = [&](auto ld) {
+    if (mine > 0) load_keys(__builtin_amdgcn_readlane(blks, 0), ld);
+    __syncthreads();
+    for (int it = 0; it < mine; ++it) {
+      const int pg = page_at(it);
+      const int blk = __builtin_amdgcn_readlane(blks, it & 63);
+      const bf16* vrow = vt + (((int64_t)blk * p.G + kvh) * V + r) * kBS + 8 * g;
+      bf16x8 vf[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) vf[n] = ld_global<bf16x8>(vrow + (int64_t)n * 16 * kBS);
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+      for (int n = 0; n < NT; ++n) vf[n] = ld(vrow + (int64_t)n * 16 * kBS);
+      f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
-    for (int u = 0; u < KB; ++u)
-      if (u < nks) {
-        const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qs + r * ldq + 32 * u + 8 * g);
-        s0 = mfma16x16x32(ka[u], q8, s0);
-        s1 = mfma16x16x32(kb[u], q8, s1);
+      for (int u = 0; u < KB; ++u)
+        if (KD > 0 || u < nks) {
+          const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qs + r * ldq + 32 * u + 8 * g);
+          s0 = mfma16x16x32(ka[u], q8, s0);
+          s1 = mfma16x16x32(kb[u], q8, s1);
+        }
+      if (KD == 0 && nks > KB) {  // wider heads: the rest of the row, no prefetch
+        const bf16* k0 = key_row(blk);
+        const bf16* k1 = k0 + (int64_t)16 * p.G * D;
+        for (int s = KB; s < nks; ++s) {
+          const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qs + r * ldq + 32 * s + 8 * g);
+          s0 = mfma16x16x32(ld(k0 + 32 * s), q8, s0);
+          s1 = mfma16x16x32(ld(k1 + 32 * s), q8, s1);
+        }
       }
-    if (nks > KB) {  // wider heads: the rest of the row, no prefetch
-      const bf16* k0 = key_row(blk);
-      const bf16* k1 = k0 + (int64_t)16 * p.G * D;
-      for (int s = KB; s < nks; ++s) {
-        const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qs + r * ldq + 32 * s + 8 * g);
-        s0 = mfma16x16x32(ld_global<bf16x8>(k0 + 32 * s), q8, s0);
-        s1 = mfma16x16x32(ld_global<bf16x8>(k1 + 32 * s), q8, s1);
+      if (it + 1 < mine) {
+        if (((it + 1) & 63) == 0) blks = ids_from(it + 1);
+        load_keys(__builtin_amdgcn_readlane(blks, (it + 1) & 63), ld);
+      }
+      float sv[8];
+      const bool far = EXT && p.rel && pos - (pg * kBS + kBS - 1) >= p.rel_len - 1;
+      float bv[8];
+      if (EXT && p.rel) bias_entries(bv, far, rel_far, relc, relg, rel_lds, p.rel_len, pos - pg * kBS - 4 * g);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = pg * kBS + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4));
+        const bool seen = c_ok && key <= pos && (pos - key < p.window || (EXT && key < p.keep_first));
+        float sc = (i < 4 ? s0[i] : s1[i - 4]) * scale2;
+        if (EXT && p.softcap > 0.f) sc = cap2 * tanh_fast(sc * cap_inv);
+        if (EXT && p.rel) sc += bv[i] * kLog2e;
+        sv[i] = seen ? sc : -INFINITY;
+      }
+      bf16x8 pf;
+      const float corr = softmax_step(sv, m, l, pf);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        f32x4 o = O[n];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] *= corr;
+        O[n] = mfma16x16x32(vf[n], pf, o);
       }
     }
-    if (it + 1 < mine) {
-      if (((it + 1) & 63) == 0) blks = ids_from(it + 1);
-      load_keys(__builtin_amdgcn_readlane(blks, (it + 1) & 63));
-    }
-    float sv[8];
-    const bool far = EXT && p.rel && pos - (pg * kBS + kBS - 1) >= p.rel_len - 1;
-    float bv[8];
-    if (EXT && p.rel) bias_entries(bv, far, rel_far, relc, relg, rel_lds, p.rel_len, pos - pg * kBS - 4 * g);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int key = pg * kBS + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4));
-      const bool seen = c_ok && key <= pos && (pos - key < p.window || (EXT && key < p.keep_first));
-      float sc = (i < 4 ? s0[i] : s1[i - 4]) * scale2;
-      if (p.softcap > 0.f) sc = cap2 * tanh_fast(sc * cap_inv);
-      if (EXT && p.rel) sc += bv[i] * kLog2e;
-      sv[i] = seen ? sc : -INFINITY;
-    }
-    bf16x8 pf;
-    const float corr = softmax_step(sv, m, l, pf);
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      f32x4 o = O[n];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] *= corr;
-      O[n] = mfma16x16x32(vf[n], pf, o);
-    }
-  }
+  };
+  if (__builtin_expect(past, 0))  // the allocating walk, that of few and short rows, in line
+    walk_pages([](const bf16* a) { return ld_once<bf16x8>(a); });
+  else
+    walk_pages([](const bf16* a) { return ld_global<bf16x8>(a); });
   const int ldm = V + 2;
   if (c_ok) {
     float* my = mg + (wave * cols + r) * ldm;
@@ -974,15 +993,20 @@ void launch_decode_waves(int num_work, const SinkAttnParams& p, const bf16* vt, 
     lds += cols * rel_lds * sizeof(float);
   }
   const int parts = p.nparts > 1 ? p.nparts : 1;
-  hipLaunchKernelGGL((sink_decode_kernel<NT, 4, NW, EXT>), dim3(num_work, p.G, (rep + 15) / 16 * parts), dim3(NW * 64), lds,
-                     st, p, vt, rel_lds);
+  auto go = [&](auto kd) {
+    hipLaunchKernelGGL((sink_decode_kernel<NT, decltype(kd)::value, NW, EXT>), dim3(num_work, p.G, (rep + 15) / 16 * parts),
+                       dim3(NW * 64), lds, st, p, vt, rel_lds);
+  };
+  constexpr int KD = NT % 2 == 0 && NT <= 8 ? NT / 2 : 0;  // keys as wide as the values: their k-steps at compile time
+  if (KD > 0 && p.D == p.V) go(std::integral_constant<int, KD>{});
+  else go(std::integral_constant<int, 0>{});
   if (parts > 1)
     hipLaunchKernelGGL(sink_combine_kernel, dim3((num_work * p.H + 3) / 4), dim3(256), 0, st, p, num_work);
 }
 
 template <int NT>
 void launch_decode(int num_work, const SinkAttnParams& p, const bf16* vt, hipStream_t st) {
-  const bool ext = p.rel || p.keep_first > 0;
+  const bool ext = p.rel || p.keep_first > 0 || p.softcap > 0.f;
   if (decode_lds(p, 8) <= kFlashLds) {
     if (ext) launch_decode_waves<NT, 8, true>(num_work, p, vt, st);
     else launch_decode_waves<NT, 8, false>(num_work, p, vt, st);

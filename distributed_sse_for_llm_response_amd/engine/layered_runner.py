@@ -134,6 +134,10 @@ from .weights import LayeredWeights
 
 ATTN_ROWS_TILE = 4    # query rows per work item of the row-wise attention kernel (prompt portions)
 FLASH_DECODE_WAVES = 512  # waves a decode attention launch aims for (two per CU)
+# Working set of a decode step, in bytes, up to which allocating loads of its pages pay: more than the 256 MB behind the L2s,
+# since part of the pages is still found there.  A byte of recurrent state, read and written back, counts half as much again.
+WALK_CACHED = 340e6
+WALK_STATE = 1.5
 SINK_DECODE_GROUPS = 512  # workgroups a decode launch of the sink attention aims for (two per CU)
 SINK_DECODE_PAGES = 32    # fewest pages of a full cache that a workgroup's stretch of a split walk is worth
 SINK_ROWS_TILE = 16   # query rows per work item of the sink attention's MFMA form (one head per wave)
@@ -161,6 +165,8 @@ class LayeredRunner(RunnerBase):
         self._tile_rows = []   # row counts of the shared-page sink attention's work items that this design's layers use
         self._plain_scans = []  # one row of the operands (q, k, v, channel decays or None) of each recurrence without the delta rule
         self._latents = set()  # (heads, rank, rotated width) of the latent attentions on the MFMA form
+        self.walked = torch.zeros(1, device=self.device, dtype=torch.int32)  # tokens of the live sequences (decode_prep)
+        self._slot_bytes = None  # bytes of one slot's recurrent states, counted by _walk_once
         self.num_blocks = num_blocks
         self.prenorm = getattr(cfg, "family", "") == "surodra"   # pre-norm blocks with matrix-state mixers
         self.multistream = getattr(cfg, "family", "") == "dironex"  # pre-norm blocks on several residual streams
@@ -618,7 +624,8 @@ class LayeredRunner(RunnerBase):
                                    Lw.sink, small[:, :H], ao, a.window, a.scale, rows, vt)
             elif vt is not None and ops.sink_decode_ok(self.dtype, H, G, D, V):  # decode rows: a group's heads side by side
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
-                                   g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, 1, vt)
+                                   g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, 1, vt,
+                                   walked=self.walked, once=self._walk_once(g["ws"].numel()))
             elif vt is not None and V <= ops.layers.SINK_SPLIT_MAX_V:  # tile 0, keys split over the waves
                 ops.sink_attention(qa, self.kv.k[ri], self.kv.v[ri], g["bt"], g["qs"], g["ql"], g["ctx"], g["ws"],
                                    g["wt"], Lw.sink, small[:, :H], ao, a.window, a.scale, SINK_ROWS_TILE, vt, True)
@@ -1187,7 +1194,20 @@ class LayeredRunner(RunnerBase):
             else:
                 work, form = (g["ws"], g["wt"]), (g["qt"], None, False)
             ops.sink_attention(qa, kc, vc, g["bt"], g["qs"], g["ql"], g["ctx"], *work, sink, gate, out, NO_WINDOW, a.scale,
-                               *form, out_scale=out_scale, part=self._walk_part if nparts > 1 else None, nparts=nparts)
+                               *form, out_scale=out_scale, part=self._walk_part if nparts > 1 else None, nparts=nparts,
+                               walked=self.walked, once=self._walk_once(g["ws"].numel()))
+
+    def _walk_once(self, rows: int) -> float:
+        """Bytes of pages that one layer's decode attention may walk and still find enough of them on the chip a step later:
+        its share of what the rows' states leave of it.  Beyond that the pages are read past the caches.  Both sides on one
+        MI355X, past the caches against allocating (us per step): six attention layers, states of 2 MB a row: 8 rows of 1500
+        tokens 731 / 714, 16 of 700 700 / 691, 16 of 500 675 / 649, but 16 of 2000 794 / 820, 32 of 500 742 / 769, 64 of 100
+        790 / 810, 64 of 500 925 / 965; two layers, states of 12.6 MB: 8 of 1500 608 / 586, 16 of 250 616 / 610, but 16 of 1000
+        649 / 670, 32 of 250 737 / 752."""
+        if self._slot_bytes is None:
+            caches = [getattr(self.state, k, {}) for k in ("state", "norm", "tail")]
+            self._slot_bytes = sum(t[0].numel() * t.element_size() for c in caches for t in c.values())
+        return max(1.0, (WALK_CACHED - rows * WALK_STATE * self._slot_bytes) / max(1, len(self.kv.k)))
 
     def _walk_parts(self, rows: int, a) -> int:
         """Workgroups that share a decode row's walk over all of its pages: as many as fill the chip, as long as each has
@@ -1383,7 +1403,7 @@ class LayeredRunner(RunnerBase):
         (q_len 0) write no cache row and touch no state."""
         r = slice(0, B)
         ops.decode_prep(self.active[r], self.positions[r], self.block_tables[r], self.slots[r], self.ctx_len[r],
-                        self.q_len[r], self.kv.num_blocks)
+                        self.q_len[r], self.kv.num_blocks, self.walked)
         rows = ("resid", "xb", "ym", "streams", "hn", "hc", "cat")
         d = {k: (v[:B] if k in rows and v is not None else v) for k, v in self._dec.items()}
         prev = (self.prev_ids[r], self.prev_ids[r], self.q_len[r]) if self.pair else None
@@ -1521,7 +1541,7 @@ class LayeredRunner(RunnerBase):
         M = B + T
         r = slice(0, B)
         ops.decode_prep(self.active[r], self.positions[r], self.block_tables[r], self.slots[r], self.ctx_len[r],
-                        self.q_len[r], self.kv.num_blocks)
+                        self.q_len[r], self.kv.num_blocks, self.walked)
         ids = torch.cat([self.ids[r], g["ids"]])
         pos = torch.cat([self.positions[r], g["pos"]])
         slots = torch.cat([self.slots[r], g["slots"]])

@@ -173,11 +173,13 @@ def silu_mul(gu, h):
         ref.silu_mul(gu, h)
 
 
-def decode_prep(active, positions, block_tables, slots, ctx_len, q_len, num_blocks: int = 2**31 - 1):
+def decode_prep(active, positions, block_tables, slots, ctx_len, q_len, num_blocks: int = 2**31 - 1, walked=None):
     if _hip(active):
-        torch.ops.dsse.decode_prep(active, positions, block_tables, slots, ctx_len, q_len, num_blocks)
+        torch.ops.dsse.decode_prep(active, positions, block_tables, slots, ctx_len, q_len, num_blocks, walked)
     else:
         ref.decode_prep(active, positions, block_tables, slots, ctx_len, q_len)
+        if walked is not None:
+            walked[0] = ctx_len[:active.numel()].sum()
 
 
 def ring_advance(counter):

@@ -278,7 +278,8 @@ def sink_flash_lds(dim: int) -> int:
 
 def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, work_seq, work_tile, sink, gate, out,
                    window: int, scale: float, qt: int, vt=None, split: bool = False, softcap: float = 0.0, out_rope=None,
-                   rel=None, keep_first: int = 0, out_scale: float = 1.0, part=None, nparts: int = 1):
+                   rel=None, keep_first: int = 0, out_scale: float = 1.0, part=None, nparts: int = 1,
+                   walked=None, once: float = 0.0):
     """Causal softmax attention of q [T, H, D] over paged keys [pages, 32, G, D] and values [pages, 32, G, V] (grouped
     heads), scores and weights in fp32; sink [H] adds exp(sink) to each head's denominator, gate [T, H] multiplies the
     head's output by its sigmoid.  `qt` query rows per work item (work_seq, work_tile).  With vt (transposed value
@@ -294,11 +295,13 @@ def sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, wor
     distances from N - 1 on) is added to the score.  keep_first: the sequence's first keep_first keys stay visible when the
     window has passed them.  A gate of H * V columns multiplies the heads element by element.  out (rows may be a column
     slice of a wider buffer) is multiplied by out_scale before it is rounded.  part (fp32, [work items, H, nparts, V + 2]):
-    the decode form splits each row's walk over nparts (at most 16) workgroups and joins them in a second launch."""
+    the decode form splits each row's walk over nparts (at most 16) workgroups and joins them in a second launch.  walked (int32
+    [1], the rows' tokens together) and once: with more bytes of pages than that the decode form reads them past the caches;
+    the result is the same."""
     if _hip(q):
         torch.ops.dsse.sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, work_seq, work_tile,
                                       sink, gate, out, window, scale, qt, vt, split, softcap, out_rope, rel, keep_first,
-                                      out_scale, part, nparts)
+                                      out_scale, part, nparts, walked, once)
     else:
         lref.sink_attention(q, kcache, vcache, block_tables, q_start, q_len, ctx_len, sink, gate, out, window, scale, vt,
                             softcap, out_rope, rel, keep_first, out_scale)
