@@ -116,6 +116,8 @@ struct SampleParams {
 extern "C" {
 hipError_t dsse_skinny_gemm(int mode, int mt, int nt, int kw, const void* X, int ldx, int M,
                             const void* W, int K, int N, const dsse::GemmEpi* ep, hipStream_t st);
+hipError_t dsse_norm_gemm(int mode, int kw, const float* resid, const void* norm_w, float eps, int M, const void* W, int K,
+                          int N, const dsse::GemmEpi* ep, hipStream_t st);
 hipError_t dsse_gemm_stream(int mode, int mt, int nt, int nw, int rd, int S, int partial_only, const void* X, int ldx, int M,
                             const void* W, int K, int N, const dsse::GemmEpi* ep, float* part, hipStream_t st);
 hipError_t dsse_gemm_ring(int mode, int nw, int S, int partial_only, int ring2, const void* X, int ldx, int M,

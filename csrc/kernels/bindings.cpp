@@ -791,9 +791,9 @@ void gated_gemm(const Tensor& x, const Tensor& w, Tensor& out, bool gelu) {
 void gemm_silu(const Tensor& x, const Tensor& w, Tensor& out) { gated_gemm(x, w, out, false); }
 void gemm_gelu(const Tensor& x, const Tensor& w, Tensor& out) { gated_gemm(x, w, out, true); }
 
-void gemm_qkv_rope(const Tensor& x, const Tensor& w, const Tensor& positions, const Tensor& slots,
-                   const Tensor& rope, Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh,
-                   int64_t nkv) {
+// Checks and epilogue of the QKV projection of x's rows
+dsse::GemmEpi qkv_epi(const Tensor& x, const Tensor& w, const Tensor& positions, const Tensor& slots, const Tensor& rope,
+                      Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh, int64_t nkv) {
   for (auto* t : {&positions, &slots, &rope}) check_gpu(*t, "metadata");
   check_gpu(q_out, "q_out");
   check_gpu(k_cache, "k_cache");
@@ -821,7 +821,71 @@ void gemm_qkv_rope(const Tensor& x, const Tensor& w, const Tensor& positions, co
   ep.nkv = (int)nkv;
   ep.num_slots = (int)(k_cache.size(0) * dsse::kBS);
   ep.rope_len = (int)rope.size(0);
+  return ep;
+}
+
+void gemm_qkv_rope(const Tensor& x, const Tensor& w, const Tensor& positions, const Tensor& slots,
+                   const Tensor& rope, Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh,
+                   int64_t nkv) {
+  dsse::GemmEpi ep = qkv_epi(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv);
   run_gemm(dsse::kQkvRope, x, w, ep);
+}
+
+// Products of RMS-normalised fp32 rows with the norm inside the launch (gemm_skinny.hip norm_gemm_kernel): up to four rows (32 KB
+// of them normalised, two rows of more than 4096), whole float4s of a row for every thread, and only where the plain product would take the skinny kernel with one column tile per wave.
+bool norm_gemm_ok(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || M > (K <= 4096 ? 4 : 2) || K < 1024 || K > 8192 || N < 16 || N % 16 || N * K * 2 >= (1LL << 31)) return false;
+  if (gemm_impl((int)M, (int)N, (int)K) != 0) return false;
+  int mt, nt, kw;
+  pick_tiles((int)M, (int)N, (int)K, dsse::kStoreF32, mt, nt, kw);
+  if (mt != 1 || nt != 1 || (kw != 4 && kw != 8) || K % (256 * kw)) return false;
+  const int64_t per = K / (256 * kw);
+  return kw == 4 ? per <= 3 : per >= 2 && per <= 4;
+}
+
+void run_norm_gemm(int mode, const Tensor& resid, const Tensor& norm_w, double eps, const Tensor& w, dsse::GemmEpi& ep) {
+  check_gpu(resid, "resid");
+  check_gpu(norm_w, "norm_w");
+  check_gpu(w, "w");
+  check_dtype(resid, at::kFloat, "resid");
+  check_dtype(norm_w, at::kBFloat16, "norm_w");
+  check_dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(resid.dim() == 2 && w.dim() == 2 && w.size(1) == resid.size(1) && norm_w.numel() == resid.size(1),
+              "resid [M, K], w [N, K], norm_w [K]");
+  TORCH_CHECK(norm_gemm_ok(resid.size(0), w.size(0), resid.size(1)), "no kernel for this product of normalised rows (norm_gemm_ok)");
+  for (const Tensor* t : {&resid, &norm_w, &w})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "operands must be 16-byte aligned");
+  int mt, nt, kw;
+  pick_tiles((int)resid.size(0), (int)w.size(0), (int)resid.size(1), mode, mt, nt, kw);
+  DSSE_CHECK_HIP(dsse_norm_gemm(mode, kw, resid.data_ptr<float>(), norm_w.data_ptr(), (float)eps, (int)resid.size(0), w.data_ptr(),
+                                (int)w.size(1), (int)w.size(0), &ep, cur_stream()));
+}
+
+void norm_gemm_out(const Tensor& resid, const Tensor& norm_w, double eps, const Tensor& w, Tensor& out) {
+  check_gpu(out, "out");
+  check_dtype(out, at::kFloat, "out");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == resid.size(0) && out.size(1) == w.size(0), "out must be [M, N]");
+  dsse::GemmEpi ep{};
+  ep.out = out.data_ptr();
+  ep.ldo = (int)out.size(1);
+  run_norm_gemm(dsse::kStoreF32, resid, norm_w, eps, w, ep);
+}
+
+void norm_gemm_silu(const Tensor& resid, const Tensor& norm_w, double eps, const Tensor& w, Tensor& out) {
+  check_gpu(out, "out");
+  check_dtype(out, at::kBFloat16, "out");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == resid.size(0) && out.size(1) * 2 == w.size(0), "out must be [M, N / 2]");
+  dsse::GemmEpi ep{};
+  ep.out = out.data_ptr();
+  ep.ldo = (int)out.size(1);
+  run_norm_gemm(dsse::kSiluMul, resid, norm_w, eps, w, ep);
+}
+
+void norm_gemm_qkv_rope(const Tensor& resid, const Tensor& norm_w, double eps, const Tensor& w, const Tensor& positions,
+                        const Tensor& slots, const Tensor& rope, Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh,
+                        int64_t nkv) {
+  dsse::GemmEpi ep = qkv_epi(resid, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv);
+  run_norm_gemm(dsse::kQkvRope, resid, norm_w, eps, w, ep);
 }
 
 void rmsnorm(Tensor& resid, const Tensor& w, Tensor& y, double eps, const c10::optional<Tensor>& delta,
@@ -1430,6 +1494,11 @@ TORCH_LIBRARY(dsse, m) {
   m.def("gemm_gelu(Tensor x, Tensor w, Tensor(a!) out) -> ()");
   m.def("gemm_qkv_rope(Tensor x, Tensor w, Tensor positions, Tensor slots, Tensor rope, Tensor(a!) q_out, "
         "Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv) -> ()");
+  m.def("norm_gemm_ok(int M, int N, int K) -> bool", &norm_gemm_ok);
+  m.def("norm_gemm_out(Tensor resid, Tensor norm_w, float eps, Tensor w, Tensor(a!) out) -> ()");
+  m.def("norm_gemm_silu(Tensor resid, Tensor norm_w, float eps, Tensor w, Tensor(a!) out) -> ()");
+  m.def("norm_gemm_qkv_rope(Tensor resid, Tensor norm_w, float eps, Tensor w, Tensor positions, Tensor slots, Tensor rope, "
+        "Tensor(a!) q_out, Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv) -> ()");
   m.def("rmsnorm(Tensor(a!) resid, Tensor w, Tensor(b!) y, float eps, Tensor? delta=None, Tensor? embed=None, "
         "Tensor? ids=None, Tensor? part=None, int nsplit=0) -> ()");
   m.def("gemm_resid_split(Tensor x, Tensor w, Tensor(a!) resid, Tensor(b!) part) -> int");
@@ -1483,6 +1552,9 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("gemm_out_parts", &gemm_out_parts);
   m.impl("gemm_out_split", &gemm_out_split);
   m.impl("gemm_silu", &gemm_silu);
+  m.impl("norm_gemm_out", &norm_gemm_out);
+  m.impl("norm_gemm_silu", &norm_gemm_silu);
+  m.impl("norm_gemm_qkv_rope", &norm_gemm_qkv_rope);
   m.impl("gemm_gelu", &gemm_gelu);
   m.impl("gemm_qkv_rope", &gemm_qkv_rope);
   m.impl("rmsnorm", &rmsnorm);

@@ -54,43 +54,12 @@ DEV void mma_chunk(f32x4 (&acc)[MT][NT], const bf16x8 (&wf)[NT][4], const bf16x8
       for (int t = 0; t < NT; ++t) acc[mt][t] = mfma16x16x32(xf[mt][s], wf[t][s], acc[mt][t]);
 }
 
+// The waves' sums of the K slices meet in wave 0, which applies the mode.
 template <int MT, int NT, int KW, int MODE>
-__global__ void __launch_bounds__(64 * KW)
-skinny_gemm_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restrict__ W, int K,
-                   int N, GemmEpi ep) {
+DEV void skinny_finish(f32x4 (&acc)[MT][NT], int M, int n0, const GemmEpi& ep) {
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT;
-
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const bf16* wp[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) wp[t] = W + (size_t)((n0 >> 4) + t) * (K >> 7) * kTileChunk + lane * 8;
-  const bf16* xp[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = min(16 * mt + r, M - 1);
-    xp[mt] = X + (size_t)m * ldx + 32 * g;
-  }
-
-  const int nchunks = K >> 7;
-  bf16x8 wa[NT][4], xa[MT][4], wb[NT][4], xb[MT][4];
-  int c = w;
-  if (c < nchunks) load_chunk<MT, NT>(wa, xa, wp, xp, c);
-  for (; c < nchunks; c += 2 * KW) {
-    if (c + KW < nchunks) load_chunk<MT, NT>(wb, xb, wp, xp, c + KW);
-    mma_chunk<MT, NT>(acc, wa, xa);
-    if (c + KW >= nchunks) break;
-    if (c + 2 * KW < nchunks) load_chunk<MT, NT>(wa, xa, wp, xp, c + 2 * KW);
-    mma_chunk<MT, NT>(acc, wb, xb);
-  }
-
   if constexpr (KW > 1) {
     __shared__ float red[KW - 1][MT * NT * 4][64];
     if (w > 0) {
@@ -168,6 +137,135 @@ skinny_gemm_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __res
 }
 
 template <int MT, int NT, int KW, int MODE>
+__global__ void __launch_bounds__(64 * KW)
+skinny_gemm_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restrict__ W, int K,
+                   int N, GemmEpi ep) {
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT;
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[mt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const bf16* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = W + (size_t)((n0 >> 4) + t) * (K >> 7) * kTileChunk + lane * 8;
+  const bf16* xp[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = min(16 * mt + r, M - 1);
+    xp[mt] = X + (size_t)m * ldx + 32 * g;
+  }
+
+  const int nchunks = K >> 7;
+  bf16x8 wa[NT][4], xa[MT][4], wb[NT][4], xb[MT][4];
+  int c = w;
+  if (c < nchunks) load_chunk<MT, NT>(wa, xa, wp, xp, c);
+  for (; c < nchunks; c += 2 * KW) {
+    if (c + KW < nchunks) load_chunk<MT, NT>(wb, xb, wp, xp, c + KW);
+    mma_chunk<MT, NT>(acc, wa, xa);
+    if (c + KW >= nchunks) break;
+    if (c + 2 * KW < nchunks) load_chunk<MT, NT>(wa, xa, wp, xp, c + 2 * KW);
+    mma_chunk<MT, NT>(acc, wb, xb);
+  }
+  skinny_finish<MT, NT, KW, MODE>(acc, M, n0, ep);
+}
+
+// The same product of RMS-normalised rows, for the few rows of a small decode step: every workgroup normalises the fp32 residual
+// rows itself, into LDS, while its first weights are under way, and a launch that did nothing else disappears.
+//
+// What bounds it: the weights, read once.  The rows come from L2 and are requested before the weights, since loads come back in
+// order; 256 KW elements divide a row, so a thread holds PER whole float4s of each.  Measured, 65 norms inside 32 layers of 4096
+// (qkv 6144, gate / up 28672 wide) and the head, the whole step: 1 row 3.00 -> 2.79 ms, 2 rows 3.06 -> 2.83, 3 rows 3.12 -> 2.92,
+// 4 rows 3.17 -> 3.06: a workgroup's own norm work grows with the rows, the launch it saves does not.  With rows and steps counted at
+// run time (sums per step, divisions, predicated loads) 1 row took 2.88 ms and 4 rows 3.60.
+template <int KW, int PER, int ROWS, int MODE>
+__global__ void __launch_bounds__(64 * KW)
+norm_gemm_kernel(const float* __restrict__ resid, const bf16* __restrict__ norm_w, float eps, const bf16* __restrict__ W, GemmEpi ep) {
+  constexpr int kStep = 256 * KW, K = PER * kStep, kChunks = K >> 7;
+  __shared__ __attribute__((aligned(16))) bf16 rows[ROWS][K];
+  __shared__ float sums[ROWS][KW];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4;
+  f32x4 v[ROWS][PER];
+  bf16x4 nw[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) v[m][i] = ld_global<f32x4>(resid + m * K + i * kStep + 4 * tid);
+    nw[i] = ld_global<bf16x4>(norm_w + i * kStep + 4 * tid);
+  }
+  const bf16* wp = W + (size_t)blockIdx.x * kChunks * kTileChunk + lane * 8;
+  bf16x8 wa[4], wb[4];
+  auto load_w = [&](bf16x8 (&wf)[4], int c) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) wf[s] = ld_once<bf16x8>(wp + (size_t)c * kTileChunk + 512 * s);
+  };
+  static_assert(kChunks >= 2 * KW, "two chunks for every wave");
+  load_w(wa, w);
+  load_w(wb, w + KW);
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    f32x4 sq = v[m][0] * v[m][0];
+#pragma unroll
+    for (int i = 1; i < PER; ++i) sq += v[m][i] * v[m][i];
+    const float ss = wave_sum((sq[0] + sq[1]) + (sq[2] + sq[3]));
+    if (lane == 0) sums[m][w] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    float tot = 0.f;
+#pragma unroll
+    for (int u = 0; u < KW; ++u) tot += sums[m][u];
+    const float inv = rsqrtf(tot / (float)K + eps);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = f2bf(v[m][i][e] * inv * bf2f(nw[i][e]));
+      *reinterpret_cast<bf16x4*>(&rows[m][i * kStep + 4 * tid]) = o;
+    }
+  }
+  __syncthreads();
+  const bf16* xp = &rows[min(r, ROWS - 1)][32 * g];
+  f32x4 acc[1][1] = {{f32x4{0.f, 0.f, 0.f, 0.f}}};
+  auto mma = [&](const bf16x8 (&wf)[4], int c) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      acc[0][0] = mfma16x16x32(*reinterpret_cast<const bf16x8*>(xp + (c << 7) + 8 * s), wf[s], acc[0][0]);
+  };
+#pragma unroll
+  for (int c = 0; c < kChunks / KW; c += 2) {  // the wave's chunks w, w + KW, ..: two per 256 KW elements of a row
+    mma(wa, w + c * KW);
+    if (c + 2 < kChunks / KW) load_w(wa, w + (c + 2) * KW);
+    mma(wb, w + (c + 1) * KW);
+    if (c + 3 < kChunks / KW) load_w(wb, w + (c + 3) * KW);
+  }
+  skinny_finish<1, 1, KW, MODE>(acc, ROWS, blockIdx.x * 16, ep);
+}
+
+template <int MODE>
+static hipError_t launch_norm(int kw, const float* resid, const bf16* nw, float eps, int M, const bf16* W, int K, int N,
+                              const GemmEpi& ep, hipStream_t st) {
+#define NORM_CASE(KW_, PER_, ROWS_)                                                                                               \
+  if (kw == KW_ && K == 256 * KW_ * PER_ && M == ROWS_) {                                                                         \
+    hipLaunchKernelGGL((norm_gemm_kernel<KW_, PER_, ROWS_, MODE>), dim3(N / 16), dim3(64 * KW_), 0, st, resid, nw, eps, W, ep); \
+    return hipGetLastError();                                                                                                     \
+  }
+#define NORM_ROWS(KW_, PER_) NORM_CASE(KW_, PER_, 1) NORM_CASE(KW_, PER_, 2)
+#define NORM_FOUR(KW_, PER_) NORM_ROWS(KW_, PER_) NORM_CASE(KW_, PER_, 3) NORM_CASE(KW_, PER_, 4)
+  NORM_FOUR(4, 1) NORM_FOUR(4, 2) NORM_FOUR(4, 3) NORM_FOUR(8, 2) NORM_ROWS(8, 3) NORM_ROWS(8, 4)
+#undef NORM_FOUR
+#undef NORM_ROWS
+#undef NORM_CASE
+  return hipErrorInvalidValue;
+}
+
+template <int MT, int NT, int KW, int MODE>
 static hipError_t launch_t(const bf16* X, int ldx, int M, const bf16* W, int K, int N,
                            const GemmEpi& ep, hipStream_t st) {
   dim3 grid(N / (16 * NT)), block(64 * KW);
@@ -207,6 +305,20 @@ extern "C" hipError_t dsse_skinny_gemm(int mode, int mt, int nt, int kw, const v
     case kResidAdd: return launch_mode<kResidAdd>(mt, nt, kw, x, ldx, M, w, K, N, *ep, st);
     case kSiluMul: return launch_mode<kSiluMul>(mt, nt, kw, x, ldx, M, w, K, N, *ep, st);
     case kQkvRope: return launch_mode<kQkvRope>(mt, nt, kw, x, ldx, M, w, K, N, *ep, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+// norm_gemm_kernel: M rows of K contiguous floats; M and K as launch_norm lists, N % 16 == 0
+extern "C" hipError_t dsse_norm_gemm(int mode, int kw, const float* resid, const void* norm_w, float eps, int M, const void* W,
+                                     int K, int N, const dsse::GemmEpi* ep, hipStream_t st) {
+  using namespace dsse;
+  const bf16* nw = reinterpret_cast<const bf16*>(norm_w);
+  const bf16* w = reinterpret_cast<const bf16*>(W);
+  switch (mode) {
+    case kStoreF32: return launch_norm<kStoreF32>(kw, resid, nw, eps, M, w, K, N, *ep, st);
+    case kSiluMul: return launch_norm<kSiluMul>(kw, resid, nw, eps, M, w, K, N, *ep, st);
+    case kQkvRope: return launch_norm<kQkvRope>(kw, resid, nw, eps, M, w, K, N, *ep, st);
   }
   return hipErrorInvalidValue;
 }

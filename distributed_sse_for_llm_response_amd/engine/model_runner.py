@@ -418,6 +418,22 @@ class ModelRunner(RunnerBase):
         if B > DECODE_GEMM_MAX_M:
             self._decode_layers_wide(B, resid, x, part, nparts)
             return
+        if self._norms_inside(B):
+            # a few rows: the projections normalise the residual rows themselves, no norm launches
+            for li, L in enumerate(w.layers):
+                kc, vc = self.kv.k[li], self.kv.v[li]
+                ops.norm_gemm_qkv_rope(resid, L.attn_norm, eps, L.wqkv_t, self.positions[r], self.slots[r], self.rope,
+                                       self.q[r], kc, vc, nh, nkv)
+                ops.paged_attention(0, self.q[r].view(B, nh, 128), kc, vc, self.block_tables[r], self.q_start[r],
+                                    self.q_len[r], self.ctx_len[r], self.work_seq[r], self.work_tile[r],
+                                    self.attn[r].view(B, nh, 128), self.part_o, self.part_ml, part, nparts)
+                ops.gemm_resid(self.attn[r], L.wo_t, resid)
+                ops.norm_gemm_silu(resid, L.ffn_norm, eps, L.wgu_t, self.h[r])
+                ops.gemm_resid(self.h[r], L.wd_t, resid)
+            ops.norm_gemm_out(resid, w.final_norm, eps, w.lm_head_t, self.logits[r])
+            self._sample_commit(B)
+            ops.ring_advance(self.ring_counter)
+            return
         for li, L in enumerate(w.layers):
             self._qkv_attention(li, L, B, x, part, nparts)
             self._resid_proj(self.attn[r], L.wo_t, resid, L.ffn_norm, x, self.tmp[r])
@@ -427,6 +443,15 @@ class ModelRunner(RunnerBase):
         ops.gemm_out(x, w.lm_head_t, self.logits[r])
         self._sample_commit(B)
         ops.ring_advance(self.ring_counter)
+
+    def _norms_inside(self, B: int) -> bool:
+        """Whether a decode step of B rows runs its norms inside the projections that read them (one rank: across ranks
+        the norm follows the all-reduce)."""
+        w = self.w
+        if self.comm.size > 1 or self.device.type != "cuda":
+            return False
+        L = w.layers[0]
+        return all(ops.norm_gemm_ok(B, t.shape[0], self.cfg.hidden_size) for t in (L.wqkv_t, L.wgu_t, w.lm_head_t))
 
     def _decode_layers_wide(self, B: int, resid, x, part: int, nparts: int) -> None:
         """Decode step for buckets above DECODE_GEMM_MAX_M sequences (256 streams per GPU).

@@ -101,6 +101,36 @@ def gemm_qkv_rope(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv
         ref.gemm_qkv_rope(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
 
 
+def norm_gemm_ok(M: int, N: int, K: int) -> bool:
+    """Whether M normalised rows times a weight [N, K] run as one launch (the norm_gemm ops)."""
+    load_library(required=True)
+    return bool(torch.ops.dsse.norm_gemm_ok(M, N, K))
+
+
+def norm_gemm_out(resid, norm_w, eps, w, out):
+    """gemm_out of rmsnorm(resid) * norm_w: fp32 resid [M, K], fp32 out; the norm runs inside the launch."""
+    if _hip(resid):
+        torch.ops.dsse.norm_gemm_out(resid, norm_w, eps, w, out)
+    else:
+        ref.gemm_out(ref.normed(resid, norm_w, eps), w, out)
+
+
+def norm_gemm_silu(resid, norm_w, eps, w, out):
+    """gemm_silu of rmsnorm(resid) * norm_w, likewise."""
+    if _hip(resid):
+        torch.ops.dsse.norm_gemm_silu(resid, norm_w, eps, w, out)
+    else:
+        ref.gemm_silu(ref.normed(resid, norm_w, eps), w, out)
+
+
+def norm_gemm_qkv_rope(resid, norm_w, eps, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv):
+    """gemm_qkv_rope of rmsnorm(resid) * norm_w, likewise."""
+    if _hip(resid):
+        torch.ops.dsse.norm_gemm_qkv_rope(resid, norm_w, eps, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
+    else:
+        ref.gemm_qkv_rope(ref.normed(resid, norm_w, eps), w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
+
+
 def gemm_resid_split(x, w, resid, part) -> int:
     """resid += x · wᵀ, or (when the X-in-LDS kernel splits K) write fp32 slabs [S, M, N] into `part`
     and return S so the following rmsnorm(part=..., nsplit=S) folds the reduction into the norm."""

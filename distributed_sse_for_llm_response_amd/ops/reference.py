@@ -155,6 +155,12 @@ def rmsnorm(resid, w, y, eps, delta=None, embed=None, ids=None, part=None, nspli
     y.copy_((r * torch.rsqrt(r.pow(2).mean(-1, keepdim=True) + eps) * w.float()).to(y.dtype))
 
 
+def normed(resid, w, eps):
+    y = torch.empty(resid.shape, dtype=torch.bfloat16, device=resid.device)
+    rmsnorm(resid, w, y, eps)
+    return y
+
+
 def decode_prep(active, positions, block_tables, slots, ctx_len, q_len, num_blocks: int = 2**31 - 1):
     B = active.numel()
     for b in range(B):
