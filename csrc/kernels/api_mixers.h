@@ -49,6 +49,8 @@ struct NormRopeList {
   static constexpr int kMost = 3;
   NormRopeParams p[kMost];
   int gy[kMost];         // workgroups per row (set by the launch)
+  bool fours[kMost];     // four numbers per lane, pages of 32 rows (both set by the launch)
+  bool pages[kMost];
   int n;
 };
 

@@ -149,6 +149,119 @@ DEV void norm_rope_row(const NormRopeParams& p, int gy, float* strips, float* re
   }
 }
 
+// The same with four neighbouring numbers to a lane: a head of 4 n numbers is n lanes, a wave takes 64 / n heads, sums and rotation
+// partners (half / 4 lanes away) come from shuffles; no strips, no barriers.  norm_rope_fours() says which sets it takes.  1500
+// rows, by ones / by fours: unit q and k of 8 heads of 128 9.8 / 7.3 us, rotation of 16 and 16 heads in place 15.1 / 8.7, row-normed
+// and rotated q and k with v (16, 8, 8 heads) 17.7 / 12.3; 300 rows 8.1 / 4.8.
+template <typename OutT>
+DEV void norm_rope_fours_row(const NormRopeParams& p, int gy, float* red) {
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int n = p.D >> 2, e = 4 * (lane & (n - 1)), hpw = 64 / n, N = p.nh * p.D;
+  const float* x = p.x + (int64_t)row * p.ldx;
+  float inv_row = 1.0f;
+  if (p.kind == 1) {
+    f32x4 sq{0.f, 0.f, 0.f, 0.f};
+    for (int d = 4 * threadIdx.x; d < N; d += 4 * blockDim.x) {
+      const f32x4 v = ld4(x + d);
+      sq += v * v;
+    }
+    inv_row = 1.0f / sqrtf(block_sum256((sq[0] + sq[1]) + (sq[2] + sq[3]), red) / (float)N + p.eps);
+  }
+  const int orow = p.out_rows ? p.out_rows[row] : row;
+  if (orow < 0 || orow >= p.num_out_rows) return;  // uniform for the workgroup; after the only block-wide barrier
+  OutT* out = reinterpret_cast<OutT*>(p.out) + (int64_t)orow * p.ldo;
+  const int dims = p.rope ? 2 * p.half : 0;
+  f32x4 cs0{1.f, 0.f, 1.f, 0.f}, cs1 = cs0;  // (cos, sin) of the lane's four numbers
+  float side = 0.f;                          // how their partners enter: v cos + side * partner sin
+  if (e < dims) {
+    int pos = p.positions[row];
+    pos = pos < 0 ? 0 : (pos >= p.rope_len ? p.rope_len - 1 : pos);
+    const float* c = reinterpret_cast<const float*>(p.rope + (int64_t)pos * p.half + (e < p.half ? e : e - p.half));
+    cs0 = ld4(c), cs1 = ld4(c + 4);
+    side = e < p.half ? -1.f : 1.f;
+  }
+  f32x4 w{1.f, 1.f, 1.f, 1.f};
+  if (p.kind == 3 && p.norm_w) w = ld4(p.norm_w + e);
+  for (int h0 = nw * hpw * blockIdx.y; h0 < p.nh; h0 += nw * hpw * gy) {
+    const int h = h0 + wave * hpw + lane / n;
+    const bool on = h < p.nh;
+    f32x4 v = ld4(x + (on ? h : 0) * p.D + e);
+    float inv = inv_row;
+    if (p.kind >= 2) {
+      float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+      for (int o = n >> 1; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+      inv = 1.0f / sqrtf((p.kind == 3 ? ss / (float)p.D : ss) + p.eps);
+    } else if (p.kind == 1) {
+      w = ld4(p.norm_w + (on ? h : 0) * p.D + e);
+    }
+    v = v * inv * w;
+    if (dims) {
+      f32x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = side * __shfl_xor(v[i], p.half >> 2);
+      v = f32x4{v[0] * cs0[0] + o[0] * cs0[1], v[1] * cs0[2] + o[1] * cs0[3], v[2] * cs1[0] + o[2] * cs1[1], v[3] * cs1[2] + o[3] * cs1[3]};
+    }
+    v = v * p.scale;
+    if (!on) continue;
+    st4(out + h * p.D + e, v);
+    if (p.out_t) {  // the same numbers once more where the MFMA attention's value operand wants them
+      const int page = orow / kBS, off = orow % kBS;
+      const int at = ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4 + (off & 3);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        reinterpret_cast<OutT*>(p.out_t)[(((int64_t)page * p.nh + h) * p.D + e + i) * kBS + at] = (OutT)v[i];
+    }
+  }
+}
+
+// Values on their way into pages and transposed pages: a workgroup takes 32 rows of one head, so that a whole page's 64-byte pieces
+// of the transposed one (a value's 32 tokens) are written by one thread each -- by token they are 2-byte writes from 32 workgroups
+// behind eight L2s: 1500 rows of 8 heads of 128 12.8 -> 6.3 us, beside queries and keys 19.9 -> 14.3.  Rows that make no whole page
+// in order go by token.  items: (32 rows, head) pairs, counted over the workgroups of the set.
+DEV void value_pages(const NormRopeParams& p, int item, bf16* tile) {
+  const int n = p.D >> 2, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ldt = p.D + 4;
+  const int t0 = item / p.nh * kBS, h = item % p.nh, rows = p.T - t0 < kBS ? p.T - t0 : kBS;
+  const int mine = (lane & 31) < rows ? p.out_rows[t0 + (lane & 31)] : -1;
+  const int slot = mine >= 0 && mine < p.num_out_rows ? mine : -1;  // of row lane & 31
+  const int first = __shfl(slot, 0);
+  const bool whole = rows == kBS && first >= 0 && first % kBS == 0 && __all(slot == first + (lane & 31));
+  const int rpp = 256 / n, e = 4 * (threadIdx.x & (n - 1));  // rows of a pass of the workgroup
+  for (int r = threadIdx.x / n; r < kBS; r += rpp) {
+    const int s = __shfl(slot, r);
+    if (r >= rows) continue;
+    const f32x4 v = ld4(p.x + (int64_t)(t0 + r) * p.ldx + h * p.D + e) * p.scale;
+    const bf16x4 b{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+    *reinterpret_cast<bf16x4*>(tile + r * ldt + e) = b;
+    if (s >= 0) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(p.out) + (int64_t)s * p.ldo + h * p.D + e) = b;
+  }
+  __syncthreads();
+  bf16* pages = reinterpret_cast<bf16*>(p.out_t);
+  if (whole) {
+    bf16* dst = pages + ((int64_t)(first / kBS) * p.nh + h) * p.D * kBS;
+    for (int i = threadIdx.x; i < 4 * p.D; i += 256) {  // (value, 8 places): tokens 4 q .. + 3 and 16 + 4 q .. + 3
+      const int d = i >> 2, q = i & 3;
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = tile[(4 * q + (j & 3) + 16 * (j >> 2)) * ldt + d];
+      *reinterpret_cast<bf16x8*>(dst + (int64_t)d * kBS + 8 * q) = o;
+    }
+    return;
+  }
+  for (int r = wave; r < rows; r += 4) {
+    const int s = __builtin_amdgcn_readlane(slot, r);
+    if (s < 0) continue;
+    const int page = s / kBS, off = s % kBS, at = ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4 + (off & 3);
+    for (int d = lane; d < p.D; d += 64) pages[(((int64_t)page * p.nh + h) * p.D + d) * kBS + at] = tile[r * ldt + d];
+  }
+}
+
+// Heads of 32, 64, 128 or 256 numbers in 16-byte pieces, rotation partners a power of two of lanes apart
+inline bool norm_rope_fours(const NormRopeParams& p) {
+  auto power = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
+  return p.D % 32 == 0 && p.D <= 256 && power(p.D) && p.ldx % 4 == 0 && p.ldo % 4 == 0 && fours({p.x, p.out, p.norm_w, p.rope}) &&
+         (!p.rope || (p.half % 4 == 0 && power(p.half / 4) && 2 * p.half <= p.D));
+}
+
 // A layer's queries, keys and values (blockIdx.z) in one launch.  What bounds it in a decode step: the launch, 4 to 5 us whatever it
 // moves.  Surodra-wide, 16 rows, ten launches fewer (two of them gates): 703 -> 678 us; 1500 prompt rows of surodra-mid 1813 -> 1792.
 template <int WAVES>
@@ -158,6 +271,16 @@ __global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopeList
   const NormRopeParams& p = l.p[blockIdx.z];
   const int gy = l.gy[blockIdx.z];
   if ((int)blockIdx.y >= gy) return;  // uniform: another set's share of the grid
+  if (l.pages[blockIdx.z]) {
+    const int item = blockIdx.y * gridDim.x + blockIdx.x;
+    if (item < (p.T + kBS - 1) / kBS * p.nh) value_pages(p, item, reinterpret_cast<bf16*>(strips));
+    return;
+  }
+  if (l.fours[blockIdx.z]) {
+    if (p.out_f32) norm_rope_fours_row<float>(p, gy, red);
+    else norm_rope_fours_row<bf16>(p, gy, red);
+    return;
+  }
   if (p.out_f32) norm_rope_row<float, WAVES>(p, gy, strips, red);
   else norm_rope_row<bf16, WAVES>(p, gy, strips, red);
 }
@@ -198,6 +321,27 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* o, co
   for (int i = lane; i < V; i += 64) ss += oh[i] * oh[i];
   const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)V + eps);
   for (int i = lane; i < V; i += 64) dst[i] = (T)(oh[i] * inv * (w ? w[i] : 1.0f) * (gate_kind == 1 ? sigmoid_f(g[i]) : silu_f(g[i])));
+}
+
+// The same for heads of 32, 64, 128 or 256 values, V / 4 lanes each: 16-byte pieces, 256 / V heads to a wave (1500 rows of 16 heads of
+// 128: 10.4 -> 7.7 us)
+template <typename T>
+__global__ __launch_bounds__(256) void gated_head_norm_fours_kernel(const float* o, const float* w, const float* gate, int ldg, T* out,
+                                                                    int64_t items, int H, int V, float eps, int gate_kind) {
+  const int n = V >> 2, e = 4 * (threadIdx.x & (n - 1));
+  const int64_t item = (int64_t)blockIdx.x * (256 / n) + threadIdx.x / n;  // (row, head)
+  if (item >= items) return;  // whole heads: the lanes of a head leave together
+  const int64_t row = item / H;
+  const f32x4 v = ld4(o + item * V + e), g = ld4(gate + row * ldg + (item - row * H) * V + e);
+  f32x4 k{1.f, 1.f, 1.f, 1.f};
+  if (w) k = ld4(w + e);
+  float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+  for (int x = n >> 1; x >= 1; x >>= 1) ss += __shfl_xor(ss, x);
+  const float inv = 1.0f / sqrtf(ss / (float)V + eps);
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = v[i] * inv * k[i] * (gate_kind == 1 ? sigmoid_f(g[i]) : silu_f(g[i]));
+  st4(out + item * V + e, r);
 }
 
 __global__ __launch_bounds__(256) void rms_mix_kernel(const float* ya, int na, const float* wa, const float* yb, int nb, const float* wb,
@@ -302,25 +446,34 @@ extern "C" hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st) 
   for (int i = 0; i < l.n; ++i) {
     const dsse::NormRopeParams& p = l.p[i];
     if (p.T != l.p[0].T || p.D > dsse::kMaxHeadDim) return hipErrorInvalidValue;
-    if (p.kind == 1 && p.T <= 512 && p.nh > 4) waves = std::max(waves, std::min(p.nh, 16));
-    width = std::max(width, p.D);
+    l.fours[i] = dsse::norm_rope_fours(p);
+    // a row's workgroup of up to 16 waves; in fours 96 rows of 16 heads take 4.7 us with four waves and 5.5 with 16, 64 rows 4.6 / 4.5
+    if (p.kind == 1 && p.T <= (l.fours[i] ? 64 : 512) && p.nh > 4) waves = std::max(waves, std::min(p.nh, 16));
+    if (!l.fours[i]) width = std::max(width, p.D);
   }
   const int T = l.p[0].T;
   if (T <= 0) return hipSuccess;
-  // four heads to a workgroup while the rows alone leave the chip idle, then more of them: a workgroup's start (lengths, places,
+  size_t lds = 0;
+  // one walk of the heads per workgroup while the rows alone leave the chip idle, then more of them: a workgroup's start (lengths, places,
   // position) costs as much as a group of narrow heads.  One group / all groups per workgroup / this rule, rows x heads x width:
   // 512 x 32 x 64 normed in place 8.4 / 11.4 / 8.2 us, 1000 x 32 x 128 15.3 / 17.5 / 14.7; rotated into bf16, 4096 x 16 x 64
   // 16.8 / 11.2 / 11.4, 4096 x 64 x 64 54.1 / 33.7 / 35.5, 1500 x 32 x 128 16.7 / 15.6 / 16.1.
   const int each = T <= 512 ? 1 : (T < 1500 ? 2 : (T < 3000 ? 4 : 8));
   for (int i = 0; i < l.n; ++i) {
     const dsse::NormRopeParams& p = l.p[i];
-    const int groups = (p.nh + waves - 1) / waves;
+    const int heads = waves * (l.fours[i] ? 256 / p.D : 1), groups = (p.nh + heads - 1) / heads;  // of one walk
     l.gy[i] = p.nh <= 0 ? 0 : (p.kind == 1 ? 1 : std::min((groups + each - 1) / each, 65535));
+    // from 128 rows on: with fewer they are decode rows, each in a page of its own
+    l.pages[i] = waves == 4 && l.fours[i] && p.out_t && dsse::fours({p.out_t}) && p.out_rows && !p.out_f32 && p.kind == 0 && !p.rope && p.nh > 0 && T >= 128;
+    if (l.pages[i]) {
+      l.gy[i] = (int)(((int64_t)((T + dsse::kBS - 1) / dsse::kBS) * p.nh + T - 1) / T);
+      lds = std::max(lds, (size_t)dsse::kBS * (p.D + 4) * sizeof(bf16));
+    }
     most = std::max(most, l.gy[i]);
   }
   if (most <= 0) return hipSuccess;
   const dim3 grid(T, most, l.n);
-  const size_t lds = (size_t)waves * width * sizeof(float);
+  lds = std::max(lds, (size_t)waves * width * sizeof(float));
   if (waves == 4) hipLaunchKernelGGL(dsse::norm_rope_rows_kernel<4>, grid, dim3(256), lds, st, l);
   else hipLaunchKernelGGL(dsse::norm_rope_rows_kernel<16>, grid, dim3(64 * waves), lds, st, l);
   return hipGetLastError();
@@ -338,6 +491,17 @@ extern "C" hipError_t dsse_gate_math(float* x, int ld, int M, int N, int kind, c
 extern "C" hipError_t dsse_gated_head_norm(const float* o, const float* w, const float* gate, int ldg, void* out, int M,
                                            int H, int V, float eps, int gate_kind, int f32, hipStream_t st) {
   if (M <= 0 || H <= 0) return hipSuccess;
+  if (V % 32 == 0 && V <= 256 && (V & (V - 1)) == 0 && ldg % 4 == 0 && dsse::fours({o, w, gate, out})) {
+    const int64_t items = (int64_t)M * H, heads = 1024 / V;
+    const dim3 grid((unsigned)((items + heads - 1) / heads));
+    if (f32)
+      hipLaunchKernelGGL(dsse::gated_head_norm_fours_kernel<float>, grid, dim3(256), 0, st, o, w, gate, ldg,
+                         reinterpret_cast<float*>(out), items, H, V, eps, gate_kind);
+    else
+      hipLaunchKernelGGL(dsse::gated_head_norm_fours_kernel<bf16>, grid, dim3(256), 0, st, o, w, gate, ldg,
+                         reinterpret_cast<bf16*>(out), items, H, V, eps, gate_kind);
+    return hipGetLastError();
+  }
   const int blocks = (int)(((int64_t)M * H + 3) / 4);
   if (f32)
     hipLaunchKernelGGL(dsse::gated_head_norm_kernel<float>, dim3(blocks), dim3(256), 0, st, o, w, gate, ldg,

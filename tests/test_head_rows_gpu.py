@@ -1,0 +1,80 @@
+"""Heads in pieces of four numbers: norms and rotations with a head's lanes side by side, values written page by page, gated head
+norms -- at the narrowest and widest heads of that form, more heads than a walk takes, partial rotations, rows that make whole pages
+and rows that do not."""
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.ops import layers_reference as lref
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-5
+PAGE = 32
+
+
+def c(t):
+    return None if t is None else t.cuda()
+
+
+def near(got, want, steps):
+    """Within `steps` roundings of the result's type of the largest value."""
+    unit = 2.0 ** -9 if got.dtype == torch.bfloat16 else 2.0 ** -24
+    assert (got.cpu().double() - want.double()).abs().max() <= steps * unit * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("T,nh,D,half", [(1, 1, 32, 4), (3, 9, 32, 16), (65, 16, 128, 64), (64, 5, 64, 8), (700, 3, 256, 128), (130, 33, 64, 0)])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_heads_in_fours(T, nh, D, half, kind, dtype):
+    g = torch.Generator().manual_seed(T + D)
+    wide = torch.randn(T, nh * D + 8, generator=g)
+    w = torch.randn(nh * D if kind == 1 else D, generator=g) if kind in (1, 3) else None
+    rope = torch.randn(11, half, 2, generator=g) if half else None
+    pos = torch.randint(-1, 13, (T,), generator=g, dtype=torch.int32)  # clamped into the table
+    steps = nh * D / 256 + 24  # a row's squares in sequence, the root, a rotation
+    want, got = torch.zeros(T, nh, D, dtype=dtype), torch.zeros(T, nh, D, dtype=dtype, device="cuda")
+    view = lambda t: t[:, 4:4 + nh * D].unflatten(1, (nh, D))  # noqa: E731
+    lref.norm_rope_rows(view(wide), w, pos, rope, want, None, kind, EPS, 0.7)
+    dev = c(wide)
+    ops.norm_rope_rows(view(dev), c(w), c(pos), c(rope), got, None, kind, EPS, 0.7)
+    near(got, want, 2 if dtype == torch.bfloat16 else steps)
+    if dtype == torch.float32:  # in place: nothing beside the heads changes
+        ops.norm_rope_rows(view(dev), c(w), c(pos), c(rope), view(dev), None, kind, EPS, 0.7)
+        near(view(dev), want, steps)
+        assert torch.equal(dev[:, :4].cpu(), wide[:, :4]) and torch.equal(dev[:, -4:].cpu(), wide[:, -4:])
+
+
+@pytest.mark.parametrize("nh,D", [(1, 32), (3, 64), (8, 128), (2, 256)])
+@pytest.mark.parametrize("T", [127, 128, 200])
+def test_values_page_by_page(nh, D, T):
+    """Rows 0-31 a whole page, 32-63 the same shifted by a token, then one page backwards, skipped and out-of-range rows, a rest."""
+    g = torch.Generator().manual_seed(nh * D + T)
+    rows = torch.full((T,), -1, dtype=torch.int32)
+    rows[:32] = torch.arange(32) + 2 * PAGE
+    rows[32:63] = torch.arange(31) + 3 * PAGE + 1
+    rows[63] = 4 * PAGE + 5
+    rows[64:96] = torch.arange(31, -1, -1) + 5 * PAGE
+    rows[100:T] = torch.arange(T - 100) + 6 * PAGE + (7 if T < 128 else 0)
+    x = torch.randn(T, nh, D, generator=g)
+    pos = torch.zeros(T, dtype=torch.int32)
+    pages = int(rows.max()) // PAGE + 2
+    out, out_t = torch.full((pages, PAGE, nh, D), 7.0).to(torch.bfloat16), torch.full((pages, nh, D, PAGE), 7.0).to(torch.bfloat16)
+    rows[97] = pages * PAGE + 3
+    assert rows[rows >= 0].unique().numel() == int((rows >= 0).sum())
+    got, got_t = c(out.clone()), c(out_t.clone())
+    lref.norm_rope_rows(x, None, pos, None, out, rows, 0, 0.0, 1.0, out_t)
+    ops.norm_rope_rows(c(x), None, c(pos), None, got, c(rows), 0, 0.0, 1.0, got_t)
+    assert torch.equal(got.cpu(), out) and torch.equal(got_t.cpu(), out_t)
+
+
+@pytest.mark.parametrize("M,H,V", [(1, 1, 32), (5, 3, 64), (33, 7, 128), (2, 5, 256)])
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gated_heads_in_fours(M, H, V, kind, dtype):
+    g = torch.Generator().manual_seed(M + V)
+    o, wide = torch.randn(M, H, V, generator=g), torch.randn(M, H * V + 8, generator=g)
+    for w in (torch.randn(V, generator=g), None):
+        want, got = torch.zeros(M, H * V, dtype=dtype), torch.zeros(M, H * V, dtype=dtype, device="cuda")
+        lref.gated_head_norm(o, w, wide[:, 4:4 + H * V], EPS, want, kind)
+        ops.gated_head_norm(c(o), c(w), c(wide)[:, 4:4 + H * V], EPS, got, kind)
+        near(got, want, 2 if dtype == torch.bfloat16 else 30)  # 32-256 squares, a root, an exponential, four products
