@@ -42,6 +42,7 @@ struct NormRopeParams {
                          // norm_w [D] (one gain vector for all heads)
   float eps, scale;
   int out_f32;
+  const float* bias;     // [nh * D], added before everything else, or null (dsse_norm_rope_all_fours only)
 };
 
 // Up to three sets of heads of the same rows in one launch: none reads or writes what another writes (each may work in place)
@@ -255,6 +256,7 @@ hipError_t dsse_moe_route(const float* z, int ldz, const float* corr, int M, int
 hipError_t dsse_stream_step(const dsse::StreamStepParams* p, hipStream_t st);
 hipError_t dsse_gated_act(const float* gu, int ldg, void* h, int M, int F, int kind, int f32, hipStream_t st);
 hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st);
+bool dsse_norm_rope_all_fours(const dsse::NormRopeList& l);
 hipError_t dsse_sink_attention(int num_work, const dsse::SinkAttnParams* p, hipStream_t st);
 // MFMA form for prompt portions (bf16, D % 32 == 0, V / 16 in {1..8, 10, 12, 16, 20, 24, 32}): 16-row tiles, values from the
 // transposed pages vt [pages, G, V, kBS] (keys permuted inside a page as the MFMA's k axis wants them)

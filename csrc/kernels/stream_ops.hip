@@ -186,6 +186,7 @@ DEV void norm_rope_fours_row(const NormRopeParams& p, int gy, float* red) {
     const int h = h0 + wave * hpw + lane / n;
     const bool on = h < p.nh;
     f32x4 v = ld4(x + (on ? h : 0) * p.D + e);
+    if (p.bias) v += ld4(p.bias + (on ? h : 0) * p.D + e);
     float inv = inv_row;
     if (p.kind >= 2) {
       float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
@@ -229,7 +230,9 @@ DEV void value_pages(const NormRopeParams& p, int item, bf16* tile) {
   for (int r = threadIdx.x / n; r < kBS; r += rpp) {
     const int s = __shfl(slot, r);
     if (r >= rows) continue;
-    const f32x4 v = ld4(p.x + (int64_t)(t0 + r) * p.ldx + h * p.D + e) * p.scale;
+    f32x4 v = ld4(p.x + (int64_t)(t0 + r) * p.ldx + h * p.D + e);
+    if (p.bias) v += ld4(p.bias + h * p.D + e);
+    v = v * p.scale;
     const bf16x4 b{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
     *reinterpret_cast<bf16x4*>(tile + r * ldt + e) = b;
     if (s >= 0) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(p.out) + (int64_t)s * p.ldo + h * p.D + e) = b;
@@ -258,7 +261,7 @@ DEV void value_pages(const NormRopeParams& p, int item, bf16* tile) {
 // Heads of 32, 64, 128 or 256 numbers in 16-byte pieces, rotation partners a power of two of lanes apart
 inline bool norm_rope_fours(const NormRopeParams& p) {
   auto power = [](int n) { return n > 0 && (n & (n - 1)) == 0; };
-  return p.D % 32 == 0 && p.D <= 256 && power(p.D) && p.ldx % 4 == 0 && p.ldo % 4 == 0 && fours({p.x, p.out, p.norm_w, p.rope}) &&
+  return p.D % 32 == 0 && p.D <= 256 && power(p.D) && p.ldx % 4 == 0 && p.ldo % 4 == 0 && fours({p.x, p.out, p.norm_w, p.rope, p.bias}) &&
          (!p.rope || (p.half % 4 == 0 && power(p.half / 4) && 2 * p.half <= p.D));
 }
 
@@ -438,6 +441,13 @@ extern "C" hipError_t dsse_gated_act(const float* gu, int ldg, void* h, int M, i
     hipLaunchKernelGGL(dsse::gated_act_kernel<bf16>, dim3(blocks), dim3(256), 0, st, gu, ldg, reinterpret_cast<bf16*>(h),
                        M, F, kind);
   return hipGetLastError();
+}
+
+// Every set in fours: the only form that adds biases
+extern "C" bool dsse_norm_rope_all_fours(const dsse::NormRopeList& l) {
+  for (int i = 0; i < l.n; ++i)
+    if (!dsse::norm_rope_fours(l.p[i]) || (l.p[i].kind == 1 && l.p[i].bias)) return false;
+  return true;
 }
 
 extern "C" hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st) {

@@ -78,3 +78,35 @@ def test_gated_heads_in_fours(M, H, V, kind, dtype):
         lref.gated_head_norm(o, w, wide[:, 4:4 + H * V], EPS, want, kind)
         ops.gated_head_norm(c(o), c(w), c(wide)[:, 4:4 + H * V], EPS, got, kind)
         near(got, want, 2 if dtype == torch.bfloat16 else 30)  # 32-256 squares, a root, an exponential, four products
+
+
+@pytest.mark.parametrize("H,G,D,V", [(1, 1, 4, 0), (3, 2, 8, 4), (2, 1, 128, 0), (5, 1, 132, 64)])
+@pytest.mark.parametrize("K", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_convolved_rows_in_fours(H, G, D, V, K, dtype):
+    """Prompt portions that start, continue, are shorter than the taps, one inactive; a skipped row and one out of the pages."""
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32)  # noqa: E731
+    g = torch.Generator().manual_seed(D + K)
+    C, VW, lens, ctx = (H + G) * D, V or D, [9, 2, 0, 41], [9, 35, 3, 73]
+    T, qs = sum(lens), [0, 9, 11, 11]
+    x = torch.randn(T, 4 + C + G * V + 4, generator=g)
+    taps = torch.randn(C, K, generator=g) if K else None
+    tail = torch.randn(5, K - 1, C, generator=g) if K > 1 else None
+    rope = torch.randn(70, 2 if D < 128 else 64, 2, generator=g)  # shorter than the last position
+    factor = torch.rand(60, generator=g) if V else None
+    slots = torch.cat([96 * s + torch.arange(n - m, n, dtype=torch.int32) for s, (m, n) in enumerate(zip(lens, ctx))]).to(torch.int32)
+    slots[-1], slots[3] = 96 * 4 + 7, -1
+    caches = [torch.zeros(12, PAGE, G, D, dtype=dtype), torch.zeros(12, PAGE, G, VW, dtype=dtype), torch.zeros(12, G, VW, PAGE, dtype=dtype)]
+    for qt in (4, 16):
+        want, got = [t.clone() for t in caches], [c(t) for t in caches]
+        q_ref, q, t0, t1 = torch.zeros(T, H, D), torch.zeros(T, H, D, device="cuda"), None if tail is None else tail.clone(), c(tail)
+        meta = (i32(qs), i32(lens), i32(ctx), i32([4, 0, 2, 1]))
+        work = [(s, t) for s, n in enumerate(lens) for t in range(-(-n // qt))]
+        lref.conv_qkv_rows(x[:, 4:], taps, t0, *meta, H, G, D, V, rope, factor, slots, q_ref, *want)
+        ops.conv_qkv_rows(c(x)[:, 4:], c(taps), t1, *map(c, meta), c(i32([s for s, _ in work])), c(i32([t for _, t in work])), qt, H, G,
+                          D, V, c(rope), c(factor), c(slots), q, *got)
+        near(q, q_ref, 12)  # four products and sums, a rotation, a factor
+        for a, r in zip(got, want):
+            near(a, r, 12 if dtype == torch.float32 else 2)
+        if K > 1:
+            assert torch.equal(t1.cpu(), t0)
