@@ -541,7 +541,7 @@ class LayeredRunner(RunnerBase):
     @staticmethod
     def _cols(buf, c0: int, heads: int, width: int):
         """Columns [c0, c0 + heads * width) of a row-major fp32 buffer as [rows, heads, width] (a view)."""
-        return buf[:, c0:c0 + heads * width].unflatten(1, (heads, width))
+        return buf[:, c0:c0 + heads * width].view(-1, heads, width)
 
     def _scan_rows(self, buf, c0: int, H: int, D: int, V: int):
         """Queries, keys and values that lie side by side from column c0 on."""
@@ -1310,6 +1310,8 @@ class LayeredRunner(RunnerBase):
         norms it for the next layer; the last outputs are added before the head's norm.  Both sublayers of a layer run at
         the same time: the mixer's launches are latency-sized, the experts' stream weights."""
         cfg, w, eps = self.cfg, self.w, self.cfg.eps
+        # a captured step forks for nothing on the host
+        capturing = self._side_stream is not None and torch.cuda.is_current_stream_capturing()
         ops.embed_rows(ids, w.embed, d["resid"], None, cfg.embed_scale, pos, self._pos_table)
         none = (None, 1, None, 1)
         pending = none  # sublayer outputs that are not in the stream yet: (rows, parts per row) of both
@@ -1318,7 +1320,7 @@ class LayeredRunner(RunnerBase):
             ops.add_norm_rows(y, nsum, None, d["resid"], Lw.norm1, eps, d["xb"], d["hn"] if L.mlp is not None else None, y2, nsum2)
             if L.mlp is None:
                 pending = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups) + (None, 1)
-            elif self._side_stream is None:
+            elif self._side_stream is None or not (capturing or self._worth_a_fork(L, M)):
                 mixed = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
                 pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d) + mixed
             else:
@@ -1334,6 +1336,17 @@ class LayeredRunner(RunnerBase):
                 trace.append(d["resid"].clone())
         if pending[0] is not None:
             ops.add_norm_rows(pending[0], pending[1], None, d["resid"], None, eps, None, None, *pending[2:])
+
+    def _worth_a_fork(self, L, M: int) -> bool:
+        """Whether M rows keep the GPU longer in one layer than the host needs to issue it with a fork and a join: two waits across
+        streams of some 17 us each and their events, 210 us a layer in all against 137 on one stream.  The layer's time from its
+        weights at 5 TB/s, its products at 500 TFLOP/s and 60 us of small launches.  One stream / two, six layers of 2048 wide with
+        16 experts of 1408: 64 rows 825 / 1230 us, 150 rows 1042 / 1280, 300 rows 1183 / 1298, but 500 rows 1367 / 1309, 800 rows
+        1631 / 1356; 4096 wide with experts of 3584: 64 rows 2086 / 2177, 200 rows 2795 / 2664, 500 rows 3509 / 3239."""
+        f, m, W = L.mlp, L.mixer, self.cfg.width
+        met = (2 * m.heads + 2 * m.kv_heads) * m.dim + m.heads * m.vdim  # columns of the mixer's projections
+        ff = 3 * (f.experts * f.ff + f.shared_ff), 3 * (f.top * f.ff + f.shared_ff)
+        return 60 + (ff[0] + met) * W * 2 / 5e6 + 2 * M * (ff[1] + met) * W / 5e8 >= 210
 
     def _attention_joint(self, li: int, m, Lw, M: int, d: dict, slots, groups: list):
         """Windowed attention with a distance bias over this layer's pages, or over those of the layer it takes keys and

@@ -11,11 +11,15 @@ import torch
 from . import layers_reference as lref
 
 
-def _hip(t: torch.Tensor) -> bool:
-    if t.is_cuda:
-        from . import load_library
+_load = None  # ops.load_library: a statement that imports it costs every launch half a microsecond
 
-        load_library(required=True)
+
+def _hip(t: torch.Tensor) -> bool:
+    global _load
+    if t.is_cuda:
+        if _load is None:
+            from . import load_library as _load
+        _load(required=True)
         return True
     return False
 
