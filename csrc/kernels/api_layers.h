@@ -170,6 +170,8 @@ struct MoeGroupedParams {
 // Shapes that the expert GEMMs on LDS-DMA take (moe_pipe.hip, moe_stream.hip): reduction lengths of whole 64-element steps,
 // two at least; 16-byte-aligned operands; every operand inside a 2 GiB buffer range.
 bool moe_lines_ok(const MoeGroupedParams& p);
+// Shapes that the exact mode's expert GEMMs on LDS-DMA take (moe_exact.hip)
+bool moe_exact_ok(const MoeGroupedParams& p);
 // Which form those take: the register-direct kernels of moe.hip (few rows of small experts), the stream, the pipeline
 enum class MoeForm { kDirect, kStream, kPipe };
 MoeForm moe_form(const MoeGroupedParams& p);
@@ -225,6 +227,7 @@ hipError_t dsse_conv_state(const dsse::ConvStateParams* p, hipStream_t st);
 hipError_t dsse_lru_scan(const dsse::LruScanParams* p, hipStream_t st);
 hipError_t dsse_moe_router(const dsse::MoeRouterParams* p, hipStream_t st);
 hipError_t dsse_moe_ffn(const dsse::MoeFfnParams* p, hipStream_t st);
+hipError_t dsse_moe_exact(const dsse::MoeGroupedParams* p, hipStream_t st);
 hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStream_t st);
 hipError_t dsse_moe_route_rows(const dsse::MoeRouteRowsParams* p, hipStream_t st);
 hipError_t dsse_moe_topk(const float* z, int M, int E, int top, int* topk_idx, float* topk_w, hipStream_t st);

@@ -725,6 +725,7 @@ extern "C" hipError_t dsse_moe_grouped(const dsse::MoeGroupedParams* p, hipStrea
     const dsse::MoeForm form = dsse::moe_form(*p);
     if (form != dsse::MoeForm::kDirect) return form == dsse::MoeForm::kStream ? dsse_moe_stream(p, st) : dsse_moe_pipe(p, st);
   }
+  if (dsse::moe_exact_ok(*p)) return dsse_moe_exact(p, st);
   // other prompt-sized steps in bf16 with rows of whole 16-byte pieces: operands staged through registers and LDS
   if (!p->f32 && p->lds_tiles && p->W % 8 == 0 && p->F % 8 == 0 && p->Fs % 8 == 0 && p->ldh % 8 == 0) {
     dim3 l1((fmax + 63) / 64, p->max_tiles), l2((p->W + 127) / 128, p->max_tiles), l3((fmax + 127) / 128, p->max_tiles);
