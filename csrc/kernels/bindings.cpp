@@ -169,6 +169,10 @@ SCfg pick_stream(int M, int N, int K, int mode = -1) {
   // 8 waves per workgroup when that still gives ~one workgroup per CU without split-K (gate_up,
   // LM head), else 4 (narrow O / down / QKV: more, shorter workgroups; measured, profiles/gemm_stream_r1.md)
   c.nw = env_int("s_nw", (N / (16 * c.nt)) / 8 >= 192 ? 8 : 4);
+  // 17 to 64 rows (the ring): 8 also where workgroups of 4 would be more than one round of the CUs.  16640 x 4096, 4 / 8 waves: 17 rows
+  // 36.0 / 27.5 us, 64 rows 43.6 / 33.2
+  const bool ring = M > 16 && M <= 64;
+  if (ring && c.nt == 1 && env_int("s_nw", 0) == 0 && N / 64 > 256 && N % 128 == 0) c.nw = 8;
   if (c.nt == 2 && c.mt <= 4) c.nw = 8;  // instantiated (nt, nw): (1, 8), (2, 8), (1, 4) — gemm_stream.hip
   if (c.nt == 2 && c.mt >= 8) c.nw = 4;   // mt 8 / 16: (1, 8), (1, 4), (2, 4)
   // 7 waves when that puts exactly one workgroup on each CU where 8 leaves CUs idle (gate_up at TP = 1:
@@ -198,11 +202,14 @@ SCfg pick_stream(int M, int N, int K, int mode = -1) {
   const int wgs = N / (16 * c.nt) / c.nw * (M > 16 * c.mt ? (M + 63) / 64 : 1), slices = K / (128 * cps);
   int S = env_int("s_split", 0);
   if (S <= 0 || slices % S != 0) {
-    // smallest split that gives ~one workgroup per CU (256 CUs), never more than 1.25x that
+    // smallest split that gives ~one workgroup per CU (256 CUs), never more than 1.25x that; on the ring never more: a second round
+    // takes as long as the first.  320 workgroups of two slices / 160 of one: 10240 x 4096, 17 rows 23.7 / 19.8 us, 64 rows 28.8 /
+    // 22.6; 9216 x 2048, 64 rows 19.1 / 12.6; 260 / 130, 8320 x 4096, 64 rows 27.9 / 22.1
+    const int most = ring ? 256 : 320;
     S = 1;
     for (int d = 1; d <= slices; ++d) {
       if (slices % d) continue;
-      if (wgs * d > 320) break;
+      if (wgs * d > most) break;
       S = d;
       if (wgs * d >= 192) break;
     }
