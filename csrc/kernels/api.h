@@ -145,6 +145,9 @@ hipError_t dsse_rmsnorm(int mode, int M, float* resid, int H, const void* delta,
 hipError_t dsse_rope_kv_write(int T, const void* qkv, int hq, int hkv, const int* positions,
                               const int* slots, const float2* rope, void* q_out, void* k_cache,
                               void* v_cache, int num_slots, int rope_len, hipStream_t st);
+hipError_t dsse_rope_kv_slices(int T, const float* part, int S, int hq, int hkv, const int* positions, const int* slots,
+                               const float2* rope, void* q_out, void* k_cache, void* v_cache, int num_slots, int rope_len,
+                               hipStream_t st);
 hipError_t dsse_silu_mul(int T, int F, const void* gu, void* h, hipStream_t st);
 hipError_t dsse_decode_prep(int B, const int* active, const int* positions, const int* block_tables,
                             int max_blocks, int num_blocks, int* slots, int* ctx_len, int* q_len, int* walked, hipStream_t st);

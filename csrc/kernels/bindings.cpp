@@ -942,7 +942,8 @@ void rmsnorm(Tensor& resid, const Tensor& w, Tensor& y, double eps, const c10::o
 }
 
 void rope_kv_write(const Tensor& qkv, const Tensor& positions, const Tensor& slots, const Tensor& rope,
-                   Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh, int64_t nkv) {
+                   Tensor& q_out, Tensor& k_cache, Tensor& v_cache, int64_t nh, int64_t nkv, const std::optional<Tensor>& part,
+                   int64_t nsplit) {
   check_gpu(qkv, "qkv");
   check_dtype(qkv, at::kBFloat16, "qkv");
   const int T = (int)qkv.size(0);
@@ -950,6 +951,18 @@ void rope_kv_write(const Tensor& qkv, const Tensor& positions, const Tensor& slo
   TORCH_CHECK(positions.numel() >= T && slots.numel() >= T, "metadata too short");
   TORCH_CHECK(q_out.numel() >= (int64_t)T * nh * 128, "q_out too small");
   TORCH_CHECK(k_cache.size(1) == nkv && v_cache.size(1) == nkv, "cache head mismatch");
+  if (nsplit > 0) {  // qkv's rows still as fp32 K slices [nsplit, T, width]; qkv itself is neither read nor written
+    TORCH_CHECK(part.has_value(), "slices without their tensor");
+    check_gpu(*part, "part");
+    check_dtype(*part, at::kFloat, "part");
+    TORCH_CHECK(part->numel() >= nsplit * qkv.numel() && reinterpret_cast<uintptr_t>(part->data_ptr()) % 16 == 0,
+                "part must hold the slices, 16-byte aligned");
+    DSSE_CHECK_HIP(dsse_rope_kv_slices(T, part->data_ptr<float>(), (int)nsplit, (int)nh, (int)nkv, positions.data_ptr<int>(),
+                                       slots.data_ptr<int>(), reinterpret_cast<const float2*>(rope.data_ptr<float>()),
+                                       q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                                       (int)(k_cache.size(0) * dsse::kBS), (int)rope.size(0), cur_stream()));
+    return;
+  }
   DSSE_CHECK_HIP(dsse_rope_kv_write(T, qkv.data_ptr(), (int)nh, (int)nkv, positions.data_ptr<int>(),
                                     slots.data_ptr<int>(),
                                     reinterpret_cast<const float2*>(rope.data_ptr<float>()),
@@ -1513,7 +1526,7 @@ TORCH_LIBRARY(dsse, m) {
   m.def("gemm_out_split(Tensor x, Tensor w, Tensor(a!) out, Tensor(b!) part) -> int");
   m.def("refresh_env() -> ()", &refresh_env);
   m.def("rope_kv_write(Tensor qkv, Tensor positions, Tensor slots, Tensor rope, Tensor(a!) q_out, "
-        "Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv) -> ()");
+        "Tensor(b!) k_cache, Tensor(c!) v_cache, int nh, int nkv, Tensor? part=None, int nsplit=0) -> ()");
   m.def("silu_mul(Tensor gu, Tensor(a!) h) -> ()");
   m.def("decode_prep(Tensor active, Tensor positions, Tensor block_tables, Tensor(a!) slots, "
         "Tensor(b!) ctx_len, Tensor(c!) q_len, int num_blocks=2147483647, Tensor(d!)? walked=None) -> ()");

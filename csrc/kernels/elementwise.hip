@@ -103,11 +103,11 @@ rmsnorm_kernel(float* __restrict__ resid, int H, const bf16* __restrict__ delta,
 // qkv: [T, (hq + 2 hkv) * 128] bf16 in the engine's permuted column order (inside each 16-column
 // tile j of a head: columns 0..7 = dims 8j..8j+7, columns 8..15 = dims 64+8j..64+8j+7).
 // A token's rows: each thread rotates 8 pairs of one (unit, tile j) with 16-byte loads and stores.
-DEV void rope_kv_rows(const bf16* __restrict__ qkv, int hq, int hkv, const int* __restrict__ positions,
+// load(col): eight neighbouring numbers of the row in bf16.
+template <typename Load>
+DEV void rope_kv_rows(Load load, int hq, int hkv, const int* __restrict__ positions,
                       const int* __restrict__ slots, const float2* __restrict__ rope, bf16* __restrict__ q_out,
                       bf16* __restrict__ k_cache, int num_slots, int rope_len, int t) {
-  const int ncols = (hq + 2 * hkv) * 128;
-  const bf16* row = qkv + (size_t)t * ncols;
   const int pos = DSSE_IDX(positions[t], rope_len, 0);
   const int slot = slots[t] < 0 ? -1 : DSSE_IDX(slots[t], num_slots, -1);
   const int blk = slot >= 0 ? slot / kPageTok : 0, off = slot >= 0 ? slot % kPageTok : 0;
@@ -117,8 +117,8 @@ DEV void rope_kv_rows(const bf16* __restrict__ qkv, int hq, int hkv, const int* 
     bf16* dst = u < hq ? q_out + ((size_t)t * hq + u) * 128
                        : (slot >= 0 ? k_cache + (((size_t)blk * hkv + (u - hq)) * kPageTok + off) * 128 : nullptr);
     if (dst == nullptr) continue;
-    const bf16x8 x1 = ld_bf16x8(row + u * 128 + 16 * j);
-    const bf16x8 x2 = ld_bf16x8(row + u * 128 + 16 * j + 8);
+    const bf16x8 x1 = load(u * 128 + 16 * j);
+    const bf16x8 x2 = load(u * 128 + 16 * j + 8);
     const float4* cs4 = reinterpret_cast<const float4*>(rope + (size_t)pos * 64 + 8 * j);
     bf16x8 o1, o2;
 #pragma unroll
@@ -183,13 +183,69 @@ rope_kv_v_kernel(const bf16* __restrict__ qkv, int T, int hq, int hkv, const int
                  const int* __restrict__ slots, const float2* __restrict__ rope, bf16* __restrict__ q_out,
                  bf16* __restrict__ k_cache, bf16* __restrict__ v_cache, int num_slots, int rope_len) {
   if ((int)blockIdx.x < T) {
-    rope_kv_rows(qkv, hq, hkv, positions, slots, rope, q_out, k_cache, num_slots, rope_len, blockIdx.x);
+    const bf16* row = qkv + (size_t)blockIdx.x * (hq + 2 * hkv) * 128;
+    rope_kv_rows([=](int col) { return ld_bf16x8(row + col); }, hq, hkv, positions, slots, rope, q_out, k_cache, num_slots, rope_len,
+                 blockIdx.x);
     return;
   }
   const int vb = blockIdx.x - T, hpairs = (hkv + 1) / 2;
   const int h = 2 * (vb % hpairs) + (threadIdx.x >> 7);
   if (h >= hkv) return;  // wave-uniform (128-thread halves)
   v_page_write(qkv, T, hq, hkv, slots, v_cache, num_slots, (vb / hpairs) * kPageTok, h, threadIdx.x & 127);
+}
+
+// The same from the K slices of a split projection, fp32 [S, T, (hq + 2 hkv) * 128]: their sum is rounded to bf16 as the reduction
+// launch rounds it, and that launch, its bf16 rows and their way back fall away.  Blocks [0, T) rotate q and k, the blocks after them
+// take 32 rows of one kv head's values, 16 of them to a thread.  384 rows of 32 + 8 + 8 heads in
+// five slices beside the rest of a mixed step of 64 streams and 300 prompt rows: 9.1 + 9.1 -> 11 us a layer, the step 9037 -> 8815.
+template <typename V>
+DEV V slice_sum(const float* p, size_t slab, int S) {
+  return add_parts<V>(S, [&](int s) { return ld_global<V>(p + s * slab); });
+}
+
+__global__ void __launch_bounds__(256)
+rope_kv_slices_kernel(const float* __restrict__ part, int S, int T, int hq, int hkv, const int* __restrict__ positions,
+                      const int* __restrict__ slots, const float2* __restrict__ rope, bf16* __restrict__ q_out,
+                      bf16* __restrict__ k_cache, bf16* __restrict__ v_cache, int num_slots, int rope_len) {
+  const int ncols = (hq + 2 * hkv) * 128;
+  const size_t slab = (size_t)T * ncols;
+  if ((int)blockIdx.x < T) {
+    const float* row = part + (size_t)blockIdx.x * ncols;
+    auto load = [=](int col) {
+      const f32x4 a = slice_sum<f32x4>(row + col, slab, S), b = slice_sum<f32x4>(row + col + 4, slab, S);
+      return bf16x8{f2bf(a[0]), f2bf(a[1]), f2bf(a[2]), f2bf(a[3]), f2bf(b[0]), f2bf(b[1]), f2bf(b[2]), f2bf(b[3])};
+    };
+    rope_kv_rows(load, hq, hkv, positions, slots, rope, q_out, k_cache, num_slots, rope_len, blockIdx.x);
+    return;
+  }
+  const int vb = blockIdx.x - T, h = vb % hkv, t0 = vb / hkv * kPageTok, lane = threadIdx.x & 63;
+  const int d = threadIdx.x & 127, r0 = 16 * (threadIdx.x >> 7);  // uniform for the wave
+  const int tl = t0 + (lane & 31);
+  const int my_slot = tl < T ? (slots[tl] < 0 ? -1 : DSSE_IDX(slots[tl], num_slots, -1)) : -1;
+  const int s0 = __shfl(my_slot, 0);
+  const bool whole = __all(s0 >= 0 && s0 % kPageTok == 0 && my_slot == s0 + (lane & 31));
+  const int col = d < 64 ? 16 * (d >> 3) + (d & 7) : 16 * ((d - 64) >> 3) + 8 + (d & 7);  // as in v_page_write
+  const float* src = part + (size_t)t0 * ncols + (hq + hkv + h) * 128 + col;
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = 0.f;
+  for (int s = 0; s < S; ++s) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] += src[s * slab + (size_t)(t0 + r0 + i < T ? r0 + i : T - 1 - t0) * ncols];
+  }
+  if (whole) {
+    bf16* dst = v_cache + (((size_t)(s0 / kPageTok) * hkv + h) * 128 + d) * kPageTok + (r0 >> 2);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)  // tokens r0 + 4 q .. + 3
+      *reinterpret_cast<bf16x4*>(dst + 8 * q) = bf16x4{f2bf(v[4 * q]), f2bf(v[4 * q + 1]), f2bf(v[4 * q + 2]), f2bf(v[4 * q + 3])};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int sl = __builtin_amdgcn_readlane(my_slot, r0 + i);  // -1 past the last row
+    if (sl < 0) continue;
+    v_cache[(((size_t)(sl / kPageTok) * hkv + h) * 128 + d) * kPageTok + vperm_tok(sl % kPageTok)] = f2bf(v[i]);
+  }
 }
 
 // ---- SiLU·mul over the interleaved gate/up output of a library GEMM (prefill) ---------------
@@ -296,6 +352,17 @@ extern "C" hipError_t dsse_rope_kv_write(int T, const void* qkv, int hq, int hkv
   hipLaunchKernelGGL(rope_kv_v_kernel, dim3(T + vblocks), dim3(256), 0, st, reinterpret_cast<const bf16*>(qkv), T,
                      hq, hkv, positions, slots, rope, reinterpret_cast<bf16*>(q_out), reinterpret_cast<bf16*>(k_cache),
                      reinterpret_cast<bf16*>(v_cache), num_slots, rope_len);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t dsse_rope_kv_slices(int T, const float* part, int S, int hq, int hkv, const int* positions, const int* slots,
+                                          const float2* rope, void* q_out, void* k_cache, void* v_cache, int num_slots, int rope_len,
+                                          hipStream_t st) {
+  if (T <= 0) return hipSuccess;
+  const int vblocks = (T + kPageTok - 1) / kPageTok * hkv;
+  hipLaunchKernelGGL(rope_kv_slices_kernel, dim3(T + vblocks), dim3(256), 0, st, part, S, T, hq, hkv, positions, slots, rope,
+                     reinterpret_cast<bf16*>(q_out), reinterpret_cast<bf16*>(k_cache), reinterpret_cast<bf16*>(v_cache), num_slots,
+                     rope_len);
   return hipGetLastError();
 }
 

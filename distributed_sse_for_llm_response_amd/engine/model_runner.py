@@ -690,6 +690,16 @@ class ModelRunner(RunnerBase):
         """out = a·wᵀ in bf16 on the engine's tiled-layout GEMMs (every row count: no library GEMM)."""
         ops.gemm_out(a, wt, out)
 
+    def _qkv_rows(self, x, L, qkv, pos, slots, q, kc, vc) -> None:
+        """QKV projection, RoPE and K/V write of prompt rows.  K slices of a split projection stay in split_part (free here: the
+        previous norm consumed it) and are summed where they are rotated."""
+        ns, rows = 0, x.shape[0]
+        if self.comm.size == 1 and rows <= PREFILL_SLAB_ROWS:  # (slices that split_part cannot hold: the whole product)
+            ns = ops.gemm_out_split(x, L.wqkv_t, qkv, self.split_part)
+        else:
+            self._proj(x, L.wqkv_t, qkv)
+        ops.rope_kv_write(qkv, pos, slots, self.rope, q, kc, vc, self.w.nh, self.w.nkv, self.split_part if ns else None, ns)
+
     def _gate_up(self, x, L, h) -> None:
         """h = SiLU(x·W_gateᵀ)·(x·W_upᵀ) with the fused SiLU·mul epilogue (gate / up rows interleaved by 8)."""
         ops.gemm_silu(x, L.wgu_t, h)
@@ -892,8 +902,7 @@ class ModelRunner(RunnerBase):
             # per-element RoPE epilogue measured +200 us per 8192-row layer (profiles/r2/prefill_kernels_8k.md), and
             # at 512 rows (gemm_qkv_rope, one launch fewer) 9.21-9.37 vs 9.15-9.33 ms TTFT, alternating
             # (profiles/r6/ttft512_qkv_fused_ab_r6.log)
-            self._proj(x, L.wqkv_t, qkv)
-            ops.rope_kv_write(qkv, d["pos"], d["slots"], self.rope, q, self.kv.k[li], self.kv.v[li], nh, nkv)
+            self._qkv_rows(x, L, qkv, d["pos"], d["slots"], q, self.kv.k[li], self.kv.v[li])
             if d.get("fslots"):
                 ops.flash_prefill_split(q, self.kv.k[li], self.kv.v[li], d["bt"], d["qs"], d["ql"], d["ctx"],
                                         d["fw"], d["fc"], attn, d["fpo"], d["fpm"], d["fslots"])
@@ -997,8 +1006,7 @@ class ModelRunner(RunnerBase):
         nl = len(w.layers)
         for li, L in enumerate(w.layers):
             kc, vc = self.kv.k[li], self.kv.v[li]
-            self._proj(x, L.wqkv_t, qkv)
-            ops.rope_kv_write(qkv, pos, slots, self.rope, q, kc, vc, nh, nkv)
+            self._qkv_rows(x, L, qkv, pos, slots, q, kc, vc)
             ops.paged_attention(0, q[r], kc, vc, self.block_tables[r], self.q_start[r], self.q_len[r],
                                 self.ctx_len[r], self.work_seq[r], self.work_tile[r], attn[r], self.part_o,
                                 self.part_ml, dpart, dnparts)

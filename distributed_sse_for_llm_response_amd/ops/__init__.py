@@ -189,9 +189,9 @@ def rmsnorm(resid, w, y, eps, delta=None, embed=None, ids=None, part=None, nspli
         ref.rmsnorm(resid, w, y, eps, delta, embed, ids, part, nsplit)
 
 
-def rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv):
+def rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv, part=None, nsplit: int = 0):
     if _hip(qkv):
-        torch.ops.dsse.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
+        torch.ops.dsse.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv, part, nsplit)
     else:
         ref.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
 
