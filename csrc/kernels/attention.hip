@@ -512,11 +512,12 @@ extern "C" hipError_t dsse_paged_attention(int mode, int num_work, const dsse::A
       hipLaunchKernelGGL((attn_combine_kernel<1>), dim3(num_work, p->hkv, 1), dim3(256), 0, st, *p);
   } else if (mode == 0) {
     // decode: p->kwv (attn_kwv in DSSE_KERNEL_CFG, read by the bindings) = waves per workgroup splitting the keys (1/2/4/8).
-    // Measured (profiles/attention_decode_r1.md): 4 key-split waves are best up to ~1k workgroups (64 streams x
-    // 8 kv heads: 29 us at 560 keys, 5.1 TB/s), one wave per (sequence, kv head) above (256 streams: 100 vs
-    // 109 us, 5.9 TB/s).  (A next-page register prefetch variant cost 2-10 % and was removed.)
+    // 1 / 2 / 4 waves, us, 512 keys on average (0.7 to 1.3 of it), 8 kv heads, non-temporal loads: 64 streams 122 / 28.6 / 29.6,
+    // 128 streams 138 / 54.2 / 55.9, 256 streams 173 / 108 / 100; 256 streams of 128 keys 36.9 / 25.8 / 25.9.  (A next-page
+    // register prefetch variant cost 2-10 % and was removed.)
     const dim3 grid(num_work, p->hkv, p->nparts);
-    const int kwv = p->kwv ? p->kwv : (grid.x * grid.y * grid.z >= 2048 ? 1 : 4);
+    const unsigned nwg = grid.x * grid.y * grid.z;
+    const int kwv = p->kwv ? p->kwv : (nwg >= 512 && nwg < 1536 ? 2 : 4);
     const int pd = p->pd == 2 && kwv <= 2 ? 2 : 1;  // attn_pd=2 (DSSE_KERNEL_CFG): 2-page register ring (1 / 2 waves)
     if (kwv == 8) hipLaunchKernelGGL((paged_attention_kernel<1, 8, 1>), grid, dim3(512), 0, st, *p);
     else if (kwv == 1 && pd == 2) hipLaunchKernelGGL((paged_attention_kernel<1, 1, 2>), grid, dim3(64), 0, st, *p);
