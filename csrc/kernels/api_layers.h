@@ -24,6 +24,8 @@ struct GemmRmParams {
   int f32;           // element type of x / w / bias: 0 bf16, 1 fp32
   int vecx, vecw;    // 16-byte fragment loads allowed (base, row and batch strides aligned)
 };
+// gemm_rm_strip.hip: rows 48 or 80; fp32 operands of whole 128-byte chunks (gemm_rowmajor.hip lds_ok)
+hipError_t gemm_rm_strip(int rows, const GemmRmParams& p, hipStream_t st);
 
 struct ScalarNormParams {
   const float* y;    // [M * nsum, W] sublayer output, a row's nsum consecutive parts are summed (mode 0) -- unused in mode 1

@@ -105,6 +105,15 @@ struct QkvRowsParams {
   int f32;
 };
 
+// gated_head_norm of a scan's read-out, made where the read-out is
+struct ScanGate {
+  const float* w;        // [V] or null
+  const float* gate;     // [T, H V] rows ldg apart
+  void* out;             // [T, H V], or null: the read-out itself
+  int ldg, kind, f32;
+  float eps;
+};
+
 struct MatrixScanParams {
   const float* q;        // [T, G, D] rows ldq apart
   const float* k;        // rows ldk apart
@@ -130,7 +139,9 @@ struct MatrixScanParams {
   int no_out;            // 1: a pass that only produces end states
   int portions;          // 1: the rows are prompt portions (many rows per sequence): the wave-local kernel
   float* a_out;          // [nseq, H, D] product of the chunk's per-channel decays (decay_kind 3) or null
+  ScanGate gated;
 };
+bool matrix_scan_gated_ok(const MatrixScanParams& p);
 
 // Workspace floats of the chunked form (matrix_chunk.hip) for `rows` rows, of them `longest` in the longest sequence (0 = not
 // known); 0 where the walk by tokens is taken: by its time, and for shapes that the chunks do not take.  They take key widths

@@ -389,14 +389,14 @@ void gate_pair(Tensor& x, const Tensor& p1, const Tensor& p2) {
   gate_rows(x, 3, p1, p2, 1.0);
 }
 
-void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
-                 Tensor& state, const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
-                 const Tensor& state_slot, Tensor& out, double q_scale, int64_t longest) {
+// Checks and parameters of matrix_scan without its output
+dsse::MatrixScanParams scan_params(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
+                                   Tensor& state, const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
+                                   const Tensor& state_slot, double q_scale) {
   head_view(q, "q");
   head_view(k, "k");
   head_view(v, "v");
   f32t(state, "state");
-  f32t(out, "out");
   dsse::MatrixScanParams p{};
   const int T = (int)v.size(0);
   p.H = (int)v.size(1), p.V = (int)v.size(2), p.G = (int)k.size(1), p.D = (int)k.size(2);
@@ -404,7 +404,6 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   TORCH_CHECK(p.D <= 512, "key width <= 512");
   TORCH_CHECK(state.dim() == 4 && state.size(1) == p.H && state.size(2) == p.D && state.size(3) == p.V,
               "state must be [slots, H, D, V]");
-  TORCH_CHECK(out.dim() == 3 && out.sizes() == v.sizes(), "out must be [T, H, V]");
   p.nseq = (int)q_len.numel();
   seq_meta(q_start, q_len, ctx_len, p.nseq);
   i32(state_slot, "state_slot");
@@ -441,9 +440,19 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
   p.q_len = q_len.data_ptr<int>();
   p.ctx_len = ctx_len.data_ptr<int>();
   p.state_slot = state_slot.data_ptr<int>();
-  p.out = out.data_ptr<float>();
   p.q_scale = (float)q_scale;
   p.portions = T > 2 * p.nseq;  // more than a row or two per sequence: prompt portions, not a decode step
+  return p;
+}
+
+void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
+                 Tensor& state, const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
+                 const Tensor& state_slot, Tensor& out, double q_scale, int64_t longest) {
+  dsse::MatrixScanParams p = scan_params(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, q_scale);
+  f32t(out, "out");
+  TORCH_CHECK(out.dim() == 3 && out.sizes() == v.sizes(), "out must be [T, H, V]");
+  p.out = out.data_ptr<float>();
+  const int T = (int)v.size(0);
   TORCH_CHECK(longest >= 0 && longest <= T, "longest must be 0 (not known) .. T rows");
   if (const int64_t floats = dsse::scan_chunk_floats(p, T, longest)) {
     Tensor ws = at::empty({floats}, v.options());
@@ -451,6 +460,27 @@ void matrix_scan(const Tensor& q, const Tensor& k, const Tensor& v, const OptTen
     return;
   }
   DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
+}
+
+// matrix_scan and gated_head_norm of its output in one launch where the decode rows' form takes them; false: nothing done
+bool matrix_scan_gated(const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& decay, const OptTensor& beta,
+                       Tensor& state, const Tensor& q_start, const Tensor& q_len, const Tensor& ctx_len,
+                       const Tensor& state_slot, const OptTensor& w, const Tensor& gate, double eps, Tensor& out, double q_scale,
+                       int64_t kind) {
+  dsse::MatrixScanParams p = scan_params(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, q_scale);
+  const int64_t T = v.size(0), cols = (int64_t)p.H * p.V;
+  col_view(gate, "gate");
+  f32t(gate, "gate", false);
+  gpu(out, "out");
+  TORCH_CHECK(gate.size(0) == T && gate.size(1) == cols && out.dim() == 2 && out.size(0) == T && out.size(1) == cols,
+              "gate and out must be [T, H V]");
+  p.gated.w = opt_f32(w, "w", p.V);
+  p.gated.gate = gate.data_ptr<float>();
+  p.gated.ldg = (int)gate.stride(0), p.gated.kind = (int)kind, p.gated.eps = (float)eps;
+  p.gated.out = out.data_ptr(), p.gated.f32 = elem(out, "out");
+  if (!dsse::matrix_scan_gated_ok(p)) return false;
+  DSSE_CHECK_HIP(dsse_matrix_scan(&p, cur_stream()));
+  return true;
 }
 
 // What the choice of a form looks at: shapes, row pitches and addresses.  decay: the decays where the caller has them, [T, H, D] when
@@ -946,6 +976,9 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
   m.def("gate_pair(Tensor(a!) x, Tensor p1, Tensor p2) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
         "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor(b!) out, float q_scale=1.0, int longest=0) -> ()");
+  m.def("matrix_scan_gated(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "
+        "Tensor q_len, Tensor ctx_len, Tensor state_slot, Tensor? w, Tensor gate, float eps, Tensor(b!) out, float q_scale=1.0, "
+        "int kind=0) -> bool");
   m.def("matrix_scan_two_levels(Tensor q, Tensor k, Tensor v, bool channels, int rows, int nseq, int longest, "
         "Tensor? decay=None) -> bool");
   m.def("matrix_scan_by_chunks(Tensor q, Tensor k, Tensor v, bool delta, bool channels, int rows, int nseq, int longest, "
@@ -980,6 +1013,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("gate_math", &gate_math);
   m.impl("gate_pair", &gate_pair);
   m.impl("matrix_scan", &matrix_scan);
+  m.impl("matrix_scan_gated", &matrix_scan_gated);
   m.impl("matrix_scan_chunked", &matrix_scan_chunked);
   m.impl("gated_head_norm", &gated_head_norm);
   m.impl("rms_mix", &rms_mix);

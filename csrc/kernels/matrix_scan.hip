@@ -421,8 +421,14 @@ hipError_t launch(const MatrixScanParams& p, hipStream_t st) {
 // What bounds it: the state, read and written once -- 67 MB at 16 sequences of 32 heads of 128 x 128 -- behind one chain of
 // loads (lengths, then everything else).  matrix_scan_kernel, which stages blocks of tokens for eight waves, took 37 us with
 // the delta rule there, this 11; 128 sequences 258 and 82; one sequence 5.7 and 4.2.  A sequence with several rows walks them, the next row's operands in flight.
-template <int NR, bool DELTA>
-__global__ __launch_bounds__(256) void matrix_scan_step_kernel(MatrixScanParams p) {
+//
+// Out: with an element type the workgroup has all columns of its head and leaves the head's gated norm of the read-out (`gated`)
+// instead of the read-out: a launch of 3 us and 12 bytes a value less.  16 sequences of 32 heads of 128 x 128, six such launches in a
+// step 643 -> 634 us, one sequence 505 -> 495.
+template <int NR, bool DELTA, typename Out = void>
+__global__ __launch_bounds__(std::is_void_v<Out> ? 256 : 1024) void matrix_scan_step_kernel(MatrixScanParams p) {
+  constexpr bool kGated = !std::is_void_v<Out>;
+  __shared__ __attribute__((aligned(16))) float head[kGated ? 256 : 4];
   const int seq = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
   const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (tile * kScanCols >= p.V) return;  // uniform for the wave
@@ -483,7 +489,29 @@ __global__ __launch_bounds__(256) void matrix_scan_step_kernel(MatrixScanParams 
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = groups16_sum(o[e]);
-    if (dr == 0) st4(p.out + ((int64_t)(row0 + t) * p.H + h) * p.V + j, o);
+    if constexpr (!kGated) {
+      if (dr == 0) st4(p.out + ((int64_t)(row0 + t) * p.H + h) * p.V + j, o);
+    } else {
+      const ScanGate& n = p.gated;
+      if (dr == 0) *reinterpret_cast<f32x4*>(head + j) = o;
+      __syncthreads();
+      if (threadIdx.x < 64) {  // V / 4 lanes of the first wave
+        const int e = 4 * lane;
+        const bool on = e < p.V;
+        const f32x4 y = on ? *reinterpret_cast<const f32x4*>(head + e) : f32x4{0.f, 0.f, 0.f, 0.f};  // (ld4 is of global memory)
+        const float inv = 1.0f / sqrtf(wave_sum((y[0] * y[0] + y[1] * y[1]) + (y[2] * y[2] + y[3] * y[3])) / (float)p.V + n.eps);
+        if (on) {
+          const int64_t col = (int64_t)h * p.V + e;
+          const f32x4 gate = ld4(n.gate + (row0 + t) * (int64_t)n.ldg + col);
+          f32x4 w{1.f, 1.f, 1.f, 1.f}, r;
+          if (n.w) w = ld4(n.w + e);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = y[i] * inv * w[i] * (n.kind == 1 ? 1.0f : gate[i]) / (1.0f + expf(-gate[i]));
+          st4(reinterpret_cast<Out*>(n.out) + (row0 + t) * (int64_t)p.H * p.V + col, r);
+        }
+      }
+      if (t + 1 < ql) __syncthreads();  // read before the next row's
+    }
   }
 #pragma unroll
   for (int i = 0; i < NR; ++i) st4(st + 16 * i * kScanCols, S[i]);
@@ -491,6 +519,15 @@ __global__ __launch_bounds__(256) void matrix_scan_step_kernel(MatrixScanParams 
 
 template <int NR>
 hipError_t launch_step(const MatrixScanParams& p, hipStream_t st) {
+  if (p.gated.out) {
+    const dim3 heads(1, p.H, p.nseq), all(4 * p.V);
+    auto go = [&](auto delta, auto out) {
+      hipLaunchKernelGGL((matrix_scan_step_kernel<NR, decltype(delta)::value, decltype(out)>), heads, all, 0, st, p);
+    };
+    if (p.gated.f32) p.beta ? go(std::true_type{}, 0.f) : go(std::false_type{}, 0.f);
+    else p.beta ? go(std::true_type{}, bf16{}) : go(std::false_type{}, bf16{});
+    return hipGetLastError();
+  }
   const dim3 grid((p.V + 4 * kScanCols - 1) / (4 * kScanCols), p.H, p.nseq);
   if (p.beta) hipLaunchKernelGGL((matrix_scan_step_kernel<NR, true>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((matrix_scan_step_kernel<NR, false>), grid, dim3(256), 0, st, p);
@@ -500,9 +537,17 @@ hipError_t launch_step(const MatrixScanParams& p, hipStream_t st) {
 }  // namespace
 }  // namespace dsse
 
+// Decode rows that the step kernel takes with the gated norm inside: all columns of a head in one workgroup
+bool dsse::matrix_scan_gated_ok(const MatrixScanParams& p) {
+  const ScanGate& n = p.gated;
+  return n.out && !p.portions && !p.src_idx && p.V % kScanCols == 0 && p.V <= 256 && (p.D == 16 || p.D == 32 || p.D == 64 || p.D == 128) &&
+         p.ldv % 4 == 0 && n.ldg % 4 == 0 && fours({p.state, p.v, n.gate, n.w, n.out});
+}
+
 extern "C" hipError_t dsse_matrix_scan(const dsse::MatrixScanParams* p, hipStream_t st) {
   if (p->nseq <= 0 || p->H <= 0) return hipSuccess;
   if (p->D < 1 || p->D > 512 || p->V < 1 || p->G < 1 || p->H % p->G) return hipErrorInvalidValue;
+  if (p->gated.out && !dsse::matrix_scan_gated_ok(*p)) return hipErrorInvalidValue;
   if (p->portions || p->src_idx) {  // prompt portions (and every pass of the two-level walk): all sums inside a wave (rows per lane = D / 16 rounded up to a power of two)
     if (p->D <= 16) return dsse::launch_wave<1, 16>(*p, st);
     if (p->D <= 32) return dsse::launch_wave<2, 16>(*p, st);
@@ -511,7 +556,7 @@ extern "C" hipError_t dsse_matrix_scan(const dsse::MatrixScanParams* p, hipStrea
     if (p->D <= 256) return dsse::launch_wave<16, 8>(*p, st);
     return dsse::launch_wave<32, 4>(*p, st);
   }
-  if (p->V % dsse::kScanCols == 0 && p->ldv % 4 == 0 && dsse::fours({p->state, p->v, p->out})) {
+  if (p->V % dsse::kScanCols == 0 && p->ldv % 4 == 0 && dsse::fours({p->state, p->v, p->out})) {  // (out null: gated)
     if (p->D == 16) return dsse::launch_step<1>(*p, st);
     if (p->D == 32) return dsse::launch_step<2>(*p, st);
     if (p->D == 64) return dsse::launch_step<4>(*p, st);

@@ -551,6 +551,12 @@ class LayeredRunner(RunnerBase):
                   o_w, o_t, y):
         """Recurrence over every sequence group, per-head output norm times the SiLU gate, output projection (_out)."""
         o = d["o"][:M * H * V].view(M, H, V)
+        ao = d["ao"][:M * H * V].view(M, H * V)
+        if len(groups) == 1 and groups[0]["qt"] == 1:  # decode rows: norm and gate inside the step
+            g = groups[0]
+            if ops.matrix_scan_gated(q, k, v, decay, beta, self.state.state[ri], g["qs"], g["ql"], g["ctx"], g["ss"], Lw_norm, gate,
+                                     self.cfg.eps, ao, q_scale):
+                return self._out(ao, o_w, o_t, y)
         for g in groups:
             D, chan = k.shape[2], decay is not None and decay.dim() == 3
             if beta is None and self._two_levels(g, q, k, v, decay if chan else None):
@@ -562,7 +568,6 @@ class LayeredRunner(RunnerBase):
             else:
                 ops.matrix_scan(q, k, v, decay, beta, self.state.state[ri], g["qs"], g["ql"], g["ctx"], g["ss"], o,
                                 q_scale, g.get("longest", 0))
-        ao = d["ao"][:M * H * V].view(M, H * V)
         ops.gated_head_norm(o, Lw_norm, gate, self.cfg.eps, ao)
         return self._out(ao, o_w, o_t, y)
 

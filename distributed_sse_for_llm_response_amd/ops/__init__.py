@@ -329,7 +329,7 @@ def kernel_checks(clear: bool = True, raise_on_error: bool = True) -> list:
 
 
 from .layers import (conv_state, embed_rows, gate_math, gate_pair, gated_act, gated_head_norm, gemm_rm, latent_attention,  # noqa: E402,F401
-                     latent_flash_ok, latent_flash_part_floats, latent_kv_write, latent_tile_rows, logit_cap, lru_scan, matrix_scan,
+                     latent_flash_ok, latent_flash_part_floats, latent_kv_write, latent_tile_rows, logit_cap, lru_scan, matrix_scan, matrix_scan_gated,
                      matrix_scan_chunked, matrix_scan_two_levels,
                      moe_ffn, moe_grouped, moe_parts, moe_router, moe_topk, moe_topk_lists, norm_rope_rows, norm_rope_list, rms_mix, scalar_norm, sink_attention,
                      sink_flash_ok, sink_flash_lds, sink_tile_rows, sink_decode_ok, moe_route_rows, stream_step, stream_mix, act_rows, moe_route, embed_pair_rows, add_norm_rows,

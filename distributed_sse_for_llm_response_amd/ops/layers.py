@@ -345,6 +345,16 @@ def matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot
         lref.matrix_scan(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, out, q_scale)
 
 
+def matrix_scan_gated(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, w, gate, eps, out, q_scale: float = 1.0,
+                      kind: int = 0) -> bool:
+    """matrix_scan and gated_head_norm(w, gate, eps, kind) of what it reads out, in one launch; rows of idle sequences keep what
+    `out` held.  False: not decode rows or not shapes that the launch takes, nothing is done."""
+    if not _hip(v):
+        return False
+    return torch.ops.dsse.matrix_scan_gated(q, k, v, decay, beta, state, q_start, q_len, ctx_len, state_slot, w, gate, eps, out, q_scale,
+                                            kind)
+
+
 def scan_state_plain(state):
     """A GPU matrix state [slots, H, D, V] as the plain [.., D, V] matrices it stands for.  The scan kernels keep an
     entry tile-major ([H][V / 16][D][16]) when V is a multiple of 16; CPU tensors are plain already."""

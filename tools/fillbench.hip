@@ -2,6 +2,9 @@
 // X footprints of 2 MiB (one XCD's L2) and 8 MiB (spills the 4 MiB L2 into the Infinity Cache)): how many bytes
 // per second one CU can bring on chip, by path.
 //
+// Read its results as lower bounds: every piece pays a 64-bit modulo for its address, and pieces that hit the L2 arrive at 125 to 147
+// GB/s per CU without it.
+//
 // The decode GEMMs at 64-256 rows all measured ~35-39 GB/s of LDS-DMA fill per CU (gemm_ring at 64 rows,
 // gemm_tiled at 256 rows and at 8192 rows alike: profiles/r3/fillbench.md), which bounds them whatever the
 // MFMA work.  This program measures the paths separately and together, one 256-thread workgroup per CU:
