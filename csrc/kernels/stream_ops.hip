@@ -200,7 +200,9 @@ DEV void norm_rope_fours_row(const NormRopeParams& p, int gy, float* red) {
       f32x4 o;
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = side * __shfl_xor(v[i], p.half >> 2);
-      v = f32x4{v[0] * cs0[0] + o[0] * cs0[1], v[1] * cs0[2] + o[1] * cs0[3], v[2] * cs1[0] + o[2] * cs1[1], v[3] * cs1[2] + o[3] * cs1[3]};
+      // numbers past the rotated ones stay as they are, whatever they were paired with: 0 * inf is no zero
+      if (e < dims)
+        v = f32x4{v[0] * cs0[0] + o[0] * cs0[1], v[1] * cs0[2] + o[1] * cs0[3], v[2] * cs1[0] + o[2] * cs1[1], v[3] * cs1[2] + o[3] * cs1[3]};
     }
     v = v * p.scale;
     if (!on) continue;

@@ -110,3 +110,25 @@ def test_convolved_rows_in_fours(H, G, D, V, K, dtype):
             near(a, r, 12 if dtype == torch.float32 else 2)
         if K > 1:
             assert torch.equal(t1.cpu(), t0)
+
+
+@pytest.mark.parametrize("D,half", [(32, 4), (64, 8), (128, 32)])
+@pytest.mark.parametrize("kind", [0, 1, 3])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_what_is_not_finite_stays_where_it_was(D, half, kind, bad):
+    """A partial rotation beside an infinite or undefined number: of the numbers that are not rotated only that one is touched (no
+    norm), or what the reference says (a norm carries it through its sum)."""
+    g = torch.Generator().manual_seed(D)
+    x = torch.randn(5, 3, D, generator=g)
+    x[1, 1, 2 * half] = bad          # the first number past the rotated ones
+    x[2, 0, D - 1] = bad
+    x[3, 2, 1] = bad                 # a rotated one: its partner too
+    w = torch.randn(3 * D if kind == 1 else D, generator=g) if kind else None
+    rope, pos = torch.randn(7, half, 2, generator=g), torch.arange(5, dtype=torch.int32)
+    want, got = torch.zeros(5, 3, D), torch.zeros(5, 3, D, device="cuda")
+    lref.norm_rope_rows(x, w, pos, rope, want, None, kind, EPS, 0.7)
+    ops.norm_rope_rows(c(x), c(w), c(pos), c(rope), got, None, kind, EPS, 0.7)
+    got = got.cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    ok = torch.isfinite(want)
+    near(got[ok], want[ok], 24)
