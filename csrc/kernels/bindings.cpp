@@ -955,8 +955,9 @@ void rope_kv_write(const Tensor& qkv, const Tensor& positions, const Tensor& slo
     TORCH_CHECK(part.has_value(), "slices without their tensor");
     check_gpu(*part, "part");
     check_dtype(*part, at::kFloat, "part");
-    TORCH_CHECK(part->numel() >= nsplit * qkv.numel() && reinterpret_cast<uintptr_t>(part->data_ptr()) % 16 == 0,
-                "part must hold the slices, 16-byte aligned");
+    TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (nh + 2 * nkv) * 128 && part->numel() >= nsplit * qkv.numel() &&
+                    reinterpret_cast<uintptr_t>(part->data_ptr()) % 16 == 0,
+                "part must hold the slices of rows of nh + 2 nkv heads, 16-byte aligned");
     DSSE_CHECK_HIP(dsse_rope_kv_slices(T, part->data_ptr<float>(), (int)nsplit, (int)nh, (int)nkv, positions.data_ptr<int>(),
                                        slots.data_ptr<int>(), reinterpret_cast<const float2*>(rope.data_ptr<float>()),
                                        q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),

@@ -193,7 +193,7 @@ def rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv,
     if _hip(qkv):
         torch.ops.dsse.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv, part, nsplit)
     else:
-        ref.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv)
+        ref.rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv, part, nsplit)
 
 
 def silu_mul(gu, h):

@@ -128,8 +128,12 @@ def gemm_qkv_rope(x, w, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv
     _write_kv(rot[:, nh:], qkv[:, nh + nkv:], slots[:M], k_cache, v_cache)
 
 
-def rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv):
+def rope_kv_write(qkv, positions, slots, rope, q_out, k_cache, v_cache, nh, nkv, part=None, nsplit=0):
     T = qkv.shape[0]
+    if nsplit > 0:  # the rows as fp32 K slices [nsplit, T, width]; qkv itself is not read
+        if part is None or part.dtype != torch.float32 or part.numel() < nsplit * qkv.numel():
+            raise RuntimeError("part must hold the fp32 slices of qkv's rows")
+        qkv = part.reshape(-1)[:nsplit * qkv.numel()].view(nsplit, *qkv.shape).sum(0).to(qkv.dtype)
     u = _unpermute_units(qkv.float(), nh + 2 * nkv)
     rot = _rope(u[:, : nh + nkv], positions[:T], rope)
     q_out.view(-1)[: T * nh * HEAD_DIM].copy_(rot[:, :nh].reshape(-1).to(q_out.dtype))

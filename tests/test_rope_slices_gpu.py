@@ -40,3 +40,11 @@ def test_refused():
     for part in (None, z(2 * 384, dtype=torch.float32), z(4 * 384)):
         with pytest.raises(RuntimeError):
             ops.rope_kv_write(*args, part, 2)
+
+
+def test_rows_of_another_width_are_refused():
+    z = lambda *s, dtype=torch.bfloat16: torch.zeros(*s, dtype=dtype, device="cuda")  # noqa: E731
+    i = z(2, dtype=torch.int32)
+    with pytest.raises(RuntimeError):  # one head's worth of columns too few for nh + 2 nkv heads
+        ops.rope_kv_write(z(2, 256), i, i, z(4, 64, 2, dtype=torch.float32), z(2, 1, 128), z(1, 1, 32, 128), z(1, 1, 128, 32), 1, 1,
+                          z(2, 2, 256, dtype=torch.float32), 2)
