@@ -256,13 +256,14 @@ class LayeredRunner(RunnerBase):
     # ------------------------------------------------------------------ buffers
     def _buffers(self, M: int, clear: bool = True) -> dict:
         """Activations of a step of M rows.  clear=False (a prompt pass: every row belongs to a portion): what each step writes
-        whole before it reads it is not zeroed first -- a dozen fills and launches per pass."""
+        whole before it reads it is not zeroed first -- a dozen fills and launches per pass.  The output projections' parts (y, y2)
+        and their mix (ym) are never zeroed: a product writes every row of them, an idle sequence's too."""
         cfg, dev = self.cfg, self.device
         new = torch.zeros if clear else torch.empty
         f32 = dict(device=dev, dtype=torch.float32)
         el = dict(device=dev, dtype=self.dtype)
         W = cfg.width
-        d = {"resid": new(M, W, **f32), "xb": new(M, W, **el), "y": new(self._part_rows(M) * W, **f32)}
+        d = {"resid": new(M, W, **f32), "xb": new(M, W, **el), "y": torch.empty(self._part_rows(M) * W, **f32)}
         if self.joint:
             d.update(self._joint_buffers(M, new))
             return d
@@ -490,7 +491,7 @@ class LayeredRunner(RunnerBase):
             if L.mlp is not None:
                 ff = max(ff, L.mlp.ff)
                 gu = max(gu, 0 if self.w.layers[i].mlp.gu is None else 2 * L.mlp.ff)
-        y2 = {"y2": new(self._part_rows(M) * cfg.width, **f32), "ym": new(M, cfg.width, **f32)} if any(L.kind == "parallel" for L in cfg.layers) else {}
+        y2 = {"y2": torch.empty(self._part_rows(M) * cfg.width, **f32), "ym": torch.empty(M, cfg.width, **f32)} if any(L.kind == "parallel" for L in cfg.layers) else {}
         return {**y2, "big": new(M * big, **f32),
                 "cv": new(M * cv, **f32), "z": new(M * z, **f32),
                 "qa": new(M * qa, **f32), "o": new(M * o, **f32), "ao": new(M * o, **el),
