@@ -69,8 +69,8 @@ extern "C" hipError_t dsse_qkv_rows(const dsse::QkvRowsParams* p, hipStream_t st
   if (p->T <= 0) return hipSuccess;
   if (p->D > 64 * dsse::kHeadRegs || p->V > 64 * dsse::kHeadRegs) return hipErrorInvalidValue;
   // queries, keys and values as three sets of heads where all go by fours (stream_ops.hip) and the rows fill more than one round of
-  // workgroups.  Heads 16 + 8 + 8 of 128, this kernel / by fours: 128 rows 4.2 / 4.5 us, 300 rows 6.6 / 5.3, 1024 rows 16.4 / 9.5,
-  // 3000 rows 37 / 19; 32 + 8 + 8, 1024 rows 20.6 / 12.3.
+  // workgroups.  Heads 16 + 8 + 8 of 128, this kernel / by fours: 192 decode rows 6.2 / 6.2 us, 256 8.0 / 7.2, prompts of 300 rows 6.3 / 4.8
+  // (three of them 6.4 / 5.0), 1500 rows 21.3 / 11.6, 3000 rows 36 / 19.
   dsse::NormRopeList l{};
   auto set = [&](int nh, int D, int col, int kind, void* out, const int* rows) {
     dsse::NormRopeParams& s = l.p[l.n++];

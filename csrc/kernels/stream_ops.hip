@@ -217,47 +217,55 @@ DEV void norm_rope_fours_row(const NormRopeParams& p, int gy, float* red) {
   }
 }
 
-// Values on their way into pages and transposed pages: a workgroup takes 32 rows of one head, so that a whole page's 64-byte pieces
-// of the transposed one (a value's 32 tokens) are written by one thread each -- by token they are 2-byte writes from 32 workgroups
-// behind eight L2s: 1500 rows of 8 heads of 128 12.8 -> 6.3 us, beside queries and keys 19.9 -> 14.3.  Rows that make no whole page
-// in order go by token.  items: (32 rows, head) pairs, counted over the workgroups of the set.
-DEV void value_pages(const NormRopeParams& p, int item, bf16* tile) {
-  const int n = p.D >> 2, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ldt = p.D + 4;
-  const int t0 = item / p.nh * kBS, h = item % p.nh, rows = p.T - t0 < kBS ? p.T - t0 : kBS;
-  const int mine = (lane & 31) < rows ? p.out_rows[t0 + (lane & 31)] : -1;
-  const int slot = mine >= 0 && mine < p.num_out_rows ? mine : -1;  // of row lane & 31
-  const int first = __shfl(slot, 0);
-  const bool whole = rows == kBS && first >= 0 && first % kBS == 0 && __all(slot == first + (lane & 31));
-  const int rpp = 256 / n, e = 4 * (threadIdx.x & (n - 1));  // rows of a pass of the workgroup
-  for (int r = threadIdx.x / n; r < kBS; r += rpp) {
-    const int s = __shfl(slot, r);
-    if (r >= rows) continue;
-    f32x4 v = ld4(p.x + (int64_t)(t0 + r) * p.ldx + h * p.D + e);
-    if (p.bias) v += ld4(p.bias + h * p.D + e);
-    v = v * p.scale;
-    const bf16x4 b{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
-    *reinterpret_cast<bf16x4*>(tile + r * ldt + e) = b;
-    if (s >= 0) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(p.out) + (int64_t)s * p.ldo + h * p.D + e) = b;
-  }
-  __syncthreads();
-  bf16* pages = reinterpret_cast<bf16*>(p.out_t);
-  if (whole) {
-    bf16* dst = pages + ((int64_t)(first / kBS) * p.nh + h) * p.D * kBS;
-    for (int i = threadIdx.x; i < 4 * p.D; i += 256) {  // (value, 8 places): tokens 4 q .. + 3 and 16 + 4 q .. + 3
-      const int d = i >> 2, q = i & 3;
+// Values on their way into pages and transposed pages.  By token the transposed ones are 2-byte writes from 32 workgroups behind eight
+// L2s; where the 32 packed rows around a row are one page in order, wherever in the launch they begin, the page's workgroups take
+// columns instead: each a part of the page's columns for all of its 32 rows, so that a value's 32 tokens, 64 bytes, are written at
+// once.  The others go by token.  Both kinds move a row's worth of numbers per workgroup, behind one load of the slots.  8 heads of
+// 128, us, all by token / whole pages only at multiples of 32 packed rows, a workgroup to 32 rows of a head / this: one prompt of 1500 rows
+// 13.2 / 6.0 / 5.0, three of together 1500 13.0 / 8.9 / 5.1, of 300 4.9 / 5.6 / 3.9, 344 rows behind 20 decode rows 5.4 / 6.2 / 4.1; beside
+// queries and keys 23.7 / 14.0 / 13.6, 23.7 / 18.4 / 13.7, 9.5 / 6.5 / 5.4, 11.3 / 7.5 / 5.8, and 192 decode rows 8.6 / 8.1 / 6.9 (8 of 64, one
+// prompt of 1500: 15.3 / 9.5 / 10.6).
+constexpr int kPageCols = 64;  // columns that pass through LDS together
+constexpr int kPageLds = kBS * (kPageCols + 4) * sizeof(bf16);
+
+// Returns false, in every thread, where the row's page is not whole.  gy workgroups of the set per row.
+DEV bool value_pages(const NormRopeParams& p, int gy, bf16* tile) {
+  const int row = blockIdx.x, lane = threadIdx.x & 63;
+  const int near = row + lane - (kBS - 1);  // lane kBS - 1: the row itself
+  const int slot = near >= 0 && near < p.T ? p.out_rows[near] : -1;
+  const int own = __shfl(slot, kBS - 1);
+  if (own < 0 || own >= p.num_out_rows) return false;
+  const int off = own % kBS, first = own - off, from = kBS - 1 - off;  // the lane of the page's first row
+  const int i = lane - from;
+  if (first + kBS > p.num_out_rows || !__all(i < 0 || i >= kBS || slot == first + i)) return false;
+  const int t0 = row - off, N = p.nh * p.D;
+  const int each = max((N / 4 + kBS * gy - 1) / (kBS * gy), 8);  // groups of four columns of a workgroup: whole lines of x
+  const int g0 = (off * gy + (int)blockIdx.y) * each, g1 = min(g0 + each, N / 4);
+  bf16* out = reinterpret_cast<bf16*>(p.out) + (int64_t)first * p.ldo;
+  bf16* pages = reinterpret_cast<bf16*>(p.out_t) + (int64_t)first * N;
+  constexpr int ldt = kPageCols + 4;
+  for (int g = g0; g < g1; g += kPageCols / 4) {
+    const int n = min(kPageCols / 4, g1 - g);
+    for (int u = threadIdx.x; u < kBS * n; u += blockDim.x) {
+      const int r = u / n, q = u - r * n, d = 4 * (g + q);
+      f32x4 v = ld4(p.x + (int64_t)(t0 + r) * p.ldx + d);
+      if (p.bias) v += ld4(p.bias + d);
+      v = v * p.scale;
+      const bf16x4 b{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+      *reinterpret_cast<bf16x4*>(tile + r * ldt + 4 * q) = b;
+      *reinterpret_cast<bf16x4*>(out + (int64_t)r * p.ldo + d) = b;
+    }
+    __syncthreads();
+    for (int u = threadIdx.x; u < 16 * n; u += blockDim.x) {  // (column, 8 places): tokens 4 q .. + 3 and 16 + 4 q .. + 3
+      const int d = u >> 2, q = u & 3;
       bf16x8 o;
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = tile[(4 * q + (j & 3) + 16 * (j >> 2)) * ldt + d];
-      *reinterpret_cast<bf16x8*>(dst + (int64_t)d * kBS + 8 * q) = o;
+      *reinterpret_cast<bf16x8*>(pages + (int64_t)(4 * g + d) * kBS + 8 * q) = o;
     }
-    return;
+    __syncthreads();
   }
-  for (int r = wave; r < rows; r += 4) {
-    const int s = __builtin_amdgcn_readlane(slot, r);
-    if (s < 0) continue;
-    const int page = s / kBS, off = s % kBS, at = ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4 + (off & 3);
-    for (int d = lane; d < p.D; d += 64) pages[(((int64_t)page * p.nh + h) * p.D + d) * kBS + at] = tile[r * ldt + d];
-  }
+  return true;
 }
 
 // Heads of 32, 64, 128 or 256 numbers in 16-byte pieces, rotation partners a power of two of lanes apart
@@ -276,11 +284,7 @@ __global__ __launch_bounds__(64 * WAVES) void norm_rope_rows_kernel(NormRopeList
   const NormRopeParams& p = l.p[blockIdx.z];
   const int gy = l.gy[blockIdx.z];
   if ((int)blockIdx.y >= gy) return;  // uniform: another set's share of the grid
-  if (l.pages[blockIdx.z]) {
-    const int item = blockIdx.y * gridDim.x + blockIdx.x;
-    if (item < (p.T + kBS - 1) / kBS * p.nh) value_pages(p, item, reinterpret_cast<bf16*>(strips));
-    return;
-  }
+  if (l.pages[blockIdx.z] && value_pages(p, gy, reinterpret_cast<bf16*>(strips))) return;
   if (l.fours[blockIdx.z]) {
     if (p.out_f32) norm_rope_fours_row<float>(p, gy, red);
     else norm_rope_fours_row<bf16>(p, gy, red);
@@ -477,10 +481,7 @@ extern "C" hipError_t dsse_norm_rope_rows(dsse::NormRopeList l, hipStream_t st) 
     l.gy[i] = p.nh <= 0 ? 0 : (p.kind == 1 ? 1 : std::min((groups + each - 1) / each, 65535));
     // from 128 rows on: with fewer they are decode rows, each in a page of its own
     l.pages[i] = waves == 4 && l.fours[i] && p.out_t && dsse::fours({p.out_t}) && p.out_rows && !p.out_f32 && p.kind == 0 && !p.rope && p.nh > 0 && T >= 128;
-    if (l.pages[i]) {
-      l.gy[i] = (int)(((int64_t)((T + dsse::kBS - 1) / dsse::kBS) * p.nh + T - 1) / T);
-      lds = std::max(lds, (size_t)dsse::kBS * (p.D + 4) * sizeof(bf16));
-    }
+    if (l.pages[i]) lds = std::max(lds, (size_t)dsse::kPageLds);
     most = std::max(most, l.gy[i]);
   }
   if (most <= 0) return hipSuccess;

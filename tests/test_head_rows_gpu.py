@@ -132,3 +132,23 @@ def test_what_is_not_finite_stays_where_it_was(D, half, kind, bad):
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
     ok = torch.isfinite(want)
     near(got[ok], want[ok], 24)
+
+
+@pytest.mark.parametrize("nh,D", [(1, 32), (3, 32), (3, 64), (8, 128), (5, 256), (40, 64)])
+def test_pages_that_begin_anywhere_in_the_launch(nh, D):
+    """Decode rows in pages of their own, then prompts of whole and partial pages that begin at no multiple of 32 packed rows, a page
+    whose first rows are not in the launch, and one whose last are not."""
+    g = torch.Generator().manual_seed(nh + D)
+    rows = [PAGE * (20 + b) + (5 * b) % PAGE for b in range(7)] + list(range(PAGE * 40 + 9, PAGE * 42))  # the rest of a page, then a whole one
+    rows += list(range(71)) + [PAGE * 60 + 1, PAGE * 60] + list(range(PAGE * 10, PAGE * 10 + 64)) + list(range(PAGE * 50, PAGE * 50 + 30))
+    T, pages = len(rows), 62
+    assert T >= 128 and len(set(rows)) == T
+    rows = torch.tensor(rows, dtype=torch.int32)
+    x, pos = torch.randn(T, nh * D + 4, generator=g)[:, 4:].unflatten(1, (nh, D)), torch.zeros(T, dtype=torch.int32)
+    out, out_t = torch.full((pages, PAGE, nh, D), 7.0).to(torch.bfloat16), torch.full((pages, nh, D, PAGE), 7.0).to(torch.bfloat16)
+    got, got_t = c(out.clone()), c(out_t.clone())
+    lref.norm_rope_rows(x, None, pos, None, out, rows, 0, 0.0, 0.5, out_t)
+    wide = torch.zeros(T, nh * D + 4, device="cuda")
+    wide[:, 4:] = c(x.flatten(1))
+    ops.norm_rope_rows(wide[:, 4:].unflatten(1, (nh, D)), None, c(pos), None, got, c(rows), 0, 0.0, 0.5, got_t)
+    assert torch.equal(got.cpu(), out) and torch.equal(got_t.cpu(), out_t)
