@@ -38,7 +38,13 @@ DEV float block_sum(float v, float* red) {
 constexpr int kKeep = 4;
 
 template <int VEC>
-struct Pack { float v[VEC]; };
+struct Pack {
+  float v[VEC];
+  DEV void operator+=(const Pack& o) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) v[j] += o.v[j];
+  }
+};
 
 template <int VEC>
 DEV Pack<VEC> ld_pack(const float* p) {
@@ -101,12 +107,7 @@ __global__ __launch_bounds__(256) void stream_mix_kernel(StreamMixParams p) {
       for (int s = 0; s < S; ++s) xs[s] = ld_pack<VEC>(x + (int64_t)s * W + d);
     }
     if (y) {
-      Pack<VEC> yv = ld_pack<VEC>(y + d);
-      for (int k = 1; k < p.nsum; ++k) {
-        const Pack<VEC> t = ld_pack<VEC>(y + (int64_t)k * W + d);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) yv.v[j] += t.v[j];
-      }
+      const Pack<VEC> yv = add_parts<Pack<VEC>>(p.nsum, [&](int k) { return ld_pack<VEC>(y + (int64_t)k * W + d); });
 #pragma unroll
       for (int t = 0; t < S; ++t)
 #pragma unroll

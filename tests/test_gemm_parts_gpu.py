@@ -72,3 +72,26 @@ def test_norms_add_parts(gpu, W, na, nb):
     close(got, want), close(gx, wx)
     with pytest.raises(RuntimeError):
         ops.add_norm_rows(c(ya), na, None, got, c(w), 1e-5, gx, None, c(yb), nb + 1)
+
+
+# the residual streams and the token inputs: vector and scalar rows, parts up to and past a group of four
+@pytest.mark.parametrize("W", [64, 130, 2048])
+@pytest.mark.parametrize("parts", [1, 5, 9])
+def test_streams_and_token_inputs_add_parts(gpu, W, parts):
+    M, S, F, g = 5, 2, 24, torch.Generator().manual_seed(W + parts)
+    r = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    c = lambda t: t.to(gpu)  # noqa: E731
+    close = lambda a, b: torch.testing.assert_close(a.cpu(), b, rtol=2e-5, atol=5e-5)  # noqa: E731
+    y, streams, outw, mix, inw, nw = r(M * parts, W), r(M, S, W), r(S), r(S, S), r(S), r(W)
+    want, wh, wt = streams.clone(), torch.zeros(M, W), torch.zeros(M, W)
+    got, gh, gt = c(streams.clone()), torch.zeros(M, W, device=gpu), torch.zeros(M, W, device=gpu)
+    lref.stream_mix(y, parts, 0.6, want, None, None, 1.0, outw, mix, inw, nw, 1e-5, wh, wt)
+    ops.stream_mix(c(y), parts, 0.6, got, None, None, 1.0, c(outw), c(mix), c(inw), c(nw), 1e-5, gh, gt)
+    close(got, want), close(gh, wh), close(gt, wt)
+
+    resid, ga, sn, go = r(M, W), r(W), r(W), r(W)
+    gate_w, proj_w, table, ids = r(F, W) / W ** 0.5, r(W, F) / F ** 0.5, r(30, F), torch.arange(M, dtype=torch.int32)
+    want, wx, got, gx = resid.clone(), torch.zeros(M, W), c(resid.clone()), torch.zeros(M, W, device=gpu)
+    lref.token_side_rows(y, parts, ga, want, ids, table, 0, gate_w, proj_w, sn, go, 1e-5, wx, None)
+    ops.token_side_rows(c(y), parts, c(ga), got, c(ids), c(table), 0, c(gate_w), c(proj_w), c(sn), c(go), 1e-5, gx, None)
+    close(got, want), close(gx, wx)
