@@ -26,6 +26,8 @@ struct GemmRmParams {
 };
 // gemm_rm_strip.hip: rows 48 or 80; fp32 operands of whole 128-byte chunks (gemm_rowmajor.hip lds_ok)
 hipError_t gemm_rm_strip(int rows, const GemmRmParams& p, hipStream_t st);
+// gemm_rowmajor.hip: rows of the fp32 form for many tiles: 64 (64 x 64 tiles), 48 or 80 (strips)
+int gemm_rm_form_rows(int M, int N, int batch);
 
 struct ScalarNormParams {
   const float* y;    // [M * nsum, W] sublayer output, a row's nsum consecutive parts are summed (mode 0) -- unused in mode 1

@@ -676,6 +676,8 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor(d!)? scratch=None, bool alone=False, int longest=0) -> ()");
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
+  m.def("gemm_rm_form_rows(int M, int N, int batch=1) -> int",
+        [](int64_t M, int64_t N, int64_t batch) { return (int64_t)dsse::gemm_rm_form_rows((int)M, (int)N, (int)batch); });
   m.def("moe_plan(int M, int W, int F, int Fs, int E, int top, bool gated) -> int", &moe_plan);
   m.def("moe_parts(Tensor x, int top, Tensor? gate, Tensor up, Tensor down, Tensor? sgate, Tensor? sup, Tensor? sdown, Tensor h) -> int");
   m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "

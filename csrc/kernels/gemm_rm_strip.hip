@@ -1,4 +1,4 @@
-// The row-major GEMM of the exact mode in strips: chosen, and compared with the 64 x 64 tiles, in gemm_rowmajor.hip (launch_rows).
+// The row-major GEMM of the exact mode in strips: chosen, and compared with the 64 x 64 tiles, in gemm_rowmajor.hip (gemm_rm_form_rows).
 #include "api_layers.h"
 #include "frag.h"
 #include "lds_dma.h"

@@ -297,18 +297,10 @@ hipError_t launch_lds(const GemmRmParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// 64 x 64 tiles or strips of 48 or 80 rows, whichever the busiest CU is through first.  A CU's tiles of K = 2048 take 28 us each as
-// strips of 48 rows (one or three of them 24 more: alone on its CU a strip waits for its fragments), 36 as 64 x 64, 46 of 80 rows (one
-// 10 more).  Strips of 96 rows were the faster form nowhere by more than 3 %.
+// 64 x 64 tiles or strips of 48 or 80 rows, whichever are through first
 hipError_t launch_rows(const GemmRmParams& p, hipStream_t st) {
-  auto tiles = [&](int rows) {  // of the busiest CU
-    return ((int64_t)((p.M + rows - 1) / rows) * ((p.N + 63) / 64) * p.batch + 255) / 256;
-  };
-  const int64_t n48 = tiles(48), n64 = tiles(64), n80 = tiles(80);
-  const int64_t t48 = 28 * n48 + (n48 == 1 || n48 == 3 ? 24 : 0), t64 = 36 * n64, t80 = 46 * n80 + (n80 == 1 ? 10 : 0);
-  if (t48 < t64 && t48 <= t80) return gemm_rm_strip(48, p, st);
-  if (t80 < t64) return gemm_rm_strip(80, p, st);
-  return launch_lds<float, 2, 1>(p, st);
+  const int rows = gemm_rm_form_rows(p.M, p.N, p.batch);
+  return rows == 64 ? launch_lds<float, 2, 1>(p, st) : gemm_rm_strip(rows, p, st);
 }
 
 // Whole 128-byte chunks of 16-byte-aligned rows, each operand inside a 2 GiB buffer range
@@ -330,7 +322,7 @@ hipError_t dispatch(const GemmRmParams& p, hipStream_t st) {
     return hipGetLastError();
   }
   if (lds_ok<T>(p)) {
-    // 64 x 64 tiles (fp32: or strips, launch_rows) while they fill the CUs; two wave groups per tile when there is one tile per CU at most (nothing else
+    // 64 x 64 tiles (fp32: or strips, gemm_rm_form_rows) while they fill the CUs; two wave groups per tile when there is one tile per CU at most (nothing else
     // would run while a wave waits for its fragments: 400 rows of 2048 x 2048 in fp32 45.4 -> 42.2 us); 32 x 32 tiles, four
     // groups each, while those make one round (64 rows of 2048 x 8192 in fp32 157 -> 50 us, 400 rows of 576 x 4096 in bf16
     // 19 -> 11 us).  A second round of them pays in fp32 (bound by the matrix rate) where the groups have four chunks each;
@@ -353,6 +345,32 @@ hipError_t dispatch(const GemmRmParams& p, hipStream_t st) {
 }
 
 }  // namespace
+
+// LDS holds two workgroups of each form per CU, so a launch runs in rounds of 512, and what is left for the last one counts: 257
+// workgroups and more take a round's time; fewer share no CU and take more than half of it, since a workgroup alone on its CU waits for its
+// fragments; from some 160 on they go in pairs to the CUs that are free first, except for the longest ones.  Units: 1 us at K = 2048.  Over 171
+// products (K 512, 2048 and 4096, 2048 to 16384 columns, 80 to 800 rows) the choice is within 0.3 % of the best of the three forms, 4 %
+// at the worst.  us at K = 2048, 48 rows / 64 x 64 / 80 rows: 8192 columns, 330 rows 108 / 136 / 140, 400 rows 140 / 138 / 141; 12288, 130
+// rows 89 / 108 / 91, 240 rows 110 / 130 / 140; 16384, 130 rows 99 / 135 / 92, 330 rows 194 / 209 / 228, 400 rows 247 / 247 / 228; one round of
+// K = 224 (longer ones of 64 x 64 tiles are split over wave groups): 330 x 2048 7.6 / 9.0 / 10.6, 400 x 2048 10.4 / 9.1 / 10.7.  Strips of 96
+// rows were the faster form nowhere by more than 3 %.
+int gemm_rm_form_rows(int M, int N, int batch) {
+  struct Form {
+    int rows, round, alone, paired, only;  // a round; up to 160, up to 256 workgroups behind full rounds; up to 256 and no others
+  };
+  static constexpr Form kForms[3] = {{64, 69, 39, 62, 53}, {48, 54, 34, 40, 52}, {80, 90, 50, 50, 55}};
+  int best = 0;
+  int64_t least = 0;
+  for (const Form& f : kForms) {
+    const int64_t tiles = (int64_t)((M + f.rows - 1) / f.rows) * ((N + 63) / 64) * batch, full = tiles / 512, left = tiles % 512;
+    int64_t t = full * f.round;
+    if (left > 256) t += f.round;
+    else if (left > 0) t += full == 0 ? f.only : (left > 160 ? f.paired : f.alone);
+    if (!best || t < least) best = f.rows, least = t;
+  }
+  return best;
+}
+
 }  // namespace dsse
 
 extern "C" hipError_t dsse_gemm_rm(const dsse::GemmRmParams* p, hipStream_t st) {

@@ -14,7 +14,7 @@ def _bound(K):
     return 4.0 * (K + 1) ** 0.5 * 2.0 ** -24
 
 
-# (48-row strips: 130 and 97 rows; 80-row strips: 400, 330 and 81 rows; 64 x 64: 256) x columns that end inside a strip's 64
+# (48-row strips: 130, 81, 240 and 800 rows; 80-row strips: 400 and 330; 64 x 64: 97 and 256) x columns that end inside a strip's 64
 @pytest.mark.parametrize("M,N,K,Z", [(130, 8200, 96, 1), (97, 16390, 128, 1), (400, 6272, 160, 1), (330, 2051, 96, 3), (400, 16384, 32, 1),
                                      (81, 16300, 256, 1), (256, 8192, 96, 1), (240, 12000, 2048, 1), (800, 3300, 544, 1)])
 def test_strips(M, N, K, Z):
