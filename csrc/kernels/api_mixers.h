@@ -87,6 +87,12 @@ struct SinkAttnParams {
   float once;            // ... pages of more bytes than this in one launch are read non-temporally
 };
 
+// Whether a decode launch of `rows` rows with `tokens` cached tokens together walks more than `once` bytes of bf16 pages
+__host__ __device__ inline bool sink_reads_past(float tokens, float rows, int window, int G, int D, int V, float once) {
+  const float seen = rows * (float)window;
+  return (tokens < seen ? tokens : seen) * (float)(G * 2 * (D + V)) > once;
+}
+
 // Whether the exact mode's shared-page form (sink_exact.hip) takes a launch of num_work items of p.qt rows: fp32, head widths up
 // to 128 in multiples of 16, 16 / 32 / 64 rows per item with groups of 4 / 2 / 1 heads, no output rotation, 16-byte-aligned rows.
 bool sink_exact_ok(const SinkAttnParams& p, int64_t num_work);

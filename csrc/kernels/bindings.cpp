@@ -1413,6 +1413,12 @@ void ar_gather(const Tensor& cand, Tensor& out, const Tensor& peers, int64_t ran
 
 int64_t kernels_abi_version() { return 16; }
 
+// The streaming and ring kernels' (waves per workgroup, K slices) for a product that takes one of them; (0, 0): none does
+std::tuple<int64_t, int64_t> stream_plan(int64_t M, int64_t N, int64_t K) {
+  const SCfg c = pick_stream((int)M, (int)N, (int)K);
+  return c.ok ? std::tuple<int64_t, int64_t>{c.nw, c.S} : std::tuple<int64_t, int64_t>{0, 0};
+}
+
 // The dispatch's choice for an (M, N, K) projection: (impl, tiled cfg, split, fix, model estimate in us) -- impl as
 // gemm_impl (4 = tiled / pipe); cfg / split / fix / estimate only for impl 4 (tools/bench_decode_gemm.py --plan).
 std::tuple<int64_t, int64_t, int64_t, bool, double> gemm_plan(int64_t M, int64_t N, int64_t K, bool slab_consumer) {
@@ -1557,6 +1563,7 @@ TORCH_LIBRARY(dsse, m) {
         "Tensor(c!) err) -> ()");
   m.def("kernels_abi_version() -> int", &kernels_abi_version);
   m.def("gemm_plan(int M, int N, int K, bool slab_consumer=False) -> (int, int, int, bool, float)", &gemm_plan);
+  m.def("stream_plan(int M, int N, int K) -> (int, int)", &stream_plan);
   m.def("gemm_fix_timeouts(int device=0) -> int", &gemm_fix_timeouts);
   m.def("gemm_fix_stamps(int device=0) -> Tensor", &gemm_fix_stamps);
   m.def("step_stamps_arm(int device=0, int cap=0) -> bool", &step_stamps_arm);

@@ -972,6 +972,10 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "float scale, int qt, Tensor? vt=None, bool split=False, float softcap=0.0, Tensor? out_rope=None, "
         "Tensor? rel=None, int keep_first=0, float out_scale=1.0, Tensor(b!)? part=None, int nparts=1, "
         "Tensor? walked=None, float once=0.0) -> ()");
+  m.def("sink_reads_past(int tokens, int rows, int window, int G, int D, int V, float once) -> bool",
+        [](int64_t tokens, int64_t rows, int64_t window, int64_t G, int64_t D, int64_t V, double once) {
+          return dsse::sink_reads_past((float)tokens, (float)rows, (int)std::min<int64_t>(window, INT32_MAX), (int)G, (int)D, (int)V, (float)once);
+        });
   m.def("gate_math(Tensor(a!) x, int kind, Tensor? p1=None, Tensor? p2=None, float c=1.0) -> ()");
   m.def("gate_pair(Tensor(a!) x, Tensor p1, Tensor p2) -> ()");
   m.def("matrix_scan(Tensor q, Tensor k, Tensor v, Tensor? decay, Tensor? beta, Tensor(a!) state, Tensor q_start, "

@@ -770,8 +770,7 @@ __global__ __launch_bounds__(NW * 64) void sink_decode_kernel(SinkAttnParams p, 
   };
   int blks = ids_from(0);
   // all rows decide alike; one column tile only: a second one reads the pages again
-  const bool past = !EXT && rep <= 16 && p.walked &&
-                    fminf((float)*p.walked, (float)gridDim.x * (float)p.window) * (float)(p.G * 2 * (D + V)) > p.once;
+  const bool past = !EXT && rep <= 16 && p.walked && sink_reads_past((float)*p.walked, (float)gridDim.x, p.window, p.G, D, V, p.once);
   bf16* qs = reinterpret_cast<bf16*>(smem_raw);
   float* rels = reinterpret_cast<float*>(smem_raw + 16 * ldq * sizeof(bf16));   // [cols][rel_lds]
   float* mg = rels + cols * rel_lds;                                            // [NW][cols][V + 2]

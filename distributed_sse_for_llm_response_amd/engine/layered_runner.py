@@ -1345,10 +1345,13 @@ class LayeredRunner(RunnerBase):
 
     def _worth_a_fork(self, L, M: int) -> bool:
         """Whether M rows keep the GPU longer in one layer than the host needs to issue it with a fork and a join: two waits across
-        streams of some 17 us each and their events, 210 us a layer in all against 137 on one stream.  The layer's time from its
-        weights at 5 TB/s, its products at 500 TFLOP/s and 60 us of small launches.  One stream / two, six layers of 2048 wide with
-        16 experts of 1408: 64 rows 825 / 1230 us, 150 rows 1042 / 1280, 300 rows 1183 / 1298, but 500 rows 1367 / 1309, 800 rows
-        1631 / 1356; 4096 wide with experts of 3584: 64 rows 2086 / 2177, 200 rows 2795 / 2664, 500 rows 3509 / 3239."""
+        streams of some 17 us each and their events, 210 us a layer in all against 137 on one stream.  The layer's time is estimated from
+        the weights of all experts at 5 TB/s, its products at 500 TFLOP/s and 60 us of small launches, which is on the high side (64 rows of the
+        wider model 461 us a layer, 342 measured): the line is where the measured times cross.  One stream / two, means of five processes,
+        six layers of 2048 wide with 16 experts of 1408: 64 rows 823 / 1120 us, 150 rows 1029 / 1207, 300 rows 1160 / 1233, but 400 rows
+        1278 / 1252, 700 rows 1442 / 1250, 1024 rows 1859 / 1513 (500 rows 1342 / 1437 all the same); 4096 wide with experts of 3584, always
+        two: 32 rows 2025 / 1957, 64 rows 2110 / 2050, 200 rows 2771 / 2624, 500 rows 3463 / 3274, where 8 rows (1478 / 1524), 16 (1912 /
+        2007) and 128 (2493 / 2586) would be 3 to 5 % faster on one."""
         f, m, W = L.mlp, L.mixer, self.cfg.width
         met = (2 * m.heads + 2 * m.kv_heads) * m.dim + m.heads * m.vdim  # columns of the mixer's projections
         ff = 3 * (f.experts * f.ff + f.shared_ff), 3 * (f.top * f.ff + f.shared_ff)

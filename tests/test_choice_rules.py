@@ -1,0 +1,67 @@
+"""Rules that choose between forms of equal results, on both sides of their lines as measured: host code only."""
+from types import SimpleNamespace as NS
+
+import pytest
+import torch
+
+from distributed_sse_for_llm_response_amd import ops
+from distributed_sse_for_llm_response_amd.engine.layered_runner import LayeredRunner
+from distributed_sse_for_llm_response_amd.models import registry
+
+
+# attention layers of 8 heads of 128 + 128 in bf16, bytes of a row's states: which rows x tokens read their pages past the caches
+@pytest.mark.parametrize("layers,state,rows,tokens,past", [
+    (6, 2.0e6, 8, 1500, False), (6, 2.0e6, 16, 700, False), (6, 2.0e6, 16, 500, False), (6, 2.0e6, 16, 2000, True), (6, 2.0e6, 32, 500, True),
+    (6, 2.0e6, 64, 100, True), (6, 2.0e6, 64, 500, True), (2, 12.6e6, 8, 1500, False), (2, 12.6e6, 16, 250, False), (2, 12.6e6, 16, 1000, True),
+    (2, 12.6e6, 32, 250, True)])
+def test_pages_past_the_caches(layers, state, rows, tokens, past):
+    r = NS(_slot_bytes=state, kv=NS(k=range(layers)))
+    ops.load_library(required=True)
+    assert torch.ops.dsse.sink_reads_past(rows * tokens, rows, 2 ** 31 - 1, 8, 128, 128, LayeredRunner._walk_once(r, rows)) == past
+
+
+# the kernel's side of the rule: a window bounds what a row walks, keys and values of other widths count what they hold
+@pytest.mark.parametrize("tokens,rows,window,G,D,V,share,past", [
+    (1056, 6, 10 ** 9, 8, 128, 128, 0.9, True), (1056, 6, 10 ** 9, 8, 128, 128, 6.0, False), (1056, 6, 45, 2, 64, 64, 0.9, False),
+    (1056, 6, 45, 2, 64, 64, 0.25, True), (1056, 6, 10 ** 9, 2, 64, 128, 0.99, True), (1056, 6, 10 ** 9, 2, 64, 128, 1.01, False), (0, 6, 10 ** 9, 8, 128, 128, 0.9, False)])
+def test_bytes_of_a_walk(tokens, rows, window, G, D, V, share, past):
+    ops.load_library(required=True)
+    assert torch.ops.dsse.sink_reads_past(tokens, rows, window, G, D, V, share * 1056 * G * 2 * (D + V)) == past
+
+
+def test_bytes_of_a_slot():
+    """What the rule counts as a row's state: one slot of every recurrent cache, idle rows of a bucket like live ones."""
+    fam, cfg, _ = registry.resolve("lobidra-tiny")
+    w = registry.load_weights(fam, cfg, None, device=torch.device("cpu"), seed=0, dtype=torch.float32)
+    r = registry.make_runner(fam, w, num_blocks=8, max_batch=4, max_model_len=64, device=torch.device("cpu"))
+    one, four = r._walk_once(1), r._walk_once(4)
+    caches = [t for k in ("state", "norm", "tail") for t in getattr(r.state, k, {}).values()]
+    assert caches and r._slot_bytes == sum(t.numel() * t.element_size() // t.shape[0] for t in caches)
+    assert one > four >= 1.0
+    assert abs((one - four) * len(r.kv.k) - 3 * 1.5 * r._slot_bytes) <= 64.0
+
+
+# joint layers on two streams: the 2048 wide model from some 400 rows on, the 4096 wide one always
+@pytest.mark.parametrize("model,rows,two", [("kagorax-mid", 64, False), ("kagorax-mid", 150, False), ("kagorax-mid", 300, False), ("kagorax-mid", 400, True),
+                                            ("kagorax-mid", 1024, True), ("kagorax-wide", 32, True), ("kagorax-wide", 64, True),
+                                            ("kagorax-wide", 200, True), ("kagorax-wide", 500, True)])
+def test_joint_layers_on_two_streams(model, rows, two):
+    cfg = registry.resolve(model)[1]
+    layer = next(L for L in cfg.layers if L.mlp is not None)
+    assert LayeredRunner._worth_a_fork(NS(cfg=cfg), layer, rows) == two
+
+
+# 17 to 64 rows: one round of workgroups, eight waves where four would make more; 65 rows and 16 keep the wider line
+@pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K,waves,slices", [(4096, 4096, 4, 4), (8192, 512, 4, 1), (8192, 4096, 4, 2), (8256, 4096, 4, 1), (10240, 1024, 4, 1), (10240, 4096, 4, 1),
+                                              (16384, 512, 4, 1), (16448, 512, 4, 1), (16512, 512, 8, 1), (24448, 512, 8, 1), (32768, 4096, 8, 1)])
+def test_one_round_of_workgroups(M, N, K, waves, slices):
+    ops.load_library(required=True)
+    assert torch.ops.dsse.stream_plan(M, N, K) == (waves, slices)
+
+
+@pytest.mark.parametrize("M,N,K,want", [(16, 10240, 4096, (4, 2)), (65, 10240, 4096, (4, 2)), (65, 16512, 512, (4, 1)), (33, 28672, 4096, (7, 1)),
+                                        (17, 28672, 4096, (8, 1)), (33, 60, 4096, (0, 0))])
+def test_other_rows(M, N, K, want):
+    ops.load_library(required=True)
+    assert torch.ops.dsse.stream_plan(M, N, K) == want
