@@ -324,10 +324,9 @@ struct TCfg {
   double est_us = 0;   // the cost model's estimate (pipe_plan), 0 for the table's choices
 };
 
-// Cost model of one gemm_pipe launch (round 6, profiles/r6/gemm_model_r6.md).  A workgroup is bound by its LDS
-// fill (X rows + weight rows through LDS-DMA: fitted, ~44 GB/s per CU; the path itself carries 125 and more from L2)
-// or by its MFMA issue (~5.0 TFLOP/s
-// per CU, the kernel's rate at 8192 rows), plus ~3.3 us of pipeline fill and epilogue; one 128 KiB workgroup per CU,
+// Cost model of one gemm_pipe launch (profiles/r6/gemm_model_r6.md).  A workgroup is bound by its LDS
+// fill (X rows + weight rows through LDS-DMA: ~44 GB/s per CU, fitted; tools/fillbench.hip draws 45 to 47 of half rows from L2, half
+// weights from memory) or by its MFMA issue (~5.0 TFLOP/s per CU, the kernel's rate at 8192 rows), plus ~3.3 us of pipeline fill and epilogue; one 128 KiB workgroup per CU,
 // so the grid runs in rounds of 256, a partial last round at 0.67 + 0.33 x its fill of a full one's time.  Split K
 // costs the fp32 partial tiles: combined in the launch (FIX) ~7 us of store / release / wait plus the last arriver
 // reading S - 1 slots at ~26 GB/s (the stamps of profiles/r6/pipe_fix_stamps_r6.log), or left as slabs for the

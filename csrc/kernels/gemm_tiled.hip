@@ -58,8 +58,8 @@ DEV void glds16(const void* src, char* lds_base) {
 constexpr bool kBurst = DSSE_TILED_BURST;  // A/B build only: every tile issues its stage in one burst
 
 // ROWS: one tile holds all rows (65 to 256, MT of 3 to 8 sub-tiles per wave row) and 128 columns, so that every weight is fetched
-// once, non-temporal, and no row that is not there is fetched; four stages where they fit.  What bounds it is how fast this schedule
-// fills LDS, 45 GB/s per CU: (rows + 128) x 128 bytes per K step.  Mistral's gate_up at 160 rows: 57 us (0.86 us per step) against
+// once, non-temporal, and no row that is not there is fetched; four stages where they fit.  What bounds it is the LDS fill, 45 GB/s
+// per CU of rows from L2 and weights from memory together: (rows + 128) x 128 bytes per K step.  Mistral's gate_up at 160 rows: 57 us (0.86 us per step) against
 // 69 with two row blocks of 128 x 256; with 192 rows computed for 160 the same, with 256 66.  A column
 // block begins at a K step of its own and wraps around: X has just been written on other XCDs, and workgroups that ask for different
 // parts of it bring it into their XCD's L2 for each other (160-stream decode step 6201 -> 6075 us, 200-row prompt 6277 -> 6108).

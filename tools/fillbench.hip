@@ -1,20 +1,16 @@
-// Per-CU fill-rate microbenchmark (round 3; round 6: 4 or 8 waves per workgroup, up to 32 KiB in flight per wave,
-// X footprints of 2 MiB (one XCD's L2) and 8 MiB (spills the 4 MiB L2 into the Infinity Cache)): how many bytes
-// per second one CU can bring on chip, by path.
+// Per-CU fill-rate microbenchmark: how many bytes per second one CU can bring on chip, by path, with 4 or 8 waves per workgroup, up to
+// 20 KiB in flight per wave, and X footprints of 2 MiB (one XCD's L2) and 8 MiB (more than its 4 MiB).
 //
-// Read its results as lower bounds: every piece pays a 64-bit modulo for its address, and pieces that hit the L2 arrive at 125 to 147
-// GB/s per CU without it.
-//
-// The decode GEMMs at 64-256 rows all measured ~35-39 GB/s of LDS-DMA fill per CU (gemm_ring at 64 rows,
-// gemm_tiled at 256 rows and at 8192 rows alike: profiles/r3/fillbench.md), which bounds them whatever the
-// MFMA work.  This program measures the paths separately and together, one 256-thread workgroup per CU:
+// On one MI355X (profiles/floors/fillbench.txt), GB/s per CU: X alone 90 with four waves, 140 with eight, weights alone 27 to 28 (6.9 to 7.2
+// TB/s for the chip), half of each 45 to 47, of which the weights are 6 TB/s.  The decode GEMMs at 64-256 rows measured 35-39 of such a
+// mix.  One workgroup per CU:
 //   mode 0  X: global_load_lds_dwordx4 (LDS-DMA) of an L2-resident 2 MiB buffer, every wave loading
 //   mode 1  W: global_load_dwordx4 into VGPRs (nt) streaming a 2 GiB buffer once (HBM)
 //   mode 2  W: buffer_load ... lds (LDS-DMA, nt) streaming the 2 GiB buffer (the ring GEMM's weight path)
 //   mode 3  waves 0-1 as mode 0, waves 2-3 as mode 1 (the two paths at once, separate vmcnt counters)
 //   mode 4  waves 0-1 as mode 0, waves 2-3 as mode 2
 // with D 1-KiB pieces in flight per wave.  Prints GB/s per CU and chip-wide.
-//   hipcc --offload-arch=gfx950 -O3 -o fillbench tools/fillbench.hip && ./fillbench
+//   hipcc --offload-arch=gfx950 -O3 -Xclang -target-feature -Xclang -packed-fp32-ops -o fillbench tools/fillbench.hip && ./fillbench
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -69,7 +65,7 @@ __global__ void __launch_bounds__(512) fill_kernel(const char* __restrict__ x, c
   if (x_role) {
     const size_t start = ((size_t)blockIdx.x * NW + wave) * 4096;
     for (int i = 0; i < iters; ++i) {
-      const size_t off = (start + (size_t)i * 1024) % xb;  // 1-KiB aligned, inside the X buffer
+      const size_t off = (start + (size_t)i * 1024) & (xb - 1);  // 1-KiB aligned, inside the X buffer (xb a power of two)
       glds(x + off + lane * 16, ring + (i % D) * 1024);
       wait_vm<D>();
     }
