@@ -70,7 +70,8 @@ extern "C" hipError_t dsse_qkv_rows(const dsse::QkvRowsParams* p, hipStream_t st
   if (p->D > 64 * dsse::kHeadRegs || p->V > 64 * dsse::kHeadRegs) return hipErrorInvalidValue;
   // queries, keys and values as three sets of heads where all go by fours (stream_ops.hip) and the rows fill more than one round of
   // workgroups.  Heads 16 + 8 + 8 of 128, this kernel / by fours: 192 decode rows 6.2 / 6.2 us, 256 8.0 / 7.2, prompts of 300 rows 6.3 / 4.8
-  // (three of them 6.4 / 5.0), 1500 rows 21.3 / 11.6, 3000 rows 36 / 19.
+  // (three of them 6.4 / 5.0), 1500 rows 21.3 / 11.6, 3000 rows 36 / 19.  Beside the experts' products of a captured step more, smaller
+  // workgroups are through sooner: the decode step of 192 streams 1005 / 1030 us, 224 streams 1101 / 1098, 256 streams 1136 / 1121.
   dsse::NormRopeList l{};
   auto set = [&](int nh, int D, int col, int kind, void* out, const int* rows) {
     dsse::NormRopeParams& s = l.p[l.n++];
@@ -85,7 +86,7 @@ extern "C" hipError_t dsse_qkv_rows(const dsse::QkvRowsParams* p, hipStream_t st
     set(p->G, p->V, (p->H + p->G) * p->D, 0, p->v, p->slots);
     l.p[2].out_t = p->vt;
   }
-  if (p->T >= 192 && dsse_norm_rope_all_fours(l)) return dsse_norm_rope_rows(l, st);
+  if (p->T > 192 && dsse_norm_rope_all_fours(l)) return dsse_norm_rope_rows(l, st);
   const int heads = p->H + (p->k ? 2 * p->G : 0);
   const dim3 grid(p->T, (heads + 3) / 4);
   if (p->f32) hipLaunchKernelGGL(dsse::qkv_rows_kernel<float>, grid, dim3(256), 0, st, *p);

@@ -138,6 +138,7 @@ FLASH_DECODE_WAVES = 512  # waves a decode attention launch aims for (two per CU
 # since part of the pages is still found there.  A byte of recurrent state, read and written back, counts half as much again.
 WALK_CACHED = 340e6
 WALK_STATE = 1.5
+WALK_ROWS = 2  # prompt rows whose products take a joint layer as long as a decode row's walk through its pages, some 0.4 us
 SINK_DECODE_GROUPS = 512  # workgroups a decode launch of the sink attention aims for (two per CU)
 SINK_DECODE_PAGES = 32    # fewest pages of a full cache that a workgroup's stretch of a split walk is worth
 SINK_ROWS_TILE = 16   # query rows per work item of the sink attention's MFMA form (one head per wave)
@@ -1318,6 +1319,7 @@ class LayeredRunner(RunnerBase):
         cfg, w, eps = self.cfg, self.w, self.cfg.eps
         # a captured step forks for nothing on the host
         capturing = self._side_stream is not None and torch.cuda.is_current_stream_capturing()
+        met = M + WALK_ROWS * sum(g["ws"].numel() for g in groups if g["qt"] == 1)  # a mixed step's decode rows walk their pages
         ops.embed_rows(ids, w.embed, d["resid"], None, cfg.embed_scale, pos, self._pos_table)
         none = (None, 1, None, 1)
         pending = none  # sublayer outputs that are not in the stream yet: (rows, parts per row) of both
@@ -1326,7 +1328,7 @@ class LayeredRunner(RunnerBase):
             ops.add_norm_rows(y, nsum, None, d["resid"], Lw.norm1, eps, d["xb"], d["hn"] if L.mlp is not None else None, y2, nsum2)
             if L.mlp is None:
                 pending = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups) + (None, 1)
-            elif self._side_stream is None or not (capturing or self._worth_a_fork(L, M)):
+            elif self._side_stream is None or not (capturing or self._worth_a_fork(L, met)):
                 mixed = self._attention_joint(i, L.mixer, Lw.mix, M, d, slots, groups)
                 pending = self._input_weighted_ff(L.mlp, Lw.mlp, M, d) + mixed
             else:
@@ -1351,7 +1353,9 @@ class LayeredRunner(RunnerBase):
         six layers of 2048 wide with 16 experts of 1408: 64 rows 823 / 1120 us, 150 rows 1029 / 1207, 300 rows 1160 / 1233, but 400 rows
         1278 / 1252, 700 rows 1442 / 1250, 1024 rows 1859 / 1513 (500 rows 1342 / 1437 all the same); 4096 wide with experts of 3584, always
         two: 32 rows 2025 / 1957, 64 rows 2110 / 2050, 200 rows 2771 / 2624, 500 rows 3463 / 3274, where 8 rows (1478 / 1524), 16 (1912 /
-        2007) and 128 (2493 / 2586) would be 3 to 5 % faster on one."""
+        2007) and 128 (2493 / 2586) would be 3 to 5 % faster on one.  Mixed steps, 2048 wide, streams of 400 tokens + prompt rows: 16 + 128
+        1194 / 1336, 64 + 64 1200 / 1267, 16 + 300 1311 / 1348, 64 + 190 1370 / 1426, but 64 + 300 1450 / 1359, 128 + 64 1495 / 1414, 128 + 128 1523 /
+        1432: a decode row counts as WALK_ROWS more; 4096 wide, 64 + 128 3004 / 2755, 128 + 128 3365 / 2990."""
         f, m, W = L.mlp, L.mixer, self.cfg.width
         met = (2 * m.heads + 2 * m.kv_heads) * m.dim + m.heads * m.vdim  # columns of the mixer's projections
         ff = 3 * (f.experts * f.ff + f.shared_ff), 3 * (f.top * f.ff + f.shared_ff)

@@ -51,6 +51,29 @@ def test_joint_layers_on_two_streams(model, rows, two):
     assert LayeredRunner._worth_a_fork(NS(cfg=cfg), layer, rows) == two
 
 
+# mixed steps: decode rows with their walks beside prompt rows
+@pytest.mark.parametrize("streams,rows,two", [(4, 64, False), (16, 128, False), (64, 32, False), (64, 64, False), (16, 300, False), (64, 190, False), (64, 300, True), (128, 64, True),
+                                              (128, 300, True)])
+def test_mixed_steps_on_two_streams(streams, rows, two):
+    cfg = registry.resolve("kagorax-mid")[1]
+    layer = next(L for L in cfg.layers if L.mlp is not None)
+    taken = []
+
+    def rule(L, M):
+        taken.append(LayeredRunner._worth_a_fork(NS(cfg=cfg), L, M))
+        raise StopIteration
+
+    groups = [{"qt": 1, "ws": torch.zeros(streams)}, {"qt": 4, "ws": torch.zeros(rows // 4)}]
+    runner = NS(cfg=NS(layers=[layer], eps=cfg.eps, embed_scale=1.0), w=NS(layers=[NS(norm1=None)], embed=None), _side_stream=True, _pos_table=None, _worth_a_fork=rule)
+    with pytest.MonkeyPatch.context() as m:
+        for name in ("embed_rows", "add_norm_rows"):
+            m.setattr(ops, name, lambda *a, **k: None)
+        m.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        with pytest.raises(StopIteration):
+            LayeredRunner._joint_layers(runner, streams + rows, dict.fromkeys(("resid", "xb", "hn")), None, None, None, groups, None)
+    assert taken == [two]
+
+
 # 17 to 64 rows: one round of workgroups, eight waves where four would make more; 65 rows and 16 keep the wider line
 @pytest.mark.parametrize("M", [17, 33, 64])
 @pytest.mark.parametrize("N,K,waves,slices", [(4096, 4096, 4, 4), (8192, 512, 4, 1), (8192, 4096, 4, 2), (8256, 4096, 4, 1), (10240, 1024, 4, 1), (10240, 4096, 4, 1),
