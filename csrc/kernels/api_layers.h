@@ -156,10 +156,11 @@ struct MoeGroupedParams {
   const void* sgate;     // shared expert (slot `top`, expert index E) or null
   const void* sup;
   const void* sdown;
-  int* sorted;           // [max_tiles * 64] ids (row * S + slot) grouped by expert, -1 = pad
+  int* sorted;           // [max_tiles * 64] ids (row * S + slot) grouped by expert, -1 = pad; 64 counters behind them, left at 0
   int* tile_expert;      // [max_tiles]
   int* num_tiles;        // [1]
   void* h;               // [M * S, ldh] element type
+  float* ws;             // [kMoeCutFloats]: the pieces of tiles that are cut over K (moe_pipe.hip), or null: none is
   float* o;              // [M * parts, W]: a row's parts are its slots, and the further slices of the shared expert's
   int M, W, F, Fs, E, top, S, ldh, max_tiles;
   int parts;             // S, or S + n: the shared expert's down product in n + 1 slices of its hidden units (moe_parts)
@@ -167,9 +168,10 @@ struct MoeGroupedParams {
   int aligned;           // 1: sorted / tile_expert / num_tiles are already made (moe_route_rows)
   int lds_tiles;         // 1: enough rows for the LDS-staged tiles (prompt portions); 0: the register-direct kernels
   int f32;
-  int form, once;        // 0: by cost; else (moe_form, moe_once of DSSE_KERNEL_CFG) form 1 stream, 2 pipeline, 3 register-direct where that
-                         // one takes the step; once 1 / 2: the pipeline's non-temporal weights on / off
+  int form, once, cut;   // 0: by cost; else (moe_form, moe_once, moe_cut of DSSE_KERNEL_CFG) form 1 stream, 2 pipeline, 3 register-direct where that
+                         // one takes the step; once 1 / 2: the pipeline's non-temporal weights on / off; cut: pieces of its last round's tiles
 };
+constexpr int64_t kMoeCutFloats = 8 * 16 * 65536;  // of moe_pipe.hip: 8 XCDs, 16 pieces of 256 x 256 at most
 
 // Shapes that the expert GEMMs on LDS-DMA take (moe_pipe.hip, moe_stream.hip): reduction lengths of whole 64-element steps,
 // two at least; 16-byte-aligned operands; every operand inside a 2 GiB buffer range.

@@ -536,6 +536,12 @@ void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, 
   p.form = dsse::kernel_cfg_int("moe_form", 0), p.once = dsse::kernel_cfg_int("moe_once", 0);
   TORCH_CHECK(p.parts == p.S || (dsse::moe_lines_ok(p) && dsse::moe_form(p) != dsse::MoeForm::kDirect && p.Fs / 64 >= 2 * (p.parts - p.S + 1)),
               "moe_grouped: this step's shared expert cannot be computed in ", p.parts - p.S + 1, " slices (moe_parts)");
+  at::Tensor ws;
+  if (p.M && dsse::moe_lines_ok(p) && dsse::moe_form(p) == dsse::MoeForm::kPipe) {
+    ws = at::empty({dsse::kMoeCutFloats}, o.options());
+    p.ws = ws.data_ptr<float>();
+    p.cut = std::clamp(dsse::kernel_cfg_int("moe_cut", 0), 0, 8);
+  }
   DSSE_CHECK_HIP(dsse_moe_grouped(&p, cur_stream()));
 }
 

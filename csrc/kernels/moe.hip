@@ -148,7 +148,8 @@ __global__ __launch_bounds__(256) void moe_ffn_kernel(MoeFfnParams p) {
 // GEMM launches serve a decode step (a few rows per expert) and a prompt portion (hundreds).
 //
 //   moe_align     one workgroup: per-expert counts -> tile-padded offsets -> sorted ids (pads -1), the expert of every
-//                 tile and the tile count.  The order of ids inside an expert is whatever the atomics give; a row's
+//                 tile and the tile count, and 64 zeros behind the list (moe_pipe's counters; the scratch holds a tile more than any
+//                 list: sum of ceil(ids of an expert / 64) <= ids / 64 + 63 / 64 per expert).  The order of ids inside an expert is whatever the atomics give; a row's
 //                 result does not depend on its place in a tile.
 //   moe_gate_up   h[id, f] = silu(gate_e[f] . x[row]) * (up_e[f] . x[row])       (element type)
 //   moe_down      o[id, :] = weight(id) * down_e . h[id]                          (fp32)
@@ -196,6 +197,7 @@ DEV void align_ids(int M, int S, int top, int E, Choice choice, int* sorted, int
   __syncthreads();
   const int total = off[NE];
   for (int i = threadIdx.x; i < total; i += blockDim.x) sorted[i] = -1;
+  if (threadIdx.x < kMoeRows) sorted[total + threadIdx.x] = 0;
   for (int e = threadIdx.x; e < NE; e += blockDim.x)
     for (int t = off[e] / kMoeRows; t < off[e + 1] / kMoeRows; ++t) tile_expert[t] = e;
   for (int t = total / kMoeRows + threadIdx.x; t < max_tiles; t += blockDim.x) tile_expert[t] = -1;

@@ -16,7 +16,8 @@
 //     for rows that are not there;
 //   * MODE 0: a column tile pair is (gate rows, up rows) of the same 16 hidden units, so silu(gate) * up needs no exchange;
 //   * order: the shared expert's tiles first (the tallest), then the routed ones; each XCD owns a contiguous eighth of both,
-//     row tiles fastest within groups of 8, so a weight panel's readers share an L2 at about the same time.
+//     row tiles fastest within groups of 8, so a weight panel's readers share an L2 at about the same time;
+//   * a few tiles past an XCD's last whole round are cut over K, so that the launch does not wait for one of them.
 //
 // Every workgroup finds its tile by itself from the work list of 64-row tiles (the experts ascend, so ballots over the list
 // give every expert's place); the host knows only a bound of the tile count.
@@ -39,7 +40,18 @@ constexpr int kA = 256 * 128;   // row image of one K step: 256 rows x 64 bf16
 constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 bf16
 constexpr int kBuf = kA + kB;
 constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), their weights (256 floats), their rows of the result (256 ints)
-constexpr size_t kLDS = kIds + 3 * 256 * 4;
+constexpr int kSay = kIds + 3 * 256 * 4;  // one word: whether this workgroup ends a cut tile
+constexpr size_t kLDS = kSay + 16;
+
+// The last round where only a few tiles are left for it: each XCD runs its tiles in rounds of one per CU, and the tiles past the last whole
+// round are cut over K.  Every piece leaves its fp32 sums in `ws`, and the one that finishes last -- a counter, nobody waits -- adds them in the
+// order of the pieces and runs the epilogue.
+constexpr int kCUs = 32;              // per XCD
+constexpr int kMostCut = 8;           // pieces of a tile
+constexpr int kPieces = 16;           // pieces per XCD
+constexpr int kCutTiles = 4;          // cut tiles per XCD: the counters are 16-bit halves of the first of the 64 ints behind the work list
+constexpr int kSlot = 8 * 32 * 64;    // f32x4 of one piece: [wave][row tile, column tile][lane]
+static_assert(8 * kPieces * kSlot * 4 == kMoeCutFloats && 8 * kCutTiles <= 2 * 64, "workspace and counters");
 
 struct Place {
   int first;  // the expert's first list tile
@@ -80,8 +92,11 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
   auto blocks = [&](int F) { return ((MODE == 1 ? p.W : F) + kCols - 1) / kCols; };
 
   List list{p.tile_expert, __builtin_amdgcn_readfirstlane(ld_global<int>(p.num_tiles)), lane, {}};
+  auto read_list = [&]() {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) list.v[c] = list.chunk(c);
+    for (int c = 0; c < 4; ++c) list.v[c] = list.chunk(c);
+  };
+  read_list();
   // list tiles of routed experts, and the row tiles they make: one per started `tall` list tiles of an expert
   int routed = 0, row_tiles = 0;
   auto walk = [&](auto f) {  // f(tile, its expert, its index inside the expert, it opens a row tile, row tiles before it)
@@ -106,13 +121,28 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
   const int nb_r = blocks(p.F), nb_s = blocks(p.Fs);
   const int slices = MODE == 1 ? p.parts - p.S + 1 : 1;  // of the shared expert's hidden units
   const int tiles_s = (shared + tall - 1) / tall * nb_s, total_s = tiles_s * slices, total_r = row_tiles * nb_r;
+  // Pieces pay where they are few -- tiles of a round that is half empty run faster than those of a full one -- and long, and where no
+  // shared expert's longer walk is what the launch waits for (MODE 1).  Without / with, one MI355X, work list and both products, us: 16 experts, top
+  // 2 and a shared one, 2048 x 1408, 1024 rows (264 tiles, one left per XCD) 152 / 144; 4096 x 3584, 200 rows 320 / 300, 1300 567 / 541,
+  // 1500 609 / 584, 3000 1030 / 1007.  With more than these left it turns: 2048 x 1408, three or four tiles left, 1100 rows 151 / 154, five to eight 1300
+  // rows 154 / 163, 1500 165 / 170; 16 K steps, 1024 x 2048, 2500 rows 174 / 178.
+  const int steps_r = (MODE == 1 ? p.F : p.W) >> 6, steps_s = total_s ? (MODE == 1 ? p.Fs / slices : p.W) >> 6 : steps_r;
+  const int most_left = p.cut ? kCutTiles : steps_r < 32 || steps_s > steps_r ? 0 : min(kCutTiles, steps_r / 16);
+  const int most_cut = p.cut ? min(p.cut, min(steps_r, steps_s) / 2) : kMostCut;
 
-  for (int v = blockIdx.x; ; v += gridDim.x) {  // one tile; a second round only if a choice list is not what it should be
-    const int x = v & 7, u = v >> 3;
+  // One tile; a second round only if a choice list is not what it should be (the list is read again for it: no registers for it in the K loop)
+  for (int v = blockIdx.x; ; v += gridDim.x, read_list()) {
+    const int x = v & 7, item = v >> 3;
     const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0;
     const int r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
-    if (u >= (total_s + 7) / 8 + (total_r + 7) / 8) return;  // past every XCD's share
+    if (item >= (total_s + 7) / 8 + (total_r + 7) / 8 + kPieces) return;  // past every XCD's share
+    // the tiles past the last whole round, each in `cut` pieces
+    const int left = (ns + nr) % kCUs;
+    const int cut = !p.ws || left < 1 || left > most_left ? 1 : min(most_cut, kPieces / left);
+    const int whole = cut > 1 ? ns + nr - left : ns + nr;
+    const int u = item < whole ? item : whole + (item - whole) / cut;
     if (u >= ns + nr) continue;
+    const int piece = item < whole ? 0 : (item - whole) % cut, of = item < whole ? 1 : cut;
     const bool sh = u < ns;
     Place pl;
     int e;
@@ -146,8 +176,9 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
 
     const int Fe = sh ? p.Fs : p.F;
     const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
-    const int slice = sh ? (s0 + u) / tiles_s : 0, cut = sh ? slices : 1;
-    const int first = (K >> 6) * slice / cut, nk = (K >> 6) * (slice + 1) / cut - first;  // its K steps
+    const int slice = sh ? (s0 + u) / tiles_s : 0, parts = sh ? slices : 1;
+    const int k0 = (K >> 6) * slice / parts, kn = (K >> 6) * (slice + 1) / parts - k0;  // its K steps
+    const int first = k0 + kn * piece / of, nk = k0 + kn * (piece + 1) / of - first;    // this piece's
     const int off = ONCE ? n0 / kCols % nk : 0;
     const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
     const int ldx = MODE == 1 ? p.ldh : p.W;
@@ -296,6 +327,50 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     step(t, std::integral_constant<int, 2>{});
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // the two rows' barrier counts meet
 
+    if (of > 1) {
+      f32x4* slots = reinterpret_cast<f32x4*>(p.ws) + (size_t)(x * kPieces + (u - whole) * cut) * kSlot;
+      int at = w * 32 * 64 + lane;
+      asm volatile("" : "+v"(at));  // addresses of this part are not made before the K loop, whose registers are full
+#pragma unroll
+      for (int m = 0; m < 8; ++m)
+        if ((m & 3) < QI)  // uniform
+#pragma unroll
+          for (int n = 0; n < 4; ++n) slots[(size_t)piece * kSlot + at + (4 * m + n) * 64] = acc[m][n];
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      int* say = reinterpret_cast<int*>(smem + kSay);
+      if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const int c = x * kCutTiles + u - whole, shift = 16 * (c & 1);
+        int* count = p.sorted + (size_t)list.n * 64 + (c >> 1);
+        const int before = __hip_atomic_fetch_add(count, 1 << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> shift & 0xffff;
+        *say = before == of - 1;
+        if (before == of - 1) __hip_atomic_fetch_sub(count, of << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (!__builtin_amdgcn_readfirstlane(*say)) continue;
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(slots, (uint32_t)(of * kSlot * 16));
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        if ((m & 3) >= QI) continue;  // uniform
+#pragma unroll
+        for (int c0 = 0; c0 < kMostCut; c0 += 4) {
+          if (c0 >= of) continue;  // uniform
+          f32x4 t[4][4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c)  // pieces that do not exist read as zeros, without traffic
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+              t[c][n] = __builtin_bit_cast(
+                  f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                             rs, c0 + c < of ? (uint32_t)(((c0 + c) * kSlot + at + (4 * m + n) * 64) * 16) : kOOB, 0, 0));
+#pragma unroll
+          for (int n = 0; n < 4; ++n) acc[m][n] = (c0 ? acc[m][n] + t[0][n] : t[0][n]) + t[1][n] + t[2][n] + t[3][n];
+        }
+      }
+    }
+
 #pragma unroll
     for (int qm = 0; qm < 2; ++qm)
 #pragma unroll
@@ -443,7 +518,7 @@ hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
     attr_set = true;
   }
   const int tall = MODE == 1 ? down_height(p, p.parts - p.S + 1).tall : moe_pipe_height(p, MODE);
-  const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8);
+  const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8 + (p.ws ? mp::kPieces : 0));
   hipLaunchKernelGGL((moe_pipe_kernel<MODE, ONCE>), dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
   return hipGetLastError();
 }
@@ -454,7 +529,7 @@ hipError_t launch_moe_pipes(const MoeGroupedParams& p, hipStream_t st) {
   return e != hipSuccess ? e : launch_moe_pipe<1, ONCE>(p, st);
 }
 
-bool pieces(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+bool sixteens(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
 
@@ -465,8 +540,8 @@ bool moe_lines_ok(const MoeGroupedParams& p) {
   if (p.f32 || p.W % 64 || p.W < 128 || p.F % 64 || p.F < 128 || (shared && (p.Fs % 64 || p.Fs < 128)) || p.ldh % 8)
     return false;
   if ((int64_t)p.M * p.W * 2 >= kRange || ids * p.ldh * 2 >= kRange || widest * p.W * 2 >= kRange) return false;
-  if (!pieces(p.x) || !pieces(p.h) || !pieces(p.up) || !pieces(p.down) || (p.gate && !pieces(p.gate))) return false;
-  return !shared || (pieces(p.sgate) && pieces(p.sup) && pieces(p.sdown));
+  if (!sixteens(p.x) || !sixteens(p.h) || !sixteens(p.up) || !sixteens(p.down) || (p.gate && !sixteens(p.gate))) return false;
+  return !shared || (sixteens(p.sgate) && sixteens(p.sup) && sixteens(p.sdown));
 }
 
 // Two slices where they end sooner.  One / two, work list, both products and the norm that adds the parts, in us: 2048 x 1408, 16 experts,

@@ -63,3 +63,50 @@ def test_pipelined_experts(gpu, pipe, M, W, F, Fs, E, top, first, gated, weight_
     err = (o.cpu().double() - ref.double()).norm() / ref.double().norm()
     assert float(err) <= 2.0 ** -8
     assert float((o.cpu() - ref).abs().max()) <= 2.0 ** -5 * float(ref.abs().max())
+
+
+# Tiles cut over K: two and more pieces of two K steps and odd ones, every height of a row tile, a shared expert, experts without a gate, a walk
+# that starts in the middle, 257 tiles (a whole round and one tile), and once by the rule itself (33 K steps).  The list's counters are zero again
+# afterwards: a second call on the same list gives the same bits.
+@pytest.mark.parametrize("M,W,F,Fs,E,top,first,gated,cut", [
+    (70, 256, 256, 0, 2, 1, 64, True, 2), (130, 448, 320, 448, 3, 2, 65, True, 3), (300, 1088, 192, 0, 4, 1, 193, True, 8), (513, 576, 320, 192, 3, 1, 257, True, 4),
+    (700, 512, 256, 0, 3, 1, 256, False, 4), (257, 512, 128, 0, 257, 1, 1, True, 4), (200, 2112, 256, 320, 2, 2, 40, True, 0)])
+@pytest.mark.parametrize("once", [1, 2], ids=["once", "plain"])
+def test_cut_tiles(gpu, monkeypatch, M, W, F, Fs, E, top, first, gated, cut, once):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2, moe_once=once, moe_cut=cut))
+    ops.refresh_env()
+    try:
+        g = torch.Generator().manual_seed(M + W + F)
+
+        def rnd(*s):
+            return (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16()
+
+        x = torch.randn(M, W, generator=g).bfloat16()
+        gate, up, down = rnd(E, F, W) if gated else None, rnd(E, F, W), rnd(E, W, F)
+        sh = (rnd(Fs, W), rnd(Fs, W), rnd(W, Fs)) if Fs else (None, None, None)
+        S = top + (1 if Fs else 0)
+        start = torch.arange(M) % E if E == M else torch.randint(0, max(1, E - 1), (M,), generator=g) + 1
+        start[torch.randperm(M, generator=g)[:first]] = 0
+        idx = ((start[:, None] + torch.arange(top)) % E).int()
+        w = torch.rand(M, S, generator=g) + 0.25
+        ref = torch.zeros(M * S, W)
+        lref.moe_grouped(x, idx, w, gate, up, down, *sh, ref)
+        tiles = -(-M * S // 64) + E + 1  # as few as the operator takes
+        c = lambda t: None if t is None else t.to(gpu)  # noqa: E731
+        lists = (torch.full((tiles * 64,), 7, dtype=torch.int32, device=gpu), torch.zeros(tiles, dtype=torch.int32, device=gpu),
+                 torch.zeros(1, dtype=torch.int32, device=gpu))
+        args = (c(x), c(idx), c(w), c(gate), c(up), c(down), *(c(t) for t in sh), *lists)
+        outs = []
+        for aligned in (False, True):
+            o = torch.full((M * S, W), float("nan"), device=gpu)
+            ops.moe_grouped(*args, torch.zeros(M * S, max(F, Fs), dtype=torch.bfloat16, device=gpu), o, aligned=aligned)
+            outs.append(o.cpu())
+            n = int(lists[2])
+            assert int(lists[0][n * 64:(n + 1) * 64].abs().sum()) == 0
+        assert torch.equal(*outs)
+        err = (outs[0].double() - ref.double()).norm() / ref.double().norm()
+        assert float(err) <= 2.0 ** -8  # as above: one rounding of the hidden values, fp32 sums
+        assert float((outs[0] - ref).abs().max()) <= 2.0 ** -5 * float(ref.abs().max())
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
