@@ -132,6 +132,9 @@ size_t dsse_gemm_pipe_fix_floats(int bm, int S, int M, int N);
 size_t dsse_gemm_ring_fix_floats(int nw, int S, int M, int N);
 hipError_t dsse_paged_attention(int mode, int num_work, const dsse::AttnParams* p, hipStream_t st);
 hipError_t dsse_flash_prefill(int num_work, const dsse::AttnParams* p, hipStream_t st);
+hipError_t dsse_attn_combine(int num_work, const dsse::AttnParams* p, hipStream_t st);
+// decode rows d (mode 0) and prompt tiles f (mode 2) of one layer in one launch; hipErrorNotSupported: nothing done, not its sizes
+hipError_t dsse_mixed_attention(int rows, const dsse::AttnParams* d, int num_work, const dsse::AttnParams* f, hipStream_t st);
 hipError_t dsse_sample(int B, const dsse::SampleParams* p, hipStream_t st);
 hipError_t dsse_sample_pick(int B, int world, const void* cand, const dsse::SampleParams* p,
                             hipStream_t st);
@@ -167,6 +170,7 @@ hipError_t dsse_check_gemm_skinny(int* out, int clear);
 hipError_t dsse_check_gemm_stream(int* out, int clear);
 hipError_t dsse_check_attention(int* out, int clear);
 hipError_t dsse_check_attention_prefill(int* out, int clear);
+hipError_t dsse_check_attention_mixed(int* out, int clear);
 hipError_t dsse_check_elementwise(int* out, int clear);
 hipError_t dsse_check_sampler(int* out, int clear);
 hipError_t dsse_check_gemm_tiled(int* out, int clear);

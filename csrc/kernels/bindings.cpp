@@ -1100,6 +1100,34 @@ void paged_attention(int64_t mode, const Tensor& q, const Tensor& k_cache, const
   else DSSE_CHECK_HIP(dsse_paged_attention((int)mode, num_work, &p, cur_stream()));
 }
 
+// Attention of a mixed step: decode rows (paged_attention mode 0) and prompt tiles (mode 2) over the same q, pages and result; one launch
+// where the kernel takes the step (dsse_mixed_attention), else both.
+void mixed_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, Tensor& out, Tensor& part_o, Tensor& part_ml,
+                     at::TensorList rows, int64_t part, int64_t nparts, at::TensorList tiles, int64_t tile_part) {
+  check_gpu(q, "q");
+  check_dtype(q, at::kBFloat16, "q");
+  TORCH_CHECK(q.dim() == 3 && q.size(2) == 128 && out.sizes() == q.sizes(), "q and out must be [T, Hq, 128]");
+  TORCH_CHECK(rows.size() == 6 && tiles.size() == 6, "block_tables, q_start, q_len, ctx_len, work_seq, work_tile of decode rows and of prompt tiles");
+  const int hq = (int)q.size(1), hkv = (int)k_cache.size(1);
+  TORCH_CHECK(hq % hkv == 0 && (hq / hkv == 1 || hq / hkv == 2 || hq / hkv == 4), "flash prefill supports G in {1, 2, 4}");
+  auto params = [&](at::TensorList m, int64_t len, int64_t n, int qw, int kwv) {
+    dsse::AttnParams p = attn_params(hq, k_cache, v_cache, m[0], m[1], m[2], m[3], m[4], m[5], out, part_o, part_ml, len, n, qw, kwv);
+    p.q = reinterpret_cast<const bf16*>(q.data_ptr());
+    return p;
+  };
+  dsse::AttnParams d = params(rows, part, nparts, 1, 4), f = params(tiles, tile_part, 1, 4, 1);
+  const int nr = (int)rows[4].numel(), nt = (int)tiles[4].numel();
+  if (env_int("attn_mixed", 1) && !env_int("flash_hg", 0)) {
+    const hipError_t e = dsse_mixed_attention(nr, &d, nt, &f, cur_stream());
+    if (e == hipSuccess) return;
+    TORCH_CHECK(e == hipErrorNotSupported, "dsse kernel launch failed: ", hipGetErrorString(e));
+  }
+  attn_last_arriver(d, nr, q.device());
+  DSSE_CHECK_HIP(dsse_paged_attention(0, nr, &d, cur_stream()));
+  f.kwv = 0;
+  DSSE_CHECK_HIP(dsse_flash_prefill(nt, &f, cur_stream()));
+}
+
 // Flash prefill with the key split (round 6): `work` = [seq | tile | (kb0, kb1) pairs | slot] over nw items (int32,
 // 5 nw), `comb` = [(seq, tile, first slot, slots)] over the split tiles (int32, 4 nc).  Items with slot -1 write `out`;
 // the others leave partial O / (max, sum) in slots [0, nslots) of part_o / part_ml and flash_combine_kernel merges
@@ -1448,19 +1476,19 @@ bool kernels_checked() { return true; }
 bool kernels_checked() { return false; }
 #endif
 
-// Checked build: [7, 4] int32 (line, value, bound, count) of the first out-of-range index per kernel file,
+// Checked build: [8, 4] int32 (line, value, bound, count) of the first out-of-range index per kernel file,
 // in the order of kCheckFiles; all zeros in the default build.  Synchronises the device.
-const char* const kCheckFiles[7] = {"gemm_skinny.hip", "gemm_stream.hip", "attention.hip", "attention_prefill.hip",
-                                    "elementwise.hip", "sampler.hip", "gemm_tiled.hip"};
+const char* const kCheckFiles[8] = {"gemm_skinny.hip", "gemm_stream.hip", "attention.hip", "attention_prefill.hip",
+                                    "elementwise.hip", "sampler.hip", "gemm_tiled.hip", "attention_mixed.hip"};
 Tensor kernel_checks(bool clear) {
   using Reader = hipError_t (*)(int*, int);
-  static const Reader readers[7] = {dsse_check_gemm_skinny, dsse_check_gemm_stream, dsse_check_attention,
+  static const Reader readers[8] = {dsse_check_gemm_skinny, dsse_check_gemm_stream, dsse_check_attention,
                                     dsse_check_attention_prefill, dsse_check_elementwise, dsse_check_sampler,
-                                    dsse_check_gemm_tiled};
-  Tensor out = at::zeros({7, 4}, at::kInt);
+                                    dsse_check_gemm_tiled, dsse_check_attention_mixed};
+  Tensor out = at::zeros({8, 4}, at::kInt);
   if (!kernels_checked()) return out;
   DSSE_CHECK_HIP(hipDeviceSynchronize());
-  for (int i = 0; i < 7; ++i) DSSE_CHECK_HIP(readers[i](out.data_ptr<int>() + 4 * i, clear ? 1 : 0));
+  for (int i = 0; i < 8; ++i) DSSE_CHECK_HIP(readers[i](out.data_ptr<int>() + 4 * i, clear ? 1 : 0));
   return out;
 }
 // Stamps build: step-anatomy records (common.h stamps::record) of the ring GEMMs and RMSNorms.  step_stamps_arm
@@ -1537,6 +1565,8 @@ TORCH_LIBRARY(dsse, m) {
   m.def("decode_prep(Tensor active, Tensor positions, Tensor block_tables, Tensor(a!) slots, "
         "Tensor(b!) ctx_len, Tensor(c!) q_len, int num_blocks=2147483647, Tensor(d!)? walked=None) -> ()");
   m.def("ring_advance(Tensor(a!) counter) -> ()");
+  m.def("mixed_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) out, Tensor(b!) part_o, Tensor(c!) part_ml, Tensor[] rows, int part, "
+        "int nparts, Tensor[] tiles, int tile_part) -> ()");
   m.def("paged_attention(int mode, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor q_start, Tensor q_len, Tensor ctx_len, Tensor work_seq, Tensor work_tile, Tensor(a!) out, "
         "Tensor(b!) part_o, Tensor(c!) part_ml, int part, int nparts) -> ()");
@@ -1589,6 +1619,7 @@ TORCH_LIBRARY_IMPL(dsse, CUDA, m) {
   m.impl("silu_mul", &silu_mul);
   m.impl("decode_prep", &decode_prep);
   m.impl("ring_advance", &ring_advance);
+  m.impl("mixed_attention", &mixed_attention);
   m.impl("paged_attention", &paged_attention);
   m.impl("flash_prefill_split", &flash_prefill_split);
   m.impl("qkv_attention_decode", &qkv_attention_decode);

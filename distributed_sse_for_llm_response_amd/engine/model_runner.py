@@ -1007,11 +1007,10 @@ class ModelRunner(RunnerBase):
         for li, L in enumerate(w.layers):
             kc, vc = self.kv.k[li], self.kv.v[li]
             self._qkv_rows(x, L, qkv, pos, slots, q, kc, vc)
-            ops.paged_attention(0, q[r], kc, vc, self.block_tables[r], self.q_start[r], self.q_len[r],
-                                self.ctx_len[r], self.work_seq[r], self.work_tile[r], attn[r], self.part_o,
-                                self.part_ml, dpart, dnparts)
-            ops.paged_attention(2, q, kc, vc, d["bt"], d["qs"], d["ql"], d["ctx"], d["ws"], d["wt"], attn,
-                                self.part_o, self.part_ml, d["part"], 1)
+            ops.mixed_attention(q, kc, vc, attn, self.part_o, self.part_ml,
+                                (self.block_tables[r], self.q_start[r], self.q_len[r], self.ctx_len[r], self.work_seq[r],
+                                 self.work_tile[r]), dpart, dnparts, tuple(d[k] for k in ("bt", "qs", "ql", "ctx", "ws", "wt")),
+                                d["part"])
             self._resid_proj(attn.view(M, nh * 128), L.wo_t, resid, L.ffn_norm, x, tmp)
             self._gate_up(x, L, h)
             w_next = w.layers[li + 1].attn_norm if li + 1 < nl else w.final_norm

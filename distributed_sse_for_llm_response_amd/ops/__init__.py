@@ -231,6 +231,18 @@ def paged_attention(mode, q, k_cache, v_cache, block_tables, q_start, q_len, ctx
                             out, part_o, part_ml, part, nparts)
 
 
+def mixed_attention(q, k_cache, v_cache, out, part_o, part_ml, rows, part, nparts, tiles, tile_part):
+    """A mixed step's attention: paged_attention of decode rows (mode 0) and of 64-query prompt tiles (mode 2) over the same
+    q, pages and out, in one launch where the kernel takes both.  rows, tiles: (block_tables, q_start, q_len, ctx_len,
+    work_seq, work_tile) of either kind; part, nparts: the decode rows' key partitions; tile_part: mode 2's part."""
+    if _hip(q):
+        torch.ops.dsse.mixed_attention(q, k_cache, v_cache, out, part_o, part_ml, list(rows), part, nparts, list(tiles), tile_part)
+    else:
+        n = rows[4].numel()
+        paged_attention(0, q[:n], k_cache, v_cache, *rows, out[:n], part_o, part_ml, part, nparts)
+        paged_attention(2, q, k_cache, v_cache, *tiles, out, part_o, part_ml, tile_part, 1)
+
+
 def flash_prefill_split(q, k_cache, v_cache, block_tables, q_start, q_len, ctx_len, work, comb, out, part_o, part_ml,
                         nslots: int) -> None:
     """Flash prefill with long causal tiles split over key ranges (work = [seq | tile | (kb0, kb1) pairs | slot],
