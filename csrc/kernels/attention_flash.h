@@ -2,16 +2,13 @@
 // beside decode rows.  Layout and schedule are described in attention_prefill.hip.
 #pragma once
 #include "api.h"
+#include "lds_dma.h"
+
+#include <type_traits>
 
 namespace dsse {
 namespace flash {
 namespace {
-DEV void glds16(const void* src, char* lds_base) {
-  __builtin_amdgcn_global_load_lds(const_cast<void*>(src),
-                                   reinterpret_cast<__attribute__((address_space(3))) void*>(
-                                       reinterpret_cast<uintptr_t>(lds_base)),
-                                   16, 0, 0);
-}
 constexpr int kD = 128;
 constexpr int kBQ = 64;    // query tokens per workgroup
 constexpr int kBK = 64;    // keys per block (2 pages)
@@ -34,8 +31,8 @@ DEV int page_block(const int* bt, int pg, int npages, const AttnParams& p) {
 // workgroups: short prompts, where one workgroup per (tile, kv head) leaves most CUs idle -- a 512-token prompt is 64
 // workgroups; each then stages its K/V itself, which the L2 serves)
 // STAMP (diagnostic build, DSSE_FLASH_STAMPS): every wave of the first kStampWgs workgroups records the shader clock at
-// six points of each key block (before / after the barrier in front of QKᵀ, before / after the barrier in front of
-// softmax + PV, after the DMA issue, after the softmax) into 24 KiB of LDS past the ring, copied to `stamps` at the end; tools/flash_stamps.py reads them.
+// six points of each key block (before / after the barrier in front of the products, before / after the barrier in front of
+// the softmax, after the softmax, after the issue of the last Vᵀ reads) into 24 KiB of LDS past the ring, copied to `stamps` at the end; tools/flash_stamps.py reads them.
 constexpr int kStampBlocks = 128, kStampWgs = 32, kStampsPerBlock = 6;
 template <int G, int HG, bool STAMP>
 DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* smem) {  // smem: kRing blocks of kStage
@@ -64,7 +61,6 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
   const int jb = p.work_kb ? p.work_kb[2 * item] : 0;
   const int je = p.work_kb ? min(nblk, p.work_kb[2 * item + 1]) : nblk;
   const int pslot = p.work_slot ? p.work_slot[item] : -1;
-  const int w_last_pos = pos0 + min(qlen, q0 + 32) - 1;  // last visible key of this wave
   const int w_first_pos = pos0 + q0;
   const int head = h * G + hs * HG + wh;
   const int* bt = p.block_tables + (size_t)b * p.max_blocks;
@@ -86,59 +82,39 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
 #pragma unroll
     for (int s = 0; s < 4; ++s) asm volatile("" ::"v"(qf[qt][s]));
 
-  // LDS-DMA: a block is 32 x 1 KiB DMA instructions, IPW per wave.  Instruction q < 16 fills keys 4q..4q+3
-  // (lane -> key 4q + lane / 16, LDS slot lane % 16 = chunk ^ swz(key)); q >= 16 fills Vᵀ rows d = 8 (q - 16)
-  // + lane / 8 (slot lane % 8 = chunk ^ ((d >> 1) & 7), chunk = page * 4 + 8-token group).  The swizzles sit
-  // on the source address because the DMA writes LDS lane-linearly; the reads are unchanged.  Blocks past the
-  // last are issued too (pages clamp to the context, nobody reads them): a branch around the DMA made the
-  // compiler's waitcnt placement drain every load in flight.
-  constexpr int IPW = 32 / NW;
-  // Lane-constant parts of the DMA sources (element offsets inside a page block of this kv head) and, for the Vᵀ
-  // pieces, which of the block's two pages the lane's chunk comes from: per block only the two page bases change
-  // (scalar), so a piece costs a select and one 64-bit add instead of a per-lane 64-bit multiply-add.
-  uint32_t loff[IPW];
-  bool vhi[IPW];
+  // LDS-DMA: a block is 32 x 1 KiB DMA instructions, IPW per wave, each a contiguous KiB of one page of this kv head.  Instruction q < 16 fills
+  // keys 4q..4q+3 (lane -> key 4q + lane / 16, LDS slot lane % 16 = chunk ^ swz(key)); q >= 16 fills 16 rows d of one page's Vᵀ image (lane -> row
+  // lane / 4, slot lane % 4 = chunk ^ vswz(row)).  The swizzles sit on the source address because the DMA writes LDS lane-linearly.  Blocks past
+  // the last are issued too (pages clamp to the context, nobody reads them): a branch around the DMA made the compiler's waitcnt
+  // placement drain every load in flight.  A wave's instructions are all K or all Vᵀ, of one page (of both where a wave has 16).
+  constexpr int IPW = 32 / NW, NP = IPW > 8 ? 2 : 1;
+  static_assert(IPW % 4 == 0, "a lane's offset inside the KiB repeats every 4 instructions");
+  auto vswz = [](int row) { return (4 - (row >> 2)) & 3; };  // reads of lane (r, g): 16 distinct slots in every group of lanes that LDS serves together
+  const bool kpiece = w * IPW < 16;  // wave-uniform
+  uint32_t loff[4];
 #pragma unroll
-  for (int i = 0; i < IPW; ++i) {
-    const int q = w * IPW + i;  // wave-uniform
-    if (q < 16) {
-      const int key = 4 * q + (lane >> 4), c = (lane & 15) ^ swz(key & 15);
-      loff[i] = (key & 31) * kD + 8 * c;
-      vhi[i] = false;
-    } else {
-      const int d = 8 * (q - 16) + (lane >> 3), c = (lane & 7) ^ ((d >> 1) & 7);
-      loff[i] = d * kBS + 8 * (c & 3);
-      vhi[i] = c >= 4;
-    }
-  }
+  for (int i = 0; i < 4; ++i)
+    loff[i] = kpiece ? (lane >> 4) * 256 + (((lane & 15) ^ swz(4 * i + (lane >> 4))) << 4) : (lane >> 2) * 64 + (((lane & 3) ^ vswz(lane >> 2)) << 4);
   const size_t pstride = (size_t)p.hkv * kBS * kD;  // elements per page block (all kv heads)
-  const bf16* kh = p.k_cache + (size_t)h * kBS * kD;
-  const bf16* vh = p.v_cache + (size_t)h * kD * kBS;
-  // Page-table entries are read one block ahead: the scalar load of block j + 1's pages is in flight while block j
+  const bf16* head_pages = (kpiece ? p.k_cache : p.v_cache) + (size_t)h * kBS * kD;
+  // Page-table entries are read one block ahead: the scalar load of block j + 1's page is in flight while block j
   // is issued and retired by the next LDS wait, not by a dependent wait in front of this block's DMA.
-  int pg0 = page_block(bt, 2 * jb, npages, p), pg1 = page_block(bt, 2 * jb + 1, npages, p);
-  int jn = jb;  // next block to issue (blocks are issued in order)
-  // (the page bases are pinned in SGPR pairs: left to itself the compiler folds the per-lane select of two bases into
-  // a per-lane select of the page index followed by a per-lane 64-bit multiply)
-  auto sbase = [&](const bf16* head, int blk) {
-    uint64_t u = reinterpret_cast<uint64_t>(head + (size_t)blk * pstride);
-    asm volatile("" : "+s"(u));
-    return u;
-  };
-  auto issue_block = [&](int slot) {
-    const int blk0 = pg0, blk1 = pg1;
-    ++jn;
-    pg0 = page_block(bt, 2 * jn, npages, p);
-    pg1 = page_block(bt, 2 * jn + 1, npages, p);
-    char* base = smem + slot * kStage;
-    const bool kpiece = w * IPW < 16;  // wave-uniform: a wave's pieces are all K or all Vᵀ (IPW divides 16)
-    const uint64_t b0 = sbase(kpiece ? kh : vh, blk0), b1 = sbase(kpiece ? kh : vh, blk1);
+  const int par = (w * IPW & 15) >> 3;  // the block's page that the wave begins in
+  int pg[NP];
+  auto next_pages = [&](int j) {
 #pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-      const int q = w * IPW + i;  // wave-uniform
-      const uint64_t b = kpiece ? (q >= 8 ? b1 : b0) : (vhi[i] ? b1 : b0);
-      glds16(reinterpret_cast<const bf16*>(b + 2ull * loff[i]), base + q * 1024);
-    }
+    for (int n = 0; n < NP; ++n) pg[n] = page_block(bt, 2 * j + par + n, npages, p);
+  };
+  next_pages(jb);
+  int jn = jb;  // next block to issue (blocks are issued in order)
+  auto issue_block = [&](int slot) {
+    __amdgpu_buffer_rsrc_t page[NP];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) page[n] = make_rsrc(head_pages + (size_t)pg[n] * pstride, kBS * kD * 2);
+    next_pages(++jn);
+    char* base = smem + slot * kStage + w * IPW * 1024;
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) lds_dma(page[i / 8], base + i * 1024, loff[i & 3], ((w * IPW + i) & 7) * 1024);
   };
 
   f32x4 o[8][2];
@@ -153,13 +129,12 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
   f32x4 s4[4][2];  // Sᵀ[key tile kt][query tile qt] of the current block, live across the mid-block barrier
 
   // Lane-constant parts of the fragment addresses: K row 16 kt + r, chunk (4g + s) ^ swz(r) = kt * 4096 + kofs[s];
-  // Vᵀ row d = 16 dt + r, chunk (4t + g) ^ ((d >> 1) & 7) = (4t + g) ^ ((r >> 1) & 7) = dt * 2048 + vofs[t].  With the
+  // Vᵀ page t, row d = 16 dt + r, chunk g ^ vswz(r) = t * 8192 + dt * 1024 + vofs.  With the
   // slot a compile-time constant (the block loop is unrolled by the ring) every read is one base VGPR + an immediate.
-  int kofs[4], vofs[2];
+  int kofs[4];
 #pragma unroll
   for (int s2 = 0; s2 < 4; ++s2) kofs[s2] = r * 256 + (((4 * g + s2) ^ swz(r)) << 4);
-#pragma unroll
-  for (int t = 0; t < 2; ++t) vofs[t] = kKBytes + r * 128 + (((4 * t + g) ^ ((r >> 1) & 7)) << 4);
+  const int vofs = kKBytes + r * 64 + ((g ^ vswz(r)) << 4);
 
   unsigned* st_lds = reinterpret_cast<unsigned*>(smem + kRing * kStage) + w * kStampsPerBlock * kStampBlocks;
   auto stamp = [&](int j, int i) {
@@ -167,159 +142,171 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
       if (lane == 0 && j < kStampBlocks) st_lds[kStampsPerBlock * j + i] = (unsigned)__builtin_amdgcn_s_memtime();
     }
   };
-  // phase 1: Sᵀ = K·Qᵀ of the block in LDS slot `buf`; a key tile's 4 fragments are read one tile ahead
-  auto qk = [&](int buf) {
+  bf16x8 vf[2][8];  // Vᵀ fragments of a block's two pages, read while its softmax is computed: a wave by itself gets 16 bytes per lane out of
+                    // LDS every 46 clocks, the time of three MFMAs, so the reads of a block are spread over both its phases
+  bf16x8 pf[2][2];  // Pᵀ fragments [query tile][page] of the block whose products come next
+  bf16x8 kf[4][4];
+  auto read_k = [&](int buf, int kt) {
     const char* kb = smem + buf * kStage;
-    bf16x8 kf[2][4];
 #pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) kf[0][s2] = *reinterpret_cast<const bf16x8*>(kb + kofs[s2]);
-    __builtin_amdgcn_s_setprio(1);
+    for (int s2 = 0; s2 < 4; ++s2) kf[kt][s2] = *reinterpret_cast<const bf16x8*>(kb + kt * 4096 + kofs[s2]);
+  };
+  auto read_v = [&](int buf, int t) {
+    const char* vb0 = smem + buf * kStage;
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      if (kt < 3) {
+    for (int dt = 0; dt < 8; ++dt) vf[t][dt] = *reinterpret_cast<const bf16x8*>(vb0 + t * 8192 + dt * 1024 + vofs);
+  };
+  // Oᵀ[d tile][query tile] += Vᵀ · Pᵀ of one page
+  auto pv = [&](int t) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2)
-          kf[(kt + 1) & 1][s2] = *reinterpret_cast<const bf16x8*>(kb + (kt + 1) * 4096 + kofs[s2]);
-      }
+    for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt) o[dt][qt] = mfma16x16x32(vf[t][dt], pf[qt][t], o[dt][qt]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Sᵀ = K·Qᵀ of the block in LDS slot `buf`, whose first two tiles' fragments are read
+  auto qk = [&](int buf) {
+    read_k(buf, 2);
+    read_k(buf, 3);
+#pragma unroll
+    for (int k2 = 0; k2 < 4; k2 += 2) {  // two key tiles at a time: four chains of products
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) s4[kt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) s4[kt][qt] = mfma16x16x32(kf[kt & 1][s2], qf[qt][s2], s4[kt][qt]);
+        for (int kt = k2; kt < k2 + 2; ++kt)
+#pragma unroll
+          for (int qt = 0; qt < 2; ++qt)
+            s4[kt][qt] = mfma16x16x32(kf[kt][s2], qf[qt][s2], s2 ? s4[kt][qt] : f32x4{0.f, 0.f, 0.f, 0.f});
     }
-    __builtin_amdgcn_s_setprio(0);
   };
-  // phase 2: online softmax of block j and Oᵀ += Vᵀ·Pᵀ
-  auto sm_pv = [&](int j, int buf) {
+  // Online softmax of block j.  The running max (log2 units) only moves when a score exceeds it by more than kRescaleThr, so after the first blocks
+  // O and l are not rescaled at all (P <= 2^thr stays well inside bf16 / fp32 range; the final O / l is unchanged).  Decided per wave (any
+  // lane, each for the keys that it holds), and off the critical chain: the first half of the exponentials is made from the max as it was
+  // and made again where it moved.
+  auto softmax = [&](int j) {
     const int key0 = j * kBK;
-    const bool need_mask = key0 + kBK - 1 > w_first_pos;  // some key of the block is after some query
-    bf16x8 pf[2][2];  // [qt][page t]
+    if (key0 + kBK - 1 > w_first_pos) {  // some key of the block is after some query: masked scores become -1e30
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-      const int qpos = pos0 + q0 + 16 * qt + r;
-      const bool qvalid = q0 + 16 * qt + r < qlen;
-      // max over the RAW scores (scale_log2 > 0 commutes with max); masked scores become -1e30
-      float mx = -1e30f;
-      if (need_mask) {
+      for (int qt = 0; qt < 2; ++qt) {
+        const int qpos = q0 + 16 * qt + r < qlen ? pos0 + q0 + 16 * qt + r : -1;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = key0 + 16 * kt + 4 * g + i;
-            const float v = (qvalid && key <= qpos) ? s4[kt][qt][i] : -1e30f;
-            s4[kt][qt][i] = v;
-            mx = fmaxf(mx, v);
-          }
-      } else {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s4[kt][qt][i]);
+          for (int i = 0; i < 4; ++i) s4[kt][qt][i] = key0 + 16 * kt + 4 * g + i <= qpos ? s4[kt][qt][i] : -1e30f;
       }
-      mx = rows4_max(mx);
-      // Deferred rescale: the running max (log2 units) only moves when a query's block max exceeds it by
-      // more than kRescaleThr, so after the first blocks O and l are not rescaled at all (P <= 2^thr stays
-      // well inside bf16 / fp32 range; the final O / l is unchanged).  Decided per wave (any lane).
-      const float m_blk = mx * sc;
-      if (__any(m_blk > m_run[qt] + kRescaleThr)) {
-        const float m_new = fmaxf(m_run[qt], m_blk);
-        // a column with no visible key yet keeps m = -1e30 and must produce p = 0, not exp2(0)
+    }
+    // raw v_exp_f32 (no denormal range reduction: arguments are <= thr and underflow to 0 is wanted), the scale folded into one FMA; a
+    // query with no visible key yet keeps m = -1e30 and must produce p = 0, not exp2(0)
+    f32x4 e[2][2];
+    auto make = [&](f32x4& to, int kt, int qt) {
+      const float m_use = m_run[qt] < -1e29f ? 0.f : m_run[qt];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[kt][qt][i], sc, -m_use));
+    };
+    auto half = [&]() {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) make(e[kt][qt], kt, qt);
+    };
+    float mx[2];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {  // over the raw scores (scale_log2 > 0 commutes with max)
+      float a = s4[0][qt][0], b = s4[2][qt][0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) {
+        a = fmaxf(a, s4[i >> 2][qt][i & 3]);
+        b = fmaxf(b, s4[2 + (i >> 2)][qt][i & 3]);
+      }
+      mx[qt] = fmaxf(a, b);
+    }
+    half();
+    if (__any(mx[0] * sc > m_run[0] + kRescaleThr || mx[1] * sc > m_run[1] + kRescaleThr)) {
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt) {
+        const float m_new = fmaxf(m_run[qt], rows4_max(mx[qt]) * sc);
         const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - (m_new < -1e29f ? 0.f : m_new));
         l_part[qt] *= alpha;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-          o[dt][qt][0] *= alpha;
-          o[dt][qt][1] *= alpha;
-          o[dt][qt][2] *= alpha;
-          o[dt][qt][3] *= alpha;
-        }
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[dt][qt][i] *= alpha;
         m_run[qt] = m_new;
       }
-      const float m_use = m_run[qt] < -1e29f ? 0.f : m_run[qt];
-      // raw v_exp_f32 (no denormal range reduction: arguments are <= thr and underflow to 0 is wanted); the scale
-      // is folded into one packed FMA per score pair and the row sum is a packed add (VALU is this loop's bound:
-      // profiles/r4/pmc_flash_prefill_r4.md)
-      const f32x2 scv = {sc, sc}, mv = {-m_use, -m_use};
+      half();
+    }
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
+    for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          f32x2 v = {s4[kt][qt][i], s4[kt][qt][i + 1]};
-          v = __builtin_elementwise_fma(v, scv, mv);
-          v[0] = __builtin_amdgcn_exp2f(v[0]);
-          v[1] = __builtin_amdgcn_exp2f(v[1]);
-          s4[kt][qt][i] = v[0];
-          s4[kt][qt][i + 1] = v[1];
-          l_part[qt] += v;
-        }
-      // Pᵀ fragments: page t = key tiles 2t (keys 4g+i) and 2t+1 (keys 16+4g+i)
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int qt = 0; qt < 2; ++qt) {
+        if (kt < 2) s4[kt][qt] = e[kt][qt];
+        else make(s4[kt][qt], kt, qt);
+        // Pᵀ fragments: page t = key tiles 2t (keys 4g+i) and 2t+1 (keys 16+4g+i)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          pf[qt][t][i] = f2bf(s4[2 * t][qt][i]);
-          pf[qt][t][4 + i] = f2bf(s4[2 * t + 1][qt][i]);
+          l_part[qt][i & 1] += s4[kt][qt][i];
+          pf[qt][kt >> 1][4 * (kt & 1) + i] = f2bf(s4[kt][qt][i]);
         }
-    }
-    stamp(j, 5);
-    // Oᵀ[d tile][query tile] += Vᵀ · Pᵀ: the 8 fragments of a page read before its 16 MFMAs
-    const char* vb0 = smem + buf * kStage;
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      bf16x8 vf[8];
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) vf[dt] = *reinterpret_cast<const bf16x8*>(vb0 + dt * 2048 + vofs[t]);
-      // keep the 8 reads ahead of the MFMAs (the scheduler otherwise pairs 2 reads with a full lgkmcnt wait)
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) o[dt][qt] = mfma16x16x32(vf[dt], pf[qt][t], o[dt][qt]);
-    }
-    __builtin_amdgcn_s_setprio(0);
+      }
   };
 
-  // Barrier accounting (absolute barriers, counted from the loop entry of the leading half; the lagging half,
-  // wq = 1, passes one extra barrier first and one fewer at the end).  Leading half: QKᵀ(j) in interval 2j,
-  // softmax/PV(j) in 2j + 1; lagging half one interval later.  So block j is read in intervals 2j .. 2j + 2:
+  // Two phases per block, the products PV(j - 1), QKᵀ(j) and the softmax of block j, with a barrier before each.  Barrier accounting
+  // (absolute barriers, counted from the loop entry of the leading half; the lagging half, wq = 1, passes one extra barrier first and
+  // one fewer at the end).  Leading half: products of j in interval 2j, softmax in 2j + 1; lagging half one interval later.  So block j
+  // is read from interval 2j (its K, leading) to 2j + 3 (its Vᵀ, lagging):
   //   RAW  every wave's DMA of block j has retired (its own counted vmcnt) before barrier 2j;
-  //   WAR  block j + 4 reuses j's slot; its DMA is issued at the start of softmax/PV(j + 1), i.e. in interval
-  //        2j + 3 (leading) or 2j + 4 (lagging), after every read of block j (the last in interval 2j + 2).
-  // Each wave issues block j + 3 at the start of its softmax/PV(j) phase, so at the barrier before QKᵀ(j) the
-  // leading half has blocks up to j + 2 issued (wait: all but the 2 youngest blocks), and at the barrier before
-  // softmax/PV(j), which for the lagging half is absolute barrier 2(j + 1), the lagging half needs block j + 1
-  // with blocks up to j + 2 issued (wait: all but the youngest).
+  //   WAR  block j + 4 reuses j's slot; its DMA is issued among the products of j + 2, in interval 2j + 4 or 2j + 5.
+  // At barrier 2j either half has blocks up to j + 1 issued and waits for j: all but the youngest.
   const bool lag = wq == 1;
   issue_block(0);
   issue_block(1);
-  issue_block(2);
-  if (lag) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * IPW) : "memory");
-  // unrolled by the ring size: each block's LDS slot is a compile-time offset (no per-read address arithmetic)
-  for (int j0 = jb; j0 < je; j0 += kRing) {
-#pragma unroll
-    for (int k = 0; k < kRing; ++k) {
-      const int j = j0 + k;  // LDS slot k = (j - jb) % kRing: block jb went to slot 0
-      if (j < je) {
-        const bool vis = j * kBK <= w_last_pos;  // this wave sees at least one key of the block
-        stamp(j, 0);
-        if (!lag) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * IPW) : "memory");
-        else asm volatile("s_barrier" ::: "memory");
-        stamp(j, 1);
-        if (vis) qk(k);
-        stamp(j, 2);
-        if (!lag) asm volatile("s_barrier" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
-        stamp(j, 3);
-        issue_block((k + 3) % kRing);  // block j + 3
-        stamp(j, 4);
-        if (vis) sm_pv(j, k);
-      }
+  if (lag) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
+  auto step = [&](int j, auto slot, auto first) {  // slot: (j - jb) % kRing
+    constexpr int k = decltype(slot)::value;
+    stamp(j, 0);
+    if (!lag) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
+    else asm volatile("s_barrier" ::: "memory");
+    stamp(j, 1);
+    __builtin_amdgcn_s_setprio(1);
+    if constexpr (!decltype(first)::value) {
+      pv(0);
+      read_k(k, 0);
+      read_k(k, 1);
+      issue_block((k + 2) % kRing);  // block j + 2
+      pv(1);
+    } else {
+      read_k(k, 0);
+      read_k(k, 1);
+      issue_block((k + 2) % kRing);
     }
+    qk(k);
+    __builtin_amdgcn_s_setprio(0);
+    stamp(j, 2);
+    if (!lag) asm volatile("s_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
+    stamp(j, 3);
+    read_v(k, 0);
+    softmax(j);
+    stamp(j, 4);
+    __builtin_amdgcn_sched_barrier(0);
+    read_v(k, 1);
+    stamp(j, 5);
+  };
+  // unrolled by the ring size: each block's LDS slot is a compile-time offset (no per-read address arithmetic)
+  if (jb < je) step(jb, std::integral_constant<int, 0>{}, std::true_type{});
+  for (int j = jb + 1; j < je; j += kRing) {
+    step(j, std::integral_constant<int, 1>{}, std::false_type{});
+    if (j + 1 < je) step(j + 1, std::integral_constant<int, 2>{}, std::false_type{});
+    if (j + 2 < je) step(j + 2, std::integral_constant<int, 3>{}, std::false_type{});
+    if (j + 3 < je) step(j + 3, std::integral_constant<int, 0>{}, std::false_type{});
   }
   if (!lag) asm volatile("s_barrier" ::: "memory");
+  if (jb < je) {
+    pv(0);
+    pv(1);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA may still write this workgroup's LDS after it exits
   if constexpr (STAMP) {
     if (block < kStampWgs) {

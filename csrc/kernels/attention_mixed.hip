@@ -1,13 +1,13 @@
 // Attention of a mixed step in one launch: prompt tiles (attention_flash.h) and decode rows (attention_decode.h) of one layer.
 //
 // What bounds it: a step of 64 streams and 300 prompt rows has 40 prompt tiles, each a chain of key blocks on one of 256 CUs, and decode rows,
-// which are bound by their pages.  One after the other they took 20 and 30 us; here the tiles' workgroups are the first of the grid and the
+// which are bound by their pages.  One after the other they take 16 and 30 us; here the tiles' workgroups are the first of the grid and the
 // other CUs read pages meanwhile.  A workgroup has the tile kernel's 8 waves and LDS, so a CU holds one: its waves take 8 / KWV (row, kv head, key
 // partition) items of KWV waves each.
 //
-// Two launches / one, us, one MI355X, 32 heads over 8: 64 streams of 512 keys + 300 rows 50.9 / 40.2, + 64 rows 43.1 / 34.5, 32 + 300 40.2 / 32.2, 16
-// of 500 + 200 30.3 / 19.9, 4 of 300 + 100 19.7 / 14.9, 2 of 64 + 32 13.4 / 9.1, 128 of 500 + 300 78.1 / 63.0, 128 of 128 + 384 41.3 / 28.0, 192 of
-// 300 + 256 68.0 / 55.9, 16 of 4000 + 256 77.5 / 65.8, 64 of 512 + 256 rows behind 3000 148 / 117; one kv head, 64 + 256 29.5 / 24.4.
+// Two launches / one, us, one MI355X, 32 heads over 8: 64 streams of 512 keys + 300 rows 47.5 / 37.8, + 64 rows 42.1 / 33.3, 32 + 300 37.0 / 31.3, 16
+// of 500 + 200 27.9 / 19.2, 4 of 300 + 100 18.2 / 13.5, 2 of 64 + 32 12.4 / 8.1, 128 of 500 + 300 74.5 / 61.1, 128 of 128 + 384 37.2 / 27.7, 192 of
+// 300 + 256 65.3 / 56.4, 16 of 4000 + 256 75.1 / 63.8, 64 of 512 + 256 rows behind 3000 112 / 80; one kv head, 64 + 256 26.5 / 21.2.
 #include "attention_decode.h"
 #include "attention_flash.h"
 
@@ -53,9 +53,9 @@ extern "C" hipError_t dsse_mixed_attention(int rows, const dsse::AttnParams* d, 
   using namespace dsse;
   if (d->group != 4 || f->group != 4 || rows <= 0 || num_work <= 0) return hipErrorNotSupported;
   const int tiles = num_work * f->hkv, items = rows * d->hkv * d->nparts;
-  // Waves per item, 2 / 4 / 8, us: 1024 items of 500 keys 63.0 / 65.2 / 65.7, 800 of 300 31.0 / 34.0 / 37.0; 512 of 512 43.7 / 40.2 / 41.7, of 1000
-  // (16 rows of 4000 in four partitions) 83.8 / 65.8 / 68.3, of 375 37.7 / 38.4 / 36.9, of 256 29.5 / 32.2 / 30.0; 384 of 170 22.3 / 21.2 / 19.9, 128 of
-  // 75 16.7 / 16.5 / 14.9.  (Two pages in flight per wave are 0 to 5 us behind one; one wave per item 73 us at 512 keys.)
+  // Waves per item, 2 / 4 / 8, us: 1024 items of 500 keys 61.1 / 62.4 / 66.4, 800 of 300 31.1 / 33.7 / 37.2; 512 of 512 43.6 / 37.8 / 41.2, of 1000
+  // (16 rows of 4000 in four partitions) 85.0 / 63.8 / 67.1, of 375 37.9 / 35.5 / 36.4, of 256 29.2 / 31.3 / 29.4; 384 of 170 22.2 / 19.0 / 19.2, 128 of
+  // 75 15.3 / 15.1 / 13.5.  (Two pages in flight per wave are 0 to 5 us behind one; one wave per item 73 us at 512 keys.)
   const int kwv = d->kwv ? d->kwv : items > 640 ? 2 : items > 384 ? 4 : 8;
   const hipError_t e = kwv <= 2 ? launch<2>(tiles, rows, *d, *f, st) : kwv == 4 ? launch<4>(tiles, rows, *d, *f, st) : launch<8>(tiles, rows, *d, *f, st);
   return e == hipSuccess && d->nparts > 1 ? dsse_attn_combine(rows, d, st) : e;

@@ -13,16 +13,20 @@
 //                in one lane column, and the exponentiated scores are already the B operand of
 //                Oᵀ = Vᵀ·Pᵀ — the V cache stores each page transposed with the token permutation
 //                vperm(), so lane group g's 8 keys {4g..4g+3, 16+4g..16+4g+3} are one 16-byte run;
-//   LDS images = K [64 keys][256 B] with the XOR-swizzled 16-byte chunks of gemm_xlds, Vᵀ [128 d]
-//                [128 B] with chunk ^= (d >> 1) & 7: both read with conflict-free ds_read_b128;
+//   LDS images = K [64 keys][256 B] with the XOR-swizzled 16-byte chunks of gemm_xlds, a page's Vᵀ [128 d][64 B] with
+//                chunk ^= (-(d >> 2)) & 3: both read with conflict-free ds_read_b128, both filled by instructions that read
+//                one contiguous KiB of a page;
 //   softmax    = online, base 2, masked scores contribute exactly 0 (fully masked columns stay 0).
 //
-// Schedule (round 4): two phases per key block, QKᵀ(j) | softmax(j) + PV(j), one barrier before each, and the
-// two query halves staggered by one barrier.  Waves w and w + 4 share a SIMD (G = 4: the same head, the two
-// query halves), so while one runs the 32 MFMAs of its QKᵀ the other runs its softmax VALU work and then its PV
-// MFMAs: the SIMD sees MFMA work from one wave under the other's exp / max / convert chain.  The round-1..3 form
-// (all waves in lockstep, one barrier per two blocks) measured MFMA busy 22 %, 34 % of wave time waiting on
-// dependencies (profiles/pmc_flash_prefill_r1.md): both waves of a SIMD reached their softmax at the same time.
+// Schedule: two phases per key block with a barrier before each, the products PV(j - 1) and QKᵀ(j) | softmax(j), and the two
+// query halves staggered by one barrier.  Waves w and w + 4 share a SIMD (G = 4: the same head, the two query halves), so one
+// runs its 64 MFMAs (1075 clocks) while the other runs its softmax (32 exponentials per lane and what goes with them: some 1100
+// clocks beside MFMAs).  Vᵀ fragments are read in the softmax phase, K fragments under the PV products; the running max is off the
+// critical chain (the softmax's comment).  One MI355X, 32 heads over 8, us: 8192 tokens 594 (925 TFLOP/s) with QKᵀ | softmax + PV as the
+// phases, a block's maximum before its exponentials and Vᵀ read right before its products, 467 (1175) now; 6000 377 / 293, 4096 184 / 145, 2048
+// 82 / 62, 1024 44 / 34, 512 27 / 21, 300 18.6 / 15.1, four of 2048 193 / 156; 16 heads over 8, 8192 tokens 681 / 365.  Left out in a copy, the
+// LDS reads are 85 us of the 465, the DMA 6, the softmax 46; reads of a block further ahead, DMA in other places and other wave
+// priorities 0 to 4 % slower.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>

@@ -3,8 +3,9 @@
     DSSE_FLASH_STAMPS=/tmp/fs.bin python tools/bench_prefill_attn.py --T 8192 && python tools/flash_stamps.py /tmp/fs.bin
 
 The file holds [32 workgroups][8 waves][128 blocks][6] u32 shader-clock values per key block: a = before the barrier
-in front of QKᵀ, b = after it, c = after QKᵀ, d = after the barrier in front of softmax + PV, e = after the DMA issue
-of block j + 3, f = after the softmax (the next block's a closes PV).  Prints, per query half (leading waves 0-3, lagging waves 4-7), the median cycles per block of
+in front of the products PV(j - 1) and QKᵀ(j), b = after it, c = after the products, d = after the barrier in front of the
+softmax, e = after the softmax, f = after the issue of the last Vᵀ reads.  A stamp waits for the LDS reads in flight, so the
+stamped kernel is slower than the other.  Prints, per query half (leading waves 0-3, lagging waves 4-7), the median cycles per block of
 each segment over the steady blocks (the first 4 and the last 2 of each wave are skipped).
 """
 import argparse
@@ -30,7 +31,7 @@ def main():
             seg = np.stack([b - a, c - b, d - c, e - d, f - e, a_next - f, a_next - a], axis=1)[4:n - 2]
             seg = seg % (1 << 32)  # 32-bit clock wrap
             rows["leading (w 0-3)" if w < 4 else "lagging (w 4-7)"].append(seg)
-    print("| half | barrier before QK | QK | barrier before SM+PV | DMA issue | softmax | PV | block |")
+    print("| half | barrier before products | products | barrier before softmax | softmax | V reads | loop | block |")
     print("|---|---|---|---|---|---|---|---|")
     for k, v in rows.items():
         if not v:
