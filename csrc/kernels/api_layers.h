@@ -26,6 +26,11 @@ struct GemmRmParams {
 };
 // gemm_rm_strip.hip: rows 48 or 80; fp32 operands of whole 128-byte chunks (gemm_rowmajor.hip lds_ok)
 hipError_t gemm_rm_strip(int rows, const GemmRmParams& p, hipStream_t st);
+// gemm_rm_split.hip: the same operands, and what the form takes in us at K = 2048
+hipError_t gemm_rm_split(const GemmRmParams& p, hipStream_t st);
+int64_t gemm_rm_split_us(int M, int N, int batch);
+int gemm_rm_split_form(int M, int N, int batch);  // 10 TM + TN of its tiles
+bool gemm_rm_split_pays(int M, int N, int K, int batch);  // gemm_rowmajor.hip
 // gemm_rowmajor.hip: rows of the fp32 form for many tiles: 64 (64 x 64 tiles), 48 or 80 (strips)
 int gemm_rm_form_rows(int M, int N, int batch);
 

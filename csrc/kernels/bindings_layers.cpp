@@ -682,6 +682,10 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         "Tensor(d!)? scratch=None, bool alone=False, int longest=0) -> ()");
   m.def("moe_router(Tensor x, Tensor w, Tensor? b, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
   m.def("moe_topk(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w) -> ()");
+  m.def("gemm_rm_split_form(int M, int N, int K, int batch=1) -> int",  // 0: another form
+        [](int64_t M, int64_t N, int64_t K, int64_t batch) {
+          return (int64_t)(dsse::gemm_rm_split_pays((int)M, (int)N, (int)K, (int)batch) ? dsse::gemm_rm_split_form((int)M, (int)N, (int)batch) : 0);
+        });
   m.def("gemm_rm_form_rows(int M, int N, int batch=1) -> int",
         [](int64_t M, int64_t N, int64_t batch) { return (int64_t)dsse::gemm_rm_form_rows((int)M, (int)N, (int)batch); });
   m.def("moe_plan(int M, int W, int F, int Fs, int E, int top, bool gated) -> int", &moe_plan);

@@ -322,6 +322,9 @@ hipError_t dispatch(const GemmRmParams& p, hipStream_t st) {
     return hipGetLastError();
   }
   if (lds_ok<T>(p)) {
+    if constexpr (sizeof(T) == 4) {
+      if (gemm_rm_split_pays(p.M, p.N, p.K, p.batch)) return gemm_rm_split(p, st);
+    }
     // 64 x 64 tiles (fp32: or strips, gemm_rm_form_rows) while they fill the CUs; two wave groups per tile when there is one tile per CU at most (nothing else
     // would run while a wave waits for its fragments: 400 rows of 2048 x 2048 in fp32 45.4 -> 42.2 us); 32 x 32 tiles, four
     // groups each, while those make one round (64 rows of 2048 x 8192 in fp32 157 -> 50 us, 400 rows of 576 x 4096 in bf16
@@ -354,13 +357,13 @@ hipError_t dispatch(const GemmRmParams& p, hipStream_t st) {
 // rows 89 / 108 / 91, 240 rows 110 / 130 / 140; 16384, 130 rows 99 / 135 / 92, 330 rows 194 / 209 / 228, 400 rows 247 / 247 / 228; one round of
 // K = 224 (longer ones of 64 x 64 tiles are split over wave groups): 330 x 2048 7.6 / 9.0 / 10.6, 400 x 2048 10.4 / 9.1 / 10.7.  Strips of 96
 // rows were the faster form nowhere by more than 3 %.
-int gemm_rm_form_rows(int M, int N, int batch) {
+namespace {
+int rows_us(int M, int N, int batch, int64_t& least) {
   struct Form {
     int rows, round, alone, paired, only;  // a round; up to 160, up to 256 workgroups behind full rounds; up to 256 and no others
   };
   static constexpr Form kForms[3] = {{64, 69, 39, 62, 53}, {48, 54, 34, 40, 52}, {80, 90, 50, 50, 55}};
   int best = 0;
-  int64_t least = 0;
   for (const Form& f : kForms) {
     const int64_t tiles = (int64_t)((M + f.rows - 1) / f.rows) * ((N + 63) / 64) * batch, full = tiles / 512, left = tiles % 512;
     int64_t t = full * f.round;
@@ -369,6 +372,28 @@ int gemm_rm_form_rows(int M, int N, int batch) {
     if (!best || t < least) best = f.rows, least = t;
   }
   return best;
+}
+}  // namespace
+
+// Whether the tiles of gemm_rm_split.hip are through before the forms below.  From K = 512 on by what both take, in us at K = 2048 (`rows_us`; tiles of
+// 32 x 32 one round 16.5 and two 32, 64 x 64 tiles with two wave groups 41), with 3 % for the figures' own error: over 552 products of
+// 20 to 1500 rows, 128 to 16384 columns, K 128 to 8192, others / chosen 1.10 in the mean (1.64 at the most: 257 to 512 tiles of 32 x 32), 0.93 at the least.  With
+// 4 to 15 chunks by tiles of 32 x 32: K = 128 up to 512 of them 1.12 to 1.27, up to 1024 0.90 to 1.04; K = 256 up to 1024 0.96 to 1.54, more 0.78 to 1.03.
+bool gemm_rm_split_pays(int M, int N, int K, int batch) {
+  const int chunks = K / 32;
+  auto tiles = [&](int t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
+  const int64_t small = tiles(32);
+  if (chunks < 16) return chunks >= 4 && small <= (chunks < 8 ? 512 : 1024);
+  int64_t us;
+  if (small <= 512) us = small <= 256 ? 16 : 32;
+  else if (tiles(64) <= 256) us = 41;
+  else rows_us(M, N, batch, us);
+  return 100 * gemm_rm_split_us(M, N, batch) < 97 * us;
+}
+
+int gemm_rm_form_rows(int M, int N, int batch) {
+  int64_t us = 0;
+  return rows_us(M, N, batch, us);
 }
 
 }  // namespace dsse
