@@ -33,8 +33,15 @@
 //     address arithmetic); rows past M read as zeros (out-of-range offsets, no memory traffic); the last two steps
 //     issue nothing past the end and count their waits exactly;
 //   * XCD-aware tile order (bijective remap, groups of 8 row blocks swept by column) as gemm_tiled.hip;
-//   * epilogues: bf16 store staged through LDS (16-byte row stores), SiLU·mul, fp32 / residual / QKV+RoPE /
-//     split-K partial slabs through gemm_epilogue.h.
+//   * epilogues: bf16 results and SiLU / GELU·mul through a wave's own 4 KiB of LDS (16-byte row stores), fp32 / residual / QKV+RoPE /
+//     split-K partial slabs through gemm_epilogue.h;
+//   * from two rounds of tiles on a workgroup stays on its CU and takes every 256th tile: the requests past a tile's last step are the next
+//     one's first, and its results leave while they are under way.  A round a launch at a time / this, one MI355X, us: 8192 x 28672 x 4096 SiLU
+//     1425 / 1373, 8192 x 28672 x 2048 784 / 764, x 1024 480 / 445; 8192 x 4096 x 4096 196.5 / 193.5, x 2048 108 / 105, x 1024 64.5 / 60.0;
+//     1500 x 16384 x 2048 GELU 93 / 89.
+#include <algorithm>
+#include <type_traits>
+
 #include "gemm_epilogue.h"
 #include "lds_dma.h"
 
@@ -58,7 +65,23 @@ DEV unsigned long long now() { return DSSE_PIPE_STAMPS ? __builtin_amdgcn_s_memr
 constexpr int kA = 256 * 128;     // A image of one K step: 256 rows x 64 bf16, swizzled 16-byte pieces
 constexpr int kB = 16 * 2048;     // B image: 16 column tiles x two 1 KiB k-step blocks
 constexpr int kBuf = kA + kB;     // 64 KiB per K step
-constexpr size_t kLDS = 2 * (size_t)kBuf;
+constexpr int kStage = 4096;      // a wave's rows of the result on their way to 16-byte stores, beside the two images
+constexpr size_t kLDS = 2 * (size_t)kBuf + 8 * kStage;
+constexpr int kCUs = 256;
+
+// bf16 results: products with the weights as their first operand, so that a lane has four columns of a row, and rows that leave through LDS as 16-byte
+// stores, this many per tile and wave, those of rows and columns that are not there included (past their descriptor's range).  0: fp32 results and
+// scattered ones, a row's 16 columns in 16 lanes.  (fp32 slabs as 16-byte stores, straight or through LDS: 1024 x 2048 x 2048 17.3 / 20.0 / 17.9 us, 2048 x
+// 4096 x 4096 61.5 / 63.7 / 59.7.)
+template <int MODE, int QI>
+constexpr int stores() {
+  return MODE == kStoreBf16 ? 4 * QI : MODE == kSiluMul ? 2 * QI : 0;
+}
+
+// Whether 16 bytes of a bf16 result row are one aligned store
+__host__ __device__ inline bool wide_results(const GemmEpi& ep) {
+  return reinterpret_cast<uintptr_t>(ep.out) % 16 == 0 && ep.ldo % 8 == 0;
+}
 
 }  // namespace gp
 
@@ -90,60 +113,66 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
   constexpr int QR = BM / 4, QI = QR / 16;  // X rows per quadrant, MFMA row tiles per quadrant
   static_assert(BM == 256 || BM == 192 || BM == 128, "row tile");
   const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256, ntile = nbm * nbn;
-  const int nwg = gridDim.x;
-  const int bid = blockIdx.x, xcd = bid % 8, q8 = nwg / 8, rem = nwg % 8;
-  const int lid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + bid / 8;
   // split slices: FIX keeps a tile's S slices adjacent in the remapped order, so they run on one XCD and the last
   // arriver reads the other slices' plain-stored slots from its own L2; the slab form (consumer-reduced) keeps
   // them ntile apart
-  const int S_ = nwg / ntile;
-  const int ks = FIX ? lid % S_ : lid / ntile, tl = FIX ? lid / S_ : lid % ntile;
-  constexpr int GM = 8;
-  const int grp = tl / (GM * nbn), first = grp * GM, gsz = min(GM, nbm - first);
-  const int bm = first + (tl % (GM * nbn)) % gsz, bn = (tl % (GM * nbn)) / gsz;
-  const int m0 = bm * BM, n0 = bn * 256;
-  const int k0 = ks * Kr, nk = Kr >> 6;
-  const int KC = K >> 7;
+  const int S_ = K / Kr, nwg = ntile * S_, nk = Kr >> 6, KC = K >> 7;
+  struct Tile {
+    int m0, n0, ks, tl;
+  };
+  auto decode = [&](int bid) {
+    constexpr int GM = 8;
+    const int xcd = bid % 8, q8 = nwg / 8, rem = nwg % 8;
+    const int lid = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + bid / 8;
+    const int ks = FIX ? lid % S_ : lid / ntile, tl = FIX ? lid / S_ : lid % ntile;
+    const int grp = tl / (GM * nbn), first = grp * GM, gsz = min(GM, nbm - first);
+    return Tile{(first + (tl % (GM * nbn)) % gsz) * BM, (tl % (GM * nbn)) / gsz * 256, ks, tl};
+  };
+  int bid = blockIdx.x;
+  Tile at = decode(bid);
 
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, (uint32_t)(((size_t)(M - 1) * ldx + K) * 2));
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(W, (uint32_t)((size_t)N * K * 2));
 
-  // ---- per-lane DMA offsets (bytes), fixed for the whole K loop: [half q][instruction i] of this wave
+  // ---- per-lane DMA offsets (bytes), fixed for a tile's K loop: [half q][instruction i] of this wave
   uint32_t a_vo[2][2], b_vo[2][2];
   int a_lo[2][2], b_lo[2][2];  // LDS byte offsets inside a buffer
 #pragma unroll
   for (int q = 0; q < 2; ++q)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int j = 2 * w + i;                                     // instruction j of the 16 of this half
-      const int rb = (j >> 3) * 128 + q * 64 + (j & 7) * 8;        // first of its 8 rows
-      const int row = rb + (lane >> 3), sr = (j & 7) * 8 + (lane >> 3);  // LDS slot row, slot row in the quadrant
-      const int xrow = m0 + (j >> 3) * (BM / 2) + q * QR + sr;          // the X row it holds
-      const int pc = (lane & 7) ^ piece_swizzle(row);
-      a_lo[q][i] = rb * 128;
-      a_vo[q][i] = sr < QR && xrow < M ? (uint32_t)(((size_t)xrow * ldx + 32 * (pc >> 1) + 8 * (pc & 1)) * 2) : kOOB;
-      const int tb = (j >> 2) * 4 + q * 2 + ((j >> 1) & 1), sub = j & 1;  // column tile of the block, k sub-step
-      b_lo[q][i] = kA + tb * 2048 + sub * 1024;
-      b_vo[q][i] = n0 + 16 * tb < N ? (uint32_t)((((size_t)(n0 / 16 + tb) * KC) * kTileChunk + sub * 512 + lane * 8) * 2) : kOOB;
+      const int j = 2 * w + i;  // instruction j of the 16 of this half
+      a_lo[q][i] = ((j >> 3) * 128 + q * 64 + (j & 7) * 8) * 128;
+      b_lo[q][i] = kA + ((j >> 2) * 4 + q * 2 + ((j >> 1) & 1)) * 2048 + (j & 1) * 1024;
     }
-  // K step t: X columns 128c + 16h + (piece offsets), W chunk c, k sub-steps 2h, 2h+1
-  auto a_so = [&](int t) {
-    const int kk = k0 + 64 * t;
-    return (uint32_t)(((kk >> 7) * 128 + 16 * ((kk >> 6) & 1)) * 2);
+  auto offsets = [&](const Tile& to) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int j = 2 * w + i;
+        const int row = (j >> 3) * 128 + q * 64 + (j & 7) * 8 + (lane >> 3), sr = (j & 7) * 8 + (lane >> 3);  // LDS slot row, slot row in the quadrant
+        const int xrow = to.m0 + (j >> 3) * (BM / 2) + q * QR + sr;                                       // the X row it holds
+        const int pc = (lane & 7) ^ piece_swizzle(row);
+        a_vo[q][i] = sr < QR && xrow < M ? (uint32_t)(((size_t)xrow * ldx + 32 * (pc >> 1) + 8 * (pc & 1)) * 2) : kOOB;
+        const int tb = (j >> 2) * 4 + q * 2 + ((j >> 1) & 1), sub = j & 1;  // column tile of the block, k sub-step
+        b_vo[q][i] = to.n0 + 16 * tb < N ? (uint32_t)((((size_t)(to.n0 / 16 + tb) * KC) * kTileChunk + sub * 512 + lane * 8) * 2) : kOOB;
+      }
   };
-  auto b_so = [&](int t) {
-    const int kk = k0 + 64 * t;
-    return (uint32_t)(((kk >> 7) * kTileChunk + ((kk >> 6) & 1) * 1024) * 2);
-  };
+  offsets(at);
+  // K steps count on from tile to tile; step t lies at column kk: X columns 128c + 16h + (piece offsets), W chunk c, k sub-steps 2h, 2h+1
+  int k_at = at.ks * Kr;  // column of step 0, had the tile begun there
   auto issue_a = [&](int q, int t) {
     char* base = smem + (t & 1) * kBuf;
-    const uint32_t so = __builtin_amdgcn_readfirstlane(a_so(t));
+    const int kk = k_at + 64 * t;
+    const uint32_t so = __builtin_amdgcn_readfirstlane((uint32_t)(((kk >> 7) * 128 + 16 * ((kk >> 6) & 1)) * 2));
 #pragma unroll
     for (int i = 0; i < 2; ++i) lds_dma(xr, base + a_lo[q][i], a_vo[q][i], so);
   };
   auto issue_b = [&](int q, int t) {
     char* base = smem + (t & 1) * kBuf;
-    const uint32_t so = __builtin_amdgcn_readfirstlane(b_so(t));
+    const int kk = k_at + 64 * t;
+    const uint32_t so = __builtin_amdgcn_readfirstlane((uint32_t)(((kk >> 7) * kTileChunk + ((kk >> 6) & 1) * 1024) * 2));
 #pragma unroll
     for (int i = 0; i < 2; ++i) lds_dma(wr, base + b_lo[q][i], b_vo[q][i], so);
   };
@@ -156,11 +185,8 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     const int row = wm * 128 + r;
     a_rd[sp] = row * 128 + (((2 * g + sp) ^ piece_swizzle(row)) << 4);
   }
+  constexpr bool kTurned = stores<MODE, QI>() > 0;
   f32x4 acc[8][4];
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
   bf16x8 a[4][2], b[4][2];
   auto read_a = [&](const char* buf, int qm) {
 #pragma unroll
@@ -186,33 +212,44 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       for (int i = 0; i < QI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[4 * qm + i][2 * qn + j] = mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j]);
+          acc[4 * qm + i][2 * qn + j] = kTurned ? mfma16x16x32(b[2 * qn + j][sp], a[i][sp], acc[4 * qm + i][2 * qn + j])
+                                                : mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j]);
     __builtin_amdgcn_s_setprio(0);
     asm volatile("s_barrier" ::: "memory");
   };
 
-  {
-    // prologue: step 0 whole, then A0 / B0 of step 1 (its B1 / A1 go out in phases 0 / 1 of step 0)
-    issue_a(0, 0);
-    issue_b(0, 0);
-    issue_b(1, 0);
-    issue_a(1, 0);
-    issue_a(0, 1);
-    issue_b(0, 1);
-    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // A0 / B0 of step 0 landed everywhere
-    if (wm == 1) asm volatile("s_barrier" ::: "memory");  // wave row 1 runs one barrier behind row 0
+  // prologue: step 0 whole, then A0 / B0 of step 1 (its B1 / A1 go out in phases 0 / 1 of step 0)
+  issue_a(0, 0);
+  issue_b(0, 0);
+  issue_b(1, 0);
+  issue_a(1, 0);
+  issue_a(0, 1);
+  issue_b(0, 1);
+  asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // A0 / B0 of step 0 landed everywhere
+  if (wm == 1) asm volatile("s_barrier" ::: "memory");  // wave row 1 runs one barrier behind row 0
+  // A workgroup goes on to its next tile without a pause: the requests past a tile's last step are those of the next one's first, and its
+  // results leave while they are under way.
+  int t0 = 0;  // the tile's first step
+  for (;; t0 += nk) {
+    const bool more = !FIX && stores<MODE, QI>() > 0 && bid + (int)gridDim.x < nwg;  // uniform
+    const Tile next = decode(more ? bid + (int)gridDim.x : bid);
+#pragma unroll
+    for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // TAIL 0 = steady, 1 = step t+1 exists but t+2 does not, 2 = last step.  RAW: B1(t) waited in phase 0 and read
     // in phase 1, A1(t) waited in 1 and read in 2, A0 / B0(t+1) waited in 3 and read in phase 0 of t+1 (the
     // barrier that opens the reading phase follows every wave's wait).  WAR: B1 of buffer (t+1)&1 was last read in
     // phase 1 of t-1, A1 in phase 2 of t-1, A0 / B0 of buffer t&1 in phase 0 of t -- each restaged >= 2 phases later.
-    auto step_even = [&](int t, auto tail_tag) {
-      constexpr int TAIL = decltype(tail_tag)::value;
+    // OUT: stores of the tile before, which the wave has issued between the requests that are waited for here and the younger ones.
+    auto step_even = [&](int t, auto tail_tag, auto out_tag) {
+      constexpr int TAIL = decltype(tail_tag)::value, OUT = decltype(out_tag)::value;
       const char* buf = smem + (t & 1) * kBuf;
       read_a(buf, 0);
       read_b(buf, 0);
       if constexpr (TAIL < 2) {
         issue_b(1, t + 1);
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // B-half 1 of step t
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + OUT) : "memory");  // B-half 1 of step t
       } else {
         asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
       }
@@ -220,29 +257,39 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       read_b(buf, 1);
       if constexpr (TAIL < 2) {
         issue_a(1, t + 1);
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // A-half 1 of step t
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + OUT) : "memory");  // A-half 1 of step t
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       }
       mma(0, 1);
       read_a(buf, 1);
+      if (TAIL == 0 && OUT == 0 && t == t0 + nk - 2) {  // step t + 2 is the next tile's first
+        offsets(next);
+        k_at = next.ks * Kr - 64 * (t + 2);
+      }
       if constexpr (TAIL == 0) issue_a(0, t + 2);
       mma(1, 1);
       if constexpr (TAIL == 0) {
         issue_b(0, t + 2);
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // A0 / B0 of step t+1
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + OUT) : "memory");  // A0 / B0 of step t+1
       } else if constexpr (TAIL == 1) {
         asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
       }
       mma(1, 0);
     };
-    int t = 0;
-    for (; t < nk - 2; ++t) step_even(t, std::integral_constant<int, 0>{});
-    step_even(t++, std::integral_constant<int, 1>{});  // nk >= 2 (host contract)
-    step_even(t, std::integral_constant<int, 2>{});
-  }
-  // balance the barrier count of the two rows
-  if (wm == 0) asm volatile("s_barrier" ::: "memory");
+    typedef std::integral_constant<int, 0> None;
+    int t = t0;
+    if constexpr (stores<MODE, QI>() > 0 && !FIX) {
+      if (t0 > 0) step_even(t++, None{}, std::integral_constant<int, stores<MODE, QI>()>{});  // nk >= 4 (host contract)
+    }
+    const int end = t0 + (more ? nk : nk - 2);
+    for (; t < end; ++t) step_even(t, None{}, None{});
+    if (!more) {
+      step_even(t++, std::integral_constant<int, 1>{}, None{});  // nk >= 2 (host contract)
+      step_even(t, std::integral_constant<int, 2>{}, None{});
+      // balance the barrier count of the two rows
+      if (wm == 0) asm volatile("s_barrier" ::: "memory");
+    }
 
   if constexpr (FIX) {
     const int S = S_;
@@ -253,7 +300,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       __syncthreads();  // every wave past its last LDS read: word 0 of the LDS carries the ticket
       stamp(ep, 1, now());
       int* sflag = reinterpret_cast<int*>(smem);
-      if (threadIdx.x == 0) sflag[0] = __hip_atomic_fetch_add(cnt + tl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (threadIdx.x == 0) sflag[0] = __hip_atomic_fetch_add(cnt + at.tl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       const int ticket = __builtin_amdgcn_readfirstlane(sflag[0]);  // wave-uniform: no waterfall around the rsrc
       stamp(ep, 2, now());
@@ -262,7 +309,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
         asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
         stamp(ep, 6, ((unsigned long long)ticket << 32) | (xcc & 0xF));
       }
-      f32x4* slots = reinterpret_cast<f32x4*>(part) + (size_t)tl * (S - 1) * kSlotF4;
+      f32x4* slots = reinterpret_cast<f32x4*>(part) + (size_t)at.tl * (S - 1) * kSlotF4;
       const int lane_off = w * (8 * QI * 64) + lane;
       if (ticket < S - 1) {
         // plain stores (they stay in this XCD's L2 for the same-XCD reader), every wave drained, then ONE agent-scope
@@ -280,14 +327,14 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
         if (threadIdx.x == 0) {
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __hip_atomic_fetch_add(cnt + kFixTiles + tl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_add(cnt + kFixTiles + at.tl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         stamp(ep, 4, now());
         return;
       }
       if (threadIdx.x == 0) {
         unsigned spins = 0;
-        while (__hip_atomic_load(cnt + kFixTiles + tl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1) {
+        while (__hip_atomic_load(cnt + kFixTiles + at.tl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1) {
           __builtin_amdgcn_s_sleep(2);
           if (++spins > (1u << 22)) {  // ~0.1 s: a writer never counted itself (cannot happen); flag, do not hang
             __hip_atomic_fetch_add(cnt - 4, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -297,8 +344,8 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         // every other slice already took its ticket and counted itself: nothing touches this pair again in
         // this launch, so the last arriver leaves it zero for the next one
-        __hip_atomic_store(cnt + tl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(cnt + kFixTiles + tl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(cnt + at.tl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(cnt + kFixTiles + at.tl, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -331,61 +378,84 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     }
   }
 
-  // acc[4 qm + i] holds X rows row0 + QR qm + 16 i (i < QI)
-  const int row0 = m0 + wm * (BM / 2), tile0 = n0 / 16 + wn * 4;
-  const bool cols = tile0 * 16 < N;  // uniform; N % 128 == 0: a wave's 64 columns are all there or none is
-  auto mrow = [&](int mt) { return row0 + QR * (mt >> 2) + 16 * (mt & 3); };
-  if constexpr (MODE == kStoreBf16) {
-    // stage the wave's 128 x 64 bf16 tile in LDS (all DMA retired, everyone past its last fragment read), then
-    // 16-byte row stores: 8 lanes per 128-byte row, 8 rows per instruction
-    __syncthreads();
-    if (!cols) return;
-    bf16* st = reinterpret_cast<bf16*>(smem + w * (128 * 64 * 2));
+    // acc[4 qm + i][nt]: X rows row0 + QR qm + 16 i (i < QI), column tile tile0 + nt; turned, lane (r, g) has row r, columns 4 g .. 4 g + 3
+    const int row0 = at.m0 + wm * (BM / 2), tile0 = at.n0 / 16 + wn * 4;
+    const bool cols = tile0 * 16 < N;  // uniform; N % 128 == 0: a wave's 64 columns are all there or none is
+    auto mt_of = [](int k) { return k / QI * 4 + k % QI; };  // k < 2 QI
+    auto row_of = [&](int k) { return row0 + QR * (k / QI) + 16 * (k % QI); };
+    if (!kTurned || !wide_results(ep)) {  // uniform; such a launch has a workgroup per tile
+      if (!cols) return;
+      float* part_ks = partial_of(ep, part, at.ks, M, N);
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
+      for (int k = 0; k < 2 * QI; ++k)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int rr = 16 * mt + 4 * g + i, cc = 16 * nt + r;
-          // 16-byte chunk (cc >> 3) of row rr at chunk slot (cc >> 3) ^ (rr & 7): conflict-spread writes and reads
-          st[rr * 64 + ((((cc >> 3) ^ (rr & 7)) << 3) | (cc & 7))] = f2bf(acc[mt][nt][i]);
+          for (int i = 0; i < 4; ++i) {
+            const float v = acc[mt_of(k)][nt][i];
+            const float partner = MODE == kQkvRope || MODE == kSiluMul ? __shfl_xor(v, kTurned ? 32 : 8) : 0.f;
+            epilogue<MODE>(ep, part_ks, M, N, row_of(k) + (kTurned ? r : 4 * g + i), tile0 + nt, kTurned ? 4 * g + i : r, v, partner);
+          }
+      if constexpr (FIX) stamp(ep, 5, now());
+      return;
+    }
+    bf16* st = reinterpret_cast<bf16*>(smem + 2 * kBuf + w * kStage);
+    // the wave's rows, from its first column on
+    const int col0 = MODE == kSiluMul ? tile0 * 8 : tile0 * 16;
+    const __amdgpu_buffer_rsrc_t to = make_rsrc(reinterpret_cast<bf16*>(ep.out) + (size_t)min(row0, M - 1) * ep.ldo + (cols ? col0 : 0), 0x7fffffffu);
+    auto put = [&](const bf16x8& v, int m, int piece) {
+      typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), to,
+                                             cols && m < M ? (uint32_t)(m - row0) * (uint32_t)ep.ldo * 2 + 16 * piece : kOOB, 0, 0);
+    };
+    if constexpr (MODE == kStoreBf16) {
+      // through the wave's LDS, 32 rows at a time: 16-byte row stores, 8 lanes per 128-byte row, 8 rows per instruction
+#pragma unroll
+      for (int k = 0; k < 2 * QI; k += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) {
+            bf16x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = f2bf(acc[mt_of(k + u)][nt][i]);
+            // piece 2 nt + g / 2 of row r at piece slot ^ (r & 7): conflict-spread writes and reads
+            *reinterpret_cast<bf16x4*>(st + (16 * u + r) * 64 + (((2 * nt + (g >> 1)) ^ (r & 7)) << 3) + 4 * (g & 1)) = v;
+          }
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const int rr = 8 * it + (lane >> 3), ch = lane & 7;
+          const bf16x8 v = *reinterpret_cast<const bf16x8*>(st + rr * 64 + ((ch ^ (rr & 7)) << 3));
+          put(v, row_of(k + (it >> 1)) + (rr & 15), ch);
         }
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's own LDS image is complete
-    bf16* out = reinterpret_cast<bf16*>(ep.out);
+      }
+    } else if constexpr (MODE == kSiluMul) {
+      // gate rows 0-7 and up rows 8-15 of a column tile: lanes 0-31 and 32-63.  Of two row tiles, the lower lanes take the first and the upper ones the second.
 #pragma unroll
-    for (int it = 0; it < 16; ++it) {
-      const int rr = 8 * it + (lane >> 3), ch = lane & 7;
-      if ((rr & 63) >= QR) continue;  // BM 192: slot rows 48-63 of a quadrant hold no X row
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(st + rr * 64 + ((ch ^ (rr & 7)) << 3));
-      const int m = row0 + QR * (rr >> 6) + (rr & 63);
-      if (m < M) *reinterpret_cast<bf16x8*>(out + (size_t)m * ep.ldo + n0 + wn * 64 + ch * 8) = v;
+      for (int k = 0; k < 2 * QI; k += 2) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+          bf16x4 v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[mt_of(k)][nt][i]), __float_as_uint(acc[mt_of(k + 1)][nt][i]), false, false);
+            v[i] = f2bf(gate_act(ep, __uint_as_float(x[0])) * __uint_as_float(x[1]));
+          }
+          const int rr = 16 * (g >> 1) + r;  // 32 rows of four 16-byte pieces
+          *reinterpret_cast<bf16x4*>(st + rr * 32 + ((nt ^ (rr >> 1 & 3)) << 3) + 4 * (g & 1)) = v;
+        }
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+          const int rr = 16 * it + (lane >> 2), ch = lane & 3;
+          const bf16x8 v = *reinterpret_cast<const bf16x8*>(st + rr * 32 + ((ch ^ (rr >> 1 & 3)) << 3));
+          put(v, row_of(k + it) + (rr & 15), ch);
+        }
+      }
     }
     if constexpr (FIX) stamp(ep, 5, now());
-    return;
-  }
-  if (!cols) return;
-  if constexpr (MODE == kSiluMul) {
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-        if ((mt & 3) < QI) silu_epilogue4(ep, M, mrow(mt) + 4 * g, tile0 + nt, r, acc[mt][nt]);
-    if constexpr (FIX) stamp(ep, 5, now());
-    return;
-  }
-  float* part_ks = partial_of(ep, part, ks, M, N);
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt) {
-    if ((mt & 3) >= QI) continue;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float v = acc[mt][nt][i];
-        const float partner = (MODE == kQkvRope) ? __shfl_xor(v, 8) : 0.f;
-        epilogue<MODE>(ep, part_ks, M, N, mrow(mt) + 4 * g + i, tile0 + nt, r, v, partner);
-      }
+    if (!more) return;
+    bid += gridDim.x;
+    at = next;
   }
 }
 
@@ -398,8 +468,9 @@ static hipError_t launch_pipe_bm(const bf16* X, int ldx, int M, const bf16* W, i
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)gp::kLDS);
     attr_set = true;
   }
-  const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256;
-  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(nbm * nbn * S), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
+  const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256, n = nbm * nbn * S;
+  const bool stay = !FIX && n >= 2 * gp::kCUs && gp::stores<MODE, BM / 64>() > 0 && K / S >= 256 && gp::wide_results(ep) && kernel_cfg_int("pipe_stay", 1);
+  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(stay ? std::min(n, gp::kCUs) : n), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
                      N, K / S, ep, part);
   return hipGetLastError();
 }
