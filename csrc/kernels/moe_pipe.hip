@@ -41,7 +41,8 @@ constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 
 constexpr int kBuf = kA + kB;
 constexpr int kIds = 2 * kBuf;  // the tile's ids (256 ints), their weights (256 floats), their rows of the result (256 ints)
 constexpr int kSay = kIds + 3 * 256 * 4;  // one word: whether this workgroup ends a cut tile
-constexpr size_t kLDS = kSay + 16;
+constexpr int kStage = kSay + 16;  // 2 KiB per wave: 16 rows of its hidden units on their way to 16-byte stores
+constexpr size_t kLDS = kStage + 8 * 2048;
 
 // The last round where only a few tiles are left for it: each XCD runs its tiles in rounds of one per CU, and the tiles past the last whole
 // round are cut over K.  Every piece leaves its fp32 sums in `ws`, and the one that finishes last -- a counter, nobody waits -- adds them in the
@@ -274,7 +275,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            acc[4 * qm + i][2 * qn + j] = mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j]);
+            acc[4 * qm + i][2 * qn + j] = MODE == 1 ? mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j])
+                                                    : mfma16x16x32(b[2 * qn + j][sp], a[i][sp], acc[4 * qm + i][2 * qn + j]);
       }
       __builtin_amdgcn_s_setprio(0);
       asm volatile("s_barrier" ::: "memory");
@@ -371,6 +373,46 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
       }
     }
 
+    if constexpr (MODE != 1) {
+      // The weights were the products' first operand: a lane has four hidden units of a row, which leaves through the wave's LDS in pieces of 16 bytes.
+      // Two-byte stores from 16 lanes a row, expf and a division / this, work list and both products, us: 1024 rows of 2048 x 1408 157 / 152, 400
+      // 111 / 106; 4096 x 3584, 2048 rows 756 / 732, 3000 995 / 965.
+      constexpr int kPer = MODE == 0 ? 4 : 8;  // pieces of a row
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // addresses of this part are not made before the K loop either
+      const int r = ln & 15, g = ln >> 4;
+      const int f0 = n0 + wn * 8 * kPer;
+      char* st = smem + kStage + w * 2048;
+      if (f0 < N)  // uniform: N % 64 == 0
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          if ((m & 3) >= QI) continue;  // uniform
+          const int first_row = (wm * 2 + (m >> 2)) * QR + 16 * (m & 3);
+          const float wt = s_w[first_row + r];
+#pragma unroll
+          for (int q = 0; q < kPer / 2; ++q) {
+            bf16x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (MODE == 0) {
+                v[e] = (bf16)(silu(acc[m][2 * q][e] * wt) * (acc[m][2 * q + 1][e] * wt));
+              } else {
+                const float z = acc[m][q][e] * wt;
+                v[e] = (bf16)(z > 0.0f ? z * z : 0.0f);
+              }
+            }
+            *reinterpret_cast<bf16x4*>(st + r * 16 * kPer + (((2 * q + (g >> 1)) ^ (r >> (MODE == 0 ? 1 : 0) & (kPer - 1))) << 4) + 8 * (g & 1)) = v;
+          }
+#pragma unroll
+          for (int it = 0; it < kPer / 4; ++it) {
+            const int rr = it * 8 + ln / kPer, piece = ln % kPer;
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(st + rr * 16 * kPer + ((piece ^ (rr >> (MODE == 0 ? 1 : 0) & (kPer - 1))) << 4));
+            const int id = s_id[first_row + rr];
+            if (id >= 0) *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(p.h) + (int64_t)id * p.ldh + f0 + 8 * piece) = v;
+          }
+        }
+      continue;
+    }
 #pragma unroll
     for (int qm = 0; qm < 2; ++qm)
 #pragma unroll
@@ -379,28 +421,12 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         for (int j = 0; j < 4; ++j) {
           if (i >= QI) continue;  // uniform
           const int at = (wm * 2 + qm) * QR + 16 * i + 4 * g + j;
-          const int id = s_id[at];
-          if (id < 0) continue;
+          if (s_id[at] < 0) continue;
           const float wt = s_w[at];
-          const f32x4(&c)[4] = acc[4 * qm + i];
-          if (MODE == 0) {
 #pragma unroll
-            for (int qn = 0; qn < 2; ++qn) {
-              const int f = n0 + (wn * 2 + qn) * 16 + r;
-              const float gv = c[2 * qn][j] * wt;
-              if (f < N)
-                reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] =
-                    (bf16)(gv / (1.0f + expf(-gv)) * (c[2 * qn + 1][j] * wt));
-            }
-          } else {
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-              const int f = n0 + (wn * 4 + n) * 16 + r;
-              if (f >= N) continue;
-              const float v = c[n][j] * wt;
-              if (MODE == 1) p.o[(int64_t)s_o[at] * p.W + f] = v;
-              else reinterpret_cast<bf16*>(p.h)[(int64_t)id * p.ldh + f] = (bf16)(v > 0.0f ? v * v : 0.0f);
-            }
+          for (int n = 0; n < 4; ++n) {
+            const int f = n0 + (wn * 4 + n) * 16 + r;
+            if (f < N) p.o[(int64_t)s_o[at] * p.W + f] = acc[4 * qm + i][n][j] * wt;
           }
         }
   }
