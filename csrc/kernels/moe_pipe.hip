@@ -275,8 +275,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            acc[4 * qm + i][2 * qn + j] = MODE == 1 ? mfma16x16x32(a[i][sp], b[2 * qn + j][sp], acc[4 * qm + i][2 * qn + j])
-                                                    : mfma16x16x32(b[2 * qn + j][sp], a[i][sp], acc[4 * qm + i][2 * qn + j]);
+            acc[4 * qm + i][2 * qn + j] = mfma16x16x32(b[2 * qn + j][sp], a[i][sp], acc[4 * qm + i][2 * qn + j]);
       }
       __builtin_amdgcn_s_setprio(0);
       asm volatile("s_barrier" ::: "memory");
@@ -373,16 +372,16 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
       }
     }
 
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // addresses of this part are not made before the K loop either
+    const int r = ln & 15, g = ln >> 4;
+    char* st = smem + kStage + w * 2048;
     if constexpr (MODE != 1) {
       // The weights were the products' first operand: a lane has four hidden units of a row, which leaves through the wave's LDS in pieces of 16 bytes.
       // Two-byte stores from 16 lanes a row, expf and a division / this, work list and both products, us: 1024 rows of 2048 x 1408 157 / 152, 400
       // 111 / 106; 4096 x 3584, 2048 rows 756 / 732, 3000 995 / 965.
       constexpr int kPer = MODE == 0 ? 4 : 8;  // pieces of a row
-      int ln = lane;
-      asm volatile("" : "+v"(ln));  // addresses of this part are not made before the K loop either
-      const int r = ln & 15, g = ln >> 4;
       const int f0 = n0 + wn * 8 * kPer;
-      char* st = smem + kStage + w * 2048;
       if (f0 < N)  // uniform: N % 64 == 0
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
@@ -413,22 +412,26 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         }
       continue;
     }
+    // fp32 rows, 128 bytes of 16 of them at a time
 #pragma unroll
-    for (int qm = 0; qm < 2; ++qm)
+    for (int m = 0; m < 8; ++m) {
+      if ((m & 3) >= QI) continue;  // uniform
+      const int first_row = (wm * 2 + (m >> 2)) * QR + 16 * (m & 3);
+      const float wt = s_w[first_row + r];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int q = 0; q < 2; ++q) {
+        const int f0 = n0 + wn * 64 + 32 * q;
+        if (f0 >= N) continue;  // uniform: N % 64 == 0
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (i >= QI) continue;  // uniform
-          const int at = (wm * 2 + qm) * QR + 16 * i + 4 * g + j;
-          if (s_id[at] < 0) continue;
-          const float wt = s_w[at];
+        for (int n = 0; n < 2; ++n) *reinterpret_cast<f32x4*>(st + r * 128 + (((4 * n + g) ^ (r & 7)) << 4)) = acc[m][2 * q + n] * wt;
 #pragma unroll
-          for (int n = 0; n < 4; ++n) {
-            const int f = n0 + (wn * 4 + n) * 16 + r;
-            if (f < N) p.o[(int64_t)s_o[at] * p.W + f] = acc[4 * qm + i][n][j] * wt;
-          }
+        for (int it = 0; it < 2; ++it) {
+          const int rr = it * 8 + (ln >> 3), piece = ln & 7, at = first_row + rr;
+          const f32x4 v = *reinterpret_cast<const f32x4*>(st + rr * 128 + ((piece ^ (rr & 7)) << 4));
+          if (s_id[at] >= 0) *reinterpret_cast<f32x4*>(p.o + (int64_t)s_o[at] * p.W + f0 + 4 * piece) = v;
         }
+      }
+    }
   }
 }
 
