@@ -383,6 +383,25 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     const bool cols = tile0 * 16 < N;  // uniform; N % 128 == 0: a wave's 64 columns are all there or none is
     auto mt_of = [](int k) { return k / QI * 4 + k % QI; };  // k < 2 QI
     auto row_of = [&](int k) { return row0 + QR * (k / QI) + 16 * (k % QI); };
+    if constexpr (MODE == kPartial || MODE == kStoreF32) {
+      // a row's offset once for its four column tiles; rows that are not there are past the descriptor's range (a branch and an address per value / this, us:
+      // 384 x 4096 x 4096 24.0 / 23.5, 300 x 2048 x 2048 12.6 / 12.3, 1500 x 2048 x 2048 21.4 / 21.1, 2048 x 4096 x 4096 63 / 61.5)
+      if (!cols) return;
+      const int ldo = MODE == kPartial ? (ep.parts ? ep.parts : 1) * N : ep.ldo;
+      float* out = MODE == kPartial ? partial_of(ep, part, at.ks, M, N) : reinterpret_cast<float*>(ep.out);
+      const __amdgpu_buffer_rsrc_t to = make_rsrc(out + (size_t)min(row0, M - 1) * ldo + tile0 * 16, 0x7fffffffu);
+#pragma unroll
+      for (int k = 0; k < 2 * QI; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = row_of(k) + 4 * g + i;
+          const uint32_t row = m < M ? (uint32_t)(m - row0) * (uint32_t)ldo * 4 + 4 * r : kOOB;
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[mt_of(k)][nt][i]), to, row + 64 * nt, 0, 0);
+        }
+      if constexpr (FIX) stamp(ep, 5, now());
+      return;
+    }
     if (!kTurned || !wide_results(ep)) {  // uniform; such a launch has a workgroup per tile
       if (!cols) return;
       float* part_ks = partial_of(ep, part, at.ks, M, N);
