@@ -23,8 +23,8 @@
 // give every expert's place); the host knows only a bound of the tile count.
 //
 // Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
-// experts, top 2, shared 7168: 2369 -> 1014 us (1042 TFLOP/s); 2048 rows: 1695 -> 775; 1024 rows of 2048 x 1408, shared
-// 2816: 245 -> 168; 1024 rows of 1024 x 512, 8 experts: 49 -> 41.  Up to 192 rows moe_stream.hip takes
+// experts, top 2, shared 7168: 2369 -> 953 us (1109 TFLOP/s); 2048 rows: 1695 -> 720; 1024 rows of 2048 x 1408, shared
+// 2816: 245 -> 150; 1024 rows of 1024 x 512, 8 experts: 49 -> 38.  Up to 192 rows moe_stream.hip takes
 // the sizes whose weights it need not read twice, or the kernels of moe.hip a few rows of small experts (moe_form).
 #include <algorithm>
 #include <cmath>
