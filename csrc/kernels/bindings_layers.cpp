@@ -628,6 +628,20 @@ int64_t moe_plan(int64_t M, int64_t W, int64_t F, int64_t Fs, int64_t E, int64_t
   return form == dsse::MoeForm::kPipe ? 0 : (form == dsse::MoeForm::kStream ? 1 : 2);
 }
 
+// What the workgroups of the expert GEMM pipeline take, rows[e] rows of expert e: [n, 9] of XCD, expert, row tile, column block, slice, piece, of,
+// first K step, K steps.  product: 0 gate and up, 1 down, 2 up alone; cut: as moe_cut of DSSE_KERNEL_CFG
+Tensor moe_pipe_walks(at::IntArrayRef rows, int64_t W, int64_t F, int64_t Fs, int64_t top, int64_t product, int64_t parts, int64_t cut) {
+  dsse::MoeGroupedParams p{};
+  std::vector<int> r(rows.begin(), rows.end());
+  int64_t ids = 0;
+  for (int n : r) ids += n;
+  TORCH_CHECK(top > 0 && ids > 0 && ids % top == 0 && W >= 128 && F >= 128 && (Fs == 0 || Fs >= 128) && product >= 0 && product <= 2, "moe_pipe_walks");
+  p.M = (int)(ids / top), p.W = (int)W, p.F = (int)F, p.Fs = (int)Fs, p.E = (int)r.size(), p.top = (int)top, p.S = (int)top + (Fs > 0 ? 1 : 0);
+  p.parts = parts ? (int)parts : p.S, p.cut = (int)cut;
+  const std::vector<int> w = dsse::moe_pipe_walks(p, (int)product, r.data());
+  return at::tensor(w, at::kInt).view({-1, 9});
+}
+
 // moe_topk and the work list of moe_grouped (aligned) in one launch, for decode-sized steps; false: nothing done, the step is larger.
 bool moe_topk_lists(const Tensor& logits, Tensor& topk_idx, Tensor& topk_w, Tensor& sorted, Tensor& tile_expert,
                     Tensor& num_tiles, bool shared) {
@@ -688,6 +702,7 @@ TORCH_LIBRARY_FRAGMENT(dsse, m) {
         });
   m.def("gemm_rm_form_rows(int M, int N, int batch=1) -> int",
         [](int64_t M, int64_t N, int64_t batch) { return (int64_t)dsse::gemm_rm_form_rows((int)M, (int)N, (int)batch); });
+  m.def("moe_pipe_walks(int[] rows, int W, int F, int Fs, int top, int product, int parts=0, int cut=0) -> Tensor", &moe_pipe_walks);
   m.def("moe_plan(int M, int W, int F, int Fs, int E, int top, bool gated) -> int", &moe_plan);
   m.def("moe_parts(Tensor x, int top, Tensor? gate, Tensor up, Tensor down, Tensor? sgate, Tensor? sup, Tensor? sdown, Tensor h) -> int");
   m.def("moe_topk_lists(Tensor logits, Tensor(a!) topk_idx, Tensor(b!) topk_w, Tensor(c!) sorted, Tensor(d!) tile_expert, "

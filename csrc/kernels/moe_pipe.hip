@@ -28,13 +28,16 @@
 // the sizes whose weights it need not read twice, or the kernels of moe.hip a few rows of small experts (moe_form).
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "lds_dma.h"
+#include "moe_cut.h"
 #include "moe_rows.h"
 
 namespace dsse {
 namespace {
 namespace mp {
+using namespace moe_cut;
 
 constexpr int kA = 256 * 128;   // row image of one K step: 256 rows x 64 bf16
 constexpr int kB = 256 * 128;   // weight image: 16 column tiles x 16 rows x 64 bf16
@@ -44,13 +47,7 @@ constexpr int kSay = kIds + 3 * 256 * 4;  // one word: whether this workgroup en
 constexpr int kStage = kSay + 16;  // 2 KiB per wave: 16 rows of its hidden units on their way to 16-byte stores
 constexpr size_t kLDS = kStage + 8 * 2048;
 
-// The last round where only a few tiles are left for it: each XCD runs its tiles in rounds of one per CU, and the tiles past the last whole
-// round are cut over K.  Every piece leaves its fp32 sums in `ws`, and the one that finishes last -- a counter, nobody waits -- adds them in the
-// order of the pieces and runs the epilogue.
-constexpr int kCUs = 32;              // per XCD
-constexpr int kMostCut = 8;           // pieces of a tile
-constexpr int kPieces = 16;           // pieces per XCD
-constexpr int kCutTiles = 4;          // cut tiles per XCD: the counters are 16-bit halves of the first of the 64 ints behind the work list
+// Tiles cut over K (moe_cut.h): the counters are 16-bit halves of the first of the 64 ints behind the work list
 constexpr int kSlot = 8 * 32 * 64;    // f32x4 of one piece: [wave][row tile, column tile][lane]
 static_assert(8 * kPieces * kSlot * 4 == kMoeCutFloats && 8 * kCutTiles <= 2 * 64, "workspace and counters");
 
@@ -122,14 +119,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
   const int nb_r = blocks(p.F), nb_s = blocks(p.Fs);
   const int slices = MODE == 1 ? p.parts - p.S + 1 : 1;  // of the shared expert's hidden units
   const int tiles_s = (shared + tall - 1) / tall * nb_s, total_s = tiles_s * slices, total_r = row_tiles * nb_r;
-  // Pieces pay where they are few -- tiles of a round that is half empty run faster than those of a full one -- and long, and where no
-  // shared expert's longer walk is what the launch waits for (MODE 1).  Without / with, one MI355X, work list and both products, us: 16 experts, top
-  // 2 and a shared one, 2048 x 1408, 1024 rows (264 tiles, one left per XCD) 152 / 144; 4096 x 3584, 200 rows 320 / 300, 1300 567 / 541,
-  // 1500 609 / 584, 3000 1030 / 1007.  With more than these left it turns: 2048 x 1408, three or four tiles left, 1100 rows 151 / 154, five to eight 1300
-  // rows 154 / 163, 1500 165 / 170; 16 K steps, 1024 x 2048, 2500 rows 174 / 178.
   const int steps_r = (MODE == 1 ? p.F : p.W) >> 6, steps_s = total_s ? (MODE == 1 ? p.Fs / slices : p.W) >> 6 : steps_r;
-  const int most_left = p.cut ? kCutTiles : steps_r < 32 || steps_s > steps_r ? 0 : min(kCutTiles, steps_r / 16);
-  const int most_cut = p.cut ? min(p.cut, min(steps_r, steps_s) / 2) : kMostCut;
+  const Cut most = most_cut(steps_r, steps_s, p.ws ? p.cut : 1);
 
   // One tile; a second round only if a choice list is not what it should be (the list is read again for it: no registers for it in the K loop)
   for (int v = blockIdx.x; ; v += gridDim.x, read_list()) {
@@ -137,13 +128,9 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0;
     const int r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
     if (item >= (total_s + 7) / 8 + (total_r + 7) / 8 + kPieces) return;  // past every XCD's share
-    // the tiles past the last whole round, each in `cut` pieces
-    const int left = (ns + nr) % kCUs;
-    const int cut = !p.ws || left < 1 || left > most_left ? 1 : min(most_cut, kPieces / left);
-    const int whole = cut > 1 ? ns + nr - left : ns + nr;
-    const int u = item < whole ? item : whole + (item - whole) / cut;
+    Item it = item_of(item, ns + nr, most);
+    const int u = it.u;
     if (u >= ns + nr) continue;
-    const int piece = item < whole ? 0 : (item - whole) % cut, of = item < whole ? 1 : cut;
     const bool sh = u < ns;
     Place pl;
     int e;
@@ -167,10 +154,9 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
       list.each([&](int, int ve) { pl.tiles += __popcll(__ballot(ve == e)); });
       pl.at = at - opener * nb_r;
     }
-    // groups of 8 row tiles swept column by column
-    const int nb = sh ? nb_s : nb_r, T = (pl.tiles + tall - 1) / tall, q = (pl.tiles + T - 1) / T;
-    const int grp = pl.at / (8 * nb), gsz = min(8, T - 8 * grp), in = pl.at - grp * 8 * nb;
-    const int rt = 8 * grp + in % gsz, n0 = in / gsz * kCols;
+    const int T = (pl.tiles + tall - 1) / tall, q = (pl.tiles + T - 1) / T;
+    const Spot spot = spot_of(pl.at, T, sh ? nb_s : nb_r);
+    const int rt = spot.row_tile, n0 = spot.block * kCols;
     const int t0 = pl.first + rt * q;
     const int rows64 = min(q, pl.tiles - rt * q);  // list tiles of this row tile: 1..4, or none (T q > tiles + q)
     if (rows64 <= 0) continue;
@@ -179,7 +165,12 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
     const int slice = sh ? (s0 + u) / tiles_s : 0, parts = sh ? slices : 1;
     const int k0 = (K >> 6) * slice / parts, kn = (K >> 6) * (slice + 1) / parts - k0;  // its K steps
-    const int first = k0 + kn * piece / of, nk = k0 + kn * (piece + 1) / of - first;    // this piece's
+    if (!cuts(it, kn)) {  // its first piece takes it whole
+      if (it.piece) continue;
+      it.of = 1;
+    }
+    const Walk mine = walk_of(k0, kn, it.piece, it.of);  // this piece's
+    const int first = mine.first, nk = mine.steps;
     const int off = ONCE ? n0 / kCols % nk : 0;
     const bf16* X = reinterpret_cast<const bf16*>(MODE == 1 ? p.h : p.x);
     const int ldx = MODE == 1 ? p.ldh : p.W;
@@ -324,25 +315,26 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     };
     int t = 0;
     for (; t < nk - 2; ++t) step(t, std::integral_constant<int, 0>{});
-    step(t++, std::integral_constant<int, 1>{});  // nk >= 2 (moe_lines_ok)
+    step(t++, std::integral_constant<int, 1>{});  // nk >= 2: a tile's (moe_lines_ok; bindings for slices), a piece's (cuts)
     step(t, std::integral_constant<int, 2>{});
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // the two rows' barrier counts meet
 
-    if (of > 1) {
-      f32x4* slots = reinterpret_cast<f32x4*>(p.ws) + (size_t)(x * kPieces + (u - whole) * cut) * kSlot;
+    if (it.of > 1) {
+      const int of = it.of;
+      f32x4* slots = reinterpret_cast<f32x4*>(p.ws) + (size_t)(x * kPieces + (u - it.whole) * of) * kSlot;
       int at = w * 32 * 64 + lane;
       asm volatile("" : "+v"(at));  // addresses of this part are not made before the K loop, whose registers are full
 #pragma unroll
       for (int m = 0; m < 8; ++m)
         if ((m & 3) < QI)  // uniform
 #pragma unroll
-          for (int n = 0; n < 4; ++n) slots[(size_t)piece * kSlot + at + (4 * m + n) * 64] = acc[m][n];
+          for (int n = 0; n < 4; ++n) slots[(size_t)it.piece * kSlot + at + (4 * m + n) * 64] = acc[m][n];
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       int* say = reinterpret_cast<int*>(smem + kSay);
       if (threadIdx.x == 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const int c = x * kCutTiles + u - whole, shift = 16 * (c & 1);
+        const int c = x * kCutTiles + u - it.whole, shift = 16 * (c & 1);
         int* count = p.sorted + (size_t)list.n * 64 + (c >> 1);
         const int before = __hip_atomic_fetch_add(count, 1 << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> shift & 0xffff;
         *say = before == of - 1;
@@ -571,6 +563,42 @@ bool moe_lines_ok(const MoeGroupedParams& p) {
   if ((int64_t)p.M * p.W * 2 >= kRange || ids * p.ldh * 2 >= kRange || widest * p.W * 2 >= kRange) return false;
   if (!sixteens(p.x) || !sixteens(p.h) || !sixteens(p.up) || !sixteens(p.down) || (p.gate && !sixteens(p.gate))) return false;
   return !shared || (sixteens(p.sgate) && sixteens(p.sup) && sixteens(p.sdown));
+}
+
+// What every workgroup of a product takes, rows[e] rows of expert e: {XCD, expert (E: the shared one), row tile, column block, slice, piece, of,
+// first K step, K steps}, by the kernel's own rules on the host
+std::vector<int> moe_pipe_walks(const MoeGroupedParams& p, int mode, const int* rows) {
+  using namespace moe_cut;
+  const int tall = mode == 1 ? down_height(p, p.parts - p.S + 1).tall : moe_pipe_height(p, mode);
+  const int nb_r = (int)col_blocks(p, mode, p.F), nb_s = (int)col_blocks(p, mode, p.Fs), slices = mode == 1 ? p.parts - p.S + 1 : 1;
+  const int shared = p.S > p.top ? (p.M + 63) / 64 : 0, tiles_s = (shared + tall - 1) / tall * nb_s, total_s = tiles_s * slices;
+  auto row_tiles = [&](int e) { return ((rows[e] + 63) / 64 + tall - 1) / tall; };
+  int total_r = 0;
+  for (int e = 0; e < p.E; ++e) total_r += row_tiles(e) * nb_r;
+  const int steps_r = (mode == 1 ? p.F : p.W) >> 6, steps_s = total_s ? (mode == 1 ? p.Fs / slices : p.W) >> 6 : steps_r;
+  const Cut most = most_cut(steps_r, steps_s, p.cut);
+  std::vector<int> out;
+  for (int x = 0; x < 8; ++x) {
+    const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0, r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
+    for (int item = 0; item < (total_s + 7) / 8 + (total_r + 7) / 8 + kPieces; ++item) {
+      Item it = item_of(item, ns + nr, most);
+      if (it.u >= ns + nr) continue;
+      const bool sh = it.u < ns;
+      int e = p.E, at = sh ? (s0 + it.u) % tiles_s : r0 + it.u - ns;
+      if (!sh)
+        for (e = 0; at >= row_tiles(e) * nb_r; ++e) at -= row_tiles(e) * nb_r;
+      const int slice = sh ? (s0 + it.u) / tiles_s : 0, parts = sh ? slices : 1, K = mode == 1 ? (sh ? p.Fs : p.F) : p.W;
+      const int k0 = (K >> 6) * slice / parts, kn = (K >> 6) * (slice + 1) / parts - k0;
+      const Spot spot = spot_of(at, sh ? (shared + tall - 1) / tall : row_tiles(e), sh ? nb_s : nb_r);
+      if (!cuts(it, kn)) {
+        if (it.piece) continue;
+        it.of = 1;
+      }
+      const Walk mine = walk_of(k0, kn, it.piece, it.of);
+      out.insert(out.end(), {x, e, spot.row_tile, spot.block, slice, it.piece, it.of, mine.first, mine.steps});
+    }
+  }
+  return out;
 }
 
 // Two slices where they end sooner.  One / two, work list, both products and the norm that adds the parts, in us: 2048 x 1408, 16 experts,

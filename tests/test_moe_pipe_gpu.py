@@ -110,3 +110,38 @@ def test_cut_tiles(gpu, monkeypatch, M, W, F, Fs, E, top, first, gated, cut, onc
     finally:
         monkeypatch.undo()
         ops.refresh_env()
+
+
+# Down products that the rule itself cuts (32 K steps and more), with a shared expert of so few hidden units that its tiles, the last of some XCDs, stay
+# whole; its hidden units in one and in two slices
+@pytest.mark.parametrize("M,W,F,Fs,E,top,slices,pieces", [
+    (300, 256, 2048, 128, 8, 1, 1, 8), (300, 512, 4096, 512, 8, 2, 1, 1), (300, 512, 4096, 512, 8, 2, 2, 1), (700, 256, 8192, 256, 4, 1, 2, 5)])
+@pytest.mark.parametrize("once", [1, 2], ids=["once", "plain"])
+def test_down_products_cut_by_the_rule(gpu, monkeypatch, M, W, F, Fs, E, top, slices, pieces, once):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2, moe_once=once))
+    ops.refresh_env()
+    try:
+        g = torch.Generator().manual_seed(M + F)
+        c = lambda t: t.to(gpu)  # noqa: E731
+        rnd = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16()  # noqa: E731
+        x, gate, up, down, sh = torch.randn(M, W, generator=g).bfloat16(), rnd(E, F, W), rnd(E, F, W), rnd(E, W, F), (rnd(Fs, W), rnd(Fs, W), rnd(W, Fs))
+        S, parts = top + 1, top + slices
+        idx = ((torch.arange(M)[:, None] + torch.arange(top)) % E).int()
+        walks = torch.ops.dsse.moe_pipe_walks(torch.bincount(idx.flatten(), minlength=E).tolist(), W, F, Fs, top, 1, parts)
+        assert int(walks[:, 6].max()) == pieces
+        w = torch.rand(M, S, generator=g) + 0.25
+        ref = torch.zeros(M * S, W)
+        lref.moe_grouped(x, idx, w, gate, up, down, *sh, ref)
+        tiles = -(-M * S // 64) + E + 1
+        o = torch.full((M * parts, W), float("nan"), device=gpu)
+        ops.moe_grouped(*(c(t) for t in (x, idx, w, gate, up, down, *sh)), torch.zeros(tiles * 64, dtype=torch.int32, device=gpu),
+                        torch.zeros(tiles, dtype=torch.int32, device=gpu), torch.zeros(1, dtype=torch.int32, device=gpu),
+                        torch.zeros(M * S, F, dtype=torch.bfloat16, device=gpu), o, parts=parts)
+        got, ref = o.cpu().view(M, parts, W), ref.view(M, S, W)
+        got = torch.cat([got[:, :top], got[:, top:].sum(1, keepdim=True)], 1)
+        for a, b in ((got[:, :top], ref[:, :top]), (got[:, top:], ref[:, top:])):  # as above, the shared expert by itself
+            assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -8
+            assert float((a - b).abs().max()) <= 2.0 ** -5 * float(b.abs().max())
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
