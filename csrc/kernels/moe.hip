@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void moe_ffn_kernel(MoeFfnParams p) {
 //   moe_align     one workgroup: per-expert counts -> tile-padded offsets -> sorted ids (pads -1), the expert of every
 //                 tile and the tile count, and 64 zeros behind the list (moe_pipe's counters; the scratch holds a tile more than any
 //                 list: sum of ceil(ids of an expert / 64) <= ids / 64 + 63 / 64 per expert).  The order of ids inside an expert is whatever the atomics give; a row's
-//                 result does not depend on its place in a tile.
+//                 result does not depend on its place (moe_pipe cuts all row tiles of a column block over K, or none).
 //   moe_gate_up   h[id, f] = silu(gate_e[f] . x[row]) * (up_e[f] . x[row])       (element type)
 //   moe_down      o[id, :] = weight(id) * down_e . h[id]                          (fp32)
 // The residual norm that follows sums a row's S slots (scalar_norm nsum).

@@ -50,9 +50,6 @@ __host__ __device__ inline Item item_of(int item, int tiles, Cut most) {
   return u < tiles ? Item{u, (item - whole) % cut, cut, whole} : Item{tiles, 0, 1, whole};
 }
 
-// Whether a tile of kn K steps is cut.  The last tiles of an XCD may be a shared expert's, whose walk may be short.
-__host__ __device__ inline bool cuts(const Item& it, int kn) { return it.of > 1 && kn >= kLeast * it.of; }
-
 // Tile `at` of an expert of T row tiles and nb column blocks: groups of 8 row tiles swept column by column
 struct Spot {
   int row_tile, block;
@@ -60,6 +57,15 @@ struct Spot {
 __host__ __device__ inline Spot spot_of(int at, int T, int nb) {
   const int grp = at / (8 * nb), gsz = T - 8 * grp < 8 ? T - 8 * grp : 8, in = at - grp * 8 * nb;
   return Spot{8 * grp + in % gsz, in / gsz};
+}
+
+// Whether a tile of kn K steps is cut.  The last tiles of an XCD may be a shared expert's, whose walk may be short.  And a routed tile is cut only with
+// all T row tiles of its column block: which of them holds a row is up to the atomics that made the work list, so where one had another order of sums, the
+// same call would not give the same bits again.  (A shared expert's rows are in order.)  ns, tiles: the XCD's shared tiles, all of its tiles.
+__host__ __device__ inline bool cuts(const Item& it, int kn, int ns, int tiles, int row_tile, int T) {
+  if (it.of == 1 || kn < kLeast * it.of) return false;
+  const int block = it.u - row_tile;  // the block's first tile: T <= 8 follow each other, and no more than kCutTiles are cut
+  return it.u < ns || (block >= it.whole && block >= ns && block + T <= tiles);
 }
 
 struct Walk {

@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     const int K = MODE == 1 ? Fe : p.W, N = MODE == 1 ? p.W : Fe;
     const int slice = sh ? (s0 + u) / tiles_s : 0, parts = sh ? slices : 1;
     const int k0 = (K >> 6) * slice / parts, kn = (K >> 6) * (slice + 1) / parts - k0;  // its K steps
-    if (!cuts(it, kn)) {  // its first piece takes it whole
+    if (!cuts(it, kn, ns, ns + nr, rt, T)) {  // its first piece takes it whole
       if (it.piece) continue;
       it.of = 1;
     }
@@ -589,8 +589,9 @@ std::vector<int> moe_pipe_walks(const MoeGroupedParams& p, int mode, const int* 
         for (e = 0; at >= row_tiles(e) * nb_r; ++e) at -= row_tiles(e) * nb_r;
       const int slice = sh ? (s0 + it.u) / tiles_s : 0, parts = sh ? slices : 1, K = mode == 1 ? (sh ? p.Fs : p.F) : p.W;
       const int k0 = (K >> 6) * slice / parts, kn = (K >> 6) * (slice + 1) / parts - k0;
-      const Spot spot = spot_of(at, sh ? (shared + tall - 1) / tall : row_tiles(e), sh ? nb_s : nb_r);
-      if (!cuts(it, kn)) {
+      const int T = sh ? (shared + tall - 1) / tall : row_tiles(e);
+      const Spot spot = spot_of(at, T, sh ? nb_s : nb_r);
+      if (!cuts(it, kn, ns, ns + nr, spot.row_tile, T)) {
         if (it.piece) continue;
         it.of = 1;
       }

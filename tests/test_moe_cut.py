@@ -25,6 +25,9 @@ def _check(walks, steps_r, steps_s, experts):
         for rt, block in {k[1:3] for k in tiles if k[0] == e}:
             walk = sorted((t[3], t[4]) for k, p in tiles.items() if k[:3] == (e, rt, block) for t in p)
             assert walk[0][0] == 0 and sum(n for _, n in walk) == (steps_s if e == experts else steps_r)
+    # which of an expert's row tiles holds a row is not fixed, so the sums of a column block have one order in all of them
+    for e, block in {(k[0], k[2]) for k in tiles if k[0] < experts}:
+        assert len({len(p) for k, p in tiles.items() if (k[0], k[2]) == (e, block)}) == 1
     return {k: len(p) for k, p in tiles.items()}
 
 
@@ -32,7 +35,7 @@ def _check(walks, steps_r, steps_s, experts):
 # that leaves experts without rows; a step whose last tiles are routed
 @pytest.mark.parametrize("M,W,F,Fs,E,top,parts", [
     (300, 256, 2048, 128, 8, 1, 0), (300, 512, 4096, 512, 8, 2, 0), (300, 512, 4096, 512, 8, 2, 4), (1024, 2048, 1408, 2816, 16, 2, 0), (3000, 4096, 3584, 7168, 16, 2, 0),
-    (3000, 4096, 3584, 7168, 16, 2, 4), (700, 256, 8192, 256, 4, 1, 3)])
+    (3000, 4096, 3584, 7168, 16, 2, 4), (700, 256, 8192, 256, 4, 1, 3), (350, 2112, 320, 0, 3, 1, 0), (600, 2048, 256, 0, 2, 1, 0)])
 @pytest.mark.parametrize("cut", [0, 1, 3, 8])
 @pytest.mark.parametrize("uneven", [False, True])
 def test_pieces(M, W, F, Fs, E, top, parts, cut, uneven):

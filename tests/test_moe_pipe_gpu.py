@@ -115,7 +115,7 @@ def test_cut_tiles(gpu, monkeypatch, M, W, F, Fs, E, top, first, gated, cut, onc
 # Down products that the rule itself cuts (32 K steps and more), with a shared expert of so few hidden units that its tiles, the last of some XCDs, stay
 # whole; its hidden units in one and in two slices
 @pytest.mark.parametrize("M,W,F,Fs,E,top,slices,pieces", [
-    (300, 256, 2048, 128, 8, 1, 1, 8), (300, 512, 4096, 512, 8, 2, 1, 1), (300, 512, 4096, 512, 8, 2, 2, 1), (700, 256, 8192, 256, 4, 1, 2, 5)])
+    (300, 256, 2048, 128, 8, 1, 1, 8), (300, 512, 4096, 512, 8, 2, 1, 1), (300, 512, 4096, 512, 8, 2, 2, 1), (300, 512, 4096, 512, 4, 1, 2, 4)])
 @pytest.mark.parametrize("once", [1, 2], ids=["once", "plain"])
 def test_down_products_cut_by_the_rule(gpu, monkeypatch, M, W, F, Fs, E, top, slices, pieces, once):
     monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2, moe_once=once))
@@ -142,6 +142,39 @@ def test_down_products_cut_by_the_rule(gpu, monkeypatch, M, W, F, Fs, E, top, sl
         for a, b in ((got[:, :top], ref[:, :top]), (got[:, top:], ref[:, top:])):  # as above, the shared expert by itself
             assert float((a.double() - b.double()).norm() / b.double().norm()) <= 2.0 ** -8
             assert float((a - b).abs().max()) <= 2.0 ** -5 * float(b.abs().max())
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
+
+
+# The order of an expert's rows in the work list is whatever its atomics give; any of them gives the same bits, also where the last tiles are cut
+# over K: an expert in two row tiles, one of which is among them (by the rule and by force), and both
+@pytest.mark.parametrize("M,W,F,E,cut", [(350, 2112, 320, 3, 0), (600, 2048, 256, 2, 0), (700, 512, 384, 2, 2), (3000, 2048, 512, 8, 0)])
+def test_bits_do_not_depend_on_the_order_of_the_list(gpu, monkeypatch, M, W, F, E, cut):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2, moe_cut=cut))
+    ops.refresh_env()
+    try:
+        g = torch.Generator().manual_seed(M + F)
+        rnd = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16().to(gpu)  # noqa: E731
+        x, gate, up, down = rnd(M, W), rnd(E, F, W), rnd(E, F, W), rnd(E, W, F)
+        idx, w = (torch.arange(M)[:, None] % E).int().to(gpu), torch.rand(M, 1, generator=g).to(gpu)
+        tiles = -(-M // 64) + E + 1
+        lists = (torch.zeros(tiles * 64, dtype=torch.int32, device=gpu), torch.zeros(tiles, dtype=torch.int32, device=gpu), torch.zeros(1, dtype=torch.int32, device=gpu))
+        outs = []
+        for turn in range(3):
+            if turn:  # an order of its own inside every expert
+                ids, at = lists[0].cpu(), 0
+                for e in range(E):
+                    rows = M // E + (e < M % E)
+                    ids[at:at + rows] = torch.arange(e, M, E, dtype=torch.int32)[torch.randperm(rows, generator=g)]
+                    at += -(-rows // 64) * 64
+                lists[0].copy_(ids)
+            o = torch.full((M, W), float("nan"), device=gpu)
+            h = torch.zeros(M, F, dtype=torch.bfloat16, device=gpu)
+            ops.moe_grouped(x, idx, w, gate, up, down, None, None, None, *lists, h, o, aligned=turn > 0)
+            outs.append((h.cpu(), o.cpu()))
+        for h, o in outs[1:]:
+            assert torch.equal(h, outs[0][0]) and torch.equal(o, outs[0][1])
     finally:
         monkeypatch.undo()
         ops.refresh_env()
