@@ -17,13 +17,11 @@ DEV int vperm_tok(int off) { return ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4
 // gate and up rows written once and read once by a launch of their own: surodra-mid, 1500 rows of 2 x 8192, 1792 -> 1730 us a pass
 // (two layers), 200 rows 948 -> 813, decode of 16 rows of surodra-wide 678 -> 666.  Both are one formula with other factors: with a
 // branch per value the exponentials of a wave's values do not overlap, SiLU of 28672 x 4096, 100 rows, 50.7 -> 54.4 us, now 1.00 of
-// the first.  SiLU's exponent is z exactly: the square is bounded, so its factor of zero stays zero.  log2 e is in the factors, and the reciprocal is the
-// instruction's, 1 ulp, where a division took ten more instructions: 64 values a lane at a tile's end, 8192 x 28672 x 4096 1373 -> 1288 us, 3000 rows 555 -> 519, 1500 x 16384 x
-// 2048 GELU 89 -> 84; error of the bf16 results against 64 bits the same to five digits (0.0016562 at 2048 rows).
+// the first.  SiLU's exponent is z exactly: the square is bounded, so its factor of zero stays zero.  (The reciprocal instruction in place of the division is 5 % of
+// 8192 x 28672 x 4096, but one more rounding, and quotients below 2^-126 become zero.)
 DEV float gate_act(const GemmEpi& ep, float z) {
-  constexpr float kLog2e = 1.4426950408889634f, kGelu = 1.5957691216057308f;
-  const float c1 = -kLog2e * (ep.gelu ? kGelu : 1.0f), c3 = -kLog2e * (ep.gelu ? kGelu * 0.044715f : 0.0f);
-  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * __builtin_fmaf(c3, fminf(z * z, 1e30f), c1)));
+  const float c1 = ep.gelu ? 1.5957691216057308f : 1.0f, c3 = ep.gelu ? 1.5957691216057308f * 0.044715f : 0.0f;
+  return z / (1.0f + __expf(-(z * __builtin_fmaf(c3, fminf(z * z, 1e30f), c1))));
 }
 
 template <int MODE>
