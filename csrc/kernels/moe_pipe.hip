@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     char* st = smem + kStage + w * 2048;
     if constexpr (MODE != 1) {
       // The weights were the products' first operand: a lane has four hidden units of a row, which leaves through the wave's LDS in pieces of 16 bytes.
-      // Two-byte stores from 16 lanes a row, expf and a division / this, work list and both products, us: 1024 rows of 2048 x 1408 157 / 152, 400
+      // Two-byte stores from 16 lanes a row / this, work list and both products, us: 1024 rows of 2048 x 1408 157 / 152, 400
       // 111 / 106; 4096 x 3584, 2048 rows 756 / 732, 3000 995 / 965.
       constexpr int kPer = MODE == 0 ? 4 : 8;  // pieces of a row
       const int f0 = n0 + wn * 8 * kPer;
@@ -386,7 +386,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               if (MODE == 0) {
-                v[e] = (bf16)(silu(acc[m][2 * q][e] * wt) * (acc[m][2 * q + 1][e] * wt));
+                const float gv = acc[m][2 * q][e] * wt;
+                v[e] = (bf16)(gv / (1.0f + expf(-gv)) * (acc[m][2 * q + 1][e] * wt));
               } else {
                 const float z = acc[m][q][e] * wt;
                 v[e] = (bf16)(z > 0.0f ? z * z : 0.0f);

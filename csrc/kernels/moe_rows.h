@@ -24,8 +24,5 @@ DEV float in_weight(const MoeGroupedParams& p, int id) {
   return k < p.top ? slot_weight(p, row, k) : 1.0f;
 }
 
-// z / (1 + exp(-z)) by the exponential and reciprocal instructions, for results that are rounded to bf16
-DEV float silu(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z)); }
-
 }  // namespace
 }  // namespace dsse

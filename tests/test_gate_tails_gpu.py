@@ -1,4 +1,4 @@
-"""SiLU and GELU of every gate that bf16 holds, in the epilogues of the dense GEMMs, against float64: far below zero the
+"""SiLU and GELU of every gate that bf16 holds, in the epilogues of the dense and of the expert GEMMs, against float64: far below zero the
 result is small, not zero."""
 import pytest
 import torch
@@ -39,3 +39,25 @@ def test_dense(gpu, M, act):
     (ops.gemm_silu if act == "silu" else ops.gemm_gelu)(x.to(gpu), tile_weight(w[gate_up_perm(F)].contiguous()).to(gpu), out)
     for row in {0, M // 2, M - 1}:
         _check(out[row, :z.numel()].cpu(), want)
+
+
+@pytest.mark.parametrize("form", [1, 2, 3], ids=["stream", "pipeline", "direct"])
+def test_experts(gpu, monkeypatch, form):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=form))
+    ops.refresh_env()
+    try:
+        z, want = _gates("silu")
+        M, W, F = 70, 128, -(-z.numel() // 256) * 256
+        x = torch.zeros(M, W, dtype=torch.bfloat16)
+        x[:, 0] = 1
+        gate, up, down = (torch.zeros(1, *s, dtype=torch.bfloat16) for s in ((F, W), (F, W), (W, F)))
+        gate[0, :z.numel(), 0], up[0, :, 0] = z, 1
+        h, o = torch.zeros(M, F, dtype=torch.bfloat16, device=gpu), torch.zeros(M, W, device=gpu)
+        lists = (torch.zeros(n, dtype=torch.int32, device=gpu) for n in (4 * 64, 4, 1))
+        ops.moe_grouped(x.to(gpu), torch.zeros(M, 1, dtype=torch.int32, device=gpu), torch.ones(M, 1, device=gpu), gate.to(gpu), up.to(gpu), down.to(gpu),
+                        None, None, None, *lists, h, o)
+        for row in (0, M - 1):
+            _check(h[row, :z.numel()].cpu(), want)
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
