@@ -191,6 +191,7 @@ MoeForm moe_form(const MoeGroupedParams& p);
 // Parts of a row of o that the step is best computed in: S, or S + 1 where the shared expert's hidden units are worth two slices (moe_pipe.hip)
 constexpr int kMoeSlices = 2;
 int moe_parts(const MoeGroupedParams& p);
+bool moe_pipe_cuts(const MoeGroupedParams& p);  // moe_pipe.hip: whether a product of the step may cut tiles over K, and so needs ws
 std::vector<int> moe_pipe_walks(const MoeGroupedParams& p, int mode, const int* rows);  // moe_pipe.hip
 
 // Router, choice and work list of a decode-sized step in one launch.

@@ -538,9 +538,11 @@ void moe_grouped(const Tensor& x, const Tensor& topk_idx, const Tensor& topk_w, 
               "moe_grouped: this step's shared expert cannot be computed in ", p.parts - p.S + 1, " slices (moe_parts)");
   at::Tensor ws;
   if (p.M && dsse::moe_lines_ok(p) && dsse::moe_form(p) == dsse::MoeForm::kPipe) {
-    ws = at::empty({dsse::kMoeCutFloats}, o.options());
-    p.ws = ws.data_ptr<float>();
     p.cut = std::clamp(dsse::kernel_cfg_int("moe_cut", 0), 0, 8);
+    if (dsse::moe_pipe_cuts(p)) {
+      ws = at::empty({dsse::kMoeCutFloats}, o.options());
+      p.ws = ws.data_ptr<float>();
+    }
   }
   DSSE_CHECK_HIP(dsse_moe_grouped(&p, cur_stream()));
 }

@@ -34,6 +34,9 @@ __host__ __device__ inline Cut most_cut(int steps_r, int steps_s, int forced) {
   return Cut{steps_r < 32 || steps_s > steps_r ? 0 : left, kMostCut};
 }
 
+// Workgroups per XCD beyond one for each tile
+__host__ __device__ inline int pieces_room(Cut most) { return most.left > 0 && most.pieces > 1 ? kPieces : 0; }
+
 struct Item {
   int u;          // the tile, or the count of them: none
   int piece, of;  // its piece

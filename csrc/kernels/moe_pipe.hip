@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
   const int nb_r = blocks(p.F), nb_s = blocks(p.Fs);
   const int slices = MODE == 1 ? p.parts - p.S + 1 : 1;  // of the shared expert's hidden units
   const int tiles_s = (shared + tall - 1) / tall * nb_s, total_s = tiles_s * slices, total_r = row_tiles * nb_r;
-  const int steps_r = (MODE == 1 ? p.F : p.W) >> 6, steps_s = total_s ? (MODE == 1 ? p.Fs / slices : p.W) >> 6 : steps_r;
+  const int steps_r = (MODE == 1 ? p.F : p.W) >> 6, steps_s = total_s ? (MODE == 1 ? p.Fs / slices : p.W) >> 6 : steps_r;  // (as may_cut)
   const Cut most = most_cut(steps_r, steps_s, p.ws ? p.cut : 1);
 
   // One tile; a second round only if a choice list is not what it should be (the list is read again for it: no registers for it in the K loop)
@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     const int x = v & 7, item = v >> 3;
     const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0;
     const int r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
-    if (item >= (total_s + 7) / 8 + (total_r + 7) / 8 + kPieces) return;  // past every XCD's share
+    if (item >= (total_s + 7) / 8 + (total_r + 7) / 8 + pieces_room(most)) return;  // past every XCD's share
     Item it = item_of(item, ns + nr, most);
     const int u = it.u;
     if (u >= ns + nr) continue;
@@ -531,6 +531,12 @@ Height down_height(const MoeGroupedParams& p, int slices) {
   return best;
 }
 
+// The rule of the kernel, for every list that the step may have
+moe_cut::Cut may_cut(const MoeGroupedParams& p, int mode) {
+  const int steps_r = (mode == 1 ? p.F : p.W) >> 6, steps_s = mode == 1 && p.S > p.top ? p.Fs / (p.parts - p.S + 1) >> 6 : steps_r;
+  return moe_cut::most_cut(steps_r, steps_s, p.cut);
+}
+
 template <int MODE, bool ONCE>
 hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
   static bool attr_set = false;
@@ -540,7 +546,7 @@ hipError_t launch_moe_pipe(const MoeGroupedParams& p, hipStream_t st) {
     attr_set = true;
   }
   const int tall = MODE == 1 ? down_height(p, p.parts - p.S + 1).tall : moe_pipe_height(p, MODE);
-  const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8 + (p.ws ? mp::kPieces : 0));
+  const int64_t grid = 8 * ((routed_tiles(p, MODE, tall) + 7) / 8 + (shared_tiles(p, MODE, tall) + 7) / 8 + (p.ws ? moe_cut::pieces_room(may_cut(p, MODE)) : 0));
   hipLaunchKernelGGL((moe_pipe_kernel<MODE, ONCE>), dim3((unsigned)grid), dim3(512), mp::kLDS, st, p, tall);
   return hipGetLastError();
 }
@@ -554,6 +560,10 @@ hipError_t launch_moe_pipes(const MoeGroupedParams& p, hipStream_t st) {
 bool sixteens(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
+
+bool moe_pipe_cuts(const MoeGroupedParams& p) {
+  return moe_cut::pieces_room(may_cut(p, p.gate ? 0 : 2)) > 0 || moe_cut::pieces_room(may_cut(p, 1)) > 0;
+}
 
 bool moe_lines_ok(const MoeGroupedParams& p) {
   constexpr int64_t kRange = (int64_t)1 << 31;
@@ -581,7 +591,7 @@ std::vector<int> moe_pipe_walks(const MoeGroupedParams& p, int mode, const int* 
   std::vector<int> out;
   for (int x = 0; x < 8; ++x) {
     const int s0 = total_s * x / 8, ns = total_s * (x + 1) / 8 - s0, r0 = total_r * x / 8, nr = total_r * (x + 1) / 8 - r0;
-    for (int item = 0; item < (total_s + 7) / 8 + (total_r + 7) / 8 + kPieces; ++item) {
+    for (int item = 0; item < (total_s + 7) / 8 + (total_r + 7) / 8 + pieces_room(most); ++item) {
       Item it = item_of(item, ns + nr, most);
       if (it.u >= ns + nr) continue;
       const bool sh = it.u < ns;

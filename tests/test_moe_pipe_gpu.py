@@ -178,3 +178,24 @@ def test_bits_do_not_depend_on_the_order_of_the_list(gpu, monkeypatch, M, W, F, 
     finally:
         monkeypatch.undo()
         ops.refresh_env()
+
+
+# 16 K steps are never cut: no workspace; 32 may be
+@pytest.mark.parametrize("W,F,cuts", [(1024, 512, False), (2048, 512, True), (1024, 2048, True)])
+def test_workspace_only_where_a_tile_may_be_cut(gpu, monkeypatch, W, F, cuts):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2))
+    ops.refresh_env()
+    try:
+        M, E = 300, 4
+        z = lambda *s, **k: torch.zeros(*s, device=gpu, **k)  # noqa: E731
+        b, i = {"dtype": torch.bfloat16}, {"dtype": torch.int32}
+        args = (z(M, W, **b), z(M, 1, **i), z(M, 1), z(E, F, W, **b), z(E, F, W, **b), z(E, W, F, **b), None, None, None, z(10 * 64, **i), z(10, **i), z(1, **i),
+                z(M, F, **b), z(M, W))
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        ops.moe_grouped(*args)
+        assert (torch.cuda.max_memory_allocated() - before > 0) == cuts
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
