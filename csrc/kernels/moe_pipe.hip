@@ -405,7 +405,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         }
       continue;
     }
-    // fp32 rows, 128 bytes of 16 of them at a time
+    // fp32 rows, 128 bytes of 16 of them at a time, wherever o begins (memory takes 16 bytes at any multiple of four)
+    typedef f32x4 __attribute__((aligned(4))) f32x4_any;
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
       if ((m & 3) >= QI) continue;  // uniform
@@ -421,7 +422,7 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
         for (int it = 0; it < 2; ++it) {
           const int rr = it * 8 + (ln >> 3), piece = ln & 7, at = first_row + rr;
           const f32x4 v = *reinterpret_cast<const f32x4*>(st + rr * 128 + ((piece ^ (rr & 7)) << 4));
-          if (s_id[at] >= 0) *reinterpret_cast<f32x4*>(p.o + (int64_t)s_o[at] * p.W + f0 + 4 * piece) = v;
+          if (s_id[at] >= 0) *reinterpret_cast<f32x4_any*>(p.o + (int64_t)s_o[at] * p.W + f0 + 4 * piece) = v;
         }
       }
     }

@@ -199,3 +199,30 @@ def test_workspace_only_where_a_tile_may_be_cut(gpu, monkeypatch, W, F, cuts):
     finally:
         monkeypatch.undo()
         ops.refresh_env()
+
+
+# results that begin four bytes past a multiple of 16: the same bits, nothing beside them
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_results_of_any_alignment(gpu, monkeypatch, shift):
+    monkeypatch.setenv("DSSE_KERNEL_CFG", ops.kernel_cfg_env(moe_form=2))
+    ops.refresh_env()
+    try:
+        M, W, F, E, top = 300, 320, 192, 4, 2
+        g = torch.Generator().manual_seed(shift)
+        rnd = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16().to(gpu)  # noqa: E731
+        x, gate, up, down = rnd(M, W), rnd(E, F, W), rnd(E, F, W), rnd(E, W, F)
+        idx, w = ((torch.arange(M)[:, None] + torch.arange(top)) % E).int().to(gpu), torch.rand(M, top, generator=g).to(gpu)
+        n = M * top * W
+        bufs = []
+        for at in (0, shift):
+            tiles = -(-M * top // 64) + E + 1
+            lists = (torch.zeros(k, dtype=torch.int32, device=gpu) for k in (tiles * 64, tiles, 1))
+            buf = torch.full((n + 8,), float("nan"), device=gpu)
+            ops.moe_grouped(x, idx, w, gate, up, down, None, None, None, *lists, torch.zeros(M * top, F, dtype=torch.bfloat16, device=gpu),
+                            buf[at:at + n].view(M * top, W))
+            assert torch.isnan(buf[:at]).all() and torch.isnan(buf[at + n:]).all()
+            bufs.append(buf[at:at + n])
+        assert torch.equal(*bufs)
+    finally:
+        monkeypatch.undo()
+        ops.refresh_env()
