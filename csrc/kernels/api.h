@@ -129,6 +129,7 @@ hipError_t dsse_gemm_tiled(int mode, int cfg, int S, int partial_only, const voi
 hipError_t dsse_gemm_pipe(int mode, int bm, int S, int partial_only, const void* X, int ldx, int M, const void* W,
                           int K, int N, const dsse::GemmEpi* ep, float* part, hipStream_t st);
 size_t dsse_gemm_pipe_fix_floats(int bm, int S, int M, int N);
+int dsse_gemm_pipe_pairs(int tiles);  // times 256 workgroups of a launch that take two tiles each
 size_t dsse_gemm_ring_fix_floats(int nw, int S, int M, int N);
 hipError_t dsse_paged_attention(int mode, int num_work, const dsse::AttnParams* p, hipStream_t st);
 hipError_t dsse_flash_prefill(int num_work, const dsse::AttnParams* p, hipStream_t st);

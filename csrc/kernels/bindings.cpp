@@ -1593,6 +1593,7 @@ TORCH_LIBRARY(dsse, m) {
   m.def("kernels_abi_version() -> int", &kernels_abi_version);
   m.def("gemm_plan(int M, int N, int K, bool slab_consumer=False) -> (int, int, int, bool, float)", &gemm_plan);
   m.def("stream_plan(int M, int N, int K) -> (int, int)", &stream_plan);
+  m.def("gemm_pipe_pairs(int tiles) -> int", [](int64_t tiles) { return (int64_t)dsse_gemm_pipe_pairs((int)tiles); });
   m.def("gemm_fix_timeouts(int device=0) -> int", &gemm_fix_timeouts);
   m.def("gemm_fix_stamps(int device=0) -> Tensor", &gemm_fix_stamps);
   m.def("step_stamps_arm(int device=0, int cap=0) -> bool", &step_stamps_arm);

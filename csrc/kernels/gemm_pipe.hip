@@ -35,10 +35,9 @@
 //   * XCD-aware tile order (bijective remap, groups of 8 row blocks swept by column) as gemm_tiled.hip;
 //   * epilogues: bf16 results and SiLU / GELU·mul through a wave's own 4 KiB of LDS (16-byte row stores), fp32 / residual / QKV+RoPE /
 //     split-K partial slabs through gemm_epilogue.h;
-//   * from two rounds of tiles on a workgroup stays on its CU and takes every 256th tile: the requests past a tile's last step are the next
-//     one's first, and its results leave while they are under way.  A round a launch at a time / this, one MI355X, us: 8192 x 28672 x 4096 SiLU
-//     1425 / 1373, 8192 x 28672 x 2048 784 / 764, x 1024 480 / 445; 8192 x 4096 x 4096 196.5 / 193.5, x 2048 108 / 105, x 1024 64.5 / 60.0;
-//     1500 x 16384 x 2048 GELU 93 / 89.
+//   * from three rounds of tiles on most workgroups take two (pairs_of): the requests past the first tile's last step are the second
+//     one's first, and the first one's results leave while they are under way.  One tile each / this, one MI355X, us: 8192 x 28672 x 4096 SiLU
+//     1410 / 1397, 8192 x 28672 x 2048 775 / 765, x 1024 466 / 446; 3000 x 28672 x 4096 565 / 564, 3000 x 16384 x 2048 GELU 167 / 164.
 #include <algorithm>
 #include <type_traits>
 
@@ -78,6 +77,12 @@ constexpr int stores() {
   return MODE == kStoreBf16 ? 4 * QI : MODE == kSiluMul ? 2 * QI : 0;
 }
 
+// How many times kCUs workgroups of a launch of n tiles take two tiles each: as long as a round of single tiles follows.  Which CU a workgroup gets is decided
+// when one is free, so a CU that another stream holds (the collectives beside a tensor-parallel prompt) costs what it does without pairs: with one workgroup
+// per CU for all rounds, 8192 x 28672 x 4096 beside 16 held CUs took 2417 us and not 1574, 3000 rows 983 and not 633; with pairs up to the last
+// tile, 8192 x 4096 x 4096 332 and not 267.  In time units of a tile, no count of tiles from 512 to 4096 ends later beside 8 to 64 held CUs than without pairs.
+inline int pairs_of(int n) { return n < kCUs ? 0 : (n - kCUs) / (2 * kCUs); }
+
 // Whether 16 bytes of a bf16 result row are one aligned store
 __host__ __device__ inline bool wide_results(const GemmEpi& ep) {
   return reinterpret_cast<uintptr_t>(ep.out) % 16 == 0 && ep.ldo % 8 == 0;
@@ -101,7 +106,7 @@ __host__ __device__ inline bool wide_results(const GemmEpi& ep) {
 template <int MODE, int BM, bool FIX = false>
 __global__ void __launch_bounds__(512)
 gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restrict__ W, int K, int N, int Kr,
-                 GemmEpi ep, float* __restrict__ part) {
+                 GemmEpi ep, float* __restrict__ part, int pairs) {
   using namespace gp;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -128,7 +133,10 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     const int grp = tl / (GM * nbn), first = grp * GM, gsz = min(GM, nbm - first);
     return Tile{(first + (tl % (GM * nbn)) % gsz) * BM, (tl % (GM * nbn)) / gsz * 256, ks, tl};
   };
-  int bid = blockIdx.x;
+  // the first `pairs` times kCUs workgroups take two tiles each, kCUs apart, the others one
+  const bool two = (int)blockIdx.x < pairs * kCUs;
+  int bid = two ? blockIdx.x + blockIdx.x / kCUs * kCUs : blockIdx.x + pairs * kCUs;
+  const int second = bid + kCUs;
   Tile at = decode(bid);
 
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(X, (uint32_t)(((size_t)(M - 1) * ldx + K) * 2));
@@ -227,12 +235,12 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
   issue_b(0, 1);
   asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // A0 / B0 of step 0 landed everywhere
   if (wm == 1) asm volatile("s_barrier" ::: "memory");  // wave row 1 runs one barrier behind row 0
-  // A workgroup goes on to its next tile without a pause: the requests past a tile's last step are those of the next one's first, and its
-  // results leave while they are under way.
+  // A workgroup goes on to its second tile without a pause: the requests past the first one's last step are those of the second one's first, and the
+  // first one's results leave while they are under way.
   int t0 = 0;  // the tile's first step
   for (;; t0 += nk) {
-    const bool more = !FIX && stores<MODE, QI>() > 0 && bid + (int)gridDim.x < nwg;  // uniform
-    const Tile next = decode(more ? bid + (int)gridDim.x : bid);
+    const bool more = !FIX && stores<MODE, QI>() > 0 && two && bid < second;  // uniform
+    const Tile next = decode(more ? second : bid);
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
@@ -473,7 +481,7 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
     }
     if constexpr (FIX) stamp(ep, 5, now());
     if (!more) return;
-    bid += gridDim.x;
+    bid = second;
     at = next;
   }
 }
@@ -488,9 +496,9 @@ static hipError_t launch_pipe_bm(const bf16* X, int ldx, int M, const bf16* W, i
     attr_set = true;
   }
   const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256, n = nbm * nbn * S;
-  const bool stay = !FIX && n >= 2 * gp::kCUs && gp::stores<MODE, BM / 64>() > 0 && K / S >= 256 && gp::wide_results(ep) && kernel_cfg_int("pipe_stay", 1);
-  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(stay ? std::min(n, gp::kCUs) : n), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
-                     N, K / S, ep, part);
+  const int pairs = !FIX && gp::stores<MODE, BM / 64>() > 0 && K / S >= 256 && gp::wide_results(ep) && kernel_cfg_int("pipe_stay", 1) ? gp::pairs_of(n) : 0;
+  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(n - pairs * gp::kCUs), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
+                     N, K / S, ep, part, pairs);
   return hipGetLastError();
 }
 template <int MODE, bool FIX = false>
@@ -539,6 +547,8 @@ extern "C" hipError_t dsse_gemm_pipe(int mode, int bm, int S, int partial_only, 
   if (e != hipSuccess || partial_only) return e;
   return launch_splitk_reduce(mode, part, S, M, N, *ep, st);
 }
+
+extern "C" int dsse_gemm_pipe_pairs(int tiles) { return dsse::gp::pairs_of(tiles); }
 
 // Workspace floats of the in-launch fix-up (partial_only = 2): S - 1 register-order slots per tile.
 extern "C" size_t dsse_gemm_pipe_fix_floats(int bm, int S, int M, int N) {

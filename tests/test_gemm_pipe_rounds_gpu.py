@@ -1,4 +1,4 @@
-"""The 256 x 256 pipeline where a workgroup goes on from tile to tile (two rounds of 256 tiles and more): the fewest K steps that it takes, one more
+"""The 256 x 256 pipeline from two rounds of 256 tiles on, from three on with workgroups that go on to a second tile: the fewest K steps that they take, one more
 and an odd count, a last round of a few tiles, ragged rows, a half-empty last column block, every tile height; results that are not aligned to 16 bytes."""
 import pytest
 import torch
@@ -19,8 +19,11 @@ def tile(monkeypatch):
     ops.refresh_env()
 
 
-# tiles of 256 / 192 / 128 rows x 256 columns: 513, 531, 989 and 533 of them; the half-empty column block as it is planned
-@pytest.mark.parametrize("cfg,M,N,K", [("8", 2050, 14592, 256), ("8", 2300, 15104, 384), ("9", 8200, 5888, 256), ("10", 1537, 10496, 640), (None, 4200, 8320, 2048)])
+# tiles of 256 / 192 / 128 rows x 256 columns: 513, 531, 989, 533 and 561 of them, the half-empty column block as it is planned; and 774, 801, 780, 825 and 1287:
+# one round of pairs and two
+@pytest.mark.parametrize("cfg,M,N,K", [
+    ("8", 2050, 14592, 256), ("8", 2300, 15104, 384), ("9", 8200, 5888, 256), ("10", 1537, 10496, 640), (None, 4200, 8320, 2048),
+    ("8", 2050, 22016, 256), ("8", 2300, 22784, 384), ("10", 1537, 15360, 640), (None, 6200, 8320, 2048), ("8", 2050, 36608, 384)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_rounds(gpu, tile, cfg, M, N, K, shift):
     tile(cfg)
