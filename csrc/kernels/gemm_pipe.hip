@@ -65,7 +65,6 @@ constexpr int kA = 256 * 128;     // A image of one K step: 256 rows x 64 bf16, 
 constexpr int kB = 16 * 2048;     // B image: 16 column tiles x two 1 KiB k-step blocks
 constexpr int kBuf = kA + kB;     // 64 KiB per K step
 constexpr int kStage = 4096;      // a wave's rows of the result on their way to 16-byte stores, beside the two images
-constexpr size_t kLDS = 2 * (size_t)kBuf + 8 * kStage;
 constexpr int kCUs = 256;
 
 // bf16 results: products with the weights as their first operand, so that a lane has four columns of a row, and rows that leave through LDS as 16-byte
@@ -82,6 +81,11 @@ constexpr int stores() {
 // per CU for all rounds, 8192 x 28672 x 4096 beside 16 held CUs took 2417 us and not 1574, 3000 rows 983 and not 633; with pairs up to the last
 // tile, 8192 x 4096 x 4096 332 and not 267.  In time units of a tile, no count of tiles from 512 to 4096 ends later beside 8 to 64 held CUs than without pairs.
 inline int pairs_of(int n) { return n < kCUs ? 0 : (n - kCUs) / (2 * kCUs); }
+
+template <int MODE, int QI>
+constexpr size_t lds() {
+  return 2 * (size_t)kBuf + (stores<MODE, QI>() > 0 ? 8 * kStage : 0);
+}
 
 // Whether 16 bytes of a bf16 result row are one aligned store
 __host__ __device__ inline bool wide_results(const GemmEpi& ep) {
@@ -489,15 +493,16 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
 template <int MODE, int BM, bool FIX>
 static hipError_t launch_pipe_bm(const bf16* X, int ldx, int M, const bf16* W, int K, int N, int S, const GemmEpi& ep,
                                  float* part, hipStream_t st) {
+  constexpr size_t kLDS = gp::lds<MODE, BM / 64>();
   static bool attr_set = false;
   if (!attr_set) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pipe_kernel<MODE, BM, FIX>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gp::kLDS);
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLDS);
     attr_set = true;
   }
   const int nbm = (M + BM - 1) / BM, nbn = (N + 255) / 256, n = nbm * nbn * S;
   const int pairs = !FIX && gp::stores<MODE, BM / 64>() > 0 && K / S >= 256 && gp::wide_results(ep) && kernel_cfg_int("pipe_stay", 1) ? gp::pairs_of(n) : 0;
-  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(n - pairs * gp::kCUs), dim3(512), gp::kLDS, st, X, ldx, M, W, K,
+  hipLaunchKernelGGL((gemm_pipe_kernel<MODE, BM, FIX>), dim3(n - pairs * gp::kCUs), dim3(512), kLDS, st, X, ldx, M, W, K,
                      N, K / S, ep, part, pairs);
   return hipGetLastError();
 }
