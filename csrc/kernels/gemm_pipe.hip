@@ -401,13 +401,15 @@ gemm_pipe_kernel(const bf16* __restrict__ X, int ldx, int M, const bf16* __restr
       if (!cols) return;
       const int ldo = MODE == kPartial ? (ep.parts ? ep.parts : 1) * N : ep.ldo;
       float* out = MODE == kPartial ? partial_of(ep, part, at.ks, M, N) : reinterpret_cast<float*>(ep.out);
-      const __amdgpu_buffer_rsrc_t to = make_rsrc(out + (size_t)min(row0, M - 1) * ldo + tile0 * 16, 0x7fffffffu);
+      // a weight of up to 2 GiB has 2^23 columns at K = 128 (slices and all): a wave's rows span up to 127 * 4 * 2^23 bytes, so nearly all of a descriptor's 4 GiB
+      constexpr uint32_t kPast = 0xfffffe00u;
+      const __amdgpu_buffer_rsrc_t to = make_rsrc(out + (size_t)min(row0, M - 1) * ldo + tile0 * 16, kPast);
 #pragma unroll
       for (int k = 0; k < 2 * QI; ++k)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int m = row_of(k) + 4 * g + i;
-          const uint32_t row = m < M ? (uint32_t)(m - row0) * (uint32_t)ldo * 4 + 4 * r : kOOB;
+          const uint32_t row = m < M ? (uint32_t)(m - row0) * (uint32_t)ldo * 4 + 4 * r : kPast;
 #pragma unroll
           for (int nt = 0; nt < 4; ++nt) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[mt_of(k)][nt][i]), to, row + 64 * nt, 0, 0);
         }
