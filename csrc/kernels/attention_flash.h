@@ -61,7 +61,10 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
   const int jb = p.work_kb ? p.work_kb[2 * item] : 0;
   const int je = p.work_kb ? min(nblk, p.work_kb[2 * item + 1]) : nblk;
   const int pslot = p.work_slot ? p.work_slot[item] : -1;
-  const int w_first_pos = pos0 + q0;
+  const int w_first_pos = pos0 + q0, w_last_pos = pos0 + min(qlen, q0 + 32) - 1;
+  // Key blocks from jv on (the tile's last one, or none) are after all of this wave's queries: skipped, since a weight of zero does not keep a value that is
+  // not finite out of the sum
+  const int jv = min(je, w_last_pos / kBK + 1);
   const int head = h * G + hs * HG + wh;
   const int* bt = p.block_tables + (size_t)b * p.max_blocks;
   const int npages = (kmax + kBS - 1) / kBS;
@@ -295,15 +298,22 @@ DEV void flash_prefill(const AttnParams& p, unsigned* stamps, int block, char* s
     stamp(j, 5);
   };
   // unrolled by the ring size: each block's LDS slot is a compile-time offset (no per-read address arithmetic)
-  if (jb < je) step(jb, std::integral_constant<int, 0>{}, std::true_type{});
-  for (int j = jb + 1; j < je; j += kRing) {
+  if (jb < jv) step(jb, std::integral_constant<int, 0>{}, std::true_type{});
+  for (int j = jb + 1; j < jv; j += kRing) {
     step(j, std::integral_constant<int, 1>{}, std::false_type{});
-    if (j + 1 < je) step(j + 1, std::integral_constant<int, 2>{}, std::false_type{});
-    if (j + 2 < je) step(j + 2, std::integral_constant<int, 3>{}, std::false_type{});
-    if (j + 3 < je) step(j + 3, std::integral_constant<int, 0>{}, std::false_type{});
+    if (j + 1 < jv) step(j + 1, std::integral_constant<int, 2>{}, std::false_type{});
+    if (j + 2 < jv) step(j + 2, std::integral_constant<int, 3>{}, std::false_type{});
+    if (j + 3 < jv) step(j + 3, std::integral_constant<int, 0>{}, std::false_type{});
+  }
+  for (int j = max(jb, jv); j < je; ++j) {  // the barriers and the DMA of a step
+    if (!lag) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
+    else asm volatile("s_barrier" ::: "memory");
+    issue_block((j - jb + 2) % kRing);
+    if (!lag) asm volatile("s_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(IPW) : "memory");
   }
   if (!lag) asm volatile("s_barrier" ::: "memory");
-  if (jb < je) {
+  if (jb < jv) {
     pv(0);
     pv(1);
   }
