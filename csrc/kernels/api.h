@@ -136,6 +136,7 @@ hipError_t dsse_flash_prefill(int num_work, const dsse::AttnParams* p, hipStream
 hipError_t dsse_attn_combine(int num_work, const dsse::AttnParams* p, hipStream_t st);
 // decode rows d (mode 0) and prompt tiles f (mode 2) of one layer in one launch; hipErrorNotSupported: nothing done, not its sizes
 hipError_t dsse_mixed_attention(int rows, const dsse::AttnParams* d, int num_work, const dsse::AttnParams* f, hipStream_t st);
+int dsse_mixed_attention_waves(int group, int rows, int hkv, int nparts, int num_work, int forced);  // waves per decode item, 0: not its sizes
 hipError_t dsse_sample(int B, const dsse::SampleParams* p, hipStream_t st);
 hipError_t dsse_sample_pick(int B, int world, const void* cand, const dsse::SampleParams* p,
                             hipStream_t st);

@@ -49,15 +49,22 @@ hipError_t launch(int tiles, int rows, const AttnParams& d, const AttnParams& f,
 }  // namespace
 }  // namespace dsse
 
+// Waves per (row, kv head, key partition) item of the one launch; 0: the step goes in two.  By the count of items, since how many keys an item has is known on
+// the device only.  2 / 4 / 8, us: 1024 items of 500 keys 61.1 / 62.4 / 66.4, 800 of 300 31.1 / 33.7 / 37.2; 512 of 512 43.6 / 37.8 / 41.2, of 1000
+// (16 rows of 4000 in four partitions) 85.0 / 63.8 / 67.1, of 375 37.9 / 35.5 / 36.4; 384 of 170 22.2 / 19.0 / 19.2, 128 of 75 15.3 / 15.1 / 13.5.  What the
+// rule gives away: 512 of 256 keys 29.2 / 31.3 / 29.4.  (Two pages in flight per wave are 0 to 5 us behind one; one wave per item 73 us at 512 keys.)
+extern "C" int dsse_mixed_attention_waves(int group, int rows, int hkv, int nparts, int num_work, int forced) {
+  if (group != 4 || rows <= 0 || num_work <= 0) return 0;
+  const int items = rows * hkv * nparts, kwv = forced ? forced : items > 640 ? 2 : items > 384 ? 4 : 8;
+  return kwv < 2 ? 2 : kwv;
+}
+
 extern "C" hipError_t dsse_mixed_attention(int rows, const dsse::AttnParams* d, int num_work, const dsse::AttnParams* f, hipStream_t st) {
   using namespace dsse;
-  if (d->group != 4 || f->group != 4 || rows <= 0 || num_work <= 0) return hipErrorNotSupported;
-  const int tiles = num_work * f->hkv, items = rows * d->hkv * d->nparts;
-  // Waves per item, 2 / 4 / 8, us: 1024 items of 500 keys 61.1 / 62.4 / 66.4, 800 of 300 31.1 / 33.7 / 37.2; 512 of 512 43.6 / 37.8 / 41.2, of 1000
-  // (16 rows of 4000 in four partitions) 85.0 / 63.8 / 67.1, of 375 37.9 / 35.5 / 36.4, of 256 29.2 / 31.3 / 29.4; 384 of 170 22.2 / 19.0 / 19.2, 128 of
-  // 75 15.3 / 15.1 / 13.5.  (Two pages in flight per wave are 0 to 5 us behind one; one wave per item 73 us at 512 keys.)
-  const int kwv = d->kwv ? d->kwv : items > 640 ? 2 : items > 384 ? 4 : 8;
-  const hipError_t e = kwv <= 2 ? launch<2>(tiles, rows, *d, *f, st) : kwv == 4 ? launch<4>(tiles, rows, *d, *f, st) : launch<8>(tiles, rows, *d, *f, st);
+  const int kwv = f->group == d->group ? dsse_mixed_attention_waves(d->group, rows, d->hkv, d->nparts, num_work, d->kwv) : 0;
+  if (!kwv) return hipErrorNotSupported;
+  const int tiles = num_work * f->hkv;
+  const hipError_t e = kwv == 2 ? launch<2>(tiles, rows, *d, *f, st) : kwv == 4 ? launch<4>(tiles, rows, *d, *f, st) : launch<8>(tiles, rows, *d, *f, st);
   return e == hipSuccess && d->nparts > 1 ? dsse_attn_combine(rows, d, st) : e;
 }
 

@@ -1100,6 +1100,14 @@ void paged_attention(int64_t mode, const Tensor& q, const Tensor& k_cache, const
   else DSSE_CHECK_HIP(dsse_paged_attention((int)mode, num_work, &p, cur_stream()));
 }
 
+bool one_mixed_launch() { return env_int("attn_mixed", 1) && !env_int("flash_hg", 0); }
+
+// Waves per (row, kv head, key partition) item where mixed_attention is one launch, 0 where it is two
+int64_t mixed_attention_waves(int64_t rows, int64_t hq, int64_t hkv, int64_t nparts, int64_t num_work) {
+  TORCH_CHECK(hkv > 0 && hq % hkv == 0, "heads");
+  return one_mixed_launch() ? dsse_mixed_attention_waves((int)(hq / hkv), (int)rows, (int)hkv, (int)nparts, (int)num_work, env_int("attn_kwv", 0)) : 0;
+}
+
 // Attention of a mixed step: decode rows (paged_attention mode 0) and prompt tiles (mode 2) over the same q, pages and result; one launch
 // where the kernel takes the step (dsse_mixed_attention), else both.
 void mixed_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, Tensor& out, Tensor& part_o, Tensor& part_ml,
@@ -1117,7 +1125,7 @@ void mixed_attention(const Tensor& q, const Tensor& k_cache, const Tensor& v_cac
   };
   dsse::AttnParams d = params(rows, part, nparts, 1, 4), f = params(tiles, tile_part, 1, 4, 1);
   const int nr = (int)rows[4].numel(), nt = (int)tiles[4].numel();
-  if (env_int("attn_mixed", 1) && !env_int("flash_hg", 0)) {
+  if (one_mixed_launch()) {
     const hipError_t e = dsse_mixed_attention(nr, &d, nt, &f, cur_stream());
     if (e == hipSuccess) return;
     TORCH_CHECK(e == hipErrorNotSupported, "dsse kernel launch failed: ", hipGetErrorString(e));
@@ -1593,6 +1601,7 @@ TORCH_LIBRARY(dsse, m) {
   m.def("kernels_abi_version() -> int", &kernels_abi_version);
   m.def("gemm_plan(int M, int N, int K, bool slab_consumer=False) -> (int, int, int, bool, float)", &gemm_plan);
   m.def("stream_plan(int M, int N, int K) -> (int, int)", &stream_plan);
+  m.def("mixed_attention_waves(int rows, int hq, int hkv, int nparts, int tiles) -> int", &mixed_attention_waves);
   m.def("gemm_pipe_pairs(int tiles) -> int", [](int64_t tiles) { return (int64_t)dsse_gemm_pipe_pairs((int)tiles); });
   m.def("gemm_fix_timeouts(int device=0) -> int", &gemm_fix_timeouts);
   m.def("gemm_fix_stamps(int device=0) -> Tensor", &gemm_fix_stamps);

@@ -12,13 +12,13 @@ pytestmark = pytest.mark.gpu
 
 # decode contexts on both sides of a page, an idle slot, prompts that end inside a tile, begin behind cached tokens or have one row, padded work items;
 # counts of (row, kv head, partition) items that 2, 4 and 8 waves each take, and that leave groups of a workgroup without one; partitions that
-# are empty; one kv head; groups of heads that go in two launches
-@pytest.mark.parametrize("ctxs,nparts,prompts,hq,hkv", [
-    ([1, 31, 32, 33, 300], 1, [(45, 45)], 32, 8), ([40, 700], 3, [(64, 64), (1, 90)], 32, 8), ([5], 1, [(130, 200)], 4, 1),
-    ([17] * 49, 1, [(65, 65)], 32, 8), ([33, 64] * 41, 1, [(3, 3)], 32, 8), ([600] * 7, 2, [(300, 1000)], 32, 8), ([77] * 3, 1, [(70, 70)], 16, 8),
-    ([90] * 97, 1, [(20, 20)], 4, 1)])
+# are empty; one kv head; groups of heads that go in two launches (waves 0)
+@pytest.mark.parametrize("ctxs,nparts,prompts,hq,hkv,waves", [
+    ([1, 31, 32, 33, 300], 1, [(45, 45)], 32, 8, 8), ([40, 700], 3, [(64, 64), (1, 90)], 32, 8, 8), ([5], 1, [(130, 200)], 4, 1, 8),
+    ([17] * 49, 1, [(65, 65)], 32, 8, 4), ([33, 64] * 41, 1, [(3, 3)], 32, 8, 2), ([600] * 7, 2, [(300, 1000)], 32, 8, 8), ([77] * 3, 1, [(70, 70)], 16, 8, 0),
+    ([90] * 97, 1, [(20, 20)], 4, 1, 8)])
 @pytest.mark.parametrize("idle", [False, True])
-def test_mixed_attention(gpu, ctxs, nparts, prompts, hq, hkv, idle):
+def test_mixed_attention(gpu, ctxs, nparts, prompts, hq, hkv, waves, idle):
     g = torch.Generator().manual_seed(sum(ctxs) + hq + len(prompts))
     B, C = len(ctxs), sum(n for n, _ in prompts)
     lens = ctxs + [c for _, c in prompts]
@@ -45,6 +45,7 @@ def test_mixed_attention(gpu, ctxs, nparts, prompts, hq, hkv, idle):
         row += n
     items += [(len(prompts), 0)] * 3  # padded items point at an empty sequence
     tiles = (bt[B:], i32(qs + [0]), i32(ql + [0]), i32([c for _, c in prompts] + [0]), i32([s for s, _ in items]), i32([t for _, t in items]))
+    assert torch.ops.dsse.mixed_attention_waves(B, hq, hkv, nparts, len(items)) == waves
     part = 0 if nparts > 1 else math.ceil(max(ctxs) / 128) * 128
     ref = torch.zeros_like(q)
     R.paged_attention(0, q[:B], kc, vc, *rows, ref[:B])
