@@ -8,13 +8,6 @@
 namespace dsse {
 namespace {
 
-template <int E> struct Part;
-template <> struct Part<1> { typedef float V; };
-template <> struct Part<2> { typedef __attribute__((ext_vector_type(2))) float V; };
-
-DEV float part_at(float v, int) { return v; }
-DEV float part_at(Part<2>::V v, int e) { return v[e]; }
-
 // Tiles of 16 TM rows x 16 TN columns; KW waves, each with 32 / KW k of every chunk of 32 for all TM TN accumulators, meet in LDS at the end.
 //
 // What bounds it: the fp32 matrix rate, and behind it the DMA instructions: one that misses L1 keeps its wave from issuing for some 40 clocks, whatever is
@@ -27,7 +20,8 @@ template <int TM, int TN, int KW, int STAGES>
 __global__ __launch_bounds__(64 * KW) void gemm_rm_split_kernel(GemmRmParams p) {
   constexpr int kRows = 16 * TM, kCols = 16 * TN, kPieces = 2 * (TM + TN), kPer = (kPieces + KW - 1) / KW;  // DMA instructions (8 rows), per wave
   constexpr int kSlot = KW * kPer * 1024, E = 8 / KW, T = TM * TN;
-  typedef typename Part<E>::V V;
+  static_assert(KW == 4, "a wave's part of a fragment is two k");
+  typedef __attribute__((ext_vector_type(2))) float V;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -86,7 +80,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_rm_split_kernel(GemmRmParams p) 
       constexpr int q = decltype(m)::value;
       if constexpr (q < kProducts) {
         constexpr int e = q / T, i = T - 1 - q % T;
-        acc[i] = mfma16x16x4(part_at(a[cur][i / TN], e), part_at(b[cur][i % TN], e), acc[i]);
+        acc[i] = mfma16x16x4(a[cur][i / TN][e], b[cur][i % TN][e], acc[i]);
         __builtin_amdgcn_sched_barrier(0);
         constexpr int s0 = q * kSide / kProducts, s1 = (q + 1) * kSide / kProducts;
 #pragma unroll
