@@ -8,7 +8,7 @@
 //   workgroup  = one KV head x 64 query tokens; 2G waves (G = Hq/Hkv q heads x 2 halves of 32
 //                queries), so every K/V byte staged in LDS feeds 2G waves (GQA reuse in LDS);
 //   key loop   = 64 keys (two 32-token pages) per block, a 4-block LDS ring (4 x 32 KiB) filled by LDS-DMA
-//                three blocks ahead;
+//                two blocks ahead;
 //   scores     = Sᵀ = K·Qᵀ (keys on MFMA rows, queries on lanes): a query's softmax statistics live
 //                in one lane column, and the exponentiated scores are already the B operand of
 //                Oᵀ = Vᵀ·Pᵀ — the V cache stores each page transposed with the token permutation
