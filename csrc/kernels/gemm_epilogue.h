@@ -17,8 +17,8 @@ DEV int vperm_tok(int off) { return ((off & 15) >> 2) * 8 + ((off >> 4) & 1) * 4
 // gate and up rows written once and read once by a launch of their own: surodra-mid, 1500 rows of 2 x 8192, 1792 -> 1730 us a pass
 // (two layers), 200 rows 948 -> 813, decode of 16 rows of surodra-wide 678 -> 666.  Both are one formula with other factors: with a
 // branch per value the exponentials of a wave's values do not overlap, SiLU of 28672 x 4096, 100 rows, 50.7 -> 54.4 us, now 1.00 of
-// the first.  SiLU's exponent is z exactly: the square is bounded, so its factor of zero stays zero.  (The reciprocal instruction in place of the division is 5 % of
-// 8192 x 28672 x 4096, but one more rounding, and quotients below 2^-126 become zero.)
+// the first.  SiLU's exponent is z exactly: the square is bounded, so its factor of zero stays zero.  (The reciprocal instruction in place of the division is 2 to 3 % of
+// 8192 and 3000 rows of 28672 x 4096, but one more rounding, and quotients below 2^-126 become zero.)
 DEV float gate_act(const GemmEpi& ep, float z) {
   const float c1 = ep.gelu ? 1.5957691216057308f : 1.0f, c3 = ep.gelu ? 1.5957691216057308f * 0.044715f : 0.0f;
   return z / (1.0f + __expf(-(z * __builtin_fmaf(c3, fminf(z * z, 1e30f), c1))));

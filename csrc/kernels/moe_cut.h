@@ -21,10 +21,10 @@ struct Cut {
 
 // steps_r, steps_s: K steps of a routed and of a shared tile (steps_r where there is none); forced: 0, or pieces by force (1: no tile is cut).
 // Pieces pay where they are few -- tiles of a round that is half empty run faster than those of a full one -- and long, and where no
-// shared expert's longer walk is what the launch waits for (down products).  Without / with, one MI355X, work list and both products, us: 16 experts, top
-// 2 and a shared one, 2048 x 1408, 1024 rows (264 tiles, one left per XCD) 152 / 144; 4096 x 3584, 200 rows 320 / 300, 1300 567 / 541,
-// 1500 609 / 584, 3000 1030 / 1007.  With more than these left it turns: 2048 x 1408, three or four tiles left, 1100 rows 151 / 154, five to eight 1300
-// rows 154 / 163, 1500 165 / 170; 16 K steps, 1024 x 2048, 2500 rows 174 / 178.
+// shared expert's longer walk is what the launch waits for (down products).  Without / with, one MI355X, work list and both products, us, mean of six random
+// choices: 16 experts, top 2 and a shared one, 2048 x 1408, 1024 rows (264 tiles, one left per XCD) 164 / 154; 4096 x 3584, 1300 rows 553 / 526, 1500
+// 592 / 568, 3000 1017 / 1005; 200 and 700 rows, whose experts' tiles are not left over, 311 and 405 in both.  With more than these left it turns (forced): 2048 x
+// 1408, three or four tiles left, 1100 rows 151 / 154, five to eight 1300 rows 154 / 163, 1500 165 / 170; 16 K steps, 1024 x 2048, 2500 rows 174 / 178.
 __host__ __device__ inline Cut most_cut(int steps_r, int steps_s, int forced) {
   if (forced) {
     const int fit = (steps_r < steps_s ? steps_r : steps_s) / kLeast;

@@ -23,8 +23,8 @@
 // give every expert's place); the host knows only a bound of the tile count.
 //
 // Measured (one MI355X, work list and both products, against the 64-row tiles of moe.hip): 3000 rows of 4096 x 3584, 16
-// experts, top 2, shared 7168: 2369 -> 953 us (1109 TFLOP/s); 2048 rows: 1695 -> 720; 1024 rows of 2048 x 1408, shared
-// 2816: 245 -> 150; 1024 rows of 1024 x 512, 8 experts: 49 -> 38.  Up to 192 rows moe_stream.hip takes
+// experts, top 2, shared 7168: 2369 -> 1005 us (1052 TFLOP/s); 2048 rows: 1695 -> 757; 1024 rows of 2048 x 1408, shared
+// 2816: 245 -> 154; 1024 rows of 1024 x 512, 8 experts: 49 -> 39.  Up to 192 rows moe_stream.hip takes
 // the sizes whose weights it need not read twice, or the kernels of moe.hip a few rows of small experts (moe_form).
 #include <algorithm>
 #include <cmath>
@@ -370,8 +370,8 @@ __global__ void __launch_bounds__(512) moe_pipe_kernel(MoeGroupedParams p, int t
     char* st = smem + kStage + w * 2048;
     if constexpr (MODE != 1) {
       // The weights were the products' first operand: a lane has four hidden units of a row, which leaves through the wave's LDS in pieces of 16 bytes.
-      // Two-byte stores from 16 lanes a row / this, work list and both products, us: 1024 rows of 2048 x 1408 157 / 152, 400
-      // 111 / 106; 4096 x 3584, 2048 rows 756 / 732, 3000 995 / 965.
+      // Two-byte stores from 16 lanes a row (the down product's: four bytes, 64 of four rows) / this, work list and both products, no tile cut, us: 1024
+      // rows of 2048 x 1408 166 / 164, 400 111 / 108; 4096 x 3584, 1300 rows 564 / 553, 2048 769 / 756, 3000 1029 / 1017.
       constexpr int kPer = MODE == 0 ? 4 : 8;  // pieces of a row
       const int f0 = n0 + wn * 8 * kPer;
       if (f0 < N)  // uniform: N % 64 == 0
